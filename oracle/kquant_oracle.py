@@ -28,9 +28,10 @@ _ref: Optional[ctypes.CDLL] = None
 
 
 def build(with_reference: bool = True) -> None:
-    """Compile the oracle, and the reference harness when the checkout is present."""
+    """Compile the oracle, and the reference harness when the checkout is present (an empty
+    directory in its place is no checkout)."""
     subprocess.run(["make", "-C", str(HERE), "all"], check=True, capture_output=True)
-    if with_reference and REFERENCE_ROOT.exists():
+    if with_reference and (REFERENCE_ROOT / "neuralfn").is_dir():
         subprocess.run(["make", "-C", str(HERE), "ref"], check=True, capture_output=True)
 
 
