@@ -1,4 +1,5 @@
-"""Build recipe for the HIP library and the host-side library (quantizer, GGUF tensor table).
+"""Build recipe for the HIP library, the Python front end in front of it and the host-side
+library (quantizer, GGUF tensor table).
 
 `build_all()` compiles every source for gfx950 with hipcc and links
 `neuralfn_amd/lib/libnfn_mi355_tile_ops.so` (and the benchmark's measurement aids into
@@ -21,6 +22,7 @@ OBJ_DIR = PACKAGE / "build"
 TILE_OPS_LIB = LIB_DIR / "libnfn_mi355_tile_ops.so"
 PROBES_LIB = LIB_DIR / "libnfn_mi355_probes.so"
 HOST_LIB = LIB_DIR / "libnfn_mi355_kquant_host.so"
+FRONT_END = PACKAGE / "_front_end.so"  # a Python extension module: imported as neuralfn_amd._front_end
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -101,10 +103,24 @@ def build_host() -> Path:
     return HOST_LIB
 
 
+def build_front_end() -> Path:
+    """The extension module that turns tensors into C ABI calls (host code; torch's headers and libraries)."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    includes = [*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"]]
+    libraries = cpp_extension.library_paths("cuda")
+    _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+          "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", *(f"-isystem{path}" for path in includes),
+          str(CSRC / "python" / "front_end.cpp"), "-o", str(FRONT_END),
+          *(f"-L{path}" for path in libraries), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"])
+    return FRONT_END
+
+
 def build_all() -> None:
     build_tile_ops()
     build_probes()
     build_host()
+    build_front_end()
 
 
 if __name__ == "__main__":

@@ -11,9 +11,7 @@ from __future__ import annotations
 import ctypes
 
 from . import tile_ops
-from .tile_ops import (BlockAttentionDescriptor, CacheCommitDescriptor,
-                       FusedDecodeAttentionDescriptor, GqaDecodeDescriptor, PackedWeight, check,
-                       load)
+from .tile_ops import CacheCommitDescriptor, PackedWeight, check, load
 
 ROPE_HALF_SPLIT = 0
 ROPE_INTERLEAVED = 1
@@ -70,23 +68,8 @@ def qk_norm_scale_rope(query, key, query_weight=None, key_weight=None, eps: floa
                        query_centered: bool = False, key_centered: bool = False) -> None:
     """In place: per-head RMS norm, query scale, rope.  query [heads, head_dim] or
     [rows, heads, head_dim] (then key [rows, kv_heads, head_dim], row r at position + r)."""
-    stream = _stream()
-    q_descriptor = query_weight.descriptor(stream) if query_weight is not None else None
-    k_descriptor = key_weight.descriptor(stream) if key_weight is not None else None
-    q_pointer = ctypes.byref(q_descriptor) if q_descriptor is not None else None
-    k_pointer = ctypes.byref(k_descriptor) if k_descriptor is not None else None
-    if query.dim() == 3:
-        rows, query_heads, head_dim = query.shape
-        check(load().nfn_native_tile_glimmer_qk_norm_scale_rope_batch_float32_v1(
-            query.data_ptr(), key.data_ptr(), q_pointer, k_pointer, rows, query_heads,
-            key.shape[1], head_dim, eps, query_centered, key_centered, query_scale, position,
-            theta, layout, apply_rope, stream), "qk_norm_scale_rope_batch")
-        return
-    query_heads, head_dim = query.shape
-    check(load().nfn_native_tile_glimmer_qk_norm_scale_rope_float32_v1(
-        query.data_ptr(), key.data_ptr(), q_pointer, k_pointer, query_heads, key.shape[0],
-        head_dim, eps, query_centered, key_centered, query_scale, position, theta, layout,
-        apply_rope, stream), "qk_norm_scale_rope")
+    tile_ops.native().qk_norm_scale_rope(query, key, query_weight, key_weight, eps, query_scale, position, theta,
+                                         layout, apply_rope, query_centered, key_centered)
 
 
 def fused_decode_attention(query, key, value, key_cache, value_cache, position: int,
@@ -100,46 +83,9 @@ def fused_decode_attention(query, key, value, key_cache, value_cache, position: 
     With `device_position` (an int64 tensor of one element) the kernels read the position when
     they run and `position` / `first_key_position` are ignored; `sliding_window` then bounds a
     local layer's keys.  With `workspace` (gqa_decode_workspace) the attention is the split form."""
-    import torch
-    if out is None:
-        out = torch.empty_like(query)
-    stream = _stream()
-    d = FusedDecodeAttentionDescriptor()
-    d.struct_size = ctypes.sizeof(d)
-    d.version = 1
-    d.query, d.key, d.current_value = query.data_ptr(), key.data_ptr(), value.data_ptr()
-    d.key_cache_bf16, d.value_cache_bf16 = key_cache.data_ptr(), value_cache.data_ptr()
-    d.output = out.data_ptr()
-    if query_weight is not None:
-        d.query_norm_weight = query_weight.descriptor(stream)
-        d.has_query_norm_weight = 1
-    if key_weight is not None:
-        d.key_norm_weight = key_weight.descriptor(stream)
-        d.has_key_norm_weight = 1
-    d.query_heads, d.head_dim = query.shape
-    d.kv_heads = key.shape[0]
-    d.position, d.first_key_position = position, first_key_position
-    d.cache_capacity, d.cache_row_stride = key_cache.shape
-    d.norm_eps, d.query_scale, d.rope_theta = eps, query_scale, theta
-    d.attention_scale = attention_scale
-    d.rope_layout = layout
-    d.apply_rope = 1 if apply_rope else 0
-    d.cuda_stream = stream
-    if workspace is not None and device_position is not None:
-        check(load().nfn_mi355_fused_decode_attention_split_device_position_v1(
-            ctypes.byref(d), device_position.data_ptr(), sliding_window, workspace.data_ptr(),
-            workspace.numel()), "fused_decode_attention_split_device_position")
-    elif workspace is not None:
-        check(load().nfn_mi355_fused_decode_attention_split_v1(
-            ctypes.byref(d), workspace.data_ptr(), workspace.numel()), "fused_decode_attention_split")
-    elif device_position is not None:
-        check(load().nfn_native_tile_glimmer_fused_decode_attention_device_position_float32_v1(
-            ctypes.byref(d), device_position.data_ptr(), sliding_window),
-            "fused_decode_attention_device_position")
-    else:
-        check(load().nfn_native_tile_glimmer_fused_decode_attention_float32_v1(ctypes.byref(d)),
-              "fused_decode_attention")
-    return out
+    return tile_ops.native().fused_decode_attention(
+        query, key, value, key_cache, value_cache, position, first_key_position, attention_scale, query_weight,
+        key_weight, eps, query_scale, theta, layout, apply_rope, out, device_position, sliding_window, workspace)
 
 
 def lend_attention_workspace(workspace=None, stream=None) -> None:
@@ -167,28 +113,8 @@ def gqa_decode(query, current_key, current_value, key_cache, value_cache, positi
                first_key_position: int, scale: float, out=None, workspace=None):
     """query [query_heads, head_dim]; current_key/value [kv_heads, head_dim]; caches uint16
     (or bfloat16) [capacity, row_stride].  With `workspace` the split form runs."""
-    import torch
-    if out is None:
-        out = torch.empty_like(query)
-    d = GqaDecodeDescriptor()
-    d.struct_size = ctypes.sizeof(d)
-    d.version = 1
-    d.query, d.current_key, d.current_value = (query.data_ptr(), current_key.data_ptr(),
-                                               current_value.data_ptr())
-    d.key_cache_bf16, d.value_cache_bf16 = key_cache.data_ptr(), value_cache.data_ptr()
-    d.output = out.data_ptr()
-    d.query_heads, d.head_dim = query.shape
-    d.kv_heads = current_key.shape[0]
-    d.position, d.first_key_position = position, first_key_position
-    d.cache_capacity, d.cache_row_stride = key_cache.shape
-    d.scale = scale
-    d.cuda_stream = _stream()
-    if workspace is not None:
-        check(load().nfn_mi355_gqa_decode_split_v1(ctypes.byref(d), workspace.data_ptr(),
-                                                   workspace.numel()), "gqa_decode_split")
-    else:
-        check(load().nfn_native_tile_glimmer_gqa_decode_float32_v1(ctypes.byref(d)), "gqa_decode")
-    return out
+    return tile_ops.native().gqa_decode(query, current_key, current_value, key_cache, value_cache, position,
+                                        first_key_position, scale, out, workspace)
 
 
 def cache_commit(keys, values, key_cache, value_cache, position: int, rows: int = 0) -> None:
@@ -213,30 +139,8 @@ def block_attention(query, block_key, block_value, key_cache, value_cache, conte
                     sliding_window: int, scale: float, causal: bool, out=None, workspace=None):
     """query [query_rows, query_heads, head_dim]; block_key/value [block_rows, kv_heads, head_dim].
     With `workspace` (any 16-byte aligned uint8 tensor, e.g. gqa_decode_workspace) the split form."""
-    import torch
-    if out is None:
-        out = torch.empty_like(query)
-    d = BlockAttentionDescriptor()
-    d.struct_size = ctypes.sizeof(d)
-    d.version = 1
-    d.flags = BLOCK_ATTENTION_CAUSAL if causal else 0
-    d.query, d.block_key, d.block_value = (query.data_ptr(), block_key.data_ptr(),
-                                           block_value.data_ptr())
-    d.key_cache_bf16, d.value_cache_bf16 = key_cache.data_ptr(), value_cache.data_ptr()
-    d.output = out.data_ptr()
-    d.query_rows, d.query_heads, d.head_dim = query.shape
-    d.block_rows, d.kv_heads = block_key.shape[0], block_key.shape[1]
-    d.context_length, d.sliding_window = context_length, sliding_window
-    d.cache_capacity, d.cache_row_stride = key_cache.shape
-    d.scale = scale
-    d.cuda_stream = _stream()
-    if workspace is not None:
-        check(load().nfn_mi355_dflash_block_attention_split_v1(
-            ctypes.byref(d), workspace.data_ptr(), workspace.numel()), "block_attention_split")
-    else:
-        check(load().nfn_native_tile_dflash_block_attention_float32_v1(ctypes.byref(d)),
-              "block_attention")
-    return out
+    return tile_ops.native().block_attention(query, block_key, block_value, key_cache, value_cache, context_length,
+                                             sliding_window, scale, causal, out, workspace)
 
 
 def logit_transform(logits, multiplier: float, softcap: float) -> None:

@@ -5,6 +5,10 @@ harness for this ABI (tools/bench_muse_glimmer_packed_linear.py:28-43, 560-640):
 device pointers as integers, a 72-byte descriptor per packed matrix, an int
 status per call.  torch is used only to own device memory and streams.
 
+The calls of a decode step go through the extension module _front_end (csrc/python/front_end.cpp),
+which puts the same descriptors together natively: a launch costs the host 2.8 us here, the same
+call assembled with ctypes 7.5 to 13 us more.
+
 There is no CPU fallback: if the library is missing, loading raises.
 """
 from __future__ import annotations
@@ -273,6 +277,25 @@ def load(path: Optional[Path] = None) -> ctypes.CDLL:
     return lib
 
 
+_front = None
+
+
+def native():
+    """The extension module with the library's entry points bound; raises if either is not built."""
+    global _front
+    if _front is None:
+        import torch  # noqa: F401  (the module links against torch's libraries)
+        lib = load()
+        try:
+            from . import _front_end
+        except ImportError as error:
+            raise RuntimeError("neuralfn_amd._front_end is not built; run `python -m neuralfn_amd.build`") from error
+        _front_end.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+                         for name in _front_end.entry_points()}, check)
+        _front = _front_end
+    return _front
+
+
 class TileOpsError(RuntimeError):
     def __init__(self, operation: str, status: int):
         text = load().nfn_native_tile_ops_error_string(status)
@@ -296,8 +319,7 @@ def make_descriptor(encoding: int, data_ptr: int, output_dim: int, input_dim: in
 
 
 def _stream_handle() -> int:
-    import torch
-    return int(torch.cuda.current_stream().cuda_stream)
+    return native().stream_handle()
 
 
 @dataclass
@@ -353,14 +375,7 @@ def dequantize(weight: PackedWeight):
 
 def linear(weight: PackedWeight, x, bias=None):
     """nfn_native_tile_linear_packed_weight_float32_v1: any row count."""
-    import torch
-    rows = x.shape[0]
-    out = torch.empty((rows, weight.output_dim), dtype=torch.float32, device=x.device)
-    descriptor = weight.descriptor(_stream_handle())
-    check(load().nfn_native_tile_linear_packed_weight_float32_v1(
-        ctypes.byref(descriptor), x.data_ptr(), bias.data_ptr() if bias is not None else None,
-        out.data_ptr(), rows, bias is not None), "linear_packed_weight")
-    return out
+    return native().linear(weight, x, bias)
 
 
 def small_batch_workspace(rows: int, input_dim: int, device="cuda:0"):
@@ -371,37 +386,13 @@ def small_batch_workspace(rows: int, input_dim: int, device="cuda:0"):
     return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
 
-_MULTI = {
-    ("mmq", "plain"): "nfn_native_tile_k_quant_mmq_multi_linear_float32_v1",
-    ("mmq", "gated"): "nfn_native_tile_k_quant_mmq_multi_linear_gated_float32_v1",
-    ("mmq", "swiglu"): "nfn_native_tile_k_quant_mmq_multi_linear_swiglu_float32_v1",
-    ("mmvq", "plain"): "nfn_native_tile_k_quant_mmvq_multi_linear_float32_v1",
-    ("mmvq", "gated"): "nfn_native_tile_k_quant_mmvq_multi_linear_gated_float32_v1",
-    ("mmvq", "swiglu"): "nfn_native_tile_k_quant_mmvq_multi_linear_swiglu_float32_v1",
-}
-
-
 def multi_linear(weights: Sequence[PackedWeight], x, workspace, second=None, family: str = "mmq",
                  prologue: str = "plain", outputs=None):
     """1..4 projections of one shared input, rows 1..16.
 
     prologue "gated": x / (1 + exp(-second));  "swiglu": x is gate, second is up.
     """
-    import torch
-    rows = x.shape[0]
-    stream = _stream_handle()
-    if outputs is None:
-        outputs = [torch.empty((rows, w.output_dim), dtype=torch.float32, device=x.device)
-                   for w in weights]
-    descriptors = [w.descriptor(stream) for w in weights]
-    function = getattr(load(), _MULTI[(family, prologue)])
-    args = [_descriptor_array(descriptors), x.data_ptr()]
-    if prologue != "plain":
-        args.append(second.data_ptr() if second is not None else None)
-    args += [_pointer_array(outputs), len(weights), rows, workspace.data_ptr(),
-             workspace.numel(), stream]
-    check(function(*args), _MULTI[(family, prologue)])
-    return outputs
+    return native().multi_linear(weights, x, workspace, second, family, prologue, outputs)
 
 
 def multi_linear_prequantized(weights: Sequence[PackedWeight], rows: int, workspace, outputs=None,
@@ -409,18 +400,7 @@ def multi_linear_prequantized(weights: Sequence[PackedWeight], rows: int, worksp
     """Projections of the input whose quantized form an earlier call left in `workspace`:
     family "mmvq": the activation records of a verifier-family call or of the one-row dual-RMS
     handoff; family "mmq": the fp16 rows of the 5..16-row dual-RMS handoff."""
-    import torch
-    stream = _stream_handle()
-    if outputs is None:
-        outputs = [torch.empty((rows, w.output_dim), dtype=torch.float32, device=workspace.device)
-                   for w in weights]
-    descriptors = [w.descriptor(stream) for w in weights]
-    name = ("nfn_native_tile_k_quant_mmvq_multi_linear_prequantized_float32_v1" if family == "mmvq"
-            else "nfn_mi355_k_quant_mmq_multi_linear_prequantized_float32_v1")
-    check(getattr(load(), name)(
-        _descriptor_array(descriptors), _pointer_array(outputs), len(weights), rows,
-        workspace.data_ptr(), workspace.numel(), stream), f"{family}_multi_linear_prequantized")
-    return outputs
+    return native().multi_linear_prequantized(weights, rows, workspace, outputs, family == "mmvq")
 
 
 def rms_norm(x, weight: Optional[PackedWeight] = None, centered: bool = False, eps: float = 1e-6,
@@ -471,35 +451,9 @@ def dual_rms_add_capture(x, residual, first_weight: Optional[PackedWeight] = Non
     of `normalized` is left there for multi_linear_prequantized: one row, family "mmvq";
     5..16 rows, family "mmq" (`handoff_family`), or 4..16 rows, family "mmvq".
     """
-    import torch
-    rows, width = x.shape
-    stream = _stream_handle()
-    hidden = torch.empty_like(x)
-    normalized = torch.empty_like(x)
-    captured = torch.empty_like(x)
-    first = first_weight.descriptor(stream) if first_weight is not None else None
-    second = second_weight.descriptor(stream) if second_weight is not None else None
-    arguments = [x.data_ptr(), ctypes.byref(first) if first is not None else None,
-                 residual.data_ptr(), hidden.data_ptr(),
-                 ctypes.byref(second) if second is not None else None, normalized.data_ptr(),
-                 captured.data_ptr(), rows, width, first_eps, first_centered, second_eps,
-                 second_centered]
-    if handoff_workspace is None:
-        check(load().nfn_native_tile_glimmer_dual_rms_add_capture_float32_v1(*arguments, stream),
-              "dual_rms_add_capture")
-    elif rows == 1:
-        check(load().nfn_native_tile_glimmer_dual_rms_add_capture_mmvq_q8_float32_v1(
-            *arguments, handoff_workspace.data_ptr(), handoff_workspace.numel(), stream),
-            "dual_rms_add_capture_mmvq_q8")
-    elif handoff_family == "mmvq":
-        check(load().nfn_mi355_dual_rms_add_capture_mmvq_rows_float32_v1(
-            *arguments, handoff_workspace.data_ptr(), handoff_workspace.numel(), stream),
-            "dual_rms_add_capture_mmvq_rows")
-    else:
-        check(load().nfn_mi355_dual_rms_add_capture_mmq_f16_float32_v1(
-            *arguments, handoff_workspace.data_ptr(), handoff_workspace.numel(), stream),
-            "dual_rms_add_capture_mmq_f16")
-    return hidden, normalized, captured
+    return native().dual_rms_add_capture(x, residual, first_weight, first_centered, second_weight,
+                                         second_centered, first_eps, second_eps, handoff_workspace,
+                                         handoff_family == "mmvq")
 
 
 def dual_rms_multi_linear(x, residual, weights: Sequence[PackedWeight],
@@ -510,23 +464,8 @@ def dual_rms_multi_linear(x, residual, weights: Sequence[PackedWeight],
     """nfn_mi355_dual_rms_mmvq_multi_linear_float32_v1: one row through the two normalisations
     and the projections of their result in one launch.
     Returns (hidden, normalized, residual_output, outputs)."""
-    import torch
-    stream = _stream_handle()
-    width = x.shape[1]
-    hidden, normalized, captured = torch.empty_like(x), torch.empty_like(x), torch.empty_like(x)
-    if outputs is None:
-        outputs = [torch.empty((1, w.output_dim), dtype=torch.float32, device=x.device)
-                   for w in weights]
-    first = first_weight.descriptor(stream) if first_weight is not None else None
-    second = second_weight.descriptor(stream) if second_weight is not None else None
-    descriptors = [w.descriptor(stream) for w in weights]
-    check(load().nfn_mi355_dual_rms_mmvq_multi_linear_float32_v1(
-        x.data_ptr(), ctypes.byref(first) if first is not None else None, residual.data_ptr(),
-        hidden.data_ptr(), ctypes.byref(second) if second is not None else None,
-        normalized.data_ptr(), captured.data_ptr(), width, first_eps, first_centered, second_eps,
-        second_centered, _descriptor_array(descriptors), _pointer_array(outputs), len(weights),
-        stream), "dual_rms_mmvq_multi_linear")
-    return hidden, normalized, captured, outputs
+    return native().dual_rms_multi_linear(x, residual, weights, first_weight, first_centered, second_weight,
+                                          second_centered, first_eps, second_eps, outputs)
 
 
 def dual_rms_multi_linear_supported(weights: Sequence[PackedWeight], width: int) -> bool:
@@ -538,29 +477,13 @@ def dual_rms_multi_linear_supported(weights: Sequence[PackedWeight], width: int)
 
 def mmvq_linear(weight: PackedWeight, x, workspace, out=None):
     """nfn_native_tile_k_quant_mmvq_linear_float32_v1: the one-row decode GEMV."""
-    import torch
-    stream = _stream_handle()
-    if out is None:
-        out = torch.empty((1, weight.output_dim), dtype=torch.float32, device=x.device)
-    descriptor = weight.descriptor(stream)
-    check(load().nfn_native_tile_k_quant_mmvq_linear_float32_v1(
-        ctypes.byref(descriptor), x.data_ptr(), out.data_ptr(), workspace.data_ptr(),
-        workspace.numel(), stream), "mmvq_linear")
-    return out
+    return native().mmvq_linear(weight, x, workspace, out)
 
 
 def gate_up_swiglu(gate: PackedWeight, up: PackedWeight, x, out=None):
     """nfn_mi355_k_quant_mmvq_gate_up_swiglu_float32_v1: one token through the gate and up
     projections with the SwiGLU activation at the row ends."""
-    import torch
-    stream = _stream_handle()
-    if out is None:
-        out = torch.empty((1, gate.output_dim), dtype=torch.float32, device=x.device)
-    gate_descriptor, up_descriptor = gate.descriptor(stream), up.descriptor(stream)
-    check(load().nfn_mi355_k_quant_mmvq_gate_up_swiglu_float32_v1(
-        ctypes.byref(gate_descriptor), ctypes.byref(up_descriptor), x.data_ptr(), out.data_ptr(),
-        stream), "gate_up_swiglu")
-    return out
+    return native().gate_up_swiglu(gate, up, x, out)
 
 
 def gate_up_swiglu_supported(gate: PackedWeight, up: PackedWeight) -> bool:
@@ -574,16 +497,7 @@ def gate_up_swiglu_rows(gate: PackedWeight, up: PackedWeight, x, rows: int, work
     """nfn_mi355_k_quant_mmq_gate_up_swiglu_float32_v1: a block of 5..16 rows through the gate and
     up projections with the SwiGLU activation applied to the pair of results.  x None: the
     workspace holds the rows as dual_rms_add_capture(handoff_workspace=...) left them."""
-    import torch
-    stream = _stream_handle()
-    if out is None:
-        out = torch.empty((rows, gate.output_dim), dtype=torch.float32, device=workspace.device)
-    gate_descriptor, up_descriptor = gate.descriptor(stream), up.descriptor(stream)
-    check(load().nfn_mi355_k_quant_mmq_gate_up_swiglu_float32_v1(
-        ctypes.byref(gate_descriptor), ctypes.byref(up_descriptor),
-        None if x is None else x.data_ptr(), out.data_ptr(), rows, workspace.data_ptr(),
-        workspace.numel(), stream), "gate_up_swiglu_rows")
-    return out
+    return native().gate_up_swiglu_rows(gate, up, x, rows, workspace, out)
 
 
 def gate_up_swiglu_rows_supported(gate: PackedWeight, up: PackedWeight, rows: int) -> bool:
@@ -664,23 +578,7 @@ def swiglu(gate, up):
 
 def lm_head_argmax(weight: PackedWeight, x, workspace=None, indices=None, maxima=None):
     """nfn_mi355_lm_head_argmax_v1: GEMV + argmax, logits never stored."""
-    import torch
-    rows = x.shape[0]
-    stream = _stream_handle()
-    if workspace is None:
-        nbytes = load().nfn_mi355_lm_head_argmax_workspace_bytes_v1(rows, weight.output_dim)
-        if nbytes <= 0:
-            raise ValueError("lm_head_argmax supports 1..16 rows")
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    if indices is None:
-        indices = torch.empty(rows, dtype=torch.int64, device=x.device)
-    if maxima is None:
-        maxima = torch.empty(rows, dtype=torch.float32, device=x.device)
-    descriptor = weight.descriptor(stream)
-    check(load().nfn_mi355_lm_head_argmax_v1(
-        ctypes.byref(descriptor), x.data_ptr(), indices.data_ptr(), maxima.data_ptr(), rows,
-        workspace.data_ptr(), workspace.numel(), stream), "lm_head_argmax")
-    return indices, maxima
+    return native().lm_head_argmax(weight, x, workspace, indices, maxima)
 
 
 STATIC_SCRATCH_EXCEEDED = 0x4e46  # NFN_MI355_STATUS_STATIC_SCRATCH_EXCEEDED
@@ -700,22 +598,7 @@ def lm_head_argmax_no_alloc(weight: PackedWeight, x, indices, maxima):
 
 def gemm(weight: PackedWeight, x, mode: int = GEMM_F16, workspace=None, out=None):
     """nfn_mi355_k_quant_gemm_float32_v1: prefill dequant-GEMM, any row count."""
-    import torch
-    rows = x.shape[0]
-    stream = _stream_handle()
-    if workspace is None:
-        nbytes = load().nfn_mi355_k_quant_gemm_workspace_bytes_v1(
-            rows, weight.input_dim, weight.output_dim, mode)
-        if nbytes <= 0:
-            raise ValueError("unsupported GEMM geometry or mode")
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    if out is None:
-        out = torch.empty((rows, weight.output_dim), dtype=torch.float32, device=x.device)
-    descriptor = weight.descriptor(stream)
-    check(load().nfn_mi355_k_quant_gemm_float32_v1(
-        ctypes.byref(descriptor), x.data_ptr(), out.data_ptr(), rows, workspace.data_ptr(),
-        workspace.numel(), mode, stream), "k_quant_gemm")
-    return out
+    return native().gemm(weight, x, mode, workspace, out)
 
 
 def gemm_plan(encoding: int, rows: int, input_dim: int, output_dim: int, mode: int = GEMM_F16):
@@ -730,20 +613,4 @@ def gemm_plan(encoding: int, rows: int, input_dim: int, output_dim: int, mode: i
 def gemm_multi(weights: Sequence[PackedWeight], x, mode: int = GEMM_F16, workspace=None,
                outputs=None):
     """nfn_mi355_k_quant_gemm_multi_float32_v1: 1..4 projections of one input, converted once."""
-    import torch
-    rows = x.shape[0]
-    stream = _stream_handle()
-    if workspace is None:
-        nbytes = max(load().nfn_mi355_k_quant_gemm_workspace_bytes_v1(
-            rows, w.input_dim, w.output_dim, mode) for w in weights)
-        if nbytes <= 0:
-            raise ValueError("unsupported GEMM geometry or mode")
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    if outputs is None:
-        outputs = [torch.empty((rows, w.output_dim), dtype=torch.float32, device=x.device)
-                   for w in weights]
-    descriptors = [w.descriptor(stream) for w in weights]
-    check(load().nfn_mi355_k_quant_gemm_multi_float32_v1(
-        _descriptor_array(descriptors), x.data_ptr(), _pointer_array(outputs), len(weights), rows,
-        workspace.data_ptr(), workspace.numel(), mode, stream), "k_quant_gemm_multi")
-    return outputs
+    return native().gemm_multi(weights, x, mode, workspace, outputs)

@@ -245,3 +245,17 @@ def test_the_reference_engines_own_loader_opens_the_library():
     status = harness.nfn_ref_loader_probe(b"libnfn_mi355_tile_ops.so", str(runtime).encode(),
                                           report, len(report))
     assert status == 1 and "absolute" in report.value.decode()
+
+
+def test_front_end_binds_declared_entry_points_and_checks_its_arguments():
+    """The extension module in front of the C ABI: it binds names of the header only, and what the
+    ctypes form refused with an exception before the call it refuses with one of the same kind."""
+    torch = pytest.importorskip("torch")
+    front = tile_ops.native()
+    assert set(front.entry_points()) <= set(tile_ops.SIGNATURES)
+    x, scratch = torch.zeros((1, 256)), torch.zeros(4096, dtype=torch.uint8)
+    weight = tile_ops.PackedWeight(tile_ops.kquant.Q4_K, 2, 256, torch.zeros(288, dtype=torch.uint8))
+    with pytest.raises(TypeError):
+        tile_ops.multi_linear([weight], None, scratch)
+    with pytest.raises(KeyError):
+        tile_ops.multi_linear([weight], x, scratch, family="mmx")
