@@ -90,7 +90,7 @@ int nfn_native_tile_packed_weight_dequantize_float32_v1(
 /* ---- generic float-activation linear, any row count (tile_ops.h:614-620):
  *      float weights times float activations, no quantization of the input.
  *      It has no workspace argument, so every row count keeps that float
- *      arithmetic (17 rows and more on the float matrix instruction);
+ *      arithmetic (four rows and more on the bf16 matrix instruction, the floats cut into exact terms);
  *      nfn_mi355_k_quant_gemm_float32_v1 is the fp16 matrix-core route. -- */
 int nfn_native_tile_linear_packed_weight_float32_v1(
     const NfnNativeTilePackedWeightDescriptorV1* descriptor,

@@ -231,34 +231,6 @@ const char* nfn_native_tile_ops_error_string(int code) {
 
 }  // extern "C"
 
-namespace {
-
-// The generic linear has two exact kernels: the vector one decodes every weight once per 8
-// input rows, the matrix-core one once per 128.  Rates measured on MI355X at 6,656 columns:
-// the vector kernel decodes 4.6e11 (Q4_K, Q5_K), 3.0e11 (Q6_K) or 2.4e11 (others) weights a
-// second and a launch of it takes at least 6 us; a 128 x 64 tile of the matrix-core kernel
-// takes 300 us alone on its compute unit (3.6e11 flop/s) and 229 us when the unit works
-// through several (4.8e11 flop/s).
-bool float_matrix_cores_pay(const Descriptor& weight, std::int64_t rows) {
-    if (rows <= 16 || !gemm_f32_supports(weight, rows)) return false;
-    const double weights =
-        static_cast<double>(weight.output_dim) * static_cast<double>(weight.input_dim);
-    const double decoded_per_us = weight.encoding == kEncQ4K || weight.encoding == kEncQ5K ? 4.6e5
-                                  : weight.encoding == kEncQ6K                             ? 3.0e5
-                                                                                           : 2.4e5;
-    // the vector kernel's passes of eight rows are workgroups of one launch, not launches one
-    // after another: the launch floor counts once
-    const double vector_work_us = static_cast<double>((rows + 7) / 8) * weights / decoded_per_us;
-    const double vector_us = vector_work_us < 6.0 ? 6.0 : vector_work_us;
-    const double tile_flop = 128.0 * 64.0 * 2.0 * static_cast<double>(weight.input_dim);
-    const double passes = gemm_f32_tile_passes(weight, rows);
-    const double alone_us = tile_flop / 3.6e5;
-    const double matrix_us = passes * tile_flop / 4.8e5 < alone_us ? alone_us : passes * tile_flop / 4.8e5;
-    return matrix_us + 4.0 < vector_us;
-}
-
-}  // namespace
-
 extern "C" {
 
 int nfn_native_tile_packed_weight_validate_v1(const Descriptor* descriptor) {
@@ -284,10 +256,15 @@ int nfn_native_tile_linear_packed_weight_float32_v1(const Descriptor* descriptor
         return kInvalid;
     }
     const hipStream_t stream = as_stream(normalized.cuda_stream);
-    if (float_matrix_cores_pay(normalized, rows)) {
-        launch_gemm_f32(normalized, input, has_bias ? bias : nullptr, output, rows, stream);
+    if (linear_rows_supports(normalized, rows)) {
+        launch_linear_rows(normalized, input, has_bias ? bias : nullptr, output, rows, stream);
         return launch_status();
     }
+    if (linear_exact_supports(normalized, rows)) {
+        launch_linear_exact(normalized, input, has_bias ? bias : nullptr, output, rows, stream);
+        return launch_status();
+    }
+    // odd widths: the kernel that takes any
     ProjectionSet set{};
     set.count = 1;
     set.input_dim = normalized.input_dim;

@@ -1,0 +1,253 @@
+// Exact float dot products of packed weight rows with one to three input rows: device code shared
+// by the generic linear (linear_rows.hip) and the one-row lm_head of the formats without a
+// streaming kernel of their own (lm_head.hip).
+//
+// The decoded weight d * sc * q - d_min * m is one fused multiply-add: d * sc and d_min * m are
+// exact in float (at most 19 bits), and so is d * sc * q (at most 24), so that the fused form
+// rounds where the CPU engine's two products and a subtraction round
+// (neuralfn/csrc/native_gpt2/resident_glimmer.cpp:542-616).  A code byte becomes a float in one
+// instruction: 2.25 vector instructions a weight before the products with the input rows.
+//
+// The input rows lie in LDS, 64 columns (a unit) at a pitch of 68 floats: a lane owns whole units,
+// and neighbouring lanes' 16-byte reads then fall into distinct banks.  A wave takes two weight
+// rows at a time, so that an input value read from LDS serves both, and requests a pair's packed
+// bytes one turn ahead.
+#pragma once
+
+#include <type_traits>
+#include <utility>
+
+#include "common.hpp"
+
+namespace nfn {
+
+typedef float exact_f32x4 __attribute__((ext_vector_type(4)));
+typedef std::uint32_t exact_u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef std::uint32_t exact_u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+
+constexpr int kExactPitch = 68;  // floats from one unit to the next in LDS
+constexpr int kExactWaves = 8;
+constexpr int kExactPair = 2;    // weight rows a wave takes at a time
+
+// LDS bytes of `rows` input rows
+constexpr std::int64_t exact_rows_lds(std::int64_t rows, std::int64_t input_dim) {
+    return rows * ((input_dim + 63) / 64) * kExactPitch * 4;
+}
+
+// What a lane holds of one unit of a weight row.  values<I>(): columns 4 I .. 4 I + 3 of it.
+template <std::uint32_t ENC>
+struct ExactUnit;
+
+__device__ __forceinline__ float code_byte(std::uint32_t word, int index) {
+    return static_cast<float>((word >> (8 * index)) & 255u);
+}
+
+template <std::uint32_t ENC>
+struct ExactUnitOfQ4KOrQ5K {
+    exact_u32x4_a4 header, codes[2], fifth[2];
+    __device__ __forceinline__ void load(const std::uint8_t* row, int unit) {
+        const std::uint8_t* block = row + (unit >> 2) * static_cast<int>(block_bytes(ENC));
+        const std::uint8_t* source = block + (ENC == kEncQ5K ? 48 : 16) + (unit & 3) * 32;
+        header = *reinterpret_cast<const exact_u32x4_a4*>(block);
+        codes[0] = *reinterpret_cast<const exact_u32x4_a4*>(source);
+        codes[1] = *reinterpret_cast<const exact_u32x4_a4*>(source + 16);
+        if constexpr (ENC == kEncQ5K) {
+            fifth[0] = *reinterpret_cast<const exact_u32x4_a4*>(block + 16);
+            fifth[1] = *reinterpret_cast<const exact_u32x4_a4*>(block + 32);
+        }
+    }
+    // scales and minimums of the unit's two sub-blocks (k_scale_min's indexing, without a branch)
+    float scale[2], offset[2];
+    int group;
+    __device__ __forceinline__ void prepare(int unit) {
+        group = unit & 3;
+        const float d = half_bits_to_float(header[0] & 0xffffu), dmin = half_bits_to_float(header[0] >> 16);
+#pragma unroll
+        for (int step = 0; step < 2; ++step) {
+            const int sub = 2 * group + step, shift = 8 * (sub & 3), upper = -(sub >> 2);
+            const int y = static_cast<int>(header[1] >> shift), z = static_cast<int>(header[2] >> shift);
+            const int w = static_cast<int>(header[3] >> shift);
+            const int sc = ((y & 63) & ~upper) | (((w & 15) | (((y >> 6) & 3) << 4)) & upper);
+            const int m = ((z & 63) & ~upper) | ((((w >> 4) & 15) | (((z >> 6) & 3) << 4)) & upper);
+            scale[step] = d * static_cast<float>(sc);
+            offset[step] = -(dmin * static_cast<float>(m));
+        }
+    }
+    template <int I>
+    __device__ __forceinline__ exact_f32x4 values() const {
+        constexpr int kStep = I / 8, kWord = I % 8;
+        std::uint32_t q = (codes[kWord / 4][kWord % 4] >> (4 * kStep)) & 0x0f0f0f0fu;
+        if constexpr (ENC == kEncQ5K) {
+            q |= ((fifth[kWord / 4][kWord % 4] >> (2 * group + kStep)) & 0x01010101u) << 4;
+        }
+        exact_f32x4 w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = fmaf(scale[kStep], code_byte(q, j), offset[kStep]);
+        return w;
+    }
+};
+template <>
+struct ExactUnit<kEncQ4K> : ExactUnitOfQ4KOrQ5K<kEncQ4K> {};
+template <>
+struct ExactUnit<kEncQ5K> : ExactUnitOfQ4KOrQ5K<kEncQ5K> {};
+
+template <>
+struct ExactUnit<kEncQ6K> {
+    exact_u32x4_a2 low[4], high[2];
+    std::uint32_t codes_of_scale, d;
+    float scale[4];
+    int upper;
+    __device__ __forceinline__ void load(const std::uint8_t* row, int unit) {
+        const std::uint8_t* block = row + (unit >> 2) * 210;
+        const std::uint8_t* lower = block + ((unit >> 1) & 1) * 64;
+        const std::uint8_t* top = block + 128 + ((unit >> 1) & 1) * 32;
+#pragma unroll
+        for (int piece = 0; piece < 4; ++piece) {
+            low[piece] = *reinterpret_cast<const exact_u32x4_a2*>(lower + 16 * piece);
+        }
+        high[0] = *reinterpret_cast<const exact_u32x4_a2*>(top);
+        high[1] = *reinterpret_cast<const exact_u32x4_a2*>(top + 16);
+        const auto* pairs = reinterpret_cast<const std::uint16_t*>(block + 192 + 4 * (unit & 3));
+        codes_of_scale = pairs[0] | (static_cast<std::uint32_t>(pairs[1]) << 16);
+        d = *reinterpret_cast<const std::uint16_t*>(block + 208);
+    }
+    __device__ __forceinline__ void prepare(int unit) {
+        upper = (unit & 1) * 4;  // quarters 2 and 3 of the half block: high nibbles, high-bit pairs 2 and 3
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            scale[k] = half_bits_to_float(d) * static_cast<float>(static_cast<std::int8_t>(codes_of_scale >> (8 * k)));
+        }
+    }
+    template <int I>
+    __device__ __forceinline__ exact_f32x4 values() const {
+        constexpr int kStep = I / 8, kWord = I % 8;
+        const std::uint32_t q = ((low[2 * kStep + kWord / 4][kWord % 4] >> upper) & 0x0f0f0f0fu) |
+            (((high[kWord / 4][kWord % 4] >> (upper + 2 * kStep)) & 0x03030303u) << 4);
+        const float factor = scale[2 * kStep + kWord / 4];
+        exact_f32x4 w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = fmaf(factor, code_byte(q, j), -32.0f * factor);
+        return w;
+    }
+};
+
+template <>
+struct ExactUnit<kEncQ8_0> {
+    // two 34-byte blocks: 17 words, the codes of the first block half a word off
+    std::uint32_t words[17];
+    float scale[2];
+    __device__ __forceinline__ void load(const std::uint8_t* row, int unit) {
+        const std::uint8_t* source = row + unit * 68;
+#pragma unroll
+        for (int piece = 0; piece < 4; ++piece) {
+            const exact_u32x4_a2 four = *reinterpret_cast<const exact_u32x4_a2*>(source + 16 * piece);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) words[4 * piece + j] = four[j];
+        }
+        typedef std::uint32_t u32_a2 __attribute__((aligned(2)));
+        words[16] = *reinterpret_cast<const u32_a2*>(source + 64);
+    }
+    __device__ __forceinline__ void prepare(int) {
+        scale[0] = half_bits_to_float(words[0] & 0xffffu);
+        scale[1] = half_bits_to_float(words[8] >> 16);
+    }
+    template <int I>
+    __device__ __forceinline__ exact_f32x4 values() const {
+        constexpr int kStep = I / 8, kWord = I % 8;
+        const std::uint32_t q = (kStep == 0 ? __builtin_amdgcn_alignbyte(words[kWord + 1], words[kWord], 2)
+                                            : words[9 + kWord]) ^ 0x80808080u;  // the byte q + 128
+        exact_f32x4 w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = fmaf(scale[kStep], code_byte(q, j), -128.0f * scale[kStep]);
+        return w;
+    }
+};
+
+template <std::uint32_t ENC>
+constexpr bool kExactRowsFormat = ENC == kEncQ4K || ENC == kEncQ5K || ENC == kEncQ6K || ENC == kEncQ8_0;
+
+// The workgroup's copy of the input rows: [row][unit][kExactPitch].
+template <int R>
+__device__ __forceinline__ void exact_rows_stage(const float* __restrict__ input, std::int64_t input_dim,
+                                                 float* staged) {
+    const int units = static_cast<int>(input_dim >> 6);
+    for (int index = threadIdx.x; index < R * units * 16; index += kExactWaves * kWave) {
+        const int row = index / (units * 16), piece = index % (units * 16);
+        typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+        const exact_f32x4 x = *reinterpret_cast<const f32x4_a4*>(input + row * input_dim + 4 * piece);
+        *reinterpret_cast<exact_f32x4*>(staged + (row * units + (piece >> 4)) * kExactPitch + 4 * (piece & 15)) = x;
+    }
+    __syncthreads();
+}
+
+template <typename F, int... I>
+__device__ __forceinline__ void for_each_piece(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+// Calls take(row, sums) for the weight rows `first`, `first + step`, ... below `output_dim`, two at a
+// time (rows 2 p and 2 p + 1); sums[r]: this wave's total for input row r, in every lane.  A row's
+// sum does not depend on the launch: lane l adds the units l, l + 64, ... in rising order, four
+// columns at a time, and the lanes meet in a butterfly.
+template <std::uint32_t ENC, int R, typename Take>
+__device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__ data, std::int64_t row_stride,
+                                                std::int64_t output_dim, std::int64_t input_dim,
+                                                const float* staged, std::int64_t first_pair, std::int64_t pair_step,
+                                                std::int64_t end_pair, Take&& take) {
+    const int lane = threadIdx.x & 63;
+    const int units = static_cast<int>(input_dim >> 6);
+    const int turns = (units + 63) / 64;
+    if (first_pair >= end_pair) return;
+    ExactUnit<ENC> now[kExactPair], next[kExactPair];
+    auto load = [&](ExactUnit<ENC> (&into)[kExactPair], std::int64_t pair, int turn) {
+        const int unit = min(lane + 64 * turn, units - 1);
+#pragma unroll
+        for (int k = 0; k < kExactPair; ++k) {
+            into[k].load(data + min(pair * kExactPair + k, output_dim - 1) * row_stride, unit);
+        }
+    };
+    load(now, first_pair, 0);
+    for (std::int64_t pair = first_pair; pair < end_pair; pair += pair_step) {
+        float sums[kExactPair][R] = {};
+        for (int turn = 0; turn < turns; ++turn) {
+            const bool more = turn + 1 < turns;
+            // (unconditional: behind the last pair its own bytes are read again)
+            load(next, more ? pair : pair + pair_step < end_pair ? pair + pair_step : pair, more ? turn + 1 : 0);
+            const int unit = lane + 64 * turn;
+            if (unit < units) {
+#pragma unroll
+                for (int k = 0; k < kExactPair; ++k) now[k].prepare(unit);
+                const float* x = staged + unit * kExactPitch;
+                const auto four = [&](auto index) {
+                    constexpr int kI = decltype(index)::value;
+                    exact_f32x4 w[kExactPair];
+#pragma unroll
+                    for (int k = 0; k < kExactPair; ++k) w[k] = now[k].template values<kI>();
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const exact_f32x4 v =
+                            *reinterpret_cast<const exact_f32x4*>(x + r * units * kExactPitch + 4 * kI);
+#pragma unroll
+                        for (int k = 0; k < kExactPair; ++k) {
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) sums[k][r] = fmaf(v[j], w[k][j], sums[k][r]);
+                        }
+                    }
+                };
+                for_each_piece(four, std::make_integer_sequence<int, 16>{});
+            }
+#pragma unroll
+            for (int k = 0; k < kExactPair; ++k) now[k] = next[k];
+        }
+#pragma unroll
+        for (int k = 0; k < kExactPair; ++k) {
+            const std::int64_t row = pair * kExactPair + k;
+            float totals[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) totals[r] = wave_sum(sums[k][r]);
+            if (row < output_dim) take(row, totals);
+        }
+    }
+}
+
+}  // namespace nfn

@@ -6,11 +6,12 @@
 // and multiplied with the float activations as they are; only the order of the
 // float additions differs from the engine's double accumulation
 // (resident_glimmer.cpp:655-679).  It serves
-//   nfn_native_tile_linear_packed_weight_float32_v1 for rows <= 16 and for the
-//   encodings without a matrix-core kernel (reference kernel:
+//   nfn_native_tile_linear_packed_weight_float32_v1 for widths that the tuned
+//   exact kernels (linear_rows.hip, linear_exact.hip) do not take (reference kernel:
 //   neuralfn/csrc/tile_cuda/kernels.cu:1398-1525),
-//   and the verifier entry points, whose contract is that every row gets the
-//   one-row arithmetic (neuralfn/csrc/native_train/tile_ops.h:685-688): the
+//   and the small-batch entry points for float and bf16 weights and odd widths; in the
+//   verifier's, whose contract is that every row gets the one-row arithmetic
+//   (neuralfn/csrc/native_train/tile_ops.h:685-688), it matters that the
 //   per-row order of operations here does not depend on R.
 #include "common.hpp"
 #include "gemv_f32_device.hpp"

@@ -1,0 +1,783 @@
+// The exact tier on the bf16 matrix cores: many input rows of one projection, float in, float
+// out, every weight at its decoded value.
+//
+// A float is the sum of three bf16 numbers (24 significant bits cut into 8 + 8 + 8 by
+// truncation, nothing left over), and the integer code of a packed weight is one bf16 number
+// (at most eight significant bits).  v_mfma_f32_32x32x16_bf16 multiplies bf16 exactly and adds
+// in float, so three of them per code give the product of the float activations with the codes,
+// at a sixteenth of the cycles of the float instruction each: 3/16 of v_mfma_f32_32x32x2_f32's
+// time.  A sub-block's scale d * sc is exact in float (11 + 6 or 7 bits) and multiplies the
+// sub-block's sums on their way into the accumulators; the minimum's part d_min * m times the
+// sub-block's sum of activations goes in by one float matrix instruction per 64 columns.  A
+// one-hot input row returns the dequantized weight bit for bit: d * sc * q is exact, the
+// subtraction of d_min * m is the one rounding that the decode has.  Float weights are cut into
+// three terms as well (eight products of the nine: the one left out is below 2^-32 of the
+// product), bf16 weights are one term.
+//
+// A workgroup's waves share one tile and cut K between them; their sums meet in LDS at the end, in
+// a fixed order.  Two forms:
+//   linear_exact_small_kernel, a tile of 32 MT x 32 NT, each wave streaming its own operands straight
+//   into registers (no LDS, no barrier in the loop): what a problem of a few tiles needs (38 rows x
+//   332 outputs are 22 of 32 x 32 for 256 compute units), there is no long walk over K;
+//   linear_exact_kernel, a tile of 32 MT input rows x 128 weight rows for two waves (64 weight rows
+//   each) in each of four K groups.  The two cut the activations of a step of 32 columns between
+//   them and hand the terms over in LDS.
+// What bounds both is the vector cache: a load instruction that reads 16 bytes from each of 32 rows
+// looks up 32 lines for 1 KB, and a unit pulls some 20 GB/s that way.  (Requests two steps ahead
+// instead of one, and the matrix instructions of a step before its other work instead of between it,
+// made no difference.)  Measured at 4,096 -> 6,656, against the vector kernel (16 rows) and the
+// float matrix instruction (200, 512 rows) before: Q4_K 134 -> 16 us at 16 rows, 203 -> 69 at 200,
+// 311 -> 135 at 512; Q8_0 368 -> 29, 180 -> 90, 279 -> 178; F32 406 -> 30, 172 -> 131, 271 -> 254.
+//
+// The entry point, nfn_native_tile_linear_packed_weight_float32_v1, has no workspace argument
+// (neuralfn/csrc/native_train/tile_ops.h:614-620; reference kernel
+// neuralfn/csrc/tile_cuda/kernels.cu:26943-26983), so nothing is converted ahead of the launch.
+// Weight layouts and decode: neuralfn/csrc/native_gpt2/resident_glimmer.cpp:542-616.
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace nfn {
+
+namespace {
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef std::uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef std::uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef std::uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef std::uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+
+__device__ __forceinline__ bf16x8 as_bf16(u32x4 words) { return __builtin_bit_cast(bf16x8, words); }
+
+// the upper halves of two floats, `low` in the lower half: two bf16 numbers by truncation
+__device__ __forceinline__ std::uint32_t upper_halves(float low, float high) {
+    return __builtin_amdgcn_perm(__float_as_uint(high), __float_as_uint(low), 0x07060302u);
+}
+
+// Two of the eight values of a fragment: word `pair` of its three terms.
+__device__ __forceinline__ void cut_pair(float x0, float x1, std::uint32_t& a, std::uint32_t& b, std::uint32_t& c) {
+    a = upper_halves(x0, x1);
+    const float y0 = x0 - __uint_as_float(__float_as_uint(x0) & 0xffff0000u);
+    const float y1 = x1 - __uint_as_float(__float_as_uint(x1) & 0xffff0000u);
+    b = upper_halves(y0, y1);
+    const float z0 = y0 - __uint_as_float(__float_as_uint(y0) & 0xffff0000u);
+    const float z1 = y1 - __uint_as_float(__float_as_uint(y1) & 0xffff0000u);
+    c = upper_halves(z0, z1);
+}
+
+// Eight floats as three bf16 fragments whose sum they are.
+struct Terms {
+    bf16x8 first, second, third;
+};
+__device__ __forceinline__ Terms cut(const float (&x)[8]) {
+    u32x4 a, b, c;
+#pragma unroll
+    for (int pair = 0; pair < 4; ++pair) {
+        std::uint32_t wa, wb, wc;
+        cut_pair(x[2 * pair], x[2 * pair + 1], wa, wb, wc);
+        a[pair] = wa;
+        b[pair] = wb;
+        c[pair] = wc;
+    }
+    return Terms{as_bf16(a), as_bf16(b), as_bf16(c)};
+}
+
+__device__ __forceinline__ float sum_of(const float (&x)[8]) {
+    return ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+}
+
+// four code bytes (0..255) less `offset` as four bf16 numbers
+__device__ __forceinline__ void codes_to_bf16(std::uint32_t bytes, float offset, std::uint32_t& low,
+                                              std::uint32_t& high) {
+    const float q0 = static_cast<float>(bytes & 255u) - offset;
+    const float q1 = static_cast<float>((bytes >> 8) & 255u) - offset;
+    const float q2 = static_cast<float>((bytes >> 16) & 255u) - offset;
+    const float q3 = static_cast<float>(bytes >> 24) - offset;
+    low = upper_halves(q0, q1);
+    high = upper_halves(q2, q3);
+}
+
+// -----------------------------------------------------------------------------------------------
+// What a lane holds of one weight row for 64 columns (a unit: two steps of 32).  The lane's
+// columns of a step: kWide formats 16 half + 8 chunk + j, the others 16 chunk + 8 half + j
+// (half = lane / 32, chunk = 0 or 1, j = 0..7); the matrix instruction does not care which
+// column carries which k index as long as both operands agree, and 16 neighbouring code bytes
+// are one load.  Q6_K has a scale per 16 columns, which a chunk's instructions must not mix.
+//   load(row, unit, half); words(step, chunk, word, ..): four codes as bf16; scale(step, chunk);
+//   minimum(step): d_min * m
+// -----------------------------------------------------------------------------------------------
+template <std::uint32_t ENC>
+struct Unit;
+
+template <std::uint32_t ENC>
+struct UnitOfQ4KOrQ5K {
+    static constexpr bool kWide = true, kScaled = true, kMinimum = true, kScalePerChunk = false;
+    u32x4_a4 header, codes, fifth;
+    int group;
+    __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half) {
+        const std::uint8_t* block = row + (unit >> 2) * static_cast<int>(block_bytes(ENC));
+        group = unit & 3;
+        header = *reinterpret_cast<const u32x4_a4*>(block);
+        codes = *reinterpret_cast<const u32x4_a4*>(block + (ENC == kEncQ5K ? 48 : 16) + group * 32 + half * 16);
+        if constexpr (ENC == kEncQ5K) fifth = *reinterpret_cast<const u32x4_a4*>(block + 16 + half * 16);
+    }
+    __device__ __forceinline__ void words(int step, int chunk, int word, std::uint32_t& low, std::uint32_t& high) const {
+        std::uint32_t q = (codes[2 * chunk + word] >> (4 * step)) & 0x0f0f0f0fu;
+        if constexpr (ENC == kEncQ5K) {
+            q |= ((fifth[2 * chunk + word] >> (2 * group + step)) & 0x01010101u) << 4;
+        }
+        codes_to_bf16(q, 0.0f, low, high);
+    }
+    // scale and minimum bytes of sub-block 2 group + step (k_scale_min's indexing, without a branch)
+    __device__ __forceinline__ float scale(int step, int) const {
+        const int sub = 2 * group + step, shift = 8 * (sub & 3), upper = -(sub >> 2);
+        const int y = static_cast<int>(header[1] >> shift), w = static_cast<int>(header[3] >> shift);
+        const int code = ((y & 63) & ~upper) | (((w & 15) | (((y >> 6) & 3) << 4)) & upper);
+        return half_bits_to_float(header[0] & 0xffffu) * static_cast<float>(code);
+    }
+    __device__ __forceinline__ float minimum(int step) const {
+        const int sub = 2 * group + step, shift = 8 * (sub & 3), upper = -(sub >> 2);
+        const int z = static_cast<int>(header[2] >> shift), w = static_cast<int>(header[3] >> shift);
+        const int code = ((z & 63) & ~upper) | ((((w >> 4) & 15) | (((z >> 6) & 3) << 4)) & upper);
+        return half_bits_to_float(header[0] >> 16) * static_cast<float>(code);
+    }
+};
+template <>
+struct Unit<kEncQ4K> : UnitOfQ4KOrQ5K<kEncQ4K> {};
+template <>
+struct Unit<kEncQ5K> : UnitOfQ4KOrQ5K<kEncQ5K> {};
+
+template <>
+struct Unit<kEncQ6K> {
+    static constexpr bool kWide = false, kScaled = true, kMinimum = false, kScalePerChunk = true;
+    u32x2_a2 low[2][2], high[2];  // [step][chunk], [chunk]
+    std::uint32_t scales;         // the unit's four sub-scales, (step, chunk) at byte 2 step + chunk
+    std::uint32_t d;
+    int upper;
+    __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half) {
+        const std::uint8_t* block = row + (unit >> 2) * 210;
+        const int half_block = (unit >> 1) & 1;
+        upper = unit & 1;  // quarters 2 and 3 of the half block: high nibbles, high-bit pairs 2 and 3
+#pragma unroll
+        for (int chunk = 0; chunk < 2; ++chunk) {
+            const int position = 16 * chunk + 8 * half;
+            low[0][chunk] = *reinterpret_cast<const u32x2_a2*>(block + half_block * 64 + position);
+            low[1][chunk] = *reinterpret_cast<const u32x2_a2*>(block + half_block * 64 + 32 + position);
+            high[chunk] = *reinterpret_cast<const u32x2_a2*>(block + 128 + half_block * 32 + position);
+        }
+        const auto* pairs = reinterpret_cast<const std::uint16_t*>(block + 192 + 4 * (unit & 3));
+        scales = pairs[0] | (static_cast<std::uint32_t>(pairs[1]) << 16);
+        d = *reinterpret_cast<const std::uint16_t*>(block + 208);
+    }
+    __device__ __forceinline__ void words(int step, int chunk, int word, std::uint32_t& even, std::uint32_t& odd) const {
+        const std::uint32_t q = ((low[step][chunk][word] >> (4 * upper)) & 0x0f0f0f0fu) |
+            (((high[chunk][word] >> (4 * upper + 2 * step)) & 0x03030303u) << 4);
+        codes_to_bf16(q, 32.0f, even, odd);
+    }
+    __device__ __forceinline__ float scale(int step, int chunk) const {
+        const int code = static_cast<std::int8_t>(scales >> (8 * (2 * step + chunk)));
+        return half_bits_to_float(d) * static_cast<float>(code);
+    }
+    __device__ __forceinline__ float minimum(int) const { return 0.0f; }
+};
+
+template <>
+struct Unit<kEncQ8_0> {
+    static constexpr bool kWide = true, kScaled = true, kMinimum = false, kScalePerChunk = false;
+    u32x4_a2 codes[2];
+    std::uint32_t d[2];
+    // (`steps`: the row's 32-column blocks; a row of an odd number of them reads its last one twice)
+    __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half, int steps) {
+#pragma unroll
+        for (int step = 0; step < 2; ++step) {
+            const std::uint8_t* block = row + min(2 * unit + step, steps - 1) * 34;
+            codes[step] = *reinterpret_cast<const u32x4_a2*>(block + 2 + 16 * half);
+            d[step] = *reinterpret_cast<const std::uint16_t*>(block);
+        }
+    }
+    __device__ __forceinline__ void words(int step, int chunk, int word, std::uint32_t& even, std::uint32_t& odd) const {
+        // (flipping the sign bit turns the code q into the byte q + 128)
+        codes_to_bf16(codes[step][2 * chunk + word] ^ 0x80808080u, 128.0f, even, odd);
+    }
+    __device__ __forceinline__ float scale(int step, int) const { return half_bits_to_float(d[step]); }
+    __device__ __forceinline__ float minimum(int) const { return 0.0f; }
+};
+
+template <>
+struct Unit<kEncBF16> {
+    static constexpr bool kWide = true, kScaled = false, kMinimum = false, kScalePerChunk = false;
+    u32x4_a2 values[2][2];
+    __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half, int steps) {
+#pragma unroll
+        for (int step = 0; step < 2; ++step) {
+            const std::uint8_t* source = row + min(2 * unit + step, steps - 1) * 64 + 32 * half;
+            values[step][0] = *reinterpret_cast<const u32x4_a2*>(source);
+            values[step][1] = *reinterpret_cast<const u32x4_a2*>(source + 16);
+        }
+    }
+    __device__ __forceinline__ void words(int step, int chunk, int word, std::uint32_t& low, std::uint32_t& high) const {
+        low = values[step][chunk][2 * word];
+        high = values[step][chunk][2 * word + 1];
+    }
+    __device__ __forceinline__ float scale(int, int) const { return 1.0f; }
+};
+
+template <>
+struct Unit<kEncF32> {
+    static constexpr bool kWide = true, kScaled = false, kMinimum = false;
+    f32x4_a4 values[2][2][2];  // [step][chunk][piece]
+    __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half, int steps) {
+#pragma unroll
+        for (int step = 0; step < 2; ++step) {
+            const auto* source = reinterpret_cast<const float*>(row) + min(2 * unit + step, steps - 1) * 32 + 16 * half;
+#pragma unroll
+            for (int piece = 0; piece < 4; ++piece) {
+                values[step][piece >> 1][piece & 1] = *reinterpret_cast<const f32x4_a4*>(source + 4 * piece);
+            }
+        }
+    }
+    __device__ __forceinline__ Terms terms(int step, int chunk) const {
+        float eight[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) eight[j] = values[step][chunk][j >> 2][j & 3];
+        return cut(eight);
+    }
+};
+
+// the codes of one chunk
+template <std::uint32_t ENC>
+__device__ __forceinline__ bf16x8 fragment_of(const Unit<ENC>& unit, int step, int chunk) {
+    u32x4 out;
+#pragma unroll
+    for (int word = 0; word < 2; ++word) {
+        std::uint32_t low, high;
+        unit.words(step, chunk, word, low, high);
+        out[2 * word] = low;
+        out[2 * word + 1] = high;
+    }
+    return as_bf16(out);
+}
+
+template <std::uint32_t ENC>
+constexpr bool kWholeBlocks = ENC == kEncQ4K || ENC == kEncQ5K || ENC == kEncQ6K;
+
+__device__ __forceinline__ f32x16 product(bf16x8 a, bf16x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+// the small terms first
+__device__ __forceinline__ f32x16 product(const Terms& a, bf16x8 b, f32x16 c) {
+    return product(a.first, b, product(a.second, b, product(a.third, b, c)));
+}
+__device__ __forceinline__ f32x16 product(const Terms& a, const Terms& b, f32x16 c) {
+    c = product(a.second, b.third, product(a.third, b.second, c));
+    c = product(a.second, b.second, product(a.first, b.third, product(a.third, b.first, c)));
+    return product(a.first, b.first, product(a.second, b.first, product(a.first, b.second, c)));
+}
+
+// One step of 32 columns of one wave: 32 MT input rows (their terms in `a`) by 32 weight rows.
+template <std::uint32_t ENC, int MT>
+__device__ __forceinline__ void multiply(f32x16 (&acc)[MT], const Terms (&a)[MT][2], const Unit<ENC>& unit, int step) {
+    using Slice = Unit<ENC>;
+    if constexpr (!Slice::kScaled) {
+#pragma unroll
+        for (int chunk = 0; chunk < 2; ++chunk) {
+            if constexpr (ENC == kEncF32) {
+                const Terms b = unit.terms(step, chunk);
+#pragma unroll
+                for (int m = 0; m < MT; ++m) acc[m] = product(a[m][chunk], b, acc[m]);
+            } else {
+                const bf16x8 b = fragment_of<ENC>(unit, step, chunk);
+#pragma unroll
+                for (int m = 0; m < MT; ++m) acc[m] = product(a[m][chunk], b, acc[m]);
+            }
+        }
+    } else if constexpr (Slice::kScalePerChunk) {
+#pragma unroll
+        for (int chunk = 0; chunk < 2; ++chunk) {
+            const bf16x8 b = fragment_of<ENC>(unit, step, chunk);
+            const float scale = unit.scale(step, chunk);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const f32x16 sums = product(a[m][chunk], b, f32x16{});
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[m][r] = fmaf(scale, sums[r], acc[m][r]);
+            }
+        }
+    } else {
+        const bf16x8 b0 = fragment_of<ENC>(unit, step, 0), b1 = fragment_of<ENC>(unit, step, 1);
+        const float scale = unit.scale(step, 0);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            f32x16 sums = product(a[m][0].third, b0, f32x16{});
+            sums = product(a[m][1].third, b1, sums);
+            sums = product(a[m][0].second, b0, sums);
+            sums = product(a[m][1].second, b1, sums);
+            sums = product(a[m][0].first, b0, sums);
+            sums = product(a[m][1].first, b1, sums);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[m][r] = fmaf(scale, sums[r], acc[m][r]);
+        }
+    }
+}
+
+template <std::uint32_t ENC>
+__device__ __forceinline__ void load_unit(Unit<ENC>& into, const std::uint8_t* row, int unit, int half, int steps) {
+    if constexpr (kWholeBlocks<ENC>) {
+        into.load(row, unit, half);
+    } else {
+        into.load(row, unit, half, steps);
+    }
+}
+
+// The sums of a tile's waves meet, 32 x 32 outputs at a time: register r of lane l is row
+// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.  GROUPS sets of sums, set g in meeting[g]; the
+// workgroup's wave `wave` of WAVES adds up and stores its registers' worth.
+template <int GROUPS, int WAVES>
+__device__ __forceinline__ void add_up_and_store(const float (*meeting)[16 * kWave], int wave, int lane,
+                                                 const float* bias, float* output, std::int64_t rows,
+                                                 std::int64_t output_dim, std::int64_t row0, std::int64_t column) {
+#pragma unroll
+    for (int part = 0; part < 16 / WAVES; ++part) {
+        const int r = part * WAVES + wave;
+        float total = meeting[0][r * kWave + lane];
+#pragma unroll
+        for (int g = 1; g < GROUPS; ++g) total += meeting[g][r * kWave + lane];
+        const std::int64_t row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        if (row < rows && column < output_dim) {
+            output[row * output_dim + column] = total + (bias != nullptr ? bias[column] : 0.0f);
+        }
+    }
+}
+
+// WAVES waves share a tile of 32 MT input rows x 32 NT weight rows.
+template <std::uint32_t ENC, int MT, int NT, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exact_small_kernel(
+    const std::uint8_t* __restrict__ data, std::int64_t row_stride, const float* __restrict__ input,
+    const float* __restrict__ bias, float* __restrict__ output, std::int64_t rows, std::int64_t input_dim,
+    std::int64_t output_dim, int row_tiles) {
+    using Slice = Unit<ENC>;
+    constexpr int kLow = Slice::kWide ? 16 : 8, kNext = Slice::kWide ? 8 : 16;  // lane's columns: kLow half + kNext chunk
+    __shared__ float meeting[WAVES][16 * kWave];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int inner = lane & 31, half = lane >> 5;
+    const std::int64_t row0 = static_cast<std::int64_t>(blockIdx.x % row_tiles) * (32 * MT);
+    const std::int64_t col0 = static_cast<std::int64_t>(blockIdx.x / row_tiles) * (32 * NT);
+    // Rows past the end read the last one again; their results are not stored.
+    const float* x_row[MT];
+    const std::uint8_t* w_row[NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) x_row[m] = input + min(row0 + 32 * m + inner, rows - 1) * input_dim + kLow * half;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) w_row[n] = data + min(col0 + 32 * n + inner, output_dim - 1) * row_stride;
+    const int steps = static_cast<int>(input_dim / 32);
+    const int units = (steps + 1) / 2;
+    const int first_unit = units * wave / WAVES, end_unit = units * (wave + 1) / WAVES;
+    const int last_step = min(2 * end_unit, steps) - 1;
+
+    f32x16 acc[NT][MT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[n][m] = f32x16{};
+    }
+    f32x4_a4 x[MT][2][2];  // [row tile][chunk][piece] of the step ahead
+    const auto load_inputs = [&](int step) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+#pragma unroll
+            for (int piece = 0; piece < 4; ++piece) {
+                x[m][piece >> 1][piece & 1] = *reinterpret_cast<const f32x4_a4*>(
+                    x_row[m] + static_cast<std::int64_t>(step) * 32 + kNext * (piece >> 1) + 4 * (piece & 1));
+            }
+        }
+    };
+    if (first_unit < end_unit) {
+        Slice now[NT], next[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) load_unit<ENC>(now[n], w_row[n], first_unit, half, steps);
+        load_inputs(2 * first_unit);
+        for (int unit = first_unit; unit < end_unit; ++unit) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n) load_unit<ENC>(next[n], w_row[n], min(unit + 1, end_unit - 1), half, steps);
+            float partial[MT][2];
+#pragma unroll
+            for (int step = 0; step < 2; ++step) {
+                if (!kWholeBlocks<ENC> && 2 * unit + step > last_step) break;  // (uniform: a row's odd last block)
+                Terms a[MT][2];
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    partial[m][step] = 0.0f;
+#pragma unroll
+                    for (int chunk = 0; chunk < 2; ++chunk) {
+                        float eight[8];
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) eight[j] = x[m][chunk][j >> 2][j & 3];
+                        a[m][chunk] = cut(eight);
+                        if constexpr (Slice::kMinimum) partial[m][step] += sum_of(eight);
+                    }
+                }
+                load_inputs(min(2 * unit + step + 1, last_step));
+#pragma unroll
+                for (int n = 0; n < NT; ++n) multiply<ENC, MT>(acc[n], a, now[n], step);
+            }
+            if constexpr (Slice::kMinimum) {
+                // k index = half: the lower lanes bring step 0's sums and minimums, the upper ones
+                // step 1's.  A lane holds half of its row's sum of each step; the other half is 32
+                // lanes away.
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    const float other = __shfl_xor(half != 0 ? partial[m][0] : partial[m][1], 32);
+                    const float total = (half != 0 ? partial[m][1] : partial[m][0]) + other;
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+                        const float least = -(half != 0 ? now[n].minimum(1) : now[n].minimum(0));
+                        acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x2f32(total, least, acc[n][m], 0, 0, 0);
+                    }
+                }
+            }
+#pragma unroll
+            for (int n = 0; n < NT; ++n) now[n] = next[n];
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            if (n + m > 0) __syncthreads();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) meeting[wave][r * kWave + lane] = acc[n][m][r];
+            __syncthreads();
+            add_up_and_store<WAVES, WAVES>(meeting, wave, lane, bias, output, rows, output_dim, row0 + 32 * m,
+                                           col0 + 32 * n + inner);
+        }
+    }
+}
+
+// -- the large form --------------------------------------------------------------------------------
+
+constexpr int kGroups = 4;                      // K groups of a workgroup
+constexpr int kPartners = 2;                    // waves of a K group, 64 weight rows each
+constexpr int kLargeWaves = kGroups * kPartners;
+constexpr int kOctetBytes = 32 * 16 + 32;       // eight columns of 32 rows, as bf16; the padding keeps the
+                                                // writes of four lanes that share a row in distinct banks
+constexpr int kTermBytes = 4 * kOctetBytes;     // one term of 32 rows x 32 columns
+template <int MT>
+constexpr int kStepBytes = 3 * MT * kTermBytes;  // one step of a K group: [term][row tile][octet][row]
+template <int MT>
+constexpr int kSumBytes = 4 * 32 * MT * 4;       // sums of the activations, [step % 4][row]
+template <int MT>
+constexpr int kGroupBytes = 2 * kStepBytes<MT> + kSumBytes<MT>;
+template <int MT>
+constexpr int kLargeLds = kGroups * kGroupBytes<MT>;
+static_assert(kLargeLds<1> >= kGroups * kPartners * 16 * kWave * 4, "the waves' sums meet in the same memory");
+
+template <std::uint32_t ENC, int MT>
+__global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
+    const std::uint8_t* __restrict__ data, std::int64_t row_stride, const float* __restrict__ input,
+    const float* __restrict__ bias, float* __restrict__ output, std::int64_t rows, std::int64_t input_dim,
+    std::int64_t output_dim, int row_tiles) {
+    using Slice = Unit<ENC>;
+    extern __shared__ __attribute__((aligned(16))) std::uint8_t lds[];
+    constexpr int kItems = 2 * MT;  // quads (four columns of a row) that a lane cuts per step
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int group = wave / kPartners, partner = wave % kPartners;
+    const int inner = lane & 31, half = lane >> 5;
+    // row tiles next to each other share their weight rows, which come from L2 for all but one
+    const std::int64_t row0 = static_cast<std::int64_t>(blockIdx.x % row_tiles) * (32 * MT);
+    const std::int64_t col0 = static_cast<std::int64_t>(blockIdx.x / row_tiles) * (64 * kPartners) + 64 * partner;
+    const int steps = static_cast<int>(input_dim / 32);
+    const int units = (steps + 1) / 2;
+    const int first_unit = units * group / kGroups, end_unit = units * (group + 1) / kGroups;
+    const int turns = (units + kGroups - 1) / kGroups;  // the longest group's units: all groups meet at the barriers
+
+    // cutter's role: quad lane % 8 of the rows 8 (2 item + partner) + lane / 8: a load instruction
+    // reads whole 128-byte lines of eight rows
+    std::uint8_t* const own = lds + group * kGroupBytes<MT>;
+    float* const sums = reinterpret_cast<float*>(own + 2 * kStepBytes<MT>);
+    const int quad = lane & 7;
+    const float* x_row[kItems];
+#pragma unroll
+    for (int item = 0; item < kItems; ++item) {
+        x_row[item] = input + min(row0 + 8 * (2 * item + partner) + (lane >> 3), rows - 1) * input_dim + 4 * quad;
+    }
+    const int target = (quad >> 1) * kOctetBytes + (8 * partner + (lane >> 3)) * 16 + (quad & 1) * 8;
+    f32x4_a4 x[kItems];
+    const auto load_input = [&](int item, int step) {
+        x[item] = *reinterpret_cast<const f32x4_a4*>(x_row[item] + static_cast<std::int64_t>(min(step, steps - 1)) * 32);
+    };
+    const auto cut_input = [&](int item, int step) {
+        std::uint32_t a0, b0, c0, a1, b1, c1;
+        cut_pair(x[item][0], x[item][1], a0, b0, c0);
+        cut_pair(x[item][2], x[item][3], a1, b1, c1);
+        std::uint8_t* const stage = own + (step & 1) * kStepBytes<MT> + (item >> 1) * kTermBytes + target + (item & 1) * 256;
+        *reinterpret_cast<uint2*>(stage) = make_uint2(c0, c1);
+        *reinterpret_cast<uint2*>(stage + MT * kTermBytes) = make_uint2(b0, b1);
+        *reinterpret_cast<uint2*>(stage + 2 * MT * kTermBytes) = make_uint2(a0, a1);
+        if constexpr (Slice::kMinimum) {
+            float total = (x[item][0] + x[item][1]) + (x[item][2] + x[item][3]);
+            total += __shfl_xor(total, 1);
+            total += __shfl_xor(total, 2);
+            total += __shfl_xor(total, 4);  // (the eight lanes of a row store the same sum)
+            sums[(step & 3) * 32 * MT + 8 * (2 * item + partner) + (lane >> 3)] = total;
+        }
+    };
+    // multiplier's role: the lane's fragment of a term, octets 2 half + chunk (wide) or 2 chunk + half.
+    // Fragments in the order in which they are used: the small terms first, chunk by chunk where a
+    // scale belongs to a chunk.
+    constexpr int kHalfOctets = Slice::kWide ? 2 : 1, kChunkOctets = Slice::kWide ? 1 : 2;
+    constexpr int kUses = 6, kSum = Slice::kScalePerChunk ? 3 : 6;  // products of a tile, of one scale
+    const auto chunk_of = [](int use) { return Slice::kScalePerChunk ? use / 3 : use & 1; };
+    const auto term_of = [](int use) { return Slice::kScalePerChunk ? use % 3 : use >> 1; };
+    const std::uint8_t* const fragments = own + half * kHalfOctets * kOctetBytes + inner * 16;
+    const auto read_fragment = [&](int use, int m, int step) {
+        return *reinterpret_cast<const bf16x8*>(fragments + (step & 1) * kStepBytes<MT> + term_of(use) * MT * kTermBytes +
+                                                m * kTermBytes + chunk_of(use) * kChunkOctets * kOctetBytes);
+    };
+
+    const std::uint8_t* w_row[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) w_row[n] = data + min(col0 + 32 * n + inner, output_dim - 1) * row_stride;
+    f32x16 acc[2][MT];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[n][m] = f32x16{};
+    }
+    Slice even[2], odd[2];  // packed bytes of the units to come, by the unit's place in the group's run
+    bf16x8 a[kUses];
+    u32x4 b[2][2];  // [n][chunk]: codes; those of n = 0 are decoded a step ahead, those of n = 1 under the first tile
+    float scale[2][2], scale_before[2];
+    const auto load_weights = [&](Slice (&into)[2], int unit) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n) load_unit<ENC>(into[n], w_row[n], min(unit, end_unit - 1), half, steps);
+    };
+    const auto decode_piece = [&](const Slice& source, int n, int step, int piece) {
+        const int chunk = piece >> 1, word = piece & 1;
+        std::uint32_t low, high;
+        source.words(step, chunk, word, low, high);
+        b[n][chunk][2 * word] = low;
+        b[n][chunk][2 * word + 1] = high;
+        if (word == 1) scale[n][chunk] = source.scale(step, chunk);
+    };
+    if (first_unit < end_unit) {
+        load_weights(even, first_unit);
+        load_weights(odd, first_unit + 1);
+#pragma unroll
+        for (int item = 0; item < kItems; ++item) load_input(item, 2 * first_unit);
+#pragma unroll
+        for (int item = 0; item < kItems; ++item) {
+            cut_input(item, 2 * first_unit);
+            load_input(item, 2 * first_unit + 1);
+        }
+#pragma unroll
+        for (int piece = 0; piece < 4; ++piece) decode_piece(even[0], 0, 0, piece);
+    }
+    __syncthreads();
+    if (first_unit < end_unit) {
+#pragma unroll
+        for (int use = 0; use < kUses; ++use) a[use] = read_fragment(use, 0, 2 * first_unit);
+    }
+
+    // One unit, two steps: `own_bytes` holds its packed bytes, `next_bytes` those of the unit behind it.
+    const auto pass = [&](Slice (&own_bytes)[2], const Slice (&next_bytes)[2], int unit) {
+        float least[2] = {};
+#pragma unroll
+        for (int step = 0; step < 2; ++step) {
+            const int at = 2 * unit + step;
+            // A step is 12 MT slots of one matrix instruction each, fenced against reordering: what
+            // stands between two of them is issued in their shadow (32 cycles, eight vector
+            // instructions).  The waves of a unit run in step, so that nothing else would overlap.
+            // Slots bring: the scaling of the sums before; the next step's activations cut and
+            // handed over (before the last tile, whose slots read the next step's fragments) and
+            // their successors requested; codes.
+            constexpr int kSlots = 12 * MT, kHandOver = kSlots - kUses, kPerPiece = MT == 1 ? 2 : 4;
+            f32x16 partial[2];
+#pragma unroll
+            for (int slot = 0; slot < kSlots; ++slot) {
+                const int tile = slot / kUses, use = slot % kUses, m = tile >> 1, n = tile & 1;
+                const int sum = slot / kSum;  // sums since the step's start; partial[sum & 1]
+                __builtin_amdgcn_sched_barrier(0);
+                if (slot == kHandOver) {
+                    __syncthreads();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if constexpr (Slice::kScaled) {
+                    partial[sum & 1] = product(a[use], as_bf16(b[n][chunk_of(use)]),
+                                               slot % kSum == 0 ? f32x16{} : partial[sum & 1]);
+                    if (sum > 0 && slot % kSum >= 1 && slot % kSum <= 2) {
+                        const int before = sum - 1, at_tile = before * kSum / kUses;
+                        const float factor = slot >= kHandOver && (at_tile & 1) == 0 ? scale_before[Slice::kScalePerChunk ? before & 1 : 0]
+                                                                   : scale[at_tile & 1][Slice::kScalePerChunk ? before & 1 : 0];
+#pragma unroll
+                        for (int r = 8 * (slot % kSum - 1); r < 8 * (slot % kSum); ++r) {
+                            acc[at_tile & 1][at_tile >> 1][r] =
+                                fmaf(factor, partial[before & 1][r], acc[at_tile & 1][at_tile >> 1][r]);
+                        }
+                    }
+                } else {
+                    acc[n][m] = product(a[use], as_bf16(b[n][chunk_of(use)]), acc[n][m]);
+                }
+                if (n == 1) a[use] = m + 1 < MT ? read_fragment(use, m + 1, at) : read_fragment(use, 0, at + 1);
+                if (slot % kPerPiece == 0 && slot / kPerPiece < kItems) {
+                    cut_input(slot / kPerPiece, at + 1);
+                    load_input(slot / kPerPiece, at + 2);
+                }
+                if (slot < 4) decode_piece(own_bytes[1], 1, step, slot);
+                if (slot == 4 && step == 1) {
+                    if constexpr (Slice::kMinimum) {
+#pragma unroll
+                        for (int k = 0; k < 2; ++k) least[k] = -(half != 0 ? own_bytes[k].minimum(1) : own_bytes[k].minimum(0));
+                    }
+                    load_weights(own_bytes, unit + 2);
+                }
+                if (slot == kHandOver) {  // (the last sums of n = 0 are scaled below, with the old factors)
+                    scale_before[0] = scale[0][0];
+                    scale_before[1] = scale[0][1];
+                }
+                if (slot > kHandOver && slot <= kHandOver + 4) {
+                    decode_piece(step == 0 ? own_bytes[0] : next_bytes[0], 0, 1 - step, slot - kHandOver - 1);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (Slice::kScaled) {  // the last sums
+                const float factor = scale[1][Slice::kScalePerChunk ? 1 : 0];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    acc[1][MT - 1][r] = fmaf(factor, partial[(kSlots / kSum - 1) & 1][r], acc[1][MT - 1][r]);
+                }
+            }
+            if constexpr (Slice::kMinimum) {
+                // k index = half: the lower lanes bring step 0's sums and minimums, the upper step 1's
+#pragma unroll
+                for (int m = 0; m < MT && step == 1; ++m) {
+                    const float total = sums[((2 * unit + half) & 3) * 32 * MT + 32 * m + inner];
+#pragma unroll
+                    for (int n = 0; n < 2; ++n) {
+                        acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x2f32(total, least[n], acc[n][m], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    };
+    // (uniform: a group without a unit left waits out the turn's two barriers)
+    for (int turn = 0; turn < turns; turn += 2) {
+        const int unit = first_unit + turn;
+        if (unit < end_unit) {
+            pass(even, odd, unit);
+        } else {
+            __syncthreads();
+            __syncthreads();
+        }
+        if (turn + 1 < turns) {
+            if (unit + 1 < end_unit) {
+                pass(odd, even, unit + 1);
+            } else {
+                __syncthreads();
+                __syncthreads();
+            }
+        }
+    }
+    __syncthreads();
+
+    // meeting[group] of either partner's 32 x 32 outputs: partner p's sets lie behind each other
+    float(*meeting)[16 * kWave] = reinterpret_cast<float(*)[16 * kWave]>(lds);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            if (n + m > 0) __syncthreads();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) meeting[partner * kGroups + group][r * kWave + lane] = acc[n][m][r];
+            __syncthreads();
+            add_up_and_store<kGroups, kGroups>(meeting + partner * kGroups, group, lane, bias, output, rows, output_dim,
+                                               row0 + 32 * m, col0 + 32 * n + inner);
+        }
+    }
+}
+
+template <std::uint32_t ENC, int MT>
+void launch_large(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
+                  hipStream_t stream) {
+    const std::int64_t row_tiles = (rows + 32 * MT - 1) / (32 * MT);
+    const std::int64_t column_tiles = (weight.output_dim + 64 * kPartners - 1) / (64 * kPartners);
+    allow_large_lds<linear_exact_kernel<ENC, MT>>();
+    hipLaunchKernelGGL((linear_exact_kernel<ENC, MT>), dim3(static_cast<unsigned>(row_tiles * column_tiles)),
+                       dim3(kLargeWaves * kWave), kLargeLds<MT>, stream, weight.data, weight.row_stride_bytes, input,
+                       bias, output, rows, weight.input_dim, weight.output_dim, static_cast<int>(row_tiles));
+}
+
+template <std::uint32_t ENC, int MT, int NT, int WAVES>
+void launch_small(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
+                  hipStream_t stream) {
+    const std::int64_t row_tiles = (rows + 32 * MT - 1) / (32 * MT);
+    const std::int64_t column_tiles = (weight.output_dim + 32 * NT - 1) / (32 * NT);
+    hipLaunchKernelGGL((linear_exact_small_kernel<ENC, MT, NT, WAVES>),
+                       dim3(static_cast<unsigned>(row_tiles * column_tiles)), dim3(WAVES * kWave), 0, stream,
+                       weight.data, weight.row_stride_bytes, input, bias, output, rows, weight.input_dim,
+                       weight.output_dim, static_cast<int>(row_tiles));
+}
+
+template <std::uint32_t ENC>
+void launch_for(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
+                hipStream_t stream) {
+    // What bounds all forms is the look-up of lines in the unit's vector cache, which a round of
+    // tiles, one workgroup a unit, makes as often however many of its rows are real.  A round of
+    // 32 x 32, 32 x 64, 32 x 128 and 64 x 128 tiles was measured at 21, 27, 43 and 65 us for Q4_K
+    // (33, 46, 78, 90 for Q8_0) at 4,096 columns, of 32 x 32, 64 x 32 and 64 x 64 tiles at 31, 45
+    // and 68 us for F32: the form with the cheapest rounds takes the call.
+    const std::int64_t units = compute_units();
+    const auto rounds = [&](std::int64_t height, std::int64_t width) {
+        const std::int64_t tiles = (rows + height - 1) / height * ((weight.output_dim + width - 1) / width);
+        return static_cast<double>((tiles + units - 1) / units);
+    };
+    const double cost_small = rounds(32, 32);
+    if constexpr (ENC == kEncF32) {
+        const double cost_high = 1.4 * rounds(64, 32), cost_square = 2.1 * rounds(64, 64);
+        if (cost_square <= cost_high && cost_square <= cost_small) {
+            launch_small<ENC, 2, 2, 4>(weight, input, bias, output, rows, stream);
+        } else if (cost_high <= cost_small) {
+            launch_small<ENC, 2, 1, 4>(weight, input, bias, output, rows, stream);
+        } else {
+            launch_small<ENC, 1, 1, 8>(weight, input, bias, output, rows, stream);
+        }
+    } else {
+        const bool whole = weight.input_dim % 64 == 0;
+        const double cost_wide = 1.35 * rounds(32, 64);
+        const double cost_low = whole ? 2.1 * rounds(32, 128) : 1e30, cost_high = whole ? 2.9 * rounds(64, 128) : 1e30;
+        if (cost_high <= cost_low && cost_high <= cost_wide && cost_high <= cost_small) {
+            launch_large<ENC, 2>(weight, input, bias, output, rows, stream);
+        } else if (cost_low <= cost_wide && cost_low <= cost_small) {
+            launch_large<ENC, 1>(weight, input, bias, output, rows, stream);
+        } else if (cost_wide <= cost_small) {
+            launch_small<ENC, 1, 2, 8>(weight, input, bias, output, rows, stream);
+        } else {
+            launch_small<ENC, 1, 1, 16>(weight, input, bias, output, rows, stream);
+        }
+    }
+}
+
+}  // namespace
+
+bool linear_exact_supports(const Descriptor& weight, std::int64_t rows) {
+    const std::int64_t tiles = ((rows + 31) / 32) * ((weight.output_dim + 31) / 32);
+    return rows > 0 && weight.input_dim > 0 && weight.input_dim % 32 == 0 && block_bytes(weight.encoding) != 0 &&
+           weight.input_dim <= (std::int64_t(1) << 30) && tiles < (std::int64_t(1) << 31);
+}
+
+void launch_linear_exact(const Descriptor& weight, const float* input, const float* bias, float* output,
+                         std::int64_t rows, hipStream_t stream) {
+    switch (weight.encoding) {
+        case kEncQ4K: launch_for<kEncQ4K>(weight, input, bias, output, rows, stream); break;
+        case kEncQ5K: launch_for<kEncQ5K>(weight, input, bias, output, rows, stream); break;
+        case kEncQ6K: launch_for<kEncQ6K>(weight, input, bias, output, rows, stream); break;
+        case kEncQ8_0: launch_for<kEncQ8_0>(weight, input, bias, output, rows, stream); break;
+        case kEncBF16: launch_for<kEncBF16>(weight, input, bias, output, rows, stream); break;
+        default: launch_for<kEncF32>(weight, input, bias, output, rows, stream); break;
+    }
+}
+
+}  // namespace nfn

@@ -1,0 +1,234 @@
+// The exact tier at one to three input rows: float activations from LDS, packed weights streamed
+// once, a wave per pair of weight rows (exact_rows.hpp).  What bounds it is the weight stream for
+// one row and the vector ALU (2.25 instructions to decode a weight, one per product) beyond.
+// Rows past three are cheaper on the matrix cores (linear_exact.hip), where a product costs
+// nothing on the vector ALU.  4,096 -> 6,656 of Q4_K at 1 / 3 rows: 30.4 / 40.3 -> 6.3 / 9.0 us
+// against the wave-per-row kernel that loaded two bytes a lane.
+#include "common.hpp"
+#include "exact_rows.hpp"
+#include "kernels.hpp"
+
+namespace nfn {
+
+namespace {
+
+constexpr std::int64_t kMaxLds = 160 * 1024;
+constexpr std::int64_t kMaxDenseLds = 159 * 1024;  // beside the waves' meeting place
+
+template <std::uint32_t ENC, int R>
+__global__ __launch_bounds__(kExactWaves * kWave) void linear_rows_kernel(
+    const std::uint8_t* __restrict__ data, std::int64_t row_stride, const float* __restrict__ input,
+    const float* __restrict__ bias, float* __restrict__ output, std::int64_t input_dim, std::int64_t output_dim) {
+    extern __shared__ __attribute__((aligned(16))) float staged[];
+    exact_rows_stage<R>(input, input_dim, staged);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const std::int64_t pairs = (output_dim + kExactPair - 1) / kExactPair;
+    exact_rows_walk<ENC, R>(data, row_stride, output_dim, input_dim, staged,
+                            static_cast<std::int64_t>(blockIdx.x) * kExactWaves + wave,
+                            static_cast<std::int64_t>(gridDim.x) * kExactWaves, pairs,
+                            [&](std::int64_t row, const float (&sums)[R]) {
+                                if ((threadIdx.x & 63) != 0) return;
+                                const float offset = bias != nullptr ? bias[row] : 0.0f;
+#pragma unroll
+                                for (int r = 0; r < R; ++r) output[r * output_dim + row] = sums[r] + offset;
+                            });
+}
+
+template <std::uint32_t ENC, int R>
+void launch_rows(const Descriptor& weight, const float* input, const float* bias, float* output, hipStream_t stream) {
+    const std::int64_t pairs = (weight.output_dim + kExactPair - 1) / kExactPair;
+    const std::int64_t lds = exact_rows_lds(R, weight.input_dim);
+    // as many workgroups as the units hold at once, every wave with the same number of pairs
+    const std::int64_t resident = std::int64_t(compute_units()) * (lds <= 40 * 1024 ? 4 : lds <= 80 * 1024 ? 2 : 1);
+    const std::int64_t most = (pairs + kExactWaves - 1) / kExactWaves;
+    const std::int64_t turns = (most + resident - 1) / resident;
+    const std::int64_t groups = (most + turns - 1) / turns;
+    allow_large_lds<linear_rows_kernel<ENC, R>>();
+    hipLaunchKernelGGL((linear_rows_kernel<ENC, R>), dim3(static_cast<unsigned>(groups)), dim3(kExactWaves * kWave),
+                       static_cast<unsigned>(lds), stream, weight.data, weight.row_stride_bytes, input, bias, output,
+                       weight.input_dim, weight.output_dim);
+}
+
+// Float and bf16 weights: a wave (SPLIT = 1) or the workgroup's eight waves together (SPLIT = 8, for
+// few weight rows) take a pair of weight rows; a lane reads 16 neighbouring bytes of each, the
+// next turn's requested before this one's are used.  Bound by the weight stream.
+typedef std::uint32_t dense_u32x4 __attribute__((ext_vector_type(4), aligned(2)));
+
+template <std::uint32_t ENC, int R, int SPLIT>
+__global__ __launch_bounds__(kExactWaves * kWave) void dense_rows_kernel(
+    const std::uint8_t* __restrict__ data, std::int64_t row_stride, const float* __restrict__ input,
+    const float* __restrict__ bias, float* __restrict__ output, std::int64_t input_dim, std::int64_t output_dim) {
+    constexpr int kValues = ENC == kEncF32 ? 4 : 8;  // of 16 bytes
+    extern __shared__ __attribute__((aligned(16))) float staged[];
+    __shared__ float meeting[kExactWaves][kExactPair * R];
+    typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+    const int columns = static_cast<int>(input_dim);
+    for (int index = threadIdx.x * 4; index < R * columns; index += kExactWaves * kWave * 4) {
+        *reinterpret_cast<exact_f32x4*>(staged + index) = *reinterpret_cast<const f32x4_a4*>(input + index);
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int pieces = columns / kValues;
+    const int stride = SPLIT == 1 ? kWave : SPLIT * kWave;  // pieces from one turn to the next
+    const int first = SPLIT == 1 ? lane : wave * kWave + lane;
+    const std::int64_t pairs = (output_dim + kExactPair - 1) / kExactPair;
+    const std::int64_t step = SPLIT == 1 ? static_cast<std::int64_t>(gridDim.x) * kExactWaves : gridDim.x;
+    for (std::int64_t pair = SPLIT == 1 ? static_cast<std::int64_t>(blockIdx.x) * kExactWaves + wave : blockIdx.x;
+         pair < pairs; pair += step) {
+        const std::uint8_t* row[kExactPair];
+#pragma unroll
+        for (int k = 0; k < kExactPair; ++k) row[k] = data + min(pair * kExactPair + k, output_dim - 1) * row_stride;
+        constexpr int kAhead = 4;
+        dense_u32x4 held[kAhead][kExactPair];
+        const auto load = [&](dense_u32x4 (&into)[kExactPair], int piece) {
+#pragma unroll
+            for (int k = 0; k < kExactPair; ++k) {
+                into[k] = *reinterpret_cast<const dense_u32x4*>(row[k] + static_cast<std::int64_t>(min(piece, pieces - 1)) * 16);
+            }
+        };
+#pragma unroll
+        for (int turn = 0; turn < kAhead; ++turn) load(held[turn], first + turn * stride);
+        float sums[kExactPair][R] = {};
+        for (int base = first; base < pieces; base += kAhead * stride) {
+#pragma unroll
+            for (int turn = 0; turn < kAhead; ++turn) {
+                const int piece = base + turn * stride;
+                float w[kExactPair][kValues];
+#pragma unroll
+                for (int k = 0; k < kExactPair; ++k) {
+#pragma unroll
+                    for (int j = 0; j < kValues; ++j) {
+                        if constexpr (ENC == kEncF32) {
+                            w[k][j] = __uint_as_float(held[turn][k][j]);
+                        } else {
+                            w[k][j] = __uint_as_float(j & 1 ? held[turn][k][j / 2] & 0xffff0000u
+                                                            : held[turn][k][j / 2] << 16);
+                        }
+                    }
+                }
+                load(held[turn], piece + kAhead * stride);
+                if (piece < pieces) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+#pragma unroll
+                        for (int quad = 0; quad < kValues / 4; ++quad) {
+                            const exact_f32x4 v =
+                                *reinterpret_cast<const exact_f32x4*>(staged + r * columns + piece * kValues + 4 * quad);
+#pragma unroll
+                            for (int k = 0; k < kExactPair; ++k) {
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) sums[k][r] = fmaf(v[j], w[k][4 * quad + j], sums[k][r]);
+                            }
+                        }
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kExactPair; ++k) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) sums[k][r] = wave_sum(sums[k][r]);
+        }
+        if constexpr (SPLIT == 1) {
+            if (lane == 0) {
+#pragma unroll
+                for (int k = 0; k < kExactPair; ++k) {
+                    const std::int64_t at = pair * kExactPair + k;
+                    if (at < output_dim) {
+                        const float offset = bias != nullptr ? bias[at] : 0.0f;
+#pragma unroll
+                        for (int r = 0; r < R; ++r) output[r * output_dim + at] = sums[k][r] + offset;
+                    }
+                }
+            }
+        } else {
+            __syncthreads();
+            if (lane == 0) {
+#pragma unroll
+                for (int k = 0; k < kExactPair; ++k) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r) meeting[wave][k * R + r] = sums[k][r];
+                }
+            }
+            __syncthreads();
+            if (threadIdx.x < kExactPair * R) {
+                const int k = threadIdx.x / R, r = threadIdx.x % R;
+                const std::int64_t at = pair * kExactPair + k;
+                float total = meeting[0][threadIdx.x];
+#pragma unroll
+                for (int w = 1; w < kExactWaves; ++w) total += meeting[w][threadIdx.x];
+                if (at < output_dim) output[r * output_dim + at] = total + (bias != nullptr ? bias[at] : 0.0f);
+            }
+        }
+    }
+}
+
+template <std::uint32_t ENC, int R>
+void launch_dense(const Descriptor& weight, const float* input, const float* bias, float* output, hipStream_t stream) {
+    const std::int64_t pairs = (weight.output_dim + kExactPair - 1) / kExactPair;
+    const std::int64_t lds = R * weight.input_dim * 4;
+    const std::int64_t resident = std::int64_t(compute_units()) * (lds <= 40 * 1024 ? 4 : lds <= 78 * 1024 ? 2 : 1);
+    // few pairs: a workgroup each, so that eight waves walk the row instead of one
+    const bool split = pairs <= 2 * std::int64_t(compute_units());
+    const std::int64_t most = split ? pairs : (pairs + kExactWaves - 1) / kExactWaves;
+    const unsigned groups = static_cast<unsigned>(most < resident ? most : resident);
+    if (split) {
+        allow_large_lds<dense_rows_kernel<ENC, R, kExactWaves>>(kMaxDenseLds);
+        hipLaunchKernelGGL((dense_rows_kernel<ENC, R, kExactWaves>), dim3(groups), dim3(kExactWaves * kWave),
+                           static_cast<unsigned>(lds), stream, weight.data, weight.row_stride_bytes, input, bias, output,
+                           weight.input_dim, weight.output_dim);
+    } else {
+        allow_large_lds<dense_rows_kernel<ENC, R, 1>>(kMaxDenseLds);
+        hipLaunchKernelGGL((dense_rows_kernel<ENC, R, 1>), dim3(groups), dim3(kExactWaves * kWave),
+                           static_cast<unsigned>(lds), stream, weight.data, weight.row_stride_bytes, input, bias, output,
+                           weight.input_dim, weight.output_dim);
+    }
+}
+
+template <std::uint32_t ENC>
+void launch_for(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
+                hipStream_t stream) {
+    const auto launch = [&](auto count) {
+        constexpr int kRows = decltype(count)::value;
+        if constexpr (kExactRowsFormat<ENC>) {
+            launch_rows<ENC, kRows>(weight, input, bias, output, stream);
+        } else {
+            launch_dense<ENC, kRows>(weight, input, bias, output, stream);
+        }
+    };
+    if (rows == 1) {
+        launch(std::integral_constant<int, 1>{});
+    } else if (rows == 2) {
+        launch(std::integral_constant<int, 2>{});
+    } else {
+        launch(std::integral_constant<int, 3>{});
+    }
+}
+
+}  // namespace
+
+bool linear_rows_supports(const Descriptor& weight, std::int64_t rows) {
+    if (rows < 1 || rows > 3) return false;
+    switch (weight.encoding) {
+        case kEncQ4K: case kEncQ5K: case kEncQ6K: case kEncQ8_0:
+            return weight.input_dim % 64 == 0 && exact_rows_lds(rows, weight.input_dim) <= kMaxLds;
+        case kEncF32: case kEncBF16:
+            return weight.input_dim % 8 == 0 && rows * weight.input_dim * 4 <= kMaxDenseLds;
+        default: return false;
+    }
+}
+
+void launch_linear_rows(const Descriptor& weight, const float* input, const float* bias, float* output,
+                        std::int64_t rows, hipStream_t stream) {
+    switch (weight.encoding) {
+        case kEncQ4K: launch_for<kEncQ4K>(weight, input, bias, output, rows, stream); break;
+        case kEncQ5K: launch_for<kEncQ5K>(weight, input, bias, output, rows, stream); break;
+        case kEncQ6K: launch_for<kEncQ6K>(weight, input, bias, output, rows, stream); break;
+        case kEncQ8_0: launch_for<kEncQ8_0>(weight, input, bias, output, rows, stream); break;
+        case kEncBF16: launch_for<kEncBF16>(weight, input, bias, output, rows, stream); break;
+        default: launch_for<kEncF32>(weight, input, bias, output, rows, stream); break;
+    }
+}
+
+}  // namespace nfn

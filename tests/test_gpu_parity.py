@@ -175,6 +175,32 @@ def test_generic_linear_many_rows_against_oracle(cuda, oracle, encoding, rows):
     assert normalised_error(y, expected) <= 1e-5
 
 
+@pytest.mark.parametrize("rows,out_dim,in_dim", [
+    (1, 1, 256), (2, 67, 4352), (3, 130, 512),    # one pass over the weights, rows in LDS
+    (1, 3, 16384), (3, 40, 16384),                # ... of rows that fill LDS, or do not fit it
+    (4, 33, 288), (31, 65, 768), (47, 129, 288),  # 32 x 32 tiles; an odd last step of 32 columns
+    (60, 5000, 256), (100, 6600, 320), (200, 6600, 512),  # 32 x 64, 32 x 128 and 64 x 128 tiles (F32: up to 64 x 64)
+])
+@pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
+def test_exact_linear_forms_at_their_edges(cuda, oracle, encoding, rows, out_dim, in_dim):
+    """Every form of the exact linear against the oracle's double sums, a row six orders of
+    magnitude larger than the others among them.  Bound: a float sum of K terms is off by at
+    most K 2^-24 of the sum of magnitudes; with random signs by about sqrt(K) of that, and the
+    largest output of a row is some four standard deviations: 1e-5 covers K = 16,384."""
+    if in_dim % kquant.BLOCKS[encoding][0]:
+        in_dim += 256 - in_dim % 256  # whole blocks
+    packed = kquant.quantize(encoding, kquant.synthetic_weights(5 + rows, out_dim, in_dim))
+    x = kquant.synthetic_activations(6 + rows, rows, in_dim) + np.float32(0.3)
+    x[rows - 1] *= np.float32(1e6)
+    bias = np.linspace(-1, 1, out_dim, dtype=np.float32)
+    weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    y = tile_ops.linear(weight, to_device(x, cuda), to_device(bias, cuda)).cpu().numpy()
+    expected = oracle.linear(encoding, packed, out_dim, in_dim, x, bias=bias)
+    for row in {0, rows // 2, rows - 1}:
+        assert normalised_error(y[row], expected[row]) <= 1e-5, row
+    assert normalised_error(y[: rows - 1], expected[: rows - 1]) <= 1e-5 if rows > 1 else True
+
+
 # ------------------------------------------------------------ public Q8_1 path
 
 def crafted_q8_input(rows, in_dim):
