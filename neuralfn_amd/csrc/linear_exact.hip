@@ -331,13 +331,29 @@ __device__ __forceinline__ void load_unit(Unit<ENC>& into, const std::uint8_t* r
     }
 }
 
+// One output the plain way: decoded weights times the activations as they are.
+__device__ __forceinline__ float plain_dot(std::uint32_t encoding, const std::uint8_t* row, const float* x,
+                                           std::int64_t input_dim) {
+    float total = 0.0f;
+#pragma unroll 1
+    for (std::int64_t column = 0; column < input_dim; ++column) {
+        total = fmaf(x[column], weight_value(encoding, row, column), total);
+    }
+    return total;
+}
+
 // The sums of a tile's waves meet, 32 x 32 outputs at a time: register r of lane l is row
 // 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.  GROUPS sets of sums, set g in meeting[g]; the
 // workgroup's wave `wave` of WAVES adds up and stores its registers' worth.
-template <int GROUPS, int WAVES>
+// A sum that is not finite is taken again the plain way: infinity less its own upper half is NaN
+// where the product with the weight is infinite, and the products with the codes leave the
+// float range before those with the weights, which are smaller, do.
+template <std::uint32_t ENC, int GROUPS, int WAVES>
 __device__ __forceinline__ void add_up_and_store(const float (*meeting)[16 * kWave], int wave, int lane,
-                                                 const float* bias, float* output, std::int64_t rows,
-                                                 std::int64_t output_dim, std::int64_t row0, std::int64_t column) {
+                                                 const std::uint8_t* data, std::int64_t row_stride, const float* input,
+                                                 std::int64_t input_dim, const float* bias, float* output,
+                                                 std::int64_t rows, std::int64_t output_dim, std::int64_t row0,
+                                                 std::int64_t column) {
 #pragma unroll
     for (int part = 0; part < 16 / WAVES; ++part) {
         const int r = part * WAVES + wave;
@@ -346,6 +362,7 @@ __device__ __forceinline__ void add_up_and_store(const float (*meeting)[16 * kWa
         for (int g = 1; g < GROUPS; ++g) total += meeting[g][r * kWave + lane];
         const std::int64_t row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
         if (row < rows && column < output_dim) {
+            if (!isfinite(total)) total = plain_dot(ENC, data + column * row_stride, input + row * input_dim, input_dim);
             output[row * output_dim + column] = total + (bias != nullptr ? bias[column] : 0.0f);
         }
     }
@@ -450,8 +467,8 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
 #pragma unroll
             for (int r = 0; r < 16; ++r) meeting[wave][r * kWave + lane] = acc[n][m][r];
             __syncthreads();
-            add_up_and_store<WAVES, WAVES>(meeting, wave, lane, bias, output, rows, output_dim, row0 + 32 * m,
-                                           col0 + 32 * n + inner);
+            add_up_and_store<ENC, WAVES, WAVES>(meeting, wave, lane, data, row_stride, input, input_dim, bias, output,
+                                                rows, output_dim, row0 + 32 * m, col0 + 32 * n + inner);
         }
     }
 }
@@ -693,8 +710,9 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
 #pragma unroll
             for (int r = 0; r < 16; ++r) meeting[partner * kGroups + group][r * kWave + lane] = acc[n][m][r];
             __syncthreads();
-            add_up_and_store<kGroups, kGroups>(meeting + partner * kGroups, group, lane, bias, output, rows, output_dim,
-                                               row0 + 32 * m, col0 + 32 * n + inner);
+            add_up_and_store<ENC, kGroups, kGroups>(meeting + partner * kGroups, group, lane, data, row_stride, input,
+                                                    input_dim, bias, output, rows, output_dim, row0 + 32 * m,
+                                                    col0 + 32 * n + inner);
         }
     }
 }

@@ -201,6 +201,28 @@ def test_exact_linear_forms_at_their_edges(cuda, oracle, encoding, rows, out_dim
     assert normalised_error(y[: rows - 1], expected[: rows - 1]) <= 1e-5 if rows > 1 else True
 
 
+@pytest.mark.parametrize("rows,out_dim,in_dim", [(3, 67, 512), (5, 67, 512), (60, 5000, 256), (100, 6600, 256), (200, 6600, 256)])
+@pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
+def test_exact_linear_of_infinities_nan_and_large_activations(cuda, oracle, encoding, rows, out_dim, in_dim):
+    """Activations that are infinite, NaN or whose products with the codes (but not with the
+    weights) leave the float range: what the products with the decoded weights give."""
+    packed = kquant.quantize(encoding, kquant.synthetic_weights(5 + rows, out_dim, in_dim))
+    x = kquant.synthetic_activations(6 + rows, rows, in_dim)
+    x[0, 37] = np.inf
+    x[1, 200] = np.nan
+    x[2] *= np.float32(3e37) / np.abs(x[2]).max()
+    weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    y = tile_ops.linear(weight, to_device(x, cuda)).cpu().numpy()
+    w = oracle.dequantize(encoding, packed, out_dim, in_dim).reshape(out_dim, in_dim).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        expected = x.astype(np.float64) @ w.T
+    assert np.array_equal(np.isnan(y), np.isnan(expected))
+    infinite = np.isinf(expected)
+    assert infinite[0].any() and np.array_equal(np.isinf(y), infinite) and np.array_equal(y[infinite], expected[infinite])
+    for row in {2, rows - 1}:
+        assert normalised_error(y[row], expected[row]) <= 1e-5, row
+
+
 # ------------------------------------------------------------ public Q8_1 path
 
 def crafted_q8_input(rows, in_dim):
