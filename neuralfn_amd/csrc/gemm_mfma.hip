@@ -29,7 +29,7 @@
 // against reordering, so that the dequantization, the LDS traffic and the
 // global loads of later steps are issued in the shadow of the matrix
 // instructions; weight fragments are read one K chunk ahead, packed bytes are
-// loaded three steps before they are decoded.  Consecutive workgroups walk M first: with 8 XCDs picking
+// loaded three steps before they are decoded (Q6_K: two).  Consecutive workgroups walk M first: with 8 XCDs picking
 // workgroups round robin each XCD keeps one or two 256-row slices of X in its
 // L2 while the packed weights stream through.
 //
@@ -58,6 +58,9 @@ constexpr int kFragmentBytes = 1024;  // 32 rows x 16 K values of fp16 in operan
 
 struct __attribute__((packed, aligned(2))) Chunk16 {
     std::uint32_t v[4];
+};
+struct __attribute__((packed, aligned(2))) Chunk8 {
+    std::uint32_t v[2];
 };
 
 // ---------------------------------------------------------------------------
@@ -176,14 +179,26 @@ __global__ __launch_bounds__(256) void prepare_activations_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// What one thread holds of the packed weights of one K step: its row's 16
-// bytes of codes for positions 16*half .. 16*half+15 of both 32-value groups
-// of the step.  Decoding is cut into pieces of
+// What one thread holds of the packed weights: 32 weights of a K step, in two runs of 16.
+//   Q4_K, Q5_K: positions 16*part .. 16*part+15 of both 32-value groups of the step, of one row;
+//               two neighbouring lanes share a row.
+//   Q6_K, Q8_0: the step's columns 16*part .. 16*part+15 of two rows, 64 apart; four neighbouring
+//               lanes share a row.  A Q6_K slice serves the two steps of a half block, whose
+//               codes share their bytes.
+// A load instruction looks up every cache line that its lanes touch, and with a row a lane
+// (64 lines for 1 KB, more where the pieces straddle lines) those look-ups, not the matrix
+// instructions, bounded Q6_K: three such loads a step, 2,048 x 16,384 -> 6,656 in 764 us where
+// Q4_K took 467.  Lanes that share a row share its lines: 556 (Q6_K), Q8_0 687 -> 542, Q5_K 507 ->
+// 490, Q4_K 461; 17 rows 98 -> 66 us (Q6_K), 86 -> 64 (Q8_0).
+// Decoding is cut into pieces of
 // at most eight vector instructions so that each fits behind one matrix
 // instruction: prepare_bits() and prepare_scales() derive the fp16 scale
 // constants; group_a<I>() / group_b<I>() decode code word I into positions
-// 4I..4I+3 of the first / second group (two packed fp16 pairs).
+// 4I..4I+3 of the first / second run (two packed fp16 pairs).
 // ---------------------------------------------------------------------------
+struct WeightRows {
+    const std::uint8_t *first, *second;  // (second: Q6_K and Q8_0)
+};
 template <std::uint32_t ENC>
 struct PackedSlice;
 // what all K steps of one 256-value block share; loaded once per block
@@ -202,8 +217,8 @@ template <>
 struct PackedSlice<kEncQ4K> {
     u32x4 codes;
     KBlockScales c;
-    __device__ __forceinline__ void load(const std::uint8_t* row, int block, int pair, int half) {
-        codes = *reinterpret_cast<const u32x4*>(row + block * 144 + 16 + pair * 32 + half * 16);
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
+        codes = *reinterpret_cast<const u32x4*>(rows.first + block * 144 + 16 + pair * 32 + part * 16);
     }
     __device__ __forceinline__ void prepare_bits(const BlockHeader<kEncQ4K>& header, int pair, int) {
         c.bits(header.words, pair);
@@ -235,10 +250,10 @@ struct PackedSlice<kEncQ5K> {
     u32x4 codes, high;
     KBlockScales c;
     int high_shift;
-    __device__ __forceinline__ void load(const std::uint8_t* row, int block, int pair, int half) {
-        const std::uint8_t* p = row + block * 176;
-        high = *reinterpret_cast<const u32x4*>(p + 16 + half * 16);
-        codes = *reinterpret_cast<const u32x4*>(p + 48 + pair * 32 + half * 16);
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
+        const std::uint8_t* p = rows.first + block * 176;
+        high = *reinterpret_cast<const u32x4*>(p + 16 + part * 16);
+        codes = *reinterpret_cast<const u32x4*>(p + 48 + pair * 32 + part * 16);
     }
     __device__ __forceinline__ void prepare_bits(const BlockHeader<kEncQ5K>& header, int pair, int) {
         c.bits(header.words, pair);
@@ -262,65 +277,53 @@ struct PackedSlice<kEncQ5K> {
 };
 
 template <>
-struct BlockHeader<kEncQ6K> {
-    // sixteen int8 sub-scales in four words, then d; five plain words, so that the
-    // struct has no padding for a copy to carry through scratch memory
-    std::uint32_t scales_x, scales_y, scales_z, scales_w;
-    std::uint32_t d_bits;
-    __device__ __forceinline__ void load(const std::uint8_t* row, int block) {
-        const std::uint8_t* p = row + block * 210;
-        const Chunk16 s = *reinterpret_cast<const Chunk16*>(p + 192);
-        scales_x = s.v[0];
-        scales_y = s.v[1];
-        scales_z = s.v[2];
-        scales_w = s.v[3];
-        d_bits = *reinterpret_cast<const std::uint16_t*>(p + 208);
-    }
+struct BlockHeader<kEncQ6K> {  // the scales come with the slice
+    __device__ __forceinline__ void load(const std::uint8_t*, int) {}
 };
 
 template <>
 struct PackedSlice<kEncQ6K> {
-    // a K step of 64 is two quarters (32 values each) of one half of the block:
-    // quarters (0,1) or (2,3); `pair` = 2*half_of_block + (quarters 2,3 ? 1 : 0)
-    u32x4 low_a, low_b, high;
+    // a K step of 64 is two quarters (32 values each) of one half of the block: quarters (0,1) or
+    // (2,3), the low or the high nibbles of the half's 64 bytes; `pair` = 2 * half + (quarters 2,3 ? 1 : 0)
+    u32x4 low_a, high_a, low_b, high_b;
+    std::uint32_t scales_a[2], scales_b[2], d_a, d_b;  // the half's eight sub-scales; [0]: quarters 0,1
     f16x2 scale_a, scale_b;
-    int upper, sa, sb;
-    __device__ __forceinline__ void load(const std::uint8_t* row, int block, int pair, int half) {
-        const std::uint8_t* p = row + block * 210;
-        const int block_half = pair >> 1;
-        const Chunk16 la = *reinterpret_cast<const Chunk16*>(p + block_half * 64 + half * 16);
-        const Chunk16 lb = *reinterpret_cast<const Chunk16*>(p + block_half * 64 + 32 + half * 16);
-        const Chunk16 hb = *reinterpret_cast<const Chunk16*>(p + 128 + block_half * 32 + half * 16);
-        low_a = u32x4{la.v[0], la.v[1], la.v[2], la.v[3]};
-        low_b = u32x4{lb.v[0], lb.v[1], lb.v[2], lb.v[3]};
-        high = u32x4{hb.v[0], hb.v[1], hb.v[2], hb.v[3]};
+    int upper, high_shift, sa, sb;
+    __device__ __forceinline__ static void load_row(const std::uint8_t* p, int half, int part, u32x4& low, u32x4& high,
+                                                    std::uint32_t (&scales)[2], std::uint32_t& d) {
+        const Chunk16 l = *reinterpret_cast<const Chunk16*>(p + half * 64 + part * 16);
+        const Chunk16 h = *reinterpret_cast<const Chunk16*>(p + 128 + half * 32 + (part & 1) * 16);
+        const Chunk8 sc = *reinterpret_cast<const Chunk8*>(p + 192 + half * 8);
+        low = u32x4{l.v[0], l.v[1], l.v[2], l.v[3]};
+        high = u32x4{h.v[0], h.v[1], h.v[2], h.v[3]};
+        scales[0] = sc.v[0];
+        scales[1] = sc.v[1];
+        d = *reinterpret_cast<const std::uint16_t*>(p + 208);
     }
-    __device__ __forceinline__ void prepare_bits(const BlockHeader<kEncQ6K>& header, int pair,
-                                                 int half) {
-        // sub-scale index = 8*half_of_block + 2*quarter + position/16: the step's four
-        // are word `pair` of the sixteen, and this thread's 16 positions share one per quarter
-        const std::uint32_t sub_scales = pair == 0 ? header.scales_x
-            : pair == 1 ? header.scales_y : pair == 2 ? header.scales_z : header.scales_w;
-        sa = static_cast<std::int8_t>((sub_scales >> (8 * half)) & 0xffu);
-        sb = static_cast<std::int8_t>((sub_scales >> (8 * (2 + half))) & 0xffu);
-        upper = (pair & 1) * 4;  // quarters 2,3: high nibbles, high-bit pairs 4..7
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
+        load_row(rows.first + block * 210, pair >> 1, part, low_a, high_a, scales_a, d_a);
+        load_row(rows.second + block * 210, pair >> 1, part, low_b, high_b, scales_b, d_b);
     }
-    __device__ __forceinline__ void prepare_scales(const BlockHeader<kEncQ6K>& header) {
-        const float d = half_bits_to_float(header.d_bits);
-        scale_a = splat(d * static_cast<float>(sa));
-        scale_b = splat(d * static_cast<float>(sb));
+    __device__ __forceinline__ void prepare_bits(const BlockHeader<kEncQ6K>&, int pair, int part) {
+        // sub-scale of the run: 2*quarter + position/16 = 4 * (pair & 1) + part of the half's eight
+        sa = static_cast<std::int8_t>((scales_a[pair & 1] >> (8 * part)) & 0xffu);
+        sb = static_cast<std::int8_t>((scales_b[pair & 1] >> (8 * part)) & 0xffu);
+        upper = (pair & 1) * 4;                   // quarters 2,3: high nibbles,
+        high_shift = upper + 2 * (part >> 1);     // bit pairs 2 and 3 of the high bits
+    }
+    __device__ __forceinline__ void prepare_scales(const BlockHeader<kEncQ6K>&) {
+        scale_a = splat(half_bits_to_float(d_a) * static_cast<float>(sa));
+        scale_b = splat(half_bits_to_float(d_b) * static_cast<float>(sb));
     }
     // bias: 1024 + the format's offset of 32
     template <int I>
     __device__ __forceinline__ void group_a(std::uint32_t (&out)[2]) const {
-        const std::uint32_t top = high[I] >> upper;  // bits 0,1: first quarter
-        const std::uint32_t q = ((low_a[I] >> upper) & 0x0f0f0f0fu) | ((top & 0x03030303u) << 4);
+        const std::uint32_t q = ((low_a[I] >> upper) & 0x0f0f0f0fu) | (((high_a[I] >> high_shift) & 0x03030303u) << 4);
         scale_bytes(q, splat(-1056.0f), scale_a, splat(0.0f), out[0], out[1]);
     }
     template <int I>
     __device__ __forceinline__ void group_b(std::uint32_t (&out)[2]) const {
-        const std::uint32_t top = high[I] >> upper;  // bits 2,3: second quarter
-        const std::uint32_t q = ((low_b[I] >> upper) & 0x0f0f0f0fu) | ((top & 0x0c0c0c0cu) << 2);
+        const std::uint32_t q = ((low_b[I] >> upper) & 0x0f0f0f0fu) | (((high_b[I] >> high_shift) & 0x03030303u) << 4);
         scale_bytes(q, splat(-1056.0f), scale_b, splat(0.0f), out[0], out[1]);
     }
 };
@@ -336,14 +339,15 @@ struct PackedSlice<kEncQ8_0> {
     u32x4 codes_a, codes_b;
     std::uint32_t d_a, d_b;
     f16x2 scale_a, scale_b;
-    __device__ __forceinline__ void load(const std::uint8_t* row, int block, int pair, int half) {
-        const std::uint8_t* p = row + (block * 8 + pair * 2) * 34;
-        const Chunk16 a = *reinterpret_cast<const Chunk16*>(p + 2 + half * 16);
-        const Chunk16 b = *reinterpret_cast<const Chunk16*>(p + 34 + 2 + half * 16);
-        codes_a = u32x4{a.v[0], a.v[1], a.v[2], a.v[3]};
-        codes_b = u32x4{b.v[0], b.v[1], b.v[2], b.v[3]};
-        d_a = *reinterpret_cast<const std::uint16_t*>(p);
-        d_b = *reinterpret_cast<const std::uint16_t*>(p + 34);
+    __device__ __forceinline__ static void load_row(const std::uint8_t* p, int part, u32x4& codes, std::uint32_t& d) {
+        const Chunk16 c = *reinterpret_cast<const Chunk16*>(p + 2 + (part & 1) * 16);
+        codes = u32x4{c.v[0], c.v[1], c.v[2], c.v[3]};
+        d = *reinterpret_cast<const std::uint16_t*>(p);
+    }
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
+        const int offset = (block * 8 + pair * 2 + (part >> 1)) * 34;
+        load_row(rows.first + offset, part, codes_a, d_a);
+        load_row(rows.second + offset, part, codes_b, d_b);
     }
     __device__ __forceinline__ void prepare_bits(const BlockHeader<kEncQ8_0>&, int, int) {}
     __device__ __forceinline__ void prepare_scales(const BlockHeader<kEncQ8_0>&) {
@@ -362,6 +366,16 @@ struct PackedSlice<kEncQ8_0> {
         scale_bytes(codes_b[I] ^ 0x80808080u, splat(-1152.0f), scale_b, splat(0.0f), out[0], out[1]);
     }
 };
+
+// lanes that share a weight row
+template <std::uint32_t ENC>
+constexpr int kParts = ENC == kEncQ4K || ENC == kEncQ5K ? 2 : 4;
+// a slice serves two steps
+template <std::uint32_t ENC>
+constexpr bool kHalfBlocks = ENC == kEncQ6K;
+// from the first run of 16 to the second, in the stage
+template <std::uint32_t ENC>
+constexpr int kSecondRun = kParts<ENC> == 2 ? 64 : 64 * kRowBytes;
 
 // The activation fragments of one K step for one wave: row blocks 0 and 1,
 // K chunks 0..3, in named registers (an array here ends up in scratch memory).
@@ -401,19 +415,19 @@ struct WeightFragments {
 //   b_next:   packed weights of the next step: dequantized into the other
 //             stage with the scales in `header`, then refilled with the packed
 //             bytes of `fetch_step`
-template <std::uint32_t ENC, int RB>
+template <std::uint32_t ENC, int RB, bool REFILL>
 __device__ __forceinline__ void k_step(
     v16f (&acc)[RB][4], ActivationSlice& a_now, WeightFragments& current,
     const std::uint8_t* b_read, const std::uint8_t* b_read_next, std::uint8_t* b_write,
-    PackedSlice<ENC>& b_next, const BlockHeader<ENC>& header, int decode_pair, int b_half,
-    const std::uint8_t* a_fetch, std::int64_t row_block_bytes, const std::uint8_t* b_global,
+    PackedSlice<ENC>& b_next, const BlockHeader<ENC>& header, int decode_pair, int b_part,
+    const std::uint8_t* a_fetch, std::int64_t row_block_bytes, const WeightRows& b_global,
     int fetch_step) {
     WeightFragments ahead;
     std::uint32_t w[2], v[2];
 
     if constexpr (RB == 1) {
         // One row block per wave: 16 slots carry the same side work.
-        NFN_SLOT(a_now.r0k0, current.c0, acc[0][0], b_next.prepare_bits(header, decode_pair, b_half))
+        NFN_SLOT(a_now.r0k0, current.c0, acc[0][0], b_next.prepare_bits(header, decode_pair, b_part))
         NFN_SLOT(a_now.r0k0, current.c1, acc[0][1], b_next.prepare_scales(header);
                  ahead.c0 = NFN_READ_WEIGHTS(b_read, 0, 1))
         NFN_SLOT(a_now.r0k0, current.c2, acc[0][2], b_next.template group_a<0>(w);
@@ -429,12 +443,12 @@ __device__ __forceinline__ void k_step(
         NFN_SLOT(a_now.r0k1, ahead.c2, acc[0][2], b_next.template group_b<0>(w);
                  current.c2 = NFN_READ_WEIGHTS(b_read, 2, 2))
         NFN_SLOT(a_now.r0k1, ahead.c3, acc[0][3], b_next.template group_b<1>(v);
-                 NFN_WRITE16(b_write + 64, w[0], w[1], v[0], v[1]); current.c3 = NFN_READ_WEIGHTS(b_read, 3, 2))
+                 NFN_WRITE16(b_write + kSecondRun<ENC>, w[0], w[1], v[0], v[1]); current.c3 = NFN_READ_WEIGHTS(b_read, 3, 2))
         NFN_SLOT(a_now.r0k2, current.c0, acc[0][0], b_next.template group_b<2>(w);
                  ahead.c0 = NFN_READ_WEIGHTS(b_read, 0, 3);
                  a_now.r0k1 = NFN_LOAD_ACTIVATIONS(a_fetch, 0, 1))
         NFN_SLOT(a_now.r0k2, current.c1, acc[0][1], b_next.template group_b<3>(v);
-                 NFN_WRITE16(b_write + 80, w[0], w[1], v[0], v[1]); ahead.c1 = NFN_READ_WEIGHTS(b_read, 1, 3))
+                 NFN_WRITE16(b_write + kSecondRun<ENC> + 16, w[0], w[1], v[0], v[1]); ahead.c1 = NFN_READ_WEIGHTS(b_read, 1, 3))
         NFN_SLOT(a_now.r0k2, current.c2, acc[0][2], ahead.c2 = NFN_READ_WEIGHTS(b_read, 2, 3))
         NFN_SLOT(a_now.r0k2, current.c3, acc[0][3], ahead.c3 = NFN_READ_WEIGHTS(b_read, 3, 3))
         __syncthreads();
@@ -445,13 +459,13 @@ __device__ __forceinline__ void k_step(
         NFN_SLOT(a_now.r0k3, ahead.c3, acc[0][3], current.c3 = NFN_READ_WEIGHTS(b_read_next, 3, 0))
         a_now.r0k3 = NFN_LOAD_ACTIVATIONS(a_fetch, 0, 3);
         NFN_FENCE();
-        b_next.load(b_global, fetch_step >> 2, fetch_step & 3, b_half);
+        if constexpr (REFILL) b_next.load(b_global, fetch_step >> 2, fetch_step & 3, b_part);
         NFN_FENCE();
         return;
     } else {
     // K chunk 0: read chunk 1, decode; every decoded group of four values is
     // written to the other stage at once (8 bytes), which keeps few registers live
-    NFN_SLOT(a_now.r0k0, current.c0, acc[0][0], b_next.prepare_bits(header, decode_pair, b_half))
+    NFN_SLOT(a_now.r0k0, current.c0, acc[0][0], b_next.prepare_bits(header, decode_pair, b_part))
     NFN_SLOT(a_now.r0k0, current.c1, acc[0][1], b_next.prepare_scales(header);
              ahead.c0 = NFN_READ_WEIGHTS(b_read, 0, 1))
     NFN_SLOT(a_now.r0k0, current.c2, acc[0][2], b_next.template group_a<0>(w);
@@ -466,13 +480,13 @@ __device__ __forceinline__ void k_step(
     NFN_SLOT(a_now.r1k0, current.c2, acc[1][2], b_next.template group_b<0>(w);
              ahead.c3 = NFN_READ_WEIGHTS(b_read, 3, 1))
     NFN_SLOT(a_now.r1k0, current.c3, acc[1][3], b_next.template group_b<1>(v);
-             NFN_WRITE16(b_write + 64, w[0], w[1], v[0], v[1]))
+             NFN_WRITE16(b_write + kSecondRun<ENC>, w[0], w[1], v[0], v[1]))
     // K chunk 1: read chunk 2, finish decoding
     NFN_SLOT(a_now.r0k1, ahead.c0, acc[0][0], b_next.template group_b<2>(w);
              current.c0 = NFN_READ_WEIGHTS(b_read, 0, 2);
              a_now.r1k0 = NFN_LOAD_ACTIVATIONS(a_fetch, 1, 0))
     NFN_SLOT(a_now.r0k1, ahead.c1, acc[0][1], b_next.template group_b<3>(v);
-             NFN_WRITE16(b_write + 80, w[0], w[1], v[0], v[1]))
+             NFN_WRITE16(b_write + kSecondRun<ENC> + 16, w[0], w[1], v[0], v[1]))
     NFN_SLOT(a_now.r0k1, ahead.c2, acc[0][2], current.c1 = NFN_READ_WEIGHTS(b_read, 1, 2))
     NFN_SLOT(a_now.r0k1, ahead.c3, acc[0][3], (void)0)
     NFN_SLOT(a_now.r1k1, ahead.c0, acc[1][0], current.c2 = NFN_READ_WEIGHTS(b_read, 2, 2);
@@ -511,7 +525,7 @@ __device__ __forceinline__ void k_step(
     NFN_SLOT(a_now.r1k3, ahead.c3, acc[1][3], (void)0)
     a_now.r1k3 = NFN_LOAD_ACTIVATIONS(a_fetch, 1, 3);
     NFN_FENCE();
-    b_next.load(b_global, fetch_step >> 2, fetch_step & 3, b_half);
+    if constexpr (REFILL) b_next.load(b_global, fetch_step >> 2, fetch_step & 3, b_part);
     NFN_FENCE();
     }
 }
@@ -523,9 +537,9 @@ constexpr int kBlockBytes = ENC == kEncQ4K ? 144 : ENC == kEncQ5K ? 176 : ENC ==
 // Workgroups per compute unit (= waves per SIMD): as many as the registers
 // allow; while one wave waits at the barrier or for LDS, another keeps the
 // matrix pipe busy.  With 256-row tiles the Q6_K decode holds too much live
-// state for two.
+// state for two (of 22 registers in scratch memory with two).
 template <std::uint32_t ENC, int RB>
-constexpr int kWavesPerSimd = ENC == kEncQ6K ? RB == 1 ? 2 : 1 : RB == 1 ? (ENC == kEncQ5K ? 2 : 3) : 2;
+constexpr int kWavesPerSimd = ENC == kEncQ6K ? RB == 1 ? 2 : 1 : RB == 1 && ENC == kEncQ4K ? 3 : 2;
 
 // RB: 32-row blocks per wave; the workgroup's tile is 128*RB rows by 128 columns.
 template <std::uint32_t ENC, int RB>
@@ -558,14 +572,17 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     const std::uint8_t* a_global = activations + (m0 / 32 + wave * RB) * row_block_bytes +
         static_cast<std::int64_t>(first_block) * 16 * kFragmentBytes + lane * 16;
     constexpr int kStepBytes = (kBK / 16) * kFragmentBytes;
-    // weights: thread -> (row, which 16 positions of the two 32-value groups)
-    // (sixteen consecutive lanes write sixteen consecutive stage rows: with rows of 144 bytes
-    // their 16-byte pieces fall into distinct banks, as the fragment reads do)
-    const int b_row = tid & 127;
-    const int b_half = tid >> 7;
-    const std::uint8_t* b_global = weights + min(n0 + b_row, output_dim - 1) * row_stride +
-        static_cast<std::int64_t>(first_block) * kBlockBytes<ENC>;
-    const int b_target = b_row * kRowBytes + b_half * 32;
+    // weights: thread -> (row, which run of 16).  Eight consecutive lanes write their 16-byte
+    // pieces into distinct banks: with stage rows of 36 words and runs of 8, rows k and k + 1
+    // times four runs do, and so do rows k, k + 1, k + 4, k + 5 times two.
+    const int b_part = tid & (kParts<ENC> - 1);
+    const int b_turn = tid / kParts<ENC>;
+    const int b_row = kParts<ENC> == 4 ? b_turn : (b_turn & ~6) | ((b_turn & 2) << 1) | ((b_turn & 4) >> 1);
+    const std::int64_t b_skip = static_cast<std::int64_t>(first_block) * kBlockBytes<ENC>;
+    WeightRows b_global;
+    b_global.first = weights + min(n0 + b_row, output_dim - 1) * row_stride + b_skip;
+    b_global.second = weights + min(n0 + b_row + 64, output_dim - 1) * row_stride + b_skip;
+    const int b_target = b_row * kRowBytes + b_part * 32;
 
     v16f acc[RB][4];
 #pragma unroll
@@ -590,12 +607,16 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     PackedSlice<ENC> b0, b1, b2, b3;
     BlockHeader<ENC> header_even, header_odd;  // blocks 0, 2, 4 ... and 1, 3, 5 ...
     const int last_block = (steps >> 2) - 1;
-    header_even.load(b_global, 0);
-    header_odd.load(b_global, min(1, last_block));
-    b0.load(b_global, 0, 0, b_half);
-    b1.load(b_global, 0, 1, b_half);
-    b2.load(b_global, 0, 2, b_half);
-    b3.load(b_global, 0, 3, b_half);
+    header_even.load(b_global.first, 0);
+    header_odd.load(b_global.first, min(1, last_block));
+    b0.load(b_global, 0, 0, b_part);
+    if constexpr (kHalfBlocks<ENC>) {
+        b1.load(b_global, 0, 2, b_part);
+    } else {
+        b1.load(b_global, 0, 1, b_part);
+        b2.load(b_global, 0, 2, b_part);
+        b3.load(b_global, 0, 3, b_part);
+    }
     a_now.r0k0 = NFN_LOAD_ACTIVATIONS(a_global, 0, 0);
     a_now.r0k1 = NFN_LOAD_ACTIVATIONS(a_global, 0, 1);
     a_now.r0k2 = NFN_LOAD_ACTIVATIONS(a_global, 0, 2);
@@ -608,7 +629,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     }
     {
         std::uint32_t wa[4][2], wb[4][2];
-        b0.prepare_bits(header_even, 0, b_half);
+        b0.prepare_bits(header_even, 0, b_part);
         b0.prepare_scales(header_even);
         b0.template group_a<0>(wa[0]);
         b0.template group_a<1>(wa[1]);
@@ -621,10 +642,10 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
         std::uint8_t* target = lds + b_target;
         NFN_WRITE16(target, wa[0][0], wa[0][1], wa[1][0], wa[1][1]);
         NFN_WRITE16(target + 16, wa[2][0], wa[2][1], wa[3][0], wa[3][1]);
-        NFN_WRITE16(target + 64, wb[0][0], wb[0][1], wb[1][0], wb[1][1]);
-        NFN_WRITE16(target + 80, wb[2][0], wb[2][1], wb[3][0], wb[3][1]);
+        NFN_WRITE16(target + kSecondRun<ENC>, wb[0][0], wb[0][1], wb[1][0], wb[1][1]);
+        NFN_WRITE16(target + kSecondRun<ENC> + 16, wb[2][0], wb[2][1], wb[3][0], wb[3][1]);
     }
-    b0.load(b_global, min(1, last_block), 0, b_half);  // step 4, or step 0 again
+    if constexpr (!kHalfBlocks<ENC>) b0.load(b_global, min(1, last_block), 0, b_part);  // step 4, or step 0 again
     __syncthreads();
 
     const int operand = (lane & 31) * kRowBytes + (lane >> 5) * 16;
@@ -650,15 +671,20 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     // step s+5 and the activation slice step s+1.  `now` holds the scales of
     // this block, `next` those of the following one (needed by the fourth step,
     // which decodes the first step of that block).
+    // (Q6_K: b0 holds a block's first half, which the first and, of the next block, the fourth step
+    // decode, b1 the second.)
     auto block_of_four = [&](int step, const BlockHeader<ENC>& now, const BlockHeader<ENC>& next) {
-        k_step<ENC, RB>(acc, a_now, current, b_read0, b_read1, b_write1, b1, now, 1, b_half,
-                    activations_of(step + 1), row_block_bytes, b_global, min(step + 5, last));
-        k_step<ENC, RB>(acc, a_now, current, b_read1, b_read0, b_write0, b2, now, 2, b_half,
-                    activations_of(step + 2), row_block_bytes, b_global, min(step + 6, last));
-        k_step<ENC, RB>(acc, a_now, current, b_read0, b_read1, b_write1, b3, now, 3, b_half,
-                    activations_of(step + 3), row_block_bytes, b_global, min(step + 7, last));
-        k_step<ENC, RB>(acc, a_now, current, b_read1, b_read0, b_write0, b0, next, 0, b_half,
-                    activations_of(step + 4), row_block_bytes, b_global, min(step + 8, last));
+        constexpr bool kHalves = kHalfBlocks<ENC>;
+        constexpr int kAhead = kHalves ? 3 : 4;  // from the step that is decoded to the one that is fetched
+        PackedSlice<ENC>&second = kHalves ? b0 : b1, &third = kHalves ? b1 : b2, &fourth = kHalves ? b1 : b3;
+        k_step<ENC, RB, true>(acc, a_now, current, b_read0, b_read1, b_write1, second, now, 1, b_part,
+                    activations_of(step + 1), row_block_bytes, b_global, min(step + 1 + kAhead, last));
+        k_step<ENC, RB, !kHalves>(acc, a_now, current, b_read1, b_read0, b_write0, third, now, 2, b_part,
+                    activations_of(step + 2), row_block_bytes, b_global, min(step + 2 + kAhead, last));
+        k_step<ENC, RB, true>(acc, a_now, current, b_read0, b_read1, b_write1, fourth, now, 3, b_part,
+                    activations_of(step + 3), row_block_bytes, b_global, min(step + 3 + kAhead, last));
+        k_step<ENC, RB, !kHalves>(acc, a_now, current, b_read1, b_read0, b_write0, b0, next, 0, b_part,
+                    activations_of(step + 4), row_block_bytes, b_global, min(step + 4 + kAhead, last));
     };
     // The two header register sets swap roles every block; the loop body is two
     // blocks so that no copy (and no wait for the load that feeds it) is needed.
@@ -668,7 +694,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     int block = 0;
     if ((last_block & 1) == 0) {
         block_of_four(0, header_even, header_odd);
-        header_even.load(b_global, min(2, last_block));
+        header_even.load(b_global.first, min(2, last_block));
         NFN_FENCE();
         const BlockHeader<ENC> second = header_odd;
         header_odd = header_even;
@@ -677,10 +703,10 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     }
     while (block < last_block) {
         block_of_four(block * 4, header_even, header_odd);
-        header_even.load(b_global, min(block + 2, last_block));
+        header_even.load(b_global.first, min(block + 2, last_block));
         NFN_FENCE();
         block_of_four(block * 4 + 4, header_odd, header_even);
-        header_odd.load(b_global, min(block + 3, last_block));
+        header_odd.load(b_global.first, min(block + 3, last_block));
         NFN_FENCE();
         block += 2;
     }
