@@ -930,7 +930,11 @@ int nfn_mi355_k_quant_gemm_plan_v1(
  * every projection runs from that copy.  All descriptors share input_dim (a
  * multiple of 256) and are Q4_K, Q5_K, Q6_K or Q8_0.  The workspace is the
  * largest of the single-projection sizes (the query above with each
- * output_dim).  Results are those of the single-projection call, bit for bit. */
+ * output_dim); with the size that the query below gives, the projections of an
+ * encoding run in one launch where they all split K.  Results are those of the
+ * single-projection call, bit for bit, with either. */
+int64_t nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1(
+    int64_t rows, int64_t input_dim, const int64_t* output_dims, int64_t operation_count, int mode);
 int nfn_mi355_k_quant_gemm_multi_float32_v1(
     const NfnNativeTilePackedWeightDescriptorV1* const* descriptors,
     const float* input,

@@ -880,7 +880,7 @@ int nfn_mi355_k_quant_gemm_float32_v1(const Descriptor* descriptor, const float*
     if (required == 0 || workspace_nbytes < required) return kInvalid;
     if (gemm_f16_supports(normalized.encoding, normalized.input_dim)) {
         if (reinterpret_cast<std::uintptr_t>(workspace) % 16 != 0) return kInvalid;
-        launch_gemm_f16(normalized, input, output, rows, workspace, as_stream(cuda_stream));
+        launch_gemm_f16(&normalized, 1, input, &output, rows, workspace, workspace_nbytes, as_stream(cuda_stream));
         return launch_status();
     }
     ProjectionSet set{};
@@ -895,6 +895,19 @@ int nfn_mi355_k_quant_gemm_float32_v1(const Descriptor* descriptor, const float*
                         as_stream(cuda_stream));
     }
     return launch_status();
+}
+
+std::int64_t nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1(std::int64_t rows, std::int64_t input_dim,
+                                                             const std::int64_t* output_dims,
+                                                             std::int64_t operation_count, int mode) {
+    if (rows <= 0 || input_dim <= 0 || input_dim % 256 != 0 || output_dims == nullptr || operation_count < 1 ||
+        operation_count > kMaxOperations || mode != NFN_MI355_GEMM_F16) {
+        return 0;
+    }
+    for (std::int64_t index = 0; index < operation_count; ++index) {
+        if (output_dims[index] <= 0) return 0;
+    }
+    return gemm_f16_multi_workspace_bytes(rows, input_dim, output_dims, static_cast<int>(operation_count));
 }
 
 int nfn_mi355_k_quant_gemm_multi_float32_v1(const Descriptor* const* descriptors, const float* input,
@@ -924,11 +937,8 @@ int nfn_mi355_k_quant_gemm_multi_float32_v1(const Descriptor* const* descriptors
         if (bytes > required) required = bytes;
     }
     if (workspace_nbytes < required) return kInvalid;
-    const hipStream_t stream = as_stream(cuda_stream);
-    convert_gemm_activations(input, rows, normalized[0].input_dim, workspace, stream);
-    for (std::int64_t index = 0; index < operation_count; ++index) {
-        launch_gemm_f16_converted(normalized[index], outputs[index], rows, workspace, stream);
-    }
+    launch_gemm_f16(normalized, static_cast<int>(operation_count), input, outputs, rows, workspace, workspace_nbytes,
+                    as_stream(cuda_stream));
     return launch_status();
 }
 

@@ -51,6 +51,7 @@ constexpr int kBM = 256;
 constexpr int kBN = 128;
 constexpr int kBK = 64;
 constexpr int kThreads = 256;
+constexpr int kMaxProjections = 4;  // of one call
 constexpr int kMaxShares = 4;  // K shares of a split launch at most
 constexpr int kRowBytes = 144;  // 64 fp16 + 16 bytes of padding
 constexpr int kStageBytes = kBN * kRowBytes;
@@ -541,31 +542,62 @@ constexpr int kBlockBytes = ENC == kEncQ4K ? 144 : ENC == kEncQ5K ? 176 : ENC ==
 template <std::uint32_t ENC, int RB>
 constexpr int kWavesPerSimd = ENC == kEncQ6K ? RB == 1 ? 2 : 1 : RB == 1 && ENC == kEncQ4K ? 3 : 2;
 
+// The projections of one launch: one encoding, one input.  Workgroup numbers run through the
+// projections, inside each through its K shares, inside each through its tiles.
+struct GemmGroup {
+    const std::uint8_t* weights[kMaxProjections];
+    float* output[kMaxProjections];    // share 0
+    float* partials[kMaxProjections];  // the other shares, one copy of the output each
+    std::int64_t output_dim[kMaxProjections];
+    std::int64_t row_stride;
+    int first[kMaxProjections];   // workgroup number (past the end for slots without a projection)
+    int tiles[kMaxProjections];
+    int shares[kMaxProjections];
+};
+
 // RB: 32-row blocks per wave; the workgroup's tile is 128*RB rows by 128 columns.
 template <std::uint32_t ENC, int RB>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB>))) void gemm_f16_kernel(
-    const std::uint8_t* __restrict__ weights, std::int64_t row_stride, std::int64_t output_dim,
-    std::int64_t input_dim, const std::uint8_t* __restrict__ activations,
-    const float* __restrict__ inverse_scale, float* __restrict__ output, std::int64_t rows,
-    int m_tiles, std::int64_t split_stride) {
+    const std::uint8_t* __restrict__ activations, const float* __restrict__ inverse_scale, std::int64_t input_dim,
+    std::int64_t rows, int m_tiles, GemmGroup group) {
     extern __shared__ __attribute__((aligned(16))) std::uint8_t lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // rows 64*wave .. +63 of the tile
-    const int m_tile = blockIdx.x % m_tiles;
-    const int n_tile = blockIdx.x / m_tiles;
+    const std::uint8_t* weights = group.weights[0];
+    float* output = group.output[0];
+    float* partials = group.partials[0];
+    std::int64_t output_dim = group.output_dim[0];
+    int first = 0, tiles = group.tiles[0], shares = group.shares[0];
+#pragma unroll
+    for (int i = 1; i < kMaxProjections; ++i) {
+        if (static_cast<int>(blockIdx.x) >= group.first[i]) {
+            weights = group.weights[i];
+            output = group.output[i];
+            partials = group.partials[i];
+            output_dim = group.output_dim[i];
+            first = group.first[i];
+            tiles = group.tiles[i];
+            shares = group.shares[i];
+        }
+    }
+    const int share = (static_cast<int>(blockIdx.x) - first) / tiles;
+    const int tile = (static_cast<int>(blockIdx.x) - first) % tiles;
+    const int m_tile = tile % m_tiles;
+    const int n_tile = tile / m_tiles;
     constexpr int kTileRows = 128 * RB;
     const std::int64_t m0 = static_cast<std::int64_t>(m_tile) * kTileRows;
     const std::int64_t n0 = static_cast<std::int64_t>(n_tile) * kBN;
-    // blockIdx.y: which share of the K dimension (whole 256-value blocks) this
-    // workgroup sums; each share writes its own copy of the output
+    // which share of the K dimension (whole 256-value blocks) this workgroup sums; each share
+    // writes its own copy of the output
     const int total_blocks = static_cast<int>(input_dim >> 8);
-    const int first_block = total_blocks * static_cast<int>(blockIdx.y) / static_cast<int>(gridDim.y);
-    const int end_block = total_blocks * (static_cast<int>(blockIdx.y) + 1) / static_cast<int>(gridDim.y);
+    const int first_block = total_blocks * share / shares;
+    const int end_block = total_blocks * (share + 1) / shares;
     const int steps = (end_block - first_block) * 4;  // a positive multiple of 4
     const int last = steps - 1;
-    output += blockIdx.y * split_stride;
+    const std::int64_t row_stride = group.row_stride;
+    if (share > 0) output = partials + (share - 1) * rows * output_dim;
 
     // activations: fragment (row block, K chunk) is 1 KB, a row block's chunks are consecutive
     const std::int64_t row_block_bytes = (input_dim / 16) * kFragmentBytes;
@@ -743,15 +775,33 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     }
 }
 
-// Sum of the K shares: output[i] = partial[0][i] + partial[1][i] + ..., in that order.
-__global__ __launch_bounds__(256) void sum_shares_kernel(const float* __restrict__ partials,
-                                                         float* __restrict__ output,
-                                                         std::int64_t count, int shares) {
+// Sum of the K shares: output[i] = share 0 (in place) + share 1 + ..., in that order;
+// blockIdx.y: the projection.
+struct ShareSums {
+    float* output[kMaxProjections];
+    const float* partials[kMaxProjections];
+    std::int64_t count[kMaxProjections];
+    int shares[kMaxProjections];
+};
+__global__ __launch_bounds__(256) void sum_shares_kernel(ShareSums sums) {
+    float* output = sums.output[0];
+    const float* partials = sums.partials[0];
+    std::int64_t count = sums.count[0];
+    int shares = sums.shares[0];
+#pragma unroll
+    for (int i = 1; i < kMaxProjections; ++i) {
+        if (static_cast<int>(blockIdx.y) == i) {
+            output = sums.output[i];
+            partials = sums.partials[i];
+            count = sums.count[i];
+            shares = sums.shares[i];
+        }
+    }
     const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
     for (std::int64_t index = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
          index < count; index += stride) {
-        float total = partials[index];
-        for (int share = 1; share < shares; ++share) total += partials[share * count + index];
+        float total = output[index];
+        for (int share = 1; share < shares; ++share) total += partials[(share - 1) * count + index];
         output[index] = total;
     }
 }
@@ -763,9 +813,15 @@ __global__ __launch_bounds__(256) void sum_shares_kernel(const float* __restrict
 // four shares) until the grid fills the units' two (256-row tiles) or three
 // (128-row tiles) workgroup slots; the shares are summed by a second launch in
 // a fixed order.  256-row tiles stay the better choice as long as two shares or
-// more fit; at most 128 rows, or a K too short to split, take 128-row tiles.
+// more fit; at most 128 rows take 128-row tiles.
 // Narrow projections (an eighth of the units' count in 256-row tiles at most) take
 // 128-row tiles and shares of six blocks or more.
+// A K too short to split takes 256-row tiles from half a workgroup a unit on: 4,096 -> 6,656, 700
+// rows (156 tiles) 82 -> 75 us for Q5_K and 94 -> 79 for Q6_K, 1,024 rows 87 -> 75; 512 rows (104
+// tiles) would lose, 56 -> 62.
+// The projections of one call run in one launch an encoding, each with the shares that it has by
+// itself, so that few workgroups of one do not wait for those of another: 17 rows into Q, K, V and
+// the gate of width 6,656 took 107 us (Q5_K) one after another and take 44, 333 rows 170 and 84.
 struct Plan {
     int row_blocks;  // 32-row blocks per wave: 2 = 256-row tiles, 1 = 128-row tiles
     int shares;
@@ -796,6 +852,7 @@ Plan plan(std::uint32_t encoding, std::int64_t rows, std::int64_t output_dim,
         std::int64_t shares = 2 * units / tall_tiles;
         if (shares > longest) shares = longest;
         if (shares >= 2) return Plan{2, static_cast<int>(shares)};
+        if (2 * tall_tiles >= units) return Plan{2, 1};
     }
     const std::int64_t tiles = (rows + 127) / 128 * n_tiles;
     std::int64_t shares = units * (encoding == kEncQ6K ? 2 : 3) / tiles;
@@ -804,36 +861,46 @@ Plan plan(std::uint32_t encoding, std::int64_t rows, std::int64_t output_dim,
     return Plan{1, static_cast<int>(shares)};
 }
 
-template <std::uint32_t ENC>
-void launch_encoding(const Descriptor& descriptor, const std::uint8_t* activations,
-                     const float* inverse_scale, float* output, float* partials,
-                     std::int64_t rows, hipStream_t stream) {
-    const std::int64_t n_tiles = (descriptor.output_dim + kBN - 1) / kBN;
-    const Plan chosen = plan(ENC, rows, descriptor.output_dim, descriptor.input_dim);
-    const std::int64_t count = rows * descriptor.output_dim;
-    float* target = chosen.shares > 1 ? partials : output;
-    const std::int64_t split_stride = chosen.shares > 1 ? count : 0;
-    if (chosen.row_blocks == 2) {
-        const int m_tiles = static_cast<int>((rows + 255) / 256);
-        hipLaunchKernelGGL((gemm_f16_kernel<ENC, 2>),
-                           dim3(static_cast<unsigned>(m_tiles * n_tiles), chosen.shares),
-                           dim3(kThreads), 2 * kStageBytes, stream, descriptor.data,
-                           descriptor.row_stride_bytes, descriptor.output_dim,
-                           descriptor.input_dim, activations, inverse_scale, target, rows, m_tiles,
-                           split_stride);
-    } else {
-        const int m_tiles = static_cast<int>((rows + 127) / 128);
-        hipLaunchKernelGGL((gemm_f16_kernel<ENC, 1>),
-                           dim3(static_cast<unsigned>(m_tiles * n_tiles), chosen.shares),
-                           dim3(kThreads), 2 * kStageBytes, stream, descriptor.data,
-                           descriptor.row_stride_bytes, descriptor.output_dim,
-                           descriptor.input_dim, activations, inverse_scale, target, rows, m_tiles,
-                           split_stride);
+template <std::uint32_t ENC, int RB>
+void launch_tiles(GemmGroup group, int count, const std::uint8_t* activations, const float* inverse_scale,
+                  std::int64_t rows, std::int64_t input_dim, hipStream_t stream) {
+    const int m_tiles = static_cast<int>((rows + 128 * RB - 1) / (128 * RB));
+    int workgroups = 0;
+    for (int i = 0; i < kMaxProjections; ++i) {
+        group.first[i] = i < count ? workgroups : 0x7fffffff;
+        if (i >= count) continue;
+        group.tiles[i] = m_tiles * static_cast<int>((group.output_dim[i] + kBN - 1) / kBN);
+        workgroups += group.tiles[i] * group.shares[i];
     }
-    if (chosen.shares > 1) {
-        const std::int64_t blocks = (count + 1023) / 1024;
-        hipLaunchKernelGGL(sum_shares_kernel, dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)),
-                           dim3(256), 0, stream, partials, output, count, chosen.shares);
+    hipLaunchKernelGGL((gemm_f16_kernel<ENC, RB>), dim3(static_cast<unsigned>(workgroups)), dim3(kThreads),
+                       2 * kStageBytes, stream, activations, inverse_scale, input_dim, rows, m_tiles, group);
+}
+
+// One launch for `count` projections of one encoding and, if any of them splits K, one for the sums.
+template <std::uint32_t ENC>
+void launch_group(const GemmGroup& group, int count, bool tall, const std::uint8_t* activations,
+                  const float* inverse_scale, std::int64_t rows, std::int64_t input_dim, hipStream_t stream) {
+    if (tall) {
+        launch_tiles<ENC, 2>(group, count, activations, inverse_scale, rows, input_dim, stream);
+    } else {
+        launch_tiles<ENC, 1>(group, count, activations, inverse_scale, rows, input_dim, stream);
+    }
+    ShareSums sums{};
+    int split = 0;
+    std::int64_t most = 0;
+    for (int i = 0; i < count; ++i) {
+        if (group.shares[i] == 1) continue;
+        sums.output[split] = group.output[i];
+        sums.partials[split] = group.partials[i];
+        sums.count[split] = rows * group.output_dim[i];
+        sums.shares[split] = group.shares[i];
+        if (sums.count[split] > most) most = sums.count[split];
+        ++split;
+    }
+    if (split > 0) {
+        const std::int64_t blocks = (most + 1023) / 1024;
+        hipLaunchKernelGGL(sum_shares_kernel, dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096), split),
+                           dim3(256), 0, stream, sums);
     }
 }
 
@@ -888,36 +955,67 @@ void convert_gemm_activations(const float* input, std::int64_t rows, std::int64_
     }
 }
 
-void launch_gemm_f16(const Descriptor& descriptor, const float* input, float* output,
-                     std::int64_t rows, void* workspace, hipStream_t stream) {
-    convert_gemm_activations(input, rows, descriptor.input_dim, workspace, stream);
-    launch_gemm_f16_converted(descriptor, output, rows, workspace, stream);
+// floats of a projection's shares behind the first
+static std::int64_t partial_floats(const Plan& chosen, std::int64_t rows, std::int64_t output_dim) {
+    return (chosen.shares - 1) * rows * output_dim;
 }
 
-void launch_gemm_f16_converted(const Descriptor& descriptor, float* output, std::int64_t rows,
-                               void* workspace, hipStream_t stream) {
-    std::uint8_t* activations = static_cast<std::uint8_t*>(workspace);
-    float* inverse_scale =
-        reinterpret_cast<float*>(activations + padded_rows(rows) * descriptor.input_dim * 2);
-    float* partials =
-        reinterpret_cast<float*>(activations + activation_bytes(rows, descriptor.input_dim));
-    switch (descriptor.encoding) {
-        case kEncQ4K:
-            launch_encoding<kEncQ4K>(descriptor, activations, inverse_scale, output, partials, rows,
-                                     stream);
-            break;
-        case kEncQ5K:
-            launch_encoding<kEncQ5K>(descriptor, activations, inverse_scale, output, partials, rows,
-                                     stream);
-            break;
-        case kEncQ6K:
-            launch_encoding<kEncQ6K>(descriptor, activations, inverse_scale, output, partials, rows,
-                                     stream);
-            break;
-        default:
-            launch_encoding<kEncQ8_0>(descriptor, activations, inverse_scale, output, partials, rows,
-                                     stream);
-            break;
+std::int64_t gemm_f16_multi_workspace_bytes(std::int64_t rows, std::int64_t input_dim, const std::int64_t* output_dims,
+                                            int count) {
+    std::int64_t largest = 0, floats = 0;
+    for (int i = 0; i < count; ++i) {
+        const std::int64_t single = gemm_f16_workspace_bytes(rows, input_dim, output_dims[i]);
+        if (single > largest) largest = single;
+        floats += partial_floats(plan(kEncQ4K, rows, output_dims[i], input_dim), rows, output_dims[i]);
+    }
+    const std::int64_t together = activation_bytes(rows, input_dim) + 4 * floats + 256;
+    return together > largest ? together : largest;
+}
+
+void launch_gemm_f16(const Descriptor* descriptors, int count, const float* input, float* const* outputs,
+                     std::int64_t rows, void* workspace, std::int64_t workspace_bytes, hipStream_t stream) {
+    const std::int64_t input_dim = descriptors[0].input_dim;
+    convert_gemm_activations(input, rows, input_dim, workspace, stream);
+    const std::uint8_t* activations = static_cast<const std::uint8_t*>(workspace);
+    const float* inverse_scale = reinterpret_cast<const float*>(activations + padded_rows(rows) * input_dim * 2);
+    float* partials = reinterpret_cast<float*>(static_cast<std::uint8_t*>(workspace) + activation_bytes(rows, input_dim));
+    const std::int64_t room = (workspace_bytes - activation_bytes(rows, input_dim)) / 4;
+    bool done[kMaxProjections] = {};
+    for (int start = 0; start < count; ++start) {
+        if (done[start]) continue;
+        // this projection and those of its encoding whose partial outputs find room beside its own
+        GemmGroup group{};
+        int members = 0;
+        std::int64_t used = 0, short_groups = 0;
+        bool tall = false;
+        for (int i = start; i < count; ++i) {
+            if (done[i] || descriptors[i].encoding != descriptors[start].encoding) continue;
+            const Plan chosen = plan(descriptors[i].encoding, rows, descriptors[i].output_dim, input_dim);
+            const std::int64_t floats = partial_floats(chosen, rows, descriptors[i].output_dim);
+            if (i != start && used + floats > room) continue;
+            done[i] = true;
+            group.weights[members] = descriptors[i].data;
+            group.row_stride = descriptors[i].row_stride_bytes;
+            group.output[members] = outputs[i];
+            group.partials[members] = partials + used;
+            group.output_dim[members] = descriptors[i].output_dim;
+            group.shares[members] = chosen.shares;
+            used += floats;
+            short_groups += (rows + 127) / 128 * ((descriptors[i].output_dim + kBN - 1) / kBN) * chosen.shares;
+            if (chosen.row_blocks == 2) tall = true;
+            ++members;
+        }
+        // 256-row tiles where a member would take them by itself, unless 128-row tiles leave half
+        // of the last one's rows out and all fit the units at two a unit (333 rows into Q, K, V and
+        // the gate of width 6,656: 84 us instead of 102 for Q5_K, 78 instead of 98 for Q4_K)
+        const bool odd = (rows + 127) / 128 % 2 != 0;
+        if (members > 1 && odd && short_groups <= 2 * compute_units()) tall = false;
+        switch (descriptors[start].encoding) {
+            case kEncQ4K: launch_group<kEncQ4K>(group, members, tall, activations, inverse_scale, rows, input_dim, stream); break;
+            case kEncQ5K: launch_group<kEncQ5K>(group, members, tall, activations, inverse_scale, rows, input_dim, stream); break;
+            case kEncQ6K: launch_group<kEncQ6K>(group, members, tall, activations, inverse_scale, rows, input_dim, stream); break;
+            default: launch_group<kEncQ8_0>(group, members, tall, activations, inverse_scale, rows, input_dim, stream); break;
+        }
     }
 }
 

@@ -17,15 +17,13 @@ bool gemm_f16_supports(std::uint32_t encoding, std::int64_t input_dim);
 // unsplit; more = one partial output per share, summed by a second launch).
 void gemm_f16_plan(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
                    std::int64_t output_dim, int* tile_rows, int* k_shares);
-// output[rows, output_dim] = input[rows, input_dim] * W^T, float accumulation.
-void launch_gemm_f16(const Descriptor& descriptor, const float* input, float* output,
-                      std::int64_t rows, void* workspace, hipStream_t stream);
-// The same in two steps, for several projections of one input: the activations
-// go to the workspace once, then each projection runs from there (the split-K
-// partial buffer behind them is reused; the launches are stream-ordered).
-void convert_gemm_activations(const float* input, std::int64_t rows, std::int64_t input_dim,
-                              void* workspace, hipStream_t stream);
-void launch_gemm_f16_converted(const Descriptor& descriptor, float* output, std::int64_t rows,
-                               void* workspace, hipStream_t stream);
+// What 1..4 projections of one input need to run in one launch an encoding; with the largest of
+// the single sizes they still run, in as many launches as it takes.
+std::int64_t gemm_f16_multi_workspace_bytes(std::int64_t rows, std::int64_t input_dim, const std::int64_t* output_dims,
+                                            int count);
+// outputs[i][rows, output_dim] = input[rows, input_dim] * W_i^T, float accumulation, for 1..4
+// projections of one input width: the input is converted once.
+void launch_gemm_f16(const Descriptor* descriptors, int count, const float* input, float* const* outputs,
+                     std::int64_t rows, void* workspace, std::int64_t workspace_bytes, hipStream_t stream);
 
 }  // namespace nfn

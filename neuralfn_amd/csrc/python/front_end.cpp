@@ -51,6 +51,7 @@ struct Raised {};
     X(nfn_mi355_lm_head_argmax_workspace_bytes_v1)                            \
     X(nfn_mi355_lm_head_argmax_v1)                                            \
     X(nfn_mi355_k_quant_gemm_workspace_bytes_v1)                              \
+    X(nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1)                        \
     X(nfn_mi355_k_quant_gemm_float32_v1)                                      \
     X(nfn_mi355_k_quant_gemm_multi_float32_v1)                                \
     X(nfn_native_tile_glimmer_qk_norm_scale_rope_float32_v1)                  \
@@ -474,11 +475,10 @@ PyObject* lm_head_argmax(Arguments a) {
 at::Tensor gemm_workspace(PyObject* given, const Descriptor* descriptors, std::int64_t count, std::int64_t rows,
                           int mode, c10::Device device) {
     if (given != Py_None) return tensor_of(given);
-    std::int64_t nbytes = 0;
-    for (std::int64_t i = 0; i < count; ++i) {
-        nbytes = std::max(nbytes, lib.nfn_mi355_k_quant_gemm_workspace_bytes_v1(
-            rows, descriptors[i].input_dim, descriptors[i].output_dim, mode));
-    }
+    c10::SmallVector<std::int64_t, 4> widths;
+    for (std::int64_t i = 0; i < count; ++i) widths.push_back(descriptors[i].output_dim);
+    const std::int64_t nbytes = count == 0 ? 0 : lib.nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1(
+        rows, descriptors[0].input_dim, widths.data(), count, mode);
     if (nbytes <= 0) raise(PyExc_ValueError, "unsupported GEMM geometry or mode");
     return new_bytes(nbytes, device);
 }

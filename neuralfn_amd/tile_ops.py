@@ -204,6 +204,7 @@ SIGNATURES = {
     "nfn_mi355_lm_head_argmax_v1": (ctypes.c_int, [_DESC, _P, _P, _P, _I64, _P, _I64, _P]),
     "nfn_mi355_lm_head_argmax_no_alloc_v1": (ctypes.c_int, [_DESC, _P, _P, _P, _I64, _P]),
     "nfn_mi355_k_quant_gemm_workspace_bytes_v1": (_I64, [_I64, _I64, _I64, ctypes.c_int]),
+    "nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1": (_I64, [_I64, _I64, _P, _I64, ctypes.c_int]),
     "nfn_mi355_k_quant_gemm_plan_v1": (
         ctypes.c_int, [ctypes.c_uint32, _I64, _I64, _I64, ctypes.c_int, _P, _P]),
     "nfn_mi355_k_quant_gemm_float32_v1": (

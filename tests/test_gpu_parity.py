@@ -1516,6 +1516,9 @@ def test_prefill_gemm_plans():
     assert tile_ops.gemm_plan(kquant.Q4_K, 200, 9216, wide) == (256, 3)
     assert tile_ops.gemm_plan(kquant.Q4_K, 200, 12544, wide) == (256, 4)
     assert tile_ops.gemm_plan(kquant.Q4_K, 2048, 6656, 16384) == (256, 1)
+    # A K too short for shares: 256-row tiles from half a workgroup a unit on.
+    assert tile_ops.gemm_plan(kquant.Q4_K, 512, 4096, 6656) == (128, 1)
+    assert tile_ops.gemm_plan(kquant.Q4_K, 700, 4096, 6656) == (256, 1)
     # A narrow projection (the K and V projections of the workload): small tiles, short shares.
     assert tile_ops.gemm_plan(kquant.Q4_K, 1024, 6656, 256) == (128, 4)
     assert tile_ops.gemm_plan(kquant.Q6_K, 2048, 6656, 256) == (128, 4)
@@ -1572,6 +1575,35 @@ def test_prefill_gemm_multi_equals_single_calls(cuda, oracle):
         kquant.Q4_K, kquant.quantize(kquant.Q4_K, kquant.synthetic_weights(72, 64, 512)), 64, 512)
     assert call(descs=descriptors[:3] + [other.descriptor(0)]) == 1  # another input width
     torch_().cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows", [17, 200, 300, 640])
+@pytest.mark.parametrize("specs", [
+    [(kquant.Q4_K, 4096), (kquant.Q4_K, 256), (kquant.Q4_K, 130), (kquant.Q4_K, 4000)],  # one launch
+    [(kquant.Q6_K, 1000), (kquant.Q8_0, 300), (kquant.Q6_K, 17), (kquant.Q8_0, 2048)],   # two, interleaved
+    [(kquant.Q5_K, 5000), (kquant.Q5_K, 129)],
+])
+def test_prefill_gemm_multi_launches_equal_single_calls(cuda, specs, rows):
+    """Projections of one encoding in one launch, each with its own K shares: the single call's bits,
+    with the workspace for one launch and with the smallest allowed (more launches); nothing is
+    written behind either."""
+    in_dim = 6656
+    weights = [tile_ops.PackedWeight.from_numpy(e, random_packed(e, n, in_dim, 80 + i), n, in_dim)
+               for i, (e, n) in enumerate(specs)]
+    x = to_device(kquant.synthetic_activations(81, rows, in_dim), cuda)
+    expected = [tile_ops.gemm(weight, x) for weight in weights]
+    lib = tile_ops.load()
+    widths = np.array([n for _, n in specs], dtype=np.int64)
+    together = lib.nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1(
+        rows, in_dim, widths.ctypes.data, len(specs), tile_ops.GEMM_F16)
+    least = max(lib.nfn_mi355_k_quant_gemm_workspace_bytes_v1(rows, in_dim, n, tile_ops.GEMM_F16) for _, n in specs)
+    assert together >= least
+    for nbytes in (together, least):
+        workspace = torch_().full((nbytes + 4096,), 0x5a, dtype=torch_().uint8, device=cuda)
+        for weight, y, single in zip(weights, tile_ops.gemm_multi(weights, x, workspace=workspace[:nbytes]), expected):
+            assert_bits_equal(y, single, kquant.NAMES[weight.encoding])
+        assert bool((workspace[nbytes:] == 0x5a).all())
+    assert lib.nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1(rows, in_dim, widths.ctypes.data, 5, tile_ops.GEMM_F16) == 0
 
 
 @pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q6_K])
