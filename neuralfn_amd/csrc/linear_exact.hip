@@ -27,7 +27,7 @@
 // instead of one, and the matrix instructions of a step before its other work instead of between it,
 // made no difference.)  Measured at 4,096 -> 6,656, against the vector kernel (16 rows) and the
 // float matrix instruction (200, 512 rows) before: Q4_K 134 -> 16 us at 16 rows, 203 -> 69 at 200,
-// 311 -> 135 at 512; Q8_0 368 -> 29, 180 -> 90, 279 -> 178; F32 406 -> 30, 172 -> 131, 271 -> 254.
+// 311 -> 135 at 512; Q8_0 368 -> 27, 180 -> 87, 279 -> 169; F32 406 -> 30, 172 -> 131, 271 -> 254.
 //
 // The entry point, nfn_native_tile_linear_packed_weight_float32_v1, has no workspace argument
 // (neuralfn/csrc/native_train/tile_ops.h:614-620; reference kernel
@@ -47,7 +47,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef std::uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef std::uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef std::uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-typedef std::uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 
 __device__ __forceinline__ bf16x8 as_bf16(u32x4 words) { return __builtin_bit_cast(bf16x8, words); }
 
@@ -105,9 +104,22 @@ __device__ __forceinline__ void codes_to_bf16(std::uint32_t bytes, float offset,
 // (half = lane / 32, chunk = 0 or 1, j = 0..7); the matrix instruction does not care which
 // column carries which k index as long as both operands agree, and 16 neighbouring code bytes
 // are one load.  Q6_K has a scale per 16 columns, which a chunk's instructions must not mix.
-//   load(row, unit, half); words(step, chunk, word, ..): four codes as bf16; scale(step, chunk);
-//   minimum(step): d_min * m
+//   load(row, unit, half); arrange(), once, when the bytes are there; words(step, chunk, word, ..):
+//   four codes as bf16; scale(step, chunk); minimum(step): d_min * m
+// Every load looks up a cache line for each of its lanes, however few bytes it brings, and those
+// look-ups bound the kernels: the two lanes of a row (half 0 and 1, 32 lanes apart) therefore
+// fetch different pieces, 16 bytes wherever a piece has them, and trade words in arrange().  Q6_K
+// takes four loads a unit instead of nine, Q8_0 three instead of four: 4,096 -> 6,656 at 16 / 200 /
+// 512 rows 24.2 / 112 / 223 -> 21.6 / 107 / 211 us for Q6_K, 28.9 / 92 / 179 -> 26.8 / 87 / 169 for Q8_0.
 // -----------------------------------------------------------------------------------------------
+// first: the lower 32 lanes' `a` and `b` (in the lower and the upper lanes), second: the upper lanes'
+struct Traded {
+    std::uint32_t first, second;
+};
+__device__ __forceinline__ Traded trade(std::uint32_t a, std::uint32_t b) {
+    const auto both = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    return Traded{both[0], both[1]};
+}
 template <std::uint32_t ENC>
 struct Unit;
 
@@ -123,6 +135,7 @@ struct UnitOfQ4KOrQ5K {
         codes = *reinterpret_cast<const u32x4_a4*>(block + (ENC == kEncQ5K ? 48 : 16) + group * 32 + half * 16);
         if constexpr (ENC == kEncQ5K) fifth = *reinterpret_cast<const u32x4_a4*>(block + 16 + half * 16);
     }
+    __device__ __forceinline__ void arrange() {}
     __device__ __forceinline__ void words(int step, int chunk, int word, std::uint32_t& low, std::uint32_t& high) const {
         std::uint32_t q = (codes[2 * chunk + word] >> (4 * step)) & 0x0f0f0f0fu;
         if constexpr (ENC == kEncQ5K) {
@@ -152,33 +165,47 @@ struct Unit<kEncQ5K> : UnitOfQ4KOrQ5K<kEncQ5K> {};
 template <>
 struct Unit<kEncQ6K> {
     static constexpr bool kWide = false, kScaled = true, kMinimum = false, kScalePerChunk = true;
-    u32x2_a2 low[2][2], high[2];  // [step][chunk], [chunk]
-    std::uint32_t scales;         // the unit's four sub-scales, (step, chunk) at byte 2 step + chunk
-    std::uint32_t d;
+    // as loaded: the 16 columns of chunk `half`; arranged: words 0 and 1 the lane's columns of
+    // chunk 0, words 2 and 3 those of chunk 1
+    u32x4_a2 low[2], high;  // low: [step]
+    std::uint32_t scales;   // the unit's four sub-scales, (step, chunk) at byte 2 step + chunk
+    std::uint32_t d;        // in the upper half
     int upper;
     __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half) {
+        typedef std::uint32_t u32_a2 __attribute__((aligned(2)));
         const std::uint8_t* block = row + (unit >> 2) * 210;
         const int half_block = (unit >> 1) & 1;
         upper = unit & 1;  // quarters 2 and 3 of the half block: high nibbles, high-bit pairs 2 and 3
+        low[0] = *reinterpret_cast<const u32x4_a2*>(block + half_block * 64 + 16 * half);
+        low[1] = *reinterpret_cast<const u32x4_a2*>(block + half_block * 64 + 32 + 16 * half);
+        high = *reinterpret_cast<const u32x4_a2*>(block + 128 + half_block * 32 + 16 * half);
+        scales = *reinterpret_cast<const u32_a2*>(block + (half != 0 ? 192 + 4 * (unit & 3) : 206));
+    }
+    __device__ __forceinline__ void arrange() {
 #pragma unroll
-        for (int chunk = 0; chunk < 2; ++chunk) {
-            const int position = 16 * chunk + 8 * half;
-            low[0][chunk] = *reinterpret_cast<const u32x2_a2*>(block + half_block * 64 + position);
-            low[1][chunk] = *reinterpret_cast<const u32x2_a2*>(block + half_block * 64 + 32 + position);
-            high[chunk] = *reinterpret_cast<const u32x2_a2*>(block + 128 + half_block * 32 + position);
+        for (int word = 0; word < 2; ++word) {
+#pragma unroll
+            for (int step = 0; step < 2; ++step) {
+                const Traded t = trade(low[step][word], low[step][word + 2]);
+                low[step][word] = t.first;
+                low[step][word + 2] = t.second;
+            }
+            const Traded t = trade(high[word], high[word + 2]);
+            high[word] = t.first;
+            high[word + 2] = t.second;
         }
-        const auto* pairs = reinterpret_cast<const std::uint16_t*>(block + 192 + 4 * (unit & 3));
-        scales = pairs[0] | (static_cast<std::uint32_t>(pairs[1]) << 16);
-        d = *reinterpret_cast<const std::uint16_t*>(block + 208);
+        const Traded t = trade(scales, scales);
+        d = t.first;
+        scales = t.second;
     }
     __device__ __forceinline__ void words(int step, int chunk, int word, std::uint32_t& even, std::uint32_t& odd) const {
-        const std::uint32_t q = ((low[step][chunk][word] >> (4 * upper)) & 0x0f0f0f0fu) |
-            (((high[chunk][word] >> (4 * upper + 2 * step)) & 0x03030303u) << 4);
+        const std::uint32_t q = ((low[step][2 * chunk + word] >> (4 * upper)) & 0x0f0f0f0fu) |
+            (((high[2 * chunk + word] >> (4 * upper + 2 * step)) & 0x03030303u) << 4);
         codes_to_bf16(q, 32.0f, even, odd);
     }
     __device__ __forceinline__ float scale(int step, int chunk) const {
         const int code = static_cast<std::int8_t>(scales >> (8 * (2 * step + chunk)));
-        return half_bits_to_float(d) * static_cast<float>(code);
+        return half_bits_to_float(d >> 16) * static_cast<float>(code);
     }
     __device__ __forceinline__ float minimum(int) const { return 0.0f; }
 };
@@ -187,15 +214,20 @@ template <>
 struct Unit<kEncQ8_0> {
     static constexpr bool kWide = true, kScaled = true, kMinimum = false, kScalePerChunk = false;
     u32x4_a2 codes[2];
-    std::uint32_t d[2];
+    std::uint32_t d[2];  // as loaded: [0] the scale of block `half`
     // (`steps`: the row's 32-column blocks; a row of an odd number of them reads its last one twice)
     __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half, int steps) {
 #pragma unroll
         for (int step = 0; step < 2; ++step) {
             const std::uint8_t* block = row + min(2 * unit + step, steps - 1) * 34;
             codes[step] = *reinterpret_cast<const u32x4_a2*>(block + 2 + 16 * half);
-            d[step] = *reinterpret_cast<const std::uint16_t*>(block);
         }
+        d[0] = *reinterpret_cast<const std::uint16_t*>(row + min(2 * unit + half, steps - 1) * 34);
+    }
+    __device__ __forceinline__ void arrange() {
+        const Traded t = trade(d[0], d[0]);
+        d[0] = t.first;
+        d[1] = t.second;
     }
     __device__ __forceinline__ void words(int step, int chunk, int word, std::uint32_t& even, std::uint32_t& odd) const {
         // (flipping the sign bit turns the code q into the byte q + 128)
@@ -217,6 +249,7 @@ struct Unit<kEncBF16> {
             values[step][1] = *reinterpret_cast<const u32x4_a2*>(source + 16);
         }
     }
+    __device__ __forceinline__ void arrange() {}
     __device__ __forceinline__ void words(int step, int chunk, int word, std::uint32_t& low, std::uint32_t& high) const {
         low = values[step][chunk][2 * word];
         high = values[step][chunk][2 * word + 1];
@@ -238,6 +271,7 @@ struct Unit<kEncF32> {
             }
         }
     }
+    __device__ __forceinline__ void arrange() {}
     __device__ __forceinline__ Terms terms(int step, int chunk) const {
         float eight[8];
 #pragma unroll
@@ -418,6 +452,8 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
         load_inputs(2 * first_unit);
         for (int unit = first_unit; unit < end_unit; ++unit) {
 #pragma unroll
+            for (int n = 0; n < NT; ++n) now[n].arrange();
+#pragma unroll
             for (int n = 0; n < NT; ++n) load_unit<ENC>(next[n], w_row[n], min(unit + 1, end_unit - 1), half, steps);
             float partial[MT][2];
 #pragma unroll
@@ -572,7 +608,8 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
 #pragma unroll
         for (int n = 0; n < 2; ++n) load_unit<ENC>(into[n], w_row[n], min(unit, end_unit - 1), half, steps);
     };
-    const auto decode_piece = [&](const Slice& source, int n, int step, int piece) {
+    const auto decode_piece = [&](Slice& source, int n, int step, int piece) {
+        if (step == 0 && piece == 0) source.arrange();  // a unit's first piece
         const int chunk = piece >> 1, word = piece & 1;
         std::uint32_t low, high;
         source.words(step, chunk, word, low, high);
@@ -600,7 +637,7 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
     }
 
     // One unit, two steps: `own_bytes` holds its packed bytes, `next_bytes` those of the unit behind it.
-    const auto pass = [&](Slice (&own_bytes)[2], const Slice (&next_bytes)[2], int unit) {
+    const auto pass = [&](Slice (&own_bytes)[2], Slice (&next_bytes)[2], int unit) {
         float least[2] = {};
 #pragma unroll
         for (int step = 0; step < 2; ++step) {
