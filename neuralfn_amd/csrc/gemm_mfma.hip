@@ -52,6 +52,8 @@ constexpr int kBN = 128;
 constexpr int kBK = 64;
 constexpr int kThreads = 256;
 constexpr int kMaxProjections = 4;  // of one call
+constexpr int kLowRows = 32;    // rows up to which every wave takes all of them
+constexpr int kLowShares = 8;   // K shares of theirs at most
 constexpr int kMaxShares = 4;  // K shares of a split launch at most
 constexpr int kRowBytes = 144;  // 64 fp16 + 16 bytes of padding
 constexpr int kStageBytes = kBN * kRowBytes;
@@ -555,6 +557,38 @@ struct GemmGroup {
     int shares[kMaxProjections];
 };
 
+// this workgroup's projection, share and tile
+struct GroupPlace {
+    const std::uint8_t* weights;
+    float *output, *partials;
+    std::int64_t output_dim;
+    int share, shares, tile;
+};
+// (a macro: a reference to a kernel's argument makes the compiler copy it to scratch memory)
+#define NFN_PLACE(place, group)                                              \
+    GroupPlace place;                                                        \
+    place.weights = group.weights[0];                                        \
+    place.output = group.output[0];                                          \
+    place.partials = group.partials[0];                                      \
+    place.output_dim = group.output_dim[0];                                  \
+    place.shares = group.shares[0];                                          \
+    {                                                                        \
+        int first = 0, tiles = group.tiles[0];                               \
+        _Pragma("unroll") for (int i = 1; i < kMaxProjections; ++i) {        \
+            if (static_cast<int>(blockIdx.x) >= group.first[i]) {            \
+                place.weights = group.weights[i];                            \
+                place.output = group.output[i];                              \
+                place.partials = group.partials[i];                          \
+                place.output_dim = group.output_dim[i];                      \
+                place.shares = group.shares[i];                              \
+                first = group.first[i];                                      \
+                tiles = group.tiles[i];                                      \
+            }                                                                \
+        }                                                                    \
+        place.share = (static_cast<int>(blockIdx.x) - first) / tiles;        \
+        place.tile = (static_cast<int>(blockIdx.x) - first) % tiles;         \
+    }
+
 // RB: 32-row blocks per wave; the workgroup's tile is 128*RB rows by 128 columns.
 template <std::uint32_t ENC, int RB>
 __global__ __launch_bounds__(kThreads)
@@ -565,27 +599,13 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // rows 64*wave .. +63 of the tile
-    const std::uint8_t* weights = group.weights[0];
-    float* output = group.output[0];
-    float* partials = group.partials[0];
-    std::int64_t output_dim = group.output_dim[0];
-    int first = 0, tiles = group.tiles[0], shares = group.shares[0];
-#pragma unroll
-    for (int i = 1; i < kMaxProjections; ++i) {
-        if (static_cast<int>(blockIdx.x) >= group.first[i]) {
-            weights = group.weights[i];
-            output = group.output[i];
-            partials = group.partials[i];
-            output_dim = group.output_dim[i];
-            first = group.first[i];
-            tiles = group.tiles[i];
-            shares = group.shares[i];
-        }
-    }
-    const int share = (static_cast<int>(blockIdx.x) - first) / tiles;
-    const int tile = (static_cast<int>(blockIdx.x) - first) % tiles;
-    const int m_tile = tile % m_tiles;
-    const int n_tile = tile / m_tiles;
+    NFN_PLACE(place, group)
+    const std::uint8_t* weights = place.weights;
+    float* output = place.output;
+    const std::int64_t output_dim = place.output_dim;
+    const int share = place.share, shares = place.shares;
+    const int m_tile = place.tile % m_tiles;
+    const int n_tile = place.tile / m_tiles;
     constexpr int kTileRows = 128 * RB;
     const std::int64_t m0 = static_cast<std::int64_t>(m_tile) * kTileRows;
     const std::int64_t n0 = static_cast<std::int64_t>(n_tile) * kBN;
@@ -597,7 +617,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     const int steps = (end_block - first_block) * 4;  // a positive multiple of 4
     const int last = steps - 1;
     const std::int64_t row_stride = group.row_stride;
-    if (share > 0) output = partials + (share - 1) * rows * output_dim;
+    if (share > 0) output = place.partials + (share - 1) * rows * output_dim;
 
     // activations: fragment (row block, K chunk) is 1 KB, a row block's chunks are consecutive
     const std::int64_t row_block_bytes = (input_dim / 16) * kFragmentBytes;
@@ -775,6 +795,181 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     }
 }
 
+// ---------------------------------------------------------------------------
+// Up to 32 rows: a wave owns 32 columns and all rows of the same 128-column tile, so that a decoded
+// weight fragment is read from LDS by one wave instead of four and by the wave that wrote it: no
+// barrier, a quarter of the LDS reads, no matrix instructions for rows that are not there.  What
+// bounds it is the latency of the packed bytes and of the fragments from L2, which are requested a
+// block and four steps ahead, and with that the number of workgroups: K is cut into up to eight
+// shares.  17 rows, width 6,656, against 128-row tiles: Q, K, V and gate 41 -> 32 us for Q4_K, 50 -> 41
+// for Q6_K; O (4,096 wide) 43 -> 21 and 52 -> 25; gate and up 68 -> 54 and 85 -> 68; down 56 -> 39
+// and 66 -> 49; Q8_0 50 -> 47, 52 -> 32, 86 -> 84, 64 -> 60.
+// ---------------------------------------------------------------------------
+struct LowActivations {
+    f16x8 chunk[4];
+};
+
+// from the first run of 16 to the second: 16 rows apart where four lanes share a row
+template <std::uint32_t ENC>
+constexpr int kLowSecondRun = kParts<ENC> == 2 ? 64 : 16 * kRowBytes;
+
+// One K step of one wave: multiplies the step in `stage` and decodes the next one into `next_stage`.
+template <std::uint32_t ENC>
+__device__ __forceinline__ void low_step(v16f& acc, LowActivations& a, const std::uint8_t* stage,
+                                         std::uint8_t* next_stage, PackedSlice<ENC>& b_next,
+                                         const BlockHeader<ENC>& header, int decode_pair, int b_part,
+                                         const std::uint8_t* a_fetch) {
+    // what a lane wrote is seen by the wave's other lanes, and no LDS access moves across
+    const auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    wave_sync();
+    f16x8 weights[4];
+#pragma unroll
+    for (int chunk = 0; chunk < 4; ++chunk) weights[chunk] = *reinterpret_cast<const f16x8*>(stage + chunk * 32);
+    wave_sync();
+    std::uint32_t w[2], v[2];
+    b_next.prepare_bits(header, decode_pair, b_part);
+    b_next.prepare_scales(header);
+    b_next.template group_a<0>(w);
+    b_next.template group_a<1>(v);
+    NFN_WRITE16(next_stage, w[0], w[1], v[0], v[1]);
+    b_next.template group_a<2>(w);
+    b_next.template group_a<3>(v);
+    NFN_WRITE16(next_stage + 16, w[0], w[1], v[0], v[1]);
+    b_next.template group_b<0>(w);
+    b_next.template group_b<1>(v);
+    NFN_WRITE16(next_stage + kLowSecondRun<ENC>, w[0], w[1], v[0], v[1]);
+    b_next.template group_b<2>(w);
+    b_next.template group_b<3>(v);
+    NFN_WRITE16(next_stage + kLowSecondRun<ENC> + 16, w[0], w[1], v[0], v[1]);
+#pragma unroll
+    for (int chunk = 0; chunk < 4; ++chunk) NFN_MFMA(a.chunk[chunk], weights[chunk], acc);
+    NFN_FENCE();
+#pragma unroll
+    for (int chunk = 0; chunk < 4; ++chunk) {
+        a.chunk[chunk] = *reinterpret_cast<const f16x8*>(a_fetch + chunk * kFragmentBytes);
+    }
+    NFN_FENCE();
+}
+
+// The packed bytes of a block of a lane's rows, requested together: the steps' pieces of a row lie
+// in the same cache lines, which do not stay in the vector cache from one step to the next.
+template <std::uint32_t ENC>
+struct LowBlock {
+    BlockHeader<ENC> header;
+    PackedSlice<ENC> s0, s1, s2, s3;  // (Q6_K: s0 the first half, s2 the second)
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int part) {
+        header.load(rows.first, block);
+        s0.load(rows, block, 0, part);
+        if constexpr (!kHalfBlocks<ENC>) s1.load(rows, block, 1, part);
+        s2.load(rows, block, 2, part);
+        if constexpr (!kHalfBlocks<ENC>) s3.load(rows, block, 3, part);
+    }
+};
+
+template <std::uint32_t ENC>
+__global__ __launch_bounds__(kThreads, 2) void gemm_f16_low_kernel(
+    const std::uint8_t* __restrict__ activations, const float* __restrict__ inverse_scale, std::int64_t input_dim,
+    std::int64_t rows, GemmGroup group) {
+    extern __shared__ __attribute__((aligned(16))) std::uint8_t lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    NFN_PLACE(place, group)
+    const std::int64_t output_dim = place.output_dim;
+    const std::int64_t n0 = static_cast<std::int64_t>(place.tile) * kBN + 32 * wave;
+    const int total_blocks = static_cast<int>(input_dim >> 8);
+    const int first_block = total_blocks * place.share / place.shares;
+    const int end_block = total_blocks * (place.share + 1) / place.shares;
+    const int steps = (end_block - first_block) * 4;
+    const int last = steps - 1;
+    const int last_block = (steps >> 2) - 1;
+    float* const output = place.share > 0 ? place.partials + (place.share - 1) * rows * output_dim : place.output;
+
+    constexpr int kStepBytes = (kBK / 16) * kFragmentBytes;
+    const std::uint8_t* a_global =
+        activations + static_cast<std::int64_t>(first_block) * 16 * kFragmentBytes + lane * 16;
+    const auto activations_of = [&](int step) {
+        return a_global + static_cast<std::int64_t>(min(step, last)) * kStepBytes;
+    };
+    // (the rows of a lane inside the wave's 32: the same bank pattern as above)
+    const int b_part = lane & (kParts<ENC> - 1);
+    const int b_turn = lane / kParts<ENC>;
+    const int b_row = kParts<ENC> == 4 ? b_turn : (b_turn & ~6) | ((b_turn & 2) << 1) | ((b_turn & 4) >> 1);
+    const std::int64_t b_skip = static_cast<std::int64_t>(first_block) * kBlockBytes<ENC>;
+    WeightRows b_global;
+    b_global.first = place.weights + min(n0 + b_row, output_dim - 1) * group.row_stride + b_skip;
+    b_global.second = place.weights + min(n0 + b_row + 16, output_dim - 1) * group.row_stride + b_skip;
+
+    v16f acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    LowActivations a0, a1, a2, a3;
+    LowBlock<ENC> even, odd;  // blocks 0, 2, 4 ... and 1, 3, 5 ...
+    even.load(b_global, 0, b_part);
+    const auto load_activations = [&](LowActivations& a, int step) {
+#pragma unroll
+        for (int chunk = 0; chunk < 4; ++chunk) {
+            a.chunk[chunk] = *reinterpret_cast<const f16x8*>(activations_of(step) + chunk * kFragmentBytes);
+        }
+    };
+    load_activations(a0, 0);
+    load_activations(a1, 1);
+    load_activations(a2, 2);
+    load_activations(a3, 3);
+
+    std::uint8_t* const mine = lds + wave * 32 * kRowBytes;
+    std::uint8_t* const write0 = mine + b_row * kRowBytes + b_part * 32;
+    std::uint8_t* const write1 = write0 + kStageBytes;
+    const std::uint8_t* const read0 = mine + (lane & 31) * kRowBytes + (lane >> 5) * 16;
+    const std::uint8_t* const read1 = read0 + kStageBytes;
+    {
+        std::uint32_t wa[4][2], wb[4][2];
+        even.s0.prepare_bits(even.header, 0, b_part);
+        even.s0.prepare_scales(even.header);
+        even.s0.template group_a<0>(wa[0]);
+        even.s0.template group_a<1>(wa[1]);
+        even.s0.template group_a<2>(wa[2]);
+        even.s0.template group_a<3>(wa[3]);
+        even.s0.template group_b<0>(wb[0]);
+        even.s0.template group_b<1>(wb[1]);
+        even.s0.template group_b<2>(wb[2]);
+        even.s0.template group_b<3>(wb[3]);
+        NFN_WRITE16(write0, wa[0][0], wa[0][1], wa[1][0], wa[1][1]);
+        NFN_WRITE16(write0 + 16, wa[2][0], wa[2][1], wa[3][0], wa[3][1]);
+        NFN_WRITE16(write0 + kLowSecondRun<ENC>, wb[0][0], wb[0][1], wb[1][0], wb[1][1]);
+        NFN_WRITE16(write0 + kLowSecondRun<ENC> + 16, wb[2][0], wb[2][1], wb[3][0], wb[3][1]);
+    }
+
+    // four steps, one block: `now` is decoded from its second step on and the first of `next`
+    const auto block_of_four = [&](int block, LowBlock<ENC>& now, LowBlock<ENC>& next) {
+        constexpr bool kHalves = kHalfBlocks<ENC>;
+        const int step = 4 * block;
+        next.load(b_global, min(block + 1, last_block), b_part);
+        NFN_FENCE();
+        low_step<ENC>(acc, a0, read0, write1, kHalves ? now.s0 : now.s1, now.header, 1, b_part,
+                          activations_of(step + 4));
+        low_step<ENC>(acc, a1, read1, write0, now.s2, now.header, 2, b_part, activations_of(step + 5));
+        low_step<ENC>(acc, a2, read0, write1, kHalves ? now.s2 : now.s3, now.header, 3, b_part,
+                          activations_of(step + 6));
+        low_step<ENC>(acc, a3, read1, write0, next.s0, next.header, 0, b_part, activations_of(step + 7));
+    };
+    for (int block = 0; block <= last_block; block += 2) {
+        block_of_four(block, even, odd);
+        if (block < last_block) block_of_four(block + 1, odd, even);
+    }
+
+    const std::int64_t n = n0 + (lane & 31);
+    const int row_base = (lane >> 5) * 4;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int row = row_base + 8 * (r >> 2) + (r & 3);
+        if (row < rows && n < output_dim) output[row * output_dim + n] = acc[r] * inverse_scale[row];
+    }
+}
+
 // Sum of the K shares: output[i] = share 0 (in place) + share 1 + ..., in that order;
 // blockIdx.y: the projection.
 struct ShareSums {
@@ -801,6 +996,7 @@ __global__ __launch_bounds__(256) void sum_shares_kernel(ShareSums sums) {
     for (std::int64_t index = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
          index < count; index += stride) {
         float total = output[index];
+#pragma unroll 4
         for (int share = 1; share < shares; ++share) total += partials[(share - 1) * count + index];
         output[index] = total;
     }
@@ -822,8 +1018,12 @@ __global__ __launch_bounds__(256) void sum_shares_kernel(ShareSums sums) {
 // The projections of one call run in one launch an encoding, each with the shares that it has by
 // itself, so that few workgroups of one do not wait for those of another: 17 rows into Q, K, V and
 // the gate of width 6,656 took 107 us (Q5_K) one after another and take 44, 333 rows 170 and 84.
+// Up to 32 rows run on the kernel that cuts the columns among the waves, with shares of three blocks
+// or more, at most eight, until there are two workgroups a unit.  (Two 32-row blocks a wave, for up
+// to 64 rows: 128-row tiles are as fast or faster where the tiles are many, 64 rows of gate and up
+// 81 us (Q4_K) and 203 (Q8_0) against 78 and 93 at 65.)
 struct Plan {
-    int row_blocks;  // 32-row blocks per wave: 2 = 256-row tiles, 1 = 128-row tiles
+    int tile_rows;  // 256 and 128 (two 32-row blocks a wave or one), 32 (all rows in every wave)
     int shares;
 };
 
@@ -831,8 +1031,16 @@ Plan plan(std::uint32_t encoding, std::int64_t rows, std::int64_t output_dim,
           std::int64_t input_dim) {
     const std::int64_t units = compute_units();
     const std::int64_t n_tiles = (output_dim + kBN - 1) / kBN;
+    if (rows <= kLowRows) {
+        std::int64_t shares = 2 * units / n_tiles;
+        const std::int64_t most = (input_dim >> 8) / 3;
+        if (shares > most) shares = most;
+        if (shares > kLowShares) shares = kLowShares;
+        if (shares < 1) shares = 1;
+        return Plan{kLowRows, static_cast<int>(shares)};
+    }
     const std::int64_t tall_tiles = (rows + 255) / 256 * n_tiles;
-    if (tall_tiles >= units) return Plan{2, 1};
+    if (tall_tiles >= units) return Plan{256, 1};
     std::int64_t longest = (input_dim >> 8) / 12;  // shares that still get twelve blocks each
     if (longest > kMaxShares) longest = kMaxShares;
     if (tall_tiles * 8 <= units) {
@@ -846,19 +1054,19 @@ Plan plan(std::uint32_t encoding, std::int64_t rows, std::int64_t output_dim,
         std::int64_t shares = units * 3 / tiles;
         if (shares > shortest) shares = shortest;
         if (shares < 1) shares = 1;
-        return Plan{1, static_cast<int>(shares)};
+        return Plan{128, static_cast<int>(shares)};
     }
     if (rows > 128) {
         std::int64_t shares = 2 * units / tall_tiles;
         if (shares > longest) shares = longest;
-        if (shares >= 2) return Plan{2, static_cast<int>(shares)};
-        if (2 * tall_tiles >= units) return Plan{2, 1};
+        if (shares >= 2) return Plan{256, static_cast<int>(shares)};
+        if (2 * tall_tiles >= units) return Plan{256, 1};
     }
     const std::int64_t tiles = (rows + 127) / 128 * n_tiles;
     std::int64_t shares = units * (encoding == kEncQ6K ? 2 : 3) / tiles;
     if (shares > longest) shares = longest;
     if (shares < 1) shares = 1;
-    return Plan{1, static_cast<int>(shares)};
+    return Plan{128, static_cast<int>(shares)};
 }
 
 template <std::uint32_t ENC, int RB>
@@ -872,8 +1080,13 @@ void launch_tiles(GemmGroup group, int count, const std::uint8_t* activations, c
         group.tiles[i] = m_tiles * static_cast<int>((group.output_dim[i] + kBN - 1) / kBN);
         workgroups += group.tiles[i] * group.shares[i];
     }
-    hipLaunchKernelGGL((gemm_f16_kernel<ENC, RB>), dim3(static_cast<unsigned>(workgroups)), dim3(kThreads),
-                       2 * kStageBytes, stream, activations, inverse_scale, input_dim, rows, m_tiles, group);
+    if (rows > kLowRows) {
+        hipLaunchKernelGGL((gemm_f16_kernel<ENC, RB>), dim3(static_cast<unsigned>(workgroups)), dim3(kThreads),
+                           2 * kStageBytes, stream, activations, inverse_scale, input_dim, rows, m_tiles, group);
+    } else {
+        hipLaunchKernelGGL(gemm_f16_low_kernel<ENC>, dim3(static_cast<unsigned>(workgroups)), dim3(kThreads),
+                           2 * kStageBytes, stream, activations, inverse_scale, input_dim, rows, group);
+    }
 }
 
 // One launch for `count` projections of one encoding and, if any of them splits K, one for the sums.
@@ -925,7 +1138,7 @@ std::int64_t gemm_f16_workspace_bytes(std::int64_t rows, std::int64_t input_dim,
 void gemm_f16_plan(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
                    std::int64_t output_dim, int* tile_rows, int* k_shares) {
     const Plan chosen = plan(encoding, rows, output_dim, input_dim);
-    *tile_rows = 128 * chosen.row_blocks;
+    *tile_rows = chosen.tile_rows;
     *k_shares = chosen.shares;
 }
 
@@ -1002,7 +1215,7 @@ void launch_gemm_f16(const Descriptor* descriptors, int count, const float* inpu
             group.shares[members] = chosen.shares;
             used += floats;
             short_groups += (rows + 127) / 128 * ((descriptors[i].output_dim + kBN - 1) / kBN) * chosen.shares;
-            if (chosen.row_blocks == 2) tall = true;
+            if (chosen.tile_rows == 256) tall = true;
             ++members;
         }
         // 256-row tiles where a member would take them by itself, unless 128-row tiles leave half

@@ -13,7 +13,7 @@ std::int64_t gemm_f16_workspace_bytes(std::int64_t rows, std::int64_t input_dim,
                                       std::int64_t output_dim);
 bool gemm_f16_supports(std::uint32_t encoding, std::int64_t input_dim);
 // How a launch of this geometry is cut on the current device: rows of the
-// output tile a workgroup owns (128 or 256) and the number of K shares (1 =
+// output tile a workgroup owns (256 or 128; 32 for up to 32 rows) and the number of K shares (1 =
 // unsplit; more = one partial output per share, summed by a second launch).
 void gemm_f16_plan(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
                    std::int64_t output_dim, int* tile_rows, int* k_shares);

@@ -1547,6 +1547,24 @@ def test_prefill_gemm_split_k(cuda, oracle, encoding, rows, in_dim, plan):
     assert np.array_equal(y.view(np.uint32), again.view(np.uint32))  # fixed summation order
 
 
+@pytest.mark.parametrize("rows,out_dim,in_dim,plan", [
+    (1, 1, 256, (32, 1)), (17, 129, 1536, (32, 2)), (32, 31, 4608, (32, 6)),   # rows of one fragment, K shares
+    (20, 97, 6656, (32, 8)), (31, 128, 2560, (32, 3)),                         # shares of unequal length
+    (17, 40000, 512, (32, 1)), (33, 129, 1536, (128, 1)),                      # enough tiles without shares; past the kernel's rows
+])
+@pytest.mark.parametrize("encoding", ALL_PACKED)
+def test_prefill_gemm_few_rows(cuda, oracle, encoding, rows, out_dim, in_dim, plan):
+    # up to 32 rows: the kernel that cuts the columns among a workgroup's waves
+    assert tile_ops.gemm_plan(encoding, rows, in_dim, out_dim) == plan
+    packed = random_packed(encoding, out_dim, in_dim, 90 + rows)
+    x = kquant.synthetic_activations(91, rows, in_dim)
+    weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    y = tile_ops.gemm(weight, to_device(x, cuda)).cpu().numpy()
+    assert normalised_error(y, oracle.linear(encoding, packed, out_dim, in_dim, x)) <= TOLERANCE
+    again = tile_ops.gemm(weight, to_device(x, cuda)).cpu().numpy()
+    assert np.array_equal(y.view(np.uint32), again.view(np.uint32))  # fixed summation order
+
+
 def test_prefill_gemm_multi_equals_single_calls(cuda, oracle):
     """nfn_mi355_k_quant_gemm_multi_float32_v1: one conversion of the input, the single call's bits."""
     rows, in_dim = 300, 1024
