@@ -184,7 +184,8 @@ __global__ __launch_bounds__(256) void prepare_activations_kernel(
 // ---------------------------------------------------------------------------
 // What one thread holds of the packed weights: 32 weights of a K step, in two runs of 16.
 //   Q4_K, Q5_K: positions 16*part .. 16*part+15 of both 32-value groups of the step, of one row;
-//               two neighbouring lanes share a row.
+//               two neighbouring lanes share a row.  Q5_K's fifth bits, which serve the whole block,
+//               come with the block's header (2,048 rows of gate and up 863 -> 836 us).
 //   Q6_K, Q8_0: the step's columns 16*part .. 16*part+15 of two rows, 64 apart; four neighbouring
 //               lanes share a row.  A Q6_K slice serves the two steps of a half block, whose
 //               codes share their bytes.
@@ -211,7 +212,7 @@ struct BlockHeader;
 template <>
 struct BlockHeader<kEncQ4K> {
     u32x4 words;  // d, dmin and the twelve scale bytes
-    __device__ __forceinline__ void load(const std::uint8_t* row, int block) {
+    __device__ __forceinline__ void load(const std::uint8_t* row, int block, int part) {
         words = *reinterpret_cast<const u32x4*>(row + block * 144);
     }
 };
@@ -243,23 +244,25 @@ struct PackedSlice<kEncQ4K> {
 template <>
 struct BlockHeader<kEncQ5K> {
     u32x4 words;  // d, dmin and the twelve scale bytes
-    __device__ __forceinline__ void load(const std::uint8_t* row, int block) {
+    u32x4 high;   // the fifth bits of the lane's positions, two for each of the block's steps
+    __device__ __forceinline__ void load(const std::uint8_t* row, int block, int part) {
         words = *reinterpret_cast<const u32x4*>(row + block * 176);
+        high = *reinterpret_cast<const u32x4*>(row + block * 176 + 16 + part * 16);
     }
 };
 
 template <>
 struct PackedSlice<kEncQ5K> {
-    u32x4 codes, high;
+    u32x4 codes;
     KBlockScales c;
+    u32x4 high;
     int high_shift;
     __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
-        const std::uint8_t* p = rows.first + block * 176;
-        high = *reinterpret_cast<const u32x4*>(p + 16 + part * 16);
-        codes = *reinterpret_cast<const u32x4*>(p + 48 + pair * 32 + part * 16);
+        codes = *reinterpret_cast<const u32x4*>(rows.first + block * 176 + 48 + pair * 32 + part * 16);
     }
     __device__ __forceinline__ void prepare_bits(const BlockHeader<kEncQ5K>& header, int pair, int) {
         c.bits(header.words, pair);
+        high = header.high;
         high_shift = 2 * pair;  // bit 2*pair: first group, bit 2*pair+1: second
     }
     __device__ __forceinline__ void prepare_scales(const BlockHeader<kEncQ5K>& header) {
@@ -281,7 +284,7 @@ struct PackedSlice<kEncQ5K> {
 
 template <>
 struct BlockHeader<kEncQ6K> {  // the scales come with the slice
-    __device__ __forceinline__ void load(const std::uint8_t*, int) {}
+    __device__ __forceinline__ void load(const std::uint8_t*, int, int) {}
 };
 
 template <>
@@ -333,7 +336,7 @@ struct PackedSlice<kEncQ6K> {
 
 template <>
 struct BlockHeader<kEncQ8_0> {  // the scales sit next to the codes
-    __device__ __forceinline__ void load(const std::uint8_t*, int) {}
+    __device__ __forceinline__ void load(const std::uint8_t*, int, int) {}
 };
 
 template <>
@@ -544,6 +547,27 @@ constexpr int kBlockBytes = ENC == kEncQ4K ? 144 : ENC == kEncQ5K ? 176 : ENC ==
 template <std::uint32_t ENC, int RB>
 constexpr int kWavesPerSimd = ENC == kEncQ6K ? RB == 1 ? 2 : 1 : RB == 1 && ENC == kEncQ4K ? 3 : 2;
 
+// The packed bytes of a block of a lane's rows.
+template <std::uint32_t ENC>
+struct Slices {
+    PackedSlice<ENC> b0, b1, b2, b3;  // of its four steps; Q6_K: b0 the first half, b1 the second
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int part) {
+        b0.load(rows, block, 0, part);
+        b1.load(rows, block, kHalfBlocks<ENC> ? 2 : 1, part);
+        if constexpr (!kHalfBlocks<ENC>) {
+            b2.load(rows, block, 2, part);
+            b3.load(rows, block, 3, part);
+        }
+    }
+};
+// Where the registers allow a second set, a block's packed bytes are requested together, one block
+// ahead: the steps' pieces of a row lie in the same cache lines, which do not stay in the vector
+// cache from one step to the next (4,096 rows of gate and up, Q4_K: 1,577 -> 1,533 us; 100 rows of
+// Q5_K 92 -> 88).  Q6_K, whose slices serve two steps, gains nothing by it, and Q8_0, whose block of a
+// row is more than two lines, loses: 100 rows of O 55 -> 69 us.
+template <std::uint32_t ENC, int RB>
+constexpr bool kWholeBlocks = (ENC == kEncQ4K && RB == 2) || (ENC == kEncQ5K && RB == 1);
+
 // The projections of one launch: one encoding, one input.  Workgroup numbers run through the
 // projections, inside each through its K shares, inside each through its tiles.
 struct GemmGroup {
@@ -656,19 +680,13 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     // The header of a 256-value block is loaded once, three or more steps
     // before the first of its four steps is decoded.
     ActivationSlice a_now;
-    PackedSlice<ENC> b0, b1, b2, b3;
+    constexpr bool kWhole = kWholeBlocks<ENC, RB>;
+    Slices<ENC> set0, set1;  // (set1: whole blocks only; the sets swap roles like the headers)
     BlockHeader<ENC> header_even, header_odd;  // blocks 0, 2, 4 ... and 1, 3, 5 ...
     const int last_block = (steps >> 2) - 1;
-    header_even.load(b_global.first, 0);
-    header_odd.load(b_global.first, min(1, last_block));
-    b0.load(b_global, 0, 0, b_part);
-    if constexpr (kHalfBlocks<ENC>) {
-        b1.load(b_global, 0, 2, b_part);
-    } else {
-        b1.load(b_global, 0, 1, b_part);
-        b2.load(b_global, 0, 2, b_part);
-        b3.load(b_global, 0, 3, b_part);
-    }
+    header_even.load(b_global.first, 0, b_part);
+    header_odd.load(b_global.first, min(1, last_block), b_part);
+    set0.load(b_global, 0, b_part);
     a_now.r0k0 = NFN_LOAD_ACTIVATIONS(a_global, 0, 0);
     a_now.r0k1 = NFN_LOAD_ACTIVATIONS(a_global, 0, 1);
     a_now.r0k2 = NFN_LOAD_ACTIVATIONS(a_global, 0, 2);
@@ -681,23 +699,23 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     }
     {
         std::uint32_t wa[4][2], wb[4][2];
-        b0.prepare_bits(header_even, 0, b_part);
-        b0.prepare_scales(header_even);
-        b0.template group_a<0>(wa[0]);
-        b0.template group_a<1>(wa[1]);
-        b0.template group_a<2>(wa[2]);
-        b0.template group_a<3>(wa[3]);
-        b0.template group_b<0>(wb[0]);
-        b0.template group_b<1>(wb[1]);
-        b0.template group_b<2>(wb[2]);
-        b0.template group_b<3>(wb[3]);
+        set0.b0.prepare_bits(header_even, 0, b_part);
+        set0.b0.prepare_scales(header_even);
+        set0.b0.template group_a<0>(wa[0]);
+        set0.b0.template group_a<1>(wa[1]);
+        set0.b0.template group_a<2>(wa[2]);
+        set0.b0.template group_a<3>(wa[3]);
+        set0.b0.template group_b<0>(wb[0]);
+        set0.b0.template group_b<1>(wb[1]);
+        set0.b0.template group_b<2>(wb[2]);
+        set0.b0.template group_b<3>(wb[3]);
         std::uint8_t* target = lds + b_target;
         NFN_WRITE16(target, wa[0][0], wa[0][1], wa[1][0], wa[1][1]);
         NFN_WRITE16(target + 16, wa[2][0], wa[2][1], wa[3][0], wa[3][1]);
         NFN_WRITE16(target + kSecondRun<ENC>, wb[0][0], wb[0][1], wb[1][0], wb[1][1]);
         NFN_WRITE16(target + kSecondRun<ENC> + 16, wb[2][0], wb[2][1], wb[3][0], wb[3][1]);
     }
-    if constexpr (!kHalfBlocks<ENC>) b0.load(b_global, min(1, last_block), 0, b_part);  // step 4, or step 0 again
+    if constexpr (!kHalfBlocks<ENC> && !kWhole) set0.b0.load(b_global, min(1, last_block), 0, b_part);  // step 4, or step 0 again
     __syncthreads();
 
     const int operand = (lane & 31) * kRowBytes + (lane >> 5) * 16;
@@ -723,19 +741,26 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     // step s+5 and the activation slice step s+1.  `now` holds the scales of
     // this block, `next` those of the following one (needed by the fourth step,
     // which decodes the first step of that block).
-    // (Q6_K: b0 holds a block's first half, which the first and, of the next block, the fourth step
+    // (Whole blocks: the next block goes to the other set at the start instead.
+    // Q6_K: b0 holds a block's first half, which the first and, of the next block, the fourth step
     // decode, b1 the second.)
-    auto block_of_four = [&](int step, const BlockHeader<ENC>& now, const BlockHeader<ENC>& next) {
+    auto block_of_four = [&](int step, const BlockHeader<ENC>& now, const BlockHeader<ENC>& next, Slices<ENC>& mine, Slices<ENC>& other) {
         constexpr bool kHalves = kHalfBlocks<ENC>;
         constexpr int kAhead = kHalves ? 3 : 4;  // from the step that is decoded to the one that is fetched
-        PackedSlice<ENC>&second = kHalves ? b0 : b1, &third = kHalves ? b1 : b2, &fourth = kHalves ? b1 : b3;
-        k_step<ENC, RB, true>(acc, a_now, current, b_read0, b_read1, b_write1, second, now, 1, b_part,
+        Slices<ENC>& after = kWhole ? other : mine;
+        if constexpr (kWhole) {
+            const int block = min((step >> 2) + 1, last_block);
+            other.load(b_global, block, b_part);
+            NFN_FENCE();
+        }
+        PackedSlice<ENC>&second = kHalves ? mine.b0 : mine.b1, &third = kHalves ? mine.b1 : mine.b2, &fourth = kHalves ? mine.b1 : mine.b3;
+        k_step<ENC, RB, !kWhole>(acc, a_now, current, b_read0, b_read1, b_write1, second, now, 1, b_part,
                     activations_of(step + 1), row_block_bytes, b_global, min(step + 1 + kAhead, last));
-        k_step<ENC, RB, !kHalves>(acc, a_now, current, b_read1, b_read0, b_write0, third, now, 2, b_part,
+        k_step<ENC, RB, !kHalves && !kWhole>(acc, a_now, current, b_read1, b_read0, b_write0, third, now, 2, b_part,
                     activations_of(step + 2), row_block_bytes, b_global, min(step + 2 + kAhead, last));
-        k_step<ENC, RB, true>(acc, a_now, current, b_read0, b_read1, b_write1, fourth, now, 3, b_part,
+        k_step<ENC, RB, !kWhole>(acc, a_now, current, b_read0, b_read1, b_write1, fourth, now, 3, b_part,
                     activations_of(step + 3), row_block_bytes, b_global, min(step + 3 + kAhead, last));
-        k_step<ENC, RB, !kHalves>(acc, a_now, current, b_read1, b_read0, b_write0, b0, next, 0, b_part,
+        k_step<ENC, RB, !kHalves && !kWhole>(acc, a_now, current, b_read1, b_read0, b_write0, after.b0, next, 0, b_part,
                     activations_of(step + 4), row_block_bytes, b_global, min(step + 4 + kAhead, last));
     };
     // The two header register sets swap roles every block; the loop body is two
@@ -745,8 +770,9 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     // around the back edge and the loads stay where they are written.
     int block = 0;
     if ((last_block & 1) == 0) {
-        block_of_four(0, header_even, header_odd);
-        header_even.load(b_global.first, min(2, last_block));
+        block_of_four(0, header_even, header_odd, set0, set1);
+        if constexpr (kWhole) set0 = set1;
+        header_even.load(b_global.first, min(2, last_block), b_part);
         NFN_FENCE();
         const BlockHeader<ENC> second = header_odd;
         header_odd = header_even;
@@ -754,11 +780,11 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
         block = 1;
     }
     while (block < last_block) {
-        block_of_four(block * 4, header_even, header_odd);
-        header_even.load(b_global.first, min(block + 2, last_block));
+        block_of_four(block * 4, header_even, header_odd, set0, set1);
+        header_even.load(b_global.first, min(block + 2, last_block), b_part);
         NFN_FENCE();
-        block_of_four(block * 4 + 4, header_odd, header_even);
-        header_odd.load(b_global.first, min(block + 3, last_block));
+        block_of_four(block * 4 + 4, header_odd, header_even, kWhole ? set1 : set0, kWhole ? set0 : set1);
+        header_odd.load(b_global.first, min(block + 3, last_block), b_part);
         NFN_FENCE();
         block += 2;
     }
@@ -855,18 +881,13 @@ __device__ __forceinline__ void low_step(v16f& acc, LowActivations& a, const std
     NFN_FENCE();
 }
 
-// The packed bytes of a block of a lane's rows, requested together: the steps' pieces of a row lie
-// in the same cache lines, which do not stay in the vector cache from one step to the next.
 template <std::uint32_t ENC>
 struct LowBlock {
     BlockHeader<ENC> header;
-    PackedSlice<ENC> s0, s1, s2, s3;  // (Q6_K: s0 the first half, s2 the second)
+    Slices<ENC> slices;
     __device__ __forceinline__ void load(const WeightRows& rows, int block, int part) {
-        header.load(rows.first, block);
-        s0.load(rows, block, 0, part);
-        if constexpr (!kHalfBlocks<ENC>) s1.load(rows, block, 1, part);
-        s2.load(rows, block, 2, part);
-        if constexpr (!kHalfBlocks<ENC>) s3.load(rows, block, 3, part);
+        header.load(rows.first, block, part);
+        slices.load(rows, block, part);
     }
 };
 
@@ -927,16 +948,16 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f16_low_kernel(
     const std::uint8_t* const read1 = read0 + kStageBytes;
     {
         std::uint32_t wa[4][2], wb[4][2];
-        even.s0.prepare_bits(even.header, 0, b_part);
-        even.s0.prepare_scales(even.header);
-        even.s0.template group_a<0>(wa[0]);
-        even.s0.template group_a<1>(wa[1]);
-        even.s0.template group_a<2>(wa[2]);
-        even.s0.template group_a<3>(wa[3]);
-        even.s0.template group_b<0>(wb[0]);
-        even.s0.template group_b<1>(wb[1]);
-        even.s0.template group_b<2>(wb[2]);
-        even.s0.template group_b<3>(wb[3]);
+        even.slices.b0.prepare_bits(even.header, 0, b_part);
+        even.slices.b0.prepare_scales(even.header);
+        even.slices.b0.template group_a<0>(wa[0]);
+        even.slices.b0.template group_a<1>(wa[1]);
+        even.slices.b0.template group_a<2>(wa[2]);
+        even.slices.b0.template group_a<3>(wa[3]);
+        even.slices.b0.template group_b<0>(wb[0]);
+        even.slices.b0.template group_b<1>(wb[1]);
+        even.slices.b0.template group_b<2>(wb[2]);
+        even.slices.b0.template group_b<3>(wb[3]);
         NFN_WRITE16(write0, wa[0][0], wa[0][1], wa[1][0], wa[1][1]);
         NFN_WRITE16(write0 + 16, wa[2][0], wa[2][1], wa[3][0], wa[3][1]);
         NFN_WRITE16(write0 + kLowSecondRun<ENC>, wb[0][0], wb[0][1], wb[1][0], wb[1][1]);
@@ -949,12 +970,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f16_low_kernel(
         const int step = 4 * block;
         next.load(b_global, min(block + 1, last_block), b_part);
         NFN_FENCE();
-        low_step<ENC>(acc, a0, read0, write1, kHalves ? now.s0 : now.s1, now.header, 1, b_part,
+        low_step<ENC>(acc, a0, read0, write1, kHalves ? now.slices.b0 : now.slices.b1, now.header, 1, b_part,
                           activations_of(step + 4));
-        low_step<ENC>(acc, a1, read1, write0, now.s2, now.header, 2, b_part, activations_of(step + 5));
-        low_step<ENC>(acc, a2, read0, write1, kHalves ? now.s2 : now.s3, now.header, 3, b_part,
+        low_step<ENC>(acc, a1, read1, write0, kHalves ? now.slices.b1 : now.slices.b2, now.header, 2, b_part, activations_of(step + 5));
+        low_step<ENC>(acc, a2, read0, write1, kHalves ? now.slices.b1 : now.slices.b3, now.header, 3, b_part,
                           activations_of(step + 6));
-        low_step<ENC>(acc, a3, read1, write0, next.s0, next.header, 0, b_part, activations_of(step + 7));
+        low_step<ENC>(acc, a3, read1, write0, next.slices.b0, next.header, 0, b_part, activations_of(step + 7));
     };
     for (int block = 0; block <= last_block; block += 2) {
         block_of_four(block, even, odd);
