@@ -617,8 +617,8 @@ def prefill_extra(device, stream, steps: int, warmup: int) -> dict:
                     "tokens/s": round(rows / ms * 1e3, 1)}
     # The same gate projection at M = 512 through the generic v1 call, the only v1 call that
     # takes more than 16 rows.  It has no workspace argument, so it stays in the exact tier:
-    # float activations against weights decoded to float, on the float matrix instruction
-    # (256 flop per cycle and compute unit, a sixteenth of the fp16 one).
+    # float activations, cut into three exact bf16 terms, against the weights' codes on the bf16
+    # matrix instruction (frac_mfma_f32: of the float one's 256 flop per cycle and compute unit).
     rows = 512
     x = torch.from_numpy(kquant.synthetic_activations(31, rows, MODEL_DIM)).to(device)
     ms = time_replays(lambda: tile_ops.linear(gate, x), 5, 2)
