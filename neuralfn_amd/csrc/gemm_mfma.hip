@@ -1152,8 +1152,13 @@ std::int64_t gemm_f16_workspace_bytes(std::int64_t rows, std::int64_t input_dim,
                                       std::int64_t output_dim) {
     // the activations, then one copy of the output per K share of a split
     // launch (the encoding with the most shares bounds the others)
-    const int shares = plan(kEncQ4K, rows, output_dim, input_dim).shares;
-    return activation_bytes(rows, input_dim) + (shares > 1 ? shares * rows * output_dim * 4 : 0) + 256;
+    const auto needed = [&](std::int64_t count) {
+        const int shares = plan(kEncQ4K, count, output_dim, input_dim).shares;
+        return activation_bytes(count, input_dim) + (shares > 1 ? shares * count * output_dim * 4 : 0) + 256;
+    };
+    // what serves a long chunk serves a short one behind it
+    const std::int64_t own = needed(rows), few = rows > kLowRows ? needed(kLowRows) : 0;
+    return own > few ? own : few;
 }
 
 void gemm_f16_plan(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,

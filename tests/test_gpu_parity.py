@@ -1519,6 +1519,11 @@ def test_prefill_gemm_plans():
     # A K too short for shares: 256-row tiles from half a workgroup a unit on.
     assert tile_ops.gemm_plan(kquant.Q4_K, 512, 4096, 6656) == (128, 1)
     assert tile_ops.gemm_plan(kquant.Q4_K, 700, 4096, 6656) == (256, 1)
+    # A workspace for a longer chunk serves a chunk of few rows, which takes more shares.
+    query = tile_ops.load().nfn_mi355_k_quant_gemm_workspace_bytes_v1
+    for in_dim, out_dim in ((256, 17), (4096, 6656), (6656, 256), (6656, 16384), (16384, 6656)):
+        few = max(query(rows, in_dim, out_dim, tile_ops.GEMM_F16) for rows in (1, 17, 32))
+        assert all(query(rows, in_dim, out_dim, tile_ops.GEMM_F16) >= few for rows in (33, 64, 128, 256, 300, 4096))
     # A narrow projection (the K and V projections of the workload): small tiles, short shares.
     assert tile_ops.gemm_plan(kquant.Q4_K, 1024, 6656, 256) == (128, 4)
     assert tile_ops.gemm_plan(kquant.Q6_K, 2048, 6656, 256) == (128, 4)
