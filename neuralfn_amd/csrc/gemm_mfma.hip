@@ -71,7 +71,7 @@ struct __attribute__((packed, aligned(2))) Chunk8 {
 // (rows past the end are zeros), in one launch that reads the input once.
 // ---------------------------------------------------------------------------
 
-// One wave per row, four rows per workgroup.  A lane owns groups of eight
+// A lane owns groups of eight
 // consecutive columns (one 16-byte piece of the fp16 copy each); rows of up to
 // 8,192 columns stay in the lane's registers between the search for the row's
 // largest magnitude and the conversion, wider rows are read again (from L2).
@@ -82,6 +82,9 @@ struct __attribute__((packed, aligned(2))) Chunk8 {
 // are the ones a round-robin placement over the eight XCDs puts on the same
 // XCD (workgroup w lands on XCD w % 8), so that the 16-byte pieces they
 // scatter into the same cache lines merge in one L2 before going to memory.
+// Rows of up to 8,192 columns take four waves each, for the loads in flight of a short prompt
+// (6,656 columns, a wave a row: 17 rows 7.6 -> 4.5 us, 333 rows 8.6 -> 6.2, 4,096 rows 52 -> 45),
+// wider ones two (four: 1,024 rows of 16,384 23.0 -> 23.8).
 // SPLIT waves share a row (each takes a contiguous part of its columns and they exchange
 // their maxima through LDS): rows of up to 16,384 columns still fit the registers.
 template <int HELD, int SPLIT>  // HELD: 8-column groups a lane keeps in registers; 0 = read the row twice
@@ -999,6 +1002,9 @@ struct ShareSums {
     std::int64_t count[kMaxProjections];
     int shares[kMaxProjections];
 };
+// PER outputs a thread, all of whose loads are under way together: one where the workgroups are few
+// anyway, four beyond (333 rows of 16,384 -> 6,656 in four shares 11.4 -> 8.7 us).
+template <int PER>
 __global__ __launch_bounds__(256) void sum_shares_kernel(ShareSums sums) {
     float* output = sums.output[0];
     const float* partials = sums.partials[0];
@@ -1013,13 +1019,20 @@ __global__ __launch_bounds__(256) void sum_shares_kernel(ShareSums sums) {
             shares = sums.shares[i];
         }
     }
-    const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
-    for (std::int64_t index = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-         index < count; index += stride) {
-        float total = output[index];
-#pragma unroll 4
-        for (int share = 1; share < shares; ++share) total += partials[(share - 1) * count + index];
-        output[index] = total;
+    for (std::int64_t base = static_cast<std::int64_t>(blockIdx.x) * (256 * PER) + threadIdx.x; base < count;
+         base += static_cast<std::int64_t>(gridDim.x) * (256 * PER)) {
+        float total[PER];
+#pragma unroll
+        for (int k = 0; k < PER; ++k) total[k] = output[min(base + 256 * k, count - 1)];
+#pragma unroll 8 / PER
+        for (int share = 1; share < shares; ++share) {
+#pragma unroll
+            for (int k = 0; k < PER; ++k) total[k] += partials[(share - 1) * count + min(base + 256 * k, count - 1)];
+        }
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            if (base + 256 * k < count) output[base + 256 * k] = total[k];
+        }
     }
 }
 
@@ -1132,9 +1145,14 @@ void launch_group(const GemmGroup& group, int count, bool tall, const std::uint8
         ++split;
     }
     if (split > 0) {
-        const std::int64_t blocks = (most + 1023) / 1024;
-        hipLaunchKernelGGL(sum_shares_kernel, dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096), split),
-                           dim3(256), 0, stream, sums);
+        const bool few = most <= 256 * 1024;
+        const std::int64_t blocks = (most + (few ? 255 : 1023)) / (few ? 256 : 1024);
+        const dim3 grid(static_cast<unsigned>(blocks < 4096 ? blocks : 4096), split);
+        if (few) {
+            hipLaunchKernelGGL(sum_shares_kernel<1>, grid, dim3(256), 0, stream, sums);
+        } else {
+            hipLaunchKernelGGL(sum_shares_kernel<4>, grid, dim3(256), 0, stream, sums);
+        }
     }
 }
 
@@ -1179,11 +1197,11 @@ void convert_gemm_activations(const float* input, std::int64_t rows, std::int64_
     float* inverse_scale = reinterpret_cast<float*>(activations + padded_rows(rows) * input_dim * 2);
     const std::int64_t groups = input_dim / 8;
     const unsigned whole_rows = static_cast<unsigned>(padded_rows(rows) / 4);  // a wave per row
-    if (groups <= 64 * 8) {
-        hipLaunchKernelGGL((prepare_activations_kernel<8, 1>), dim3(whole_rows), dim3(256), 0, stream,
+    if (groups <= 4 * 64 * 2) {
+        hipLaunchKernelGGL((prepare_activations_kernel<2, 4>), dim3(4 * whole_rows), dim3(256), 0, stream,
                            input, activations, inverse_scale, rows, input_dim);
-    } else if (groups <= 64 * 16) {
-        hipLaunchKernelGGL((prepare_activations_kernel<16, 1>), dim3(whole_rows), dim3(256), 0, stream,
+    } else if (groups <= 4 * 64 * 4) {
+        hipLaunchKernelGGL((prepare_activations_kernel<4, 4>), dim3(4 * whole_rows), dim3(256), 0, stream,
                            input, activations, inverse_scale, rows, input_dim);
     } else if (groups <= 2 * 64 * 16) {
         hipLaunchKernelGGL((prepare_activations_kernel<16, 2>), dim3(2 * whole_rows), dim3(256), 0,
