@@ -27,7 +27,7 @@
 // instead of one, and the matrix instructions of a step before its other work instead of between it,
 // made no difference.)  Measured at 4,096 -> 6,656, against the vector kernel (16 rows) and the
 // float matrix instruction (200, 512 rows) before: Q4_K 134 -> 16 us at 16 rows, 203 -> 69 at 200,
-// 311 -> 135 at 512; Q8_0 368 -> 27, 180 -> 87, 279 -> 169; F32 406 -> 30, 172 -> 131, 271 -> 254.
+// 311 -> 135 at 512; Q8_0 368 -> 27, 180 -> 81, 279 -> 162; F32 406 -> 30, 172 -> 131, 271 -> 254.
 //
 // The entry point, nfn_native_tile_linear_packed_weight_float32_v1, has no workspace argument
 // (neuralfn/csrc/native_train/tile_ops.h:614-620; reference kernel
@@ -97,6 +97,22 @@ __device__ __forceinline__ void codes_to_bf16(std::uint32_t bytes, float offset,
     low = upper_halves(q0, q1);
     high = upper_halves(q2, q3);
 }
+// ... signed ones: one instruction a code, which takes the byte with its sign (written out: from
+// plain conversions the compiler narrows the loads and runs out of registers).  200 rows 4,096 -> 6,656
+// Q8_0 89 -> 85 us; Q6_K, whose codes would take two more instructions to become signed bytes,
+// gains 4 % in the large form and loses 5 % in the small one and keeps the offset.
+#define NFN_SIGNED_BYTE(out, word, byte) \
+    asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_" #byte : "=v"(out) : "v"(word))
+__device__ __forceinline__ void signed_codes_to_bf16(std::uint32_t bytes, std::uint32_t& low, std::uint32_t& high) {
+    float q0, q1, q2, q3;
+    NFN_SIGNED_BYTE(q0, bytes, 0);
+    NFN_SIGNED_BYTE(q1, bytes, 1);
+    NFN_SIGNED_BYTE(q2, bytes, 2);
+    NFN_SIGNED_BYTE(q3, bytes, 3);
+    low = upper_halves(q0, q1);
+    high = upper_halves(q2, q3);
+}
+#undef NFN_SIGNED_BYTE
 
 // -----------------------------------------------------------------------------------------------
 // What a lane holds of one weight row for 64 columns (a unit: two steps of 32).  The lane's
@@ -230,8 +246,7 @@ struct Unit<kEncQ8_0> {
         d[1] = t.second;
     }
     __device__ __forceinline__ void words(int step, int chunk, int word, std::uint32_t& even, std::uint32_t& odd) const {
-        // (flipping the sign bit turns the code q into the byte q + 128)
-        codes_to_bf16(codes[step][2 * chunk + word] ^ 0x80808080u, 128.0f, even, odd);
+        signed_codes_to_bf16(codes[step][2 * chunk + word], even, odd);
     }
     __device__ __forceinline__ float scale(int step, int) const { return half_bits_to_float(d[step]); }
     __device__ __forceinline__ float minimum(int) const { return 0.0f; }
