@@ -187,8 +187,8 @@ __device__ __forceinline__ void for_each_piece(F&& f, std::integer_sequence<int,
 
 // Calls take(row, sums) for the weight rows `first`, `first + step`, ... below `output_dim`, two at a
 // time (rows 2 p and 2 p + 1); sums[r]: this wave's total for input row r, in every lane.  A row's
-// sum does not depend on the launch: lane l adds the units l, l + 64, ... in rising order, four
-// columns at a time, and the lanes meet in a butterfly.
+// sum does not depend on the launch: lane l adds the units l, l + 64, ... in rising order, the even
+// and the odd columns in a chain each, and the lanes meet in a butterfly.
 template <std::uint32_t ENC, int R, typename Take>
 __device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__ data, std::int64_t row_stride,
                                                 std::int64_t output_dim, std::int64_t input_dim,
@@ -208,7 +208,7 @@ __device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__
     };
     load(now, first_pair, 0);
     for (std::int64_t pair = first_pair; pair < end_pair; pair += pair_step) {
-        float sums[kExactPair][R] = {};
+        float sums[kExactPair][R][2] = {};  // even and odd columns: shorter chains, smaller errors
         for (int turn = 0; turn < turns; ++turn) {
             const bool more = turn + 1 < turns;
             // (unconditional: behind the last pair its own bytes are read again)
@@ -230,7 +230,7 @@ __device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__
 #pragma unroll
                         for (int k = 0; k < kExactPair; ++k) {
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) sums[k][r] = fmaf(v[j], w[k][j], sums[k][r]);
+                            for (int j = 0; j < 4; ++j) sums[k][r][j & 1] = fmaf(v[j], w[k][j], sums[k][r][j & 1]);
                         }
                     }
                 };
@@ -244,7 +244,7 @@ __device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__
             const std::int64_t row = pair * kExactPair + k;
             float totals[R];
 #pragma unroll
-            for (int r = 0; r < R; ++r) totals[r] = wave_sum(sums[k][r]);
+            for (int r = 0; r < R; ++r) totals[r] = wave_sum(sums[k][r][0] + sums[k][r][1]);
             if (row < output_dim) take(row, totals);
         }
     }

@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kExactWaves * kWave) void dense_rows_kernel(
         };
 #pragma unroll
         for (int turn = 0; turn < kAhead; ++turn) load(held[turn], first + turn * stride);
-        float sums[kExactPair][R] = {};
+        float sums[kExactPair][R] = {}, odd_sums[kExactPair][R] = {};  // of the even and the odd columns
         for (int base = first; base < pieces; base += kAhead * stride) {
 #pragma unroll
             for (int turn = 0; turn < kAhead; ++turn) {
@@ -118,7 +118,10 @@ __global__ __launch_bounds__(kExactWaves * kWave) void dense_rows_kernel(
 #pragma unroll
                             for (int k = 0; k < kExactPair; ++k) {
 #pragma unroll
-                                for (int j = 0; j < 4; ++j) sums[k][r] = fmaf(v[j], w[k][4 * quad + j], sums[k][r]);
+                                for (int j = 0; j < 4; ++j) {
+                                    float& sum = (j & 1) != 0 ? odd_sums[k][r] : sums[k][r];
+                                    sum = fmaf(v[j], w[k][4 * quad + j], sum);
+                                }
                             }
                         }
                     }
@@ -128,7 +131,7 @@ __global__ __launch_bounds__(kExactWaves * kWave) void dense_rows_kernel(
 #pragma unroll
         for (int k = 0; k < kExactPair; ++k) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) sums[k][r] = wave_sum(sums[k][r]);
+            for (int r = 0; r < R; ++r) sums[k][r] = wave_sum(sums[k][r] + odd_sums[k][r]);
         }
         if constexpr (SPLIT == 1) {
             if (lane == 0) {
