@@ -8,7 +8,9 @@
 // descriptor is nine stores, the stream one call and an output one allocator call.
 //
 // Nothing is kept between calls: every descriptor is made from the weight's attributes as they
-// are at the call.  The interpreter lock is given up around the entry point, as ctypes does.
+// are at the call.  The interpreter lock is given up around the entry point, as ctypes does, and
+// around nothing else: whatever may raise (a tensor without storage has no data pointer) is
+// evaluated before.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -18,6 +20,7 @@
 #include <array>
 #include <cstring>
 #include <string>
+#include <type_traits>
 
 #include "../../../include/nfn_mi355_tile_ops.h"
 
@@ -221,14 +224,26 @@ struct Projections {
     }
 };
 
+// The interpreter lock, given up for a scope; whichever way the scope ends, it is held again.
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    Unlocked() = default;
+    ~Unlocked() { PyEval_RestoreThread(state); }
+    Unlocked(const Unlocked&) = delete;
+};
+
 // Runs an entry point without the interpreter lock; a status other than 0 raises what
-// tile_ops.check raises.
-template <typename F>
-void call(const char* operation, F&& entry) {
+// tile_ops.check raises.  The arguments are numbers and pointers, evaluated by the caller under
+// the lock: nothing that could raise or run Python is left for the region.
+template <typename... Parameters, typename... Arguments>
+void call(const char* operation, int (*entry)(Parameters...), Arguments... arguments) {
+    static_assert(((std::is_arithmetic_v<Arguments> || std::is_pointer_v<Arguments> ||
+                    std::is_null_pointer_v<Arguments>) && ...), "plain values only");
     int status;
-    Py_BEGIN_ALLOW_THREADS
-    status = entry();
-    Py_END_ALLOW_THREADS
+    {
+        const Unlocked unlocked;
+        status = entry(arguments...);
+    }
     if (status != 0) {
         PyObject* nothing = PyObject_CallFunction(check_callable, "is", status, operation);
         Py_XDECREF(nothing);
@@ -300,7 +315,7 @@ PyObject* multi_linear(Arguments a) {
                                     : lib.nfn_native_tile_k_quant_mmq_multi_linear_float32_v1;
         call(verifier ? "nfn_native_tile_k_quant_mmvq_multi_linear_float32_v1"
                       : "nfn_native_tile_k_quant_mmq_multi_linear_float32_v1",
-             [&] { return entry(p.pointers.data(), first, p.outputs.data(), p.count(), rows, scratch, scratch_bytes, stream); });
+             entry, p.pointers.data(), first, p.outputs.data(), p.count(), rows, scratch, scratch_bytes, stream);
     } else {
         const auto entry = gated ? (verifier ? lib.nfn_native_tile_k_quant_mmvq_multi_linear_gated_float32_v1
                                              : lib.nfn_native_tile_k_quant_mmq_multi_linear_gated_float32_v1)
@@ -310,7 +325,7 @@ PyObject* multi_linear(Arguments a) {
                                : "nfn_native_tile_k_quant_mmq_multi_linear_gated_float32_v1")
                    : (verifier ? "nfn_native_tile_k_quant_mmvq_multi_linear_swiglu_float32_v1"
                                : "nfn_native_tile_k_quant_mmq_multi_linear_swiglu_float32_v1"),
-             [&] { return entry(p.pointers.data(), first, second, p.outputs.data(), p.count(), rows, scratch, scratch_bytes, stream); });
+             entry, p.pointers.data(), first, second, p.outputs.data(), p.count(), rows, scratch, scratch_bytes, stream);
     }
     return p.take();
 }
@@ -326,8 +341,8 @@ PyObject* multi_linear_prequantized(Arguments a) {
                                 : lib.nfn_mi355_k_quant_mmq_multi_linear_prequantized_float32_v1;
     void* scratch = workspace.data_ptr();
     const std::int64_t scratch_bytes = workspace.numel();
-    call(verifier ? "mmvq_multi_linear_prequantized" : "mmq_multi_linear_prequantized",
-         [&] { return entry(p.pointers.data(), p.outputs.data(), p.count(), rows, scratch, scratch_bytes, stream); });
+    call(verifier ? "mmvq_multi_linear_prequantized" : "mmq_multi_linear_prequantized", entry, p.pointers.data(),
+         p.outputs.data(), p.count(), rows, scratch, scratch_bytes, stream);
     return p.take();
 }
 
@@ -338,10 +353,8 @@ PyObject* mmvq_linear(Arguments a) {
     const at::Tensor& x = tensor_of(a[1]);
     const at::Tensor& workspace = tensor_of(a[2]);
     Output out(a[3], 1, descriptor.output_dim, x.device());
-    call("mmvq_linear", [&] {
-        return lib.nfn_native_tile_k_quant_mmvq_linear_float32_v1(
-            &descriptor, floats_of(x), out.data, workspace.data_ptr(), workspace.numel(), stream);
-    });
+    call("mmvq_linear", lib.nfn_native_tile_k_quant_mmvq_linear_float32_v1, &descriptor, floats_of(x), out.data,
+         workspace.data_ptr(), workspace.numel(), stream);
     return out.take();
 }
 
@@ -353,10 +366,8 @@ PyObject* linear(Arguments a) {
     const std::int64_t rows = x.size(0);
     const float* bias = floats_or_null(a[2]);
     Output out(Py_None, rows, descriptor.output_dim, x.device());
-    call("linear_packed_weight", [&] {
-        return lib.nfn_native_tile_linear_packed_weight_float32_v1(&descriptor, floats_of(x), bias, out.data, rows,
-                                                                   a[2] != Py_None);
-    });
+    call("linear_packed_weight", lib.nfn_native_tile_linear_packed_weight_float32_v1, &descriptor, floats_of(x), bias,
+         out.data, rows, a[2] != Py_None);
     return out.take();
 }
 
@@ -366,9 +377,8 @@ PyObject* gate_up_swiglu(Arguments a) {
     const Descriptor gate = descriptor_of(a[0], stream), up = descriptor_of(a[1], stream);
     const at::Tensor& x = tensor_of(a[2]);
     Output out(a[3], 1, gate.output_dim, x.device());
-    call("gate_up_swiglu", [&] {
-        return lib.nfn_mi355_k_quant_mmvq_gate_up_swiglu_float32_v1(&gate, &up, floats_of(x), out.data, stream);
-    });
+    call("gate_up_swiglu", lib.nfn_mi355_k_quant_mmvq_gate_up_swiglu_float32_v1, &gate, &up, floats_of(x), out.data,
+         stream);
     return out.take();
 }
 
@@ -380,10 +390,8 @@ PyObject* gate_up_swiglu_rows(Arguments a) {
     const std::int64_t rows = integer_of(a[3]);
     const at::Tensor& workspace = tensor_of(a[4]);
     Output out(a[5], rows, gate.output_dim, workspace.device());
-    call("gate_up_swiglu_rows", [&] {
-        return lib.nfn_mi355_k_quant_mmq_gate_up_swiglu_float32_v1(&gate, &up, x, out.data, rows, workspace.data_ptr(),
-                                                                   workspace.numel(), stream);
-    });
+    call("gate_up_swiglu_rows", lib.nfn_mi355_k_quant_mmq_gate_up_swiglu_float32_v1, &gate, &up, x, out.data, rows,
+         workspace.data_ptr(), workspace.numel(), stream);
     return out.take();
 }
 
@@ -400,11 +408,9 @@ PyObject* dual_rms_add_capture(Arguments a) {
     const float first_eps = static_cast<float>(number_of(a[6])), second_eps = static_cast<float>(number_of(a[7]));
     Output hidden(Py_None, x), normalized(Py_None, x), captured(Py_None, x);
     if (a[8] == Py_None) {
-        call("dual_rms_add_capture", [&] {
-            return lib.nfn_native_tile_glimmer_dual_rms_add_capture_float32_v1(
-                floats_of(x), first.pointer, floats_of(residual), hidden.data, second.pointer, normalized.data,
-                captured.data, rows, width, first_eps, first_centered, second_eps, second_centered, stream);
-        });
+        call("dual_rms_add_capture", lib.nfn_native_tile_glimmer_dual_rms_add_capture_float32_v1, floats_of(x),
+             first.pointer, floats_of(residual), hidden.data, second.pointer, normalized.data, captured.data, rows,
+             width, first_eps, first_centered, second_eps, second_centered, stream);
     } else {
         const at::Tensor& workspace = tensor_of(a[8]);
         const bool verifier = truth_of(a[9]);
@@ -412,11 +418,10 @@ PyObject* dual_rms_add_capture(Arguments a) {
             : verifier ? lib.nfn_mi355_dual_rms_add_capture_mmvq_rows_float32_v1
                        : lib.nfn_mi355_dual_rms_add_capture_mmq_f16_float32_v1;
         call(rows == 1 ? "dual_rms_add_capture_mmvq_q8"
-             : verifier ? "dual_rms_add_capture_mmvq_rows" : "dual_rms_add_capture_mmq_f16", [&] {
-            return entry(floats_of(x), first.pointer, floats_of(residual), hidden.data, second.pointer,
-                         normalized.data, captured.data, rows, width, first_eps, first_centered, second_eps,
-                         second_centered, workspace.data_ptr(), workspace.numel(), stream);
-        });
+             : verifier ? "dual_rms_add_capture_mmvq_rows" : "dual_rms_add_capture_mmq_f16",
+             entry, floats_of(x), first.pointer, floats_of(residual), hidden.data, second.pointer, normalized.data,
+             captured.data, rows, width, first_eps, first_centered, second_eps, second_centered, workspace.data_ptr(),
+             workspace.numel(), stream);
     }
     return Py_BuildValue("(NNN)", hidden.take(), normalized.take(), captured.take());
 }
@@ -434,12 +439,10 @@ PyObject* dual_rms_multi_linear(Arguments a) {
     const float first_eps = static_cast<float>(number_of(a[7])), second_eps = static_cast<float>(number_of(a[8]));
     Output hidden(Py_None, x), normalized(Py_None, x), captured(Py_None, x);
     Projections p(a[2], a[9], 1, x.device(), stream);
-    call("dual_rms_mmvq_multi_linear", [&] {
-        return lib.nfn_mi355_dual_rms_mmvq_multi_linear_float32_v1(
-            floats_of(x), first.pointer, floats_of(residual), hidden.data, second.pointer, normalized.data,
-            captured.data, width, first_eps, first_centered, second_eps, second_centered, p.pointers.data(),
-            p.outputs.data(), p.count(), stream);
-    });
+    call("dual_rms_mmvq_multi_linear", lib.nfn_mi355_dual_rms_mmvq_multi_linear_float32_v1, floats_of(x),
+         first.pointer, floats_of(residual), hidden.data, second.pointer, normalized.data, captured.data, width,
+         first_eps, first_centered, second_eps, second_centered, p.pointers.data(), p.outputs.data(), p.count(),
+         stream);
     return Py_BuildValue("(NNNN)", hidden.take(), normalized.take(), captured.take(), p.take());
 }
 
@@ -465,10 +468,9 @@ PyObject* lm_head_argmax(Arguments a) {
         : at::empty({rows}, at::TensorOptions().dtype(at::kLong).device(x.device()));
     const at::Tensor maxima = a[4] != Py_None ? tensor_of(a[4])
         : at::empty({rows}, at::TensorOptions().dtype(at::kFloat).device(x.device()));
-    call("lm_head_argmax", [&] {
-        return lib.nfn_mi355_lm_head_argmax_v1(&descriptor, floats_of(x), static_cast<std::int64_t*>(indices.data_ptr()),
-                                               floats_of(maxima), rows, workspace.data_ptr(), workspace.numel(), stream);
-    });
+    call("lm_head_argmax", lib.nfn_mi355_lm_head_argmax_v1, &descriptor, floats_of(x),
+         static_cast<std::int64_t*>(indices.data_ptr()), floats_of(maxima), rows, workspace.data_ptr(),
+         workspace.numel(), stream);
     return Py_BuildValue("(NN)", THPVariable_Wrap(indices), THPVariable_Wrap(maxima));
 }
 
@@ -492,10 +494,8 @@ PyObject* gemm(Arguments a) {
     const int mode = static_cast<int>(integer_of(a[2]));
     const at::Tensor workspace = gemm_workspace(a[3], &descriptor, 1, rows, mode, x.device());
     Output out(a[4], rows, descriptor.output_dim, x.device());
-    call("k_quant_gemm", [&] {
-        return lib.nfn_mi355_k_quant_gemm_float32_v1(&descriptor, floats_of(x), out.data, rows, workspace.data_ptr(),
-                                                     workspace.numel(), mode, stream);
-    });
+    call("k_quant_gemm", lib.nfn_mi355_k_quant_gemm_float32_v1, &descriptor, floats_of(x), out.data, rows,
+         workspace.data_ptr(), workspace.numel(), mode, stream);
     return out.take();
 }
 
@@ -507,10 +507,8 @@ PyObject* gemm_multi(Arguments a) {
     const int mode = static_cast<int>(integer_of(a[2]));
     Projections p(a[0], a[4], rows, x.device(), stream);
     const at::Tensor workspace = gemm_workspace(a[3], p.descriptors.data(), p.count(), rows, mode, x.device());
-    call("k_quant_gemm_multi", [&] {
-        return lib.nfn_mi355_k_quant_gemm_multi_float32_v1(p.pointers.data(), floats_of(x), p.outputs.data(), p.count(),
-                                                           rows, workspace.data_ptr(), workspace.numel(), mode, stream);
-    });
+    call("k_quant_gemm_multi", lib.nfn_mi355_k_quant_gemm_multi_float32_v1, p.pointers.data(), floats_of(x),
+         p.outputs.data(), p.count(), rows, workspace.data_ptr(), workspace.numel(), mode, stream);
     return p.take();
 }
 
@@ -527,19 +525,15 @@ PyObject* qk_norm_scale_rope(Arguments a) {
     const std::uint32_t layout = static_cast<std::uint32_t>(integer_of(a[8]));
     const bool rope = truth_of(a[9]), query_centered = truth_of(a[10]), key_centered = truth_of(a[11]);
     if (query.dim() == 3) {
-        call("qk_norm_scale_rope_batch", [&] {
-            return lib.nfn_native_tile_glimmer_qk_norm_scale_rope_batch_float32_v1(
-                floats_of(query), floats_of(key), query_weight.pointer, key_weight.pointer, query.size(0),
-                query.size(1), key.size(1), query.size(2), eps, query_centered, key_centered, scale, position, theta,
-                layout, rope, stream);
-        });
+        call("qk_norm_scale_rope_batch", lib.nfn_native_tile_glimmer_qk_norm_scale_rope_batch_float32_v1,
+             floats_of(query), floats_of(key), query_weight.pointer, key_weight.pointer, query.size(0), query.size(1),
+             key.size(1), query.size(2), eps, query_centered, key_centered, scale, position, theta, layout, rope,
+             stream);
     } else {
         if (query.dim() != 2) raise(PyExc_ValueError, "query is [heads, head_dim] or [rows, heads, head_dim]");
-        call("qk_norm_scale_rope", [&] {
-            return lib.nfn_native_tile_glimmer_qk_norm_scale_rope_float32_v1(
-                floats_of(query), floats_of(key), query_weight.pointer, key_weight.pointer, query.size(0), key.size(0),
-                query.size(1), eps, query_centered, key_centered, scale, position, theta, layout, rope, stream);
-        });
+        call("qk_norm_scale_rope", lib.nfn_native_tile_glimmer_qk_norm_scale_rope_float32_v1, floats_of(query),
+             floats_of(key), query_weight.pointer, key_weight.pointer, query.size(0), key.size(0), query.size(1), eps,
+             query_centered, key_centered, scale, position, theta, layout, rope, stream);
     }
     Py_RETURN_NONE;
 }
@@ -599,19 +593,17 @@ PyObject* fused_decode_attention(Arguments a) {
     void* scratch = split ? tensor_of(a[18]).data_ptr() : nullptr;
     const std::int64_t scratch_bytes = split ? tensor_of(a[18]).numel() : 0;
     if (split && device_position) {
-        call("fused_decode_attention_split_device_position", [&] {
-            return lib.nfn_mi355_fused_decode_attention_split_device_position_v1(&d, where, window, scratch, scratch_bytes);
-        });
+        call("fused_decode_attention_split_device_position",
+             lib.nfn_mi355_fused_decode_attention_split_device_position_v1, &d, where, window, scratch,
+             scratch_bytes);
     } else if (split) {
-        call("fused_decode_attention_split",
-             [&] { return lib.nfn_mi355_fused_decode_attention_split_v1(&d, scratch, scratch_bytes); });
+        call("fused_decode_attention_split", lib.nfn_mi355_fused_decode_attention_split_v1, &d, scratch,
+             scratch_bytes);
     } else if (device_position) {
-        call("fused_decode_attention_device_position", [&] {
-            return lib.nfn_native_tile_glimmer_fused_decode_attention_device_position_float32_v1(&d, where, window);
-        });
+        call("fused_decode_attention_device_position",
+             lib.nfn_native_tile_glimmer_fused_decode_attention_device_position_float32_v1, &d, where, window);
     } else {
-        call("fused_decode_attention",
-             [&] { return lib.nfn_native_tile_glimmer_fused_decode_attention_float32_v1(&d); });
+        call("fused_decode_attention", lib.nfn_native_tile_glimmer_fused_decode_attention_float32_v1, &d);
     }
     return out.take();
 }
@@ -646,10 +638,9 @@ PyObject* gqa_decode(Arguments a) {
     d.output = out.data;
     if (a[9] != Py_None) {
         const at::Tensor& workspace = tensor_of(a[9]);
-        call("gqa_decode_split",
-             [&] { return lib.nfn_mi355_gqa_decode_split_v1(&d, workspace.data_ptr(), workspace.numel()); });
+        call("gqa_decode_split", lib.nfn_mi355_gqa_decode_split_v1, &d, workspace.data_ptr(), workspace.numel());
     } else {
-        call("gqa_decode", [&] { return lib.nfn_native_tile_glimmer_gqa_decode_float32_v1(&d); });
+        call("gqa_decode", lib.nfn_native_tile_glimmer_gqa_decode_float32_v1, &d);
     }
     return out.take();
 }
@@ -687,11 +678,10 @@ PyObject* block_attention(Arguments a) {
     d.output = out.data;
     if (a[10] != Py_None) {
         const at::Tensor& workspace = tensor_of(a[10]);
-        call("block_attention_split", [&] {
-            return lib.nfn_mi355_dflash_block_attention_split_v1(&d, workspace.data_ptr(), workspace.numel());
-        });
+        call("block_attention_split", lib.nfn_mi355_dflash_block_attention_split_v1, &d, workspace.data_ptr(),
+             workspace.numel());
     } else {
-        call("block_attention", [&] { return lib.nfn_native_tile_dflash_block_attention_float32_v1(&d); });
+        call("block_attention", lib.nfn_native_tile_dflash_block_attention_float32_v1, &d);
     }
     return out.take();
 }
