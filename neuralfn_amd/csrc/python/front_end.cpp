@@ -185,13 +185,26 @@ at::Tensor new_floats(std::int64_t rows, std::int64_t width, c10::Device device)
     return at::empty({rows, width}, at::TensorOptions().dtype(at::kFloat).device(device));
 }
 
+// An owned reference.
+struct Reference {
+    PyObject* object = nullptr;
+    Reference() = default;
+    ~Reference() { Py_XDECREF(object); }
+    Reference(const Reference&) = delete;
+    PyObject* take() {
+        PyObject* taken = object;
+        object = nullptr;
+        return taken;
+    }
+};
+
 // The projections of one call: descriptors, output pointers and the Python object to return (the
 // caller's `outputs`, or a list of new tensors).
 struct Projections {
     c10::SmallVector<Descriptor, 4> descriptors;
     c10::SmallVector<const Descriptor*, 4> pointers;
     c10::SmallVector<float*, 4> outputs;
-    PyObject* result = nullptr;
+    Reference result;
 
     Projections(PyObject* weights, PyObject* given, std::int64_t rows, c10::Device device, void* stream) {
         const Sequence list(weights);
@@ -203,25 +216,19 @@ struct Projections {
             if (targets.size() < count) raise(PyExc_ValueError, "an output for every weight is expected");
             for (Py_ssize_t i = 0; i < count; ++i) outputs.push_back(floats_of(tensor_of(targets[i])));
             Py_INCREF(given);
-            result = given;
+            result.object = given;
             return;
         }
-        result = PyList_New(count);
-        if (result == nullptr) throw Raised{};
+        result.object = PyList_New(count);
+        if (result.object == nullptr) throw Raised{};
         for (Py_ssize_t i = 0; i < count; ++i) {
             const at::Tensor out = new_floats(rows, descriptors[i].output_dim, device);
             outputs.push_back(floats_of(out));
-            PyList_SET_ITEM(result, i, THPVariable_Wrap(out));
+            PyList_SET_ITEM(result.object, i, THPVariable_Wrap(out));
         }
     }
-    ~Projections() { Py_XDECREF(result); }
-    Projections(const Projections&) = delete;
     std::int64_t count() const { return static_cast<std::int64_t>(descriptors.size()); }
-    PyObject* take() {
-        PyObject* taken = result;
-        result = nullptr;
-        return taken;
-    }
+    PyObject* take() { return result.take(); }
 };
 
 // The interpreter lock, given up for a scope; whichever way the scope ends, it is held again.

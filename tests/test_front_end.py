@@ -129,6 +129,20 @@ stop.set()
 thread.join()
 functions = {name for name in dir(front) if not name.startswith("_")} - {"bind", "entry_points", "stream_handle"}
 assert functions == covered, functions ^ covered
+# outputs that were made before an allocation is refused are given back
+endless = tile_ops.PackedWeight(kquant.Q4_K, 1 << 50, 256, w.data)
+def refused():
+    try:
+        tile_ops.multi_linear([w, endless], x, scratch)
+    except RuntimeError:
+        return
+    raise AssertionError("an endless output was allocated")
+for _ in range(10):
+    refused()
+blocks = sys.getallocatedblocks()
+for _ in range(300):
+    refused()
+assert sys.getallocatedblocks() - blocks < 150, sys.getallocatedblocks() - blocks
 print("all refused")
 """
 
