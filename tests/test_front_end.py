@@ -23,7 +23,7 @@ inline NullStream getCurrentHIPStream() { return {}; }
 """
 
 PROGRAM = r"""
-import ctypes, importlib.machinery, importlib.util, sys, threading
+import ctypes, gc, importlib.machinery, importlib.util, sys, threading
 import torch
 sys.path.insert(0, sys.argv[1])
 from neuralfn_amd import engine_ops, kquant, tile_ops
@@ -137,12 +137,12 @@ def refused():
     except RuntimeError:
         return
     raise AssertionError("an endless output was allocated")
-for _ in range(10):
+def held():
+    return sum(type(item) is torch.Tensor for item in gc.get_objects())
+before = held()
+for _ in range(20):
     refused()
-blocks = sys.getallocatedblocks()
-for _ in range(300):
-    refused()
-assert sys.getallocatedblocks() - blocks < 150, sys.getallocatedblocks() - blocks
+assert held() == before, held() - before
 print("all refused")
 """
 
