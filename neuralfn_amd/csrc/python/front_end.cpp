@@ -15,6 +15,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <array>
@@ -705,8 +706,8 @@ PyObject* guarded(PyObject*, PyObject* const* arguments, Py_ssize_t count) {
         return Function(arguments);
     } catch (const Raised&) {
         return nullptr;
-    } catch (const std::exception& error) {
-        PyErr_SetString(PyExc_RuntimeError, error.what());
+    } catch (...) {  // as torch's own bindings raise it (no memory: torch.OutOfMemoryError)
+        torch::translate_exception_to_python(std::current_exception());
         return nullptr;
     }
 }
@@ -739,8 +740,8 @@ PyObject* bind(PyObject*, PyObject* arguments) {
 PyObject* stream_handle(PyObject*, PyObject*) {
     try {
         return PyLong_FromVoidPtr(current_stream());
-    } catch (const std::exception& error) {
-        PyErr_SetString(PyExc_RuntimeError, error.what());
+    } catch (...) {
+        torch::translate_exception_to_python(std::current_exception());
         return nullptr;
     }
 }

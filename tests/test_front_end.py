@@ -143,6 +143,14 @@ before = held()
 for _ in range(20):
     refused()
 assert held() == before, held() - before
+# the kinds of exception that torch's own methods raise
+for function in (lambda: tile_ops.linear(w, torch.tensor(0.0)), lambda: tile_ops.gemm(w, torch.tensor(0.0), workspace=scratch)):
+    try:
+        function()
+    except IndexError:
+        pass
+    else:
+        raise AssertionError("a tensor without rows is not refused")
 print("all refused")
 """
 
