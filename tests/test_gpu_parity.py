@@ -223,6 +223,35 @@ def test_exact_linear_of_infinities_nan_and_large_activations(cuda, oracle, enco
         assert normalised_error(y[row], expected[row]) <= 1e-5, row
 
 
+@pytest.mark.parametrize("exponent", [-33, -35, -36, -37])
+@pytest.mark.parametrize("rows,out_dim,in_dim", [(3, 67, 512), (5, 67, 512), (60, 5000, 256), (100, 6600, 256), (200, 6600, 256)])
+@pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
+def test_exact_linear_of_tiny_operands(cuda, oracle, encoding, rows, out_dim, in_dim, exponent):
+    """Activations, and float weights, down to the smallest normal floats: a bf16 term of one of
+    them would be below 2^-133, the smallest bf16 number.  Products and sums are normal floats, so
+    that the bound is that of the edges' test, plus half a unit of the smallest float."""
+    tiny = np.float32(10.0) ** np.float32(exponent)
+    x = kquant.synthetic_activations(6 + rows, rows, in_dim) + np.float32(0.3)
+    w = kquant.synthetic_weights(5 + rows, out_dim, in_dim, 1.0)
+    packed = kquant.quantize(encoding, w)
+    decoded = oracle.dequantize(encoding, packed, out_dim, in_dim).reshape(out_dim, in_dim).astype(np.float64)
+
+    def check(packed, decoded, x):
+        weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+        y = tile_ops.linear(weight, to_device(x, cuda)).cpu().numpy().astype(np.float64)
+        expected = x.astype(np.float64) @ decoded.T
+        for row in range(rows):
+            assert np.max(np.abs(y[row] - expected[row])) <= 1e-5 * np.max(np.abs(expected[row])) + 2.0 ** -150, row
+
+    check(packed, decoded, x * tiny)
+    mixed = x * tiny
+    mixed[:, in_dim // 2:] *= np.float32(1e6)  # tiny next to ordinary ones
+    check(packed, decoded, mixed)
+    if encoding in (kquant.F32, kquant.BF16):
+        packed = kquant.quantize(encoding, w * tiny)
+        check(packed, oracle.dequantize(encoding, packed, out_dim, in_dim).reshape(out_dim, in_dim).astype(np.float64), x)
+
+
 # ------------------------------------------------------------ public Q8_1 path
 
 def crafted_q8_input(rows, in_dim):
