@@ -405,27 +405,91 @@ __device__ __forceinline__ void load_unit(Unit<ENC>& into, const std::uint8_t* r
     }
 }
 
-// One output the plain way: decoded weights times the activations as they are.
-__device__ __forceinline__ float plain_dot(std::uint32_t encoding, const std::uint8_t* row, const float* x,
-                                           std::int64_t input_dim) {
-    float total = 0.0f;
-#pragma unroll 1
-    for (std::int64_t column = 0; column < input_dim; ++column) {
-        total = fmaf(x[column], weight_value(encoding, row, column), total);
+// 32 columns of one weight row, decoded as the dequantize entry point does; infinite scales too.
+template <std::uint32_t ENC>
+struct DecodedPiece {
+    u32x4_a2 codes[ENC == kEncF32 ? 8 : ENC == kEncBF16 ? 4 : 2], fifth[2];
+    float scale[2], offset;
+    int shift, high_shift;
+    __device__ __forceinline__ void load(const std::uint8_t* row, int piece) {
+        if constexpr (ENC == kEncF32 || ENC == kEncBF16) {
+            constexpr int kLoads = ENC == kEncF32 ? 8 : 4;
+#pragma unroll
+            for (int k = 0; k < kLoads; ++k) {
+                codes[k] = *reinterpret_cast<const u32x4_a2*>(row + (static_cast<std::int64_t>(piece) * kLoads + k) * 16);
+            }
+        } else if constexpr (ENC == kEncQ8_0) {
+            const std::uint8_t* block = row + static_cast<std::int64_t>(piece) * 34;
+            scale[0] = load_half(block);
+            codes[0] = *reinterpret_cast<const u32x4_a2*>(block + 2);
+            codes[1] = *reinterpret_cast<const u32x4_a2*>(block + 18);
+        } else if constexpr (ENC == kEncQ6K) {
+            const std::uint8_t* block = row + (piece >> 3) * 210;
+            const int half = (piece >> 2) & 1, quarter = piece & 3;
+            const float d = load_half(block + 208);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                codes[k] = *reinterpret_cast<const u32x4_a2*>(block + half * 64 + (quarter & 1) * 32 + 16 * k);
+                fifth[k] = *reinterpret_cast<const u32x4_a2*>(block + 128 + half * 32 + 16 * k);
+                scale[k] = d * static_cast<float>(static_cast<std::int8_t>(block[192 + half * 8 + quarter * 2 + k]));
+            }
+            shift = 4 * (quarter >> 1);
+            high_shift = 2 * quarter;
+        } else {
+            const std::uint8_t* block = row + (piece >> 3) * static_cast<int>(block_bytes(ENC));
+            int sc, m;
+            k_scale_min(block + 4, piece & 7, &sc, &m);
+            scale[0] = load_half(block) * static_cast<float>(sc);
+            offset = load_half(block + 2) * static_cast<float>(m);
+            const std::uint8_t* source = block + (ENC == kEncQ5K ? 48 : 16) + ((piece >> 1) & 3) * 32;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                codes[k] = *reinterpret_cast<const u32x4_a2*>(source + 16 * k);
+                if constexpr (ENC == kEncQ5K) fifth[k] = *reinterpret_cast<const u32x4_a2*>(block + 16 + 16 * k);
+            }
+            shift = 4 * (piece & 1);
+            high_shift = piece & 7;
+        }
     }
-    return total;
-}
+    // columns 4 quad .. 4 quad + 3
+    __device__ __forceinline__ void decode(int quad, float (&w)[4]) const {
+        if constexpr (ENC == kEncF32) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) w[j] = __uint_as_float(codes[quad][j]);
+        } else if constexpr (ENC == kEncBF16) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const std::uint32_t two = codes[quad >> 1][2 * (quad & 1) + (j >> 1)];
+                w[j] = __uint_as_float(j & 1 ? two & 0xffff0000u : two << 16);
+            }
+        } else {
+            const std::uint32_t word = codes[quad >> 2][quad & 3];
+            const std::uint32_t high = ENC == kEncQ5K || ENC == kEncQ6K ? fifth[quad >> 2][quad & 3] : 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (ENC == kEncQ8_0) {
+                    w[j] = scale[0] * static_cast<float>(static_cast<std::int8_t>(word >> (8 * j)));
+                } else if constexpr (ENC == kEncQ6K) {
+                    const int q = static_cast<int>((word >> (shift + 8 * j) & 15u) | (high >> (high_shift + 8 * j) & 3u) << 4);
+                    w[j] = scale[quad >> 2] * static_cast<float>(q - 32);
+                } else {
+                    int q = static_cast<int>(word >> (shift + 8 * j) & 15u);
+                    if constexpr (ENC == kEncQ5K) q |= static_cast<int>(high >> (high_shift + 8 * j) & 1u) << 4;
+                    w[j] = scale[0] * static_cast<float>(q) - offset;
+                }
+            }
+        }
+    }
+};
 
 // The sums of a tile's waves meet, 32 x 32 outputs at a time: register r of lane l is row
 // 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.  GROUPS sets of sums, set g in meeting[g]; the
-// workgroup's wave `wave` of WAVES adds up and stores its registers' worth.
-// A sum that is not finite is taken again the plain way: infinity less its own upper half is NaN
-// where the product with the weight is infinite, and the lifted products with the codes leave the
-// float range before those with the weights do.
+// workgroup's wave `wave` of WAVES adds up and stores its registers' worth.  Sums that are not
+// finite are left for take_again: a bit a lane, the word of the pass's part p in `again` of lane
+// pass * 16 / WAVES + p.
 template <std::uint32_t ENC, int GROUPS, int WAVES>
-__device__ __forceinline__ void add_up_and_store(const float (*meeting)[16 * kWave], int wave, int lane,
-                                                 const std::uint8_t* data, std::int64_t row_stride, const float* input,
-                                                 std::int64_t input_dim, const float* bias, float* output,
+__device__ __forceinline__ void add_up_and_store(const float (*meeting)[16 * kWave], int pass, std::uint64_t& again,
+                                                 int wave, int lane, const float* bias, float* output,
                                                  std::int64_t rows, std::int64_t output_dim, std::int64_t row0,
                                                  std::int64_t column) {
 #pragma unroll
@@ -439,10 +503,62 @@ __device__ __forceinline__ void add_up_and_store(const float (*meeting)[16 * kWa
 #pragma unroll
             for (int g = 0; g < width; ++g) sums[g] += sums[g + width];
         }
-        float total = sums[0] * kLower<ENC>;
+        const float total = sums[0] * kLower<ENC>;
         const std::int64_t row = row0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row < rows && column < output_dim) {
-            if (!isfinite(total)) total = plain_dot(ENC, data + column * row_stride, input + row * input_dim, input_dim);
+        const bool exists = row < rows && column < output_dim, finite = isfinite(total);
+        if (exists && finite) output[row * output_dim + column] = total + (bias != nullptr ? bias[column] : 0.0f);
+        const std::uint64_t left = __ballot(exists && !finite);
+        again = lane == pass * (16 / WAVES) + part ? left : again;
+    }
+}
+
+// One output from the decoded weights and the activations as they are.  The lanes of a wave take
+// different outputs; it ends early when all of them are NaN, which they stay.
+template <std::uint32_t ENC>
+__device__ __forceinline__ float decoded_dot(const std::uint8_t* row, const float* x, std::int64_t input_dim) {
+    float even = 0.0f, odd = 0.0f;
+    const auto take = [&](const float (&w)[4], const float* at) {
+        const f32x4_a4 v = *reinterpret_cast<const f32x4_a4*>(at);
+        even = fmaf(v[0], w[0], even);
+        odd = fmaf(v[1], w[1], odd);
+        even = fmaf(v[2], w[2], even);
+        odd = fmaf(v[3], w[3], odd);
+    };
+    const int pieces = static_cast<int>(input_dim / 32);
+#pragma unroll 1
+    for (int piece = 0; piece < pieces; ++piece) {
+        DecodedPiece<ENC> weights;
+        weights.load(row, piece);
+#pragma unroll
+        for (int quad = 0; quad < 8; ++quad) {
+            float w[4];
+            weights.decode(quad, w);
+            take(w, x + 32 * static_cast<std::int64_t>(piece) + 4 * quad);
+        }
+        if (__ballot(!isnan(even + odd)) == 0) break;
+    }
+    return even + odd;
+}
+
+// The outputs that a wave left in `again`, taken from the decoded weights: infinity less its own upper half is NaN where the product with the
+// weight is infinite, and the lifted products leave the float range (activations above some 2^90 with
+// codes, products above 2^80 with float weights) before those with the weights do.
+// place(pass, r, row, column): the row and column of this lane's bit.
+// 4,096 -> 6,656 at 200 rows (Q8_0 / Q4_K, 87 / 75 us from Python): with a NaN in one row 90 / 82 us, in
+// every row 123 / 97; an infinity or activations of 3e37 in one row 207 / 231, in every row 3.6 / 3.4 ms
+// (a byte and a weight at a time: 1.1 / 1.9 ms for one row of either kind, 29 / 64 for all).
+template <std::uint32_t ENC, int WAVES, typename Place>
+__device__ __forceinline__ void take_again(std::uint64_t again, int wave, int lane, const std::uint8_t* data,
+                                           std::int64_t row_stride, const float* input, std::int64_t input_dim,
+                                           const float* bias, float* output, std::int64_t output_dim, Place&& place) {
+    for (std::uint64_t holders = __ballot(again != 0); holders != 0; holders &= holders - 1) {
+        const int index = __builtin_ctzll(holders);
+        const std::uint32_t low = __builtin_amdgcn_readlane(static_cast<std::uint32_t>(again), index);
+        const std::uint32_t high = __builtin_amdgcn_readlane(static_cast<std::uint32_t>(again >> 32), index);
+        if (((lane < 32 ? low : high) >> (lane & 31) & 1) != 0) {
+            std::int64_t row, column;
+            place(index / (16 / WAVES), index % (16 / WAVES) * WAVES + wave, row, column);
+            const float total = decoded_dot<ENC>(data + column * row_stride, input + row * input_dim, input_dim);
             output[row * output_dim + column] = total + (bias != nullptr ? bias[column] : 0.0f);
         }
     }
@@ -541,6 +657,7 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
             for (int n = 0; n < NT; ++n) now[n] = next[n];
         }
     }
+    std::uint64_t again = 0;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
 #pragma unroll
@@ -549,10 +666,15 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
 #pragma unroll
             for (int r = 0; r < 16; ++r) meeting[wave][r * kWave + lane] = acc[n][m][r];
             __syncthreads();
-            add_up_and_store<ENC, WAVES, WAVES>(meeting, wave, lane, data, row_stride, input, input_dim, bias, output,
-                                                rows, output_dim, row0 + 32 * m, col0 + 32 * n + inner);
+            add_up_and_store<ENC, WAVES, WAVES>(meeting, n * MT + m, again, wave, lane, bias, output, rows, output_dim,
+                                                row0 + 32 * m, col0 + 32 * n + inner);
         }
     }
+    take_again<ENC, WAVES>(again, wave, lane, data, row_stride, input, input_dim, bias, output, output_dim,
+                           [&](int pass, int r, std::int64_t& row, std::int64_t& column) {
+                               row = row0 + 32 * (pass % MT) + 8 * (r >> 2) + 4 * half + (r & 3);
+                               column = col0 + 32 * (pass / MT) + inner;
+                           });
 }
 
 // -- the large form --------------------------------------------------------------------------------
@@ -571,7 +693,7 @@ template <int MT>
 constexpr int kGroupBytes = 2 * kStepBytes<MT> + kSumBytes<MT>;
 template <int MT>
 constexpr int kLargeLds = kGroups * kGroupBytes<MT>;
-static_assert(kLargeLds<1> >= kGroups * kPartners * 16 * kWave * 4, "the waves' sums meet in the same memory");
+static_assert(kLargeLds<1> >= kLargeWaves * 16 * kWave * 4, "the waves' sums meet in the same memory");
 
 template <std::uint32_t ENC, int MT>
 __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
@@ -786,6 +908,7 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
 
     // meeting[group] of either partner's 32 x 32 outputs: partner p's sets lie behind each other
     float(*meeting)[16 * kWave] = reinterpret_cast<float(*)[16 * kWave]>(lds);
+    std::uint64_t again = 0;
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
 #pragma unroll
@@ -794,11 +917,15 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
 #pragma unroll
             for (int r = 0; r < 16; ++r) meeting[partner * kGroups + group][r * kWave + lane] = acc[n][m][r];
             __syncthreads();
-            add_up_and_store<ENC, kGroups, kGroups>(meeting + partner * kGroups, group, lane, data, row_stride, input,
-                                                    input_dim, bias, output, rows, output_dim, row0 + 32 * m,
-                                                    col0 + 32 * n + inner);
+            add_up_and_store<ENC, kGroups, kGroups>(meeting + partner * kGroups, n * MT + m, again, group, lane, bias,
+                                                    output, rows, output_dim, row0 + 32 * m, col0 + 32 * n + inner);
         }
     }
+    take_again<ENC, kGroups>(again, group, lane, data, row_stride, input, input_dim, bias, output, output_dim,
+                             [&](int pass, int r, std::int64_t& row, std::int64_t& column) {
+                                 row = row0 + 32 * (pass % MT) + 8 * (r >> 2) + 4 * half + (r & 3);
+                                 column = col0 + 32 * (pass / MT) + inner;
+                             });
 }
 
 template <std::uint32_t ENC, int MT>

@@ -223,6 +223,38 @@ def test_exact_linear_of_infinities_nan_and_large_activations(cuda, oracle, enco
         assert normalised_error(y[row], expected[row]) <= 1e-5, row
 
 
+@pytest.mark.parametrize("rows,out_dim,in_dim", [(5, 67, 512), (60, 5000, 256), (100, 6600, 256), (200, 6600, 256)])
+@pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
+def test_exact_linear_of_weights_that_are_not_finite(cuda, oracle, encoding, rows, out_dim, in_dim):
+    """Infinite block scales and minimums, infinite and NaN float weights, and rows of zeros among
+    the activations: what the products with the decoded weights give."""
+    packed = kquant.quantize(encoding, kquant.synthetic_weights(5 + rows, out_dim, in_dim)).copy()
+    row_bytes = kquant.row_stride_bytes(encoding, in_dim)
+    infinity, nan = (b"\x00\x7c", b"\x00\x7e")  # halves
+    if encoding == kquant.F32:
+        infinity, nan = (np.float32(v).tobytes() for v in (np.inf, np.nan))
+    elif encoding == kquant.BF16:
+        infinity, nan = (np.float32(v).tobytes()[2:] for v in (np.inf, np.nan))
+    scale = {kquant.Q6_K: 208}.get(encoding, 0)
+    minimum = {kquant.Q4_K: 2, kquant.Q5_K: 2}.get(encoding, scale)
+    for row, offset, value in ((1, scale, infinity), (2, minimum, infinity), (out_dim - 1, scale, nan)):
+        at = row * row_bytes + offset
+        packed[at:at + len(value)] = np.frombuffer(value, dtype=np.uint8)
+    x = kquant.synthetic_activations(6 + rows, rows, in_dim)
+    x[rows - 2] = 0.0
+    weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    y = tile_ops.linear(weight, to_device(x, cuda)).cpu().numpy()
+    w = oracle.dequantize(encoding, packed, out_dim, in_dim).reshape(out_dim, in_dim).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        expected = x.astype(np.float64) @ w.T
+    assert (~np.isfinite(expected)).sum(axis=0)[[1, 2, out_dim - 1]].min() > 0
+    assert np.array_equal(np.isnan(y), np.isnan(expected))
+    infinite = np.isinf(expected)
+    assert np.array_equal(np.isinf(y), infinite) and np.array_equal(y[infinite], expected[infinite])
+    finite = np.isfinite(expected)
+    assert normalised_error(y[finite], expected[finite]) <= 1e-5
+
+
 @pytest.mark.parametrize("exponent", [-33, -35, -36, -37])
 @pytest.mark.parametrize("rows,out_dim,in_dim", [(3, 67, 512), (5, 67, 512), (60, 5000, 256), (100, 6600, 256), (200, 6600, 256)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
