@@ -134,6 +134,18 @@ __device__ __forceinline__ float load_half(const std::uint8_t* p) {
     return half_bits_to_float(static_cast<std::uint32_t>(p[0]) | (static_cast<std::uint32_t>(p[1]) << 8));
 }
 
+// The four signed bytes of a word as floats, one instruction each, which takes the byte with its
+// sign (written out: from plain conversions the compiler narrows the loads and runs out of registers).
+#define NFN_SIGNED_BYTE(out, word, byte) \
+    asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_" #byte : "=v"(out) : "v"(word))
+__device__ __forceinline__ void signed_bytes(std::uint32_t word, float (&values)[4]) {
+    NFN_SIGNED_BYTE(values[0], word, 0);
+    NFN_SIGNED_BYTE(values[1], word, 1);
+    NFN_SIGNED_BYTE(values[2], word, 2);
+    NFN_SIGNED_BYTE(values[3], word, 3);
+}
+#undef NFN_SIGNED_BYTE
+
 // float -> bf16 bits, round to nearest even; a NaN stays a NaN.
 __device__ __forceinline__ std::uint16_t to_bf16(float value) {
     const std::uint32_t bits = __float_as_uint(value);

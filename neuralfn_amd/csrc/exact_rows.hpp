@@ -6,7 +6,9 @@
 // exact in float (at most 19 bits), and so is d * sc * q (at most 24), so that the fused form
 // rounds where the CPU engine's two products and a subtraction round
 // (neuralfn/csrc/native_gpt2/resident_glimmer.cpp:542-616).  A code byte becomes a float in one
-// instruction: 2.25 vector instructions a weight before the products with the input rows.
+// instruction: 2.25 vector instructions a weight before the products with the input rows.  Formats
+// without a minimum multiply signed codes, exactly: with the offset of the codes in a fused form an
+// infinite scale would give infinity less infinity where the weight is infinite.
 //
 // The input rows lie in LDS, 64 columns (a unit) at a pitch of 68 floats: a lane owns whole units,
 // and neighbouring lanes' 16-byte reads then fall into distinct banks.  A wave takes two weight
@@ -115,18 +117,20 @@ struct ExactUnit<kEncQ6K> {
         upper = (unit & 1) * 4;  // quarters 2 and 3 of the half block: high nibbles, high-bit pairs 2 and 3
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            scale[k] = half_bits_to_float(d) * static_cast<float>(static_cast<std::int8_t>(codes_of_scale >> (8 * k)));
+            scale[k] = half_bits_to_float(d) * 0.25f * static_cast<float>(static_cast<std::int8_t>(codes_of_scale >> (8 * k)));
         }
     }
     template <int I>
     __device__ __forceinline__ exact_f32x4 values() const {
         constexpr int kStep = I / 8, kWord = I % 8;
-        const std::uint32_t q = ((low[2 * kStep + kWord / 4][kWord % 4] >> upper) & 0x0f0f0f0fu) |
-            (((high[kWord / 4][kWord % 4] >> (upper + 2 * kStep)) & 0x03030303u) << 4);
+        // in every byte 4 (q - 32): the nibble in bits 2 to 5, the high bits above, their sign flipped
+        const std::uint32_t lower = low[2 * kStep + kWord / 4][kWord % 4], above = high[kWord / 4][kWord % 4];
+        const std::uint32_t q = (__builtin_rotateright32(lower, upper - 2) & 0x3c3c3c3cu) |
+            (__builtin_rotateright32(above, upper + 2 * kStep - 6) & 0xc0c0c0c0u);
         const float factor = scale[2 * kStep + kWord / 4];
         exact_f32x4 w;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = fmaf(factor, code_byte(q, j), -32.0f * factor);
+        for (int j = 0; j < 4; ++j) w[j] = factor * static_cast<float>(static_cast<std::int8_t>((q ^ 0x80808080u) >> (8 * j)));
         return w;
     }
 };
@@ -154,11 +158,11 @@ struct ExactUnit<kEncQ8_0> {
     template <int I>
     __device__ __forceinline__ exact_f32x4 values() const {
         constexpr int kStep = I / 8, kWord = I % 8;
-        const std::uint32_t q = (kStep == 0 ? __builtin_amdgcn_alignbyte(words[kWord + 1], words[kWord], 2)
-                                            : words[9 + kWord]) ^ 0x80808080u;  // the byte q + 128
+        float code[4];
+        signed_bytes(kStep == 0 ? __builtin_amdgcn_alignbyte(words[kWord + 1], words[kWord], 2) : words[9 + kWord], code);
         exact_f32x4 w;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = fmaf(scale[kStep], code_byte(q, j), -128.0f * scale[kStep]);
+        for (int j = 0; j < 4; ++j) w[j] = scale[kStep] * code[j];
         return w;
     }
 };

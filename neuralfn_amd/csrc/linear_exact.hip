@@ -106,22 +106,15 @@ __device__ __forceinline__ void codes_to_bf16(std::uint32_t bytes, float offset,
     low = upper_halves(q0, q1);
     high = upper_halves(q2, q3);
 }
-// ... signed ones: one instruction a code, which takes the byte with its sign (written out: from
-// plain conversions the compiler narrows the loads and runs out of registers).  200 rows 4,096 -> 6,656
-// Q8_0 89 -> 85 us; Q6_K, whose codes would take two more instructions to become signed bytes,
-// gains 4 % in the large form and loses 5 % in the small one and keeps the offset.
-#define NFN_SIGNED_BYTE(out, word, byte) \
-    asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_" #byte : "=v"(out) : "v"(word))
+// ... signed ones: one instruction a code.  200 rows 4,096 -> 6,656 Q8_0 89 -> 85 us; Q6_K, whose codes
+// would take two more instructions to become signed bytes, gains 4 % in the large form and loses 5 % in
+// the small one and keeps the offset.
 __device__ __forceinline__ void signed_codes_to_bf16(std::uint32_t bytes, std::uint32_t& low, std::uint32_t& high) {
-    float q0, q1, q2, q3;
-    NFN_SIGNED_BYTE(q0, bytes, 0);
-    NFN_SIGNED_BYTE(q1, bytes, 1);
-    NFN_SIGNED_BYTE(q2, bytes, 2);
-    NFN_SIGNED_BYTE(q3, bytes, 3);
-    low = upper_halves(q0, q1);
-    high = upper_halves(q2, q3);
+    float q[4];
+    signed_bytes(bytes, q);
+    low = upper_halves(q[0], q[1]);
+    high = upper_halves(q[2], q[3]);
 }
-#undef NFN_SIGNED_BYTE
 
 // -----------------------------------------------------------------------------------------------
 // What a lane holds of one weight row for 64 columns (a unit: two steps of 32).  The lane's

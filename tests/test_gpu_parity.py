@@ -223,7 +223,7 @@ def test_exact_linear_of_infinities_nan_and_large_activations(cuda, oracle, enco
         assert normalised_error(y[row], expected[row]) <= 1e-5, row
 
 
-@pytest.mark.parametrize("rows,out_dim,in_dim", [(5, 67, 512), (60, 5000, 256), (100, 6600, 256), (200, 6600, 256)])
+@pytest.mark.parametrize("rows,out_dim,in_dim", [(2, 67, 512), (3, 67, 512), (5, 67, 512), (60, 5000, 256), (100, 6600, 256), (200, 6600, 256)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
 def test_exact_linear_of_weights_that_are_not_finite(cuda, oracle, encoding, rows, out_dim, in_dim):
     """Infinite block scales and minimums, infinite and NaN float weights, and rows of zeros among
@@ -242,6 +242,13 @@ def test_exact_linear_of_weights_that_are_not_finite(cuda, oracle, encoding, row
         packed[at:at + len(value)] = np.frombuffer(value, dtype=np.uint8)
     x = kquant.synthetic_activations(6 + rows, rows, in_dim)
     x[rows - 2] = 0.0
+    if encoding in (kquant.Q6_K, kquant.Q8_0):  # a block of positive codes, times infinity, times positive activations
+        at, nbytes = 3 * row_bytes, kquant.BLOCKS[encoding][1]
+        packed[at:at + nbytes] = 0x7f if encoding == kquant.Q8_0 else 0xff
+        if encoding == kquant.Q6_K:
+            packed[at + 192:at + 208] = 1
+        packed[at + scale:at + scale + 2] = np.frombuffer(infinity, dtype=np.uint8)
+        x[rows - 1] = np.abs(x[rows - 1]) + np.float32(0.25)
     weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
     y = tile_ops.linear(weight, to_device(x, cuda)).cpu().numpy()
     w = oracle.dequantize(encoding, packed, out_dim, in_dim).reshape(out_dim, in_dim).astype(np.float64)
@@ -251,6 +258,8 @@ def test_exact_linear_of_weights_that_are_not_finite(cuda, oracle, encoding, row
     assert np.array_equal(np.isnan(y), np.isnan(expected))
     infinite = np.isinf(expected)
     assert np.array_equal(np.isinf(y), infinite) and np.array_equal(y[infinite], expected[infinite])
+    if encoding in (kquant.Q6_K, kquant.Q8_0):
+        assert expected[rows - 1, 3] == np.inf
     finite = np.isfinite(expected)
     assert normalised_error(y[finite], expected[finite]) <= 1e-5
 
