@@ -897,6 +897,8 @@ enum {
     NFN_MI355_GEMM_INT8 = 1 /* reserved: int8 activations per 32 values on the
                                int8 MFMA; refused (workspace query returns 0) */
 };
+/* A workspace that serves a call of `rows` rows and any of fewer (which may
+ * need more: a short chunk splits K over more workgroups). */
 int64_t nfn_mi355_k_quant_gemm_workspace_bytes_v1(
     int64_t rows, int64_t input_dim, int64_t output_dim, int mode);
 int nfn_mi355_k_quant_gemm_float32_v1(

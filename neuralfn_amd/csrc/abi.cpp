@@ -875,9 +875,10 @@ int nfn_mi355_k_quant_gemm_float32_v1(const Descriptor* descriptor, const float*
         !normalize_descriptor(descriptor, &normalized)) {
         return kInvalid;
     }
-    const std::int64_t required = nfn_mi355_k_quant_gemm_workspace_bytes_v1(
-        rows, normalized.input_dim, normalized.output_dim, mode);
-    if (required == 0 || workspace_nbytes < required) return kInvalid;
+    if (normalized.input_dim % 256 != 0 || mode != NFN_MI355_GEMM_F16 ||
+        workspace_nbytes < gemm_f16_required_bytes(rows, normalized.input_dim, normalized.output_dim)) {
+        return kInvalid;
+    }
     if (gemm_f16_supports(normalized.encoding, normalized.input_dim)) {
         if (reinterpret_cast<std::uintptr_t>(workspace) % 16 != 0) return kInvalid;
         launch_gemm_f16(&normalized, 1, input, &output, rows, workspace, workspace_nbytes, as_stream(cuda_stream));
@@ -931,9 +932,8 @@ int nfn_mi355_k_quant_gemm_multi_float32_v1(const Descriptor* const* descriptors
             !gemm_f16_supports(normalized[index].encoding, normalized[index].input_dim)) {
             return kInvalid;
         }
-        const std::int64_t bytes = nfn_mi355_k_quant_gemm_workspace_bytes_v1(
-            rows, normalized[index].input_dim, normalized[index].output_dim, mode);
-        if (bytes == 0) return kInvalid;
+        const std::int64_t bytes =
+            gemm_f16_required_bytes(rows, normalized[index].input_dim, normalized[index].output_dim);
         if (bytes > required) required = bytes;
     }
     if (workspace_nbytes < required) return kInvalid;

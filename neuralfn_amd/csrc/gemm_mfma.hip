@@ -54,7 +54,7 @@ constexpr int kThreads = 256;
 constexpr int kMaxProjections = 4;  // of one call
 constexpr int kLowRows = 32;    // rows up to which every wave takes all of them
 constexpr int kLowShares = 8;   // K shares of theirs at most
-constexpr int kMaxShares = 4;  // K shares of a split launch at most
+constexpr int kMaxShares = 4;   // K shares of a split launch at most
 constexpr int kRowBytes = 144;  // 64 fp16 + 16 bytes of padding
 constexpr int kStageBytes = kBN * kRowBytes;
 constexpr int kFragmentBytes = 1024;  // 32 rows x 16 K values of fp16 in operand order
@@ -1164,19 +1164,41 @@ std::int64_t activation_bytes(std::int64_t rows, std::int64_t input_dim) {
     return (padded_rows(rows) * input_dim * 2 + padded_rows(rows) * 8 + 255) & ~std::int64_t(255);
 }
 
+// The largest of needed(count) over the row counts up to `rows`, of projections of `narrowest` outputs
+// and more: short chunks split K further than longer ones and can take more memory.  What a plan
+// gives stays the same from one multiple of 128 rows to the next, so that only those can be largest,
+// and from a tile a unit on nothing is split.
+template <typename F>
+std::int64_t largest_up_to(std::int64_t rows, std::int64_t narrowest, F&& needed) {
+    std::int64_t largest = needed(rows);
+    const auto take = [&](std::int64_t count) {
+        const std::int64_t bytes = count < rows ? needed(count) : 0;
+        if (bytes > largest) largest = bytes;
+    };
+    take(kLowRows);
+    const std::int64_t n_tiles = (narrowest + kBN - 1) / kBN, units = compute_units();
+    for (std::int64_t count = 128; count < rows && (count + 255) / 256 * n_tiles < units; count += 128) take(count);
+    return largest;
+}
+
+// floats of a projection's shares behind the first
+std::int64_t partial_floats(const Plan& chosen, std::int64_t rows, std::int64_t output_dim) {
+    return (chosen.shares - 1) * rows * output_dim;
+}
+
 }  // namespace
 
-std::int64_t gemm_f16_workspace_bytes(std::int64_t rows, std::int64_t input_dim,
-                                      std::int64_t output_dim) {
+std::int64_t gemm_f16_required_bytes(std::int64_t rows, std::int64_t input_dim, std::int64_t output_dim) {
     // the activations, then one copy of the output per K share of a split
     // launch (the encoding with the most shares bounds the others)
-    const auto needed = [&](std::int64_t count) {
-        const int shares = plan(kEncQ4K, count, output_dim, input_dim).shares;
-        return activation_bytes(count, input_dim) + (shares > 1 ? shares * count * output_dim * 4 : 0) + 256;
-    };
-    // what serves a long chunk serves a short one behind it
-    const std::int64_t own = needed(rows), few = rows > kLowRows ? needed(kLowRows) : 0;
-    return own > few ? own : few;
+    const int shares = plan(kEncQ4K, rows, output_dim, input_dim).shares;
+    return activation_bytes(rows, input_dim) + (shares > 1 ? shares * rows * output_dim * 4 : 0) + 256;
+}
+
+std::int64_t gemm_f16_workspace_bytes(std::int64_t rows, std::int64_t input_dim, std::int64_t output_dim) {
+    return largest_up_to(rows, output_dim, [&](std::int64_t count) {
+        return gemm_f16_required_bytes(count, input_dim, output_dim);
+    });
 }
 
 void gemm_f16_plan(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
@@ -1212,21 +1234,22 @@ void convert_gemm_activations(const float* input, std::int64_t rows, std::int64_
     }
 }
 
-// floats of a projection's shares behind the first
-static std::int64_t partial_floats(const Plan& chosen, std::int64_t rows, std::int64_t output_dim) {
-    return (chosen.shares - 1) * rows * output_dim;
-}
-
 std::int64_t gemm_f16_multi_workspace_bytes(std::int64_t rows, std::int64_t input_dim, const std::int64_t* output_dims,
                                             int count) {
-    std::int64_t largest = 0, floats = 0;
-    for (int i = 0; i < count; ++i) {
-        const std::int64_t single = gemm_f16_workspace_bytes(rows, input_dim, output_dims[i]);
-        if (single > largest) largest = single;
-        floats += partial_floats(plan(kEncQ4K, rows, output_dims[i], input_dim), rows, output_dims[i]);
+    std::int64_t narrowest = output_dims[0];
+    for (int i = 1; i < count; ++i) {
+        if (output_dims[i] < narrowest) narrowest = output_dims[i];
     }
-    const std::int64_t together = activation_bytes(rows, input_dim) + 4 * floats + 256;
-    return together > largest ? together : largest;
+    return largest_up_to(rows, narrowest, [&](std::int64_t chunk) {
+        std::int64_t largest = 0, floats = 0;
+        for (int i = 0; i < count; ++i) {
+            const std::int64_t single = gemm_f16_required_bytes(chunk, input_dim, output_dims[i]);
+            if (single > largest) largest = single;
+            floats += partial_floats(plan(kEncQ4K, chunk, output_dims[i], input_dim), chunk, output_dims[i]);
+        }
+        const std::int64_t together = activation_bytes(chunk, input_dim) + 4 * floats + 256;
+        return together > largest ? together : largest;
+    });
 }
 
 void launch_gemm_f16(const Descriptor* descriptors, int count, const float* input, float* const* outputs,

@@ -8,17 +8,18 @@ namespace nfn {
 // Bytes of device workspace the fp16 path needs: a row-scaled fp16 copy of the
 // activations in whole 256-row tiles, one inverse scale per row, and, where a
 // small problem splits K over several workgroups per tile, one copy of the
-// output per share.
-std::int64_t gemm_f16_workspace_bytes(std::int64_t rows, std::int64_t input_dim,
-                                      std::int64_t output_dim);
+// output per share.  required: of a call of so many rows; workspace: of any call of up to so many
+// (fewer rows can take more K shares, and with them more memory).
+std::int64_t gemm_f16_required_bytes(std::int64_t rows, std::int64_t input_dim, std::int64_t output_dim);
+std::int64_t gemm_f16_workspace_bytes(std::int64_t rows, std::int64_t input_dim, std::int64_t output_dim);
 bool gemm_f16_supports(std::uint32_t encoding, std::int64_t input_dim);
 // How a launch of this geometry is cut on the current device: rows of the
 // output tile a workgroup owns (256 or 128; 32 for up to 32 rows) and the number of K shares (1 =
 // unsplit; more = one partial output per share, summed by a second launch).
 void gemm_f16_plan(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
                    std::int64_t output_dim, int* tile_rows, int* k_shares);
-// What 1..4 projections of one input need to run in one launch an encoding; with the largest of
-// the single sizes they still run, in as many launches as it takes.
+// What 1..4 projections of one input, of up to so many rows, need to run in one launch an encoding;
+// with the largest of the single sizes they still run, in as many launches as it takes.
 std::int64_t gemm_f16_multi_workspace_bytes(std::int64_t rows, std::int64_t input_dim, const std::int64_t* output_dims,
                                             int count);
 // outputs[i][rows, output_dim] = input[rows, input_dim] * W_i^T, float accumulation, for 1..4

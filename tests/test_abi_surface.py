@@ -247,6 +247,22 @@ def test_the_reference_engines_own_loader_opens_the_library():
     assert status == 1 and "absolute" in report.value.decode()
 
 
+def test_a_prefill_workspace_serves_every_chunk_of_fewer_rows(lib):
+    """Short chunks split K over more workgroups and can need more than longer ones: the queries
+    never fall as the rows grow."""
+    import ctypes
+    single, multi = lib.nfn_mi355_k_quant_gemm_workspace_bytes_v1, lib.nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1
+    rows = sorted({1, 17, 32, 33, 64, 100, 20000, 70000} | {step + off for step in range(128, 3000, 128) for off in (0, 1)})
+    for in_dim in (256, 2048, 4096, 6656, 9216, 16384):
+        for widths in ((17,), (256,), (6656,), (16384,), (33024,), (4096, 256, 256, 4096), (16384, 16384), (640, 6656)):
+            dims = (ctypes.c_int64 * len(widths))(*widths)
+            sizes = [multi(count, in_dim, dims, len(widths), tile_ops.GEMM_F16) for count in rows]
+            assert sizes == sorted(sizes) and sizes[0] > 0, (in_dim, widths)
+            if len(widths) == 1:
+                sizes = [single(count, in_dim, widths[0], tile_ops.GEMM_F16) for count in rows]
+                assert sizes == sorted(sizes) and sizes[0] > 0, (in_dim, widths)
+
+
 def test_front_end_binds_declared_entry_points_and_checks_its_arguments():
     """The extension module in front of the C ABI: it binds names of the header only, and what the
     ctypes form refused with an exception before the call it refuses with one of the same kind."""

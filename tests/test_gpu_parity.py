@@ -1589,14 +1589,30 @@ def test_prefill_gemm_plans():
     # A K too short for shares: 256-row tiles from half a workgroup a unit on.
     assert tile_ops.gemm_plan(kquant.Q4_K, 512, 4096, 6656) == (128, 1)
     assert tile_ops.gemm_plan(kquant.Q4_K, 700, 4096, 6656) == (256, 1)
-    # A workspace for a longer chunk serves a chunk of few rows, which takes more shares.
-    query = tile_ops.load().nfn_mi355_k_quant_gemm_workspace_bytes_v1
-    for in_dim, out_dim in ((256, 17), (4096, 6656), (6656, 256), (6656, 16384), (16384, 6656)):
-        few = max(query(rows, in_dim, out_dim, tile_ops.GEMM_F16) for rows in (1, 17, 32))
-        assert all(query(rows, in_dim, out_dim, tile_ops.GEMM_F16) >= few for rows in (33, 64, 128, 256, 300, 4096))
     # A narrow projection (the K and V projections of the workload): small tiles, short shares.
     assert tile_ops.gemm_plan(kquant.Q4_K, 1024, 6656, 256) == (128, 4)
     assert tile_ops.gemm_plan(kquant.Q6_K, 2048, 6656, 256) == (128, 4)
+
+
+def test_prefill_gemm_workspace_of_a_longer_chunk(cuda):
+    """The workspace of a long chunk serves the short ones behind it, which split K further, and a
+    call takes any workspace that holds what its own plan needs: the fp16 rows in whole 256-row
+    tiles, eight bytes a row, an output per share, 256 bytes."""
+    in_dim, out_dim = 6656, 16384
+    query = tile_ops.load().nfn_mi355_k_quant_gemm_workspace_bytes_v1
+    packed = random_packed(kquant.Q4_K, out_dim, in_dim, 5)
+    weight = tile_ops.PackedWeight.from_numpy(kquant.Q4_K, packed, out_dim, in_dim)
+    large = torch_().empty(query(512, in_dim, out_dim, tile_ops.GEMM_F16), dtype=torch_().uint8, device=cuda)
+    for rows in (512, 256, 128, 17):
+        x = to_device(kquant.synthetic_activations(rows, rows, in_dim), cuda)
+        y = tile_ops.gemm(weight, x, workspace=large)
+        _, shares = tile_ops.gemm_plan(kquant.Q4_K, rows, in_dim, out_dim)
+        padded = (rows + 255) // 256 * 256
+        needed = (padded * (in_dim * 2 + 8) + 255) // 256 * 256 + (shares * rows * out_dim * 4 if shares > 1 else 0) + 256
+        assert needed <= large.numel()
+        assert_bits_equal(tile_ops.gemm(weight, x, workspace=large[:needed]), y, str(rows))
+        with pytest.raises(tile_ops.TileOpsError):
+            tile_ops.gemm(weight, x, workspace=large[:needed - 1])
 
 
 @pytest.mark.parametrize("rows,in_dim,plan", [
