@@ -943,14 +943,30 @@ void launch_small(const Descriptor& weight, const float* input, const float* bia
                        weight.output_dim, static_cast<int>(row_tiles));
 }
 
+// What a round of the larger tiles costs in rounds of 32 x 32: 32 x 64, 32 x 128 and 64 x 128 (F32:
+// 64 x 32 and 64 x 64).  From a sweep over 484 shapes an encoding (4..512 rows, 64..8,192 outputs,
+// 2,048..8,192 columns, every form of each): the middle of the values with which the rule loses least
+// to the fastest form.  Mean and largest loss, and with 1.35, 2.1 and 2.9 for all packed encodings and
+// bf16 (F32 1.4 and 2.1): Q4_K 0.00 and 1.3 % (0.31 and 15), Q5_K 0.30 and 13 (1.4 and 38; its 64 x 128
+// form keeps registers in scratch), Q6_K 0.08 and 18 (the same), Q8_0 0.00 and 0.5 (0.01 and 4), bf16
+// none (0.05 and 13), F32 0.16 and 12 (0.24 and 10).
+template <std::uint32_t ENC>
+constexpr double kRounds[3] = {1.4, 2.5, 3.9};  // Q4_K, Q5_K
+template <>
+constexpr double kRounds<kEncQ6K>[3] = {1.45, 2.1, 2.6};
+template <>
+constexpr double kRounds<kEncQ8_0>[3] = {1.45, 2.1, 2.6};
+template <>
+constexpr double kRounds<kEncBF16>[3] = {1.5, 2.0, 2.4};
+template <>
+constexpr double kRounds<kEncF32>[3] = {1.6, 2.1, 0.0};
+
 template <std::uint32_t ENC>
 void launch_for(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
                 hipStream_t stream) {
     // What bounds all forms is the look-up of lines in the unit's vector cache, which a round of
-    // tiles, one workgroup a unit, makes as often however many of its rows are real.  A round of
-    // 32 x 32, 32 x 64, 32 x 128 and 64 x 128 tiles was measured at 21, 27, 43 and 65 us for Q4_K
-    // (33, 46, 78, 90 for Q8_0) at 4,096 columns, of 32 x 32, 64 x 32 and 64 x 64 tiles at 31, 45
-    // and 68 us for F32: the form with the cheapest rounds takes the call.
+    // tiles, one workgroup a unit, makes as often however many of its rows are real: the form with
+    // the cheapest rounds takes the call.
     const std::int64_t units = compute_units();
     const auto rounds = [&](std::int64_t height, std::int64_t width) {
         const std::int64_t tiles = (rows + height - 1) / height * ((weight.output_dim + width - 1) / width);
@@ -958,7 +974,7 @@ void launch_for(const Descriptor& weight, const float* input, const float* bias,
     };
     const double cost_small = rounds(32, 32);
     if constexpr (ENC == kEncF32) {
-        const double cost_high = 1.4 * rounds(64, 32), cost_square = 2.1 * rounds(64, 64);
+        const double cost_high = kRounds<ENC>[0] * rounds(64, 32), cost_square = kRounds<ENC>[1] * rounds(64, 64);
         if (cost_square <= cost_high && cost_square <= cost_small) {
             launch_small<ENC, 2, 2, 4>(weight, input, bias, output, rows, stream);
         } else if (cost_high <= cost_small) {
@@ -968,8 +984,9 @@ void launch_for(const Descriptor& weight, const float* input, const float* bias,
         }
     } else {
         const bool whole = weight.input_dim % 64 == 0;
-        const double cost_wide = 1.35 * rounds(32, 64);
-        const double cost_low = whole ? 2.1 * rounds(32, 128) : 1e30, cost_high = whole ? 2.9 * rounds(64, 128) : 1e30;
+        const double cost_wide = kRounds<ENC>[0] * rounds(32, 64);
+        const double cost_low = whole ? kRounds<ENC>[1] * rounds(32, 128) : 1e30;
+        const double cost_high = whole ? kRounds<ENC>[2] * rounds(64, 128) : 1e30;
         if (cost_high <= cost_low && cost_high <= cost_wide && cost_high <= cost_small) {
             launch_large<ENC, 2>(weight, input, bias, output, rows, stream);
         } else if (cost_low <= cost_wide && cost_low <= cost_small) {
