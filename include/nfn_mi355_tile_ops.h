@@ -91,7 +91,11 @@ int nfn_native_tile_packed_weight_dequantize_float32_v1(
  *      float weights times float activations, no quantization of the input.
  *      It has no workspace argument, so every row count keeps that float
  *      arithmetic (four rows and more on the bf16 matrix instruction, the floats cut into exact terms);
- *      nfn_mi355_k_quant_gemm_float32_v1 is the fp16 matrix-core route. -- */
+ *      nfn_mi355_k_quant_gemm_float32_v1 is the fp16 matrix-core route.
+ *      The order of the float sums belongs to the kernel: a row's bits are the same whichever other
+ *      rows come with it among one to three rows (as many as fit LDS: 160 KB, 272 bytes for 64
+ *      columns) and among four to 32, but differ in the last place between the two and beyond.
+ *      The exact verifier entry points below are the calls whose rows equal the one-row call. -- */
 int nfn_native_tile_linear_packed_weight_float32_v1(
     const NfnNativeTilePackedWeightDescriptorV1* descriptor,
     const float* input,

@@ -201,6 +201,22 @@ def test_exact_linear_forms_at_their_edges(cuda, oracle, encoding, rows, out_dim
     assert normalised_error(y[: rows - 1], expected[: rows - 1]) <= 1e-5 if rows > 1 else True
 
 
+@pytest.mark.parametrize("out_dim,in_dim", [(67, 512), (6656, 768), (9000, 256), (33, 2048)])
+@pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
+def test_exact_linear_rows_carry_the_same_bits_within_a_form(cuda, encoding, out_dim, in_dim):
+    """What the header says of a row's bits: the same whichever other rows come with it, among one
+    to three rows and among four to 32."""
+    packed = kquant.quantize(encoding, kquant.synthetic_weights(5, out_dim, in_dim))
+    weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    x = to_device(kquant.synthetic_activations(6, 32, in_dim), cuda)
+    three, many = tile_ops.linear(weight, x[:3]), tile_ops.linear(weight, x)
+    for rows in (1, 2):
+        assert_bits_equal(tile_ops.linear(weight, x[3 - rows:3]), three[3 - rows:], f"{rows} rows")
+    for rows in (4, 5, 16, 17, 31):
+        assert_bits_equal(tile_ops.linear(weight, x[32 - rows:]), many[32 - rows:], f"{rows} rows")
+    assert normalised_error(three.cpu().numpy(), many[:3].cpu().numpy()) <= 1e-5
+
+
 @pytest.mark.parametrize("rows,out_dim,in_dim", [(3, 67, 512), (5, 67, 512), (60, 5000, 256), (100, 6600, 256), (200, 6600, 256)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
 def test_exact_linear_of_infinities_nan_and_large_activations(cuda, oracle, encoding, rows, out_dim, in_dim):
