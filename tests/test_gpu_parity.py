@@ -983,6 +983,63 @@ def test_verifier_matrix_core_rows_tensor_two_bytes_off_a_word(cuda, encoding, i
         assert_bits_equal(single, a[rows - 1:rows].contiguous(), "the one-row call on the shifted tensor")
 
 
+def shifted_copy(array, offset, device):
+    """The values of `array` in a tensor that starts `offset` bytes into an allocation and ends with it."""
+    flat = torch_().from_numpy(np.ascontiguousarray(array)).reshape(-1).view(torch_().uint8)
+    holder = torch_().empty(flat.numel() + offset, dtype=torch_().uint8, device=device)
+    holder[offset:].copy_(flat)
+    return holder[offset:]
+
+
+def shifted_floats(array, device):
+    flat = torch_().empty(array.size + 1, dtype=torch_().float32, device=device)[1:]
+    flat.copy_(torch_().from_numpy(np.ascontiguousarray(array)).reshape(-1))
+    assert flat.data_ptr() % 16 == 4
+    return flat.reshape(array.shape)
+
+
+@pytest.mark.parametrize("rows,out_dim,in_dim", [(1, 75, 768), (3, 1030, 512), (5, 75, 768), (60, 5000, 256),
+                                                 (100, 6600, 256), (200, 6600, 256)])
+@pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
+def test_exact_linear_on_tensors_off_a_word(cuda, encoding, rows, out_dim, in_dim):
+    """Every form: weights two bytes (floats four) and activations four bytes off the boundary that
+    their loads would like, at the end of their allocations: the bits of the aligned call."""
+    packed = kquant.quantize(encoding, kquant.synthetic_weights(57, out_dim, in_dim))
+    x, bias = kquant.synthetic_activations(58, rows, in_dim), kquant.synthetic_activations(59, 1, out_dim)[0]
+    aligned = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    data = shifted_copy(packed, 4 if encoding == kquant.F32 else 2, cuda)
+    shifted = tile_ops.PackedWeight(encoding, out_dim, in_dim, data)
+    assert shifted.data.data_ptr() % 16 in (2, 4)
+    expected = tile_ops.linear(aligned, to_device(x, cuda), to_device(bias, cuda))
+    assert_bits_equal(tile_ops.linear(shifted, shifted_floats(x, cuda), shifted_floats(bias, cuda)), expected)
+
+
+@pytest.mark.parametrize("encoding", ALL_PACKED)
+def test_lm_head_one_row_on_tensors_off_a_word(cuda, encoding):
+    out_dim, in_dim = 4099, 1280
+    packed = random_packed(encoding, out_dim, in_dim, 60)
+    x = kquant.synthetic_activations(61, 1, in_dim)
+    aligned = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    shifted = tile_ops.PackedWeight(encoding, out_dim, in_dim, shifted_copy(packed, 2, cuda))
+    indices, maxima = tile_ops.lm_head_argmax(aligned, to_device(x, cuda))
+    again, again_maxima = tile_ops.lm_head_argmax(shifted, shifted_floats(x, cuda))
+    assert torch_().equal(indices, again)
+    assert_bits_equal(maxima, again_maxima)
+
+
+@pytest.mark.parametrize("rows,out_dim,in_dim", [(17, 129, 1536), (96, 130, 3072), (300, 1030, 1280), (700, 6656, 512)])
+@pytest.mark.parametrize("encoding", ALL_PACKED)
+def test_prefill_gemm_on_tensors_off_a_word(cuda, encoding, rows, out_dim, in_dim):
+    """Up to 32 rows, K shares of 128-row tiles, and 256-row tiles; the output four bytes off as well."""
+    packed = random_packed(encoding, out_dim, in_dim, 62)
+    x = kquant.synthetic_activations(63, rows, in_dim)
+    aligned = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    shifted = tile_ops.PackedWeight(encoding, out_dim, in_dim, shifted_copy(packed, 2, cuda))
+    out = shifted_floats(np.zeros((rows, out_dim), dtype=np.float32), cuda)
+    expected = tile_ops.gemm(aligned, to_device(x, cuda))
+    assert_bits_equal(tile_ops.gemm(shifted, shifted_floats(x, cuda), out=out), expected)
+
+
 @pytest.mark.parametrize("in_dim", [256, 1024, 6656, 6912])
 @pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q6_K, kquant.Q8_0])
 def test_fp16_rows_last_row_of_a_tensor_and_shifted_tensors(cuda, encoding, in_dim):
