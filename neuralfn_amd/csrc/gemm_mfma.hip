@@ -3,7 +3,8 @@
 //
 // A workgroup of 4 waves owns a 256 x 128 tile of Y; wave w owns rows
 // 64w .. 64w+63 and all 128 columns, and walks K in steps of 64 with 32
-// v_mfma_f32_32x32x16_f16 per step and float accumulators.
+// v_mfma_f32_32x32x16_f16 per step and float accumulators.  (128-row tiles: half
+// the rows and instructions a wave; up to 32 rows have a kernel of their own below.)
 //
 // Activations never touch LDS.  A pre-pass converts them to fp16 once per call
 // and stores them in matrix-core operand order: for every block of 32 rows and
@@ -15,8 +16,9 @@
 // magnitude lands in [2^14, 2^15); the epilogue multiplies the row's results
 // by the inverse, so neither large nor tiny activations leave the fp16 range.
 //
-// Weights go through LDS: per step every thread turns 16 packed bytes (32
-// weights of one row of the 128 x 64 slice) into fp16 in registers with packed
+// Weights go through LDS: per step every thread turns 32 weights of the
+// 128 x 64 slice (two runs of 16: of one row for Q4_K and Q5_K, 16 packed bytes;
+// of two rows for Q6_K and Q8_0) into fp16 in registers with packed
 // fp16 arithmetic (code bytes become 1024+q by a byte permute, then
 // (x-1024)*(d*sc) - dmin*m as one packed fused multiply-add) and writes them
 // to a double-buffered stage; the packed bytes are read from HBM once per tile
@@ -29,9 +31,10 @@
 // against reordering, so that the dequantization, the LDS traffic and the
 // global loads of later steps are issued in the shadow of the matrix
 // instructions; weight fragments are read one K chunk ahead, packed bytes are
-// loaded three steps before they are decoded (Q6_K: two).  Consecutive workgroups walk M first: with 8 XCDs picking
-// workgroups round robin each XCD keeps one or two 256-row slices of X in its
-// L2 while the packed weights stream through.
+// loaded three steps before they are decoded (Q6_K: two; where the registers allow
+// it a whole block together, a block ahead).  Consecutive workgroups walk M first:
+// with 8 XCDs picking workgroups round robin each XCD keeps one or two 256-row
+// slices of X in its L2 while the packed weights stream through.
 //
 // The reference has no kernel of this kind: its small-batch path stops at 16
 // rows (neuralfn/csrc/tile_cuda/glimmer_k_mmq.cu:1326-1328) and more rows run
@@ -78,8 +81,8 @@ struct __attribute__((packed, aligned(2))) Chunk8 {
 // The row's scale is the power of two that brings that magnitude into
 // [2^14, 2^15); zero, subnormal, infinite or NaN maxima keep scale 1; padding
 // rows get inverse 0 and zeros.
-// The eight workgroups that fill one 32-row block of the operand-order copy
-// are the ones a round-robin placement over the eight XCDs puts on the same
+// The workgroups that fill one 32-row block of the operand-order copy (8, 16 or 32: four, two
+// rows or one each) are the ones a round-robin placement over the eight XCDs puts on the same
 // XCD (workgroup w lands on XCD w % 8), so that the 16-byte pieces they
 // scatter into the same cache lines merge in one L2 before going to memory.
 // Rows of up to 8,192 columns take four waves each, for the loads in flight of a short prompt
@@ -828,9 +831,10 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
 // Up to 32 rows: a wave owns 32 columns and all rows of the same 128-column tile, so that a decoded
 // weight fragment is read from LDS by one wave instead of four and by the wave that wrote it: no
 // barrier, a quarter of the LDS reads, no matrix instructions for rows that are not there.  What
-// bounds it is the latency of the packed bytes and of the fragments from L2, which are requested a
-// block and four steps ahead, and with that the number of workgroups: K is cut into up to eight
-// shares.  17 rows, width 6,656, against 128-row tiles: Q, K, V and gate 41 -> 32 us for Q4_K, 50 -> 41
+// bounds it: 17 rows of gate and up (Q4_K) take 40 us with the vector caches looking up a line in 68 % of
+// the cycles, the vector ALU busy in half of them and a quarter of the waves' time in waits; the
+// packed bytes and the fragments from L2 are requested a block and four steps ahead, and few
+// tiles leave units without work: K is cut into up to eight shares.  17 rows, width 6,656, against 128-row tiles: Q, K, V and gate 41 -> 32 us for Q4_K, 50 -> 41
 // for Q6_K; O (4,096 wide) 43 -> 21 and 52 -> 25; gate and up 68 -> 54 and 85 -> 68; down 56 -> 39
 // and 66 -> 49; Q8_0 50 -> 47, 52 -> 32, 86 -> 84, 64 -> 60.
 // ---------------------------------------------------------------------------
@@ -1218,18 +1222,18 @@ void convert_gemm_activations(const float* input, std::int64_t rows, std::int64_
     std::uint8_t* activations = static_cast<std::uint8_t*>(workspace);
     float* inverse_scale = reinterpret_cast<float*>(activations + padded_rows(rows) * input_dim * 2);
     const std::int64_t groups = input_dim / 8;
-    const unsigned whole_rows = static_cast<unsigned>(padded_rows(rows) / 4);  // a wave per row
+    const unsigned wave_a_row = static_cast<unsigned>(padded_rows(rows) / 4);  // workgroups of four rows
     if (groups <= 4 * 64 * 2) {
-        hipLaunchKernelGGL((prepare_activations_kernel<2, 4>), dim3(4 * whole_rows), dim3(256), 0, stream,
+        hipLaunchKernelGGL((prepare_activations_kernel<2, 4>), dim3(4 * wave_a_row), dim3(256), 0, stream,
                            input, activations, inverse_scale, rows, input_dim);
     } else if (groups <= 4 * 64 * 4) {
-        hipLaunchKernelGGL((prepare_activations_kernel<4, 4>), dim3(4 * whole_rows), dim3(256), 0, stream,
+        hipLaunchKernelGGL((prepare_activations_kernel<4, 4>), dim3(4 * wave_a_row), dim3(256), 0, stream,
                            input, activations, inverse_scale, rows, input_dim);
     } else if (groups <= 2 * 64 * 16) {
-        hipLaunchKernelGGL((prepare_activations_kernel<16, 2>), dim3(2 * whole_rows), dim3(256), 0,
+        hipLaunchKernelGGL((prepare_activations_kernel<16, 2>), dim3(2 * wave_a_row), dim3(256), 0,
                            stream, input, activations, inverse_scale, rows, input_dim);
     } else {
-        hipLaunchKernelGGL((prepare_activations_kernel<0, 1>), dim3(whole_rows), dim3(256), 0, stream,
+        hipLaunchKernelGGL((prepare_activations_kernel<0, 1>), dim3(wave_a_row), dim3(256), 0, stream,
                            input, activations, inverse_scale, rows, input_dim);
     }
 }

@@ -24,11 +24,16 @@
 //   each) in each of four K groups.  The two cut the activations of a step of 32 columns between
 //   them and hand the terms over in LDS.
 // What bounds both is the vector cache: a load instruction that reads 16 bytes from each of 32 rows
-// looks up 32 lines for 1 KB, and a unit pulls some 20 GB/s that way.  (Requests two steps ahead
-// instead of one, and the matrix instructions of a step before its other work instead of between it,
-// made no difference.)  Measured at 4,096 -> 6,656, against the vector kernel (16 rows) and the
-// float matrix instruction (200, 512 rows) before: Q4_K 134 -> 16 us at 16 rows, 203 -> 69 at 200,
-// 311 -> 135 at 512; Q8_0 368 -> 27, 180 -> 81, 279 -> 162; F32 406 -> 30, 172 -> 131, 271 -> 254.
+// looks up 32 lines for 1 KB, and a unit pulls some 20 GB/s that way.  200 rows of Q8_0: a look-up in
+// 70 % of the cycles, the matrix cores busy in 26 %, the vector ALU in 37, LDS in 14.  (Requests two
+// steps ahead instead of one, and the matrix instructions of a step before its other work instead of
+// between it, made no difference.)  Registers: the 64 x 128 form of Q5_K keeps thirteen registers that do
+// not change in its loop (56 bytes a lane) in scratch, with six reads of them in two units of 930
+// instructions each (its fifth bits in one word instead of four left eight there); the 64 x 64 form of
+// F32 keeps eight (36 bytes), read outside of its loop only; the others none.
+// Measured at 4,096 -> 6,656, against the vector kernel (16 rows) and the float matrix instruction (200,
+// 512 rows) before: Q4_K 134 -> 16 us at 16 rows, 203 -> 69 at 200, 311 -> 135 at 512; Q8_0 368 -> 27,
+// 180 -> 82, 279 -> 162; F32 406 -> 30, 172 -> 131, 271 -> 254.
 //
 // The entry point, nfn_native_tile_linear_packed_weight_float32_v1, has no workspace argument
 // (neuralfn/csrc/native_train/tile_ops.h:614-620; reference kernel
