@@ -27,13 +27,12 @@
 // looks up 32 lines for 1 KB, and a unit pulls some 20 GB/s that way.  200 rows of Q8_0: a look-up in
 // 70 % of the cycles, the matrix cores busy in 26 %, the vector ALU in 37, LDS in 14.  (Requests two
 // steps ahead instead of one, and the matrix instructions of a step before its other work instead of
-// between it, made no difference.)  Registers: the 64 x 128 form of Q5_K keeps thirteen registers that do
-// not change in its loop (56 bytes a lane) in scratch, with six reads of them in two units of 930
-// instructions each (its fifth bits in one word instead of four left eight there); the 64 x 64 form of
-// F32 keeps eight (36 bytes), read outside of its loop only; the others none.
+// between it, made no difference.)  The 64 x 128 form of Q5_K keeps four registers that do not change in
+// its loop in scratch (20 bytes a lane), the 64 x 64 form of F32 seven (32 bytes), read outside of its
+// loop only; the others none.
 // Measured at 4,096 -> 6,656, against the vector kernel (16 rows) and the float matrix instruction (200,
-// 512 rows) before: Q4_K 134 -> 16 us at 16 rows, 203 -> 69 at 200, 311 -> 135 at 512; Q8_0 368 -> 27,
-// 180 -> 82, 279 -> 162; F32 406 -> 30, 172 -> 131, 271 -> 254.
+// 512 rows) before: Q4_K 134 -> 16 us at 16 rows, 203 -> 68 at 200, 311 -> 135 at 512; Q8_0 368 -> 27,
+// 180 -> 80, 279 -> 162; F32 406 -> 30, 172 -> 136, 271 -> 254.
 //
 // The entry point, nfn_native_tile_linear_packed_weight_float32_v1, has no workspace argument
 // (neuralfn/csrc/native_train/tile_ops.h:614-620; reference kernel
@@ -56,8 +55,9 @@ typedef std::uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 // The factor that floats are cut with: without it the third term of an activation below 2^-110
 // would fall under 2^-133, the smallest bf16 number, and lose bits (relative error 5e-5 at 1e-36).
-// Sums of ordinary numbers keep their bits, and 200 rows of Q8_0 take 81.8 us with it and 81.5
-// without.  Float weights are cut with it too.
+// Sums of ordinary numbers keep their bits.  It costs the small forms up to 5 % (4 rows of Q4_K,
+// 5,120 -> 178: 15.2 -> 15.9 us) and the large ones little (200 rows of Q8_0 81.5 -> 81.8).  Float weights
+// are cut with it too.
 constexpr float kLift = 0x1p24f;
 template <std::uint32_t ENC>
 constexpr float kLower = ENC == kEncF32 ? 0x1p-48f : 0x1p-24f;  // ... and taken out of the sums
@@ -69,18 +69,19 @@ __device__ __forceinline__ std::uint32_t upper_halves(float low, float high) {
     return __builtin_amdgcn_perm(__float_as_uint(high), __float_as_uint(low), 0x07060302u);
 }
 
-// Two of the eight values of a fragment: word `pair` of its three terms.
+// Two of the eight values of a fragment, times kLift: word `pair` of its three terms.
 __device__ __forceinline__ void cut_pair(float x0, float x1, std::uint32_t& a, std::uint32_t& b, std::uint32_t& c) {
-    a = upper_halves(x0, x1);
-    const float y0 = x0 - __uint_as_float(__float_as_uint(x0) & 0xffff0000u);
-    const float y1 = x1 - __uint_as_float(__float_as_uint(x1) & 0xffff0000u);
+    const float l0 = x0 * kLift, l1 = x1 * kLift;
+    a = upper_halves(l0, l1);
+    const float y0 = fmaf(x0, kLift, -__uint_as_float(__float_as_uint(l0) & 0xffff0000u));
+    const float y1 = fmaf(x1, kLift, -__uint_as_float(__float_as_uint(l1) & 0xffff0000u));
     b = upper_halves(y0, y1);
     const float z0 = y0 - __uint_as_float(__float_as_uint(y0) & 0xffff0000u);
     const float z1 = y1 - __uint_as_float(__float_as_uint(y1) & 0xffff0000u);
     c = upper_halves(z0, z1);
 }
 
-// Eight floats as three bf16 fragments whose sum they are.
+// Eight floats, times kLift, as three bf16 fragments whose sum they are.
 struct Terms {
     bf16x8 first, second, third;
 };
@@ -158,11 +159,20 @@ struct UnitOfQ4KOrQ5K {
         codes = *reinterpret_cast<const u32x4_a4*>(block + (ENC == kEncQ5K ? 48 : 16) + group * 32 + half * 16);
         if constexpr (ENC == kEncQ5K) fifth = *reinterpret_cast<const u32x4_a4*>(block + 16 + half * 16);
     }
-    __device__ __forceinline__ void arrange() {}
+    __device__ __forceinline__ void arrange() {
+        if constexpr (ENC == kEncQ5K) {
+            // the unit's two bits of every byte, all four words in one (three registers a unit less)
+            std::uint32_t bits = fifth[0] >> (2 * group) & 0x03030303u;
+#pragma unroll
+            for (int word = 1; word < 4; ++word) bits |= (fifth[word] >> (2 * group) & 0x03030303u) << (2 * word);
+            fifth[0] = bits;
+        }
+    }
     __device__ __forceinline__ void words(int step, int chunk, int word, std::uint32_t& low, std::uint32_t& high) const {
         std::uint32_t q = (codes[2 * chunk + word] >> (4 * step)) & 0x0f0f0f0fu;
         if constexpr (ENC == kEncQ5K) {
-            q |= ((fifth[2 * chunk + word] >> (2 * group + step)) & 0x01010101u) << 4;
+            const int bit = 2 * (2 * chunk + word) + step;  // (constant where it is used)
+            q |= ((bit < 4 ? fifth[0] << (4 - bit) : fifth[0] >> (bit - 4)) & 0x10101010u);
         }
         codes_to_bf16(q, 0.0f, low, high);
     }
@@ -297,7 +307,7 @@ struct Unit<kEncF32> {
     __device__ __forceinline__ Terms terms(int step, int chunk) const {
         float eight[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) eight[j] = values[step][chunk][j >> 2][j & 3] * kLift;
+        for (int j = 0; j < 8; ++j) eight[j] = values[step][chunk][j >> 2][j & 3];
         return cut(eight);
     }
 };
@@ -538,28 +548,43 @@ __device__ __forceinline__ float decoded_dot(const std::uint8_t* row, const floa
     return even + odd;
 }
 
-// The outputs that a wave left in `again`, taken from the decoded weights: infinity less its own upper half is NaN where the product with the
-// weight is infinite, and the lifted products leave the float range (activations above some 2^90 with
-// codes, products above 2^80 with float weights) before those with the weights do.
-// place(pass, r, row, column): the row and column of this lane's bit.
-// 4,096 -> 6,656 at 200 rows (Q8_0 / Q4_K, 87 / 75 us from Python): with a NaN in one row 90 / 82 us, in
-// every row 123 / 97; an infinity or activations of 3e37 in one row 207 / 231, in every row 3.6 / 3.4 ms
+// The outputs that a wave left in `again`, taken from the decoded weights: infinity less its own upper
+// half is NaN where the product with the weight is infinite, and the lifted products leave the float
+// range (activations above some 2^90 with codes, products above 2^80 with float weights) before those
+// with the weights do.  MT: as in the kernels below.
+// 4,096 -> 6,656 at 200 rows (Q8_0 / Q4_K, 86 / 75 us from Python): with a NaN in one row 89 / 80 us, in
+// every row 123 / 100; an infinity or activations of 3e37 in one row 204 / 237, in every row 3.6 / 3.4 ms
 // (a byte and a weight at a time: 1.1 / 1.9 ms for one row of either kind, 29 / 64 for all).
-template <std::uint32_t ENC, int WAVES, typename Place>
-__device__ __forceinline__ void take_again(std::uint64_t again, int wave, int lane, const std::uint8_t* data,
+template <std::uint32_t ENC, int MT, int WAVES>
+__device__ __forceinline__ void take_again(std::uint64_t again, int wave, const std::uint8_t* data,
                                            std::int64_t row_stride, const float* input, std::int64_t input_dim,
-                                           const float* bias, float* output, std::int64_t output_dim, Place&& place) {
+                                           const float* bias, float* output, std::int64_t output_dim,
+                                           std::int64_t row0, std::int64_t col0) {
+    const int lane = threadIdx.x & 63;
     for (std::uint64_t holders = __ballot(again != 0); holders != 0; holders &= holders - 1) {
         const int index = __builtin_ctzll(holders);
         const std::uint32_t low = __builtin_amdgcn_readlane(static_cast<std::uint32_t>(again), index);
         const std::uint32_t high = __builtin_amdgcn_readlane(static_cast<std::uint32_t>(again >> 32), index);
         if (((lane < 32 ? low : high) >> (lane & 31) & 1) != 0) {
-            std::int64_t row, column;
-            place(index / (16 / WAVES), index % (16 / WAVES) * WAVES + wave, row, column);
+            const int pass = index / (16 / WAVES), r = index % (16 / WAVES) * WAVES + wave;
+            const std::int64_t row = row0 + 32 * (pass % MT) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            const std::int64_t column = col0 + 32 * (pass / MT) + (lane & 31);
             const float total = decoded_dot<ENC>(data + column * row_stride, input + row * input_dim, input_dim);
             output[row * output_dim + column] = total + (bias != nullptr ? bias[column] : 0.0f);
         }
     }
+}
+
+// The same as a function of its own: the small forms keep the registers and the schedule that their
+// loop has by itself (4 rows of Q6_K, 5,120 -> 178: 23.3 -> 21.8 us).  The large forms, whose loops need
+// every register, would lose some to the call.
+template <std::uint32_t ENC, int MT, int WAVES>
+__device__ __attribute__((noinline)) void take_again_apart(std::uint64_t again, int wave, const std::uint8_t* data,
+                                                           std::int64_t row_stride, const float* input,
+                                                           std::int64_t input_dim, const float* bias, float* output,
+                                                           std::int64_t output_dim, std::int64_t row0,
+                                                           std::int64_t col0) {
+    take_again<ENC, MT, WAVES>(again, wave, data, row_stride, input, input_dim, bias, output, output_dim, row0, col0);
 }
 
 // WAVES waves share a tile of 32 MT input rows x 32 NT weight rows.
@@ -627,9 +652,9 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
                     for (int chunk = 0; chunk < 2; ++chunk) {
                         float eight[8];
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) eight[j] = x[m][chunk][j >> 2][j & 3] * kLift;
+                        for (int j = 0; j < 8; ++j) eight[j] = x[m][chunk][j >> 2][j & 3];
                         a[m][chunk] = cut(eight);
-                        if constexpr (Slice::kMinimum) partial[m][step] += sum_of(eight);
+                        if constexpr (Slice::kMinimum) partial[m][step] += sum_of(eight) * kLift;
                     }
                 }
                 load_inputs(min(2 * unit + step + 1, last_step));
@@ -668,11 +693,10 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
                                                 row0 + 32 * m, col0 + 32 * n + inner);
         }
     }
-    take_again<ENC, WAVES>(again, wave, lane, data, row_stride, input, input_dim, bias, output, output_dim,
-                           [&](int pass, int r, std::int64_t& row, std::int64_t& column) {
-                               row = row0 + 32 * (pass % MT) + 8 * (r >> 2) + 4 * half + (r & 3);
-                               column = col0 + 32 * (pass / MT) + inner;
-                           });
+    if (__ballot(again != 0) != 0) {
+        take_again_apart<ENC, MT, WAVES>(again, wave, data, row_stride, input, input_dim, bias, output, output_dim, row0,
+                                         col0);
+    }
 }
 
 // -- the large form --------------------------------------------------------------------------------
@@ -718,27 +742,32 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
     std::uint8_t* const own = lds + group * kGroupBytes<MT>;
     float* const sums = reinterpret_cast<float*>(own + 2 * kStepBytes<MT>);
     const int quad = lane & 7;
-    const float* x_row[kItems];
+    // (a buffer load takes a register for the row and a scalar for the step; 64-bit addresses took eight
+    // registers and an addition a load: 200 rows of Q8_0 81.8 -> 79.6 us, of Q5_K 86 -> 80)
+    const __amdgpu_buffer_rsrc_t x_tile = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(input + row0 * input_dim), 0, 0xffffffff, 0x00020000);
+    std::uint32_t x_row[kItems];  // bytes from the tile's first row
 #pragma unroll
     for (int item = 0; item < kItems; ++item) {
-        x_row[item] = input + min(row0 + 8 * (2 * item + partner) + (lane >> 3), rows - 1) * input_dim + 4 * quad;
+        const int row = min(8 * (2 * item + partner) + (lane >> 3), static_cast<int>(min(rows - 1 - row0, std::int64_t(64))));
+        x_row[item] = 4 * (static_cast<std::uint32_t>(row) * static_cast<std::uint32_t>(input_dim) + 4 * quad);
     }
     const int target = (quad >> 1) * kOctetBytes + (8 * partner + (lane >> 3)) * 16 + (quad & 1) * 8;
     f32x4_a4 x[kItems];
     const auto load_input = [&](int item, int step) {
-        x[item] = *reinterpret_cast<const f32x4_a4*>(x_row[item] + static_cast<std::int64_t>(min(step, steps - 1)) * 32);
+        x[item] = __builtin_bit_cast(
+            f32x4_a4, __builtin_amdgcn_raw_buffer_load_b128(x_tile, x_row[item], min(step, steps - 1) * 128, 0));
     };
     const auto cut_input = [&](int item, int step) {
         std::uint32_t a0, b0, c0, a1, b1, c1;
-        const float x0 = x[item][0] * kLift, x1 = x[item][1] * kLift, x2 = x[item][2] * kLift, x3 = x[item][3] * kLift;
-        cut_pair(x0, x1, a0, b0, c0);
-        cut_pair(x2, x3, a1, b1, c1);
+        cut_pair(x[item][0], x[item][1], a0, b0, c0);
+        cut_pair(x[item][2], x[item][3], a1, b1, c1);
         std::uint8_t* const stage = own + (step & 1) * kStepBytes<MT> + (item >> 1) * kTermBytes + target + (item & 1) * 256;
         *reinterpret_cast<uint2*>(stage) = make_uint2(c0, c1);
         *reinterpret_cast<uint2*>(stage + MT * kTermBytes) = make_uint2(b0, b1);
         *reinterpret_cast<uint2*>(stage + 2 * MT * kTermBytes) = make_uint2(a0, a1);
         if constexpr (Slice::kMinimum) {
-            float total = (x0 + x1) + (x2 + x3);
+            float total = ((x[item][0] + x[item][1]) + (x[item][2] + x[item][3])) * kLift;
             total += __shfl_xor(total, 1);
             total += __shfl_xor(total, 2);
             total += __shfl_xor(total, 4);  // (the eight lanes of a row store the same sum)
@@ -919,11 +948,9 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
                                                     output, rows, output_dim, row0 + 32 * m, col0 + 32 * n + inner);
         }
     }
-    take_again<ENC, kGroups>(again, group, lane, data, row_stride, input, input_dim, bias, output, output_dim,
-                             [&](int pass, int r, std::int64_t& row, std::int64_t& column) {
-                                 row = row0 + 32 * (pass % MT) + 8 * (r >> 2) + 4 * half + (r & 3);
-                                 column = col0 + 32 * (pass / MT) + inner;
-                             });
+    if (__ballot(again != 0) != 0) {
+        take_again<ENC, MT, kGroups>(again, group, data, row_stride, input, input_dim, bias, output, output_dim, row0, col0);
+    }
 }
 
 template <std::uint32_t ENC, int MT>
@@ -1009,7 +1036,8 @@ void launch_for(const Descriptor& weight, const float* input, const float* bias,
 bool linear_exact_supports(const Descriptor& weight, std::int64_t rows) {
     const std::int64_t tiles = ((rows + 31) / 32) * ((weight.output_dim + 31) / 32);
     return rows > 0 && weight.input_dim > 0 && weight.input_dim % 32 == 0 && block_bytes(weight.encoding) != 0 &&
-           weight.input_dim <= (std::int64_t(1) << 30) && tiles < (std::int64_t(1) << 31);
+           weight.input_dim <= (std::int64_t(1) << 23) &&  // a tile's rows within 32-bit offsets
+           tiles < (std::int64_t(1) << 31);
 }
 
 void launch_linear_exact(const Descriptor& weight, const float* input, const float* bias, float* output,
