@@ -979,15 +979,14 @@ void launch_small(const Descriptor& weight, const float* input, const float* bia
 // 64 x 32 and 64 x 64).  From a sweep over 484 shapes an encoding (4..512 rows, 64..8,192 outputs,
 // 2,048..8,192 columns, every form of each): the middle of the values with which the rule loses least
 // to the fastest form.  Mean and largest loss, and with 1.35, 2.1 and 2.9 for all packed encodings and
-// bf16 (F32 1.4 and 2.1): Q4_K 0.00 and 1.3 % (0.31 and 15), Q5_K 0.30 and 13 (1.4 and 38; its 64 x 128
-// form keeps registers in scratch), Q6_K 0.08 and 18 (the same), Q8_0 0.00 and 0.5 (0.01 and 4), bf16
-// none (0.05 and 13), F32 0.16 and 12 (0.24 and 10).
+// bf16 (F32 1.4 and 2.1): Q4_K 0.01 and 3.6 % (0.31 and 12), Q5_K 0.05 and 8 (0.37 and 20), Q6_K 0.10 and
+// 23 (0.09 and 23), Q8_0 0.00 and 0.4 (0.01 and 4), bf16 none (0.05 and 14), F32 0.13 and 11 (0.39 and 11).
 template <std::uint32_t ENC>
-constexpr double kRounds[3] = {1.4, 2.5, 3.9};  // Q4_K, Q5_K
+constexpr double kRounds[3] = {1.45, 2.1, 2.6};  // Q6_K, Q8_0
 template <>
-constexpr double kRounds<kEncQ6K>[3] = {1.45, 2.1, 2.6};
+constexpr double kRounds<kEncQ4K>[3] = {1.4, 2.5, 3.9};
 template <>
-constexpr double kRounds<kEncQ8_0>[3] = {1.45, 2.1, 2.6};
+constexpr double kRounds<kEncQ5K>[3] = {1.35, 2.5, 3.6};
 template <>
 constexpr double kRounds<kEncBF16>[3] = {1.5, 2.0, 2.4};
 template <>
