@@ -4,16 +4,16 @@
 // A float times 2^24 is the sum of three bf16 numbers (24 significant bits cut into 8 + 8 + 8 by
 // truncation; the last bit of the smallest float becomes 2^-125, which bf16 holds as a normal
 // number, so that nothing is left over down to zero), and the integer code of a packed weight is
-// one bf16 number (at most eight significant bits).  Sums carry the factor to the end.  v_mfma_f32_32x32x16_bf16 multiplies bf16 exactly and adds
-// in float, so three of them per code give the product of the float activations with the codes,
-// at a sixteenth of the cycles of the float instruction each: 3/16 of v_mfma_f32_32x32x2_f32's
-// time.  A sub-block's scale d * sc is exact in float (11 + 6 or 7 bits) and multiplies the
-// sub-block's sums on their way into the accumulators; the minimum's part d_min * m times the
-// sub-block's sum of activations goes in by one float matrix instruction per 64 columns.  A
-// one-hot input row returns the dequantized weight bit for bit: d * sc * q is exact, the
-// subtraction of d_min * m is the one rounding that the decode has.  Float weights are cut into
-// three terms as well (eight products of the nine: the one left out is below 2^-32 of the
-// product), bf16 weights are one term.
+// one bf16 number (at most eight significant bits).  Sums carry the factor to the end.
+// v_mfma_f32_32x32x16_bf16 multiplies bf16 exactly and adds in float, so three of them per code give
+// the product of the float activations with the codes, at a sixteenth of the cycles of the float
+// instruction each: 3/16 of v_mfma_f32_32x32x2_f32's time.  A sub-block's scale d * sc is exact in
+// float (11 + 6 or 7 bits) and multiplies the sub-block's sums on their way into the accumulators; the
+// minimum's part d_min * m times the sub-block's sum of activations goes in by one float matrix
+// instruction per 64 columns.  A one-hot input row returns the dequantized weight bit for bit:
+// d * sc * q is exact, the subtraction of d_min * m is the one rounding that the decode has.  Float
+// weights are cut into three terms as well (eight products of the nine: the one left out is below
+// 2^-32 of the product), bf16 weights are one term.
 //
 // A workgroup's waves share one tile and cut K between them; their sums meet in LDS at the end, in
 // a fixed order.  Two forms:
@@ -25,7 +25,7 @@
 //   them and hand the terms over in LDS.
 // What bounds both is the vector cache: a load instruction that reads 16 bytes from each of 32 rows
 // looks up 32 lines for 1 KB, and a unit pulls some 20 GB/s that way.  200 rows of Q8_0: a look-up in
-// 70 % of the cycles, the matrix cores busy in 26 %, the vector ALU in 37, LDS in 14.  (Requests two
+// 72 % of the cycles, the matrix cores busy in 26 %, the vector ALU in 37, LDS in 15.  (Requests two
 // steps ahead instead of one, and the matrix instructions of a step before its other work instead of
 // between it, made no difference.)  The 64 x 128 form of Q5_K keeps four registers that do not change in
 // its loop in scratch (20 bytes a lane), the 64 x 64 form of F32 seven (32 bytes), read outside of its
