@@ -217,6 +217,22 @@ def test_exact_linear_rows_carry_the_same_bits_within_a_form(cuda, encoding, out
     assert normalised_error(three.cpu().numpy(), many[:3].cpu().numpy()) <= 1e-5
 
 
+@pytest.mark.parametrize("in_dim", [2 ** 23, 2 ** 23 + 256])
+@pytest.mark.parametrize("encoding", [kquant.Q8_0, kquant.BF16])
+def test_exact_linear_on_both_sides_of_its_longest_rows(cuda, encoding, in_dim):
+    """Past 2^23 columns the kernel for any width takes the call.  Bound: its lanes add 2^17 products
+    one after another, which with random signs is off by about sqrt(2^17) 2^-24 = 2e-5 of the result;
+    1e-4 leaves five standard deviations."""
+    torch = torch_()
+    out_dim, rows = 3, 5
+    packed = kquant.quantize(encoding, kquant.synthetic_weights(64, out_dim, in_dim))
+    weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    x = to_device(kquant.synthetic_activations(65, rows, in_dim), cuda)
+    y = tile_ops.linear(weight, x).double()
+    expected = torch.stack([(x.double() * row.double()).sum(dim=1) for row in tile_ops.dequantize(weight)], dim=1)
+    assert float((y - expected).abs().max() / expected.abs().max()) <= 1e-4
+
+
 @pytest.mark.parametrize("rows,out_dim,in_dim", [(3, 67, 512), (5, 67, 512), (60, 5000, 256), (100, 6600, 256), (200, 6600, 256)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
 def test_exact_linear_of_infinities_nan_and_large_activations(cuda, oracle, encoding, rows, out_dim, in_dim):
