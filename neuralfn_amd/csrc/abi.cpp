@@ -176,7 +176,7 @@ int run_small_batch(bool verifier, const Descriptor* const* descriptors, const f
                                     as_stream(stream));
         }
         if (verifier_rows.count > 0) {
-            launch_gemv_rows(verifier_rows, image, rows, clear.count > 0, fill_launch, as_stream(stream));
+            launch_gemv_rows(verifier_rows, image, static_cast<const std::uint8_t*>(workspace), rows, clear.count > 0, fill_launch, as_stream(stream));
         }
         dot_first = static_cast<const float*>(workspace);
         dot_second = nullptr;

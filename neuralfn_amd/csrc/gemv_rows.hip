@@ -21,9 +21,9 @@
 // through a private LDS tile per wave) and the two int8 planes of up to 16 tokens (operand A,
 // fetched in operand order from the image a quantizer launch left in the workspace beside the
 // activation records: lanes that each pick their own 16 bytes out of sixteen records cost the
-// memory pipeline four times the instructions' coalesced rate).  For Q4_K / Q5_K a second
+// memory pipeline four times the instructions' coalesced rate).  For Q4_K / Q5_K of more than eight tokens a second
 // product against the sub-block minimums, spread over K, gives the sums the minimums
-// multiply; Q6_K's offset of 32 is taken off the codes before the product.  A lane then holds,
+// multiply (fewer tokens: multiply-adds with the code sums of the records); Q6_K's offset of 32 is taken off the codes before the product.  A lane then holds,
 // for its weight row and up to 8 tokens, the integers of a unit, and replays the float tail
 // above.  Wave w takes the classes w and 15 - w (an even share of any row length), keeps the
 // four chains of a class per token in registers, and leaves (c0 + c1) + (c2 + c3) per class,
@@ -31,6 +31,16 @@
 // tree's order.  A workgroup walks the tiles blockIdx.x, blockIdx.x + gridDim.x, ... with the
 // loads of the next tile's first block in flight under the last block of the one before.
 // One pass over the weights for up to 16 tokens.
+//
+// What bounds it: a wave issues an instruction every 5 to 8 cycles and two waves fit a SIMD, so the
+// vector ALU is busy a third of the time and memory is asked in bursts (gate and up of seven
+// tokens, Q4_K: only the weights' loads 23.4 us, with the operands' 28.5, everything 35).  Up to
+// eight tokens therefore: two or four scale groups to an operand fragment (half or a quarter of
+// the operand bytes, registers for a second block of packed bytes in flight), the minimums'
+// sums from the records instead of a second pair of products, products issued around the tail
+// before.  Q4_K, 2 x 16,384 rows of 6,656 columns: 39.6 -> 31.2 us at four tokens, 41.9 -> 39.0 at
+// seven, quantizer launch included; Q5_K 44.5 -> 35.8 and 48.2 -> 43.2, Q8_0 54.1 -> 48.2 and
+// 57.0 -> 52.5, Q6_K 58.4 -> 53.3 and 63.1 -> 58.9.
 #include "common.hpp"
 #include "gemv_rows.hpp"
 #include "wave_rows.hpp"
@@ -47,7 +57,7 @@ constexpr int kRowsTile = 32;
 constexpr int kRowsWaves = 8;
 constexpr int kRowsThreads = kRowsWaves * kWave;
 constexpr int kClasses = 16;
-constexpr int kMaxRowsBlocks = 256;  // input_dim up to 65,536: the blocks whose scales a workgroup keeps
+constexpr int kMaxRowsBlocks = 256;  // input_dim up to 65,536
 
 constexpr int kImageFragments = kRowsImageFragments;
 constexpr int kImageBlock = kRowsImageBlock;
@@ -118,6 +128,9 @@ struct RowsFormat {
 struct __attribute__((packed, aligned(2))) RowsPiece {
     std::uint32_t v[4];
 };
+struct __attribute__((packed, aligned(4))) RowsWords {
+    std::uint32_t v[2];
+};
 struct __attribute__((packed, aligned(2))) RowsHalfPiece {
     std::uint32_t v[2];
 };
@@ -135,8 +148,11 @@ struct RowsPacked {
 
 // Operand A of the eight 32-value groups of a block: two sets, used by the matrix instructions
 // where they arrive.
+template <int S>
 struct RowsOperands {
-    v4i a[8];
+    static constexpr int kFragments = S;  // 8 / rows_groups(S)
+    v4i a[kFragments];
+    v2i extra;  // this lane's entry of the block's code sums and scales
 };
 
 __device__ __forceinline__ v16i mfma_i8(v4i a, v4i b, v16i c) {
@@ -164,14 +180,16 @@ __device__ __forceinline__ void rows_lds_fence() {
 // blocks has 16 on the left and 10 on the right): for tile counts that leave much of the
 // chip idle in the last pass over whole tiles (272 tiles on 256 units).
 template <std::uint32_t ENC, int S, bool SPLIT>
-__global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(
-    const std::uint8_t* __restrict__ image, int tokens, int input_dim, std::uint32_t total_tiles,
-    std::uint32_t left_groups, ProjectionSet set) {
+__global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
+    const std::uint8_t* __restrict__ image, const std::uint8_t* __restrict__ records, int tokens,
+    int input_dim, std::uint32_t total_tiles, std::uint32_t left_groups, ProjectionSet set) {
     constexpr bool kQ5 = ENC == kEncQ5K;
     using F = RowsFormat<ENC>;
     constexpr int kBlockBytes = F::kBlockBytes;
     constexpr int kQuants = kQ5 ? 48 : 16;
     constexpr int kTokens = 2 * S;
+    constexpr int kGroups = rows_groups(S);
+    constexpr bool kDeep = S <= 4;  // registers for two blocks of packed bytes in flight
     // (two buffers of class sums: the workgroup's waves meet once per tile)
     constexpr int kOwnClasses = SPLIT ? kClasses / 2 : kClasses;
     __shared__ float class_sums[2][kOwnClasses][kTokens][kRowsTile];
@@ -242,31 +260,68 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(
     };
     std::uint8_t* const my_tile = packed_tiles[wave];
     const std::uint8_t* const my_row = my_tile + j * F::kSlotBytes + F::kSlotOrigin;
-
-    // this wave's steps of a tile: the blocks of class `wave`, then those of class 15 - wave
-    // (SPLIT: the one class 8 (right half) + wave)
-    const int class0 = SPLIT ? (right_half ? 8 : 0) + wave : wave;
-    const int class1 = kClasses - 1 - wave;
-    const int count0 = class0 < blocks ? (blocks - class0 + kClasses - 1) / kClasses : 0;
-    int count1 = class1 < blocks ? (blocks - class1 + kClasses - 1) / kClasses : 0;
-    if constexpr (SPLIT) {
-        // (no second class; a value the optimizer cannot see through, so that the walk below
-        // compiles as it does for two classes: with a known zero it is scheduled with far
-        // more registers, and spills)
-        count1 = 0;
-        asm volatile("" : "+s"(count1));
+    // What the float tails take from the activation records and the image.  Up to eight tokens it comes with a
+    // block's operands, eight bytes a lane, and goes through LDS: for Q4_K and Q5_K the code sums
+    // of two neighbouring 32-value groups of a token (entry [pair of groups][token]), then the
+    // scale of every token.  More tokens leave no registers for that: the scales of all the wave's
+    // blocks are brought to LDS when it starts.
+    constexpr bool kSums = !F::kQ6 && !F::kQ8 && kDeep;
+    constexpr int kScaleEntry = kSums ? 4 * kTokens : 0;
+    constexpr int kEntries = kDeep ? kScaleEntry + kTokens : 1;
+    constexpr int kMaxSteps = kDeep ? 1 : kMaxRowsBlocks / kRowsWaves;
+    static_assert(kEntries <= kWave, "an entry a lane");
+    __shared__ __attribute__((aligned(16))) v2i extras[kRowsWaves][kEntries];
+    __shared__ __attribute__((aligned(16))) float step_scales[kRowsWaves][kMaxSteps][kDeep ? 1 : kTokens];
+    v2i* const my_extras = extras[wave];
+    const bool sums_lane = lane < kScaleEntry;
+    const int extra_entry = sums_lane ? (lane & 3) * kTokens + (lane >> 2) : lane;
+    const std::uint8_t* extra_base = nullptr;  // of block 0; from block to block `extra_stride` on
+    std::uint32_t extra_stride = 0;
+    if constexpr (kDeep) {
+        const int token = sums_lane ? min(lane >> 2, tokens - 1) : min(lane - kScaleEntry, kTokens - 1);
+        extra_base = sums_lane
+            ? records + static_cast<std::uint32_t>(token * blocks) * kActRecord + kRecordSums + (lane & 3) * 8
+            : image + kImageFragments + token * 4;
+        extra_stride = sums_lane ? kActRecord : kImageBlock;
     }
-    const int total = count0 + count1;
 
-    auto block_of = [&](int step) {
-        return step < count0 ? class0 + kClasses * step : class1 + kClasses * (step - count0);
+    // A wave's steps of a tile: the blocks of class r, then those of class 15 - r (SPLIT: of the one
+    // class r or 8 + r), r = wave for the first tile.  Rows whose blocks are no multiple of 16 give
+    // some r a block more than others (26 blocks: r = 6 and 7 have four, the others three), so r
+    // moves on by two with every tile and all waves get the same over four tiles (rows of fewer
+    // than 16 blocks leave some r nothing and stay).
+    const int role_step = kDeep && blocks >= kClasses ? 2 : 0;
+    struct Role {
+        int class0, class1, count0, total;
     };
+    const auto role_of = [&](int r) {
+        Role role;
+        role.class0 = (SPLIT && right_half ? 8 : 0) + r;
+        role.class1 = kClasses - 1 - r;
+        role.count0 = role.class0 < blocks ? (blocks - role.class0 + kClasses - 1) / kClasses : 0;
+        int count1 = role.class1 < blocks ? (blocks - role.class1 + kClasses - 1) / kClasses : 0;
+        if constexpr (SPLIT) {
+            // (no second class; a value the optimizer cannot see through, so that the walk below
+            // compiles as it does for two classes: with a known zero it is scheduled with far
+            // more registers, and spills)
+            count1 = 0;
+            asm volatile("" : "+s"(count1));
+        }
+        role.total = role.count0 + count1;
+        return role;
+    };
+    const auto block_of = [&](const Role& role, int step) {
+        return step < role.count0 ? role.class0 + kClasses * step : role.class1 + kClasses * (step - role.count0);
+    };
+    int fetch_r = wave;
+    Role fetch_role = role_of(fetch_r);
+    Role role = fetch_role;  // of the tile being worked on
     std::uint32_t fetch_tile = first_tile;
     int fetch_step = 0;
     aim(fetch_tile);
-    // the loads of the next step of the walk; past its end the last block again
-    auto fetch = [&](RowsPacked<ENC>& stage, RowsOperands& operands) {
-        const int block = min(block_of(min(fetch_step, max(total - 1, 0))), blocks - 1);
+    // the packed bytes of the next step of the walk; past its end the last block again
+    auto fetch_packed = [&](RowsPacked<ENC>& stage) {
+        const int block = min(block_of(fetch_role, min(fetch_step, max(fetch_role.total - 1, 0))), blocks - 1);
         const std::uint8_t* weights = tile_rows + static_cast<std::int64_t>(block) * kBlockBytes;
         // (a Q6_K block with an odd index lies two bytes further from a word than its row does)
         const std::uint32_t shifted = F::kQ6 ? row_parity ^ (0u - static_cast<std::uint32_t>(block & 1)) : 0u;
@@ -282,9 +337,25 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(
                 stage.chunk[i] = *reinterpret_cast<const v4u*>(weights + chunk_offset[i]);
             }
         }
+        if (++fetch_step >= fetch_role.total && fetch_tile + tile_stride < total_tiles) {
+            fetch_step = 0;
+            fetch_tile += tile_stride;
+            fetch_r = (fetch_r + role_step) & (kRowsWaves - 1);
+            fetch_role = role_of(fetch_r);
+            aim(fetch_tile);
+        }
+    };
+    // ... and the operands of a block
+    auto fetch_operands = [&](RowsOperands<S>& operands, int wanted) {
+        const int block = min(wanted, blocks - 1);
+        if constexpr (kDeep) {
+            // (the second word of a scale entry is the next token's: the image has 16)
+            operands.extra = __builtin_bit_cast(
+                v2i, *reinterpret_cast<const RowsWords*>(extra_base + static_cast<std::uint32_t>(block) * extra_stride));
+        }
         const std::uint8_t* fragments = image + static_cast<std::int64_t>(block) * kImageBlock;
 #pragma unroll
-        for (int sub = 0; sub < 8; ++sub) {
+        for (int sub = 0; sub < RowsOperands<S>::kFragments; ++sub) {
             if constexpr (F::kQ6) {
                 // the sixteen values 16 s..+15 of a 32-value group are what the image keeps for
                 // lanes 32 s..+31: this lane takes bytes 8 h..+7 of row j's sixteen, for s = 0, 1
@@ -296,15 +367,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(
                 operands.a[sub] = *reinterpret_cast<const v4i*>(fragments + sub * 1024 + lane * 16);
             }
         }
-        if (++fetch_step >= total && fetch_tile + tile_stride < total_tiles) {
-            fetch_step = 0;
-            fetch_tile += tile_stride;
-            aim(fetch_tile);
-        }
     };
-
-    constexpr int kMaxSteps = kMaxRowsBlocks / kRowsWaves;
-    __shared__ __attribute__((aligned(16))) float step_scales[kRowsWaves][kMaxSteps][16];
 
     float acc[4][S];
 #pragma unroll
@@ -335,11 +398,14 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(
         }
     };
 
-    auto compute = [&](const RowsOperands& stage, int step) {
+    auto compute = [&](const RowsOperands<S>& stage, int step) {
         const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         float scale[S];
 #pragma unroll
-        for (int slot = 0; slot < S; ++slot) scale[slot] = step_scales[wave][step][S * h + slot];
+        for (int slot = 0; slot < S; ++slot) {
+            scale[slot] = kDeep ? __int_as_float(my_extras[kScaleEntry + S * h + slot][0])
+                                : step_scales[wave][step][S * h + slot];
+        }
         if constexpr (F::kQ6) {
             // Q6_K (neuralfn/csrc/native_gpt2/resident_glimmer.cpp:591-616): per half of 128
             // values 64 bytes of low nibbles (quarters 0 / 2 in bytes 0..31, 1 / 3 in 32..63) and
@@ -387,18 +453,36 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(
                     float unit_value[S];
 #pragma unroll
                     for (int slot = 0; slot < S; ++slot) unit_value[slot] = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const v4i both = stage.a[4 * half + k];
+                    const auto product = [&](int k) {
+                        const v4i both = stage.a[(4 * half + k) / kGroups];
                         const v2i fragment = s == 0 ? v2i{both[0], both[1]} : v2i{both[2], both[3]};
-                        const v16i dots = mfma_i8_k16(fragment, codes[k], zero);
+                        return mfma_i8_k16(fragment, codes[k], zero);
+                    };
+                    const auto tail = [&](int k, const v16i& dots) {
 #pragma unroll
                         for (int slot = 0; slot < S; ++slot) {
                             // |4 (256 hi + lo)| <= 4 * 16 * 32 * 32512 < 2^27: exact in int32
-                            const int bracket = (dots[2 * slot] << 8) + dots[2 * slot + 1];
+                            const int at = (4 * half + k) % kGroups * 2 * S + 2 * slot;
+                            const int bracket = (dots[at] << 8) + dots[at + 1];
                             unit_value[slot] =
                                 fmaf(quarter_scale[2 * k + s], static_cast<float>(bracket), unit_value[slot]);
                         }
+                    };
+                    if constexpr (kDeep) {
+                        // (the next quarter's product under the tail of this one, as for Q4_K below)
+                        v16i dots[2];
+                        dots[0] = product(0);
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            if (k < 3) dots[(k + 1) & 1] = product(k + 1);
+                            __builtin_amdgcn_sched_barrier(0);
+                            tail(k, dots[k & 1]);
+                            asm volatile("" : : "v"(dots[k & 1]));
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) tail(k, product(k));
                     }
 #pragma unroll
                     for (int slot = 0; slot < S; ++slot) {
@@ -417,15 +501,17 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(
                 const RowsPiece c1 = *reinterpret_cast<const RowsPiece*>(pair + 36 + 16 * h);
                 const float d0 = half_bits_to_float(*reinterpret_cast<const std::uint16_t*>(pair));
                 const float d1 = half_bits_to_float(*reinterpret_cast<const std::uint16_t*>(pair + 34));
-                const v16i dots0 = mfma_i8(stage.a[2 * p], v4i{static_cast<int>(c0.v[0]), static_cast<int>(c0.v[1]),
+                const v16i dots0 = mfma_i8(stage.a[2 * p / kGroups], v4i{static_cast<int>(c0.v[0]), static_cast<int>(c0.v[1]),
                                                                 static_cast<int>(c0.v[2]), static_cast<int>(c0.v[3])}, zero);
-                const v16i dots1 = mfma_i8(stage.a[2 * p + 1], v4i{static_cast<int>(c1.v[0]), static_cast<int>(c1.v[1]),
+                const v16i dots1 = mfma_i8(stage.a[(2 * p + 1) / kGroups], v4i{static_cast<int>(c1.v[0]), static_cast<int>(c1.v[1]),
                                                                     static_cast<int>(c1.v[2]), static_cast<int>(c1.v[3])}, zero);
 #pragma unroll
                 for (int slot = 0; slot < S; ++slot) {
                     // |256 hi + lo| <= 32 * 127 * 32512 < 2^28: exact in int32
-                    const int bracket0 = (dots0[2 * slot] << 8) + dots0[2 * slot + 1];
-                    const int bracket1 = (dots1[2 * slot] << 8) + dots1[2 * slot + 1];
+                    const int at0 = 2 * p % kGroups * 2 * S + 2 * slot;
+                    const int at1 = (2 * p + 1) % kGroups * 2 * S + 2 * slot;
+                    const int bracket0 = (dots0[at0] << 8) + dots0[at0 + 1];
+                    const int bracket1 = (dots1[at1] << 8) + dots1[at1 + 1];
                     const float value = fmaf(d1, static_cast<float>(bracket1), d0 * static_cast<float>(bracket0));
                     acc[p][slot] = fmaf(scale[slot], value, acc[p][slot]);
                 }
@@ -449,10 +535,9 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(
             const std::uint32_t mn_hi = ((head.w >> 4) & 0x0f0f0f0fu) | ((head.z >> 2) & 0x30303030u);
             const float d = half_bits_to_float(head.x & 0xffffu);
             const float dmin = half_bits_to_float(head.x >> 16);
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
+            // the codes of pair p (sub-blocks 2p and 2p + 1), this lane's sixteen of each
+            const auto unpack = [&](int p, v4i& low, v4i& upper) {
                 const std::uint32_t packed[4] = {quants[p].x, quants[p].y, quants[p].z, quants[p].w};
-                v4i low, upper;
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
                     std::uint32_t lo = packed[w] & 0x0f0f0f0fu;
@@ -466,54 +551,117 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(
                     low[w] = static_cast<int>(lo);
                     upper[w] = static_cast<int>(up);
                 }
+            };
+            // the float tail of pair p for the token slots first..last-1 (`sums`: of the products
+            // with the minimums, for more than eight tokens)
+            const auto tail = [&](int p, const v16i& dots_a, const v16i& dots_b, const v16i& min_dots, int first,
+                                  int last) {
                 const std::uint32_t sc_word = p < 2 ? sc_lo : sc_hi;
                 const std::uint32_t mn_word = p < 2 ? mn_lo : mn_hi;
                 const int scale_a = static_cast<int>((sc_word >> (16 * (p & 1))) & 0xffu);
                 const int scale_b = static_cast<int>((sc_word >> (16 * (p & 1) + 8)) & 0xffu);
                 const int min_a = static_cast<int>((mn_word >> (16 * (p & 1))) & 0xffu);
                 const int min_b = static_cast<int>((mn_word >> (16 * (p & 1) + 8)) & 0xffu);
-                const int spread_a = static_cast<int>(__umul24(min_a, 0x010101u)) | (min_a << 24);
-                const int spread_b = static_cast<int>(__umul24(min_b, 0x010101u)) | (min_b << 24);
-                const v4i mins_a = {spread_a, spread_a, spread_a, spread_a};
-                const v4i mins_b = {spread_b, spread_b, spread_b, spread_b};
                 // the sub-block scales times 256, opaque to the optimizer: it would otherwise factor
                 // scale * (256 * hi + lo) out and pay a full 32-bit multiplication for it
                 int scale_a256, scale_b256;
                 asm("v_lshlrev_b32 %0, 8, %1" : "=v"(scale_a256) : "v"(scale_a));
                 asm("v_lshlrev_b32 %0, 8, %1" : "=v"(scale_b256) : "v"(scale_b));
-                const v16i dots_a = mfma_i8(stage.a[2 * p], low, zero);
-                const v16i dots_b = mfma_i8(stage.a[2 * p + 1], upper, zero);
-                // min_a * sum(codes of a) + min_b * sum(codes of b), per plane
-                const v16i sums = mfma_i8(stage.a[2 * p + 1], mins_b, mfma_i8(stage.a[2 * p], mins_a, zero));
 #pragma unroll
-                for (int slot = 0; slot < S; ++slot) {
-                    float codes;
-                    if constexpr (kQ5) {
-                        const int weighted_hi =
-                            __mul24(scale_a, dots_a[2 * slot]) + __mul24(scale_b, dots_b[2 * slot]);
-                        const int weighted_lo =
-                            __mul24(scale_a, dots_a[2 * slot + 1]) + __mul24(scale_b, dots_b[2 * slot + 1]);
-                        codes = fmaf(static_cast<float>(weighted_hi), 256.0f, static_cast<float>(weighted_lo));
-                    } else {
-                        // 4-bit codes: 256 * weighted_hi + weighted_lo stays below 2^31
-                        // (2 * 63 * 32 * 15 * (127 * 256 + 128)), and one conversion rounds the
-                        // exact integer as the fused multiply-add of the two exact floats does
-                        // (a chain of multiply-adds: the empty statements keep the optimizer from
-                        // turning it into a tree with one more instruction)
-                        int weighted = __mul24(scale_a256, dots_a[2 * slot]);
-                        asm("" : "+v"(weighted));
-                        weighted += __mul24(scale_b256, dots_b[2 * slot]);
-                        asm("" : "+v"(weighted));
-                        weighted += __mul24(scale_a, dots_a[2 * slot + 1]);
-                        asm("" : "+v"(weighted));
-                        weighted += __mul24(scale_b, dots_b[2 * slot + 1]);
-                        codes = static_cast<float>(weighted);
+                for (int slot = first; slot < last; slot += 2) {
+                    // (sums of both sub-blocks for two tokens)
+                    v4i sums = {0, 0, 0, 0};
+                    if constexpr (kSums) sums = *reinterpret_cast<const v4i*>(my_extras + p * kTokens + S * h + slot);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        const int at = slot + t;
+                        const int in_a = 2 * p % kGroups * 2 * S + 2 * at;
+                        const int in_b = (2 * p + 1) % kGroups * 2 * S + 2 * at;
+                        float codes;
+                        if constexpr (kQ5) {
+                            const int weighted_hi =
+                                __mul24(scale_a, dots_a[in_a]) + __mul24(scale_b, dots_b[in_b]);
+                            const int weighted_lo =
+                                __mul24(scale_a, dots_a[in_a + 1]) + __mul24(scale_b, dots_b[in_b + 1]);
+                            codes = fmaf(static_cast<float>(weighted_hi), 256.0f, static_cast<float>(weighted_lo));
+                        } else {
+                            // 4-bit codes: 256 * weighted_hi + weighted_lo stays below 2^31
+                            // (2 * 63 * 32 * 15 * (127 * 256 + 128)), and one conversion rounds the
+                            // exact integer as the fused multiply-add of the two exact floats does
+                            // (a chain of multiply-adds: the empty statements keep the optimizer from
+                            // turning it into a tree with one more instruction)
+                            int weighted = __mul24(scale_a256, dots_a[in_a]);
+                            asm("" : "+v"(weighted));
+                            weighted += __mul24(scale_b256, dots_b[in_b]);
+                            asm("" : "+v"(weighted));
+                            weighted += __mul24(scale_a, dots_a[in_a + 1]);
+                            asm("" : "+v"(weighted));
+                            weighted += __mul24(scale_b, dots_b[in_b + 1]);
+                            codes = static_cast<float>(weighted);
+                        }
+                        int weighted_min;
+                        if constexpr (kSums) {
+                            // (a group's sum of codes stays below 32 * 32,512 < 2^23)
+                            weighted_min = __mul24(min_a, sums[2 * t]);
+                            asm("" : "+v"(weighted_min));
+                            weighted_min += __mul24(min_b, sums[2 * t + 1]);
+                        } else {
+                            weighted_min = min_dots[2 * at] * 256 + min_dots[2 * at + 1];
+                        }
+                        const float value = fmaf(-dmin, static_cast<float>(weighted_min), d * codes);
+                        acc[p][at] = fmaf(scale[at], value, acc[p][at]);
                     }
-                    const int weighted_min = sums[2 * slot] * 256 + sums[2 * slot + 1];
-                    const float value = fmaf(-dmin, static_cast<float>(weighted_min), d * codes);
-                    acc[p][slot] = fmaf(scale[slot], value, acc[p][slot]);
+                }
+            };
+            if constexpr (!kSums) {
+                // min_a * sum(codes of a) + min_b * sum(codes of b) per plane as products with the
+                // minimums spread over K: more than eight tokens leave no registers for the code sums
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    v4i low, upper;
+                    unpack(p, low, upper);
+                    const std::uint32_t mn_word = p < 2 ? mn_lo : mn_hi;
+                    const int min_a = static_cast<int>((mn_word >> (16 * (p & 1))) & 0xffu);
+                    const int min_b = static_cast<int>((mn_word >> (16 * (p & 1) + 8)) & 0xffu);
+                    const int spread_a = static_cast<int>(__umul24(min_a, 0x010101u)) | (min_a << 24);
+                    const int spread_b = static_cast<int>(__umul24(min_b, 0x010101u)) | (min_b << 24);
+                    const v4i mins_a = {spread_a, spread_a, spread_a, spread_a};
+                    const v4i mins_b = {spread_b, spread_b, spread_b, spread_b};
+                    const v16i dots_a = mfma_i8(stage.a[2 * p], low, zero);
+                    const v16i dots_b = mfma_i8(stage.a[2 * p + 1], upper, zero);
+                    const v16i min_dots = mfma_i8(stage.a[2 * p + 1], mins_b, mfma_i8(stage.a[2 * p], mins_a, zero));
+                    tail(p, dots_a, dots_b, min_dots, 0, S);
+                }
+            } else {
+                // The products of pair p + 1 are issued around the tail of pair p, into a second set of
+                // result registers that stay whole until their tail has read them (the unused part of
+                // a result handed to another value would make its writer wait for the product).
+                constexpr int kHalf = S == 2 ? 2 : S / 2;
+                v16i dots_a[2], dots_b[2];
+                {
+                    v4i low, upper;
+                    unpack(0, low, upper);
+                    dots_a[0] = mfma_i8(stage.a[0], low, zero);
+                    dots_b[0] = mfma_i8(stage.a[1 / kGroups], upper, zero);
+                }
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    v4i low, upper;
+                    if (p < 3) {
+                        unpack(p + 1, low, upper);
+                        dots_a[(p + 1) & 1] = mfma_i8(stage.a[(2 * p + 2) / kGroups], low, zero);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    tail(p, dots_a[p & 1], dots_b[p & 1], zero, 0, kHalf);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (p < 3) dots_b[(p + 1) & 1] = mfma_i8(stage.a[(2 * p + 3) / kGroups], upper, zero);
+                    __builtin_amdgcn_sched_barrier(0);
+                    tail(p, dots_a[p & 1], dots_b[p & 1], zero, kHalf, S);
+                    asm volatile("" : : "v"(dots_a[p & 1]), "v"(dots_b[p & 1]));
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
+            rows_lds_fence();  // the next block's entries stay behind these reads
         }
     };
     // a class is complete: (c0 + c1) + (c2 + c3) per token goes to LDS
@@ -569,57 +717,92 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(
         work_tile += tile_stride;
     };
 
-    if (total == 0) {
+    if (role.total == 0) {
         // (rows of fewer blocks than classes: this wave only takes part in the sums)
         for (int n = 0; n < my_tiles; ++n) {
-            finish_class(class0);
-            if constexpr (!SPLIT) finish_class(class1);
+            finish_class(role.class0);
+            if constexpr (!SPLIT) finish_class(role.class1);
             finish_tile();
         }
         return;
     }
-    // One set of registers for the packed bytes, two named ones for the operands (an array of
-    // them indexed in the loop ends up in scratch memory).  A block's loads are requested when
-    // the block before has gone to LDS, so one block's arithmetic covers them; the second is
-    // requested only when the first has arrived: more requests at the start of a launch make
-    // it slower on this chip, not faster.  Past the end of the walk a request repeats the last
+    // One set of registers for the packed bytes (up to eight tokens two), two for the operands, all
+    // named (an array of them indexed in the loop ends up in scratch memory).  A block's loads are
+    // requested when the block before it (two before it) has gone to LDS, so one block's
+    // arithmetic (two blocks') covers them.  Past the end of the walk a request repeats the last
     // block, so that the number of loads in flight is the same on every path.
-    RowsPacked<ENC> packed;
-    RowsOperands even, odd;
-    fetch(packed, even);
-    // the activation scales of this wave's blocks, 16 tokens each: once into LDS (requested
-    // behind the first block's loads, so that nothing waits for them alone)
-    for (int index = lane; index < total * 16; index += kWave) {
-        const int block = block_of(index >> 4);
-        step_scales[wave][index >> 4][index & 15] = reinterpret_cast<const float*>(
-            image + static_cast<std::int64_t>(block) * kImageBlock + kImageFragments)[index & 15];
+    RowsPacked<ENC> packed_even, packed_odd;
+    RowsOperands<S> even, odd;
+    fetch_packed(packed_even);
+    fetch_operands(even, block_of(role, 0));
+    if constexpr (kDeep) {
+        fetch_packed(packed_odd);
+    } else {
+        // (requested behind the first block's loads, so that nothing waits for them alone)
+        for (int index = lane; index < role.total * kTokens; index += kWave) {
+            const int block = block_of(role, index / kTokens);
+            step_scales[wave][index / kTokens][index % kTokens] = reinterpret_cast<const float*>(
+                image + static_cast<std::int64_t>(block) * kImageBlock + kImageFragments)[index % kTokens];
+        }
     }
     int work_step = 0;
-    // (class0 = wave has at least as many blocks as class1 = 15 - wave; a class without
-    // blocks leaves the zeros the sums start from)
+    // (class0 = r has at least as many blocks as class1 = 15 - r; a class without blocks leaves
+    // the zeros the sums start from)
     auto finish_step = [&]() {
-        if (work_step == count0 - 1) finish_class(class0);
-        if (work_step == total - 1) {
-            if constexpr (!SPLIT) finish_class(class1);
+        if (work_step == role.count0 - 1) finish_class(role.class0);
+        if (work_step == role.total - 1) {
+            if constexpr (!SPLIT) finish_class(role.class1);
             finish_tile();
             work_step = 0;
+            role = role_of((role.class0 + role_step) & (kRowsWaves - 1));
         } else {
             ++work_step;
         }
     };
-    const int steps = my_tiles * total;
-    for (int step = 0; step < steps; step += 2) {
+    // the block after the one being worked on (past the end of the walk: any)
+    auto next_block = [&]() {
+        if (work_step < role.total - 1) return block_of(role, work_step + 1);
+        return (SPLIT && right_half ? 8 : 0) + ((role.class0 + role_step) & (kRowsWaves - 1));
+    };
+    // one step of the walk: its packed bytes go to LDS, the operands of the next step and the packed
+    // bytes of the one after that are requested, its products are taken
+    auto take_step = [&](RowsPacked<ENC>& packed, const RowsOperands<S>& here, RowsOperands<S>& next) {
         stage_to_lds(packed);
+        if constexpr (kDeep) {
+            if (lane < kEntries) my_extras[extra_entry] = here.extra;
+        }
         rows_lds_fence();
-        fetch(packed, odd);
-        compute(even, work_step);
+        // (in the order in which they are waited for)
+        if constexpr (!kDeep) fetch_packed(packed);
+        fetch_operands(next, next_block());
+        if constexpr (kDeep) fetch_packed(packed);
+        compute(here, work_step);
         finish_step();
-        if (step + 1 < steps) {
-            stage_to_lds(packed);
-            rows_lds_fence();
-            fetch(packed, even);
-            compute(odd, work_step);
-            finish_step();
+    };
+    // (a loop of whole pairs with one exit at its end, so that the number of loads in flight is the
+    // same wherever a wait counts them)
+    int steps = 0;
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {  // (r comes round after four tiles)
+        steps += role_of((wave + n * role_step) & (kRowsWaves - 1)).total * ((my_tiles - n + 3) >> 2);
+    }
+    if constexpr (kDeep) {
+        if (steps >= 2) {
+            do {
+                take_step(packed_even, even, odd);
+                take_step(packed_odd, odd, even);
+                steps -= 2;
+            } while (steps >= 2);
+        }
+        if (steps != 0) take_step(packed_even, even, odd);
+    } else {
+        // (nothing is in flight behind the packed bytes that a step waits for; a third copy of
+        // the step spills)
+        while (true) {
+            take_step(packed_even, even, odd);
+            if (--steps == 0) break;
+            take_step(packed_even, odd, even);
+            if (--steps == 0) break;
         }
     }
 }
@@ -689,25 +872,25 @@ RowsPlan plan_rows(std::uint32_t tiles, std::int64_t input_dim, bool may_split, 
 }
 
 template <std::uint32_t ENC, bool SPLIT>
-void launch_form(const ProjectionSet& set, const std::uint8_t* image, int tokens, std::uint32_t tiles,
-                 const RowsPlan& plan, hipStream_t stream) {
+void launch_form(const ProjectionSet& set, const std::uint8_t* image, const std::uint8_t* records,
+                 int tokens, std::uint32_t tiles, const RowsPlan& plan, hipStream_t stream) {
     const dim3 grid(plan.groups), block(kRowsThreads);
     const int input_dim = static_cast<int>(set.input_dim);
     if (tokens <= 4) {
-        hipLaunchKernelGGL((gemv_rows_kernel<ENC, 2, SPLIT>), grid, block, 0, stream, image, tokens,
+        hipLaunchKernelGGL((gemv_rows_kernel<ENC, 2, SPLIT>), grid, block, 0, stream, image, records, tokens,
                            input_dim, tiles, plan.left_groups, set);
     } else if (tokens <= 8) {
-        hipLaunchKernelGGL((gemv_rows_kernel<ENC, 4, SPLIT>), grid, block, 0, stream, image, tokens,
+        hipLaunchKernelGGL((gemv_rows_kernel<ENC, 4, SPLIT>), grid, block, 0, stream, image, records, tokens,
                            input_dim, tiles, plan.left_groups, set);
     } else {
-        hipLaunchKernelGGL((gemv_rows_kernel<ENC, 8, SPLIT>), grid, block, 0, stream, image, tokens,
+        hipLaunchKernelGGL((gemv_rows_kernel<ENC, 8, SPLIT>), grid, block, 0, stream, image, records, tokens,
                            input_dim, tiles, plan.left_groups, set);
     }
 }
 
 template <std::uint32_t ENC>
-void launch_encoding(ProjectionSet set, const std::uint8_t* image, int tokens, bool outputs_cleared,
-                     bool fill_launch, hipStream_t stream) {
+void launch_encoding(ProjectionSet set, const std::uint8_t* image, const std::uint8_t* records,
+                     int tokens, bool outputs_cleared, bool fill_launch, hipStream_t stream) {
     std::uint32_t tiles = 0;
     for (int index = 0; index < set.count; ++index) {
         set.op[index].first_tile = tiles;
@@ -715,9 +898,9 @@ void launch_encoding(ProjectionSet set, const std::uint8_t* image, int tokens, b
     }
     const RowsPlan plan = plan_rows(tiles, set.input_dim, outputs_cleared, fill_launch);
     if (plan.split) {
-        launch_form<ENC, true>(set, image, tokens, tiles, plan, stream);
+        launch_form<ENC, true>(set, image, records, tokens, tiles, plan, stream);
     } else {
-        launch_form<ENC, false>(set, image, tokens, tiles, plan, stream);
+        launch_form<ENC, false>(set, image, records, tokens, tiles, plan, stream);
     }
 }
 
@@ -795,17 +978,18 @@ void launch_fill_outputs(const ProjectionSet& clear, std::int64_t rows, hipStrea
                        static_cast<std::uint8_t*>(nullptr), 0, static_cast<int>(rows), 0, clear);
 }
 
-void launch_gemv_rows(const ProjectionSet& set, const std::uint8_t* image, std::int64_t rows,
+void launch_gemv_rows(const ProjectionSet& set, const std::uint8_t* image,
+                      const std::uint8_t* records, std::int64_t rows,
                       bool outputs_cleared, bool fill_launch, hipStream_t stream) {
     for (const std::uint32_t encoding : kRowsEncodings) {
         const ProjectionSet group = encoding_group(set, encoding);
         if (group.count == 0) continue;
         const int tokens = static_cast<int>(rows);
         switch (encoding) {
-            case kEncQ4K: launch_encoding<kEncQ4K>(group, image, tokens, outputs_cleared, fill_launch, stream); break;
-            case kEncQ5K: launch_encoding<kEncQ5K>(group, image, tokens, outputs_cleared, fill_launch, stream); break;
-            case kEncQ6K: launch_encoding<kEncQ6K>(group, image, tokens, outputs_cleared, fill_launch, stream); break;
-            default: launch_encoding<kEncQ8_0>(group, image, tokens, outputs_cleared, fill_launch, stream); break;
+            case kEncQ4K: launch_encoding<kEncQ4K>(group, image, records, tokens, outputs_cleared, fill_launch, stream); break;
+            case kEncQ5K: launch_encoding<kEncQ5K>(group, image, records, tokens, outputs_cleared, fill_launch, stream); break;
+            case kEncQ6K: launch_encoding<kEncQ6K>(group, image, records, tokens, outputs_cleared, fill_launch, stream); break;
+            default: launch_encoding<kEncQ8_0>(group, image, records, tokens, outputs_cleared, fill_launch, stream); break;
         }
     }
 }

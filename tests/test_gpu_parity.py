@@ -760,6 +760,28 @@ def test_verifier_matrix_core_rows_equal_the_one_row_kernel(cuda, oracle, encodi
                 assert_bits_equal(whole[row:row + 1].contiguous(), part, f"row {row} of {rows}")
 
 
+@pytest.mark.parametrize("in_dim", [4096, 4352, 6656])
+@pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q6_K, kquant.Q8_0])
+def test_verifier_matrix_core_rows_of_many_tiles_a_workgroup(cuda, encoding, in_dim):
+    """Up to eight tokens a wave's share of a row's blocks moves on from tile to tile (rows of 16,
+    17 and 26 blocks: even shares, one wave with a block more, two) and comes round after four
+    tiles: five and six tiles a workgroup, the last one part of a tile, against the one-row call."""
+    torch = torch_()
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    out_dim = 32 * (5 * units + units // 3) + 9
+    rows_of = torch.from_numpy(random_packed(encoding, 512, in_dim, 77).reshape(512, -1)).to(cuda)
+    chosen = torch.randint(0, 512, (out_dim,), generator=torch.Generator().manual_seed(78)).to(cuda)
+    weight = tile_ops.PackedWeight(encoding, out_dim, in_dim, rows_of.index_select(0, chosen).reshape(-1))
+    x = to_device(kquant.synthetic_activations(79, 8, in_dim), cuda)
+    one = tile_ops.small_batch_workspace(1, in_dim)
+    alone = [tile_ops.mmvq_linear(weight, x[row:row + 1], one) for row in range(8)]
+    for rows in (4, 7, 8):
+        workspace = tile_ops.small_batch_workspace(rows, in_dim)
+        batch = tile_ops.multi_linear([weight], x[:rows], workspace, family="mmvq")[0]
+        for row in range(rows):
+            assert_bits_equal(batch[row:row + 1].contiguous(), alone[row], f"row {row} of {rows}")
+
+
 @pytest.mark.parametrize("in_dim,out_dim", [(6656, 3000), (6656, 4608), (13312, 2100), (4096, 2500)])
 def test_q6k_rows_carry_the_same_bits_wherever_their_wave_starts(cuda, oracle, in_dim, out_dim):
     """The Q6_K streaming kernel hands a wave a contiguous range of rows, and how many depends on
