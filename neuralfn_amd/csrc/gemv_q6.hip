@@ -387,15 +387,17 @@ struct PassLoads {
 };
 
 // W: waves per workgroup (the activation images are shared by the workgroup,
-// so more tokens per pass want more waves behind each image).
-template <int T, int P, bool ARGMAX, int W>
+// so more tokens per pass want more waves behind each image).  FEWER: the launch has
+// `fewer_waves` of them, fewer than W.
+template <int T, int P, bool ARGMAX, int W, bool FEWER>
 __global__ __launch_bounds__(W * kWave) void gemv_q6_stream_kernel(
     const float* __restrict__ first, const float* __restrict__ second, std::int64_t input_dim,
-    int tokens, int rows_per_wave, LmHeadCandidate* __restrict__ candidates,
+    int tokens, int rows_per_wave, int fewer_waves, LmHeadCandidate* __restrict__ candidates,
     std::uint8_t* __restrict__ records_out, ProjectionSet set) {
     extern __shared__ __attribute__((aligned(16))) std::uint8_t lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = FEWER ? fewer_waves : W;
     const int blocks = static_cast<int>(input_dim >> 8);  // per row, >= 16
     const int token0 = blockIdx.y * T;
     const int pass_tokens = min(tokens - token0, T);
@@ -406,7 +408,7 @@ __global__ __launch_bounds__(W * kWave) void gemv_q6_stream_kernel(
 
     // rows and blocks of this wave: every projection owns a range of waves
     // (first_tile is its first wave), a wave a contiguous range of its rows
-    const int wave_index = static_cast<int>(blockIdx.x) * W + wave;
+    const int wave_index = static_cast<int>(blockIdx.x) * waves + wave;
     int which = 0;
 #pragma unroll
     for (int index = 1; index < 4; ++index) {
@@ -490,7 +492,7 @@ __global__ __launch_bounds__(W * kWave) void gemv_q6_stream_kernel(
     float4 early[kEarly];
 #pragma unroll
     for (int e = 0; e < kEarly; ++e) {
-        const int record = min(wave + e * W, records - 1);
+        const int record = min(wave + e * waves, records - 1);
         const int token = token_of_record<T>(record, blocks);
         const int block = record - token * blocks;
         early[e] = load_activations<P>(
@@ -516,10 +518,10 @@ __global__ __launch_bounds__(W * kWave) void gemv_q6_stream_kernel(
     };
 #pragma unroll
     for (int e = 0; e < kEarly; ++e) {
-        const int record = wave + e * W;
+        const int record = wave + e * waves;
         if (record < records) quantize_record(early[e], record);
     }
-    for (int record = wave + kEarly * W; record < records; record += W) {
+    for (int record = wave + kEarly * waves; record < records; record += waves) {
         const int token = token_of_record<T>(record, blocks);
         const int block = record - token * blocks;
         const float4 x = load_activations<P>(
@@ -673,7 +675,7 @@ __global__ __launch_bounds__(W * kWave) void gemv_q6_stream_kernel(
             const int t = threadIdx.x;
             float value = values[t];
             std::int64_t index = indices[t];
-            for (int w = 1; w < W; ++w) better(values[w * T + t], indices[w * T + t], value, index);
+            for (int w = 1; w < waves; ++w) better(values[w * T + t], indices[w * T + t], value, index);
             LmHeadCandidate candidate;
             candidate.index = index;
             candidate.value = value;
@@ -750,8 +752,6 @@ std::int64_t launch_stream(const ProjectionSet& set, const float* first, const f
                            hipStream_t stream) {
     const std::size_t lds = static_cast<std::size_t>(T) * token_image_bytes(set.input_dim >> 8) +
         W * kStagingBytes;
-    auto kernel = gemv_q6_stream_kernel<T, P, ARGMAX, W>;
-    allow_large_lds<gemv_q6_stream_kernel<T, P, ARGMAX, W>>();
     const int passes = (tokens + T - 1) / T;
     // one launch: the projections take consecutive ranges of waves
     std::int64_t rows = 0;
@@ -763,11 +763,27 @@ std::int64_t launch_stream(const ProjectionSet& set, const float* first, const f
         placed.op[index].first_tile = static_cast<std::uint32_t>(waves);
         waves += (placed.op[index].output_dim + rows_per_wave - 1) / rows_per_wave;
     }
-    const std::int64_t groups = (waves + W - 1) / W;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups), passes), dim3(W * kWave), lds,
-                       stream, first, second, set.input_dim, tokens, static_cast<int>(rows_per_wave),
-                       candidates, records_out, placed);
-    return groups;
+    const auto launch = [&](auto kernel, int waves_per_group) {
+        const std::int64_t groups = (waves + waves_per_group - 1) / waves_per_group;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups), passes), dim3(waves_per_group * kWave),
+                           lds, stream, first, second, set.input_dim, tokens, static_cast<int>(rows_per_wave),
+                           waves_per_group, candidates, records_out, placed);
+        return groups;
+    };
+    if constexpr (T == 1 && W == 16 && !ARGMAX) {
+        // Sixteen waves a workgroup that would leave a quarter of the compute units without one:
+        // as many waves as give every unit its share (16,384 -> 2,048: 12.8 -> 11.6 us with 8,
+        // -> 5,120: 20.4 -> 19.4 with 10; 13,312 -> 5,888: 21.1 -> 18.5 with 12; with 208 of 256
+        // units at work, 16,384 -> 6,656, thirteen waves on every unit take what sixteen do)
+        constexpr int kFewest = 8;  // (fewer are too few for the quantization)
+        const std::int64_t units = compute_units();
+        if (waves * 4 < units * W * 3 && waves >= units * kFewest) {
+            allow_large_lds<gemv_q6_stream_kernel<T, P, ARGMAX, W, true>>();
+            return launch(gemv_q6_stream_kernel<T, P, ARGMAX, W, true>, static_cast<int>((waves + units - 1) / units));
+        }
+    }
+    allow_large_lds<gemv_q6_stream_kernel<T, P, ARGMAX, W, false>>();
+    return launch(gemv_q6_stream_kernel<T, P, ARGMAX, W, false>, W);
 }
 
 bool streams(std::int64_t input_dim) { return (input_dim >> 8) >= kPassBlocks; }

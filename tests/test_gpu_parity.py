@@ -979,6 +979,32 @@ def test_q6_k_long_rows_one_token_and_verifier(cuda, oracle, shape):
     assert_bits_equal(one, batched[:1], "mmq at one row")
 
 
+@pytest.mark.parametrize("per_unit,in_dim,prologue", [(8.0, 12288, "plain"), (11.99, 12544, "swiglu"),
+                                                      (17.3, 16384, "plain"), (23.9, 12288, "gated")])
+def test_q6_k_long_rows_with_fewer_waves_a_workgroup(cuda, oracle, per_unit, in_dim, prologue):
+    """One token over rows of 48 blocks and more: output widths that would leave compute units
+    without a sixteen-wave workgroup run with 8 to 12 waves (one row a wave, then two, the last
+    workgroups short of rows); two rows of the verifier family take another form and give the
+    same bits."""
+    units = torch_().cuda.get_device_properties(0).multi_processor_count
+    out_dim = int(per_unit * units)
+    packed = random_packed(kquant.Q6_K, 256, in_dim, 57).reshape(256, -1)
+    chosen = np.random.default_rng(58).integers(0, 256, out_dim)
+    weight = tile_ops.PackedWeight(kquant.Q6_K, out_dim, in_dim, torch_().from_numpy(packed).to(cuda).index_select(
+        0, torch_().from_numpy(chosen).to(cuda)).reshape(-1))
+    x = kquant.synthetic_activations(59, 2, in_dim)
+    options = {} if prologue == "plain" else {"second": to_device(x, cuda), "prologue": prologue}
+    workspace = tile_ops.small_batch_workspace(2, in_dim)
+    batch = tile_ops.multi_linear([weight], to_device(x, cuda), workspace, family="mmvq", **options)[0]
+    for row in range(2):
+        here = {k: v[row:row + 1] if k == "second" else v for k, v in options.items()}
+        single = tile_ops.multi_linear([weight], to_device(x[row:row + 1], cuda), workspace, **here)[0]
+        assert_bits_equal(single, batch[row:row + 1].contiguous(), f"row {row}")
+    if prologue == "plain":
+        expected = oracle.linear(kquant.Q6_K, packed.reshape(-1), 256, in_dim, x)[:, chosen]
+        assert normalised_error(batch.cpu().numpy(), expected) <= TOLERANCE
+
+
 def test_q6_k_long_rows_tensor_two_bytes_off_a_word(cuda, oracle):
     """The streaming kernel reads word-aligned pieces when the tensor starts on a four-byte
     boundary; a tensor that does not is read the plain way and gives the same bits."""
