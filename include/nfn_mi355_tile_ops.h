@@ -918,7 +918,9 @@ int nfn_mi355_k_quant_gemm_float32_v1(
 /* How the call above cuts a problem of this geometry on the current device
  * (no counterpart in the reference; for tests and benchmarks that want to know
  * which launch form they exercised): *tile_rows = output rows per workgroup
- * tile (256 or 128; 32 for up to 32 rows), *k_shares = workgroups that share the K range of a tile
+ * tile that the K shares are cut for (256 or 128; 32 for up to 32 rows; the
+ * launch takes tiles of 512, 256 or 128 rows, whichever costs least with these
+ * shares, to the same sums), *k_shares = workgroups that share the K range of a tile
  * (1 = unsplit; with more, each writes a partial output into the workspace and
  * a second launch adds them in share order).  0 on success, 1 for an encoding
  * or width the matrix-core path does not take, or the reserved mode. */

@@ -1,9 +1,9 @@
 // Prefill dequant-GEMM on the fp16 matrix cores:
 //   Y[M, N] = X[M, K] * W[N, K]^T,  W packed (Q4_K / Q5_K / Q6_K / Q8_0).
 //
-// A workgroup of 4 waves owns a 256 x 128 tile of Y; wave w owns rows
+// A workgroup of 8 or 4 waves owns a 512 or 256 x 128 tile of Y; wave w owns rows
 // 64w .. 64w+63 and all 128 columns, and walks K in steps of 64 with 32
-// v_mfma_f32_32x32x16_f16 per step and float accumulators.  (128-row tiles: half
+// v_mfma_f32_32x32x16_f16 per step and float accumulators.  (128-row tiles: four waves, half
 // the rows and instructions a wave; up to 32 rows have a kernel of their own below.)
 //
 // Activations never touch LDS.  A pre-pass converts them to fp16 once per call
@@ -16,7 +16,7 @@
 // magnitude lands in [2^14, 2^15); the epilogue multiplies the row's results
 // by the inverse, so neither large nor tiny activations leave the fp16 range.
 //
-// Weights go through LDS: per step every thread turns 32 weights of the
+// Weights go through LDS: per step every thread turns 32 (eight waves: 16) weights of the
 // 128 x 64 slice (two runs of 16: of one row for Q4_K and Q5_K, 16 packed bytes;
 // of two rows for Q6_K and Q8_0) into fp16 in registers with packed
 // fp16 arithmetic (code bytes become 1024+q by a byte permute, then
@@ -379,6 +379,153 @@ struct PackedSlice<kEncQ8_0> {
     }
 };
 
+// The same with eight waves a workgroup: 16 weights of a K step a thread, four lanes a row.
+//   Q4_K, Q5_K: positions 8*part .. 8*part+7 of both 32-value groups of the step
+//   Q6_K, Q8_0: the step's columns 16*part .. 16*part+15
+// decode<I>() gives four of them, I = 0, 1 the first 16 bytes that the thread writes.
+template <std::uint32_t ENC>
+struct PackedRun;
+template <std::uint32_t ENC>
+struct RunHeader;
+
+template <>
+struct RunHeader<kEncQ4K> : BlockHeader<kEncQ4K> {};
+template <>
+struct RunHeader<kEncQ6K> : BlockHeader<kEncQ6K> {};
+template <>
+struct RunHeader<kEncQ8_0> : BlockHeader<kEncQ8_0> {};
+template <>
+struct RunHeader<kEncQ5K> {
+    u32x4 words;
+    std::uint32_t high[2];
+    __device__ __forceinline__ void load(const std::uint8_t* row, int block, int part) {
+        words = *reinterpret_cast<const u32x4*>(row + block * 176);
+        const uint2 bits = *reinterpret_cast<const uint2*>(row + block * 176 + 16 + part * 8);
+        high[0] = bits.x;
+        high[1] = bits.y;
+    }
+};
+
+template <>
+struct PackedRun<kEncQ4K> {
+    std::uint32_t codes[2];
+    KBlockScales c;
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
+        const uint2 both = *reinterpret_cast<const uint2*>(rows.first + block * 144 + 16 + pair * 32 + part * 8);
+        codes[0] = both.x;
+        codes[1] = both.y;
+    }
+    __device__ __forceinline__ void prepare_bits(const RunHeader<kEncQ4K>& header, int pair, int) {
+        c.bits(header.words, pair);
+    }
+    __device__ __forceinline__ void prepare_scales(const RunHeader<kEncQ4K>& header) { c.scales(header.words); }
+    template <int I>
+    __device__ __forceinline__ void decode(std::uint32_t (&out)[2]) const {
+        if constexpr (I < 2) {
+            scale_bytes(codes[I] & 0x0f0f0f0fu, splat(-1024.0f), c.scale_a, c.shift_a, out[0], out[1]);
+        } else {
+            scale_bytes((codes[I - 2] >> 4) & 0x0f0f0f0fu, splat(-1024.0f), c.scale_b, c.shift_b, out[0], out[1]);
+        }
+    }
+};
+
+template <>
+struct PackedRun<kEncQ5K> {
+    std::uint32_t codes[2], high[2];
+    KBlockScales c;
+    int high_shift;
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
+        const uint2 both = *reinterpret_cast<const uint2*>(rows.first + block * 176 + 48 + pair * 32 + part * 8);
+        codes[0] = both.x;
+        codes[1] = both.y;
+    }
+    __device__ __forceinline__ void prepare_bits(const RunHeader<kEncQ5K>& header, int pair, int) {
+        c.bits(header.words, pair);
+        high[0] = header.high[0];
+        high[1] = header.high[1];
+        high_shift = 2 * pair;
+    }
+    __device__ __forceinline__ void prepare_scales(const RunHeader<kEncQ5K>& header) { c.scales(header.words); }
+    template <int I>
+    __device__ __forceinline__ void decode(std::uint32_t (&out)[2]) const {
+        const std::uint32_t bits = high[I & 1] >> high_shift;
+        if constexpr (I < 2) {
+            const std::uint32_t q = (codes[I] & 0x0f0f0f0fu) | ((bits & 0x01010101u) << 4);
+            scale_bytes(q, splat(-1024.0f), c.scale_a, c.shift_a, out[0], out[1]);
+        } else {
+            const std::uint32_t q = ((codes[I - 2] >> 4) & 0x0f0f0f0fu) | ((bits & 0x02020202u) << 3);
+            scale_bytes(q, splat(-1024.0f), c.scale_b, c.shift_b, out[0], out[1]);
+        }
+    }
+};
+
+template <>
+struct PackedRun<kEncQ6K> {
+    u32x4 low, high;
+    std::uint32_t scales[2], d;
+    f16x2 scale;
+    int upper, high_shift, sub_scale;
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
+        PackedSlice<kEncQ6K>::load_row(rows.first + block * 210, pair >> 1, part, low, high, scales, d);
+    }
+    __device__ __forceinline__ void prepare_bits(const RunHeader<kEncQ6K>&, int pair, int part) {
+        sub_scale = static_cast<std::int8_t>((scales[pair & 1] >> (8 * part)) & 0xffu);
+        upper = (pair & 1) * 4;
+        high_shift = upper + 2 * (part >> 1);
+    }
+    __device__ __forceinline__ void prepare_scales(const RunHeader<kEncQ6K>&) {
+        scale = splat(half_bits_to_float(d) * static_cast<float>(sub_scale));
+    }
+    template <int I>
+    __device__ __forceinline__ void decode(std::uint32_t (&out)[2]) const {
+        const std::uint32_t q = ((low[I] >> upper) & 0x0f0f0f0fu) | (((high[I] >> high_shift) & 0x03030303u) << 4);
+        scale_bytes(q, splat(-1056.0f), scale, splat(0.0f), out[0], out[1]);
+    }
+};
+
+template <>
+struct PackedRun<kEncQ8_0> {
+    u32x4 codes;
+    std::uint32_t d;
+    f16x2 scale;
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
+        PackedSlice<kEncQ8_0>::load_row(rows.first + (block * 8 + pair * 2 + (part >> 1)) * 34, part, codes, d);
+    }
+    __device__ __forceinline__ void prepare_bits(const RunHeader<kEncQ8_0>&, int, int) {}
+    __device__ __forceinline__ void prepare_scales(const RunHeader<kEncQ8_0>&) {
+        const _Float16 h = __builtin_bit_cast(_Float16, static_cast<std::uint16_t>(d));
+        scale = f16x2{h, h};
+    }
+    template <int I>
+    __device__ __forceinline__ void decode(std::uint32_t (&out)[2]) const {
+        scale_bytes(codes[I] ^ 0x80808080u, splat(-1152.0f), scale, splat(0.0f), out[0], out[1]);
+    }
+};
+
+// what a thread holds and decodes with WAVES waves a workgroup
+template <std::uint32_t ENC, int WAVES>
+struct Held {
+    using Slice = PackedSlice<ENC>;
+    using Header = BlockHeader<ENC>;
+};
+template <std::uint32_t ENC>
+struct Held<ENC, 8> {
+    using Slice = PackedRun<ENC>;
+    using Header = RunHeader<ENC>;
+};
+template <int I, std::uint32_t ENC>
+__device__ __forceinline__ void decode(const PackedSlice<ENC>& slice, std::uint32_t (&out)[2]) {
+    if constexpr (I < 4) {
+        slice.template group_a<I>(out);
+    } else {
+        slice.template group_b<I - 4>(out);
+    }
+}
+template <int I, std::uint32_t ENC>
+__device__ __forceinline__ void decode(const PackedRun<ENC>& run, std::uint32_t (&out)[2]) {
+    run.template decode<I>(out);
+}
+
 // lanes that share a weight row
 template <std::uint32_t ENC>
 constexpr int kParts = ENC == kEncQ4K || ENC == kEncQ5K ? 2 : 4;
@@ -388,6 +535,9 @@ constexpr bool kHalfBlocks = ENC == kEncQ6K;
 // from the first run of 16 to the second, in the stage
 template <std::uint32_t ENC>
 constexpr int kSecondRun = kParts<ENC> == 2 ? 64 : 64 * kRowBytes;
+// eight waves: from a thread's first 16 bytes to the others
+template <std::uint32_t ENC>
+constexpr int kRunSecond = ENC == kEncQ4K || ENC == kEncQ5K ? 64 : 16;
 
 // The activation fragments of one K step for one wave: row blocks 0 and 1,
 // K chunks 0..3, in named registers (an array here ends up in scratch memory).
@@ -427,12 +577,12 @@ struct WeightFragments {
 //   b_next:   packed weights of the next step: dequantized into the other
 //             stage with the scales in `header`, then refilled with the packed
 //             bytes of `fetch_step`
-template <std::uint32_t ENC, int RB, bool REFILL>
+template <std::uint32_t ENC, int RB, int WAVES, bool REFILL>
 __device__ __forceinline__ void k_step(
     v16f (&acc)[RB][4], ActivationSlice& a_now, WeightFragments& current,
     const std::uint8_t* b_read, const std::uint8_t* b_read_next, std::uint8_t* b_write,
-    PackedSlice<ENC>& b_next, const BlockHeader<ENC>& header, int decode_pair, int b_part,
-    const std::uint8_t* a_fetch, std::int64_t row_block_bytes, const WeightRows& b_global,
+    typename Held<ENC, WAVES>::Slice& b_next, const typename Held<ENC, WAVES>::Header& header, int decode_pair,
+    int b_part, const std::uint8_t* a_fetch, std::int64_t row_block_bytes, const WeightRows& b_global,
     int fetch_step) {
     WeightFragments ahead;
     std::uint32_t w[2], v[2];
@@ -475,30 +625,35 @@ __device__ __forceinline__ void k_step(
         NFN_FENCE();
         return;
     } else {
-    // K chunk 0: read chunk 1, decode; every decoded group of four values is
-    // written to the other stage at once (8 bytes), which keeps few registers live
+    // K chunk 0: read chunk 1, decode; every decoded run of eight values is written to the other
+    // stage at once (16 bytes), which keeps few registers live
+    constexpr int kSecond = WAVES == 8 ? kRunSecond<ENC> : 16;  // of the second 16 bytes
     NFN_SLOT(a_now.r0k0, current.c0, acc[0][0], b_next.prepare_bits(header, decode_pair, b_part))
     NFN_SLOT(a_now.r0k0, current.c1, acc[0][1], b_next.prepare_scales(header);
              ahead.c0 = NFN_READ_WEIGHTS(b_read, 0, 1))
-    NFN_SLOT(a_now.r0k0, current.c2, acc[0][2], b_next.template group_a<0>(w);
+    NFN_SLOT(a_now.r0k0, current.c2, acc[0][2], decode<0>(b_next, w);
              ahead.c1 = NFN_READ_WEIGHTS(b_read, 1, 1))
-    NFN_SLOT(a_now.r0k0, current.c3, acc[0][3], b_next.template group_a<1>(v);
+    NFN_SLOT(a_now.r0k0, current.c3, acc[0][3], decode<1>(b_next, v);
              NFN_WRITE16(b_write, w[0], w[1], v[0], v[1]))
-    NFN_SLOT(a_now.r1k0, current.c0, acc[1][0], b_next.template group_a<2>(w);
+    NFN_SLOT(a_now.r1k0, current.c0, acc[1][0], decode<2>(b_next, w);
              ahead.c2 = NFN_READ_WEIGHTS(b_read, 2, 1);
              a_now.r0k0 = NFN_LOAD_ACTIVATIONS(a_fetch, 0, 0))
-    NFN_SLOT(a_now.r1k0, current.c1, acc[1][1], b_next.template group_a<3>(v);
-             NFN_WRITE16(b_write + 16, w[0], w[1], v[0], v[1]))
-    NFN_SLOT(a_now.r1k0, current.c2, acc[1][2], b_next.template group_b<0>(w);
+    NFN_SLOT(a_now.r1k0, current.c1, acc[1][1], decode<3>(b_next, v);
+             NFN_WRITE16(b_write + kSecond, w[0], w[1], v[0], v[1]))
+    NFN_SLOT(a_now.r1k0, current.c2, acc[1][2], if constexpr (WAVES == 4) decode<4>(b_next, w);
              ahead.c3 = NFN_READ_WEIGHTS(b_read, 3, 1))
-    NFN_SLOT(a_now.r1k0, current.c3, acc[1][3], b_next.template group_b<1>(v);
-             NFN_WRITE16(b_write + kSecondRun<ENC>, w[0], w[1], v[0], v[1]))
+    NFN_SLOT(a_now.r1k0, current.c3, acc[1][3], if constexpr (WAVES == 4) {
+                 decode<5>(b_next, v);
+                 NFN_WRITE16(b_write + kSecondRun<ENC>, w[0], w[1], v[0], v[1]);
+             })
     // K chunk 1: read chunk 2, finish decoding
-    NFN_SLOT(a_now.r0k1, ahead.c0, acc[0][0], b_next.template group_b<2>(w);
+    NFN_SLOT(a_now.r0k1, ahead.c0, acc[0][0], if constexpr (WAVES == 4) decode<6>(b_next, w);
              current.c0 = NFN_READ_WEIGHTS(b_read, 0, 2);
              a_now.r1k0 = NFN_LOAD_ACTIVATIONS(a_fetch, 1, 0))
-    NFN_SLOT(a_now.r0k1, ahead.c1, acc[0][1], b_next.template group_b<3>(v);
-             NFN_WRITE16(b_write + kSecondRun<ENC> + 16, w[0], w[1], v[0], v[1]))
+    NFN_SLOT(a_now.r0k1, ahead.c1, acc[0][1], if constexpr (WAVES == 4) {
+                 decode<7>(b_next, v);
+                 NFN_WRITE16(b_write + kSecondRun<ENC> + 16, w[0], w[1], v[0], v[1]);
+             })
     NFN_SLOT(a_now.r0k1, ahead.c2, acc[0][2], current.c1 = NFN_READ_WEIGHTS(b_read, 1, 2))
     NFN_SLOT(a_now.r0k1, ahead.c3, acc[0][3], (void)0)
     NFN_SLOT(a_now.r1k1, ahead.c0, acc[1][0], current.c2 = NFN_READ_WEIGHTS(b_read, 2, 2);
@@ -550,13 +705,13 @@ constexpr int kBlockBytes = ENC == kEncQ4K ? 144 : ENC == kEncQ5K ? 176 : ENC ==
 // allow; while one wave waits at the barrier or for LDS, another keeps the
 // matrix pipe busy.  With 256-row tiles the Q6_K decode holds too much live
 // state for two (of 22 registers in scratch memory with two).
-template <std::uint32_t ENC, int RB>
-constexpr int kWavesPerSimd = ENC == kEncQ6K ? RB == 1 ? 2 : 1 : RB == 1 && ENC == kEncQ4K ? 3 : 2;
+template <std::uint32_t ENC, int RB, int WAVES>
+constexpr int kWavesPerSimd = WAVES == 8 ? 2 : ENC == kEncQ6K ? RB == 1 ? 2 : 1 : RB == 1 && ENC == kEncQ4K ? 3 : 2;
 
 // The packed bytes of a block of a lane's rows.
-template <std::uint32_t ENC>
+template <std::uint32_t ENC, int WAVES>
 struct Slices {
-    PackedSlice<ENC> b0, b1, b2, b3;  // of its four steps; Q6_K: b0 the first half, b1 the second
+    typename Held<ENC, WAVES>::Slice b0, b1, b2, b3;  // of its four steps; Q6_K: b0 the first half, b1 the second
     __device__ __forceinline__ void load(const WeightRows& rows, int block, int part) {
         b0.load(rows, block, 0, part);
         b1.load(rows, block, kHalfBlocks<ENC> ? 2 : 1, part);
@@ -571,7 +726,7 @@ struct Slices {
 // cache from one step to the next (4,096 rows of gate and up, Q4_K: 1,577 -> 1,533 us; 100 rows of
 // Q5_K 92 -> 88).  Q6_K, whose slices serve two steps, gains nothing by it, and Q8_0, whose block of a
 // row is more than two lines, loses: 100 rows of O 55 -> 69 us.
-template <std::uint32_t ENC, int RB>
+template <std::uint32_t ENC, int RB, int WAVES>
 constexpr bool kWholeBlocks = (ENC == kEncQ4K && RB == 2) || (ENC == kEncQ5K && RB == 1);
 
 // The projections of one launch: one encoding, one input.  Workgroup numbers run through the
@@ -619,10 +774,10 @@ struct GroupPlace {
         place.tile = (static_cast<int>(blockIdx.x) - first) % tiles;         \
     }
 
-// RB: 32-row blocks per wave; the workgroup's tile is 128*RB rows by 128 columns.
-template <std::uint32_t ENC, int RB>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB>))) void gemm_f16_kernel(
+// RB: 32-row blocks per wave; the workgroup's tile is 32 * RB * WAVES rows by 128 columns.
+template <std::uint32_t ENC, int RB, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave)
+__attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB, WAVES>, kWavesPerSimd<ENC, RB, WAVES>))) void gemm_f16_kernel(
     const std::uint8_t* __restrict__ activations, const float* __restrict__ inverse_scale, std::int64_t input_dim,
     std::int64_t rows, int m_tiles, GemmGroup group) {
     extern __shared__ __attribute__((aligned(16))) std::uint8_t lds[];
@@ -636,7 +791,9 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     const int share = place.share, shares = place.shares;
     const int m_tile = place.tile % m_tiles;
     const int n_tile = place.tile / m_tiles;
-    constexpr int kTileRows = 128 * RB;
+    using Slice = typename Held<ENC, WAVES>::Slice;
+    using Header = typename Held<ENC, WAVES>::Header;
+    constexpr int kTileRows = 32 * RB * WAVES;
     const std::int64_t m0 = static_cast<std::int64_t>(m_tile) * kTileRows;
     const std::int64_t n0 = static_cast<std::int64_t>(n_tile) * kBN;
     // which share of the K dimension (whole 256-value blocks) this workgroup sums; each share
@@ -651,20 +808,25 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
 
     // activations: fragment (row block, K chunk) is 1 KB, a row block's chunks are consecutive
     const std::int64_t row_block_bytes = (input_dim / 16) * kFragmentBytes;
-    const std::uint8_t* a_global = activations + (m0 / 32 + wave * RB) * row_block_bytes +
+    // (a tile of 512 rows can reach past the rows the copy is padded to: its last waves take blocks
+    // that are there and store nothing)
+    int row_block = static_cast<int>(m0 / 32) + wave * RB;
+    if constexpr (WAVES == 8) row_block = min(row_block, static_cast<int>((rows + kBM - 1) / kBM * (kBM / 32)) - RB);
+    const std::uint8_t* a_global = activations + row_block * row_block_bytes +
         static_cast<std::int64_t>(first_block) * 16 * kFragmentBytes + lane * 16;
     constexpr int kStepBytes = (kBK / 16) * kFragmentBytes;
     // weights: thread -> (row, which run of 16).  Eight consecutive lanes write their 16-byte
     // pieces into distinct banks: with stage rows of 36 words and runs of 8, rows k and k + 1
     // times four runs do, and so do rows k, k + 1, k + 4, k + 5 times two.
-    const int b_part = tid & (kParts<ENC> - 1);
-    const int b_turn = tid / kParts<ENC>;
-    const int b_row = kParts<ENC> == 4 ? b_turn : (b_turn & ~6) | ((b_turn & 2) << 1) | ((b_turn & 4) >> 1);
+    constexpr int kLanes = WAVES == 8 ? 4 : kParts<ENC>;
+    const int b_part = tid & (kLanes - 1);
+    const int b_turn = tid / kLanes;
+    const int b_row = kLanes == 4 ? b_turn : (b_turn & ~6) | ((b_turn & 2) << 1) | ((b_turn & 4) >> 1);
     const std::int64_t b_skip = static_cast<std::int64_t>(first_block) * kBlockBytes<ENC>;
     WeightRows b_global;
     b_global.first = weights + min(n0 + b_row, output_dim - 1) * row_stride + b_skip;
-    b_global.second = weights + min(n0 + b_row + 64, output_dim - 1) * row_stride + b_skip;
-    const int b_target = b_row * kRowBytes + b_part * 32;
+    b_global.second = weights + min(n0 + b_row + 64, output_dim - 1) * row_stride + b_skip;  // (four waves)
+    const int b_target = b_row * kRowBytes + b_part * (WAVES == 8 && kRunSecond<ENC> == 64 ? 16 : 32);
 
     v16f acc[RB][4];
 #pragma unroll
@@ -686,9 +848,9 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     // The header of a 256-value block is loaded once, three or more steps
     // before the first of its four steps is decoded.
     ActivationSlice a_now;
-    constexpr bool kWhole = kWholeBlocks<ENC, RB>;
-    Slices<ENC> set0, set1;  // (set1: whole blocks only; the sets swap roles like the headers)
-    BlockHeader<ENC> header_even, header_odd;  // blocks 0, 2, 4 ... and 1, 3, 5 ...
+    constexpr bool kWhole = kWholeBlocks<ENC, RB, WAVES>;
+    Slices<ENC, WAVES> set0, set1;  // (set1: whole blocks only; the sets swap roles like the headers)
+    Header header_even, header_odd;  // blocks 0, 2, 4 ... and 1, 3, 5 ...
     const int last_block = (steps >> 2) - 1;
     header_even.load(b_global.first, 0, b_part);
     header_odd.load(b_global.first, min(1, last_block), b_part);
@@ -707,19 +869,23 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
         std::uint32_t wa[4][2], wb[4][2];
         set0.b0.prepare_bits(header_even, 0, b_part);
         set0.b0.prepare_scales(header_even);
-        set0.b0.template group_a<0>(wa[0]);
-        set0.b0.template group_a<1>(wa[1]);
-        set0.b0.template group_a<2>(wa[2]);
-        set0.b0.template group_a<3>(wa[3]);
-        set0.b0.template group_b<0>(wb[0]);
-        set0.b0.template group_b<1>(wb[1]);
-        set0.b0.template group_b<2>(wb[2]);
-        set0.b0.template group_b<3>(wb[3]);
+        decode<0>(set0.b0, wa[0]);
+        decode<1>(set0.b0, wa[1]);
+        decode<2>(set0.b0, wa[2]);
+        decode<3>(set0.b0, wa[3]);
+        if constexpr (WAVES == 4) {
+            decode<4>(set0.b0, wb[0]);
+            decode<5>(set0.b0, wb[1]);
+            decode<6>(set0.b0, wb[2]);
+            decode<7>(set0.b0, wb[3]);
+        }
         std::uint8_t* target = lds + b_target;
         NFN_WRITE16(target, wa[0][0], wa[0][1], wa[1][0], wa[1][1]);
-        NFN_WRITE16(target + 16, wa[2][0], wa[2][1], wa[3][0], wa[3][1]);
-        NFN_WRITE16(target + kSecondRun<ENC>, wb[0][0], wb[0][1], wb[1][0], wb[1][1]);
-        NFN_WRITE16(target + kSecondRun<ENC> + 16, wb[2][0], wb[2][1], wb[3][0], wb[3][1]);
+        NFN_WRITE16(target + (WAVES == 8 ? kRunSecond<ENC> : 16), wa[2][0], wa[2][1], wa[3][0], wa[3][1]);
+        if constexpr (WAVES == 4) {
+            NFN_WRITE16(target + kSecondRun<ENC>, wb[0][0], wb[0][1], wb[1][0], wb[1][1]);
+            NFN_WRITE16(target + kSecondRun<ENC> + 16, wb[2][0], wb[2][1], wb[3][0], wb[3][1]);
+        }
     }
     if constexpr (!kHalfBlocks<ENC> && !kWhole) set0.b0.load(b_global, min(1, last_block), 0, b_part);  // step 4, or step 0 again
     __syncthreads();
@@ -750,23 +916,24 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
     // (Whole blocks: the next block goes to the other set at the start instead.
     // Q6_K: b0 holds a block's first half, which the first and, of the next block, the fourth step
     // decode, b1 the second.)
-    auto block_of_four = [&](int step, const BlockHeader<ENC>& now, const BlockHeader<ENC>& next, Slices<ENC>& mine, Slices<ENC>& other) {
+    auto block_of_four = [&](int step, const Header& now, const Header& next, Slices<ENC, WAVES>& mine,
+                             Slices<ENC, WAVES>& other) {
         constexpr bool kHalves = kHalfBlocks<ENC>;
         constexpr int kAhead = kHalves ? 3 : 4;  // from the step that is decoded to the one that is fetched
-        Slices<ENC>& after = kWhole ? other : mine;
+        Slices<ENC, WAVES>& after = kWhole ? other : mine;
         if constexpr (kWhole) {
             const int block = min((step >> 2) + 1, last_block);
             other.load(b_global, block, b_part);
             NFN_FENCE();
         }
-        PackedSlice<ENC>&second = kHalves ? mine.b0 : mine.b1, &third = kHalves ? mine.b1 : mine.b2, &fourth = kHalves ? mine.b1 : mine.b3;
-        k_step<ENC, RB, !kWhole>(acc, a_now, current, b_read0, b_read1, b_write1, second, now, 1, b_part,
+        Slice &second = kHalves ? mine.b0 : mine.b1, &third = kHalves ? mine.b1 : mine.b2, &fourth = kHalves ? mine.b1 : mine.b3;
+        k_step<ENC, RB, WAVES, !kWhole>(acc, a_now, current, b_read0, b_read1, b_write1, second, now, 1, b_part,
                     activations_of(step + 1), row_block_bytes, b_global, min(step + 1 + kAhead, last));
-        k_step<ENC, RB, !kHalves && !kWhole>(acc, a_now, current, b_read1, b_read0, b_write0, third, now, 2, b_part,
+        k_step<ENC, RB, WAVES, !kHalves && !kWhole>(acc, a_now, current, b_read1, b_read0, b_write0, third, now, 2, b_part,
                     activations_of(step + 2), row_block_bytes, b_global, min(step + 2 + kAhead, last));
-        k_step<ENC, RB, !kWhole>(acc, a_now, current, b_read0, b_read1, b_write1, fourth, now, 3, b_part,
+        k_step<ENC, RB, WAVES, !kWhole>(acc, a_now, current, b_read0, b_read1, b_write1, fourth, now, 3, b_part,
                     activations_of(step + 3), row_block_bytes, b_global, min(step + 3 + kAhead, last));
-        k_step<ENC, RB, !kHalves && !kWhole>(acc, a_now, current, b_read1, b_read0, b_write0, after.b0, next, 0, b_part,
+        k_step<ENC, RB, WAVES, !kHalves && !kWhole>(acc, a_now, current, b_read1, b_read0, b_write0, after.b0, next, 0, b_part,
                     activations_of(step + 4), row_block_bytes, b_global, min(step + 4 + kAhead, last));
     };
     // The two header register sets swap roles every block; the loop body is two
@@ -780,7 +947,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
         if constexpr (kWhole) set0 = set1;
         header_even.load(b_global.first, min(2, last_block), b_part);
         NFN_FENCE();
-        const BlockHeader<ENC> second = header_odd;
+        const Header second = header_odd;
         header_odd = header_even;
         header_even = second;
         block = 1;
@@ -804,7 +971,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB>, kWavesPerSimd<ENC, RB
         const std::int64_t tile_row = m0 + wave * (32 * RB) + i * 32 + row_base;
         float inverse[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) inverse[r] = inverse_scale[tile_row + 8 * (r >> 2) + (r & 3)];
+        for (int r = 0; r < 16; ++r) inverse[r] = inverse_scale[(WAVES == 8 ? row_block * 32 + i * 32 + row_base : tile_row) + 8 * (r >> 2) + (r & 3)];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const std::int64_t n = n0 + j * 32 + column;
@@ -891,7 +1058,7 @@ __device__ __forceinline__ void low_step(v16f& acc, LowActivations& a, const std
 template <std::uint32_t ENC>
 struct LowBlock {
     BlockHeader<ENC> header;
-    Slices<ENC> slices;
+    Slices<ENC, 4> slices;
     __device__ __forceinline__ void load(const WeightRows& rows, int block, int part) {
         header.load(rows.first, block, part);
         slices.load(rows, block, part);
@@ -1060,6 +1227,8 @@ __global__ __launch_bounds__(256) void sum_shares_kernel(ShareSums sums) {
 // or more, at most eight, until there are two workgroups a unit.  (Two 32-row blocks a wave, for up
 // to 64 rows: 128-row tiles are as fast or faster where the tiles are many, 64 rows of gate and up
 // 81 us (Q4_K) and 203 (Q8_0) against 78 and 93 at 65.)
+// (The heights here are those that the shares are cut for.  The launch takes the one that costs
+// least with these shares, see tile_height; a sum does not depend on it.)
 struct Plan {
     int tile_rows;  // 256 and 128 (two 32-row blocks a wave or one), 32 (all rows in every wave)
     int shares;
@@ -1107,10 +1276,10 @@ Plan plan(std::uint32_t encoding, std::int64_t rows, std::int64_t output_dim,
     return Plan{128, static_cast<int>(shares)};
 }
 
-template <std::uint32_t ENC, int RB>
+template <std::uint32_t ENC, int RB, int WAVES>
 void launch_tiles(GemmGroup group, int count, const std::uint8_t* activations, const float* inverse_scale,
                   std::int64_t rows, std::int64_t input_dim, hipStream_t stream) {
-    const int m_tiles = static_cast<int>((rows + 128 * RB - 1) / (128 * RB));
+    const int m_tiles = static_cast<int>((rows + 32 * RB * WAVES - 1) / (32 * RB * WAVES));
     int workgroups = 0;
     for (int i = 0; i < kMaxProjections; ++i) {
         group.first[i] = i < count ? workgroups : 0x7fffffff;
@@ -1119,7 +1288,7 @@ void launch_tiles(GemmGroup group, int count, const std::uint8_t* activations, c
         workgroups += group.tiles[i] * group.shares[i];
     }
     if (rows > kLowRows) {
-        hipLaunchKernelGGL((gemm_f16_kernel<ENC, RB>), dim3(static_cast<unsigned>(workgroups)), dim3(kThreads),
+        hipLaunchKernelGGL((gemm_f16_kernel<ENC, RB, WAVES>), dim3(static_cast<unsigned>(workgroups)), dim3(WAVES * kWave),
                            2 * kStageBytes, stream, activations, inverse_scale, input_dim, rows, m_tiles, group);
     } else {
         hipLaunchKernelGGL(gemm_f16_low_kernel<ENC>, dim3(static_cast<unsigned>(workgroups)), dim3(kThreads),
@@ -1127,14 +1296,75 @@ void launch_tiles(GemmGroup group, int count, const std::uint8_t* activations, c
     }
 }
 
+// What a workgroup takes for 256 columns of K, in us, where one, two or three of the tile's height
+// share a compute unit and all units are at work (0: so many do not fit).
+struct TileCost {
+    int rows;
+    double block[3];
+};
+template <std::uint32_t ENC>
+constexpr TileCost kTileCosts[3] = {{512, {6.9, 0, 0}}, {256, {4.1, 7.4, 0}}, {128, {2.7, 4.5, 6.6}}};
+template <>
+constexpr TileCost kTileCosts<kEncQ5K>[3] = {{512, {6.6, 0, 0}}, {256, {4.0, 7.2, 0}}, {128, {2.9, 4.5, 0}}};
+template <>
+constexpr TileCost kTileCosts<kEncQ6K>[3] = {{512, {7.0, 0, 0}}, {256, {4.6, 0, 0}}, {128, {3.2, 5.3, 0}}};
+template <>
+constexpr TileCost kTileCosts<kEncQ8_0>[3] = {{512, {6.8, 0, 0}}, {256, {4.1, 8.0, 0}}, {128, {3.1, 5.75, 0}}};
+
+// The tile height of a launch of more than 32 rows.  The workgroups go to the units in rounds of as
+// many as fit; the last one may leave places or whole units empty, and a chip at work in part runs
+// at a higher clock, down to three quarters of the time.  The figures are fitted to 160 to 3,000
+// rows into Q, K, V and gate, O, gate and up, and down at one to four shares: the times are met to
+// 5 %, and the height chosen costs 0.2 % more than the best one on average.
+// Eight waves on 512 rows decode a weight for twice the rows, and Q6_K's registers then allow two
+// waves a SIMD instead of one: 2,048 rows of 16,384 -> 6,656 461 -> 420 us (Q4_K), 475 -> 430 (Q5_K),
+// 542 -> 434 (Q6_K), 540 -> 439 (Q8_0); 4,000 rows of gate and up 1,525 -> 1,479, 1,593 -> 1,500,
+// 1,909 -> 1,519, 1,747 -> 1,540.  Lower tiles where 512 rows leave too many units idle: 160 rows of gate
+// and up 108 us in tiles of 256 rows (128: 124, 512: 163), of O 47 in tiles of 128 (58, 85).
+template <std::uint32_t ENC>
+int tile_height(const GemmGroup& group, int count, std::int64_t rows, std::int64_t input_dim) {
+    const std::int64_t units = compute_units();
+    int best_rows = 0;
+    double best = 0;
+    for (const TileCost& tile : kTileCosts<ENC>) {
+        const std::int64_t m_tiles = (rows + tile.rows - 1) / tile.rows;
+        std::int64_t workgroups = 0, tiles = 0;
+        for (int i = 0; i < count; ++i) {
+            const std::int64_t here = m_tiles * ((group.output_dim[i] + kBN - 1) / kBN);
+            tiles += here;
+            workgroups += here * group.shares[i];
+        }
+        const int places = tile.block[2] > 0 ? 3 : tile.block[1] > 0 ? 2 : 1;
+        const std::int64_t full = workgroups / (units * places);
+        const int last = static_cast<int>((workgroups - full * units * places + units - 1) / units);
+        double rounds = static_cast<double>(full) * tile.block[places - 1];
+        if (last > 0) {
+            const double at_work = static_cast<double>(workgroups - full * units * places) / static_cast<double>(units * last);
+            const double clock = 1.0 + 0.35 * (at_work - 1.0);
+            rounds += tile.block[last - 1] * (clock > 0.75 ? clock : 0.75);
+        }
+        // (blocks of 256 columns that a workgroup walks, on average, and a fifth for its start and end)
+        const double blocks = static_cast<double>(input_dim >> 8) * static_cast<double>(tiles) / static_cast<double>(workgroups);
+        const double cost = (blocks + 0.2) * rounds;
+        if (best_rows == 0 || cost < best) {
+            best_rows = tile.rows;
+            best = cost;
+        }
+    }
+    return best_rows;
+}
+
 // One launch for `count` projections of one encoding and, if any of them splits K, one for the sums.
 template <std::uint32_t ENC>
-void launch_group(const GemmGroup& group, int count, bool tall, const std::uint8_t* activations,
+void launch_group(const GemmGroup& group, int count, const std::uint8_t* activations,
                   const float* inverse_scale, std::int64_t rows, std::int64_t input_dim, hipStream_t stream) {
-    if (tall) {
-        launch_tiles<ENC, 2>(group, count, activations, inverse_scale, rows, input_dim, stream);
+    const int height = rows <= kLowRows ? 128 : tile_height<ENC>(group, count, rows, input_dim);
+    if (height == 512) {
+        launch_tiles<ENC, 2, 8>(group, count, activations, inverse_scale, rows, input_dim, stream);
+    } else if (height == 256) {
+        launch_tiles<ENC, 2, 4>(group, count, activations, inverse_scale, rows, input_dim, stream);
     } else {
-        launch_tiles<ENC, 1>(group, count, activations, inverse_scale, rows, input_dim, stream);
+        launch_tiles<ENC, 1, 4>(group, count, activations, inverse_scale, rows, input_dim, stream);
     }
     ShareSums sums{};
     int split = 0;
@@ -1270,8 +1500,7 @@ void launch_gemm_f16(const Descriptor* descriptors, int count, const float* inpu
         // this projection and those of its encoding whose partial outputs find room beside its own
         GemmGroup group{};
         int members = 0;
-        std::int64_t used = 0, short_groups = 0;
-        bool tall = false;
+        std::int64_t used = 0;
         for (int i = start; i < count; ++i) {
             if (done[i] || descriptors[i].encoding != descriptors[start].encoding) continue;
             const Plan chosen = plan(descriptors[i].encoding, rows, descriptors[i].output_dim, input_dim);
@@ -1285,20 +1514,13 @@ void launch_gemm_f16(const Descriptor* descriptors, int count, const float* inpu
             group.output_dim[members] = descriptors[i].output_dim;
             group.shares[members] = chosen.shares;
             used += floats;
-            short_groups += (rows + 127) / 128 * ((descriptors[i].output_dim + kBN - 1) / kBN) * chosen.shares;
-            if (chosen.tile_rows == 256) tall = true;
             ++members;
         }
-        // 256-row tiles where a member would take them by itself, unless 128-row tiles leave half
-        // of the last one's rows out and all fit the units at two a unit (333 rows into Q, K, V and
-        // the gate of width 6,656: 84 us instead of 102 for Q5_K, 78 instead of 98 for Q4_K)
-        const bool odd = (rows + 127) / 128 % 2 != 0;
-        if (members > 1 && odd && short_groups <= 2 * compute_units()) tall = false;
         switch (descriptors[start].encoding) {
-            case kEncQ4K: launch_group<kEncQ4K>(group, members, tall, activations, inverse_scale, rows, input_dim, stream); break;
-            case kEncQ5K: launch_group<kEncQ5K>(group, members, tall, activations, inverse_scale, rows, input_dim, stream); break;
-            case kEncQ6K: launch_group<kEncQ6K>(group, members, tall, activations, inverse_scale, rows, input_dim, stream); break;
-            default: launch_group<kEncQ8_0>(group, members, tall, activations, inverse_scale, rows, input_dim, stream); break;
+            case kEncQ4K: launch_group<kEncQ4K>(group, members, activations, inverse_scale, rows, input_dim, stream); break;
+            case kEncQ5K: launch_group<kEncQ5K>(group, members, activations, inverse_scale, rows, input_dim, stream); break;
+            case kEncQ6K: launch_group<kEncQ6K>(group, members, activations, inverse_scale, rows, input_dim, stream); break;
+            default: launch_group<kEncQ8_0>(group, members, activations, inverse_scale, rows, input_dim, stream); break;
         }
     }
 }

@@ -1713,6 +1713,27 @@ def test_prefill_gemm_tall_tiles(cuda, oracle, encoding):
     assert normalised_error(y[picked], expected) <= TOLERANCE
 
 
+@pytest.mark.parametrize("rows,tiles,in_dim", [(600, 0.5, 256), (1000, 0.5, 512), (1200, 0.33, 768), (1537, 1.0, 1280)])
+@pytest.mark.parametrize("encoding", ALL_PACKED)
+def test_prefill_gemm_eight_waves_a_tile(cuda, oracle, encoding, rows, tiles, in_dim):
+    """Tiles of 512 rows, taken where they fill the chip: a last tile of 88, 488, 176 and one row (waves
+    past the rows that the fp16 copy is padded to), a last column tile of 125, one to five blocks of
+    K.  The oracle checks rows at the edges of waves and tiles."""
+    units = torch_().cuda.get_device_properties(0).multi_processor_count
+    out_dim = int(tiles * units) * 128 - 3
+    packed = random_packed(encoding, 256, in_dim, 46).reshape(256, -1)
+    chosen = np.random.default_rng(47).integers(0, 256, out_dim)
+    weight = tile_ops.PackedWeight(encoding, out_dim, in_dim, torch_().from_numpy(packed).to(cuda).index_select(
+        0, torch_().from_numpy(chosen).to(cuda)).reshape(-1))
+    x = kquant.synthetic_activations(76, rows, in_dim)
+    y = tile_ops.gemm(weight, to_device(x, cuda)).cpu().numpy()
+    picked = np.array(sorted({r for edge in range(0, rows + 1, 64) for r in (edge - 1, edge, edge + 31, edge + 32)
+                              if 0 <= r < rows} | {rows - 1}))
+    expected = oracle.linear(encoding, packed.reshape(-1), 256, in_dim, np.ascontiguousarray(x[picked]))[:, chosen]
+    for row, want in zip(picked, expected):
+        assert normalised_error(y[row], want) <= TOLERANCE, row
+
+
 def test_prefill_gemm_plans():
     # Host logic only.  A problem of many tiles but not one per compute unit: shares of at
     # least twelve 256-value blocks, 256-row tiles while two shares or more fit.
