@@ -23,16 +23,25 @@
 //   linear_exact_kernel, a tile of 32 MT input rows x 128 weight rows for two waves (64 weight rows
 //   each) in each of four K groups.  The two cut the activations of a step of 32 columns between
 //   them and hand the terms over in LDS.
-// What bounds both is the vector cache: a load instruction that reads 16 bytes from each of 32 rows
-// looks up 32 lines for 1 KB, and a unit pulls some 20 GB/s that way.  200 rows of Q8_0: a look-up in
-// 72 % of the cycles, the matrix cores busy in 26 %, the vector ALU in 37, LDS in 15.  (Requests two
-// steps ahead instead of one, and the matrix instructions of a step before its other work instead of
-// between it, made no difference.)  The 64 x 128 form of Q5_K keeps four registers that do not change in
-// its loop in scratch (20 bytes a lane), the 64 x 64 form of F32 seven (32 bytes), read outside of its
-// loop only; the others none.
+// What bounds the small form is the vector cache: a load instruction that reads 16 bytes from each of 32
+// rows looks up 32 lines for 1 KB, and a unit pulls some 20 GB/s that way.  The large form did the same
+// (a look-up in 72 % of the cycles, the matrix cores busy in 26 %); it loads its weights with
+// neighbouring lanes on neighbouring pieces of a row and turns them in LDS, each wave its own, and the two
+// waves of a group wait for each other alone instead of for the workgroup.  4,096 -> 6,656 at 100 / 200 /
+// 512 rows, loads as the lanes use them -> through LDS -> and with waits in pairs: Q8_0 73 / 84 / 165 -> 41 /
+// 60 / 118 -> 38 / 55 / 108 us; Q5_K 61 / 83 / 165 -> 54 / 76 / 151 -> 43 / 65 / 127 (with sums of
+// activations by DPP instead of LDS permutes); Q4_K 49 / 70 / 138 -> 46 / 72 / 142 -> 40 / 62 / 121; Q6_K 87 /
+// 105 / 208 -> 77 / 97 / 192 -> 58 / 76 / 151 (scales requested a step later, out of the registers' way);
+// bf16 58 / 67 / 131 -> 45 / 55 / 108 -> 39 / 50 / 98 (both halves of a line at once).  What is left of the
+// 55 us (200 rows of Q8_0) in parts, each by leaving it out: cutting 8, weights' loads 8, decode 5, scaling 3,
+// matrix instructions 21: two waves a SIMD overlap them in part.  (Sums of all tiles meeting in LDS at
+// once instead of tile by tile: no difference.  Requests two steps ahead instead of one, and the matrix
+// instructions of a step before its other work instead of between it: neither.)  The 64 x 128 form of Q6_K
+// keeps six registers that do not change in its loop in scratch (28 bytes a lane), the 64 x 64 form of F32
+// seven (32 bytes), read outside of its loop only; the others none.
 // Measured at 4,096 -> 6,656, against the vector kernel (16 rows) and the float matrix instruction (200,
-// 512 rows) before: Q4_K 134 -> 16 us at 16 rows, 203 -> 68 at 200, 311 -> 135 at 512; Q8_0 368 -> 27,
-// 180 -> 80, 279 -> 162; F32 406 -> 30, 172 -> 136, 271 -> 254.
+// 512 rows) before: Q4_K 134 -> 16 us at 16 rows, 203 -> 62 at 200, 311 -> 121 at 512; Q8_0 368 -> 27,
+// 180 -> 55, 279 -> 108; F32 406 -> 30, 172 -> 136, 271 -> 254.
 //
 // The entry point, nfn_native_tile_linear_packed_weight_float32_v1, has no workspace argument
 // (neuralfn/csrc/native_train/tile_ops.h:614-620; reference kernel
@@ -143,6 +152,11 @@ struct Traded {
 __device__ __forceinline__ Traded trade(std::uint32_t a, std::uint32_t b) {
     const auto both = __builtin_amdgcn_permlane32_swap(a, b, false, false);
     return Traded{both[0], both[1]};
+}
+// another lane's value, by a pattern within sixteen lanes
+template <int PATTERN>
+__device__ __forceinline__ float of_lane(float value) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(value), PATTERN, 0xf, 0xf, true));
 }
 template <std::uint32_t ENC>
 struct Unit;
@@ -713,9 +727,136 @@ template <int MT>
 constexpr int kSumBytes = 4 * 32 * MT * 4;       // sums of the activations, [step % 4][row]
 template <int MT>
 constexpr int kGroupBytes = 2 * kStepBytes<MT> + kSumBytes<MT>;
-template <int MT>
-constexpr int kLargeLds = kGroups * kGroupBytes<MT>;
-static_assert(kLargeLds<1> >= kLargeWaves * 16 * kWave * 4, "the waves' sums meet in the same memory");
+
+// A wave's 64 weight rows on their way: pieces of 16 bytes, neighbouring lanes on neighbouring pieces of
+// a row, wait in registers and lie in LDS for one unit (bf16: one step).  A row's pieces are one or two runs:
+// the first kFirst of them, then kSecond, each run of all rows an area of its own, row by row.
+template <std::uint32_t ENC>
+struct Staged {
+    static constexpr int kFirst = ENC == kEncQ4K ? 1 : ENC == kEncQ5K ? 3 : ENC == kEncQ8_0 ? 5 : 4;
+    static constexpr int kSecond = ENC == kEncQ8_0 || ENC == kEncBF16 ? 0 : 2;
+    static constexpr int kPieces = kFirst + kSecond;
+    static constexpr int kBytes = 64 * 16 * kPieces;
+    // bf16: a unit is a line a row, requested as a whole (lines come to the vector cache as such, and
+    // do not stay there for a second request), and lies in LDS a step at a time
+    static constexpr int kParts = ENC == kEncBF16 ? 2 : 1;
+    u32x4_a2 held[kParts][kPieces];
+    std::uint32_t scales[2];   // Q6_K: of the rows `inner` and 32 + inner, as Unit loads them
+    std::uint32_t from[kPieces], scales_from[2];
+    std::uint8_t* first;       // where the lane's pieces go
+    std::uint8_t* second;
+    const std::uint8_t* tile;  // the wave's first row
+
+    __device__ __forceinline__ Staged(const std::uint8_t* data, std::int64_t row_stride, std::int64_t col0,
+                                      std::int64_t output_dim, std::uint8_t* lds, int lane) {
+        const std::int64_t row0 = min(col0, output_dim - 1);
+        const int last = static_cast<int>(min(output_dim - 1 - row0, std::int64_t(63)));  // (rows past the end: the last one again)
+        const auto bytes = [&](int row) { return static_cast<std::uint32_t>(min(row, last)) * static_cast<std::uint32_t>(row_stride); };
+        tile = data + row0 * row_stride;
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            const int lanes = i < kFirst ? kFirst : kSecond, index = (i < kFirst ? i : i - kFirst) * kWave + lane;
+            const int row = index / lanes, piece = index % lanes;
+            // (Q8_0, two blocks of 34 bytes: the codes of the second one as two pieces of their own)
+            from[i] = bytes(row) + 16 * piece - (ENC == kEncQ8_0 && piece >= 2 ? 12 : 0);
+        }
+        if constexpr (ENC == kEncQ6K) {
+#pragma unroll
+            for (int n = 0; n < 2; ++n) scales_from[n] = bytes(32 * n + (lane & 31));
+        }
+        // runs of four and of two pieces would put every fourth or eighth row on the same banks
+        first = lds + (kFirst == 4 ? (lane ^ (lane >> 4)) * 16 : lane * 16);
+        second = lds + kFirst * 1024 + (lane ^ (lane >> 4 & 1)) * 16;
+    }
+    __device__ __forceinline__ void load(int unit) {
+        const std::uint8_t* one = tile;
+        const std::uint8_t* two = tile;
+        if constexpr (ENC == kEncQ8_0) {
+            one += unit * 68;
+        } else if constexpr (ENC == kEncBF16) {
+            one += unit * 128;
+        } else {
+            one += (unit >> 2) * static_cast<int>(block_bytes(ENC));
+            two = one + (ENC == kEncQ4K ? 16 + 32 * (unit & 3) : ENC == kEncQ5K ? 48 + 32 * (unit & 3) : 128 + 16 * (unit & 2));
+            if constexpr (ENC == kEncQ6K) one += 32 * (unit & 2);
+        }
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+#pragma unroll
+            for (int part = 0; part < kParts; ++part) {
+                held[part][i] = *reinterpret_cast<const u32x4_a2*>((i < kFirst ? one : two) + (from[i] + 64 * part));
+            }
+        }
+    }
+    // (Q6_K) straight into registers, when those of the unit before are taken
+    __device__ __forceinline__ void load_scales(int unit, int half) {
+        typedef std::uint32_t u32_a2 __attribute__((aligned(2)));
+        const std::uint8_t* block = tile + (unit >> 2) * 210;
+        const int place = half != 0 ? 192 + 4 * (unit & 3) : 206;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) scales[n] = *reinterpret_cast<const u32_a2*>(block + (scales_from[n] + place));
+    }
+    __device__ __forceinline__ void store(int part, int piece) const {
+        std::uint8_t* const target = piece < kFirst ? first + piece * 1024 : second + (piece - kFirst) * 1024;
+        *reinterpret_cast<u32x4*>(target) = held[part][piece];
+    }
+};
+
+// ... and back: a lane's words of row 32 n + inner
+template <std::uint32_t ENC>
+struct Taken {
+    Unit<ENC> unit;
+    std::uint32_t tail;
+    __device__ __forceinline__ void take(const std::uint8_t* lds, const Staged<ENC>& staged, int n, int at, int step, int lane) {
+        const int inner = lane & 31, half = lane >> 5;
+        const auto piece = [&](int offset) { return *reinterpret_cast<const u32x4*>(lds + offset); };
+        if constexpr (ENC == kEncQ8_0) {
+            const int row = (32 * n + inner) * 80;
+            if (step == 0) {
+                unit.codes[0] = piece(row + 16 * half);
+                tail = *reinterpret_cast<const std::uint32_t*>(lds + row + 16 + 28 * half);
+            } else {
+                unit.codes[1] = piece(row + 48 + 16 * half);
+            }
+        } else if constexpr (ENC == kEncBF16) {
+            const int row = (32 * n + inner) * 64, turn = inner >> 2 & 3;
+            unit.values[step][0] = piece(row + 16 * ((2 * half) ^ turn));
+            unit.values[step][1] = piece(row + 16 * ((2 * half + 1) ^ turn));
+        } else if (step == 0) {
+            const int second = 1024 * Staged<ENC>::kFirst + (32 * n + inner) * 32 + 16 * (half ^ (inner >> 3 & 1));
+            if constexpr (ENC == kEncQ6K) {
+                const int row = (32 * n + inner) * 64, turn = inner >> 2 & 3;
+                unit.upper = at & 1;
+                unit.low[0] = piece(row + 16 * (half ^ turn));
+                unit.low[1] = piece(row + 16 * ((2 + half) ^ turn));
+                unit.high = piece(second);
+                unit.scales = staged.scales[n];
+            } else {
+                const int row = (32 * n + inner) * 16 * Staged<ENC>::kFirst;
+                unit.group = at & 3;
+                unit.header = piece(row);
+                if constexpr (ENC == kEncQ5K) unit.fifth = piece(row + 16 + 16 * half);
+                unit.codes = piece(second);
+            }
+        }
+    }
+    // once, when the words are there
+    __device__ __forceinline__ void arrange(int step, int half) {
+        if constexpr (ENC == kEncQ8_0) {
+            // the first block's codes begin at byte 2; behind the upper lanes' lies the second block's scale
+            if (step != 0) return;
+            unit.d[0] = half != 0 ? tail >> 16 : unit.codes[0][0];
+            unit.d[0] &= 0xffffu;
+#pragma unroll
+            for (int word = 0; word < 4; ++word) {
+                unit.codes[0][word] = __builtin_amdgcn_alignbyte(word < 3 ? unit.codes[0][word + 1] : tail, unit.codes[0][word], 2);
+            }
+            unit.arrange();
+        } else if (step == 0) {
+            unit.arrange();
+        }
+    }
+};
 
 template <std::uint32_t ENC, int MT>
 __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
@@ -735,7 +876,6 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
     const int steps = static_cast<int>(input_dim / 32);
     const int units = (steps + 1) / 2;
     const int first_unit = units * group / kGroups, end_unit = units * (group + 1) / kGroups;
-    const int turns = (units + kGroups - 1) / kGroups;  // the longest group's units: all groups meet at the barriers
 
     // cutter's role: quad lane % 8 of the rows 8 (2 item + partner) + lane / 8: a load instruction
     // reads whole 128-byte lines of eight rows
@@ -768,9 +908,9 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
         *reinterpret_cast<uint2*>(stage + 2 * MT * kTermBytes) = make_uint2(a0, a1);
         if constexpr (Slice::kMinimum) {
             float total = ((x[item][0] + x[item][1]) + (x[item][2] + x[item][3])) * kLift;
-            total += __shfl_xor(total, 1);
-            total += __shfl_xor(total, 2);
-            total += __shfl_xor(total, 4);  // (the eight lanes of a row store the same sum)
+            total += of_lane<0xb1>(total);   // lane ^ 1
+            total += of_lane<0x4e>(total);   // lane ^ 2
+            total += of_lane<0x141>(total);  // the row's other four lanes (mirrored; all eight store the same sum)
             sums[(step & 3) * 32 * MT + 8 * (2 * item + partner) + (lane >> 3)] = total;
         }
     };
@@ -787,35 +927,32 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
                                                 m * kTermBytes + chunk_of(use) * kChunkOctets * kOctetBytes);
     };
 
-    const std::uint8_t* w_row[2];
-#pragma unroll
-    for (int n = 0; n < 2; ++n) w_row[n] = data + min(col0 + 32 * n + inner, output_dim - 1) * row_stride;
+    using Stage = Staged<ENC>;
+    std::uint8_t* const stage = lds + kGroups * kGroupBytes<MT> + wave * Stage::kBytes;
+    Stage weights(data, row_stride, col0, output_dim, stage, lane);
+    Taken<ENC> taken[2];
     f32x16 acc[2][MT];
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) acc[n][m] = f32x16{};
     }
-    Slice even[2], odd[2];  // packed bytes of the units to come, by the unit's place in the group's run
     bf16x8 a[kUses];
     u32x4 b[2][2];  // [n][chunk]: codes; those of n = 0 are decoded a step ahead, those of n = 1 under the first tile
     float scale[2][2], scale_before[2];
-    const auto load_weights = [&](Slice (&into)[2], int unit) {
-#pragma unroll
-        for (int n = 0; n < 2; ++n) load_unit<ENC>(into[n], w_row[n], min(unit, end_unit - 1), half, steps);
-    };
-    const auto decode_piece = [&](Slice& source, int n, int step, int piece) {
-        if (step == 0 && piece == 0) source.arrange();  // a unit's first piece
+    const auto load_weights = [&](int unit) { weights.load(min(unit, end_unit - 1)); };
+    const auto decode_piece = [&](int n, int step, int piece) {
+        Taken<ENC>& source = taken[n];
+        if (piece == 0) source.arrange(step, half);
         const int chunk = piece >> 1, word = piece & 1;
         std::uint32_t low, high;
-        source.words(step, chunk, word, low, high);
+        source.unit.words(step, chunk, word, low, high);
         b[n][chunk][2 * word] = low;
         b[n][chunk][2 * word + 1] = high;
-        if (word == 1) scale[n][chunk] = source.scale(step, chunk);
+        if (word == 1) scale[n][chunk] = source.unit.scale(step, chunk);
     };
     if (first_unit < end_unit) {
-        load_weights(even, first_unit);
-        load_weights(odd, first_unit + 1);
+        load_weights(first_unit);
 #pragma unroll
         for (int item = 0; item < kItems; ++item) load_input(item, 2 * first_unit);
 #pragma unroll
@@ -824,16 +961,50 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
             load_input(item, 2 * first_unit + 1);
         }
 #pragma unroll
-        for (int piece = 0; piece < 4; ++piece) decode_piece(even[0], 0, 0, piece);
+        for (int piece = 0; piece < Stage::kPieces; ++piece) weights.store(0, piece);
+        if constexpr (ENC == kEncQ6K) weights.load_scales(first_unit, half);
+        taken[0].take(stage, weights, 0, first_unit, 0, lane);
+        taken[1].take(stage, weights, 1, first_unit, 0, lane);
+        if constexpr (Stage::kParts == 1) load_weights(first_unit + 1);
+#pragma unroll
+        for (int piece = 0; piece < 4; ++piece) decode_piece(0, 0, piece);
     }
+    // Each wave says which step's terms it has handed over; its partner waits for that alone.  (The two
+    // take the same steps, and either says so before it waits: each wait ends.)
+    // (a word a lane: 64 writes of one word would take turns)
+    std::uint32_t* const handed = reinterpret_cast<std::uint32_t*>(lds + kGroups * kGroupBytes<MT> + kLargeWaves * Stage::kBytes);
+    handed[wave * kWave + lane] = 2 * first_unit;
     __syncthreads();
     if (first_unit < end_unit) {
 #pragma unroll
         for (int use = 0; use < kUses; ++use) a[use] = read_fragment(use, 0, 2 * first_unit);
     }
 
-    // One unit, two steps: `own_bytes` holds its packed bytes, `next_bytes` those of the unit behind it.
-    const auto pass = [&](Slice (&own_bytes)[2], Slice (&next_bytes)[2], int unit) {
+    const auto partners_step = [&] {
+        return __hip_atomic_load(&handed[(wave ^ 1) * kWave], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    const std::uint32_t partners_word = static_cast<std::uint32_t>(reinterpret_cast<std::uintptr_t>(
+        (__attribute__((address_space(3))) std::uint32_t*)(handed + (wave ^ 1) * kWave)));
+    // (in assembly: with a branch that the compiler sees, its registers no longer do)
+    const auto wait_for_partner = [&](std::uint32_t seen, int step) {
+        std::uint32_t word, place = partners_word;
+        int value = static_cast<int>(__builtin_amdgcn_readfirstlane(seen));
+        __asm__ volatile(
+            "s_cmp_lt_i32 %0, %3\n\t"
+            "s_cbranch_scc0 .Lhanded%=\n"
+            ".Lwait%=:\n\t"
+            "ds_read_b32 %1, %2\n\t"
+            "s_waitcnt lgkmcnt(0)\n\t"
+            "v_readfirstlane_b32 %0, %1\n\t"
+            "s_cmp_lt_i32 %0, %3\n\t"
+            "s_cbranch_scc1 .Lwait%=\n"
+            ".Lhanded%=:"
+            : "+s"(value), "=&v"(word)
+            : "v"(place), "s"(step)
+            : "scc", "memory");
+    };
+    // One unit, two steps.
+    const auto pass = [&](int unit) {
         float least[2] = {};
 #pragma unroll
         for (int step = 0; step < 2; ++step) {
@@ -845,14 +1016,16 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
             // handed over (before the last tile, whose slots read the next step's fragments) and
             // their successors requested; codes.
             constexpr int kSlots = 12 * MT, kHandOver = kSlots - kUses, kPerPiece = MT == 1 ? 2 : 4;
+            constexpr int kHandOut = (kItems - 1) * kPerPiece;  // the last piece of activations is cut
             f32x16 partial[2];
+            std::uint32_t seen = 0;
 #pragma unroll
             for (int slot = 0; slot < kSlots; ++slot) {
                 const int tile = slot / kUses, use = slot % kUses, m = tile >> 1, n = tile & 1;
                 const int sum = slot / kSum;  // sums since the step's start; partial[sum & 1]
                 __builtin_amdgcn_sched_barrier(0);
                 if (slot == kHandOver) {
-                    __syncthreads();
+                    wait_for_partner(seen, at + 1);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 if constexpr (Slice::kScaled) {
@@ -876,20 +1049,41 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
                     cut_input(slot / kPerPiece, at + 1);
                     load_input(slot / kPerPiece, at + 2);
                 }
-                if (slot < 4) decode_piece(own_bytes[1], 1, step, slot);
-                if (slot == 4 && step == 1) {
+                if (slot < 4) decode_piece(1, step, slot);
+                // What the next step (packed formats: the next unit) needs goes to where the wave's reads
+                // are behind it: LDS keeps a wave's order.  bf16's next unit, requested in this one, as late
+                // as its readers allow.
+                constexpr int kStores = (Stage::kPieces + 1) / 2;
+                const int first_store = Stage::kParts == 2 && step == 1 ? kHandOver - 1 - kStores : 0;
+                if ((Stage::kParts == 2 || step == 1) && slot >= first_store && slot < first_store + kStores) {
+                    const int piece = 2 * (slot - first_store);
+                    weights.store(Stage::kParts == 2 ? 1 - step : 0, piece);
+                    if (piece + 1 < Stage::kPieces) weights.store(Stage::kParts == 2 ? 1 - step : 0, piece + 1);
+                }
+                if (slot == 4) {
                     if constexpr (Slice::kMinimum) {
 #pragma unroll
-                        for (int k = 0; k < 2; ++k) least[k] = -(half != 0 ? own_bytes[k].minimum(1) : own_bytes[k].minimum(0));
+                        for (int k = 0; k < 2 && step == 1; ++k) least[k] = -(half != 0 ? taken[k].unit.minimum(1) : taken[k].unit.minimum(0));
                     }
-                    load_weights(own_bytes, unit + 2);
+                    if (step == (Stage::kParts == 2 ? 0 : 1)) load_weights(unit + (Stage::kParts == 2 ? 1 : 2));
                 }
+                if (ENC == kEncQ6K && slot == 5 && step == 0) weights.load_scales(min(unit + 1, end_unit - 1), half);
+                if (slot == kHandOut) {
+                    // (LDS takes a wave's operations in order: the terms, and the reads of what the partner will
+                    // overwrite next, are ahead of this)
+                    __asm__ volatile("" ::: "memory");
+                    __hip_atomic_store(&handed[wave * kWave + lane], at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __asm__ volatile("" ::: "memory");
+                }
+                if (slot == kHandOver - 2) seen = partners_step();
+                if (slot == kHandOver - 1) taken[0].take(stage, weights, 0, unit + step, 1 - step, lane);
+                if (slot == kHandOver + 4) taken[1].take(stage, weights, 1, unit + step, 1 - step, lane);
                 if (slot == kHandOver) {  // (the last sums of n = 0 are scaled below, with the old factors)
                     scale_before[0] = scale[0][0];
                     scale_before[1] = scale[0][1];
                 }
                 if (slot > kHandOver && slot <= kHandOver + 4) {
-                    decode_piece(step == 0 ? own_bytes[0] : next_bytes[0], 0, 1 - step, slot - kHandOver - 1);
+                    decode_piece(0, 1 - step, slot - kHandOver - 1);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -913,24 +1107,7 @@ __global__ __launch_bounds__(kLargeWaves * kWave, 2) void linear_exact_kernel(
             }
         }
     };
-    // (uniform: a group without a unit left waits out the turn's two barriers)
-    for (int turn = 0; turn < turns; turn += 2) {
-        const int unit = first_unit + turn;
-        if (unit < end_unit) {
-            pass(even, odd, unit);
-        } else {
-            __syncthreads();
-            __syncthreads();
-        }
-        if (turn + 1 < turns) {
-            if (unit + 1 < end_unit) {
-                pass(odd, even, unit + 1);
-            } else {
-                __syncthreads();
-                __syncthreads();
-            }
-        }
-    }
+    for (int unit = first_unit; unit < end_unit; ++unit) pass(unit);
     __syncthreads();
 
     // meeting[group] of either partner's 32 x 32 outputs: partner p's sets lie behind each other
@@ -958,9 +1135,11 @@ void launch_large(const Descriptor& weight, const float* input, const float* bia
                   hipStream_t stream) {
     const std::int64_t row_tiles = (rows + 32 * MT - 1) / (32 * MT);
     const std::int64_t column_tiles = (weight.output_dim + 64 * kPartners - 1) / (64 * kPartners);
+    constexpr int kLds = kGroups * kGroupBytes<MT> + kLargeWaves * (Staged<ENC>::kBytes + 4 * kWave);
+    static_assert(kLds <= 160 * 1024 && kLds >= kLargeWaves * 16 * kWave * 4, "the waves' sums meet in the same memory");
     allow_large_lds<linear_exact_kernel<ENC, MT>>();
     hipLaunchKernelGGL((linear_exact_kernel<ENC, MT>), dim3(static_cast<unsigned>(row_tiles * column_tiles)),
-                       dim3(kLargeWaves * kWave), kLargeLds<MT>, stream, weight.data, weight.row_stride_bytes, input,
+                       dim3(kLargeWaves * kWave), kLds, stream, weight.data, weight.row_stride_bytes, input,
                        bias, output, rows, weight.input_dim, weight.output_dim, static_cast<int>(row_tiles));
 }
 
@@ -976,28 +1155,35 @@ void launch_small(const Descriptor& weight, const float* input, const float* bia
 }
 
 // What a round of the larger tiles costs in rounds of 32 x 32: 32 x 64, 32 x 128 and 64 x 128 (F32:
-// 64 x 32 and 64 x 64).  From a sweep over 484 shapes an encoding (4..512 rows, 64..8,192 outputs,
+// 64 x 32 and 64 x 64).  From a sweep over 242 shapes an encoding (F32 484; 4..512 rows, 64..8,192 outputs,
 // 2,048..8,192 columns, every form of each): the middle of the values with which the rule loses least
-// to the fastest form.  Mean and largest loss, and with 1.35, 2.1 and 2.9 for all packed encodings and
-// bf16 (F32 1.4 and 2.1): Q4_K 0.01 and 3.6 % (0.31 and 12), Q5_K 0.05 and 8 (0.37 and 20), Q6_K 0.10 and
-// 23 (0.09 and 23), Q8_0 0.00 and 0.4 (0.01 and 4), bf16 none (0.05 and 14), F32 0.13 and 11 (0.39 and 11).
+// to the fastest form.  Mean and largest loss, and with 1.4, 2.5 and 3.9 (Q5_K 1.35, 2.5 and 3.6; Q6_K and
+// Q8_0 1.45, 2.1 and 2.6; bf16 1.5, 2.0 and 2.4), the prices while the large form read its weights lane
+// by lane: Q4_K none (0.37 and 13 %), Q5_K none (0.59 and 26), Q6_K 0.26 and 9, Q8_0 0.13 and 5 (1.2 and 29),
+// bf16 0.14 and 8 (3.8 and 30); F32 0.13 and 11.
 template <std::uint32_t ENC>
-constexpr double kRounds[3] = {1.45, 2.1, 2.6};  // Q6_K, Q8_0
+constexpr double kRounds[3] = {1.45, 2.1, 2.6};  // Q6_K
 template <>
-constexpr double kRounds<kEncQ4K>[3] = {1.4, 2.5, 3.9};
+constexpr double kRounds<kEncQ4K>[3] = {1.5, 1.9, 3.3};
 template <>
-constexpr double kRounds<kEncQ5K>[3] = {1.35, 2.5, 3.6};
+constexpr double kRounds<kEncQ5K>[3] = {1.5, 1.9, 3.3};
 template <>
-constexpr double kRounds<kEncBF16>[3] = {1.5, 2.0, 2.4};
+constexpr double kRounds<kEncQ8_0>[3] = {1.6, 1.3, 2.3};
+template <>
+constexpr double kRounds<kEncBF16>[3] = {1.6, 1.3, 1.4};
+// ... of 32 x 128 beyond 32 rows.  bf16, nothing to decode: below a round of 32 x 32 (36..64 rows, 2,304..4,608
+// columns 16.6..29.6 -> 15.4..27.9 us).  With fewer rows the small form looks up fewer lines (5 rows of 5,120 columns
+// 20 us against 30).
+template <std::uint32_t ENC>
+constexpr double kManyRows = ENC == kEncBF16 ? 0.95 : kRounds<ENC>[1];
 template <>
 constexpr double kRounds<kEncF32>[3] = {1.6, 2.1, 0.0};
 
 template <std::uint32_t ENC>
 void launch_for(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
                 hipStream_t stream) {
-    // What bounds all forms is the look-up of lines in the unit's vector cache, which a round of
-    // tiles, one workgroup a unit, makes as often however many of its rows are real: the form with
-    // the cheapest rounds takes the call.
+    // A round of tiles, one workgroup a unit, takes as long however many of its rows are real: the
+    // form with the cheapest rounds takes the call.
     const std::int64_t units = compute_units();
     const auto rounds = [&](std::int64_t height, std::int64_t width) {
         const std::int64_t tiles = (rows + height - 1) / height * ((weight.output_dim + width - 1) / width);
@@ -1016,7 +1202,7 @@ void launch_for(const Descriptor& weight, const float* input, const float* bias,
     } else {
         const bool whole = weight.input_dim % 64 == 0;
         const double cost_wide = kRounds<ENC>[0] * rounds(32, 64);
-        const double cost_low = whole ? kRounds<ENC>[1] * rounds(32, 128) : 1e30;
+        const double cost_low = whole ? (rows > 32 ? kManyRows<ENC> : kRounds<ENC>[1]) * rounds(32, 128) : 1e30;
         const double cost_high = whole ? kRounds<ENC>[2] * rounds(64, 128) : 1e30;
         if (cost_high <= cost_low && cost_high <= cost_wide && cost_high <= cost_small) {
             launch_large<ENC, 2>(weight, input, bias, output, rows, stream);

@@ -201,6 +201,20 @@ def test_exact_linear_forms_at_their_edges(cuda, oracle, encoding, rows, out_dim
     assert normalised_error(y[: rows - 1], expected[: rows - 1]) <= 1e-5 if rows > 1 else True
 
 
+@pytest.mark.parametrize("rows", [100, 200])  # 32 x 128 and 64 x 128 tiles
+@pytest.mark.parametrize("out_dim", [6529, 6592, 6593])  # one, 64 and 65 rows in the last tile's pair of waves
+@pytest.mark.parametrize("encoding,in_dim", [
+    (encoding, 64 * units) for encoding in ALL_PACKED + [kquant.BF16]
+    for units in ((4, 20) if kquant.BLOCKS[encoding][0] == 256 else (1, 3, 5))])  # K groups of none, one, two and five units
+def test_exact_linear_tiles_of_128_columns(cuda, oracle, encoding, in_dim, out_dim, rows):
+    """The form whose waves turn their weights in LDS and wait in pairs.  Bound: as above."""
+    packed = kquant.quantize(encoding, kquant.synthetic_weights(7 + rows, out_dim, in_dim))
+    x = kquant.synthetic_activations(8 + rows, rows, in_dim) + np.float32(0.3)
+    weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    y = tile_ops.linear(weight, to_device(x, cuda)).cpu().numpy()
+    assert normalised_error(y, oracle.linear(encoding, packed, out_dim, in_dim, x)) <= 1e-5
+
+
 @pytest.mark.parametrize("out_dim,in_dim", [(67, 512), (6656, 768), (9000, 256), (33, 2048)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
 def test_exact_linear_rows_carry_the_same_bits_within_a_form(cuda, encoding, out_dim, in_dim):
