@@ -27,8 +27,9 @@
 // for its weight row and up to 8 tokens, the integers of a unit, and replays the float tail
 // above.  Wave w takes the classes w and 15 - w (an even share of any row length), keeps the
 // four chains of a class per token in registers, and leaves (c0 + c1) + (c2 + c3) per class,
-// token and row in LDS; after one barrier a thread per (token, row) adds the 16 classes in the
-// tree's order.  A workgroup walks the tiles blockIdx.x, blockIdx.x + gridDim.x, ... with the
+// token and row in LDS; when all have, a thread per (token, row) adds the 16 classes in the
+// tree's order (up to eight tokens a tile later, the waves waiting for each other's counts in LDS; more: after a
+// barrier).  A workgroup walks the tiles blockIdx.x, blockIdx.x + gridDim.x, ... with the
 // loads of the next tile's first block in flight under the last block of the one before.
 // One pass over the weights for up to 16 tokens.
 //
@@ -40,7 +41,11 @@
 // sums from the records instead of a second pair of products, products issued around the tail
 // before.  Q4_K, 2 x 16,384 rows of 6,656 columns: 39.6 -> 31.2 us at four tokens, 41.9 -> 39.0 at
 // seven, quantizer launch included; Q5_K 44.5 -> 35.8 and 48.2 -> 43.2, Q8_0 54.1 -> 48.2 and
-// 57.0 -> 52.5, Q6_K 58.4 -> 53.3 and 63.1 -> 58.9.
+// 57.0 -> 52.5, Q6_K 58.4 -> 53.3 and 63.1 -> 58.9.  With a barrier a tile its waves waited for the one with
+// the most blocks (26 of a row are three for most waves, four for two): counts instead, at seven tokens,
+// Q4_K 39.6 -> 38.3, Q6_K 58.9 -> 55.4 us, four projections of 8,704 rows 18.5 -> 17.3 and 26.0 -> 24.4;
+// one tile a workgroup or even shares as before.  (More than eight tokens leave no memory for four tiles'
+// sums; with two, and the counts to be cleared first, 3 to 7 % slower.)
 #include "common.hpp"
 #include "gemv_rows.hpp"
 #include "wave_rows.hpp"
@@ -172,6 +177,25 @@ __device__ __forceinline__ void rows_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+__device__ __forceinline__ std::uint32_t lds_address(const int* word) {
+    return static_cast<std::uint32_t>(reinterpret_cast<std::uintptr_t>((const __attribute__((address_space(3))) int*)word));
+}
+
+// until each of the workgroup's waves has said `count` or more (the word of wave lane % 8 at `words`).  In
+// assembly, so that the requests in flight stay counted as they are.
+__device__ __forceinline__ void rows_wait_for_all(std::uint32_t words, int count) {
+    std::uint32_t word;
+    __asm__ volatile(
+        ".Lwait%=:\n\t"
+        "ds_read_b32 %0, %1\n\t"
+        "s_waitcnt lgkmcnt(0)\n\t"
+        "v_cmp_gt_i32 vcc, %2, %0\n\t"
+        "s_cbranch_vccnz .Lwait%=\n"
+        : "=&v"(word)
+        : "v"(words), "s"(count)
+        : "vcc", "memory");
+}
+
 // SPLIT: a workgroup computes one half of a row's butterfly, the classes 0..7 (the first
 // left_groups workgroups) or 8..15 (the others), a wave one class, and adds (q0 + q1) or
 // (q2 + q3) onto the output, which the quantizer launch has filled with -0: two terms commute,
@@ -192,7 +216,11 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
     constexpr bool kDeep = S <= 4;  // registers for two blocks of packed bytes in flight
     // (two buffers of class sums: the workgroup's waves meet once per tile)
     constexpr int kOwnClasses = SPLIT ? kClasses / 2 : kClasses;
-    __shared__ float class_sums[2][kOwnClasses][kTokens][kRowsTile];
+    constexpr int kTilesHeld = kDeep ? 4 : 2;
+    __shared__ float class_sums[kTilesHeld][kOwnClasses][kTokens][kRowsTile];
+    // how many tiles a wave has left its sums of [0], and added its part of [1] (a word a lane: 64 writes
+    // of one word would take turns)
+    __shared__ int said[2][kDeep ? kRowsWaves : 1][kWave];
     __shared__ __attribute__((aligned(16))) std::uint8_t packed_tiles[kRowsWaves][F::kTileBytes];
 
     const int lane = threadIdx.x & 63;
@@ -208,6 +236,14 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
     const std::uint32_t tile_stride =
         SPLIT ? (right_half ? gridDim.x - left_groups : left_groups) : gridDim.x;
     const int my_tiles = static_cast<int>((total_tiles - first_tile + tile_stride - 1) / tile_stride);
+    if (kDeep && my_tiles > 1) {
+        said[0][wave][lane] = 0;
+        said[1][wave][lane] = 0;
+        __syncthreads();
+    }
+    const auto wait_for_all = [&](int what, int count) {
+        rows_wait_for_all(lds_address(&said[what][lane & (kRowsWaves - 1)][0]), count);
+    };
     auto projection_of = [&](std::uint32_t tile) {
         int which = 0;
 #pragma unroll
@@ -665,32 +701,30 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
         }
     };
     // a class is complete: (c0 + c1) + (c2 + c3) per token goes to LDS
-    int parity = 0;
+    int work = 0;  // of the workgroup's tiles
     auto finish_class = [&](int cls) {
 #pragma unroll
         for (int slot = 0; slot < S; ++slot) {
-            class_sums[parity][cls & (kOwnClasses - 1)][S * h + slot][j] =
+            class_sums[work % kTilesHeld][cls & (kOwnClasses - 1)][S * h + slot][j] =
                 (acc[0][slot] + acc[1][slot]) + (acc[2][slot] + acc[3][slot]);
 #pragma unroll
             for (int p = 0; p < 4; ++p) acc[p][slot] = 0.0f;
         }
     };
-    // a tile is complete: after the barrier a thread per (token, row) adds the 16 classes in
+    // ... after all waves' have gone there, a thread per (token, row) adds the 16 classes of a tile in
     // the order of the one-row kernel's butterfly
-    std::uint32_t work_tile = first_tile;
-    auto finish_tile = [&]() {
-        __syncthreads();
-        const Projection op = projection_of(work_tile);
-        const std::int64_t row0 = static_cast<std::int64_t>(work_tile - op.first_tile) * kRowsTile;
+    const int token = static_cast<int>(threadIdx.x) >> 5;
+    auto add_classes = [&](int index) {
+        const std::uint32_t tile = first_tile + static_cast<std::uint32_t>(index) * tile_stride;
+        const Projection op = projection_of(tile);
+        const std::int64_t row0 = static_cast<std::int64_t>(tile - op.first_tile) * kRowsTile;
         const int valid_rows =
             static_cast<int>(min(static_cast<std::int64_t>(kRowsTile), op.output_dim - row0));
-        const int token = static_cast<int>(threadIdx.x) >> 5;
         if (token < kTokens && token < tokens && j < valid_rows) {
+            const auto& sums = class_sums[index % kTilesHeld];
             float pairs[kOwnClasses / 2];
 #pragma unroll
-            for (int m = 0; m < kOwnClasses / 2; ++m) {
-                pairs[m] = class_sums[parity][2 * m][token][j] + class_sums[parity][2 * m + 1][token][j];
-            }
+            for (int m = 0; m < kOwnClasses / 2; ++m) pairs[m] = sums[2 * m][token][j] + sums[2 * m + 1][token][j];
             float* output = op.output + (static_cast<std::int64_t>(token) * op.output_dim + row0 + j);
             if constexpr (SPLIT) {
                 // this half of the butterfly; the other workgroup's joins it in either order
@@ -713,13 +747,42 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
                 *output = (q0 + q1) + (q2 + q3);
             }
         }
-        parity ^= 1;
-        work_tile += tile_stride;
+    };
+    // A tile's waves do not meet: each says how many tiles it has left the sums of and how many it has
+    // added its part of, adds a tile's when it has finished the next one, and waits only for what it
+    // needs (a wave never waits for one that can wait for it: what is waited for lies a tile or more
+    // behind).  The last tile's meet at a barrier.
+    const auto finish_tile = [&]() {
+        if constexpr (kDeep) {
+            if (my_tiles > 1) {
+                said[0][wave][lane] = work + 1;
+                rows_lds_fence();
+            }
+            if (work > 0) {
+                if (wave * 2 < tokens) {
+                    wait_for_all(0, work);
+                    add_classes(work - 1);
+                    rows_lds_fence();
+                }
+                said[1][wave][lane] = work;
+                rows_lds_fence();
+            }
+        }
+        if (!kDeep || work + 1 == my_tiles) {
+            __syncthreads();
+            add_classes(work);
+        }
+        ++work;
+    };
+    // before the first class of a tile: its place was that of the tile kTilesHeld before
+    const auto begin_sums = [&]() {
+        if (kDeep && work >= kTilesHeld) wait_for_all(1, work - kTilesHeld + 1);
     };
 
     if (role.total == 0) {
         // (rows of fewer blocks than classes: this wave only takes part in the sums)
         for (int n = 0; n < my_tiles; ++n) {
+            begin_sums();
             finish_class(role.class0);
             if constexpr (!SPLIT) finish_class(role.class1);
             finish_tile();
@@ -749,7 +812,10 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
     // (class0 = r has at least as many blocks as class1 = 15 - r; a class without blocks leaves
     // the zeros the sums start from)
     auto finish_step = [&]() {
-        if (work_step == role.count0 - 1) finish_class(role.class0);
+        if (work_step == role.count0 - 1) {
+            begin_sums();
+            finish_class(role.class0);
+        }
         if (work_step == role.total - 1) {
             if constexpr (!SPLIT) finish_class(role.class1);
             finish_tile();

@@ -796,6 +796,22 @@ def test_verifier_matrix_core_rows_of_many_tiles_a_workgroup(cuda, encoding, in_
             assert_bits_equal(batch[row:row + 1].contiguous(), alone[row], f"row {row} of {rows}")
 
 
+@pytest.mark.parametrize("in_dim,out_dim", [(256, 42000), (1024, 50000), (6656, 8704), (6656, 13000)])
+@pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q6_K, kquant.Q8_0])
+def test_verifier_matrix_core_rows_whose_waves_wait_by_counts(cuda, encoding, in_dim, out_dim):
+    """Waves without a block of their own over six tiles, halves of tiles shared by two workgroups (one
+    and two a workgroup), tokens that leave some waves nothing to add, against the one-row call."""
+    weight = tile_ops.PackedWeight.from_numpy(encoding, random_packed(encoding, out_dim, in_dim, 81), out_dim, in_dim)
+    x = to_device(kquant.synthetic_activations(82, 8, in_dim), cuda)
+    one = tile_ops.small_batch_workspace(1, in_dim)
+    alone = [tile_ops.mmvq_linear(weight, x[row:row + 1], one) for row in range(8)]
+    for rows in (4, 5, 7, 8):
+        workspace = tile_ops.small_batch_workspace(rows, in_dim)
+        batch = tile_ops.multi_linear([weight], x[:rows], workspace, family="mmvq")[0]
+        for row in range(rows):
+            assert_bits_equal(batch[row:row + 1].contiguous(), alone[row], f"row {row} of {rows}")
+
+
 @pytest.mark.parametrize("in_dim,out_dim", [(6656, 3000), (6656, 4608), (13312, 2100), (4096, 2500)])
 def test_q6k_rows_carry_the_same_bits_wherever_their_wave_starts(cuda, oracle, in_dim, out_dim):
     """The Q6_K streaming kernel hands a wave a contiguous range of rows, and how many depends on
