@@ -17,15 +17,25 @@
 //
 // A workgroup's waves share one tile and cut K between them; their sums meet in LDS at the end, in
 // a fixed order.  Two forms:
-//   linear_exact_small_kernel, a tile of 32 MT x 32 NT, each wave streaming its own operands straight
-//   into registers (no LDS, no barrier in the loop): what a problem of a few tiles needs (38 rows x
-//   332 outputs are 22 of 32 x 32 for 256 compute units), there is no long walk over K;
+//   linear_exact_small_kernel, a tile of 32 MT x 32 NT, each wave streaming its own weights straight
+//   into registers and its own activations through LDS, where they lie cut (no barrier in the loop): what a
+//   problem of a few tiles needs (38 rows x 332 outputs are 22 of 32 x 32 for 256 compute units), there is no
+//   long walk over K;
 //   linear_exact_kernel, a tile of 32 MT input rows x 128 weight rows for two waves (64 weight rows
 //   each) in each of four K groups.  The two cut the activations of a step of 32 columns between
 //   them and hand the terms over in LDS.
-// What bounds the small form is the vector cache: a load instruction that reads 16 bytes from each of 32
-// rows looks up 32 lines for 1 KB, and a unit pulls some 20 GB/s that way.  The large form did the same
-// (a look-up in 72 % of the cycles, the matrix cores busy in 26 %); it loads its weights with
+// What bounded both is the vector cache: a load instruction that reads 16 bytes from each of 32 rows
+// looks up 32 lines for 1 KB, and a unit pulls some 20 GB/s that way.  The small form loads its activations
+// eight lanes a row instead, eight rows an instruction, and so loads and cuts only the rows that are there (by
+// eights: 8, 16 or 32), which every tile of weight rows does again: 4,096 -> 6,656 at 5 / 16 / 25 / 64 rows Q4_K
+// 15.2 / 17.4 / 19.6 / 28.7 -> 12.2 / 15.1 / 18.1 / 28.4 us, Q5_K 16.8 / 19.7 / 22.2 / 34.0 -> 13.7 / 16.3 /
+// 20.0 / 30.8, Q6_K 21.8 / 24.1 / 27.6 / 46.6 -> 20.5 / 21.5 / 25.6 / 42.0, Q8_0 24.2 / 28.2 / 31.0 / 45.9 ->
+// 21.6 / 22.8 / 25.6 / 38.3, bf16 20.4 / 23.9 / 27.1 / 38.4 -> 18.1 / 21.1 / 23.2 / 31.5, F32 32.4 / 33.5 / 35.7 /
+// 55.9 -> 28.4 / 31.2 / 33.1 / 51.6, at 200 rows 135 -> 114.  (Its buffer loads of activations as global ones take
+// registers that Q5_K does not have: 25 rows 20.0 -> 24.3.  Weights requested behind the next step's activations:
+// Q8_0 2 % faster, F32 of 64 rows 46.6 -> 55.0.)  What is left is the cut and the decode (16 waves'
+// vector instructions, 4 to 10 us) and for Q8_0, bf16 and F32 the look-ups of their weights.  The large form
+// (a look-up in 72 % of the cycles, the matrix cores busy in 26 %) loads its weights with
 // neighbouring lanes on neighbouring pieces of a row and turns them in LDS, each wave its own, and the two
 // waves of a group wait for each other alone instead of for the workgroup.  4,096 -> 6,656 at 100 / 200 /
 // 512 rows, loads as the lanes use them -> through LDS -> and with waits in pairs: Q8_0 73 / 84 / 165 -> 41 /
@@ -37,11 +47,11 @@
 // matrix instructions 21: two waves a SIMD overlap them in part.  (Sums of all tiles meeting in LDS at
 // once instead of tile by tile: no difference.  Requests two steps ahead instead of one, and the matrix
 // instructions of a step before its other work instead of between it: neither.)  The 64 x 128 form of Q6_K
-// keeps six registers that do not change in its loop in scratch (28 bytes a lane), the 64 x 64 form of F32
-// seven (32 bytes), read outside of its loop only; the others none.
+// keeps six registers that do not change in its loop in scratch (28 bytes a lane), read outside of it; the
+// 32 x 32 form of Q6_K for 17 rows and more four (32 bytes); the others none.
 // Measured at 4,096 -> 6,656, against the vector kernel (16 rows) and the float matrix instruction (200,
-// 512 rows) before: Q4_K 134 -> 16 us at 16 rows, 203 -> 62 at 200, 311 -> 121 at 512; Q8_0 368 -> 27,
-// 180 -> 55, 279 -> 108; F32 406 -> 30, 172 -> 136, 271 -> 254.
+// 512 rows) before: Q4_K 134 -> 15 us at 16 rows, 203 -> 62 at 200, 311 -> 121 at 512; Q8_0 368 -> 23,
+// 180 -> 55, 279 -> 108; F32 406 -> 31, 172 -> 114, 271 -> 217.
 //
 // The entry point, nfn_native_tile_linear_packed_weight_float32_v1, has no workspace argument
 // (neuralfn/csrc/native_train/tile_ops.h:614-620; reference kernel
@@ -307,15 +317,16 @@ template <>
 struct Unit<kEncF32> {
     static constexpr bool kWide = true, kScaled = false, kMinimum = false;
     f32x4_a4 values[2][2][2];  // [step][chunk][piece]
+    __device__ __forceinline__ void load_step(const std::uint8_t* row, int unit, int half, int steps, int step) {
+        const auto* source = reinterpret_cast<const float*>(row) + min(2 * unit + step, steps - 1) * 32 + 16 * half;
+#pragma unroll
+        for (int piece = 0; piece < 4; ++piece) {
+            values[step][piece >> 1][piece & 1] = *reinterpret_cast<const f32x4_a4*>(source + 4 * piece);
+        }
+    }
     __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half, int steps) {
 #pragma unroll
-        for (int step = 0; step < 2; ++step) {
-            const auto* source = reinterpret_cast<const float*>(row) + min(2 * unit + step, steps - 1) * 32 + 16 * half;
-#pragma unroll
-            for (int piece = 0; piece < 4; ++piece) {
-                values[step][piece >> 1][piece & 1] = *reinterpret_cast<const f32x4_a4*>(source + 4 * piece);
-            }
-        }
+        for (int step = 0; step < 2; ++step) load_step(row, unit, half, steps, step);
     }
     __device__ __forceinline__ void arrange() {}
     __device__ __forceinline__ Terms terms(int step, int chunk) const {
@@ -601,25 +612,31 @@ __device__ __attribute__((noinline)) void take_again_apart(std::uint64_t again, 
     take_again<ENC, MT, WAVES>(again, wave, data, row_stride, input, input_dim, bias, output, output_dim, row0, col0);
 }
 
-// WAVES waves share a tile of 32 MT input rows x 32 NT weight rows.
-template <std::uint32_t ENC, int MT, int NT, int WAVES>
+// A wave's activations of one step in LDS, [term][row tile][octet of columns][row] of 16 bytes; the rows
+// of an octet change places by its number, so that four lanes with a row's octets and lanes with
+// neighbouring rows of one find distinct banks.
+template <int MT>
+constexpr int kOwnTerms = 3 * MT * 4 * 512;
+template <int MT, int NT, int WAVES>
+constexpr int kSmallLds = WAVES * (kOwnTerms<MT> + 4 * 32 * MT * 4);
+
+// WAVES waves share a tile of 32 MT input rows x 32 NT weight rows, of which the first 8 ITEMS of each
+// 32 exist (the products of the others are not stored).  ITEMS = 0: each lane loads and cuts what it
+// multiplies, which spares a short walk over K the way through LDS.
+template <std::uint32_t ENC, int MT, int NT, int WAVES, int ITEMS>
 __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exact_small_kernel(
     const std::uint8_t* __restrict__ data, std::int64_t row_stride, const float* __restrict__ input,
     const float* __restrict__ bias, float* __restrict__ output, std::int64_t rows, std::int64_t input_dim,
     std::int64_t output_dim, int row_tiles) {
     using Slice = Unit<ENC>;
-    constexpr int kLow = Slice::kWide ? 16 : 8, kNext = Slice::kWide ? 8 : 16;  // lane's columns: kLow half + kNext chunk
-    __shared__ float meeting[WAVES][16 * kWave];
+    extern __shared__ __attribute__((aligned(16))) std::uint8_t lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int inner = lane & 31, half = lane >> 5;
     const std::int64_t row0 = static_cast<std::int64_t>(blockIdx.x % row_tiles) * (32 * MT);
     const std::int64_t col0 = static_cast<std::int64_t>(blockIdx.x / row_tiles) * (32 * NT);
     // Rows past the end read the last one again; their results are not stored.
-    const float* x_row[MT];
     const std::uint8_t* w_row[NT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) x_row[m] = input + min(row0 + 32 * m + inner, rows - 1) * input_dim + kLow * half;
 #pragma unroll
     for (int n = 0; n < NT; ++n) w_row[n] = data + min(col0 + 32 * n + inner, output_dim - 1) * row_stride;
     const int steps = static_cast<int>(input_dim / 32);
@@ -633,56 +650,156 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
 #pragma unroll
         for (int m = 0; m < MT; ++m) acc[n][m] = f32x16{};
     }
-    f32x4_a4 x[MT][2][2];  // [row tile][chunk][piece] of the step ahead
+    // Cutter: quad lane % 8 of the rows 8 item + lane / 8; a load instruction reads whole lines.
+    float* const sums = reinterpret_cast<float*>(lds + WAVES * kOwnTerms<MT>) + wave * 4 * 32 * MT;  // [step % 4][row]
+    const int quad = lane & 7;
+    const __amdgpu_buffer_rsrc_t x_tile = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(input + row0 * input_dim), 0, 0xffffffff, 0x00020000);
+    // (ITEMS = 0: columns 16 half + 8 chunk (kWide), 8 half + 16 chunk of row `inner`)
+    const float* const x_row = input + min(row0 + inner, rows - 1) * input_dim + (Slice::kWide ? 16 : 8) * half;
+    const int last_row = static_cast<int>(min(rows - 1 - row0, std::int64_t(32 * MT)));
+    constexpr int kLoads = ITEMS == 0 ? 4 : ITEMS;
+    std::uint32_t x_from[MT][kLoads];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+#pragma unroll
+        for (int item = 0; item < kLoads; ++item) {
+            x_from[m][item] = 4 * (static_cast<std::uint32_t>(min(32 * m + 8 * item + (lane >> 3), last_row)) *
+                                       static_cast<std::uint32_t>(input_dim) + 4 * quad);
+        }
+    }
+    f32x4_a4 x[MT][kLoads];  // of the step behind the one in LDS
     const auto load_inputs = [&](int step) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
 #pragma unroll
-            for (int piece = 0; piece < 4; ++piece) {
-                x[m][piece >> 1][piece & 1] = *reinterpret_cast<const f32x4_a4*>(
-                    x_row[m] + static_cast<std::int64_t>(step) * 32 + kNext * (piece >> 1) + 4 * (piece & 1));
+            for (int item = 0; item < kLoads; ++item) {
+                if constexpr (ITEMS == 0) {
+                    constexpr int kNext = Slice::kWide ? 8 : 16;
+                    x[m][item] = *reinterpret_cast<const f32x4_a4*>(
+                        x_row + static_cast<std::int64_t>(min(step, last_step)) * 32 + kNext * (item >> 1) + 4 * (item & 1));
+                } else {
+                    x[m][item] = __builtin_bit_cast(f32x4_a4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                  x_tile, x_from[m][item], min(step, last_step) * 128, 0));
+                }
             }
         }
     };
+    const int octet = quad >> 1;
+    // (eight rows on: 128 bytes, in the other order where the octet changes that bit)
+    const std::uint32_t target = wave * kOwnTerms<MT> + octet * 512 + ((lane >> 3) ^ (4 * octet)) * 16 + (quad & 1) * 8;
+    const auto cut_inputs = [&](int step) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+#pragma unroll
+            for (int item = 0; item < ITEMS; ++item) {
+                const f32x4_a4 v = x[m][item];
+                std::uint32_t a0, b0, c0, a1, b1, c1;
+                cut_pair(v[0], v[1], a0, b0, c0);
+                cut_pair(v[2], v[3], a1, b1, c1);
+                std::uint8_t* const to = lds + (target ^ (item * 128)) + m * 2048;
+                *reinterpret_cast<uint2*>(to) = make_uint2(a0, a1);
+                *reinterpret_cast<uint2*>(to + MT * 2048) = make_uint2(b0, b1);
+                *reinterpret_cast<uint2*>(to + 2 * MT * 2048) = make_uint2(c0, c1);
+                if constexpr (Slice::kMinimum) {
+                    float total = ((v[0] + v[1]) + (v[2] + v[3])) * kLift;
+                    total += of_lane<0xb1>(total);   // lane ^ 1
+                    total += of_lane<0x4e>(total);   // lane ^ 2
+                    total += of_lane<0x141>(total);  // the row's other four lanes (mirrored; all eight store the same sum)
+                    sums[(step & 3) * 32 * MT + 32 * m + 8 * item + (lane >> 3)] = total;
+                }
+            }
+        }
+    };
+    // Multiplier: octets 2 half + chunk (kWide) or 2 chunk + half of row `inner`
+    const int from = Slice::kWide ? 2 * half : half;
+    const std::uint32_t fragments = wave * kOwnTerms<MT> + from * 512 + (inner ^ (4 * from)) * 16;
+    constexpr std::uint32_t kOther = Slice::kWide ? 512 + 4 * 16 : 1024 + 8 * 16;  // the bits that chunk 1 changes
     if (first_unit < end_unit) {
+        // (2 x 2 tiles leave no registers for a second unit of float weights: a step's, as they are used up)
+        constexpr bool kAhead = MT * NT < 4;
         Slice now[NT], next[NT];
 #pragma unroll
         for (int n = 0; n < NT; ++n) load_unit<ENC>(now[n], w_row[n], first_unit, half, steps);
         load_inputs(2 * first_unit);
+        if constexpr (ITEMS > 0) {
+            cut_inputs(2 * first_unit);
+            load_inputs(2 * first_unit + 1);
+        }
         for (int unit = first_unit; unit < end_unit; ++unit) {
 #pragma unroll
             for (int n = 0; n < NT; ++n) now[n].arrange();
+            if constexpr (kAhead) {
 #pragma unroll
-            for (int n = 0; n < NT; ++n) load_unit<ENC>(next[n], w_row[n], min(unit + 1, end_unit - 1), half, steps);
-            float partial[MT][2];
+                for (int n = 0; n < NT; ++n) load_unit<ENC>(next[n], w_row[n], min(unit + 1, end_unit - 1), half, steps);
+            }
+            float partial[2];  // (ITEMS == 0: the lane's half of its row's sums)
 #pragma unroll
             for (int step = 0; step < 2; ++step) {
                 if (!kWholeBlocks<ENC> && 2 * unit + step > last_step) break;  // (uniform: a row's odd last block)
-                Terms a[MT][2];
-#pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    partial[m][step] = 0.0f;
+                const auto read = [&](int m, int chunk) {
+                    const std::uint8_t* const at = lds + (fragments ^ (chunk * kOther)) + m * 2048;
+                    return Terms{*reinterpret_cast<const bf16x8*>(at), *reinterpret_cast<const bf16x8*>(at + MT * 2048),
+                                 *reinterpret_cast<const bf16x8*>(at + 2 * MT * 2048)};
+                };
+                // (the cut behind the reads of what it overwrites: LDS keeps a wave's order)
+                // (of 32 rows the one past a wave's end is worth leaving out: 25 rows of Q4_K, 2,304 -> 8,000
+                // 15.2 -> 13.7 us; of fewer the branch costs as much)
+                const auto cut_next = [&] {
+                    if (ITEMS < 4 || ENC == kEncQ6K || step == 0 || unit + 1 < end_unit) cut_inputs(2 * unit + step + 1);
+                    load_inputs(2 * unit + step + 2);
+                };
+                if constexpr (ITEMS == 0) {
+                    Terms a[1][2];
+                    partial[step] = 0.0f;
 #pragma unroll
                     for (int chunk = 0; chunk < 2; ++chunk) {
                         float eight[8];
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) eight[j] = x[m][chunk][j >> 2][j & 3];
-                        a[m][chunk] = cut(eight);
-                        if constexpr (Slice::kMinimum) partial[m][step] += sum_of(eight) * kLift;
+                        for (int j = 0; j < 8; ++j) eight[j] = x[0][2 * chunk + (j >> 2)][j & 3];
+                        a[0][chunk] = cut(eight);
+                        if constexpr (Slice::kMinimum) partial[step] += sum_of(eight) * kLift;
                     }
-                }
-                load_inputs(min(2 * unit + step + 1, last_step));
+                    load_inputs(2 * unit + step + 1);
 #pragma unroll
-                for (int n = 0; n < NT; ++n) multiply<ENC, MT>(acc[n], a, now[n], step);
+                    for (int n = 0; n < NT; ++n) multiply<ENC, 1>(acc[n], a, now[n], step);
+                } else if constexpr (MT == 1) {
+                    const Terms a[1][2] = {{read(0, 0), read(0, 1)}};
+                    cut_next();
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) multiply<ENC, 1>(acc[n], a, now[n], step);
+                } else {
+                    static_assert(MT == 1 || ENC == kEncF32, "no registers for both chunks' fragments");
+#pragma unroll
+                    for (int chunk = 0; chunk < 2; ++chunk) {
+                        Terms a[MT];
+#pragma unroll
+                        for (int m = 0; m < MT; ++m) a[m] = read(m, chunk);
+#pragma unroll
+                        for (int n = 0; n < NT; ++n) {
+                            const Terms b = now[n].terms(step, chunk);
+#pragma unroll
+                            for (int m = 0; m < MT; ++m) acc[n][m] = product(a[m], b, acc[n][m]);
+                        }
+                    }
+                    if constexpr (!kAhead) {
+#pragma unroll
+                        for (int n = 0; n < NT; ++n) now[n].load_step(w_row[n], min(unit + 1, end_unit - 1), half, steps, step);
+                    }
+                    cut_next();
+                }
             }
             if constexpr (Slice::kMinimum) {
                 // k index = half: the lower lanes bring step 0's sums and minimums, the upper ones
-                // step 1's.  A lane holds half of its row's sum of each step; the other half is 32
-                // lanes away.
+                // step 1's
 #pragma unroll
                 for (int m = 0; m < MT; ++m) {
-                    const float other = __shfl_xor(half != 0 ? partial[m][0] : partial[m][1], 32);
-                    const float total = (half != 0 ? partial[m][1] : partial[m][0]) + other;
+                    float total;
+                    if constexpr (ITEMS == 0) {
+                        total = (half != 0 ? partial[1] : partial[0]) + __shfl_xor(half != 0 ? partial[0] : partial[1], 32);
+                    } else {
+                        total = sums[((2 * unit + half) & 3) * 32 * MT + 32 * m + inner];
+                    }
 #pragma unroll
                     for (int n = 0; n < NT; ++n) {
                         const float least = -(half != 0 ? now[n].minimum(1) : now[n].minimum(0));
@@ -691,9 +808,11 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
                 }
             }
 #pragma unroll
-            for (int n = 0; n < NT; ++n) now[n] = next[n];
+            for (int n = 0; n < NT; ++n) now[n] = kAhead ? next[n] : now[n];
         }
     }
+    if constexpr (ITEMS > 0) __syncthreads();
+    float(*meeting)[16 * kWave] = reinterpret_cast<float(*)[16 * kWave]>(lds);
     std::uint64_t again = 0;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
@@ -1143,24 +1262,47 @@ void launch_large(const Descriptor& weight, const float* input, const float* bia
                        bias, output, rows, weight.input_dim, weight.output_dim, static_cast<int>(row_tiles));
 }
 
-template <std::uint32_t ENC, int MT, int NT, int WAVES>
-void launch_small(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
-                  hipStream_t stream) {
+template <std::uint32_t ENC, int MT, int NT, int WAVES, int ITEMS>
+void launch_small_form(const Descriptor& weight, const float* input, const float* bias, float* output,
+                       std::int64_t rows, hipStream_t stream) {
     const std::int64_t row_tiles = (rows + 32 * MT - 1) / (32 * MT);
     const std::int64_t column_tiles = (weight.output_dim + 32 * NT - 1) / (32 * NT);
-    hipLaunchKernelGGL((linear_exact_small_kernel<ENC, MT, NT, WAVES>),
-                       dim3(static_cast<unsigned>(row_tiles * column_tiles)), dim3(WAVES * kWave), 0, stream,
+    constexpr int kLds = ITEMS == 0 ? WAVES * 16 * kWave * 4 : kSmallLds<MT, NT, WAVES>;
+    static_assert(kLds >= WAVES * 16 * kWave * 4, "the waves' sums meet in the same memory");
+    allow_large_lds<linear_exact_small_kernel<ENC, MT, NT, WAVES, ITEMS>>();
+    hipLaunchKernelGGL((linear_exact_small_kernel<ENC, MT, NT, WAVES, ITEMS>),
+                       dim3(static_cast<unsigned>(row_tiles * column_tiles)), dim3(WAVES * kWave), kLds, stream,
                        weight.data, weight.row_stride_bytes, input, bias, output, rows, weight.input_dim,
                        weight.output_dim, static_cast<int>(row_tiles));
 }
 
+template <std::uint32_t ENC, int MT, int NT, int WAVES>
+void launch_small(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
+                  hipStream_t stream) {
+    if constexpr (WAVES == 16 && kWholeBlocks<ENC>) {
+        // Walks of two or three units a wave, through LDS and not: 25 rows of Q6_K 2,048 -> 300 13.2 and 11.0 us,
+        // 3,328 -> 8,000 27.0 and 26.4, 4,096 -> 6,656 25.6 and 27.5; 16 rows 10.9 and 10.3, 15.0 and 16.2 (3,072 ->
+        // 2,000), 21.5 and 24.2; 25 rows of Q4_K 2,560 -> 8,000 14.3 and 13.7, 3,072 -> 2,000 12.9 and 13.4, and
+        // 2,048 -> 300 9.1 and 10.3.
+        const bool wide = (weight.output_dim + 31) / 32 * 3 > compute_units();
+        if (ENC == kEncQ6K ? weight.input_dim <= (rows > 16 ? 3328 : 2048) : rows > 16 && weight.input_dim <= 2560 && wide) {
+            return launch_small_form<ENC, MT, NT, WAVES, 0>(weight, input, bias, output, rows, stream);
+        }
+    }
+    if constexpr (MT == 1) {
+        if (rows <= 8) return launch_small_form<ENC, MT, NT, WAVES, 1>(weight, input, bias, output, rows, stream);
+        if (rows <= 16) return launch_small_form<ENC, MT, NT, WAVES, 2>(weight, input, bias, output, rows, stream);
+    }
+    launch_small_form<ENC, MT, NT, WAVES, 4>(weight, input, bias, output, rows, stream);
+}
+
 // What a round of the larger tiles costs in rounds of 32 x 32: 32 x 64, 32 x 128 and 64 x 128 (F32:
-// 64 x 32 and 64 x 64).  From a sweep over 242 shapes an encoding (F32 484; 4..512 rows, 64..8,192 outputs,
+// 64 x 32 and 64 x 64).  From a sweep over 242 shapes an encoding (4..512 rows, 64..8,192 outputs,
 // 2,048..8,192 columns, every form of each): the middle of the values with which the rule loses least
-// to the fastest form.  Mean and largest loss, and with 1.4, 2.5 and 3.9 (Q5_K 1.35, 2.5 and 3.6; Q6_K and
-// Q8_0 1.45, 2.1 and 2.6; bf16 1.5, 2.0 and 2.4), the prices while the large form read its weights lane
-// by lane: Q4_K none (0.37 and 13 %), Q5_K none (0.59 and 26), Q6_K 0.26 and 9, Q8_0 0.13 and 5 (1.2 and 29),
-// bf16 0.14 and 8 (3.8 and 30); F32 0.13 and 11.
+// to the fastest form.  Mean and largest loss, and with the prices before the forms loaded whole lines (Q4_K
+// 1.4, 2.5 and 3.9; Q5_K 1.35, 2.5 and 3.6; Q6_K and Q8_0 1.45, 2.1 and 2.6; bf16 1.5, 2.0 and 2.4; F32 1.6 and
+// 2.1): Q4_K 0.01 and 3 % (0.55 and 15), Q5_K 0.03 and 9 (0.73 and 20), Q6_K none, Q8_0 0.13 and 7 (0.32 and
+// 7), bf16 0.25 and 11 (the same), F32 0.03 and 6 (0.19 and 13).
 template <std::uint32_t ENC>
 constexpr double kRounds[3] = {1.45, 2.1, 2.6};  // Q6_K
 template <>
@@ -1168,16 +1310,11 @@ constexpr double kRounds<kEncQ4K>[3] = {1.5, 1.9, 3.3};
 template <>
 constexpr double kRounds<kEncQ5K>[3] = {1.5, 1.9, 3.3};
 template <>
-constexpr double kRounds<kEncQ8_0>[3] = {1.6, 1.3, 2.3};
+constexpr double kRounds<kEncQ8_0>[3] = {1.55, 1.7, 2.8};
 template <>
-constexpr double kRounds<kEncBF16>[3] = {1.6, 1.3, 1.4};
-// ... of 32 x 128 beyond 32 rows.  bf16, nothing to decode: below a round of 32 x 32 (36..64 rows, 2,304..4,608
-// columns 16.6..29.6 -> 15.4..27.9 us).  With fewer rows the small form looks up fewer lines (5 rows of 5,120 columns
-// 20 us against 30).
-template <std::uint32_t ENC>
-constexpr double kManyRows = ENC == kEncBF16 ? 0.95 : kRounds<ENC>[1];
+constexpr double kRounds<kEncBF16>[3] = {1.55, 1.9, 2.4};
 template <>
-constexpr double kRounds<kEncF32>[3] = {1.6, 2.1, 0.0};
+constexpr double kRounds<kEncF32>[3] = {1.35, 1.65, 0.0};
 
 template <std::uint32_t ENC>
 void launch_for(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
@@ -1202,7 +1339,7 @@ void launch_for(const Descriptor& weight, const float* input, const float* bias,
     } else {
         const bool whole = weight.input_dim % 64 == 0;
         const double cost_wide = kRounds<ENC>[0] * rounds(32, 64);
-        const double cost_low = whole ? (rows > 32 ? kManyRows<ENC> : kRounds<ENC>[1]) * rounds(32, 128) : 1e30;
+        const double cost_low = whole ? kRounds<ENC>[1] * rounds(32, 128) : 1e30;
         const double cost_high = whole ? kRounds<ENC>[2] * rounds(64, 128) : 1e30;
         if (cost_high <= cost_low && cost_high <= cost_wide && cost_high <= cost_small) {
             launch_large<ENC, 2>(weight, input, bias, output, rows, stream);

@@ -201,6 +201,21 @@ def test_exact_linear_forms_at_their_edges(cuda, oracle, encoding, rows, out_dim
     assert normalised_error(y[: rows - 1], expected[: rows - 1]) <= 1e-5 if rows > 1 else True
 
 
+@pytest.mark.parametrize("rows", [7, 8, 9, 16, 17, 39])  # the last and the first of those cut by 8, 16 and 32 rows
+@pytest.mark.parametrize("out_dim", [33, 3000, 8300])  # 32 x 32 (few, many) and, by two, 32 x 64 tiles (F32: 64 x 32)
+@pytest.mark.parametrize("encoding,in_dim", [
+    (encoding, in_dim) for encoding in ALL_PACKED + [kquant.F32, kquant.BF16]
+    for in_dim in ((512, 3584) if kquant.BLOCKS[encoding][0] == 256 else (544,))])
+def test_exact_linear_cuts_the_rows_that_are_there(cuda, oracle, encoding, in_dim, out_dim, rows):
+    """The forms of a few tiles: walks over K that go through LDS and short ones that do not, rows of an
+    odd number of 32 columns where the format has them.  Bound: as above."""
+    packed = kquant.quantize(encoding, kquant.synthetic_weights(9, out_dim, in_dim))
+    x = kquant.synthetic_activations(10 + rows, rows, in_dim) + np.float32(0.3)
+    weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    y = tile_ops.linear(weight, to_device(x, cuda)).cpu().numpy()
+    assert normalised_error(y, oracle.linear(encoding, packed, out_dim, in_dim, x)) <= 1e-5
+
+
 @pytest.mark.parametrize("rows", [100, 200])  # 32 x 128 and 64 x 128 tiles
 @pytest.mark.parametrize("out_dim", [6529, 6592, 6593])  # one, 64 and 65 rows in the last tile's pair of waves
 @pytest.mark.parametrize("encoding,in_dim", [
