@@ -376,8 +376,10 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
         if (++fetch_step >= fetch_role.total && fetch_tile + tile_stride < total_tiles) {
             fetch_step = 0;
             fetch_tile += tile_stride;
-            fetch_r = (fetch_r + role_step) & (kRowsWaves - 1);
-            fetch_role = role_of(fetch_r);
+            if constexpr (kDeep) {
+                fetch_r = (fetch_r + role_step) & (kRowsWaves - 1);
+                fetch_role = role_of(fetch_r);
+            }
             aim(fetch_tile);
         }
     };
@@ -820,7 +822,7 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
             if constexpr (!SPLIT) finish_class(role.class1);
             finish_tile();
             work_step = 0;
-            role = role_of((role.class0 + role_step) & (kRowsWaves - 1));
+            if constexpr (kDeep) role = role_of((role.class0 + role_step) & (kRowsWaves - 1));
         } else {
             ++work_step;
         }
@@ -828,6 +830,7 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
     // the block after the one being worked on (past the end of the walk: any)
     auto next_block = [&]() {
         if (work_step < role.total - 1) return block_of(role, work_step + 1);
+        if constexpr (!kDeep) return role.class0;
         return (SPLIT && right_half ? 8 : 0) + ((role.class0 + role_step) & (kRowsWaves - 1));
     };
     // one step of the walk: its packed bytes go to LDS, the operands of the next step and the packed
