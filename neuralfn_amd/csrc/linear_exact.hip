@@ -577,8 +577,8 @@ __device__ __forceinline__ float decoded_dot(const std::uint8_t* row, const floa
 // half is NaN where the product with the weight is infinite, and the lifted products leave the float
 // range (activations above some 2^90 with codes, products above 2^80 with float weights) before those
 // with the weights do.  MT: as in the kernels below.
-// 4,096 -> 6,656 at 200 rows (Q8_0 / Q4_K, 86 / 75 us from Python): with a NaN in one row 89 / 80 us, in
-// every row 123 / 100; an infinity or activations of 3e37 in one row 204 / 237, in every row 3.6 / 3.4 ms
+// 4,096 -> 6,656 at 200 rows (Q8_0 / Q4_K, 60 / 68 us from Python): with a NaN in one row 62 / 72 us, in
+// every row 100 / 91; an infinity or activations of 3e37 in one row 181 / 225, in every row 3.6 / 3.4 ms
 // (a byte and a weight at a time: 1.1 / 1.9 ms for one row of either kind, 29 / 64 for all).
 template <std::uint32_t ENC, int MT, int WAVES>
 __device__ __forceinline__ void take_again(std::uint64_t again, int wave, const std::uint8_t* data,
@@ -1300,9 +1300,10 @@ void launch_small(const Descriptor& weight, const float* input, const float* bia
 // 64 x 32 and 64 x 64).  From a sweep over 242 shapes an encoding (4..512 rows, 64..8,192 outputs,
 // 2,048..8,192 columns, every form of each): the middle of the values with which the rule loses least
 // to the fastest form.  Mean and largest loss, and with the prices before the forms loaded whole lines (Q4_K
-// 1.4, 2.5 and 3.9; Q5_K 1.35, 2.5 and 3.6; Q6_K and Q8_0 1.45, 2.1 and 2.6; bf16 1.5, 2.0 and 2.4; F32 1.6 and
-// 2.1): Q4_K 0.01 and 3 % (0.55 and 15), Q5_K 0.03 and 9 (0.73 and 20), Q6_K none, Q8_0 0.13 and 7 (0.32 and
-// 7), bf16 0.25 and 11 (the same), F32 0.03 and 6 (0.19 and 13).
+// 1.4, 2.5 and 3.9; Q5_K 1.35, 2.5 and 3.6; Q6_K and Q8_0 1.45, 2.1 and 2.6; bf16 1.5, 2.0 and 2.4): Q4_K 0.01 and
+// 3 % (0.55 and 15), Q5_K 0.03 and 9 (0.73 and 20), Q6_K none, Q8_0 0.13 and 7 (0.32 and 7), bf16 0.25 and 11 (the
+// same).  F32 0.19 and 13 with its old prices; 1.35 and 1.65 would lose 0.03 and 6, but send more shapes to the
+// tiles of 64 rows, whose sums round more (3.4e-7 of the result against 1.3e-7).
 template <std::uint32_t ENC>
 constexpr double kRounds[3] = {1.45, 2.1, 2.6};  // Q6_K
 template <>
@@ -1314,7 +1315,7 @@ constexpr double kRounds<kEncQ8_0>[3] = {1.55, 1.7, 2.8};
 template <>
 constexpr double kRounds<kEncBF16>[3] = {1.55, 1.9, 2.4};
 template <>
-constexpr double kRounds<kEncF32>[3] = {1.35, 1.65, 0.0};
+constexpr double kRounds<kEncF32>[3] = {1.6, 2.1, 0.0};
 
 template <std::uint32_t ENC>
 void launch_for(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
