@@ -750,24 +750,25 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
             }
         }
     };
+    // (behind what it announces: LDS takes a wave's operations in the order that the fences keep)
+    const auto say = [&](int what, int count) {
+        rows_lds_fence();
+        __hip_atomic_store(&said[what][wave][lane], count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        rows_lds_fence();
+    };
     // A tile's waves do not meet: each says how many tiles it has left the sums of and how many it has
     // added its part of, adds a tile's when it has finished the next one, and waits only for what it
     // needs (a wave never waits for one that can wait for it: what is waited for lies a tile or more
     // behind).  The last tile's meet at a barrier.
     const auto finish_tile = [&]() {
         if constexpr (kDeep) {
-            if (my_tiles > 1) {
-                said[0][wave][lane] = work + 1;
-                rows_lds_fence();
-            }
+            if (my_tiles > 1) say(0, work + 1);
             if (work > 0) {
                 if (wave * 2 < tokens) {
                     wait_for_all(0, work);
                     add_classes(work - 1);
-                    rows_lds_fence();
                 }
-                said[1][wave][lane] = work;
-                rows_lds_fence();
+                say(1, work);
             }
         }
         if (!kDeep || work + 1 == my_tiles) {
