@@ -50,6 +50,8 @@
 #include "gemv_rows.hpp"
 #include "wave_rows.hpp"
 
+#include <type_traits>
+
 namespace nfn {
 
 namespace {
@@ -835,17 +837,20 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
         return (SPLIT && right_half ? 8 : 0) + ((role.class0 + role_step) & (kRowsWaves - 1));
     };
     // one step of the walk: its packed bytes go to LDS, the operands of the next step and the packed
-    // bytes of the one after that are requested, its products are taken
-    auto take_step = [&](RowsPacked<ENC>& packed, const RowsOperands<S>& here, RowsOperands<S>& next) {
+    // bytes of the one after that are requested (`last`: nothing is left to request), its products are
+    // taken
+    auto take_step = [&](RowsPacked<ENC>& packed, const RowsOperands<S>& here, RowsOperands<S>& next, auto last) {
         stage_to_lds(packed);
         if constexpr (kDeep) {
             if (lane < kEntries) my_extras[extra_entry] = here.extra;
         }
         rows_lds_fence();
-        // (in the order in which they are waited for)
-        if constexpr (!kDeep) fetch_packed(packed);
-        fetch_operands(next, next_block());
-        if constexpr (kDeep) fetch_packed(packed);
+        if constexpr (!last) {
+            // (in the order in which they are waited for)
+            if constexpr (!kDeep) fetch_packed(packed);
+            fetch_operands(next, next_block());
+            if constexpr (kDeep) fetch_packed(packed);
+        }
         compute(here, work_step);
         finish_step();
     };
@@ -859,19 +864,27 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
     if constexpr (kDeep) {
         if (steps >= 2) {
             do {
-                take_step(packed_even, even, odd);
-                take_step(packed_odd, odd, even);
+                take_step(packed_even, even, odd, std::false_type{});
+                take_step(packed_odd, odd, even, std::false_type{});
                 steps -= 2;
             } while (steps >= 2);
         }
-        if (steps != 0) take_step(packed_even, even, odd);
+        if (steps != 0) {
+            // (a loop of one that the optimizer cannot see through, for the one form that would keep
+            // registers in scratch without it: eight of Q6_K's split form, five to eight tokens)
+            int once = 1;
+            if constexpr (F::kQ6 && SPLIT && S == 4) asm volatile("" : "+s"(once));
+            do {
+                take_step(packed_even, even, odd, std::true_type{});
+            } while (--once > 0);
+        }
     } else {
         // (nothing is in flight behind the packed bytes that a step waits for; a third copy of
         // the step spills)
         while (true) {
-            take_step(packed_even, even, odd);
+            take_step(packed_even, even, odd, std::false_type{});
             if (--steps == 0) break;
-            take_step(packed_even, odd, even);
+            take_step(packed_even, odd, even, std::false_type{});
             if (--steps == 0) break;
         }
     }
