@@ -157,7 +157,7 @@ int run_small_batch(bool verifier, const Descriptor* const* descriptors, const f
         // one of them overlaps what that launch reads.
         // (a prequantized call has no such launch: a fill launch of its own where that pays)
         const bool fill_launch = prologue == kRecords;
-        ProjectionSet clear = gemv_rows_split_set(verifier_rows, fill_launch);
+        ProjectionSet clear = gemv_rows_split_set(verifier_rows, rows, fill_launch);
         if (fill_launch) {
             launch_fill_outputs(clear, rows, as_stream(stream));
         } else {

@@ -898,11 +898,13 @@ std::uint32_t tiles_of(const ProjectionSet& set) {
     return tiles;
 }
 
-// How a launch of `tiles` tiles of rows of `blocks` blocks is shared out.  Costs in blocks a
-// SIMD works through (two of a workgroup's eight waves to a SIMD, waves w and w + 4): a whole
-// tile gives wave w the classes w and 15 - w, the split form the class w (left half) or 8 + w
-// (right half); a block and a half per work unit for its first loads, its barrier and its
-// stores (measured: 1.1 us a block, 1.6 us a unit at 16 tokens).
+// How a launch of `tiles` tiles of rows of `blocks` blocks is shared out.  Costs in half blocks that
+// the slowest SIMD works through (two of a workgroup's eight waves to a SIMD, waves w and w + 4): of
+// a whole tile wave w takes the classes w and 15 - w, of a half the class w (left) or 8 + w
+// (right).  Up to eight tokens the shares move on by two waves with every tile (rows of 16 blocks and
+// more), so a SIMD alternates between its share and that of the SIMD two further.  A block and a half
+// per tile or half for its first loads and its stores, and more than eight tokens' barrier (measured:
+// 1.1 us a block, 1.6 us a tile at 16 tokens).
 struct RowsPlan {
     bool split;
     std::uint32_t left_groups;   // split: workgroups on the left halves
@@ -910,43 +912,55 @@ struct RowsPlan {
 };
 
 // fill_launch: the outputs are filled by a launch of its own (a prequantized call has no
-// quantizer launch to do it), which the split form must win back as well (two blocks' time).
-RowsPlan plan_rows(std::uint32_t tiles, std::int64_t input_dim, bool may_split, bool fill_launch = false) {
+// quantizer launch to do it), which the split form must win back as well (two blocks' time, up to
+// eight tokens two and a half).
+// Up to eight tokens the split form is taken wherever it costs no more (equal costs of one tile a
+// workgroup are those of rows of up to eight blocks, whose right halves are empty: whole).  64 to 1,024 tiles of 2,048
+// to 16,384 columns, the four formats, four and seven tokens, 800 calls of either form: the rule takes
+// 0.2 % longer than the faster form on average, 7 % at most (prequantized 0.3 and 15; with fixed
+// shares and a tenth asked for, as for more tokens, 1.5 and 16, prequantized 1.5 and 24).  264 tiles of
+// 4,096 columns, Q6_K, seven tokens: whole 23.9 us, split 20.9; 256 of 6,656, Q8_0, four: 18.3 and 20.2.
+RowsPlan plan_rows(std::uint32_t tiles, std::int64_t input_dim, std::int64_t tokens, bool may_split, bool fill_launch) {
     const std::uint32_t units = static_cast<std::uint32_t>(compute_units());
     const int blocks = static_cast<int>(input_dim >> 8);
+    const bool few = tokens <= 8;
+    const bool moves = few && blocks >= kClasses;
     const auto count = [blocks](int cls) { return cls < blocks ? (blocks - cls + kClasses - 1) / kClasses : 0; };
-    int whole = 0, left = 0, right = 0;
+    int whole[4], left[4], right[4];
     for (int simd = 0; simd < 4; ++simd) {
-        const int a = simd, b = simd + 4;
-        const int whole_here = count(a) + count(kClasses - 1 - a) + count(b) + count(kClasses - 1 - b);
-        const int left_here = count(a) + count(b);
-        const int right_here = count(8 + a) + count(8 + b);
-        whole = whole_here > whole ? whole_here : whole;
-        left = left_here > left ? left_here : left;
-        right = right_here > right ? right_here : right;
+        left[simd] = count(simd) + count(simd + 4);
+        right[simd] = count(8 + simd) + count(12 + simd);
+        whole[simd] = left[simd] + count(kClasses - 1 - simd) + count(kClasses - 1 - (simd + 4));
     }
-    const auto passes = [tiles](std::uint32_t groups) { return (tiles + groups - 1) / groups; };
+    // a workgroup's walk over its share of the tiles, by the blocks of a SIMD
+    const auto cost = [&](const int (&share)[4], std::uint32_t groups) {
+        const std::uint64_t walk = (tiles + groups - 1) / groups, turned = moves ? walk / 2 : 0;
+        std::uint64_t worst = 0;
+        for (int simd = 0; simd < 4; ++simd) {
+            const std::uint64_t here = (walk - turned) * share[simd] + turned * share[simd ^ 2];
+            worst = here > worst ? here : worst;
+        }
+        return 2 * worst + 3 * walk;
+    };
     RowsPlan plan{false, 0, tiles < units ? tiles : units};
     if (!may_split || units < 2) return plan;
-    // costs in half blocks
-    const std::uint64_t whole_cost = static_cast<std::uint64_t>(passes(plan.groups)) * (2 * whole + 3);
+    const std::uint64_t whole_cost = cost(whole, plan.groups);
     std::uint64_t best = ~std::uint64_t(0);
     std::uint32_t best_left = 0, best_right = 0;
     for (std::uint32_t left_groups = 1; left_groups < units; ++left_groups) {
         const std::uint32_t l = left_groups < tiles ? left_groups : tiles;
         const std::uint32_t r = units - left_groups < tiles ? units - left_groups : tiles;
-        const std::uint64_t left_cost = static_cast<std::uint64_t>(passes(l)) * (2 * left + 3);
-        const std::uint64_t right_cost = static_cast<std::uint64_t>(passes(r)) * (2 * right + 3);
-        const std::uint64_t cost = left_cost > right_cost ? left_cost : right_cost;
-        if (cost < best) {
-            best = cost;
+        const std::uint64_t left_cost = cost(left, l), right_cost = cost(right, r);
+        const std::uint64_t either = left_cost > right_cost ? left_cost : right_cost;
+        if (either < best) {
+            best = either;
             best_left = l;
             best_right = r;
         }
     }
-    // (the split form has to win by a tenth: the model is that coarse)
-    if (fill_launch) best += 4;
-    if (best * 10 <= whole_cost * 9) {
+    if (fill_launch) best += few ? 5 : 4;
+    // (more than eight tokens: the split form has to win by a tenth, the model is that coarse)
+    if (few ? best < whole_cost || (best == whole_cost && tiles > units) : best * 10 <= whole_cost * 9) {
         plan.split = true;
         plan.left_groups = best_left;
         plan.groups = best_left + best_right;
@@ -979,7 +993,7 @@ void launch_encoding(ProjectionSet set, const std::uint8_t* image, const std::ui
         set.op[index].first_tile = tiles;
         tiles += static_cast<std::uint32_t>((set.op[index].output_dim + kRowsTile - 1) / kRowsTile);
     }
-    const RowsPlan plan = plan_rows(tiles, set.input_dim, outputs_cleared, fill_launch);
+    const RowsPlan plan = plan_rows(tiles, set.input_dim, tokens, outputs_cleared, fill_launch);
     if (plan.split) {
         launch_form<ENC, true>(set, image, records, tokens, tiles, plan, stream);
     } else {
@@ -1010,12 +1024,12 @@ std::int64_t gemv_rows_image_bytes(std::int64_t input_dim) {
     return (input_dim >> 8) * kImageBlock;
 }
 
-ProjectionSet gemv_rows_split_set(const ProjectionSet& set, bool fill_launch) {
+ProjectionSet gemv_rows_split_set(const ProjectionSet& set, std::int64_t rows, bool fill_launch) {
     ProjectionSet split{};
     split.input_dim = set.input_dim;
     for (const std::uint32_t encoding : kRowsEncodings) {
         const ProjectionSet group = encoding_group(set, encoding);
-        if (group.count == 0 || !plan_rows(tiles_of(group), set.input_dim, true, fill_launch).split) continue;
+        if (group.count == 0 || !plan_rows(tiles_of(group), set.input_dim, rows, true, fill_launch).split) continue;
         for (int index = 0; index < group.count; ++index) split.op[split.count++] = group.op[index];
     }
     return split;

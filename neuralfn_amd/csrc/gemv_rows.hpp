@@ -58,7 +58,7 @@ std::int64_t gemv_rows_image_bytes(std::int64_t input_dim);
 // output (the form that pays when whole tiles would leave most of the chip idle in their last
 // pass): their outputs must hold -0.0f when launch_gemv_rows starts.
 // fill_launch: the fill is a launch of its own (launch_fill_outputs), which has to pay too.
-ProjectionSet gemv_rows_split_set(const ProjectionSet& set, bool fill_launch);
+ProjectionSet gemv_rows_split_set(const ProjectionSet& set, std::int64_t rows, bool fill_launch);
 
 // Fills the outputs (rows x output_dim floats each) of the projections of `clear` with -0.0f.
 void launch_fill_outputs(const ProjectionSet& clear, std::int64_t rows, hipStream_t stream);
@@ -73,7 +73,7 @@ void launch_quantize_records(const float* first, const float* second, int prolog
 
 // rows 4..16 of the set's projections from the operand image and the records beside it.
 // outputs_cleared: the outputs of
-// gemv_rows_split_set(set, fill_launch) hold -0.0f (launch_quantize_records or
+// gemv_rows_split_set(set, rows, fill_launch) hold -0.0f (launch_quantize_records or
 // launch_fill_outputs ran with that set).
 void launch_gemv_rows(const ProjectionSet& set, const std::uint8_t* image,
                       const std::uint8_t* records, std::int64_t rows,

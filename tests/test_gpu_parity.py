@@ -827,6 +827,29 @@ def test_verifier_matrix_core_rows_whose_waves_wait_by_counts(cuda, encoding, in
             assert_bits_equal(batch[row:row + 1].contiguous(), alone[row], f"row {row} of {rows}")
 
 
+@pytest.mark.parametrize("in_dim,over", [(2048, 64), (4096, 8), (4352, 33), (6656, 64)])
+@pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q6_K, kquant.Q8_0])
+def test_verifier_matrix_core_rows_by_halves(cuda, encoding, in_dim, over):
+    """A few tiles more than compute units, up to eight tokens: halves of tiles (rows of eight blocks: the
+    right ones empty), walks of an even and an odd number of steps, the last tile part of one, with the
+    quantizer's fill of the outputs and with one of its own, against the one-row call."""
+    torch = torch_()
+    out_dim = 32 * (torch.cuda.get_device_properties(0).multi_processor_count + over) - 5
+    rows_of = torch.from_numpy(random_packed(encoding, 512, in_dim, 83).reshape(512, -1)).to(cuda)
+    chosen = torch.randint(0, 512, (out_dim,), generator=torch.Generator().manual_seed(84)).to(cuda)
+    weight = tile_ops.PackedWeight(encoding, out_dim, in_dim, rows_of.index_select(0, chosen).reshape(-1))
+    x = to_device(kquant.synthetic_activations(85, 8, in_dim), cuda)
+    one = tile_ops.small_batch_workspace(1, in_dim)
+    alone = [tile_ops.mmvq_linear(weight, x[row:row + 1], one) for row in range(8)]
+    for rows in (4, 5, 8):
+        workspace = tile_ops.small_batch_workspace(rows, in_dim)
+        batch = tile_ops.multi_linear([weight], x[:rows], workspace, family="mmvq")[0]
+        for row in range(rows):
+            assert_bits_equal(batch[row:row + 1].contiguous(), alone[row], f"row {row} of {rows}")
+        again = tile_ops.multi_linear_prequantized([weight], rows, workspace)[0]
+        assert_bits_equal(again, batch, f"{rows} rows prequantized")
+
+
 @pytest.mark.parametrize("in_dim,out_dim", [(6656, 3000), (6656, 4608), (13312, 2100), (4096, 2500)])
 def test_q6k_rows_carry_the_same_bits_wherever_their_wave_starts(cuda, oracle, in_dim, out_dim):
     """The Q6_K streaming kernel hands a wave a contiguous range of rows, and how many depends on
