@@ -60,6 +60,8 @@
 #include "common.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
+
 namespace nfn {
 
 namespace {
@@ -1297,25 +1299,33 @@ void launch_small(const Descriptor& weight, const float* input, const float* bia
 }
 
 // What a round of the larger tiles costs in rounds of 32 x 32: 32 x 64, 32 x 128 and 64 x 128 (F32:
-// 64 x 32 and 64 x 64).  From a sweep over 242 shapes an encoding (4..512 rows, 64..8,192 outputs,
-// 2,048..8,192 columns, every form of each): the middle of the values with which the rule loses least
-// to the fastest form.  Mean and largest loss, and with the prices before the forms loaded whole lines (Q4_K
-// 1.4, 2.5 and 3.9; Q5_K 1.35, 2.5 and 3.6; Q6_K and Q8_0 1.45, 2.1 and 2.6; bf16 1.5, 2.0 and 2.4): Q4_K 0.01 and
-// 3 % (0.55 and 15), Q5_K 0.03 and 9 (0.73 and 20), Q6_K none, Q8_0 0.13 and 7 (0.32 and 7), bf16 0.25 and 11 (the
-// same).  F32 0.19 and 13 with its old prices; 1.35 and 1.65 would lose 0.03 and 6, but send more shapes to the
-// tiles of 64 rows, whose sums round more (3.4e-7 of the result against 1.3e-7).
+// 64 x 32 and 64 x 64).  They choose how many waves share K, and with that how a sum rounds: 16
+// (32 x 32 tiles), eight (32 x 64) or four (the tiles of 128 columns; F32: eight, then four).  From a sweep
+// of 484 shapes an encoding (4..512 rows, 64..8,192 outputs, 2,048..8,192 columns) before the tiles of
+// 128 columns loaded whole lines.  Those would win more shapes of Q4_K and Q5_K since (257 to 512 rows into
+// 4,128 to 8,192 outputs: 1.5, 1.9 and 3.3 lose 0.01 % to the fastest form on average, these 0.6 %,
+// at most 20), with sums of half the waves: 2.6e-7 of the result (rms) instead of 2.4e-7 at 4,096 columns,
+// 3.3e-7 instead of 3.0e-7 at 8,192.  F32's 1.35 and 1.65 would gain 0.2 % with 3.4e-7 instead of 1.3e-7.
 template <std::uint32_t ENC>
-constexpr double kRounds[3] = {1.45, 2.1, 2.6};  // Q6_K
+constexpr double kRounds[3] = {1.45, 2.1, 2.6};  // Q6_K, Q8_0
 template <>
-constexpr double kRounds<kEncQ4K>[3] = {1.5, 1.9, 3.3};
+constexpr double kRounds<kEncQ4K>[3] = {1.4, 2.5, 3.9};
 template <>
-constexpr double kRounds<kEncQ5K>[3] = {1.5, 1.9, 3.3};
+constexpr double kRounds<kEncQ5K>[3] = {1.35, 2.5, 3.6};
 template <>
-constexpr double kRounds<kEncQ8_0>[3] = {1.55, 1.7, 2.8};
-template <>
-constexpr double kRounds<kEncBF16>[3] = {1.55, 1.9, 2.4};
+constexpr double kRounds<kEncBF16>[3] = {1.5, 2.0, 2.4};
 template <>
 constexpr double kRounds<kEncF32>[3] = {1.6, 2.1, 0.0};
+// A round of 64 x 128 in rounds of 32 x 128, whose sums are the same: from 242 shapes an encoding with
+// the tiles as they are (Q8_0 with 1.24: 0.3 % slower on average, 7 % at most).
+template <std::uint32_t ENC>
+constexpr double kTaller = 1.24;  // Q6_K, bf16
+template <>
+constexpr double kTaller<kEncQ4K> = 1.74;
+template <>
+constexpr double kTaller<kEncQ5K> = 1.74;
+template <>
+constexpr double kTaller<kEncQ8_0> = 1.65;
 
 template <std::uint32_t ENC>
 void launch_for(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
@@ -1340,12 +1350,14 @@ void launch_for(const Descriptor& weight, const float* input, const float* bias,
     } else {
         const bool whole = weight.input_dim % 64 == 0;
         const double cost_wide = kRounds<ENC>[0] * rounds(32, 64);
-        const double cost_low = whole ? kRounds<ENC>[1] * rounds(32, 128) : 1e30;
-        const double cost_high = whole ? kRounds<ENC>[2] * rounds(64, 128) : 1e30;
-        if (cost_high <= cost_low && cost_high <= cost_wide && cost_high <= cost_small) {
-            launch_large<ENC, 2>(weight, input, bias, output, rows, stream);
-        } else if (cost_low <= cost_wide && cost_low <= cost_small) {
-            launch_large<ENC, 1>(weight, input, bias, output, rows, stream);
+        const double low = rounds(32, 128), high = rounds(64, 128);
+        const double cost_large = whole ? std::min(kRounds<ENC>[1] * low, kRounds<ENC>[2] * high) : 1e30;
+        if (cost_large <= cost_wide && cost_large <= cost_small) {
+            if (kTaller<ENC> * high <= low) {
+                launch_large<ENC, 2>(weight, input, bias, output, rows, stream);
+            } else {
+                launch_large<ENC, 1>(weight, input, bias, output, rows, stream);
+            }
         } else if (cost_wide <= cost_small) {
             launch_small<ENC, 1, 2, 8>(weight, input, bias, output, rows, stream);
         } else {

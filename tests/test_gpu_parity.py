@@ -246,6 +246,23 @@ def test_exact_linear_rows_carry_the_same_bits_within_a_form(cuda, encoding, out
     assert normalised_error(three.cpu().numpy(), many[:3].cpu().numpy()) <= 1e-5
 
 
+@pytest.mark.parametrize("rows,out_dim", [(257, 7232), (333, 6656), (509, 5056)])
+@pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.BF16])
+def test_exact_linear_of_many_rows_rounds_as_that_of_64(cuda, encoding, rows, out_dim):
+    """Shapes where 32 x 64 tiles and those of 128 columns cost alike: they stay with the former (Q4_K, Q5_K),
+    whose sums are cut among eight waves and not four, and carry the bits of a call of 64 rows, which
+    takes 32 x 64 tiles at these widths.  (The other formats: within the bound of every form.)"""
+    in_dim = 4096
+    packed = random_packed(encoding, out_dim, in_dim, 66) if encoding != kquant.BF16 else kquant.quantize(
+        encoding, kquant.synthetic_weights(66, out_dim, in_dim))
+    weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    x = to_device(kquant.synthetic_activations(67, rows, in_dim), cuda)
+    many, few = tile_ops.linear(weight, x), tile_ops.linear(weight, x[:64])
+    if encoding in (kquant.Q4_K, kquant.Q5_K):
+        assert_bits_equal(many[:64].contiguous(), few, f"64 of {rows} rows")
+    assert normalised_error(many[:64].cpu().numpy(), few.cpu().numpy()) <= 1e-5
+
+
 @pytest.mark.parametrize("in_dim", [2 ** 23, 2 ** 23 + 256])
 @pytest.mark.parametrize("encoding", [kquant.Q8_0, kquant.BF16])
 def test_exact_linear_on_both_sides_of_its_longest_rows(cuda, encoding, in_dim):
