@@ -614,6 +614,14 @@ __device__ __attribute__((noinline)) void take_again_apart(std::uint64_t again, 
     take_again<ENC, MT, WAVES>(again, wave, data, row_stride, input, input_dim, bias, output, output_dim, row0, col0);
 }
 
+// Where a lane writes in LDS what others of its wave read.  LDS takes a wave's operations in order; this keeps
+// the compiler to it, which sees one lane's addresses only: it cannot tell that the lane itself reads
+// elsewhere.  (Fences around the writes, which nothing may pass: Q6_K up to 23 % slower, four rows of Q5_K 7.)
+__device__ __forceinline__ std::uint32_t for_others(std::uint32_t place) {
+    asm("" : "+v"(place));
+    return place;
+}
+
 // A wave's activations of one step in LDS, [term][row tile][octet of columns][row] of 16 bytes; the rows
 // of an octet change places by its number, so that four lanes with a row's octets and lanes with
 // neighbouring rows of one find distinct banks.
@@ -689,7 +697,9 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
     };
     const int octet = quad >> 1;
     // (eight rows on: 128 bytes, in the other order where the octet changes that bit)
-    const std::uint32_t target = wave * kOwnTerms<MT> + octet * 512 + ((lane >> 3) ^ (4 * octet)) * 16 + (quad & 1) * 8;
+    const std::uint32_t target =
+        for_others(wave * kOwnTerms<MT> + octet * 512 + ((lane >> 3) ^ (4 * octet)) * 16 + (quad & 1) * 8);
+    const std::uint32_t sum_target = for_others(lane >> 3);
     const auto cut_inputs = [&](int step) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
@@ -708,7 +718,7 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
                     total += of_lane<0xb1>(total);   // lane ^ 1
                     total += of_lane<0x4e>(total);   // lane ^ 2
                     total += of_lane<0x141>(total);  // the row's other four lanes (mirrored; all eight store the same sum)
-                    sums[(step & 3) * 32 * MT + 32 * m + 8 * item + (lane >> 3)] = total;
+                    sums[(step & 3) * 32 * MT + 32 * m + 8 * item + sum_target] = total;
                 }
             }
         }
@@ -886,8 +896,8 @@ struct Staged {
             for (int n = 0; n < 2; ++n) scales_from[n] = bytes(32 * n + (lane & 31));
         }
         // runs of four and of two pieces would put every fourth or eighth row on the same banks
-        first = lds + (kFirst == 4 ? (lane ^ (lane >> 4)) * 16 : lane * 16);
-        second = lds + kFirst * 1024 + (lane ^ (lane >> 4 & 1)) * 16;
+        first = lds + for_others(kFirst == 4 ? (lane ^ (lane >> 4)) * 16 : lane * 16);
+        second = lds + kFirst * 1024 + for_others((lane ^ (lane >> 4 & 1)) * 16);
     }
     __device__ __forceinline__ void load(int unit) {
         const std::uint8_t* one = tile;
