@@ -915,12 +915,11 @@ int nfn_mi355_k_quant_gemm_float32_v1(
     int mode,
     void* cuda_stream);
 
-/* How the call above cuts a problem of this geometry on the current device
- * (no counterpart in the reference; for tests and benchmarks that want to know
- * which launch form they exercised): *tile_rows = output rows per workgroup
- * tile that the K shares are cut for (256 or 128; 32 for up to 32 rows; the
- * launch takes tiles of 512, 256 or 128 rows, whichever costs least with these
- * shares, to the same sums), *k_shares = workgroups that share the K range of a tile
+/* How the call above cuts K for a problem of this geometry on the current device
+ * (no counterpart in the reference; for tests and benchmarks): *tile_rows =
+ * output rows per workgroup tile that the K shares are cut for (256 or 128; 32
+ * for up to 32 rows; which tiles the launch takes says the query below),
+ * *k_shares = workgroups that share the K range of a tile
  * (1 = unsplit; with more, each writes a partial output into the workspace and
  * a second launch adds them in share order).  0 on success, 1 for an encoding
  * or width the matrix-core path does not take, or the reserved mode. */
@@ -932,6 +931,23 @@ int nfn_mi355_k_quant_gemm_plan_v1(
     int mode,
     int* tile_rows,
     int* k_shares);
+
+/* Which launch form runs 1..4 projections of one encoding and input together (no
+ * counterpart in the reference; for tests and benchmarks): *tile_rows = output
+ * rows per workgroup tile, 512, 256 or 128, whichever costs least with the shares
+ * above (sums do not depend on it); 32 for up to 32 rows.  The projections of a
+ * call that do not find room for their shares beside each other run as several
+ * launches, each of which has a height of its own.  0 on success, 1 for an
+ * encoding, width or count the matrix-core path does not take, or the reserved
+ * mode. */
+int nfn_mi355_k_quant_gemm_tile_rows_v1(
+    uint32_t encoding,
+    int64_t rows,
+    int64_t input_dim,
+    const int64_t* output_dims,
+    int64_t operation_count,
+    int mode,
+    int* tile_rows);
 
 /* The same for 1..4 projections of one input (Q/K/V, gate/up), the way the
  * small-batch entry points group them: the activations are converted once and

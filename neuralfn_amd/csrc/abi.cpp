@@ -864,6 +864,20 @@ int nfn_mi355_k_quant_gemm_plan_v1(std::uint32_t encoding, std::int64_t rows, st
     return 0;
 }
 
+int nfn_mi355_k_quant_gemm_tile_rows_v1(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
+                                        const std::int64_t* output_dims, std::int64_t operation_count, int mode,
+                                        int* tile_rows) {
+    if (tile_rows == nullptr || output_dims == nullptr || operation_count < 1 || operation_count > 4 || rows <= 0 ||
+        input_dim <= 0 || mode != NFN_MI355_GEMM_F16 || !gemm_f16_supports(encoding, input_dim)) {
+        return kInvalid;
+    }
+    for (std::int64_t i = 0; i < operation_count; ++i) {
+        if (output_dims[i] <= 0) return kInvalid;
+    }
+    *tile_rows = gemm_f16_tile_rows(encoding, rows, input_dim, output_dims, static_cast<int>(operation_count));
+    return 0;
+}
+
 int nfn_mi355_k_quant_gemm_float32_v1(const Descriptor* descriptor, const float* input,
                                       float* output, std::int64_t rows, void* workspace,
                                       std::int64_t workspace_nbytes, int mode,

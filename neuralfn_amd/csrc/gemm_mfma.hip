@@ -1315,7 +1315,9 @@ constexpr TileCost kTileCosts<kEncQ8_0>[3] = {{512, {6.8, 0, 0}}, {256, {4.1, 8.
 // many as fit; the last one may leave places or whole units empty, and a chip at work in part runs
 // at a higher clock, down to three quarters of the time.  The figures are fitted to 160 to 3,000
 // rows into Q, K, V and gate, O, gate and up, and down at one to four shares: the times are met to
-// 5 %, and the height chosen costs 0.2 % more than the best one on average.
+// 5 %, and the height chosen costs 0.2 % more than the best one on average.  At widths they are not
+// fitted to (2,048 to 13,824 columns into 4,096 to 28,672 outputs, 48 to 4,096 rows, 448 calls) 0.2 % too,
+// 13 at most: 1,537 rows of 13,824 -> 5,120 of Q4_K run on 128 rows in 349 us, and would on 512 in 310.
 // Eight waves on 512 rows decode a weight for twice the rows, and Q6_K's registers then allow two
 // waves a SIMD instead of one: 2,048 rows of 16,384 -> 6,656 461 -> 420 us (Q4_K), 475 -> 430 (Q5_K),
 // 542 -> 434 (Q6_K), 540 -> 439 (Q8_0); 4,000 rows of gate and up 1,525 -> 1,479, 1,593 -> 1,500,
@@ -1440,6 +1442,22 @@ void gemm_f16_plan(std::uint32_t encoding, std::int64_t rows, std::int64_t input
     const Plan chosen = plan(encoding, rows, output_dim, input_dim);
     *tile_rows = chosen.tile_rows;
     *k_shares = chosen.shares;
+}
+
+int gemm_f16_tile_rows(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
+                       const std::int64_t* output_dims, int count) {
+    if (rows <= kLowRows) return kLowRows;
+    GemmGroup group{};
+    for (int i = 0; i < count; ++i) {
+        group.output_dim[i] = output_dims[i];
+        group.shares[i] = plan(encoding, rows, output_dims[i], input_dim).shares;
+    }
+    switch (encoding) {
+        case kEncQ4K: return tile_height<kEncQ4K>(group, count, rows, input_dim);
+        case kEncQ5K: return tile_height<kEncQ5K>(group, count, rows, input_dim);
+        case kEncQ6K: return tile_height<kEncQ6K>(group, count, rows, input_dim);
+        default: return tile_height<kEncQ8_0>(group, count, rows, input_dim);
+    }
 }
 
 bool gemm_f16_supports(std::uint32_t encoding, std::int64_t input_dim) {

@@ -207,6 +207,8 @@ SIGNATURES = {
     "nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1": (_I64, [_I64, _I64, _P, _I64, ctypes.c_int]),
     "nfn_mi355_k_quant_gemm_plan_v1": (
         ctypes.c_int, [ctypes.c_uint32, _I64, _I64, _I64, ctypes.c_int, _P, _P]),
+    "nfn_mi355_k_quant_gemm_tile_rows_v1": (
+        ctypes.c_int, [ctypes.c_uint32, _I64, _I64, _P, _I64, ctypes.c_int, _P]),
     "nfn_mi355_k_quant_gemm_float32_v1": (
         ctypes.c_int, [_DESC, _P, _P, _I64, _P, _I64, ctypes.c_int, _P]),
     "nfn_mi355_k_quant_gemm_multi_float32_v1": (
@@ -603,12 +605,23 @@ def gemm(weight: PackedWeight, x, mode: int = GEMM_F16, workspace=None, out=None
 
 
 def gemm_plan(encoding: int, rows: int, input_dim: int, output_dim: int, mode: int = GEMM_F16):
-    """nfn_mi355_k_quant_gemm_plan_v1: (rows per workgroup tile, K shares) of a launch."""
+    """nfn_mi355_k_quant_gemm_plan_v1: (rows of the workgroup tile that K is cut for, K shares)."""
     tile_rows, shares = ctypes.c_int(0), ctypes.c_int(0)
     check(load().nfn_mi355_k_quant_gemm_plan_v1(
         encoding, rows, input_dim, output_dim, mode, ctypes.addressof(tile_rows),
         ctypes.addressof(shares)), "k_quant_gemm_plan")
     return tile_rows.value, shares.value
+
+
+def gemm_tile_rows(encoding: int, rows: int, input_dim: int, output_dims: Sequence[int], mode: int = GEMM_F16):
+    """nfn_mi355_k_quant_gemm_tile_rows_v1: rows per workgroup tile of the launch that runs projections of
+    these widths together."""
+    tile_rows = ctypes.c_int(0)
+    widths = (ctypes.c_int64 * len(output_dims))(*output_dims)
+    check(load().nfn_mi355_k_quant_gemm_tile_rows_v1(
+        encoding, rows, input_dim, ctypes.addressof(widths), len(output_dims), mode,
+        ctypes.addressof(tile_rows)), "k_quant_gemm_tile_rows")
+    return tile_rows.value
 
 
 def gemm_multi(weights: Sequence[PackedWeight], x, mode: int = GEMM_F16, workspace=None,

@@ -1789,6 +1789,7 @@ def test_prefill_gemm_tall_tiles(cuda, oracle, encoding):
     # 256-row tile variant (smaller problems run the 128-row one); K of two
     # blocks (even count).  The oracle checks a spread of rows.
     rows, out_dim, in_dim = 512, 16384, 512
+    assert tile_ops.gemm_tile_rows(encoding, rows, in_dim, [out_dim]) == 256
     packed = random_packed(encoding, out_dim, in_dim, 43)
     x = kquant.synthetic_activations(74, rows, in_dim)
     weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
@@ -1798,14 +1799,15 @@ def test_prefill_gemm_tall_tiles(cuda, oracle, encoding):
     assert normalised_error(y[picked], expected) <= TOLERANCE
 
 
-@pytest.mark.parametrize("rows,tiles,in_dim", [(600, 0.5, 256), (1000, 0.5, 512), (1200, 0.33, 768), (1537, 1.0, 1280)])
+@pytest.mark.parametrize("rows,tiles,in_dim", [(1624, 0.25, 256), (1000, 0.5, 512), (1712, 0.25, 768), (1537, 0.25, 1280)])
 @pytest.mark.parametrize("encoding", ALL_PACKED)
 def test_prefill_gemm_eight_waves_a_tile(cuda, oracle, encoding, rows, tiles, in_dim):
-    """Tiles of 512 rows, taken where they fill the chip: a last tile of 88, 488, 176 and one row (waves
+    """Tiles of 512 rows, one on every compute unit: a last tile of 88, 488, 176 and one row (waves
     past the rows that the fp16 copy is padded to), a last column tile of 125, one to five blocks of
     K.  The oracle checks rows at the edges of waves and tiles."""
     units = torch_().cuda.get_device_properties(0).multi_processor_count
     out_dim = int(tiles * units) * 128 - 3
+    assert tile_ops.gemm_tile_rows(encoding, rows, in_dim, [out_dim]) == 512
     packed = random_packed(encoding, 256, in_dim, 46).reshape(256, -1)
     chosen = np.random.default_rng(47).integers(0, 256, out_dim)
     weight = tile_ops.PackedWeight(encoding, out_dim, in_dim, torch_().from_numpy(packed).to(cuda).index_select(
@@ -1835,6 +1837,21 @@ def test_prefill_gemm_plans():
     # A narrow projection (the K and V projections of the workload): small tiles, short shares.
     assert tile_ops.gemm_plan(kquant.Q4_K, 1024, 6656, 256) == (128, 4)
     assert tile_ops.gemm_plan(kquant.Q6_K, 2048, 6656, 256) == (128, 4)
+
+
+def test_prefill_gemm_tile_rows(cuda):
+    # Host logic only.  Low tiles where high ones would leave units idle, by the widths of the whole launch.
+    for encoding in ALL_PACKED:
+        assert tile_ops.gemm_tile_rows(encoding, 32, 6656, [4096]) == 32
+        assert tile_ops.gemm_tile_rows(encoding, 128, 6656, [4096]) == 128
+        assert tile_ops.gemm_tile_rows(encoding, 4096, 6656, [16384, 16384]) == 512
+    assert tile_ops.gemm_tile_rows(kquant.Q4_K, 160, 6656, [16384, 16384]) == 256
+    assert tile_ops.gemm_tile_rows(kquant.Q4_K, 160, 4096, [6656]) == 128
+    call, widths, out = tile_ops.load().nfn_mi355_k_quant_gemm_tile_rows_v1, (ctypes.c_int64 * 2)(128, 0), ctypes.c_int(7)
+    for encoding, count, in_dim in ((kquant.Q4_K, 2, 256), (kquant.Q4_K, 0, 256), (kquant.Q4_K, 5, 256),
+                                    (kquant.Q4_K, 1, 128), (kquant.BF16, 1, 256)):
+        assert call(encoding, 64, in_dim, ctypes.addressof(widths), count, tile_ops.GEMM_F16, ctypes.addressof(out)) == 1
+    assert call(kquant.Q4_K, 64, 256, None, 1, tile_ops.GEMM_F16, ctypes.addressof(out)) == 1 and out.value == 7
 
 
 def test_prefill_gemm_workspace_of_a_longer_chunk(cuda):
