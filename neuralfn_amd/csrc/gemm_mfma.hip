@@ -1319,9 +1319,9 @@ constexpr TileCost kTileCosts<kEncQ8_0>[3] = {{512, {6.8, 0, 0}}, {256, {4.1, 8.
 // fitted to (2,048 to 13,824 columns into 4,096 to 28,672 outputs, 48 to 4,096 rows, 448 calls) 0.2 % too,
 // 13 at most: 1,537 rows of 13,824 -> 5,120 of Q4_K run on 128 rows in 349 us, and would on 512 in 310.
 // Eight waves on 512 rows decode a weight for twice the rows, and Q6_K's registers then allow two
-// waves a SIMD instead of one: 2,048 rows of 16,384 -> 6,656 461 -> 420 us (Q4_K), 475 -> 430 (Q5_K),
-// 542 -> 434 (Q6_K), 540 -> 439 (Q8_0); 4,000 rows of gate and up 1,525 -> 1,479, 1,593 -> 1,500,
-// 1,909 -> 1,519, 1,747 -> 1,540.  Lower tiles where 512 rows leave too many units idle: 160 rows of gate
+// waves a SIMD instead of one: 2,048 rows of 16,384 -> 6,656 474 -> 441 us (Q4_K), 486 -> 446 (Q5_K),
+// 561 -> 466 (Q6_K), 548 -> 465 (Q8_0); 4,096 rows of gate and up 1,524 -> 1,467, 1,588 -> 1,501,
+// 1,837 -> 1,517, 1,743 -> 1,527 (one chip, runs in turn; faster ones take a tenth less on either side).  Lower tiles where 512 rows leave too many units idle: 160 rows of gate
 // and up 108 us in tiles of 256 rows (128: 124, 512: 163), of O 47 in tiles of 128 (58, 85).
 template <std::uint32_t ENC>
 int tile_height(const GemmGroup& group, int count, std::int64_t rows, std::int64_t input_dim) {

@@ -389,9 +389,10 @@ struct PassLoads {
 // W: waves per workgroup (the activation images are shared by the workgroup,
 // so more tokens per pass want more waves behind each image).  FEWER: the launch has
 // fewer than W.
-// At multiples of 16 KB: the instruction cache keeps a layer's kernels from one layer to the next,
-// and this one shares its sets with others where it lies.  The same instructions, a one-token layer's down
-// projection (16,384 -> 6,656): 21.9 us at 6 to 8 and 13 to 16 KB past a multiple of 16, 21.45 at 0 to 5.
+// At multiples of 16 KB: the same instructions take longer at other places, a one-token layer's down
+// projection (16,384 -> 6,656) 21.9 us at 6 to 8 and 13 to 16 KB past a multiple of 16, 21.45 at 0 to 5
+// (deep into a context; a short one 21.65 and 21.75).  Presumably the instruction cache, which keeps a layer's
+// kernels from one layer to the next; a counter run, whose launches start cold, shows the same misses.
 template <int T, int P, bool ARGMAX, int W, bool FEWER>
 __global__ __attribute__((aligned(16384))) __launch_bounds__(W * kWave) void gemv_q6_stream_kernel(
     const float* __restrict__ first, const float* __restrict__ second, std::int64_t input_dim,

@@ -33,9 +33,11 @@
 // loads of the next tile's first block in flight under the last block of the one before.
 // One pass over the weights for up to 16 tokens.
 //
-// What bounds it: a wave issues an instruction every 5 to 8 cycles and two waves fit a SIMD, so the
-// vector ALU is busy a third of the time and memory is asked in bursts (gate and up of seven
-// tokens, Q4_K: only the weights' loads 23.4 us, with the operands' 28.5, everything 35).  Up to
+// What bounds it: more than eight tokens the vector ALU (the replayed tail).  Up to eight no unit is full:
+// a wave issues an instruction every 5 to 8 cycles and two waves fit a SIMD.  Gate and up of seven tokens,
+// Q4_K, share of the cycles: vector ALU 55 %, line look-ups 39, LDS 25, matrix cores 11, and waves wait
+// 31 % of theirs; down, Q6_K, 46, 35, 43, 12 and 30; O, 208 tiles of sixteen blocks, vector ALU 33.  (Only the
+// weights' loads take 23.4 us of gate and up's, with the operands' 28.5, everything 32 to 35.)  Up to
 // eight tokens therefore: two or four scale groups to an operand fragment (half or a quarter of
 // the operand bytes, registers for a second block of packed bytes in flight), the minimums'
 // sums from the records instead of a second pair of products, products issued around the tail
@@ -145,8 +147,8 @@ struct __attribute__((packed, aligned(2))) RowsHalfPiece {
 typedef int v2i __attribute__((ext_vector_type(2)));
 
 // The packed bytes of 32 rows x one block as a wave loads them, coalesced: one set of
-// registers (they go to the LDS tile as soon as they arrive, and the next block's request
-// reuses them).
+// registers, up to eight tokens two (they go to the LDS tile as soon as they arrive, and the request of
+// the next block, or the one after it, reuses them).
 template <std::uint32_t ENC>
 struct RowsPacked {
     v4u chunk[RowsFormat<ENC>::kLoads];
@@ -216,7 +218,8 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
     constexpr int kTokens = 2 * S;
     constexpr int kGroups = rows_groups(S);
     constexpr bool kDeep = S <= 4;  // registers for two blocks of packed bytes in flight
-    // (two buffers of class sums: the workgroup's waves meet once per tile)
+    // class sums of so many tiles: two where the workgroup's waves meet at a barrier once per tile, four
+    // where they wait for each other's counts (up to eight tokens)
     constexpr int kOwnClasses = SPLIT ? kClasses / 2 : kClasses;
     constexpr int kTilesHeld = kDeep ? 4 : 2;
     __shared__ float class_sums[kTilesHeld][kOwnClasses][kTokens][kRowsTile];
@@ -326,8 +329,10 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
     // A wave's steps of a tile: the blocks of class r, then those of class 15 - r (SPLIT: of the one
     // class r or 8 + r), r = wave for the first tile.  Rows whose blocks are no multiple of 16 give
     // some r a block more than others (26 blocks: r = 6 and 7 have four, the others three), so r
-    // moves on by two with every tile and all waves get the same over four tiles (rows of fewer
-    // than 16 blocks leave some r nothing and stay).
+    // moves on by two with every tile and a wave has had every r of its parity after four tiles: even
+    // shares where the extra blocks fall on both alike (26 blocks), a block more in four tiles for
+    // one half of the waves where there is one (17 blocks: r = 0).  Rows of fewer than 16 blocks leave
+    // some r nothing and stay.
     const int role_step = kDeep && blocks >= kClasses ? 2 : 0;
     struct Role {
         int class0, class1, count0, total;
@@ -592,8 +597,8 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
                     upper[w] = static_cast<int>(up);
                 }
             };
-            // the float tail of pair p for the token slots first..last-1 (`sums`: of the products
-            // with the minimums, for more than eight tokens)
+            // the float tail of pair p for the token slots first..last-1 (min_dots: the products with
+            // the minimums, for more than eight tokens; fewer take the code sums of the records)
             const auto tail = [&](int p, const v16i& dots_a, const v16i& dots_b, const v16i& min_dots, int first,
                                   int last) {
                 const std::uint32_t sc_word = p < 2 ? sc_lo : sc_hi;

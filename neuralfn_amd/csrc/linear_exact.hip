@@ -48,7 +48,7 @@
 // once instead of tile by tile: no difference.  Requests two steps ahead instead of one, and the matrix
 // instructions of a step before its other work instead of between it: neither.)  The 64 x 128 form of Q6_K
 // keeps six registers that do not change in its loop in scratch (28 bytes a lane), read outside of it; the
-// 32 x 32 form of Q6_K for 17 rows and more four (32 bytes); the others none.
+// 32 x 32 form of Q6_K for 17 rows and more five (32 bytes); the others none.
 // Measured at 4,096 -> 6,656, against the vector kernel (16 rows) and the float matrix instruction (200,
 // 512 rows) before: Q4_K 134 -> 15 us at 16 rows, 203 -> 62 at 200, 311 -> 121 at 512; Q8_0 368 -> 23,
 // 180 -> 55, 279 -> 108; F32 406 -> 31, 172 -> 114, 271 -> 217.
