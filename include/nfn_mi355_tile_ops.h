@@ -902,7 +902,9 @@ enum {
                                int8 MFMA; refused (workspace query returns 0) */
 };
 /* A workspace that serves a call of `rows` rows and any of fewer (which may
- * need more: a short chunk splits K over more workgroups). */
+ * need more: a short chunk splits K over more workgroups).  A call takes any
+ * workspace that holds what its plan (the query below) needs; with this size it
+ * may cut K further where that is faster, and then rounds differently. */
 int64_t nfn_mi355_k_quant_gemm_workspace_bytes_v1(
     int64_t rows, int64_t input_dim, int64_t output_dim, int mode);
 int nfn_mi355_k_quant_gemm_float32_v1(
@@ -921,7 +923,8 @@ int nfn_mi355_k_quant_gemm_float32_v1(
  * for up to 32 rows; which tiles the launch takes says the query below),
  * *k_shares = workgroups that share the K range of a tile
  * (1 = unsplit; with more, each writes a partial output into the workspace and
- * a second launch adds them in share order).  0 on success, 1 for an encoding
+ * a second launch adds them in share order; a call with more workspace than this
+ * needs may take more, see above).  0 on success, 1 for an encoding
  * or width the matrix-core path does not take, or the reserved mode. */
 int nfn_mi355_k_quant_gemm_plan_v1(
     uint32_t encoding,
@@ -954,7 +957,7 @@ int nfn_mi355_k_quant_gemm_tile_rows_v1(
  * every projection runs from that copy.  All descriptors share input_dim (a
  * multiple of 256) and are Q4_K, Q5_K, Q6_K or Q8_0.  The workspace is the
  * largest of the single-projection sizes (the query above with each
- * output_dim); with the size that the query below gives, the projections of an
+ * output_dim; a smaller one that holds each plan's need is taken); with the size that the query below gives, the projections of an
  * encoding run in one launch where they all split K.  Results are those of the
  * single-projection call, bit for bit, with either. */
 int64_t nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1(

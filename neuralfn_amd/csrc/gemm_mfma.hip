@@ -44,6 +44,8 @@
 #include "f16_decode.hpp"
 #include "gemm_mfma.hpp"
 
+#include <algorithm>
+
 namespace nfn {
 
 namespace {
@@ -57,7 +59,9 @@ constexpr int kThreads = 256;
 constexpr int kMaxProjections = 4;  // of one call
 constexpr int kLowRows = 32;    // rows up to which every wave takes all of them
 constexpr int kLowShares = 8;   // K shares of theirs at most
-constexpr int kMaxShares = 4;   // K shares of a split launch at most
+constexpr int kMaxShares = 4;   // K shares of a split launch at most that plan() gives (shares_with_room: eight)
+constexpr int kLeastCutTiles = 16;  // column tiles and
+constexpr int kMostCutRows = 1024;  // rows up to which shares_with_room() looks for more
 constexpr int kRowBytes = 144;  // 64 fp16 + 16 bytes of padding
 constexpr int kStageBytes = kBN * kRowBytes;
 constexpr int kFragmentBytes = 1024;  // 32 rows x 16 K values of fp16 in operand order
@@ -1227,6 +1231,7 @@ __global__ __launch_bounds__(256) void sum_shares_kernel(ShareSums sums) {
 // or more, at most eight, until there are two workgroups a unit.  (Two 32-row blocks a wave, for up
 // to 64 rows: 128-row tiles are as fast or faster where the tiles are many, 64 rows of gate and up
 // 81 us (Q4_K) and 203 (Q8_0) against 78 and 93 at 65.)
+// (A call of more than 32 rows with room for it may cut further: shares_with_room.)
 // (The heights here are those that the shares are cut for.  The launch takes the one that costs
 // least with these shares, see tile_height; a sum does not depend on it.)
 struct Plan {
@@ -1323,18 +1328,24 @@ constexpr TileCost kTileCosts<kEncQ8_0>[3] = {{512, {6.8, 0, 0}}, {256, {4.1, 8.
 // 561 -> 466 (Q6_K), 548 -> 465 (Q8_0); 4,096 rows of gate and up 1,524 -> 1,467, 1,588 -> 1,501,
 // 1,837 -> 1,517, 1,743 -> 1,527 (one chip, runs in turn; faster ones take a tenth less on either side).  Lower tiles where 512 rows leave too many units idle: 160 rows of gate
 // and up 108 us in tiles of 256 rows (128: 124, 512: 163), of O 47 in tiles of 128 (58, 85).
-template <std::uint32_t ENC>
-int tile_height(const GemmGroup& group, int count, std::int64_t rows, std::int64_t input_dim) {
+//
+// ... and what the launch costs at that height, in us: `blocks` of 256 columns that a workgroup walks on
+// average, `extra` blocks' time for its start and end.
+struct TileChoice {
+    int rows;
+    double cost;
+};
+TileChoice cheapest_tile(const TileCost (&tiles_of)[3], const std::int64_t* output_dims, const int* shares, int count,
+                         std::int64_t rows, std::int64_t input_dim, double extra) {
     const std::int64_t units = compute_units();
-    int best_rows = 0;
-    double best = 0;
-    for (const TileCost& tile : kTileCosts<ENC>) {
+    TileChoice best{0, 0};
+    for (const TileCost& tile : tiles_of) {
         const std::int64_t m_tiles = (rows + tile.rows - 1) / tile.rows;
         std::int64_t workgroups = 0, tiles = 0;
         for (int i = 0; i < count; ++i) {
-            const std::int64_t here = m_tiles * ((group.output_dim[i] + kBN - 1) / kBN);
+            const std::int64_t here = m_tiles * ((output_dims[i] + kBN - 1) / kBN);
             tiles += here;
-            workgroups += here * group.shares[i];
+            workgroups += here * shares[i];
         }
         const int places = tile.block[2] > 0 ? 3 : tile.block[1] > 0 ? 2 : 1;
         const std::int64_t full = workgroups / (units * places);
@@ -1345,15 +1356,59 @@ int tile_height(const GemmGroup& group, int count, std::int64_t rows, std::int64
             const double clock = 1.0 + 0.35 * (at_work - 1.0);
             rounds += tile.block[last - 1] * (clock > 0.75 ? clock : 0.75);
         }
-        // (blocks of 256 columns that a workgroup walks, on average, and a fifth for its start and end)
         const double blocks = static_cast<double>(input_dim >> 8) * static_cast<double>(tiles) / static_cast<double>(workgroups);
-        const double cost = (blocks + 0.2) * rounds;
-        if (best_rows == 0 || cost < best) {
-            best_rows = tile.rows;
-            best = cost;
+        const double cost = (blocks + extra) * rounds;
+        if (best.rows == 0 || cost < best.cost) best = TileChoice{tile.rows, cost};
+    }
+    return best;
+}
+
+template <std::uint32_t ENC>
+int tile_height(const GemmGroup& group, int count, std::int64_t rows, std::int64_t input_dim) {
+    return cheapest_tile(kTileCosts<ENC>, group.output_dim, group.shares, count, rows, input_dim, 0.2).rows;
+}
+
+// K shares beyond those of plan(), where the workspace has room for them (gemm_f16_workspace_bytes asks for
+// it): plan() leaves a share twelve blocks, which leaves most of the chip idle at a K of a few thousand
+// columns into few tiles (35 rows of 4,096 -> 5,376: 42 workgroups on 256 units).  By the tiles' costs and
+// the sums' (a launch, 3 us, and 0.4 us a MB of partial outputs), shares are added if they save a
+// fifteenth of the call by itself and cost no more where two to two and a half such projections share a
+// launch: a projection has the same shares, and with them the same bits, whatever runs beside it.
+// Without the second condition 859 single calls (48 to 1,400 rows, 2,048 to 16,384 columns into 256 to
+// 16,384 outputs) take 14 % less than plan()'s on average, but Q, K, V and gate of 2,304 columns and 218
+// rows 33 -> 45 us.  With it, of 45 calls of 33 to 1,024 rows five gain (35 rows of 4,096 -> 5,376, Q4_K, 43.4 ->
+// 23.4 us; 55 of 11,776 -> 5,376, Q8_0, 54.8 -> 39.3; 33 of 16,640 -> 2,048, Q6_K, 75.7 -> 61.4) and none
+// loses.  Projections of fewer than 2,048 outputs (K and V) keep plan()'s: beside others their shares are
+// not what a launch waits for.  One table of costs (Q4_K's) for all encodings, so that the workspace
+// query, which knows none, need not ask for four.
+int shares_with_room(const Plan& least, std::int64_t rows, std::int64_t output_dim, std::int64_t input_dim) {
+    const std::int64_t n_tiles = (output_dim + kBN - 1) / kBN;
+    if (rows <= kLowRows || rows > kMostCutRows || n_tiles < kLeastCutTiles || (rows + 255) / 256 * n_tiles >= compute_units()) return least.shares;
+    // (the same for every count up to the next multiple of 128: what gemm_f16_workspace_bytes relies on)
+    const std::int64_t counted = (rows + 127) / 128 * 128;
+    const auto cost = [&](int shares, int quarters) {
+        const std::int64_t outputs = quarters * n_tiles * kBN / 4;
+        const double sums = shares == 1 ? 0.0 : 3.0 + 1.6e-6 * static_cast<double>((shares + 1) * counted * outputs);
+        return cheapest_tile(kTileCosts<kEncQ4K>, &outputs, &shares, 1, counted, input_dim, 0.0).cost + sums;
+    };
+    constexpr int kBeside[4] = {4, 8, 9, 10};  // quarters of the outputs: alone, with another, ...
+    double least_cost[4];
+    for (int i = 0; i < 4; ++i) least_cost[i] = cost(least.shares, kBeside[i]);
+    int best = least.shares;
+    double best_saved = 1.0;
+    for (const int shares : {2, 3, 4, 6, 8}) {
+        if (shares <= least.shares || 2 * shares > (input_dim >> 8)) continue;
+        double saved = 1.0;
+        for (int i = 0; i < 4; ++i) {
+            const double here = cost(shares, kBeside[i]) / least_cost[i];
+            saved *= here < (i == 0 ? 0.94 : 1.0) ? here : 2.0;
+        }
+        if (saved < best_saved) {
+            best = shares;
+            best_saved = saved;
         }
     }
-    return best_rows;
+    return best;
 }
 
 // One launch for `count` projections of one encoding and, if any of them splits K, one for the sums.
@@ -1418,8 +1473,19 @@ std::int64_t largest_up_to(std::int64_t rows, std::int64_t narrowest, F&& needed
 }
 
 // floats of a projection's shares behind the first
-std::int64_t partial_floats(const Plan& chosen, std::int64_t rows, std::int64_t output_dim) {
-    return (chosen.shares - 1) * rows * output_dim;
+std::int64_t partial_floats(int shares, std::int64_t rows, std::int64_t output_dim) {
+    return (shares - 1) * rows * output_dim;
+}
+
+// ... of the shares that a call with room for them takes, whatever the encoding (plan() gives Q4_K the most,
+// and with as many or more the other encodings take none that it does not)
+std::int64_t most_partial_floats(std::int64_t rows, std::int64_t output_dim, std::int64_t input_dim) {
+    std::int64_t most = 0;
+    for (const std::uint32_t encoding : {kEncQ4K, kEncQ6K}) {
+        const int shares = shares_with_room(plan(encoding, rows, output_dim, input_dim), rows, output_dim, input_dim);
+        most = std::max(most, partial_floats(shares, rows, output_dim));
+    }
+    return most;
 }
 
 }  // namespace
@@ -1433,7 +1499,8 @@ std::int64_t gemm_f16_required_bytes(std::int64_t rows, std::int64_t input_dim, 
 
 std::int64_t gemm_f16_workspace_bytes(std::int64_t rows, std::int64_t input_dim, std::int64_t output_dim) {
     return largest_up_to(rows, output_dim, [&](std::int64_t count) {
-        return gemm_f16_required_bytes(count, input_dim, output_dim);
+        const std::int64_t required = gemm_f16_required_bytes(count, input_dim, output_dim);
+        return std::max(required, activation_bytes(count, input_dim) + 4 * most_partial_floats(count, output_dim, input_dim) + 256);
     });
 }
 
@@ -1495,9 +1562,11 @@ std::int64_t gemm_f16_multi_workspace_bytes(std::int64_t rows, std::int64_t inpu
     return largest_up_to(rows, narrowest, [&](std::int64_t chunk) {
         std::int64_t largest = 0, floats = 0;
         for (int i = 0; i < count; ++i) {
-            const std::int64_t single = gemm_f16_required_bytes(chunk, input_dim, output_dims[i]);
+            std::int64_t single = gemm_f16_required_bytes(chunk, input_dim, output_dims[i]);
+            const std::int64_t here = most_partial_floats(chunk, output_dims[i], input_dim);
+            single = std::max(single, activation_bytes(chunk, input_dim) + 4 * here + 256);
             if (single > largest) largest = single;
-            floats += partial_floats(plan(kEncQ4K, chunk, output_dims[i], input_dim), chunk, output_dims[i]);
+            floats += here;
         }
         const std::int64_t together = activation_bytes(chunk, input_dim) + 4 * floats + 256;
         return together > largest ? together : largest;
@@ -1521,8 +1590,13 @@ void launch_gemm_f16(const Descriptor* descriptors, int count, const float* inpu
         std::int64_t used = 0;
         for (int i = start; i < count; ++i) {
             if (done[i] || descriptors[i].encoding != descriptors[start].encoding) continue;
-            const Plan chosen = plan(descriptors[i].encoding, rows, descriptors[i].output_dim, input_dim);
-            const std::int64_t floats = partial_floats(chosen, rows, descriptors[i].output_dim);
+            const Plan least = plan(descriptors[i].encoding, rows, descriptors[i].output_dim, input_dim);
+            int shares = shares_with_room(least, rows, descriptors[i].output_dim, input_dim);
+            std::int64_t floats = partial_floats(shares, rows, descriptors[i].output_dim);
+            if (floats > room) {  // a workspace of the plan's size
+                shares = least.shares;
+                floats = partial_floats(shares, rows, descriptors[i].output_dim);
+            }
             if (i != start && used + floats > room) continue;
             done[i] = true;
             group.weights[members] = descriptors[i].data;
@@ -1530,7 +1604,7 @@ void launch_gemm_f16(const Descriptor* descriptors, int count, const float* inpu
             group.output[members] = outputs[i];
             group.partials[members] = partials + used;
             group.output_dim[members] = descriptors[i].output_dim;
-            group.shares[members] = chosen.shares;
+            group.shares[members] = shares;
             used += floats;
             ++members;
         }

@@ -1875,6 +1875,35 @@ def test_prefill_gemm_workspace_of_a_longer_chunk(cuda):
             tile_ops.gemm(weight, x, workspace=large[:needed - 1])
 
 
+@pytest.mark.parametrize("rows,in_dim,out_dim", [(33, 4096, 5373), (128, 2304, 2049), (35, 11776, 5376), (97, 1024, 6144)])
+@pytest.mark.parametrize("encoding", ALL_PACKED)
+def test_prefill_gemm_cut_beyond_the_plan(cuda, oracle, encoding, rows, in_dim, out_dim):
+    """Few tiles and a K that the plan leaves whole or in long shares: with the workspace of the query the
+    call cuts further (shares of four, three and unequal lengths, a last column tile of one), with the
+    plan's it does not; both keep the bound, and projections beside each other the single call's bits."""
+    lib = tile_ops.load()
+    _, shares = tile_ops.gemm_plan(encoding, rows, in_dim, out_dim)
+    least = (256 * (in_dim * 2 + 8) + 255) // 256 * 256 + (shares * rows * out_dim * 4 if shares > 1 else 0) + 256
+    asked = lib.nfn_mi355_k_quant_gemm_workspace_bytes_v1(rows, in_dim, out_dim, tile_ops.GEMM_F16)
+    assert asked >= least
+    packed = random_packed(encoding, 256, in_dim, 46).reshape(256, -1)
+    chosen = np.random.default_rng(48).integers(0, 256, out_dim)
+    weight = tile_ops.PackedWeight(encoding, out_dim, in_dim, torch_().from_numpy(packed).to(cuda).index_select(
+        0, torch_().from_numpy(chosen).to(cuda)).reshape(-1))
+    x = kquant.synthetic_activations(77, rows, in_dim)
+    expected = oracle.linear(encoding, packed.reshape(-1), 256, in_dim, x)[:, chosen]
+    device_x = to_device(x, cuda)
+    for nbytes in (asked, least):
+        workspace = torch_().full((nbytes + 4096,), 0x5a, dtype=torch_().uint8, device=cuda)
+        y = tile_ops.gemm(weight, device_x, workspace=workspace[:nbytes])
+        assert normalised_error(y.cpu().numpy(), expected) <= TOLERANCE
+        assert bool((workspace[nbytes:] == 0x5a).all())
+    with pytest.raises(tile_ops.TileOpsError):
+        tile_ops.gemm(weight, device_x, workspace=workspace[:least - 1])
+    for y in tile_ops.gemm_multi([weight, weight], device_x):
+        assert_bits_equal(y, tile_ops.gemm(weight, device_x), kquant.NAMES[encoding])
+
+
 @pytest.mark.parametrize("rows,in_dim,plan", [
     (96, 1536, (128, 1)),    # six blocks: one share
     (96, 3072, (128, 2)),    # twelve blocks -> two shares of six
