@@ -34,9 +34,7 @@ std::int64_t first_half_rows(std::uint32_t encoding) {
     return encoding == kEncQ6K ? kFirstHalfRowsQ6 : kFirstHalfRows;
 }
 // rows from which the verifier family's Q4_K / Q5_K projections run on the int8 matrix cores
-// (one pass over the weights behind a quantizer launch; below: the dot kernel's token passes,
-// which are faster up to three rows: 9.0 / 12.4 / 13.9 us per launch of the attention
-// projections at 2 / 3 / 4 rows against 12.8 for the matrix-core kernel at any of them)
+// whatever the shape (one pass over the weights behind a quantizer launch; below: rows_kernel_pays)
 constexpr std::int64_t kFirstVerifierMatrixRows = 4;
 // Private activation records of the small-batch path, 576 bytes per token and
 // 256 values (two int8 planes of a 16-bit fixed-point code, group sums, scale,
@@ -51,14 +49,15 @@ std::int64_t record_bytes(std::int64_t rows, std::int64_t input_dim) {
 
 // Records, and behind them, from the row count on at which the verifier family runs on the
 // matrix cores, the same codes in matrix-operand order (gemv_rows.hpp).
-std::int64_t small_batch_workspace_bytes(std::int64_t rows, std::int64_t input_dim) {
+// `image`: with the operand copy from two rows on, which two and three rows use where there is room for it.
+std::int64_t small_batch_workspace_bytes(std::int64_t rows, std::int64_t input_dim, bool image = false) {
     if (rows < 1 || rows > kMaxSmallRows || input_dim <= 0 || input_dim % 128 != 0) return 0;
     const std::int64_t groups = (input_dim + 31) / 32;
     if (groups > std::numeric_limits<std::int64_t>::max() / (2 * kActivationGroupBytes * kMaxSmallRows)) {
         return 0;
     }
     std::int64_t raw = record_bytes(rows, input_dim);
-    if (rows >= kFirstVerifierMatrixRows && input_dim % 256 == 0) {
+    if ((rows >= kFirstVerifierMatrixRows || (image && rows >= 2)) && input_dim % 256 == 0) {
         raw += gemv_rows_image_bytes(input_dim);
     }
     return (raw + 255) & ~std::int64_t(255);
@@ -79,6 +78,34 @@ Projection make_projection(const Descriptor& descriptor, float* output) {
     op.encoding = descriptor.encoding;
     op.first_tile = 0;
     return op;
+}
+
+// Whether a projection runs on the exact verifier's matrix-core kernel behind its quantizer launch
+// (gemv_rows.hip) where that is a question of time: the verifier family takes it from four rows on, and the
+// one-row arithmetic of two and three rows has the same bits on either kernel.  Two launches that
+// read the activations once, against one in which every workgroup makes their codes (and a prologue's
+// functions) for itself; K: input_dim.  Times of the call before -> with it, us, one box, weights from memory.
+//   Three rows of the verifier family: K-Quants always (2,048 -> 6,144 of Q4_K 9.3 -> 7.0, 7,936 -> 39,936 76 -> 43,
+//     Q6_K 132 -> 68, SwiGLU 16,384 -> 6,656 of Q4_K 37 -> 21); Q8_0 gains from long rows or many outputs
+//     (16,384 -> 6,656 34 -> 30, 4,096 -> 32,768 35 -> 32; 4,096 -> 6,656 would lose, 12.4 -> 13.1).
+//   Two rows: K above 12,288 (SwiGLU 18,432 -> 2,304 21 -> 14, 16,384 -> 6,656 of Q6_K 38 -> 33) or, Q4_K and Q5_K, many
+//     outputs (4,096 -> 16,384 twice 25 -> 22); 6,656 -> 8,704 would lose, 13.4 -> 15.2.
+//   Three and four rows of the other family, Q4_K and Q5_K: behind a prologue (SwiGLU 18,432 -> 2,304 34 -> 14,
+//     11,776 -> 4,352 25 -> 16, gated 6,144 -> 4,352 15 -> 10), or plain from long rows into few outputs (16,384 ->
+//     4,096 20.5 -> 15.0; 5,376 -> 6,656 would lose, 10 -> 11, 4,096 -> 16,384 twice 20 -> 22).  Q8_0: four rows
+//     of 4,096 columns and more (16,384 -> 6,656 38 -> 30), three of 6,144 or many outputs.
+bool rows_kernel_pays(bool verifier, std::uint32_t encoding, int prologue, std::int64_t rows,
+                      std::int64_t output_dim, std::int64_t input_dim) {
+    constexpr std::int64_t kLongRows = 12288, kManyOutputs = 12288;
+    if (prologue == kRecords || prologue == kHalfImage || rows < 2) return false;
+    const bool q45 = encoding == kEncQ4K || encoding == kEncQ5K;
+    const bool q8 = encoding == kEncQ8_0;
+    if (rows == 2) return (!q8 && input_dim > kLongRows) || (q45 && output_dim >= kManyOutputs);
+    const bool q8_three = input_dim >= 6144 || output_dim >= kManyOutputs;
+    if (verifier) return !q8 || q8_three;
+    if (rows > 4) return false;
+    if (q8) return rows == 4 ? input_dim >= 4096 : q8_three;
+    return q45 && (prologue != kPlain || (input_dim > kLongRows && output_dim <= 8192));
 }
 
 // Shared body of the small-batch entry points.
@@ -105,7 +132,8 @@ int run_small_batch(bool verifier, const Descriptor* const* descriptors, const f
     }
     const std::int64_t required = small_batch_workspace_bytes(rows, input_dim);
     if (required == 0 || workspace_nbytes < required) return kInvalid;
-    // One or two rows, and the verifier entry points at any row count: the
+    // The exact verifier's matrix-core kernel: that family from four rows on, and where it is the faster
+    // one (rows_kernel_pays).  Else one or two rows, and the verifier entry points at any row count: the
     // vector-ALU kernels.  Otherwise 3 and 4 rows: the int8 matrix-core kernel,
     // which quantizes inside the kernel; 5..16 rows (Q6_K: 3..16): the fp16 matrix-core kernel
     // behind its conversion launch (Q8_0 below five rows: its dot kernel).
@@ -113,14 +141,17 @@ int run_small_batch(bool verifier, const Descriptor* const* descriptors, const f
     // (two rows are also faster on the dot kernels: they walk the token planes
     // against the same unpacked weights)
     const bool one_row_arithmetic = rows <= 2 || verifier;
-    const bool verifier_matrix = verifier && rows >= kFirstVerifierMatrixRows;
+    const bool always_rows = verifier && rows >= kFirstVerifierMatrixRows;
+    // (two and three rows are served without the room as well)
+    const bool room = rows >= 2 && workspace_nbytes >= small_batch_workspace_bytes(rows, input_dim, true);
     ProjectionSet dot{}, dot6{}, dot8{}, matrix{}, half{}, exact{}, verifier_rows{};
     dot.input_dim = dot6.input_dim = dot8.input_dim = matrix.input_dim = half.input_dim =
         exact.input_dim = verifier_rows.input_dim = input_dim;
     for (int index = 0; index < set.count; ++index) {
         const std::uint32_t encoding = set.op[index].encoding;
         ProjectionSet* target = &exact;
-        if (verifier_matrix && gemv_rows_supports(encoding, input_dim)) {
+        if ((always_rows || (room && rows_kernel_pays(verifier, encoding, prologue, rows, set.op[index].output_dim, input_dim))) &&
+            gemv_rows_supports(encoding, input_dim)) {
             target = &verifier_rows;
         } else if (one_row_arithmetic && gemv_dot_supports(encoding, input_dim)) {
             target = &dot;
@@ -147,7 +178,7 @@ int run_small_batch(bool verifier, const Descriptor* const* descriptors, const f
     const float* dot_first = first;
     const float* dot_second = second;
     int dot_prologue = prologue;
-    if (verifier_matrix && input_dim % 256 == 0) {
+    if ((always_rows && input_dim % 256 == 0) || verifier_rows.count > 0) {
         // The matrix-core kernel reads the activations in operand order: a quantizer launch
         // writes that image behind the records (whatever the encodings of this call, so that a
         // prequantized call behind it finds both), and the dot kernels of the other encodings
@@ -178,10 +209,12 @@ int run_small_batch(bool verifier, const Descriptor* const* descriptors, const f
         if (verifier_rows.count > 0) {
             launch_gemv_rows(verifier_rows, image, static_cast<const std::uint8_t*>(workspace), rows, clear.count > 0, fill_launch, as_stream(stream));
         }
-        dot_first = static_cast<const float*>(workspace);
-        dot_second = nullptr;
-        dot_prologue = kRecords;
-        records = nullptr;
+        if (one_row_arithmetic) {  // (the others' kernels take the activations as they are)
+            dot_first = static_cast<const float*>(workspace);
+            dot_second = nullptr;
+            dot_prologue = kRecords;
+            records = nullptr;
+        }
     }
     if (dot.count > 0) {
         launch_gemv_dot(dot, dot_first, dot_second, records, dot_prologue, rows, as_stream(stream));
@@ -352,7 +385,7 @@ int nfn_native_tile_linear_packed_weight_q8_1_multi_decode_float32_v1(
 
 std::int64_t nfn_native_tile_k_quant_mmq_workspace_bytes_v1(std::int64_t rows,
                                                             std::int64_t input_dim) {
-    return small_batch_workspace_bytes(rows, input_dim);
+    return small_batch_workspace_bytes(rows, input_dim, true);
 }
 
 int nfn_native_tile_k_quant_mmq_multi_linear_float32_v1(

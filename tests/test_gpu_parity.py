@@ -806,6 +806,54 @@ def test_verifier_matrix_core_rows_equal_the_one_row_kernel(cuda, oracle, encodi
                 assert_bits_equal(whole[row:row + 1].contiguous(), part, f"row {row} of {rows}")
 
 
+@pytest.mark.parametrize("in_dim,out_dim", [(256, 40), (2304, 33), (6656, 70), (4096, 12289), (12544, 31)])
+@pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q6_K, kquant.Q8_0])
+def test_two_and_three_rows_equal_the_one_row_kernel_on_either_kernel(cuda, oracle, encoding, in_dim, out_dim):
+    """Two and three rows of the one-row arithmetic run on the matrix cores where that is faster and the
+    workspace has room for the operands: the same bits with it, with the records alone, and from the
+    records that the call leaves.  Behind the prologues the same rows as alone."""
+    packed = random_packed(encoding, 64, in_dim, 90).reshape(64, -1)
+    chosen = torch_().from_numpy(np.random.default_rng(91).integers(0, 64, out_dim)).to(cuda)
+    weight = tile_ops.PackedWeight(encoding, out_dim, in_dim,
+                                   torch_().from_numpy(packed).to(cuda).index_select(0, chosen).reshape(-1))
+    x = to_device(kquant.synthetic_activations(92, 3, in_dim) * np.array([[1.0], [1.0e3], [1.0e-3]], dtype=np.float32), cuda)
+    second = to_device(kquant.synthetic_activations(93, 3, in_dim), cuda)
+    one = tile_ops.small_batch_workspace(1, in_dim)
+    for prologue in ("plain", "gated", "swiglu"):
+        with_second = {} if prologue == "plain" else {"prologue": prologue}
+        alone = [tile_ops.multi_linear([weight], x[r:r + 1].contiguous(), one, **with_second,
+                                       **({"second": second[r:r + 1].contiguous()} if with_second else {}))[0] for r in range(3)]
+        for rows, family in ((2, "mmq"), (2, "mmvq"), (3, "mmvq")):
+            room = tile_ops.small_batch_workspace(rows, in_dim)
+            for workspace in (room, room[:(rows * in_dim // 32 * 72 + 255) // 256 * 256]):
+                batch = tile_ops.multi_linear([weight], x[:rows], workspace, family=family, **with_second,
+                                              **({"second": second[:rows]} if with_second else {}))[0]
+                for row in range(rows):
+                    assert_bits_equal(batch[row:row + 1].contiguous(), alone[row], f"{prologue} {family} row {row} of {rows}")
+            if family == "mmvq":
+                assert_bits_equal(tile_ops.multi_linear_prequantized([weight], rows, workspace, family=family)[0], batch, "records")
+
+
+@pytest.mark.parametrize("rows,prologue", [(3, "plain"), (4, "plain"), (3, "swiglu"), (4, "gated")])
+@pytest.mark.parametrize("in_dim", [256, 6144, 12544])
+@pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q8_0])
+def test_small_batches_on_the_exact_verifiers_kernel(cuda, oracle, encoding, in_dim, rows, prologue):
+    """Small batches that the verifier's matrix-core kernel takes from the other family: row for row the
+    verifier family's bits, whether alone or beside a projection of another format."""
+    weights = [tile_ops.PackedWeight.from_numpy(e, random_packed(e, n, in_dim, 94 + n), n, in_dim)
+               for e, n in ((encoding, 77), (kquant.Q6_K, 20))]
+    x, second = (to_device(kquant.synthetic_activations(seed, rows, in_dim), cuda) for seed in (95, 96))
+    arguments = {} if prologue == "plain" else {"prologue": prologue, "second": second}
+    workspace = tile_ops.small_batch_workspace(rows, in_dim)
+    exact = tile_ops.multi_linear(weights, x, workspace, family="mmvq", **arguments)
+    alone = tile_ops.multi_linear(weights[:1], x, workspace, **arguments)[0]
+    both = tile_ops.multi_linear(weights, x, workspace, **arguments)
+    assert_bits_equal(both[0], alone, "beside another format")
+    if in_dim > 12288 or (in_dim >= 6144 if encoding == kquant.Q8_0 else prologue != "plain"):
+        assert_bits_equal(alone, exact[0], "the verifier's rows")
+    assert normalised_error(both[1].cpu().numpy(), exact[1].cpu().numpy()) <= TOLERANCE
+
+
 @pytest.mark.parametrize("in_dim", [4096, 4352, 6656])
 @pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q6_K, kquant.Q8_0])
 def test_verifier_matrix_core_rows_of_many_tiles_a_workgroup(cuda, encoding, in_dim):
