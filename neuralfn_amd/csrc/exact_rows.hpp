@@ -170,15 +170,15 @@ struct ExactUnit<kEncQ8_0> {
 template <std::uint32_t ENC>
 constexpr bool kExactRowsFormat = ENC == kEncQ4K || ENC == kEncQ5K || ENC == kEncQ6K || ENC == kEncQ8_0;
 
-// The workgroup's copy of the input rows: [row][unit][kExactPitch].
-template <int R>
+// The workgroup's copy of the input rows: [row][unit][kExactPitch].  PARTLY: the first `there` exist.
+template <int R, bool PARTLY = false>
 __device__ __forceinline__ void exact_rows_stage(const float* __restrict__ input, std::int64_t input_dim,
-                                                 float* staged) {
+                                                 float* staged, int there = R) {
     const int units = static_cast<int>(input_dim >> 6);
     for (int index = threadIdx.x; index < R * units * 16; index += kExactWaves * kWave) {
         const int row = index / (units * 16), piece = index % (units * 16);
         typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-        const exact_f32x4 x = *reinterpret_cast<const f32x4_a4*>(input + row * input_dim + 4 * piece);
+        const exact_f32x4 x = *reinterpret_cast<const f32x4_a4*>(input + (PARTLY ? min(row, there - 1) : row) * input_dim + 4 * piece);
         *reinterpret_cast<exact_f32x4*>(staged + (row * units + (piece >> 4)) * kExactPitch + 4 * (piece & 15)) = x;
     }
     __syncthreads();

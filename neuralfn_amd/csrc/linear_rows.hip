@@ -1,12 +1,17 @@
-// The exact tier at one to three input rows: float activations from LDS, packed weights streamed
-// once, a wave per pair of weight rows (exact_rows.hpp).  What bounds it is the weight stream for
-// one row and the vector ALU (2.25 instructions to decode a weight, one per product) beyond.
-// Rows past three are cheaper on the matrix cores (linear_exact.hip), where a product costs
-// nothing on the vector ALU.  4,096 -> 6,656 of Q4_K at 1 / 3 rows: 30.4 / 40.3 -> 6.3 / 9.0 us
+// The exact tier at one to three input rows, and at more of them into few outputs: float activations
+// from LDS, packed weights streamed once, a wave per pair of weight rows (exact_rows.hpp).  What bounds it
+// is the weight stream for one row and the vector ALU (2.25 instructions to decode a weight, one per
+// product) beyond.  More rows into many outputs are cheaper on the matrix cores (linear_exact.hip), where a
+// product costs nothing on the vector ALU.  Into few outputs that kernel's tiles fill a fraction of the
+// chip and walk K for as long as ever; here a workgroup takes two or three of the rows (blockIdx.y), and
+// the call is done in what three rows take until there is a workgroup a unit (rows_pay below).
+// 4,096 -> 6,656 of Q4_K at 1 / 3 rows: 30.4 / 40.3 -> 6.3 / 9.0 us
 // against the wave-per-row kernel that loaded two bytes a lane.
 #include "common.hpp"
 #include "exact_rows.hpp"
 #include "kernels.hpp"
+
+#include <algorithm>
 
 namespace nfn {
 
@@ -15,12 +20,18 @@ namespace {
 constexpr std::int64_t kMaxLds = 160 * 1024;
 constexpr std::int64_t kMaxDenseLds = 159 * 1024;  // beside the waves' meeting place
 
-template <std::uint32_t ENC, int R>
+// GROUPS: more than R rows, R of them (of the last group those that exist) a workgroup of blockIdx.y.
+// (A form of its own: the checks cost the call of up to three rows 3 %.)
+template <std::uint32_t ENC, int R, bool GROUPS>
 __global__ __launch_bounds__(kExactWaves * kWave) void linear_rows_kernel(
     const std::uint8_t* __restrict__ data, std::int64_t row_stride, const float* __restrict__ input,
-    const float* __restrict__ bias, float* __restrict__ output, std::int64_t input_dim, std::int64_t output_dim) {
+    const float* __restrict__ bias, float* __restrict__ output, std::int64_t input_dim, std::int64_t output_dim,
+    int rows) {
     extern __shared__ __attribute__((aligned(16))) float staged[];
-    exact_rows_stage<R>(input, input_dim, staged);
+    const int row0 = GROUPS ? static_cast<int>(blockIdx.y) * R : 0, there = GROUPS ? min(R, rows - row0) : R;
+    input += row0 * input_dim;
+    output += row0 * output_dim;
+    exact_rows_stage<R, GROUPS>(input, input_dim, staged, there);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const std::int64_t pairs = (output_dim + kExactPair - 1) / kExactPair;
     exact_rows_walk<ENC, R>(data, row_stride, output_dim, input_dim, staged,
@@ -30,12 +41,15 @@ __global__ __launch_bounds__(kExactWaves * kWave) void linear_rows_kernel(
                                 if ((threadIdx.x & 63) != 0) return;
                                 const float offset = bias != nullptr ? bias[row] : 0.0f;
 #pragma unroll
-                                for (int r = 0; r < R; ++r) output[r * output_dim + row] = sums[r] + offset;
+                                for (int r = 0; r < R; ++r) {
+                                    if (r < there) output[r * output_dim + row] = sums[r] + offset;
+                                }
                             });
 }
 
 template <std::uint32_t ENC, int R>
-void launch_rows(const Descriptor& weight, const float* input, const float* bias, float* output, hipStream_t stream) {
+void launch_rows(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
+                 hipStream_t stream) {
     const std::int64_t pairs = (weight.output_dim + kExactPair - 1) / kExactPair;
     const std::int64_t lds = exact_rows_lds(R, weight.input_dim);
     // as many workgroups as the units hold at once, every wave with the same number of pairs
@@ -43,10 +57,20 @@ void launch_rows(const Descriptor& weight, const float* input, const float* bias
     const std::int64_t most = (pairs + kExactWaves - 1) / kExactWaves;
     const std::int64_t turns = (most + resident - 1) / resident;
     const std::int64_t groups = (most + turns - 1) / turns;
-    allow_large_lds<linear_rows_kernel<ENC, R>>();
-    hipLaunchKernelGGL((linear_rows_kernel<ENC, R>), dim3(static_cast<unsigned>(groups)), dim3(kExactWaves * kWave),
-                       static_cast<unsigned>(lds), stream, weight.data, weight.row_stride_bytes, input, bias, output,
-                       weight.input_dim, weight.output_dim);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups), static_cast<unsigned>((rows + R - 1) / R)),
+                           dim3(kExactWaves * kWave), static_cast<unsigned>(lds), stream, weight.data,
+                           weight.row_stride_bytes, input, bias, output, weight.input_dim, weight.output_dim,
+                           static_cast<int>(rows));
+    };
+    if constexpr (R > 1) {
+        if (rows > R) {
+            allow_large_lds<linear_rows_kernel<ENC, R, true>>();
+            return launch(linear_rows_kernel<ENC, R, true>);
+        }
+    }
+    allow_large_lds<linear_rows_kernel<ENC, R, false>>();
+    launch(linear_rows_kernel<ENC, R, false>);
 }
 
 // Float and bf16 weights: a wave (SPLIT = 1) or the workgroup's eight waves together (SPLIT = 8, for
@@ -54,17 +78,23 @@ void launch_rows(const Descriptor& weight, const float* input, const float* bias
 // next turn's requested before this one's are used.  Bound by the weight stream.
 typedef std::uint32_t dense_u32x4 __attribute__((ext_vector_type(4), aligned(2)));
 
-template <std::uint32_t ENC, int R, int SPLIT>
+template <std::uint32_t ENC, int R, int SPLIT, bool GROUPS>
 __global__ __launch_bounds__(kExactWaves * kWave) void dense_rows_kernel(
     const std::uint8_t* __restrict__ data, std::int64_t row_stride, const float* __restrict__ input,
-    const float* __restrict__ bias, float* __restrict__ output, std::int64_t input_dim, std::int64_t output_dim) {
+    const float* __restrict__ bias, float* __restrict__ output, std::int64_t input_dim, std::int64_t output_dim,
+    int rows) {
     constexpr int kValues = ENC == kEncF32 ? 4 : 8;  // of 16 bytes
     extern __shared__ __attribute__((aligned(16))) float staged[];
     __shared__ float meeting[kExactWaves][kExactPair * R];
     typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
     const int columns = static_cast<int>(input_dim);
+    const int row0 = GROUPS ? static_cast<int>(blockIdx.y) * R : 0, there = GROUPS ? min(R, rows - row0) : R;
+    input += row0 * input_dim;
+    output += row0 * output_dim;
     for (int index = threadIdx.x * 4; index < R * columns; index += kExactWaves * kWave * 4) {
-        *reinterpret_cast<exact_f32x4*>(staged + index) = *reinterpret_cast<const f32x4_a4*>(input + index);
+        // (rows past the end are whatever the first one has there; their sums are not stored)
+        *reinterpret_cast<exact_f32x4*>(staged + index) =
+            *reinterpret_cast<const f32x4_a4*>(input + (!GROUPS || index < there * columns ? index : index % columns));
     }
     __syncthreads();
     const int lane = threadIdx.x & 63;
@@ -141,7 +171,9 @@ __global__ __launch_bounds__(kExactWaves * kWave) void dense_rows_kernel(
                     if (at < output_dim) {
                         const float offset = bias != nullptr ? bias[at] : 0.0f;
 #pragma unroll
-                        for (int r = 0; r < R; ++r) output[r * output_dim + at] = sums[k][r] + offset;
+                        for (int r = 0; r < R; ++r) {
+                            if (r < there) output[r * output_dim + at] = sums[k][r] + offset;
+                        }
                     }
                 }
             }
@@ -161,32 +193,42 @@ __global__ __launch_bounds__(kExactWaves * kWave) void dense_rows_kernel(
                 float total = meeting[0][threadIdx.x];
 #pragma unroll
                 for (int w = 1; w < kExactWaves; ++w) total += meeting[w][threadIdx.x];
-                if (at < output_dim) output[r * output_dim + at] = total + (bias != nullptr ? bias[at] : 0.0f);
+                if (at < output_dim && r < there) output[r * output_dim + at] = total + (bias != nullptr ? bias[at] : 0.0f);
             }
         }
     }
 }
 
 template <std::uint32_t ENC, int R>
-void launch_dense(const Descriptor& weight, const float* input, const float* bias, float* output, hipStream_t stream) {
+void launch_dense(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
+                  hipStream_t stream) {
     const std::int64_t pairs = (weight.output_dim + kExactPair - 1) / kExactPair;
     const std::int64_t lds = R * weight.input_dim * 4;
     const std::int64_t resident = std::int64_t(compute_units()) * (lds <= 40 * 1024 ? 4 : lds <= 78 * 1024 ? 2 : 1);
     // few pairs: a workgroup each, so that eight waves walk the row instead of one
-    const bool split = pairs <= 2 * std::int64_t(compute_units());
+    const bool split = pairs * ((rows + R - 1) / R) <= 2 * std::int64_t(compute_units());
     const std::int64_t most = split ? pairs : (pairs + kExactWaves - 1) / kExactWaves;
     const unsigned groups = static_cast<unsigned>(most < resident ? most : resident);
-    if (split) {
-        allow_large_lds<dense_rows_kernel<ENC, R, kExactWaves>>(kMaxDenseLds);
-        hipLaunchKernelGGL((dense_rows_kernel<ENC, R, kExactWaves>), dim3(groups), dim3(kExactWaves * kWave),
-                           static_cast<unsigned>(lds), stream, weight.data, weight.row_stride_bytes, input, bias, output,
-                           weight.input_dim, weight.output_dim);
-    } else {
-        allow_large_lds<dense_rows_kernel<ENC, R, 1>>(kMaxDenseLds);
-        hipLaunchKernelGGL((dense_rows_kernel<ENC, R, 1>), dim3(groups), dim3(kExactWaves * kWave),
-                           static_cast<unsigned>(lds), stream, weight.data, weight.row_stride_bytes, input, bias, output,
-                           weight.input_dim, weight.output_dim);
+    const unsigned row_groups = static_cast<unsigned>((rows + R - 1) / R);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(groups, row_groups), dim3(kExactWaves * kWave), static_cast<unsigned>(lds), stream,
+                           weight.data, weight.row_stride_bytes, input, bias, output, weight.input_dim,
+                           weight.output_dim, static_cast<int>(rows));
+    };
+    const auto form = [&](auto grouped) {
+        constexpr bool kGroups = decltype(grouped)::value;
+        if (split) {
+            allow_large_lds<dense_rows_kernel<ENC, R, kExactWaves, kGroups>>(kMaxDenseLds);
+            launch(dense_rows_kernel<ENC, R, kExactWaves, kGroups>);
+        } else {
+            allow_large_lds<dense_rows_kernel<ENC, R, 1, kGroups>>(kMaxDenseLds);
+            launch(dense_rows_kernel<ENC, R, 1, kGroups>);
+        }
+    };
+    if constexpr (R > 1) {
+        if (rows > R) return form(std::true_type{});
     }
+    form(std::false_type{});
 }
 
 template <std::uint32_t ENC>
@@ -195,14 +237,14 @@ void launch_for(const Descriptor& weight, const float* input, const float* bias,
     const auto launch = [&](auto count) {
         constexpr int kRows = decltype(count)::value;
         if constexpr (kExactRowsFormat<ENC>) {
-            launch_rows<ENC, kRows>(weight, input, bias, output, stream);
+            launch_rows<ENC, kRows>(weight, input, bias, output, rows, stream);
         } else {
-            launch_dense<ENC, kRows>(weight, input, bias, output, stream);
+            launch_dense<ENC, kRows>(weight, input, bias, output, rows, stream);
         }
     };
     if (rows == 1) {
         launch(std::integral_constant<int, 1>{});
-    } else if (rows == 2) {
+    } else if (rows == 2 || rows == 4) {
         launch(std::integral_constant<int, 2>{});
     } else {
         launch(std::integral_constant<int, 3>{});
@@ -211,8 +253,40 @@ void launch_for(const Descriptor& weight, const float* input, const float* bias,
 
 }  // namespace
 
+namespace {
+
+constexpr std::int64_t kMostRows = 3;  // of a workgroup
+
+// Four rows and more: while weight rows times groups of input rows fill few enough waves.  Weight rows
+// per compute unit (sixteen are a workgroup a unit) up to which it wins over linear_exact.hip, from 4 to
+// 96 rows of 2,304, 4,096 and 6,400 columns into 64 to 5,000 outputs; both in us, this one second:
+//   Q4_K, Q8_0   26, from twelve rows on (that kernel cuts more then) 37: 8 rows of 4,096 into 300 / 2,000 / 3,000
+//     outputs 10.8 and 6.8 / 11.1 and 9.9 / 11.4 and 13.5, 96 rows into 300 16.1 and 13.4
+//   Q5_K         16, from seventeen rows on 26: 8 rows into 1,100 / 2,000 11.1 and 8.0 / 11.4 and 12.9
+//   Q6_K         16, from ten rows or beyond 4,096 columns 26: 8 rows of 6,400 into 600 39.1 and 13.8, 33 45.5 and 26.6
+//   bf16, F32    14 and 25: 8 rows of 6,400 into 1,100 19.5 and 16.8, 32.3 and 17.9; 33 rows into 64 22.8 and 8.3,
+//     37.5 and 7.4
+bool rows_pay(const Descriptor& weight, std::int64_t rows) {
+    std::int64_t most = 0;
+    switch (weight.encoding) {
+        case kEncQ4K: case kEncQ8_0: most = rows >= 12 ? 37 : 26; break;
+        case kEncQ5K: most = rows > 16 ? 26 : 16; break;
+        case kEncQ6K: most = rows > 9 || weight.input_dim > 4096 ? 26 : 16; break;
+        case kEncBF16: most = 14; break;
+        case kEncF32: most = 25; break;
+        default: return false;
+    }
+    // (three rows that leave a compute unit room for one workgroup: 5 rows of 7,168 into 2,937 of Q4_K 16.7 and 17.8)
+    if (exact_rows_lds(kMostRows, weight.input_dim) > 80 * 1024) most = std::min<std::int64_t>(most, 16);
+    const std::int64_t groups = (rows + kMostRows - 1) / kMostRows;
+    return groups <= 65535 && weight.output_dim <= most * compute_units() / groups;
+}
+
+}  // namespace
+
 bool linear_rows_supports(const Descriptor& weight, std::int64_t rows) {
-    if (rows < 1 || rows > 3) return false;
+    if (rows < 1 || (rows > kMostRows && !rows_pay(weight, rows))) return false;
+    if (rows > kMostRows) rows = kMostRows;
     switch (weight.encoding) {
         case kEncQ4K: case kEncQ5K: case kEncQ6K: case kEncQ8_0:
             return weight.input_dim % 64 == 0 && exact_rows_lds(rows, weight.input_dim) <= kMaxLds;

@@ -342,6 +342,38 @@ def test_exact_linear_of_weights_that_are_not_finite(cuda, oracle, encoding, row
     assert normalised_error(y[finite], expected[finite]) <= 1e-5
 
 
+@pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
+def test_exact_linear_small_tiles_of_special_operands(cuda, oracle, encoding):
+    """The matrix-core kernel's 32 x 32 tiles (five and 17 rows into more outputs than the vector kernel takes
+    them for) with operands that are not finite, large or tiny."""
+    for rows, out_dim, in_dim in ((5, 6700, 512), (17, 2100, 256)):
+        test_exact_linear_of_infinities_nan_and_large_activations(cuda, oracle, encoding, rows, out_dim, in_dim)
+        test_exact_linear_of_weights_that_are_not_finite(cuda, oracle, encoding, rows, out_dim, in_dim)
+        test_exact_linear_of_tiny_operands(cuda, oracle, encoding, rows, out_dim, in_dim, -36)
+
+
+@pytest.mark.parametrize("rows,out_dim,in_dim", [(4, 300, 2048), (5, 33, 512), (7, 1300, 256), (12, 999, 8192), (17, 2, 64), (97, 65, 4096)])
+@pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
+def test_exact_linear_of_row_groups(cuda, oracle, encoding, rows, out_dim, in_dim):
+    """More than three rows into few outputs on the vector kernel, two or three of them a workgroup: row for
+    row the bits of the call of three rows (F32 and bf16, whose waves may share a row or not: its bound), a
+    last group of one or two, nothing written past the end."""
+    if encoding not in (kquant.F32, kquant.BF16, kquant.Q8_0):
+        in_dim = max(in_dim, 256)
+    packed = kquant.quantize(encoding, kquant.synthetic_weights(50, out_dim, in_dim))
+    x = kquant.synthetic_activations(51, rows, in_dim)
+    weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    bias = torch_().linspace(-1.0, 1.0, out_dim, device=cuda)
+    device_x = to_device(x, cuda)
+    y = tile_ops.linear(weight, device_x, bias)
+    expected = oracle.linear(encoding, packed, out_dim, in_dim, x) + bias.cpu().numpy()
+    assert normalised_error(y.cpu().numpy(), expected) <= 1e-5
+    if encoding in ALL_PACKED:
+        for first in range(0, rows, 3):
+            part = tile_ops.linear(weight, device_x[first:first + 3].contiguous(), bias)
+            assert_bits_equal(y[first:first + 3].contiguous(), part, f"rows {first} on")
+
+
 @pytest.mark.parametrize("exponent", [-33, -35, -36, -37])
 @pytest.mark.parametrize("rows,out_dim,in_dim", [(3, 67, 512), (5, 67, 512), (60, 5000, 256), (100, 6600, 256), (200, 6600, 256)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
