@@ -580,7 +580,10 @@ void launch_variant(ProjectionSet set, const float* first, const float* second,
     const std::size_t lds = static_cast<std::size_t>(T) * token_image_bytes_host(blocks);
     const int passes = (tokens + T - 1) / T;
     // (up to six workgroups per unit: 6,656 -> 65,536 streams at 5.25 TB/s with six, 5.0 with four)
-    const std::int64_t groups = decode_groups(rows, kDotWaves, 6);
+    // Normalising workgroups: one a unit.  Each normalises the row for itself, and two on a unit take turns
+    // at it: 6,656 -> 6,144 + 256 + 256 + 6,144 of Q4_K 17.3 -> 15.6 us, of Q5_K 25.3 -> 18.8 (the norms in a launch of
+    // their own: 16.0 and 19.1); + 1,024 + 1,024 18.2 -> 16.9 and 26.1 -> 21.5 (16.8, 20.1).
+    const std::int64_t groups = decode_groups(rows, kDotWaves, P == kDualNorm ? 1 : 6);
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups), passes), dim3(kDotThreads), lds,
                            stream, first, packed.a, packed.b, packed.c,
