@@ -785,6 +785,9 @@ __device__ __forceinline__ uint4 pack_as_cached(float4 low, float4 high) {
                       pair(high.z, high.w));
 }
 
+// BLOCK: of several query rows.  (One row's tiles have no rows of a block: the code for them in its kernel makes a
+// decode step of eight layers 0.5 to 1 us a layer longer.)
+template <bool BLOCK>
 __global__ __launch_bounds__(kGroupWaves * kWave) void attention_grouped_kernel(AttentionArguments a) {
     // waves x kStageBytes: a value tile per wave; at the end the waves' results
     // (maxima, denominators, accumulators: less than that) in the same memory
@@ -942,6 +945,55 @@ __global__ __launch_bounds__(kGroupWaves * kWave) void attention_grouped_kernel(
             }
         }
     };
+    // ... a tile with at most kStaged rows of the block: those are read first, a lane two dimensions, rounded
+    // and left in the wave's stage as the cache would hold them, and every lane then reads the row it
+    // needs from where it lies (one pointer, into the cache or the stage).  The choice a row above makes every
+    // request wait for the one before: a tile with a row of the block took 8 us with it.  With merge, us,
+    // 32 heads over 2: 7 rows behind 137 / 1,500 keys 20.2 / 19.6 -> 12.2 / 12.8; 48 over 8, 2 rows 19.2 / 18.5 -> 11.1 / 11.3.
+    // (Four rows a turn: eight take the block of two rows 0.5 us longer, sixteen spill.)
+    constexpr int kStaged = 32;
+    const auto load_mixed = [&](std::int64_t tile, std::int64_t slot, int in_tile, int left) {
+        constexpr int kRows = 4;
+        const float* const keys_of_block = a.block_key + (tile + left - a.context_length) * block_stride + head_offset;
+        const float* const values_of_block = a.block_value + (tile + left - a.context_length) * block_stride + head_offset;
+        wave_sync();  // the reads of the previous tile are done
+        for (int first = 0; first <= in_tile - left; first += kRows) {  // wave-uniform
+            float2 key_two[kRows], value_two[kRows];
+#pragma unroll
+            for (int r = 0; r < kRows; ++r) {
+                const std::int64_t from = (first + r < in_tile - left ? first + r : in_tile - left) * block_stride + 2 * lane;
+                key_two[r] = *reinterpret_cast<const float2*>(keys_of_block + from);
+                value_two[r] = *reinterpret_cast<const float2*>(values_of_block + from);
+            }
+#pragma unroll
+            for (int r = 0; r < kRows; ++r) {
+                std::uint32_t* const to = reinterpret_cast<std::uint32_t*>(stage + (first + r) * kStageRowBytes) + lane;
+                to[0] = static_cast<std::uint32_t>(to_bf16(key_two[r].x)) | (static_cast<std::uint32_t>(to_bf16(key_two[r].y)) << 16);
+                to[kStaged * kStageRowBytes / 4] =
+                    static_cast<std::uint32_t>(to_bf16(value_two[r].x)) | (static_cast<std::uint32_t>(to_bf16(value_two[r].y)) << 16);
+            }
+        }
+        // (the reads below may go to the stage by another path than these writes)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        wave_sync();
+        const auto row_of = [&](const std::uint16_t* cache, int staged, int wanted) {
+            const int key = wanted < in_tile ? wanted : in_tile;
+            return key < left ? reinterpret_cast<const std::uint8_t*>(cache + ring_row(slot + key) * a.cache_row_stride + head_offset)
+                              : stage + (staged + key - left) * kStageRowBytes;
+        };
+        for (int block = 0; block < 4; ++block) {
+            const std::uint8_t* const row = row_of(a.key_cache, 0, block * 16 + i) + 16 * j;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) key_raw[block][s] = *reinterpret_cast<const uint4*>(row + 64 * s);
+        }
+        for (int block = 0; block < 4; ++block) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                value_raw[block][r] = *reinterpret_cast<const uint4*>(row_of(a.value_cache, kStaged, block * 16 + 4 * j + r) + 16 * i);
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // ... before the stage is written again
+    };
     const auto is_straight = [&](std::int64_t tile, std::int64_t slot) {  // wave-uniform
         return tile + kWave - 1 <= tiled_last && tile + kWave - 1 < a.context_length &&
             slot + kWave <= capacity;
@@ -952,7 +1004,18 @@ __global__ __launch_bounds__(kGroupWaves * kWave) void attention_grouped_kernel(
          tile += tile_step, tile_slot = ring_row(tile_slot + slot_step)) {
         const int in_tile =
             static_cast<int>(tiled_last - tile < kWave - 1 ? tiled_last - tile : kWave - 1);
-        if (is_straight(tile, tile_slot)) {
+        if constexpr (BLOCK) {
+            // keys of the tile from here on are rows of the block
+            const int left = a.context_length <= tile ? 0
+                : static_cast<int>(a.context_length - tile < kWave ? a.context_length - tile : kWave);
+            if (is_straight(tile, tile_slot)) {
+                load_straight(tile_slot);
+            } else if (left <= in_tile && in_tile - left < kStaged) {
+                load_mixed(tile, tile_slot, in_tile, left);
+            } else {
+                load_general(tile, tile_slot, in_tile);
+            }
+        } else if (is_straight(tile, tile_slot)) {
             load_straight(tile_slot);
         } else {
             load_general(tile, tile_slot, in_tile);
@@ -1199,8 +1262,9 @@ bool grouped_form_fits(const AttentionArguments& arguments) {
 }
 
 // `tiles_per_group`: the most 64-key tiles one workgroup has to cover.
+// `grouped`: the matrix-core kernel wherever it fits.
 void launch_attention(const AttentionArguments& arguments, std::int64_t query_rows,
-                      std::int64_t tiles_per_group, hipStream_t stream) {
+                      std::int64_t tiles_per_group, hipStream_t stream, bool grouped = false) {
     std::int64_t waves = tiles_per_group;
     if (waves < 1) waves = 1;
     if (waves > kMaxWaves) waves = kMaxWaves;
@@ -1211,15 +1275,19 @@ void launch_attention(const AttentionArguments& arguments, std::int64_t query_ro
     // kernel pays where its workgroups are many (the split form) or where the vector
     // kernel's would not fit the chip at once (blocks of many rows).
     if (grouped_form_fits(arguments) &&
-        (arguments.partials != nullptr || query_rows * arguments.query_heads > compute_units())) {
+        (grouped || arguments.partials != nullptr || query_rows * arguments.query_heads > compute_units())) {
         static_assert(kGroupWaves == kMaxWaves, "one wave rule for both kernels");
         const std::int64_t groups = arguments.kv_heads *
             ((arguments.heads_per_kv + kGroupHeads - 1) / kGroupHeads);
-        allow_large_lds<attention_grouped_kernel>(kGroupWaves * kStageBytes);
-        hipLaunchKernelGGL(attention_grouped_kernel,
-                           dim3(static_cast<unsigned>(query_rows * groups), splits),
-                           dim3(static_cast<unsigned>(waves * kWave)),
-                           static_cast<std::size_t>(waves) * kStageBytes, stream, arguments);
+        const dim3 grid(static_cast<unsigned>(query_rows * groups), splits), block(static_cast<unsigned>(waves * kWave));
+        const std::size_t lds = static_cast<std::size_t>(waves) * kStageBytes;
+        if (query_rows == 1) {
+            allow_large_lds<attention_grouped_kernel<false>>(kGroupWaves * kStageBytes);
+            hipLaunchKernelGGL(attention_grouped_kernel<false>, grid, block, lds, stream, arguments);
+        } else {
+            allow_large_lds<attention_grouped_kernel<true>>(kGroupWaves * kStageBytes);
+            hipLaunchKernelGGL(attention_grouped_kernel<true>, grid, block, lds, stream, arguments);
+        }
         return;
     }
     const dim3 grid(static_cast<unsigned>(query_rows * arguments.query_heads), splits);
@@ -1287,6 +1355,15 @@ std::int64_t gqa_decode_split_workspace_bytes(std::int64_t query_heads, std::int
 
 namespace {
 
+// Keys of a row that a workgroup takes alone in one launch although there is a workspace: what the merge
+// takes is more than a few tiles side by side gain.  One row / seven rows of 32 heads over 2, us, split -> alone:
+// 90 keys 11.6 / 12.3 -> 7.2 / 9.1, 137 11.5 / 12.2 -> 7.3 / 9.8, 230 10.7 / 12.4 -> 9.3 / 9.9; 350 (six tiles) 10.8 / 12.7 and
+// 11.2 / 12.4.  A block's rows on the matrix cores, where the head size allows (7 rows of 137 keys on the vector
+// kernel 11.8), else up to three tiles (16 heads over 4, 4 rows of 137 keys 13.5 -> 11.8).
+bool one_launch(const AttentionArguments& a, std::int64_t tiles) {
+    return tiles <= (grouped_form_fits(a) ? 4 : 3);
+}
+
 // Split form.  `tiles`: the 64-key tiles of the longest row, or with a position in
 // device memory the most it can have (the shares are cut from each row's real key
 // count when the kernel runs; surplus shares are empty).  `partial_bytes` bounds the
@@ -1308,7 +1385,11 @@ void launch_split(AttentionArguments a, std::int64_t query_rows, std::int64_t ti
     // in 16 shares of two waves takes 11.1 us with its merge, in 32 shares of one wave 12.1 us
     // (12 or 24 shares: 11.7; 8: 11.9); long contexts and blocks are not touched by this
     // (32,768 keys: 128 shares 15.1 us, 96: 15.4, 64: 17.1; a 16-row block: 8..24 shares 16.1 us).
-    if (query_rows == 1 && grouped && 2 * splits > tiles && tiles >= 4) splits = (tiles + 1) / 2;
+    // Sixteen shares up to 48 tiles: 3,000 keys in 24 of two waves 11.9 to 12.5 us, in 16 of three 11.1 to 11.6.
+    if (query_rows == 1 && grouped && 2 * splits > tiles && tiles >= 4) {
+        splits = (tiles + 1) / 2;
+        if (tiles <= 48 && splits > 16) splits = 16;
+    }
     if (splits < 2) splits = 2;
     if (splits > partial_bytes / share_bytes) splits = partial_bytes / share_bytes;
     if (splits < 2) {
@@ -1330,8 +1411,8 @@ void launch_gqa_decode_split(const NfnNativeTileGlimmerGqaDecodeDescriptorV1& d,
                              hipStream_t stream) {
     const AttentionArguments a = decode_arguments(d);
     const std::int64_t tiles = tiles_of(a.sliding_window);
-    if (!vector_form_fits(a) || tiles < 2) {
-        launch_attention(a, 1, tiles, stream);  // nothing to split, or no vector form: one launch
+    if (!vector_form_fits(a) || one_launch(a, tiles)) {
+        launch_attention(a, 1, tiles, stream);  // little to split, or no vector form: one launch
         return;
     }
     launch_split(a, 1, tiles, partials, gqa_decode_split_workspace_bytes(d.query_heads, d.head_dim),
@@ -1381,10 +1462,10 @@ void launch_block_attention(const NfnNativeTileDFlashBlockAttentionDescriptorV1&
         if (window < longest) longest = window;
     }
     const std::int64_t tiles = tiles_of(longest);
-    if (partials != nullptr && vector_form_fits(a) && tiles >= 2) {
+    if (partials != nullptr && vector_form_fits(a) && !one_launch(a, tiles)) {
         launch_split(a, d.query_rows, tiles, partials, partial_bytes, stream);
     } else {
-        launch_attention(a, d.query_rows, tiles, stream);
+        launch_attention(a, d.query_rows, tiles, stream, partials != nullptr && tiles >= 2 && d.query_rows > 1);
     }
 }
 

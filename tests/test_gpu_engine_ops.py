@@ -443,6 +443,26 @@ def test_block_attention_split_form(cuda, oracle, causal, rows, block_rows, quer
     assert lib.nfn_mi355_dflash_block_attention_split_v1(None, workspace.data_ptr(), 1 << 20) == 1
 
 
+@pytest.mark.parametrize("rows,context", [
+    (7, 128), (7, 127), (14, 189), (2, 250), (3, 64),        # one launch: the block at a tile's start, end, over its edge
+    (16, 384), (15, 447), (14, 1500), (31, 513), (32, 640),  # split; up to 31 and 32 rows before the last one
+    (33, 640), (40, 830),                                    # more rows of the block in a tile than the stage takes
+])
+@pytest.mark.parametrize("query_heads,kv_heads", [(32, 2), (48, 8), (16, 8)])
+def test_block_attention_tiles_with_rows_of_the_block(cuda, oracle, rows, context, query_heads, kv_heads):
+    """Tiles that hold cached keys and rows of the block, in rings that wrap and that do not, on the matrix cores
+    and (two query heads a key/value head) on the vector kernel, split and in one launch."""
+    for window, capacity in ((context + rows, context + 64), (200, 256)):
+        test_block_attention_split_form(cuda, oracle, True, rows, rows, query_heads, kv_heads, context, window, capacity, 128)
+
+
+@pytest.mark.parametrize("keys", [1, 63, 64, 128, 191, 192, 255, 256, 257, 2049, 3000, 3072, 3073])
+def test_one_row_attention_in_one_launch_and_in_shares(cuda, oracle, keys):
+    """Both sides of the key counts that the number of workgroups a row is shared out over turns at."""
+    test_block_attention_split_form(cuda, oracle, True, 1, 1, 32, 4, keys, keys + 1, keys + 64, 128)
+    test_block_attention_split_form(cuda, oracle, True, 1, 1, 8, 8, keys, keys + 1, keys + 64, 64)
+
+
 def test_block_attention_fails_closed(cuda):
     lib = tile_ops.load()
     x = torch_().zeros(1 << 16, dtype=torch_().float32, device=cuda)
