@@ -90,10 +90,11 @@ Projection make_projection(const Descriptor& descriptor, float* output) {
 //     (16,384 -> 6,656 34 -> 30, 4,096 -> 32,768 35 -> 32; 4,096 -> 6,656 would lose, 12.4 -> 13.1).
 //   Two rows: K above 12,288 (SwiGLU 18,432 -> 2,304 21 -> 14, 16,384 -> 6,656 of Q6_K 38 -> 33) or, Q4_K and Q5_K, many
 //     outputs (4,096 -> 16,384 twice 25 -> 22); 6,656 -> 8,704 would lose, 13.4 -> 15.2.
-//   Three and four rows of the other family, Q4_K and Q5_K: behind a prologue (SwiGLU 18,432 -> 2,304 34 -> 14,
-//     11,776 -> 4,352 25 -> 16, gated 6,144 -> 4,352 15 -> 10), or plain from long rows into few outputs (16,384 ->
-//     4,096 20.5 -> 15.0; 5,376 -> 6,656 would lose, 10 -> 11, 4,096 -> 16,384 twice 20 -> 22).  Q8_0: four rows
-//     of 4,096 columns and more (16,384 -> 6,656 38 -> 30), three of 6,144 or many outputs.
+//   Three and four rows of the other family, Q4_K and Q5_K: K above 8,192, whatever the prologue (a fused prologue has
+//     the bits of the materialised one): SwiGLU 18,432 -> 2,304 34 -> 14, 11,776 -> 4,352 25 -> 16, plain 16,384 -> 4,096
+//     20.5 -> 15.0.  Shorter rows would gain behind a prologue (gated 6,144 -> 4,352 15 -> 10) and lose plain (5,376 ->
+//     6,656 10 -> 11, 4,096 -> 16,384 twice 20 -> 22).  Q8_0, whose bits are the one-row kernel's on either: four rows of
+//     4,096 columns and more (16,384 -> 6,656 38 -> 30), three of 6,144 or many outputs.
 bool rows_kernel_pays(bool verifier, std::uint32_t encoding, int prologue, std::int64_t rows,
                       std::int64_t output_dim, std::int64_t input_dim) {
     constexpr std::int64_t kLongRows = 12288, kManyOutputs = 12288;
@@ -105,7 +106,7 @@ bool rows_kernel_pays(bool verifier, std::uint32_t encoding, int prologue, std::
     if (verifier) return !q8 || q8_three;
     if (rows > 4) return false;
     if (q8) return rows == 4 ? input_dim >= 4096 : q8_three;
-    return q45 && (prologue != kPlain || (input_dim > kLongRows && output_dim <= 8192));
+    return q45 && input_dim > 8192;
 }
 
 // Shared body of the small-batch entry points.

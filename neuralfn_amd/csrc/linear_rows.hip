@@ -18,6 +18,12 @@ namespace nfn {
 namespace {
 
 constexpr std::int64_t kMaxLds = 160 * 1024;
+constexpr std::int64_t kMostRows = 3;  // of a workgroup
+
+// The row count that the forms are chosen for: a row of a call of four to 32 rows has the same bits
+// whichever other rows come with it, so that those calls take one form, which may not lose at 32.
+std::int64_t rows_chosen_for(std::int64_t rows) { return rows > kMostRows && rows < 32 ? 32 : rows; }
+
 constexpr std::int64_t kMaxDenseLds = 159 * 1024;  // beside the waves' meeting place
 
 // GROUPS: more than R rows, R of them (of the last group those that exist) a workgroup of blockIdx.y.
@@ -206,7 +212,9 @@ void launch_dense(const Descriptor& weight, const float* input, const float* bia
     const std::int64_t lds = R * weight.input_dim * 4;
     const std::int64_t resident = std::int64_t(compute_units()) * (lds <= 40 * 1024 ? 4 : lds <= 78 * 1024 ? 2 : 1);
     // few pairs: a workgroup each, so that eight waves walk the row instead of one
-    const bool split = pairs * ((rows + R - 1) / R) <= 2 * std::int64_t(compute_units());
+    // (a form that a row's bits hang on)
+    const std::int64_t row_groups_chosen_for = (rows_chosen_for(rows) + kMostRows - 1) / kMostRows;
+    const bool split = pairs * row_groups_chosen_for <= 2 * std::int64_t(compute_units());
     const std::int64_t most = split ? pairs : (pairs + kExactWaves - 1) / kExactWaves;
     const unsigned groups = static_cast<unsigned>(most < resident ? most : resident);
     const unsigned row_groups = static_cast<unsigned>((rows + R - 1) / R);
@@ -255,23 +263,20 @@ void launch_for(const Descriptor& weight, const float* input, const float* bias,
 
 namespace {
 
-constexpr std::int64_t kMostRows = 3;  // of a workgroup
-
 // Four rows and more: while weight rows times groups of input rows fill few enough waves.  Weight rows
-// per compute unit (sixteen are a workgroup a unit) up to which it wins over linear_exact.hip, from 4 to
-// 96 rows of 2,304, 4,096 and 6,400 columns into 64 to 5,000 outputs; both in us, this one second:
-//   Q4_K, Q8_0   26, from twelve rows on (that kernel cuts more then) 37: 8 rows of 4,096 into 300 / 2,000 / 3,000
-//     outputs 10.8 and 6.8 / 11.1 and 9.9 / 11.4 and 13.5, 96 rows into 300 16.1 and 13.4
-//   Q5_K         16, from seventeen rows on 26: 8 rows into 1,100 / 2,000 11.1 and 8.0 / 11.4 and 12.9
-//   Q6_K         16, from ten rows or beyond 4,096 columns 26: 8 rows of 6,400 into 600 39.1 and 13.8, 33 45.5 and 26.6
-//   bf16, F32    14 and 25: 8 rows of 6,400 into 1,100 19.5 and 16.8, 32.3 and 17.9; 33 rows into 64 22.8 and 8.3,
-//     37.5 and 7.4
+// per compute unit (sixteen are a workgroup a unit) up to which it wins over linear_exact.hip, from
+// 64 to 5,000 outputs of 2,304, 4,096 and 6,400 columns; both in us, this one second, 4,096 columns if not named:
+//   Q4_K, Q8_0   48 at 32 rows, 37 beyond: 33 rows into 1,100 16.4 and 14.2, 21.9 and 18.1; 8 rows into 1,100 11.0 and
+//     7.4; 96 rows into 300 16.1 and 13.4
+//   Q5_K, Q6_K   26: 33 rows into 600 17.2 and 12.5, 22.3 and 17.5, into 1,100 17.6 and 19.7, 22.6 and 27.8; 8 rows of
+//     6,400 of Q6_K into 600 39.1 and 13.8
+//   bf16, F32    14 and 25: 8 rows of 6,400 into 300 18.5 and 8.9, 31.6 and 9.2; 33 rows into 64 22.8 and 8.3, 37.5 and 7.4
 bool rows_pay(const Descriptor& weight, std::int64_t rows) {
+    rows = rows_chosen_for(rows);
     std::int64_t most = 0;
     switch (weight.encoding) {
-        case kEncQ4K: case kEncQ8_0: most = rows >= 12 ? 37 : 26; break;
-        case kEncQ5K: most = rows > 16 ? 26 : 16; break;
-        case kEncQ6K: most = rows > 9 || weight.input_dim > 4096 ? 26 : 16; break;
+        case kEncQ4K: case kEncQ8_0: most = rows <= 32 ? 48 : 37; break;
+        case kEncQ5K: case kEncQ6K: most = 26; break;
         case kEncBF16: most = 14; break;
         case kEncF32: most = 25; break;
         default: return false;

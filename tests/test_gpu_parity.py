@@ -352,7 +352,21 @@ def test_exact_linear_small_tiles_of_special_operands(cuda, oracle, encoding):
         test_exact_linear_of_tiny_operands(cuda, oracle, encoding, rows, out_dim, in_dim, -36)
 
 
-@pytest.mark.parametrize("rows,out_dim,in_dim", [(4, 300, 2048), (5, 33, 512), (7, 1300, 256), (12, 999, 8192), (17, 2, 64), (97, 65, 4096)])
+@pytest.mark.parametrize("out_dim", [90, 94, 325, 326, 581, 582, 605, 606, 1117, 1118])
+@pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
+def test_exact_linear_carries_the_same_bits_from_four_to_32_rows(cuda, encoding, out_dim):
+    """Which kernel and which form of it runs from four to 32 rows hangs on the outputs alone (their counts on
+    both sides of every line)."""
+    in_dim = 1024
+    weight = tile_ops.PackedWeight.from_numpy(
+        encoding, kquant.quantize(encoding, kquant.synthetic_weights(60, out_dim, in_dim)), out_dim, in_dim)
+    x = to_device(kquant.synthetic_activations(61, 32, in_dim), cuda)
+    all_rows = tile_ops.linear(weight, x)
+    for rows in (4, 5, 9, 12, 17, 24):
+        assert_bits_equal(tile_ops.linear(weight, x[:rows].contiguous()), all_rows[:rows].contiguous(), f"{rows} rows")
+
+
+@pytest.mark.parametrize("rows,out_dim,in_dim", [(4, 300, 2048), (5, 33, 512), (7, 605, 256), (12, 372, 8192), (17, 2, 64), (97, 65, 4096)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
 def test_exact_linear_of_row_groups(cuda, oracle, encoding, rows, out_dim, in_dim):
     """More than three rows into few outputs on the vector kernel, two or three of them a workgroup: row for
@@ -867,11 +881,12 @@ def test_two_and_three_rows_equal_the_one_row_kernel_on_either_kernel(cuda, orac
 
 
 @pytest.mark.parametrize("rows,prologue", [(3, "plain"), (4, "plain"), (3, "swiglu"), (4, "gated")])
-@pytest.mark.parametrize("in_dim", [256, 6144, 12544])
+@pytest.mark.parametrize("in_dim", [256, 8192, 8448, 12544])
 @pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q8_0])
 def test_small_batches_on_the_exact_verifiers_kernel(cuda, oracle, encoding, in_dim, rows, prologue):
     """Small batches that the verifier's matrix-core kernel takes from the other family: row for row the
-    verifier family's bits, whether alone or beside a projection of another format."""
+    verifier family's bits, whether alone or beside a projection of another format, the prologue fused
+    or materialised."""
     weights = [tile_ops.PackedWeight.from_numpy(e, random_packed(e, n, in_dim, 94 + n), n, in_dim)
                for e, n in ((encoding, 77), (kquant.Q6_K, 20))]
     x, second = (to_device(kquant.synthetic_activations(seed, rows, in_dim), cuda) for seed in (95, 96))
@@ -881,9 +896,12 @@ def test_small_batches_on_the_exact_verifiers_kernel(cuda, oracle, encoding, in_
     alone = tile_ops.multi_linear(weights[:1], x, workspace, **arguments)[0]
     both = tile_ops.multi_linear(weights, x, workspace, **arguments)
     assert_bits_equal(both[0], alone, "beside another format")
-    if in_dim > 12288 or (in_dim >= 6144 if encoding == kquant.Q8_0 else prologue != "plain"):
+    if in_dim > 8192 or encoding == kquant.Q8_0:
         assert_bits_equal(alone, exact[0], "the verifier's rows")
     assert normalised_error(both[1].cpu().numpy(), exact[1].cpu().numpy()) <= TOLERANCE
+    if prologue != "plain":
+        applied = tile_ops.sigmoid_gate(x, second) if prologue == "gated" else tile_ops.swiglu(x, second)
+        assert_bits_equal(tile_ops.multi_linear(weights[:1], applied, workspace)[0], alone, "materialised")
 
 
 @pytest.mark.parametrize("in_dim", [4096, 4352, 6656])
