@@ -90,7 +90,8 @@ int nfn_native_tile_packed_weight_dequantize_float32_v1(
 /* ---- generic float-activation linear, any row count (tile_ops.h:614-620):
  *      float weights times float activations, no quantization of the input.
  *      It has no workspace argument, so every row count keeps that float
- *      arithmetic (four rows and more on the bf16 matrix instruction, the floats cut into exact terms);
+ *      arithmetic (four rows and more on the bf16 matrix instruction, the floats cut into exact terms,
+ *      unless the outputs are few);
  *      nfn_mi355_k_quant_gemm_float32_v1 is the fp16 matrix-core route.
  *      The order of the float sums belongs to the kernel: a row's bits are the same whichever other
  *      rows come with it among one to three rows (as many as fit LDS: 160 KB, 272 bytes for 64
@@ -141,8 +142,10 @@ int nfn_native_tile_linear_packed_weight_q8_1_multi_decode_float32_v1(
 /* ---- decode / small-batch K-quant path (tile_ops.h:647-739) --------------
  * 1..4 projections that share one input, rows 1..16, Q4_K/Q5_K/Q6_K (and
  * Q8_0 here).  `workspace` is caller-owned scratch whose layout is private to
- * this library; its size comes from the query.  The query returns 0 when rows
- * is outside 1..16 or input_dim is not a multiple of 128. */
+ * this library; its size comes from the query.  (Two and three rows are also
+ * served from what their activation records alone take, by the kernel that
+ * needs no more: the same bits in the verifier family and at two rows, to
+ * rounding at three rows of the other.)  The query returns 0 when rows is outside 1..16 or input_dim is not a multiple of 128. */
 int64_t nfn_native_tile_k_quant_mmq_workspace_bytes_v1(int64_t rows, int64_t input_dim);
 int nfn_native_tile_k_quant_mmq_multi_linear_float32_v1(
     const NfnNativeTilePackedWeightDescriptorV1* const* descriptors,
@@ -1016,7 +1019,8 @@ int nfn_mi355_fused_decode_attention_split_device_position_v1(
  * of every query row are shared out over workgroups like those of the
  * one-token split form (as many shares as the workspace has room for,
  * query_rows * query_heads * (head_dim + 2) floats each; with room for fewer
- * than two the ordinary form runs).  Same descriptor, same semantics and
+ * than two, or keys that one workgroup a row takes in less time, they are not).
+ * Same descriptor, same semantics and
  * tolerance; the bits can differ from the ordinary entry point.  The workspace
  * of the one-token form is a good size for blocks of up to 16 rows. */
 int nfn_mi355_dflash_block_attention_split_v1(

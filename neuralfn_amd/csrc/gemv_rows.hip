@@ -1,4 +1,4 @@
-// Verifier rows (4..16 tokens) of K-quant projections on the int8 matrix cores, every row in
+// Verifier rows (4..16 tokens; two and three where that is faster) of K-quant projections on the int8 matrix cores, every row in
 // the one-row kernel's arithmetic bit for bit.
 //
 // The contract (neuralfn/csrc/native_train/tile_ops.h:685-688; the reference's kernel:

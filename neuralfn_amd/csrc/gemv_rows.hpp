@@ -71,7 +71,7 @@ void launch_quantize_records(const float* first, const float* second, int prolog
                              std::int64_t rows, std::int64_t input_dim, std::uint8_t* records,
                              std::uint8_t* image, const ProjectionSet& clear, hipStream_t stream);
 
-// rows 4..16 of the set's projections from the operand image and the records beside it.
+// rows 2..16 of the set's projections from the operand image and the records beside it.
 // outputs_cleared: the outputs of
 // gemv_rows_split_set(set, rows, fill_launch) hold -0.0f (launch_quantize_records or
 // launch_fill_outputs ran with that set).
