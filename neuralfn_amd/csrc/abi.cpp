@@ -824,10 +824,8 @@ bool lm_head_half_form(const nfn::Descriptor& weight, std::int64_t rows) {
         weight.output_dim <= std::numeric_limits<std::int32_t>::max() &&
         nfn::gemv_f16_supports(weight.encoding, weight.input_dim);
 }
-}  // namespace
-
-std::int64_t nfn_mi355_lm_head_argmax_workspace_bytes_v1(std::int64_t rows,
-                                                         std::int64_t output_dim) {
+// The least workspace that a call takes.
+std::int64_t lm_head_required_bytes(std::int64_t rows, std::int64_t output_dim) {
     if (rows < 1 || rows > 16 || output_dim <= 0) return 0;
     std::int64_t raw = 0;
     if (rows <= kLmHeadOtherRows) {
@@ -842,6 +840,16 @@ std::int64_t nfn_mi355_lm_head_argmax_workspace_bytes_v1(std::int64_t rows,
     }
     return (raw + 255) & ~std::int64_t(255);
 }
+}  // namespace
+
+std::int64_t nfn_mi355_lm_head_argmax_workspace_bytes_v1(std::int64_t rows,
+                                                         std::int64_t output_dim) {
+    const std::int64_t required = lm_head_required_bytes(rows, output_dim);
+    if (rows != 1 || required == 0) return required;
+    // ... with room for every workgroup that one row can be spread over (small vocabularies)
+    const std::int64_t raw = lm_head_row_groups(output_dim) * static_cast<std::int64_t>(sizeof(LmHeadCandidate));
+    return std::max(required, (raw + 255) & ~std::int64_t(255));
+}
 
 int nfn_mi355_lm_head_argmax_v1(const Descriptor* descriptor, const float* input,
                                 std::int64_t* output_indices, float* output_values,
@@ -853,8 +861,7 @@ int nfn_mi355_lm_head_argmax_v1(const Descriptor* descriptor, const float* input
         (normalized.cuda_stream != nullptr && normalized.cuda_stream != cuda_stream)) {
         return kInvalid;
     }
-    const std::int64_t required =
-        nfn_mi355_lm_head_argmax_workspace_bytes_v1(rows, normalized.output_dim);
+    const std::int64_t required = lm_head_required_bytes(rows, normalized.output_dim);
     if (required == 0 || workspace_nbytes < required) return kInvalid;
     // Five rows and more (Q6_K: two): the fp16 matrix-core kernel (one pass over the weights
     // for up to sixteen rows), the only form beyond eight rows.  Two rows and more: the int8
@@ -873,6 +880,7 @@ int nfn_mi355_lm_head_argmax_v1(const Descriptor* descriptor, const float* input
                           output_indices, output_values, as_stream(cuda_stream));
     } else {
         launch_lm_head_f32(normalized, input, rows, static_cast<LmHeadCandidate*>(workspace),
+                           workspace_nbytes / static_cast<std::int64_t>(sizeof(LmHeadCandidate)),
                            output_indices, output_values, as_stream(cuda_stream));
     }
     return launch_status();

@@ -164,10 +164,22 @@ std::int64_t lm_head_f32_blocks(std::int64_t output_dim) {
     // 16 vocabulary rows per wave, 64 per workgroup.
     return (output_dim + 63) / 64;
 }
-// (the one-row kernel's workgroups are one to 16 vocabulary rows at least: lm_head_mfma_tiles() of room)
+// Workgroups of the one-row kernel, given room for their candidates (its sums and its choice do not hang on
+// their number).  A vocabulary of up to two pairs of rows a wave at three workgroups a unit is spread over as
+// many workgroups as that takes (64 rows each would leave most units idle, or waves with four pairs
+// where others have none to hide behind): 4,608 -> 4,000 / 9,000 / 16,000 rows of Q4_K 24.4 / 24.4 / 25.2 ->
+// 11.3 / 19.1 / 22.8 us; 30,000 would take 39.3 instead of 37.0.
+std::int64_t lm_head_row_groups(std::int64_t output_dim) {
+    const std::int64_t resident = 2 * std::int64_t(compute_units());
+    const std::int64_t pairs = (output_dim + kExactPair - 1) / kExactPair;
+    const std::int64_t turns = (pairs + 12 * resident - 1) / (12 * resident);  // of eight waves, three a unit
+    if (turns <= 2) return (pairs + kExactWaves * turns - 1) / (kExactWaves * turns);
+    const std::int64_t blocks = lm_head_f32_blocks(output_dim);
+    return blocks < resident ? blocks : resident;
+}
 
 void launch_lm_head_f32(const Descriptor& descriptor, const float* input, std::int64_t rows,
-                        LmHeadCandidate* candidates, std::int64_t* indices, float* maxima,
+                        LmHeadCandidate* candidates, std::int64_t room, std::int64_t* indices, float* maxima,
                         hipStream_t stream) {
     Projection op{};
     op.data = descriptor.data;
@@ -179,15 +191,8 @@ void launch_lm_head_f32(const Descriptor& descriptor, const float* input, std::i
     // (two workgroups a compute unit; the row and the kernel's own few words have to fit LDS)
     if (rows == 1 && descriptor.input_dim % 64 == 0 &&
         exact_rows_lds(1, descriptor.input_dim) <= 159 * 1024) {
-        const std::int64_t resident = 2 * std::int64_t(compute_units());
-        std::int64_t groups = blocks < resident ? blocks : resident;
-        // A vocabulary of up to two pairs of rows a wave at three workgroups a unit is spread over as many
-        // workgroups as that takes (64 rows each would leave most units idle, or waves with four pairs
-        // where others have none to hide behind): 4,608 -> 4,000 / 9,000 / 16,000 rows of Q4_K 24.4 / 24.4 / 25.2 ->
-        // 11.3 / 19.1 / 22.8 us; 30,000 would take 39.3 instead of 37.0.
-        const std::int64_t pairs = (descriptor.output_dim + kExactPair - 1) / kExactPair;
-        const std::int64_t turns = (pairs + 12 * resident - 1) / (12 * resident);  // of eight waves, three a unit
-        if (turns <= 2) groups = (pairs + kExactWaves * turns - 1) / (kExactWaves * turns);
+        std::int64_t groups = lm_head_row_groups(descriptor.output_dim);
+        if (groups > room) groups = room;
         bool launched = true;
         switch (descriptor.encoding) {
             case kEncQ4K: launch_row<kEncQ4K>(op, descriptor.input_dim, input, candidates, groups, stream); break;

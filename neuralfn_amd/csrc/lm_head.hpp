@@ -29,8 +29,11 @@ void launch_lm_head_final(const LmHeadCandidate* candidates, std::int64_t candid
                           hipStream_t stream);
 
 std::int64_t lm_head_f32_blocks(std::int64_t output_dim);
+// workgroups of one row (each leaves a candidate) where `room` holds as many
+std::int64_t lm_head_row_groups(std::int64_t output_dim);
+// room: candidates that fit the workspace, lm_head_f32_blocks() a row at least
 void launch_lm_head_f32(const Descriptor& descriptor, const float* input, std::int64_t rows,
-                        LmHeadCandidate* candidates, std::int64_t* indices, float* maxima,
+                        LmHeadCandidate* candidates, std::int64_t room, std::int64_t* indices, float* maxima,
                         hipStream_t stream);
 
 }  // namespace nfn

@@ -1081,6 +1081,36 @@ def test_lm_head_fused_argmax_against_oracle(cuda, oracle, encoding, rows):
             assert logits[row, indices.cpu()[row].item()] >= ordered[0] - 2 * TOLERANCE * scale
 
 
+@pytest.mark.parametrize("out_dim", [33, 4096, 4097, 8192, 9001, 12288, 12289, 24576, 24577])
+@pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q8_0])
+def test_lm_head_one_row_leaves_what_lies_behind_its_workspace(cuda, encoding, out_dim):
+    """Small vocabularies are spread over more workgroups, each of which leaves a candidate: with the query's
+    workspace and with less nothing behind it is written, and the choice is that of the logits."""
+    in_dim, lib = 256, tile_ops.load()
+    packed = torch_().from_numpy(random_packed(encoding, 64, in_dim, 97).reshape(64, -1)).to(cuda)
+    chosen = torch_().from_numpy(np.random.default_rng(98).integers(0, 63, out_dim)).to(cuda)
+    chosen[out_dim - 1] = 63
+    weight = tile_ops.PackedWeight(encoding, out_dim, in_dim, packed.index_select(0, chosen).reshape(-1))
+    x = to_device(kquant.synthetic_activations(99, 1, in_dim), cuda)
+    logits = tile_ops.linear(weight, x)[0].cpu().numpy()
+    asked = lib.nfn_mi355_lm_head_argmax_workspace_bytes_v1(1, out_dim)
+    assert asked >= (out_dim + 31) // 32 * 16
+    for nbytes in (asked, asked - 16, asked - 256):
+        workspace = torch_().full((asked + 65536,), 0x5a, dtype=torch_().uint8, device=cuda)
+        indices, maxima = (torch_().zeros(1, dtype=d, device=cuda) for d in (torch_().int64, torch_().float32))
+        descriptor = weight.descriptor()
+        status = lib.nfn_mi355_lm_head_argmax_v1(ctypes.byref(descriptor), x.data_ptr(), indices.data_ptr(),
+                                                 maxima.data_ptr(), 1, workspace.data_ptr(), nbytes, None)
+        torch_().cuda.synchronize()
+        assert bool((workspace[nbytes:] == 0x5a).all())
+        if nbytes == asked:
+            assert status == 0
+        if status == 0:
+            best = logits.max()
+            assert abs(maxima.item() - best) <= 1e-5 * np.abs(logits).max()
+            assert logits[indices.item()] >= best - 2e-5 * np.abs(logits).max()
+
+
 @pytest.mark.parametrize("rows", [1, 2, 5, 16])
 def test_lm_head_fused_argmax_tie_goes_to_lowest_index(cuda, rows):
     # Identical vocabulary rows, two in one 32-row tile and one far away: the
