@@ -1336,8 +1336,7 @@ struct TileChoice {
     double cost;
 };
 TileChoice cheapest_tile(const TileCost (&tiles_of)[3], const std::int64_t* output_dims, const int* shares, int count,
-                         std::int64_t rows, std::int64_t input_dim, double extra) {
-    const std::int64_t units = compute_units();
+                         std::int64_t rows, std::int64_t input_dim, double extra, std::int64_t units) {
     TileChoice best{0, 0};
     for (const TileCost& tile : tiles_of) {
         const std::int64_t m_tiles = (rows + tile.rows - 1) / tile.rows;
@@ -1365,7 +1364,7 @@ TileChoice cheapest_tile(const TileCost (&tiles_of)[3], const std::int64_t* outp
 
 template <std::uint32_t ENC>
 int tile_height(const GemmGroup& group, int count, std::int64_t rows, std::int64_t input_dim) {
-    return cheapest_tile(kTileCosts<ENC>, group.output_dim, group.shares, count, rows, input_dim, 0.2).rows;
+    return cheapest_tile(kTileCosts<ENC>, group.output_dim, group.shares, count, rows, input_dim, 0.2, compute_units()).rows;
 }
 
 // K shares beyond those of plan(), where the workspace has room for them (gemm_f16_workspace_bytes asks for
@@ -1383,27 +1382,34 @@ int tile_height(const GemmGroup& group, int count, std::int64_t rows, std::int64
 // query, which knows none, need not ask for four.
 int shares_with_room(const Plan& least, std::int64_t rows, std::int64_t output_dim, std::int64_t input_dim) {
     const std::int64_t n_tiles = (output_dim + kBN - 1) / kBN;
-    if (rows <= kLowRows || rows > kMostCutRows || n_tiles < kLeastCutTiles || (rows + 255) / 256 * n_tiles >= compute_units()) return least.shares;
+    if (rows <= kLowRows || rows > kMostCutRows || n_tiles < kLeastCutTiles) return least.shares;
+    const std::int64_t units = compute_units();
+    if ((rows + 255) / 256 * n_tiles >= units) return least.shares;
     // (the same for every count up to the next multiple of 128: what gemm_f16_workspace_bytes relies on)
     const std::int64_t counted = (rows + 127) / 128 * 128;
     const auto cost = [&](int shares, int quarters) {
         const std::int64_t outputs = quarters * n_tiles * kBN / 4;
         const double sums = shares == 1 ? 0.0 : 3.0 + 1.6e-6 * static_cast<double>((shares + 1) * counted * outputs);
-        return cheapest_tile(kTileCosts<kEncQ4K>, &outputs, &shares, 1, counted, input_dim, 0.0).cost + sums;
+        return cheapest_tile(kTileCosts<kEncQ4K>, &outputs, &shares, 1, counted, input_dim, 0.0, units).cost + sums;
     };
-    constexpr int kBeside[4] = {4, 8, 9, 10};  // quarters of the outputs: alone, with another, ...
-    double least_cost[4];
-    for (int i = 0; i < 4; ++i) least_cost[i] = cost(least.shares, kBeside[i]);
+    // quarters of the outputs: alone, with another, ...  (The host pays for this in every call and several
+    // times in a query, so what saves too little by itself goes no further: queries of 333 / 2,048 rows into
+    // 6,656 outputs 17 / 31 -> 3 / 5 us.)
+    constexpr int kBeside[4] = {4, 8, 9, 10};
+    double least_cost[4] = {cost(least.shares, kBeside[0])};
     int best = least.shares;
     double best_saved = 1.0;
     for (const int shares : {2, 3, 4, 6, 8}) {
         if (shares <= least.shares || 2 * shares > (input_dim >> 8)) continue;
-        double saved = 1.0;
-        for (int i = 0; i < 4; ++i) {
+        double saved = cost(shares, kBeside[0]) / least_cost[0];
+        bool pays = saved < 0.94;
+        for (int i = 1; i < 4 && pays; ++i) {
+            if (least_cost[i] == 0) least_cost[i] = cost(least.shares, kBeside[i]);
             const double here = cost(shares, kBeside[i]) / least_cost[i];
-            saved *= here < (i == 0 ? 0.94 : 1.0) ? here : 2.0;
+            pays = here < 1.0;
+            saved *= here;
         }
-        if (saved < best_saved) {
+        if (pays && saved < best_saved) {
             best = shares;
             best_saved = saved;
         }
@@ -1480,10 +1486,10 @@ std::int64_t partial_floats(int shares, std::int64_t rows, std::int64_t output_d
 // ... of the shares that a call with room for them takes, whatever the encoding (plan() gives Q4_K the most,
 // and with as many or more the other encodings take none that it does not)
 std::int64_t most_partial_floats(std::int64_t rows, std::int64_t output_dim, std::int64_t input_dim) {
-    std::int64_t most = 0;
-    for (const std::uint32_t encoding : {kEncQ4K, kEncQ6K}) {
-        const int shares = shares_with_room(plan(encoding, rows, output_dim, input_dim), rows, output_dim, input_dim);
-        most = std::max(most, partial_floats(shares, rows, output_dim));
+    const Plan q4 = plan(kEncQ4K, rows, output_dim, input_dim), q6 = plan(kEncQ6K, rows, output_dim, input_dim);
+    std::int64_t most = partial_floats(shares_with_room(q4, rows, output_dim, input_dim), rows, output_dim);
+    if (q6.shares != q4.shares) {
+        most = std::max(most, partial_floats(shares_with_room(q6, rows, output_dim, input_dim), rows, output_dim));
     }
     return most;
 }
