@@ -26,15 +26,18 @@ std::int64_t rows_chosen_for(std::int64_t rows) { return rows > kMostRows && row
 
 constexpr std::int64_t kMaxDenseLds = 159 * 1024;  // beside the waves' meeting place
 
-// GROUPS: more than R rows, R of them (of the last group those that exist) a workgroup of blockIdx.y.
-// (A form of its own: the checks cost the call of up to three rows 3 %.)
-template <std::uint32_t ENC, int R, bool GROUPS>
+// GROUPS: of more than R rows, R (of the last group those that exist) a workgroup of blockIdx.y.
+// Rows is empty or the row count's int: more than R rows.
+// (A form of its own: the checks cost the call of up to three rows 3 %, and the argument alone as much, because
+// it moves the grid's size, which a wave reads before its first pair, to a second line of arguments.)
+template <std::uint32_t ENC, int R, typename... Rows>
 __global__ __launch_bounds__(kExactWaves * kWave) void linear_rows_kernel(
     const std::uint8_t* __restrict__ data, std::int64_t row_stride, const float* __restrict__ input,
     const float* __restrict__ bias, float* __restrict__ output, std::int64_t input_dim, std::int64_t output_dim,
-    int rows) {
+    Rows... rows) {
+    constexpr bool GROUPS = sizeof...(Rows) > 0;
     extern __shared__ __attribute__((aligned(16))) float staged[];
-    const int row0 = GROUPS ? static_cast<int>(blockIdx.y) * R : 0, there = GROUPS ? min(R, rows - row0) : R;
+    const int row0 = GROUPS ? static_cast<int>(blockIdx.y) * R : 0, there = min(R, (rows + ... + (GROUPS ? 0 : R)) - row0);
     input += row0 * input_dim;
     output += row0 * output_dim;
     exact_rows_stage<R, GROUPS>(input, input_dim, staged, there);
@@ -63,20 +66,19 @@ void launch_rows(const Descriptor& weight, const float* input, const float* bias
     const std::int64_t most = (pairs + kExactWaves - 1) / kExactWaves;
     const std::int64_t turns = (most + resident - 1) / resident;
     const std::int64_t groups = (most + turns - 1) / turns;
-    const auto launch = [&](auto kernel) {
+    const auto launch = [&](auto kernel, auto... count) {
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups), static_cast<unsigned>((rows + R - 1) / R)),
                            dim3(kExactWaves * kWave), static_cast<unsigned>(lds), stream, weight.data,
-                           weight.row_stride_bytes, input, bias, output, weight.input_dim, weight.output_dim,
-                           static_cast<int>(rows));
+                           weight.row_stride_bytes, input, bias, output, weight.input_dim, weight.output_dim, count...);
     };
     if constexpr (R > 1) {
         if (rows > R) {
-            allow_large_lds<linear_rows_kernel<ENC, R, true>>();
-            return launch(linear_rows_kernel<ENC, R, true>);
+            allow_large_lds<linear_rows_kernel<ENC, R, int>>();
+            return launch(linear_rows_kernel<ENC, R, int>, static_cast<int>(rows));
         }
     }
-    allow_large_lds<linear_rows_kernel<ENC, R, false>>();
-    launch(linear_rows_kernel<ENC, R, false>);
+    allow_large_lds<linear_rows_kernel<ENC, R>>();
+    launch(linear_rows_kernel<ENC, R>);
 }
 
 // Float and bf16 weights: a wave (SPLIT = 1) or the workgroup's eight waves together (SPLIT = 8, for
@@ -84,17 +86,18 @@ void launch_rows(const Descriptor& weight, const float* input, const float* bias
 // next turn's requested before this one's are used.  Bound by the weight stream.
 typedef std::uint32_t dense_u32x4 __attribute__((ext_vector_type(4), aligned(2)));
 
-template <std::uint32_t ENC, int R, int SPLIT, bool GROUPS>
+template <std::uint32_t ENC, int R, int SPLIT, typename... Rows>
 __global__ __launch_bounds__(kExactWaves * kWave) void dense_rows_kernel(
     const std::uint8_t* __restrict__ data, std::int64_t row_stride, const float* __restrict__ input,
     const float* __restrict__ bias, float* __restrict__ output, std::int64_t input_dim, std::int64_t output_dim,
-    int rows) {
+    Rows... rows) {
+    constexpr bool GROUPS = sizeof...(Rows) > 0;
     constexpr int kValues = ENC == kEncF32 ? 4 : 8;  // of 16 bytes
     extern __shared__ __attribute__((aligned(16))) float staged[];
     __shared__ float meeting[kExactWaves][kExactPair * R];
     typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
     const int columns = static_cast<int>(input_dim);
-    const int row0 = GROUPS ? static_cast<int>(blockIdx.y) * R : 0, there = GROUPS ? min(R, rows - row0) : R;
+    const int row0 = GROUPS ? static_cast<int>(blockIdx.y) * R : 0, there = min(R, (rows + ... + (GROUPS ? 0 : R)) - row0);
     input += row0 * input_dim;
     output += row0 * output_dim;
     for (int index = threadIdx.x * 4; index < R * columns; index += kExactWaves * kWave * 4) {
@@ -218,25 +221,24 @@ void launch_dense(const Descriptor& weight, const float* input, const float* bia
     const std::int64_t most = split ? pairs : (pairs + kExactWaves - 1) / kExactWaves;
     const unsigned groups = static_cast<unsigned>(most < resident ? most : resident);
     const unsigned row_groups = static_cast<unsigned>((rows + R - 1) / R);
-    const auto launch = [&](auto kernel) {
+    const auto launch = [&](auto kernel, auto... count) {
         hipLaunchKernelGGL(kernel, dim3(groups, row_groups), dim3(kExactWaves * kWave), static_cast<unsigned>(lds), stream,
                            weight.data, weight.row_stride_bytes, input, bias, output, weight.input_dim,
-                           weight.output_dim, static_cast<int>(rows));
+                           weight.output_dim, count...);
     };
-    const auto form = [&](auto grouped) {
-        constexpr bool kGroups = decltype(grouped)::value;
+    const auto form = [&](auto... count) {
         if (split) {
-            allow_large_lds<dense_rows_kernel<ENC, R, kExactWaves, kGroups>>(kMaxDenseLds);
-            launch(dense_rows_kernel<ENC, R, kExactWaves, kGroups>);
+            allow_large_lds<dense_rows_kernel<ENC, R, kExactWaves, decltype(count)...>>(kMaxDenseLds);
+            launch(dense_rows_kernel<ENC, R, kExactWaves, decltype(count)...>, count...);
         } else {
-            allow_large_lds<dense_rows_kernel<ENC, R, 1, kGroups>>(kMaxDenseLds);
-            launch(dense_rows_kernel<ENC, R, 1, kGroups>);
+            allow_large_lds<dense_rows_kernel<ENC, R, 1, decltype(count)...>>(kMaxDenseLds);
+            launch(dense_rows_kernel<ENC, R, 1, decltype(count)...>, count...);
         }
     };
     if constexpr (R > 1) {
-        if (rows > R) return form(std::true_type{});
+        if (rows > R) return form(static_cast<int>(rows));
     }
-    form(std::false_type{});
+    form();
 }
 
 template <std::uint32_t ENC>
