@@ -143,9 +143,11 @@ int nfn_native_tile_linear_packed_weight_q8_1_multi_decode_float32_v1(
  * 1..4 projections that share one input, rows 1..16, Q4_K/Q5_K/Q6_K (and
  * Q8_0 here).  `workspace` is caller-owned scratch whose layout is private to
  * this library; its size comes from the query.  (Two and three rows are also
- * served from what their activation records alone take, by the kernel that
- * needs no more: the same bits in the verifier family and at two rows, to
- * rounding at three rows of the other.)  The query returns 0 when rows is outside 1..16 or input_dim is not a multiple of 128. */
+ * served from what their activation records alone take, with the same bits.)
+ * The first group of calls, the mmq_* ones, writes nothing into it at one and two
+ * rows, so that records of a verifier call (below) survive them; from three rows
+ * on they may overwrite it.  The query returns 0 when rows is outside 1..16 or
+ * input_dim is not a multiple of 128. */
 int64_t nfn_native_tile_k_quant_mmq_workspace_bytes_v1(int64_t rows, int64_t input_dim);
 int nfn_native_tile_k_quant_mmq_multi_linear_float32_v1(
     const NfnNativeTilePackedWeightDescriptorV1* const* descriptors,

@@ -80,33 +80,28 @@ Projection make_projection(const Descriptor& descriptor, float* output) {
     return op;
 }
 
-// Whether a projection runs on the exact verifier's matrix-core kernel behind its quantizer launch
-// (gemv_rows.hip) where that is a question of time: the verifier family takes it from four rows on, and the
-// one-row arithmetic of two and three rows has the same bits on either kernel.  Two launches that
-// read the activations once, against one in which every workgroup makes their codes (and a prologue's
-// functions) for itself; K: input_dim.  Times of the call before -> with it, us, one box, weights from memory.
-//   Three rows of the verifier family: K-Quants always (2,048 -> 6,144 of Q4_K 9.3 -> 7.0, 7,936 -> 39,936 76 -> 43,
-//     Q6_K 132 -> 68, SwiGLU 16,384 -> 6,656 of Q4_K 37 -> 21); Q8_0 gains from long rows or many outputs
-//     (16,384 -> 6,656 34 -> 30, 4,096 -> 32,768 35 -> 32; 4,096 -> 6,656 would lose, 12.4 -> 13.1).
+// Whether two or three rows of the verifier family run on its matrix-core kernel behind a quantizer launch
+// (gemv_rows.hip), as from four rows on, or on the dot kernels: the same bits on either, a question of time.
+// Two launches that read the activations once, against one in which every workgroup makes their codes (and a
+// prologue's functions) for itself; K: input_dim.  Times of the call before -> with it, us, one box, weights from
+// memory.
+//   Three rows: K-Quants always (2,048 -> 6,144 of Q4_K 9.3 -> 7.0, 7,936 -> 39,936 76 -> 43, Q6_K 132 -> 68, SwiGLU
+//     16,384 -> 6,656 of Q4_K 37 -> 21); Q8_0 gains from long rows or many outputs (16,384 -> 6,656 34 -> 30, 4,096 ->
+//     32,768 35 -> 32; 4,096 -> 6,656 would lose, 12.4 -> 13.1).
 //   Two rows: K above 12,288 (SwiGLU 18,432 -> 2,304 21 -> 14, 16,384 -> 6,656 of Q6_K 38 -> 33) or, Q4_K and Q5_K, many
 //     outputs (4,096 -> 16,384 twice 25 -> 22); 6,656 -> 8,704 would lose, 13.4 -> 15.2.
-//   Three and four rows of the other family, Q4_K and Q5_K: K above 8,192, whatever the prologue (a fused prologue has
-//     the bits of the materialised one): SwiGLU 18,432 -> 2,304 34 -> 14, 11,776 -> 4,352 25 -> 16, plain 16,384 -> 4,096
-//     20.5 -> 15.0.  Shorter rows would gain behind a prologue (gated 6,144 -> 4,352 15 -> 10) and lose plain (5,376 ->
-//     6,656 10 -> 11, 4,096 -> 16,384 twice 20 -> 22).  Q8_0, whose bits are the one-row kernel's on either: four rows of
-//     4,096 columns and more (16,384 -> 6,656 38 -> 30), three of 6,144 or many outputs.
-bool rows_kernel_pays(bool verifier, std::uint32_t encoding, int prologue, std::int64_t rows,
-                      std::int64_t output_dim, std::int64_t input_dim) {
+// The other family stays on its own kernels, although they take longer for some shapes (SwiGLU 18,432 -> 2,304 of Q4_K,
+// three rows, 34 us and not 14): the quantizer launch would overwrite activation records that a verifier call left in
+// the workspace, and at three and four rows the results would not be the logits that the fused lm_head takes its
+// maximum of.
+bool rows_kernel_pays(std::uint32_t encoding, int prologue, std::int64_t rows, std::int64_t output_dim,
+                      std::int64_t input_dim) {
     constexpr std::int64_t kLongRows = 12288, kManyOutputs = 12288;
-    if (prologue == kRecords || prologue == kHalfImage || rows < 2) return false;
+    if (prologue == kRecords || rows < 2) return false;
     const bool q45 = encoding == kEncQ4K || encoding == kEncQ5K;
     const bool q8 = encoding == kEncQ8_0;
     if (rows == 2) return (!q8 && input_dim > kLongRows) || (q45 && output_dim >= kManyOutputs);
-    const bool q8_three = input_dim >= 6144 || output_dim >= kManyOutputs;
-    if (verifier) return !q8 || q8_three;
-    if (rows > 4) return false;
-    if (q8) return rows == 4 ? input_dim >= 4096 : q8_three;
-    return q45 && input_dim > 8192;
+    return !q8 || input_dim >= 6144 || output_dim >= kManyOutputs;
 }
 
 // Shared body of the small-batch entry points.
@@ -133,9 +128,9 @@ int run_small_batch(bool verifier, const Descriptor* const* descriptors, const f
     }
     const std::int64_t required = small_batch_workspace_bytes(rows, input_dim);
     if (required == 0 || workspace_nbytes < required) return kInvalid;
-    // The exact verifier's matrix-core kernel: that family from four rows on, and where it is the faster
-    // one (rows_kernel_pays).  Else one or two rows, and the verifier entry points at any row count: the
-    // vector-ALU kernels.  Otherwise 3 and 4 rows: the int8 matrix-core kernel,
+    // The verifier entry points: their matrix-core kernel from four rows on and where it is the faster one
+    // (rows_kernel_pays), else, and for one or two rows of the other family, the vector-ALU kernels.
+    // Otherwise 3 and 4 rows: the int8 matrix-core kernel,
     // which quantizes inside the kernel; 5..16 rows (Q6_K: 3..16): the fp16 matrix-core kernel
     // behind its conversion launch (Q8_0 below five rows: its dot kernel).
     // Encodings and widths without either: the float kernel.
@@ -144,14 +139,14 @@ int run_small_batch(bool verifier, const Descriptor* const* descriptors, const f
     const bool one_row_arithmetic = rows <= 2 || verifier;
     const bool always_rows = verifier && rows >= kFirstVerifierMatrixRows;
     // (two and three rows are served without the room as well)
-    const bool room = rows >= 2 && workspace_nbytes >= small_batch_workspace_bytes(rows, input_dim, true);
+    const bool room = verifier && workspace_nbytes >= small_batch_workspace_bytes(rows, input_dim, true);
     ProjectionSet dot{}, dot6{}, dot8{}, matrix{}, half{}, exact{}, verifier_rows{};
     dot.input_dim = dot6.input_dim = dot8.input_dim = matrix.input_dim = half.input_dim =
         exact.input_dim = verifier_rows.input_dim = input_dim;
     for (int index = 0; index < set.count; ++index) {
         const std::uint32_t encoding = set.op[index].encoding;
         ProjectionSet* target = &exact;
-        if ((always_rows || (room && rows_kernel_pays(verifier, encoding, prologue, rows, set.op[index].output_dim, input_dim))) &&
+        if ((always_rows || (room && rows_kernel_pays(encoding, prologue, rows, set.op[index].output_dim, input_dim))) &&
             gemv_rows_supports(encoding, input_dim)) {
             target = &verifier_rows;
         } else if (one_row_arithmetic && gemv_dot_supports(encoding, input_dim)) {
@@ -210,12 +205,10 @@ int run_small_batch(bool verifier, const Descriptor* const* descriptors, const f
         if (verifier_rows.count > 0) {
             launch_gemv_rows(verifier_rows, image, static_cast<const std::uint8_t*>(workspace), rows, clear.count > 0, fill_launch, as_stream(stream));
         }
-        if (one_row_arithmetic) {  // (the others' kernels take the activations as they are)
-            dot_first = static_cast<const float*>(workspace);
-            dot_second = nullptr;
-            dot_prologue = kRecords;
-            records = nullptr;
-        }
+        dot_first = static_cast<const float*>(workspace);
+        dot_second = nullptr;
+        dot_prologue = kRecords;
+        records = nullptr;
     }
     if (dot.count > 0) {
         launch_gemv_dot(dot, dot_first, dot_second, records, dot_prologue, rows, as_stream(stream));

@@ -883,10 +883,9 @@ def test_two_and_three_rows_equal_the_one_row_kernel_on_either_kernel(cuda, orac
 @pytest.mark.parametrize("rows,prologue", [(3, "plain"), (4, "plain"), (3, "swiglu"), (4, "gated")])
 @pytest.mark.parametrize("in_dim", [256, 8192, 8448, 12544])
 @pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q8_0])
-def test_small_batches_on_the_exact_verifiers_kernel(cuda, oracle, encoding, in_dim, rows, prologue):
-    """Small batches that the verifier's matrix-core kernel takes from the other family: row for row the
-    verifier family's bits, whether alone or beside a projection of another format, the prologue fused
-    or materialised."""
+def test_small_batches_of_three_and_four_rows(cuda, oracle, encoding, in_dim, rows, prologue):
+    """Three and four rows of the other family: the same bits alone and beside a projection of another format,
+    the prologue fused or materialised; Q8_0 in the one-row arithmetic, the rest to rounding."""
     weights = [tile_ops.PackedWeight.from_numpy(e, random_packed(e, n, in_dim, 94 + n), n, in_dim)
                for e, n in ((encoding, 77), (kquant.Q6_K, 20))]
     x, second = (to_device(kquant.synthetic_activations(seed, rows, in_dim), cuda) for seed in (95, 96))
@@ -896,12 +895,54 @@ def test_small_batches_on_the_exact_verifiers_kernel(cuda, oracle, encoding, in_
     alone = tile_ops.multi_linear(weights[:1], x, workspace, **arguments)[0]
     both = tile_ops.multi_linear(weights, x, workspace, **arguments)
     assert_bits_equal(both[0], alone, "beside another format")
-    if in_dim > 8192 or encoding == kquant.Q8_0:
+    if encoding == kquant.Q8_0:
         assert_bits_equal(alone, exact[0], "the verifier's rows")
-    assert normalised_error(both[1].cpu().numpy(), exact[1].cpu().numpy()) <= TOLERANCE
+    for got, expected in zip(both, exact):
+        assert normalised_error(got.cpu().numpy(), expected.cpu().numpy()) <= TOLERANCE
     if prologue != "plain":
         applied = tile_ops.sigmoid_gate(x, second) if prologue == "gated" else tile_ops.swiglu(x, second)
         assert_bits_equal(tile_ops.multi_linear(weights[:1], applied, workspace)[0], alone, "materialised")
+
+
+@pytest.mark.parametrize("prologue", ["plain", "gated", "swiglu"])
+@pytest.mark.parametrize("encoding,rows,out_dim,in_dim", [
+    *((encoding, 2, out_dim, in_dim) for encoding in ALL_PACKED for out_dim, in_dim in ((77, 12544), (12289, 512))),
+    *((encoding, rows, 77, 8448) for encoding in (kquant.Q4_K, kquant.Q5_K, kquant.Q8_0) for rows in (3, 4)),
+    (kquant.Q8_0, 3, 12289, 512), (kquant.Q8_0, 4, 77, 4096),
+])
+def test_small_batches_leave_the_records_of_a_verifier_call(cuda, encoding, rows, out_dim, in_dim, prologue):
+    """The other family at two rows, and at three and four where it quantizes inside its kernels, writes nothing
+    into its workspace: records that a verifier call left there serve the prequantized call behind it."""
+    packed = torch_().from_numpy(random_packed(encoding, 64, in_dim, 86).reshape(64, -1)).to(cuda)
+    chosen = torch_().from_numpy(np.random.default_rng(87).integers(0, 64, out_dim)).to(cuda)
+    weight = tile_ops.PackedWeight(encoding, out_dim, in_dim, packed.index_select(0, chosen).reshape(-1))
+    x, other, second = (to_device(kquant.synthetic_activations(seed, rows, in_dim), cuda) for seed in (88, 89, 85))
+    workspace = tile_ops.small_batch_workspace(rows, in_dim)
+    expected = tile_ops.multi_linear([weight], x, workspace, family="mmvq")[0]
+    before = workspace.clone()
+    tile_ops.multi_linear([weight], other, workspace, **({} if prologue == "plain" else {"prologue": prologue, "second": second}))
+    assert bool((workspace == before).all())
+    after = tile_ops.multi_linear_prequantized([weight], rows, workspace, family="mmvq")[0]
+    assert_bits_equal(after, expected, "from the records")
+
+
+@pytest.mark.parametrize("rows", [3, 4])
+@pytest.mark.parametrize("in_dim", [8192, 8448])
+@pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K])
+def test_lm_head_of_three_and_four_rows_is_the_maximum_of_the_calls_logits(cuda, encoding, in_dim, rows):
+    """The fused choice and its value are those of the small-batch call's logits, bit for bit, on both sides
+    of the widths at which their kernels change."""
+    out_dim = 4133
+    packed = torch_().from_numpy(random_packed(encoding, 64, in_dim, 81).reshape(64, -1)).to(cuda)
+    chosen = torch_().from_numpy(np.random.default_rng(82).integers(0, 64, out_dim)).to(cuda)
+    weight = tile_ops.PackedWeight(encoding, out_dim, in_dim, packed.index_select(0, chosen).reshape(-1))
+    x = to_device(kquant.synthetic_activations(83, rows, in_dim), cuda)
+    logits = tile_ops.multi_linear([weight], x, tile_ops.small_batch_workspace(rows, in_dim))[0]
+    indices, values = tile_ops.lm_head_argmax(weight, x)
+    best = logits.max(dim=1)
+    assert_bits_equal(values.reshape(-1), best.values, "the largest logit")
+    for row in range(rows):
+        assert indices[row].item() == int((logits[row] == best.values[row]).nonzero()[0].item())
 
 
 @pytest.mark.parametrize("in_dim", [4096, 4352, 6656])
