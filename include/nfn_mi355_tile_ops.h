@@ -924,14 +924,14 @@ int nfn_mi355_k_quant_gemm_float32_v1(
     int mode,
     void* cuda_stream);
 
-/* How the call above cuts K for a problem of this geometry on the current device
- * (no counterpart in the reference; for tests and benchmarks): *tile_rows =
+/* The least that the call above cuts K into for a problem of this geometry on the
+ * current device (no counterpart in the reference; for tests and benchmarks): *tile_rows =
  * output rows per workgroup tile that the K shares are cut for (256 or 128; 32
  * for up to 32 rows; which tiles the launch takes says the query below),
  * *k_shares = workgroups that share the K range of a tile
  * (1 = unsplit; with more, each writes a partial output into the workspace and
  * a second launch adds them in share order; a call with more workspace than this
- * needs may take more, see above).  0 on success, 1 for an encoding
+ * needs may take more: nfn_mi355_k_quant_gemm_launch_v1 says how many).  0 on success, 1 for an encoding
  * or width the matrix-core path does not take, or the reserved mode. */
 int nfn_mi355_k_quant_gemm_plan_v1(
     uint32_t encoding,
@@ -945,11 +945,10 @@ int nfn_mi355_k_quant_gemm_plan_v1(
 /* Which launch form runs 1..4 projections of one encoding and input together (no
  * counterpart in the reference; for tests and benchmarks): *tile_rows = output
  * rows per workgroup tile, 512, 256 or 128, whichever costs least with the shares
- * above (sums do not depend on it); 32 for up to 32 rows.  The projections of a
- * call that do not find room for their shares beside each other run as several
- * launches, each of which has a height of its own.  0 on success, 1 for an
- * encoding, width or count the matrix-core path does not take, or the reserved
- * mode. */
+ * that they take (sums do not depend on it); 32 for up to 32 rows.  With the
+ * workspace of the query (several projections: of the multi query below); with
+ * less, see the next call.  0 on success, 1 for an encoding, width or count the
+ * matrix-core path does not take, or the reserved mode. */
 int nfn_mi355_k_quant_gemm_tile_rows_v1(
     uint32_t encoding,
     int64_t rows,
@@ -958,6 +957,23 @@ int nfn_mi355_k_quant_gemm_tile_rows_v1(
     int64_t operation_count,
     int mode,
     int* tile_rows);
+
+/* What such a call with a workspace of `workspace_nbytes` runs (no counterpart in
+ * the reference; for tests and benchmarks): for each of the projections,
+ * tile_rows[i] = output rows per workgroup tile of the launch that takes it (those
+ * that find no room for their shares beside the others' run in another) and
+ * k_shares[i] = its K shares.  0 on success, 1 as above or for a workspace that
+ * the call would refuse. */
+int nfn_mi355_k_quant_gemm_launch_v1(
+    uint32_t encoding,
+    int64_t rows,
+    int64_t input_dim,
+    const int64_t* output_dims,
+    int64_t operation_count,
+    int mode,
+    int64_t workspace_nbytes,
+    int* tile_rows,
+    int* k_shares);
 
 /* The same for 1..4 projections of one input (Q/K/V, gate/up), the way the
  * small-batch entry points group them: the activations are converted once and

@@ -899,17 +899,35 @@ int nfn_mi355_k_quant_gemm_plan_v1(std::uint32_t encoding, std::int64_t rows, st
     return 0;
 }
 
-int nfn_mi355_k_quant_gemm_tile_rows_v1(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
-                                        const std::int64_t* output_dims, std::int64_t operation_count, int mode,
-                                        int* tile_rows) {
-    if (tile_rows == nullptr || output_dims == nullptr || operation_count < 1 || operation_count > 4 || rows <= 0 ||
-        input_dim <= 0 || mode != NFN_MI355_GEMM_F16 || !gemm_f16_supports(encoding, input_dim)) {
+int nfn_mi355_k_quant_gemm_launch_v1(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
+                                     const std::int64_t* output_dims, std::int64_t operation_count, int mode,
+                                     std::int64_t workspace_nbytes, int* tile_rows, int* k_shares) {
+    if (tile_rows == nullptr || k_shares == nullptr || output_dims == nullptr || operation_count < 1 ||
+        operation_count > kMaxOperations || rows <= 0 || input_dim <= 0 || mode != NFN_MI355_GEMM_F16 ||
+        !gemm_f16_supports(encoding, input_dim)) {
         return kInvalid;
     }
     for (std::int64_t i = 0; i < operation_count; ++i) {
-        if (output_dims[i] <= 0) return kInvalid;
+        if (output_dims[i] <= 0 || workspace_nbytes < gemm_f16_required_bytes(rows, input_dim, output_dims[i])) {
+            return kInvalid;
+        }
     }
-    *tile_rows = gemm_f16_tile_rows(encoding, rows, input_dim, output_dims, static_cast<int>(operation_count));
+    gemm_f16_launches(encoding, rows, input_dim, output_dims, static_cast<int>(operation_count), workspace_nbytes,
+                      tile_rows, k_shares);
+    return 0;
+}
+
+int nfn_mi355_k_quant_gemm_tile_rows_v1(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
+                                        const std::int64_t* output_dims, std::int64_t operation_count, int mode,
+                                        int* tile_rows) {
+    int heights[kMaxOperations], shares[kMaxOperations];
+    // (room for everything that a call may take, as with the workspace of the query)
+    if (tile_rows == nullptr ||
+        nfn_mi355_k_quant_gemm_launch_v1(encoding, rows, input_dim, output_dims, operation_count, mode,
+                                         std::numeric_limits<std::int64_t>::max(), heights, shares) != 0) {
+        return kInvalid;
+    }
+    *tile_rows = heights[0];
     return 0;
 }
 

@@ -1494,6 +1494,38 @@ std::int64_t most_partial_floats(std::int64_t rows, std::int64_t output_dim, std
     return most;
 }
 
+// The launches of a call whose workspace has `room` floats behind the activations: each takes projections of
+// one encoding whose partial outputs find room beside each other.  launch(indexes, count, shares): the
+// projections of a launch; shares[i]: of projection i.  (The plan's shares where there is no room for more.)
+template <typename F>
+void for_each_launch(const std::uint32_t* encodings, const std::int64_t* output_dims, int count, std::int64_t rows,
+                     std::int64_t input_dim, std::int64_t room, F&& launch) {
+    int shares[kMaxProjections];
+    std::int64_t floats[kMaxProjections];
+    for (int i = 0; i < count; ++i) {
+        const Plan least = plan(encodings[i], rows, output_dims[i], input_dim);
+        shares[i] = shares_with_room(least, rows, output_dims[i], input_dim);
+        floats[i] = partial_floats(shares[i], rows, output_dims[i]);
+        if (floats[i] > room) {
+            shares[i] = least.shares;
+            floats[i] = partial_floats(shares[i], rows, output_dims[i]);
+        }
+    }
+    bool done[kMaxProjections] = {};
+    for (int start = 0; start < count; ++start) {
+        if (done[start]) continue;
+        int members[kMaxProjections], found = 0;
+        std::int64_t used = 0;
+        for (int i = start; i < count; ++i) {
+            if (done[i] || encodings[i] != encodings[start] || (i != start && used + floats[i] > room)) continue;
+            done[i] = true;
+            members[found++] = i;
+            used += floats[i];
+        }
+        launch(members, found, shares);
+    }
+}
+
 }  // namespace
 
 std::int64_t gemm_f16_required_bytes(std::int64_t rows, std::int64_t input_dim, std::int64_t output_dim) {
@@ -1517,20 +1549,32 @@ void gemm_f16_plan(std::uint32_t encoding, std::int64_t rows, std::int64_t input
     *k_shares = chosen.shares;
 }
 
-int gemm_f16_tile_rows(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
-                       const std::int64_t* output_dims, int count) {
-    if (rows <= kLowRows) return kLowRows;
-    GemmGroup group{};
-    for (int i = 0; i < count; ++i) {
-        group.output_dim[i] = output_dims[i];
-        group.shares[i] = plan(encoding, rows, output_dims[i], input_dim).shares;
-    }
-    switch (encoding) {
-        case kEncQ4K: return tile_height<kEncQ4K>(group, count, rows, input_dim);
-        case kEncQ5K: return tile_height<kEncQ5K>(group, count, rows, input_dim);
-        case kEncQ6K: return tile_height<kEncQ6K>(group, count, rows, input_dim);
-        default: return tile_height<kEncQ8_0>(group, count, rows, input_dim);
-    }
+void gemm_f16_launches(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
+                       const std::int64_t* output_dims, int count, std::int64_t workspace_bytes, int* tile_rows,
+                       int* k_shares) {
+    const std::uint32_t encodings[kMaxProjections] = {encoding, encoding, encoding, encoding};
+    const std::int64_t room = (workspace_bytes - activation_bytes(rows, input_dim)) / 4;
+    for_each_launch(encodings, output_dims, count, rows, input_dim, room,
+                    [&](const int* members, int found, const int* shares) {
+        GemmGroup group{};
+        for (int m = 0; m < found; ++m) {
+            group.output_dim[m] = output_dims[members[m]];
+            group.shares[m] = shares[members[m]];
+        }
+        int height = kLowRows;
+        if (rows > kLowRows) {
+            switch (encoding) {
+                case kEncQ4K: height = tile_height<kEncQ4K>(group, found, rows, input_dim); break;
+                case kEncQ5K: height = tile_height<kEncQ5K>(group, found, rows, input_dim); break;
+                case kEncQ6K: height = tile_height<kEncQ6K>(group, found, rows, input_dim); break;
+                default: height = tile_height<kEncQ8_0>(group, found, rows, input_dim); break;
+            }
+        }
+        for (int m = 0; m < found; ++m) {
+            tile_rows[members[m]] = height;
+            k_shares[members[m]] = shares[members[m]];
+        }
+    });
 }
 
 bool gemm_f16_supports(std::uint32_t encoding, std::int64_t input_dim) {
@@ -1587,40 +1631,33 @@ void launch_gemm_f16(const Descriptor* descriptors, int count, const float* inpu
     const float* inverse_scale = reinterpret_cast<const float*>(activations + padded_rows(rows) * input_dim * 2);
     float* partials = reinterpret_cast<float*>(static_cast<std::uint8_t*>(workspace) + activation_bytes(rows, input_dim));
     const std::int64_t room = (workspace_bytes - activation_bytes(rows, input_dim)) / 4;
-    bool done[kMaxProjections] = {};
-    for (int start = 0; start < count; ++start) {
-        if (done[start]) continue;
-        // this projection and those of its encoding whose partial outputs find room beside its own
-        GemmGroup group{};
-        int members = 0;
-        std::int64_t used = 0;
-        for (int i = start; i < count; ++i) {
-            if (done[i] || descriptors[i].encoding != descriptors[start].encoding) continue;
-            const Plan least = plan(descriptors[i].encoding, rows, descriptors[i].output_dim, input_dim);
-            int shares = shares_with_room(least, rows, descriptors[i].output_dim, input_dim);
-            std::int64_t floats = partial_floats(shares, rows, descriptors[i].output_dim);
-            if (floats > room) {  // a workspace of the plan's size
-                shares = least.shares;
-                floats = partial_floats(shares, rows, descriptors[i].output_dim);
-            }
-            if (i != start && used + floats > room) continue;
-            done[i] = true;
-            group.weights[members] = descriptors[i].data;
-            group.row_stride = descriptors[i].row_stride_bytes;
-            group.output[members] = outputs[i];
-            group.partials[members] = partials + used;
-            group.output_dim[members] = descriptors[i].output_dim;
-            group.shares[members] = shares;
-            used += floats;
-            ++members;
-        }
-        switch (descriptors[start].encoding) {
-            case kEncQ4K: launch_group<kEncQ4K>(group, members, activations, inverse_scale, rows, input_dim, stream); break;
-            case kEncQ5K: launch_group<kEncQ5K>(group, members, activations, inverse_scale, rows, input_dim, stream); break;
-            case kEncQ6K: launch_group<kEncQ6K>(group, members, activations, inverse_scale, rows, input_dim, stream); break;
-            default: launch_group<kEncQ8_0>(group, members, activations, inverse_scale, rows, input_dim, stream); break;
-        }
+    std::uint32_t encodings[kMaxProjections] = {};
+    std::int64_t output_dims[kMaxProjections] = {};
+    for (int i = 0; i < count; ++i) {
+        encodings[i] = descriptors[i].encoding;
+        output_dims[i] = descriptors[i].output_dim;
     }
+    for_each_launch(encodings, output_dims, count, rows, input_dim, room,
+                    [&](const int* members, int found, const int* shares) {
+        GemmGroup group{};
+        std::int64_t used = 0;
+        for (int m = 0; m < found; ++m) {
+            const int i = members[m];
+            group.weights[m] = descriptors[i].data;
+            group.row_stride = descriptors[i].row_stride_bytes;
+            group.output[m] = outputs[i];
+            group.partials[m] = partials + used;
+            group.output_dim[m] = output_dims[i];
+            group.shares[m] = shares[i];
+            used += partial_floats(shares[i], rows, output_dims[i]);
+        }
+        switch (encodings[members[0]]) {
+            case kEncQ4K: launch_group<kEncQ4K>(group, found, activations, inverse_scale, rows, input_dim, stream); break;
+            case kEncQ5K: launch_group<kEncQ5K>(group, found, activations, inverse_scale, rows, input_dim, stream); break;
+            case kEncQ6K: launch_group<kEncQ6K>(group, found, activations, inverse_scale, rows, input_dim, stream); break;
+            default: launch_group<kEncQ8_0>(group, found, activations, inverse_scale, rows, input_dim, stream); break;
+        }
+    });
 }
 
 }  // namespace nfn

@@ -209,6 +209,8 @@ SIGNATURES = {
         ctypes.c_int, [ctypes.c_uint32, _I64, _I64, _I64, ctypes.c_int, _P, _P]),
     "nfn_mi355_k_quant_gemm_tile_rows_v1": (
         ctypes.c_int, [ctypes.c_uint32, _I64, _I64, _P, _I64, ctypes.c_int, _P]),
+    "nfn_mi355_k_quant_gemm_launch_v1": (
+        ctypes.c_int, [ctypes.c_uint32, _I64, _I64, _P, _I64, ctypes.c_int, _I64, _P, _P]),
     "nfn_mi355_k_quant_gemm_float32_v1": (
         ctypes.c_int, [_DESC, _P, _P, _I64, _P, _I64, ctypes.c_int, _P]),
     "nfn_mi355_k_quant_gemm_multi_float32_v1": (
@@ -605,7 +607,7 @@ def gemm(weight: PackedWeight, x, mode: int = GEMM_F16, workspace=None, out=None
 
 
 def gemm_plan(encoding: int, rows: int, input_dim: int, output_dim: int, mode: int = GEMM_F16):
-    """nfn_mi355_k_quant_gemm_plan_v1: (rows of the workgroup tile that K is cut for, K shares)."""
+    """nfn_mi355_k_quant_gemm_plan_v1: (rows of the workgroup tile that K is cut for, the fewest K shares)."""
     tile_rows, shares = ctypes.c_int(0), ctypes.c_int(0)
     check(load().nfn_mi355_k_quant_gemm_plan_v1(
         encoding, rows, input_dim, output_dim, mode, ctypes.addressof(tile_rows),
@@ -615,13 +617,26 @@ def gemm_plan(encoding: int, rows: int, input_dim: int, output_dim: int, mode: i
 
 def gemm_tile_rows(encoding: int, rows: int, input_dim: int, output_dims: Sequence[int], mode: int = GEMM_F16):
     """nfn_mi355_k_quant_gemm_tile_rows_v1: rows per workgroup tile of the launch that runs projections of
-    these widths together."""
+    these widths together, with the workspace of the query."""
     tile_rows = ctypes.c_int(0)
     widths = (ctypes.c_int64 * len(output_dims))(*output_dims)
     check(load().nfn_mi355_k_quant_gemm_tile_rows_v1(
         encoding, rows, input_dim, ctypes.addressof(widths), len(output_dims), mode,
         ctypes.addressof(tile_rows)), "k_quant_gemm_tile_rows")
     return tile_rows.value
+
+
+def gemm_launch(encoding: int, rows: int, input_dim: int, output_dims: Sequence[int], workspace_nbytes: int,
+                mode: int = GEMM_F16):
+    """nfn_mi355_k_quant_gemm_launch_v1: for each projection of a call with such a workspace, (rows per
+    workgroup tile of the launch that takes it, its K shares)."""
+    count = len(output_dims)
+    widths = (ctypes.c_int64 * count)(*output_dims)
+    tile_rows, shares = (ctypes.c_int * count)(), (ctypes.c_int * count)()
+    check(load().nfn_mi355_k_quant_gemm_launch_v1(
+        encoding, rows, input_dim, ctypes.addressof(widths), count, mode, workspace_nbytes,
+        ctypes.addressof(tile_rows), ctypes.addressof(shares)), "k_quant_gemm_launch")
+    return list(zip(tile_rows, shares))
 
 
 def gemm_multi(weights: Sequence[PackedWeight], x, mode: int = GEMM_F16, workspace=None,

@@ -2044,6 +2044,41 @@ def test_prefill_gemm_workspace_of_a_longer_chunk(cuda):
             tile_ops.gemm(weight, x, workspace=large[:needed - 1])
 
 
+def gemm_query(rows, in_dim, *out_dims):
+    lib = tile_ops.load()
+    if len(out_dims) == 1:
+        return lib.nfn_mi355_k_quant_gemm_workspace_bytes_v1(rows, in_dim, out_dims[0], tile_ops.GEMM_F16)
+    widths = (ctypes.c_int64 * len(out_dims))(*out_dims)
+    return lib.nfn_mi355_k_quant_gemm_multi_workspace_bytes_v1(rows, in_dim, ctypes.addressof(widths), len(out_dims),
+                                                               tile_ops.GEMM_F16)
+
+
+def test_prefill_gemm_launch_says_what_runs():
+    """Host logic only.  The height and the shares that the queries report are those of a call with the workspace at
+    hand: 257 rows of 8,704 -> 2,999 are cut in two by the plan (tiles of 128 rows), in four with room for it (256)."""
+    rows, in_dim, out_dim = 257, 8704, 2999
+    plan_bytes = (512 * (in_dim * 2 + 8) + 255) // 256 * 256 + 2 * rows * out_dim * 4 + 256
+    assert tile_ops.gemm_plan(kquant.Q4_K, rows, in_dim, out_dim) == (256, 2)
+    assert tile_ops.gemm_tile_rows(kquant.Q4_K, rows, in_dim, [out_dim]) == 256
+    assert tile_ops.gemm_launch(kquant.Q4_K, rows, in_dim, [out_dim], gemm_query(rows, in_dim, out_dim)) == [(256, 4)]
+    assert tile_ops.gemm_launch(kquant.Q4_K, rows, in_dim, [out_dim], plan_bytes) == [(128, 2)]
+    for rows in (17, 40, 333, 2000):
+        for out_dims in ([4096], [4353, 256, 2300, 5000], [16384, 16384]):
+            for encoding in ALL_PACKED:
+                launched = tile_ops.gemm_launch(encoding, rows, 4096, out_dims, gemm_query(rows, 4096, *out_dims))
+                assert {height for height, _ in launched} == {tile_ops.gemm_tile_rows(encoding, rows, 4096, out_dims)}
+                for n, (_, shares) in zip(out_dims, launched):
+                    single = tile_ops.gemm_launch(encoding, rows, 4096, [n], gemm_query(rows, 4096, n))
+                    assert single[0][1] == shares >= tile_ops.gemm_plan(encoding, rows, 4096, n)[1]
+    least = (256 * (4096 * 2 + 8) + 255) // 256 * 256 + 256
+    assert tile_ops.gemm_launch(kquant.Q4_K, 200, 4096, [16384], least)[0][1] == 1
+    for arguments in ((kquant.Q4_K, 200, 4096, [16384], least - 1), (kquant.Q4_K, 200, 4096, [], least),
+                      (kquant.Q4_K, 0, 4096, [64], least), (kquant.Q4_K, 200, 4100, [64], least),
+                      (kquant.BF16, 200, 4096, [64], least), (kquant.Q4_K, 200, 4096, [0], least)):
+        with pytest.raises(tile_ops.TileOpsError):
+            tile_ops.gemm_launch(*arguments)
+
+
 @pytest.mark.parametrize("rows,in_dim,out_dim", [(33, 4096, 5373), (128, 2304, 2049), (35, 11776, 5376), (97, 1024, 6144)])
 @pytest.mark.parametrize("encoding", ALL_PACKED)
 def test_prefill_gemm_cut_beyond_the_plan(cuda, oracle, encoding, rows, in_dim, out_dim):
