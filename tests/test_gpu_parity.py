@@ -2053,6 +2053,73 @@ def gemm_query(rows, in_dim, *out_dims):
                                                                tile_ops.GEMM_F16)
 
 
+def gemm_weight(cuda, encoding, out_dim, in_dim, seed):
+    """(weight, its 256 different rows, which of them each output has)"""
+    packed = random_packed(encoding, 256, in_dim, seed)
+    chosen = np.random.default_rng(seed + 2).integers(0, 256, out_dim)
+    device_rows = torch_().from_numpy(packed.reshape(256, -1)).to(cuda)
+    return tile_ops.PackedWeight(encoding, out_dim, in_dim, device_rows.index_select(
+        0, torch_().from_numpy(chosen).to(cuda)).reshape(-1)), packed, chosen
+
+
+@pytest.mark.parametrize("rows,in_dim,out_dim,taken", [(33, 4096, 5373, 4), (128, 2304, 2049, 4), (35, 11776, 5376, 6),
+                                                       (36, 1536, 2073, 3), (33, 11520, 2080, 8)])
+@pytest.mark.parametrize("encoding", ALL_PACKED)
+def test_prefill_gemm_cut_beyond_the_plan(cuda, oracle, encoding, rows, in_dim, out_dim, taken):
+    """Few tiles and a K that the plan leaves whole or in long shares: with the workspace of the query the
+    call cuts further (three to eight shares, some of unequal lengths, a last column tile of one), with the
+    plan's it does not; both keep the bound, and a projection beside another the single call's bits."""
+    _, shares = tile_ops.gemm_plan(encoding, rows, in_dim, out_dim)
+    least = (256 * (in_dim * 2 + 8) + 255) // 256 * 256 + (shares * rows * out_dim * 4 if shares > 1 else 0) + 256
+    asked = gemm_query(rows, in_dim, out_dim)
+    assert [tile_ops.gemm_launch(encoding, rows, in_dim, [out_dim], n)[0][1] for n in (asked, least)] == [taken, shares]
+    assert shares < taken
+    weight, packed, chosen = gemm_weight(cuda, encoding, out_dim, in_dim, 46)
+    x = kquant.synthetic_activations(77, rows, in_dim)
+    expected = oracle.linear(encoding, packed, 256, in_dim, x)[:, chosen]
+    device_x = to_device(x, cuda)
+    results = []
+    for nbytes in (asked, least):
+        workspace = torch_().full((nbytes + 4096,), 0x5a, dtype=torch_().uint8, device=cuda)
+        results.append(tile_ops.gemm(weight, device_x, workspace=workspace[:nbytes]))
+        assert normalised_error(results[-1].cpu().numpy(), expected) <= TOLERANCE
+        assert bool((workspace[nbytes:] == 0x5a).all())
+    assert not torch_().equal(*results), "the sums of more shares round differently"
+    with pytest.raises(tile_ops.TileOpsError):
+        tile_ops.gemm(weight, device_x, workspace=workspace[:least - 1])
+    for y in tile_ops.gemm_multi([weight, weight], device_x):
+        assert_bits_equal(y, tile_ops.gemm(weight, device_x), kquant.NAMES[encoding])
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("encoding", ALL_PACKED)
+def test_prefill_gemm_cut_beyond_the_plan_beside_others(cuda, encoding, mixed):
+    """Projections that the call cuts into three, six and four shares beside one that keeps the plan's two, of one
+    encoding and of two: with the grouped query's workspace in one launch an encoding, with what the largest one
+    needs in several, each time with the single calls' bits and nothing written behind the workspace."""
+    rows, in_dim, out_dims = 40, 4096, (4353, 256, 2300, 5000)
+    other = kquant.Q6_K if encoding != kquant.Q6_K else kquant.Q4_K
+    encodings = [encoding, encoding, other if mixed else encoding, encoding]
+    weights = [gemm_weight(cuda, e, n, in_dim, 49 + i)[0] for i, (e, n) in enumerate(zip(encodings, out_dims))]
+    x = to_device(kquant.synthetic_activations(78, rows, in_dim), cuda)
+    alone = [tile_ops.gemm(w, x) for w in weights]
+    together = gemm_query(rows, in_dim, *out_dims)
+    activations = (256 * (in_dim * 2 + 8) + 255) // 256 * 256
+    one = activations + 5 * rows * 2300 * 4 + 256  # (the six shares of one projection, and no other beside it)
+    for nbytes in (together, one):
+        launched = tile_ops.gemm_launch(encoding, rows, in_dim, out_dims, nbytes)
+        assert [shares for _, shares in launched] == [3, 2, 6, 4 if nbytes == together else 1]
+        workspace = torch_().full((nbytes + 4096,), 0x5a, dtype=torch_().uint8, device=cuda)
+        outputs = tile_ops.gemm_multi(weights, x, workspace=workspace[:nbytes])
+        for i, (y, single) in enumerate(zip(outputs, alone)):
+            if launched[i][1] == tile_ops.gemm_launch(encodings[i], rows, in_dim, [out_dims[i]],
+                                                      gemm_query(rows, in_dim, out_dims[i]))[0][1]:
+                assert_bits_equal(y, single, f"projection {i}")
+            else:
+                assert_bits_equal(y, tile_ops.gemm(weights[i], x, workspace=workspace[:nbytes]), f"projection {i}")
+        assert bool((workspace[nbytes:] == 0x5a).all())
+
+
 def test_prefill_gemm_launch_says_what_runs():
     """Host logic only.  The height and the shares that the queries report are those of a call with the workspace at
     hand: 257 rows of 8,704 -> 2,999 are cut in two by the plan (tiles of 128 rows), in four with room for it (256)."""
@@ -2077,35 +2144,6 @@ def test_prefill_gemm_launch_says_what_runs():
                       (kquant.BF16, 200, 4096, [64], least), (kquant.Q4_K, 200, 4096, [0], least)):
         with pytest.raises(tile_ops.TileOpsError):
             tile_ops.gemm_launch(*arguments)
-
-
-@pytest.mark.parametrize("rows,in_dim,out_dim", [(33, 4096, 5373), (128, 2304, 2049), (35, 11776, 5376), (97, 1024, 6144)])
-@pytest.mark.parametrize("encoding", ALL_PACKED)
-def test_prefill_gemm_cut_beyond_the_plan(cuda, oracle, encoding, rows, in_dim, out_dim):
-    """Few tiles and a K that the plan leaves whole or in long shares: with the workspace of the query the
-    call cuts further (shares of four, three and unequal lengths, a last column tile of one), with the
-    plan's it does not; both keep the bound, and projections beside each other the single call's bits."""
-    lib = tile_ops.load()
-    _, shares = tile_ops.gemm_plan(encoding, rows, in_dim, out_dim)
-    least = (256 * (in_dim * 2 + 8) + 255) // 256 * 256 + (shares * rows * out_dim * 4 if shares > 1 else 0) + 256
-    asked = lib.nfn_mi355_k_quant_gemm_workspace_bytes_v1(rows, in_dim, out_dim, tile_ops.GEMM_F16)
-    assert asked >= least
-    packed = random_packed(encoding, 256, in_dim, 46).reshape(256, -1)
-    chosen = np.random.default_rng(48).integers(0, 256, out_dim)
-    weight = tile_ops.PackedWeight(encoding, out_dim, in_dim, torch_().from_numpy(packed).to(cuda).index_select(
-        0, torch_().from_numpy(chosen).to(cuda)).reshape(-1))
-    x = kquant.synthetic_activations(77, rows, in_dim)
-    expected = oracle.linear(encoding, packed.reshape(-1), 256, in_dim, x)[:, chosen]
-    device_x = to_device(x, cuda)
-    for nbytes in (asked, least):
-        workspace = torch_().full((nbytes + 4096,), 0x5a, dtype=torch_().uint8, device=cuda)
-        y = tile_ops.gemm(weight, device_x, workspace=workspace[:nbytes])
-        assert normalised_error(y.cpu().numpy(), expected) <= TOLERANCE
-        assert bool((workspace[nbytes:] == 0x5a).all())
-    with pytest.raises(tile_ops.TileOpsError):
-        tile_ops.gemm(weight, device_x, workspace=workspace[:least - 1])
-    for y in tile_ops.gemm_multi([weight, weight], device_x):
-        assert_bits_equal(y, tile_ops.gemm(weight, device_x), kquant.NAMES[encoding])
 
 
 @pytest.mark.parametrize("rows,in_dim,plan", [
