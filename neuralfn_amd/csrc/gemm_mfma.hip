@@ -1239,9 +1239,8 @@ struct Plan {
     int shares;
 };
 
-Plan plan(std::uint32_t encoding, std::int64_t rows, std::int64_t output_dim,
-          std::int64_t input_dim) {
-    const std::int64_t units = compute_units();
+Plan plan(std::uint32_t encoding, std::int64_t rows, std::int64_t output_dim, std::int64_t input_dim,
+          std::int64_t units) {
     const std::int64_t n_tiles = (output_dim + kBN - 1) / kBN;
     if (rows <= kLowRows) {
         std::int64_t shares = 2 * units / n_tiles;
@@ -1316,6 +1315,21 @@ constexpr TileCost kTileCosts<kEncQ6K>[3] = {{512, {7.0, 0, 0}}, {256, {4.6, 0, 
 template <>
 constexpr TileCost kTileCosts<kEncQ8_0>[3] = {{512, {6.8, 0, 0}}, {256, {4.1, 8.0, 0}}, {128, {3.1, 5.75, 0}}};
 
+// What so many workgroups take for 256 columns each, round behind round, in us.
+template <typename Int>
+double rounds_of(const TileCost& tile, Int workgroups, Int units) {
+    const int places = tile.block[2] > 0 ? 3 : tile.block[1] > 0 ? 2 : 1;
+    const Int full = workgroups / (units * places), rest = workgroups - full * units * places;
+    double rounds = static_cast<double>(full) * tile.block[places - 1];
+    if (rest > 0) {
+        const int last = static_cast<int>((rest + units - 1) / units);
+        const double at_work = static_cast<double>(rest) / static_cast<double>(units * last);
+        const double clock = 1.0 + 0.35 * (at_work - 1.0);
+        rounds += tile.block[last - 1] * (clock > 0.75 ? clock : 0.75);
+    }
+    return rounds;
+}
+
 // The tile height of a launch of more than 32 rows.  The workgroups go to the units in rounds of as
 // many as fit; the last one may leave places or whole units empty, and a chip at work in part runs
 // at a higher clock, down to three quarters of the time.  The figures are fitted to 160 to 3,000
@@ -1346,15 +1360,7 @@ TileChoice cheapest_tile(const TileCost (&tiles_of)[3], const std::int64_t* outp
             tiles += here;
             workgroups += here * shares[i];
         }
-        const int places = tile.block[2] > 0 ? 3 : tile.block[1] > 0 ? 2 : 1;
-        const std::int64_t full = workgroups / (units * places);
-        const int last = static_cast<int>((workgroups - full * units * places + units - 1) / units);
-        double rounds = static_cast<double>(full) * tile.block[places - 1];
-        if (last > 0) {
-            const double at_work = static_cast<double>(workgroups - full * units * places) / static_cast<double>(units * last);
-            const double clock = 1.0 + 0.35 * (at_work - 1.0);
-            rounds += tile.block[last - 1] * (clock > 0.75 ? clock : 0.75);
-        }
+        const double rounds = rounds_of(tile, workgroups, units);
         const double blocks = static_cast<double>(input_dim >> 8) * static_cast<double>(tiles) / static_cast<double>(workgroups);
         const double cost = (blocks + extra) * rounds;
         if (best.rows == 0 || cost < best.cost) best = TileChoice{tile.rows, cost};
@@ -1380,29 +1386,52 @@ int tile_height(const GemmGroup& group, int count, std::int64_t rows, std::int64
 // loses.  Projections of fewer than 2,048 outputs (K and V) keep plan()'s: beside others their shares are
 // not what a launch waits for.  One table of costs (Q4_K's) for all encodings, so that the workspace
 // query, which knows none, need not ask for four.
-int shares_with_room(const Plan& least, std::int64_t rows, std::int64_t output_dim, std::int64_t input_dim) {
+int shares_with_room(const Plan& least, std::int64_t rows, std::int64_t output_dim, std::int64_t input_dim,
+                     std::int64_t units) {
     const std::int64_t n_tiles = (output_dim + kBN - 1) / kBN;
     if (rows <= kLowRows || rows > kMostCutRows || n_tiles < kLeastCutTiles) return least.shares;
-    const std::int64_t units = compute_units();
     if ((rows + 255) / 256 * n_tiles >= units) return least.shares;
-    // (the same for every count up to the next multiple of 128: what gemm_f16_workspace_bytes relies on)
-    const std::int64_t counted = (rows + 127) / 128 * 128;
-    const auto cost = [&](int shares, int quarters) {
-        const std::int64_t outputs = quarters * n_tiles * kBN / 4;
-        const double sums = shares == 1 ? 0.0 : 3.0 + 1.6e-6 * static_cast<double>((shares + 1) * counted * outputs);
-        return cheapest_tile(kTileCosts<kEncQ4K>, &outputs, &shares, 1, counted, input_dim, 0.0, units).cost + sums;
+    // (the same for every count up to the next multiple of 128: what gemm_f16_workspace_bytes relies on; and
+    // from here on every number of tiles and workgroups is a small one)
+    const int counted = static_cast<int>((rows + 127) / 128 * 128), wide = static_cast<int>(n_tiles);
+    const double blocks = static_cast<double>(input_dim >> 8);
+    const auto sums = [&](int shares, int quarters) {
+        return shares == 1 ? 0.0 : 3.0 + 1.6e-6 * static_cast<double>((shares + 1) * counted) * (quarters * wide * kBN / 4);
     };
+    const auto cost = [&](int shares, int quarters) {
+        double least_walk = 0;
+        for (const TileCost& tile : kTileCosts<kEncQ4K>) {
+            const int tiles = (counted + tile.rows - 1) / tile.rows * ((quarters * wide + 3) / 4);
+            const double walk = rounds_of(tile, tiles * shares, static_cast<int>(units));
+            if (least_walk == 0 || walk < least_walk) least_walk = walk;
+        }
+        return blocks / shares * least_walk + sums(shares, quarters);
+    };
+    // What the blocks take with every place of every unit at work: no cut gets below it.
+    double fullest = 0;
+    for (const TileCost& tile : kTileCosts<kEncQ4K>) {
+        double block = tile.block[0];
+        for (int places = 2; places <= 3; ++places) {
+            if (tile.block[places - 1] > 0) block = std::min(block, tile.block[places - 1] / places);
+        }
+        const double here = block * ((counted + tile.rows - 1) / tile.rows * wide);
+        if (fullest == 0 || here < fullest) fullest = here;
+    }
+    fullest *= blocks / static_cast<double>(units);
     // quarters of the outputs: alone, with another, ...  (The host pays for this in every call and several
-    // times in a query, so what saves too little by itself goes no further: queries of 333 / 2,048 rows into
-    // 6,656 outputs 17 / 31 -> 3 / 5 us.)
+    // times in a query, so what saves too little by itself, or cannot, goes no further, and the unit count is asked
+    // once: queries of 333 rows of 6,656 into Q, K, V and gate / of 1,000 rows of 4,096 -> 6,656 5.2 / 4.9 -> 0.4 /
+    // 0.9 us, without any further shares 2.5 / 0.8.)
     constexpr int kBeside[4] = {4, 8, 9, 10};
+    constexpr double kSaved = 0.94;
     double least_cost[4] = {cost(least.shares, kBeside[0])};
     int best = least.shares;
     double best_saved = 1.0;
     for (const int shares : {2, 3, 4, 6, 8}) {
-        if (shares <= least.shares || 2 * shares > (input_dim >> 8)) continue;
+        if (shares <= least.shares) continue;
+        if (2 * shares > (input_dim >> 8) || fullest + sums(shares, kBeside[0]) >= kSaved * least_cost[0]) break;
         double saved = cost(shares, kBeside[0]) / least_cost[0];
-        bool pays = saved < 0.94;
+        bool pays = saved < kSaved;
         for (int i = 1; i < 4 && pays; ++i) {
             if (least_cost[i] == 0) least_cost[i] = cost(least.shares, kBeside[i]);
             const double here = cost(shares, kBeside[i]) / least_cost[i];
@@ -1464,17 +1493,19 @@ std::int64_t activation_bytes(std::int64_t rows, std::int64_t input_dim) {
 // The largest of needed(count) over the row counts up to `rows`, of projections of `narrowest` outputs
 // and more: short chunks split K further than longer ones and can take more memory.  What a plan
 // gives stays the same from one multiple of 128 rows to the next, so that only those can be largest,
-// and from a tile a unit on nothing is split.
-template <typename F>
-std::int64_t largest_up_to(std::int64_t rows, std::int64_t narrowest, F&& needed) {
+// and from a tile a unit on nothing is split.  at_most(count): no less than needed() of that count and of every
+// smaller one, so that the small counts need no choice of shares.
+template <typename F, typename G>
+std::int64_t largest_up_to(std::int64_t rows, std::int64_t narrowest, std::int64_t units, F&& needed, G&& at_most) {
     std::int64_t largest = needed(rows);
-    const auto take = [&](std::int64_t count) {
-        const std::int64_t bytes = count < rows ? needed(count) : 0;
-        if (bytes > largest) largest = bytes;
-    };
-    take(kLowRows);
-    const std::int64_t n_tiles = (narrowest + kBN - 1) / kBN, units = compute_units();
-    for (std::int64_t count = 128; count < rows && (count + 255) / 256 * n_tiles < units; count += 128) take(count);
+    const std::int64_t n_tiles = (narrowest + kBN - 1) / kBN;
+    // the last count below `rows` whose tiles of 256 rows are fewer than the units
+    const std::int64_t split_rows = (units - 1) / n_tiles * 256, below = (rows - 1) / 128 * 128;
+    for (std::int64_t count = std::min(split_rows, below); count > 0; count -= 128) {
+        if (at_most(count) <= largest) return largest;
+        largest = std::max(largest, needed(count));
+    }
+    if (kLowRows < rows && at_most(kLowRows) > largest) largest = std::max(largest, needed(kLowRows));
     return largest;
 }
 
@@ -1483,15 +1514,19 @@ std::int64_t partial_floats(int shares, std::int64_t rows, std::int64_t output_d
     return (shares - 1) * rows * output_dim;
 }
 
+std::int64_t required_bytes(std::int64_t rows, std::int64_t input_dim, std::int64_t output_dim, int shares) {
+    return activation_bytes(rows, input_dim) + (shares > 1 ? shares * rows * output_dim * 4 : 0) + 256;
+}
+
 // ... of the shares that a call with room for them takes, whatever the encoding (plan() gives Q4_K the most,
-// and with as many or more the other encodings take none that it does not)
-std::int64_t most_partial_floats(std::int64_t rows, std::int64_t output_dim, std::int64_t input_dim) {
-    const Plan q4 = plan(kEncQ4K, rows, output_dim, input_dim), q6 = plan(kEncQ6K, rows, output_dim, input_dim);
-    std::int64_t most = partial_floats(shares_with_room(q4, rows, output_dim, input_dim), rows, output_dim);
-    if (q6.shares != q4.shares) {
-        most = std::max(most, partial_floats(shares_with_room(q6, rows, output_dim, input_dim), rows, output_dim));
-    }
-    return most;
+// and with as many or more the other encodings take none that it does not); *required: required_bytes().
+std::int64_t most_partial_floats(std::int64_t rows, std::int64_t output_dim, std::int64_t input_dim, std::int64_t units,
+                                 std::int64_t* required) {
+    const Plan q4 = plan(kEncQ4K, rows, output_dim, input_dim, units), q6 = plan(kEncQ6K, rows, output_dim, input_dim, units);
+    *required = required_bytes(rows, input_dim, output_dim, q4.shares);
+    int most = shares_with_room(q4, rows, output_dim, input_dim, units);
+    if (q6.shares != q4.shares) most = std::max(most, shares_with_room(q6, rows, output_dim, input_dim, units));
+    return partial_floats(most, rows, output_dim);
 }
 
 // The launches of a call whose workspace has `room` floats behind the activations: each takes projections of
@@ -1500,11 +1535,19 @@ std::int64_t most_partial_floats(std::int64_t rows, std::int64_t output_dim, std
 template <typename F>
 void for_each_launch(const std::uint32_t* encodings, const std::int64_t* output_dims, int count, std::int64_t rows,
                      std::int64_t input_dim, std::int64_t room, F&& launch) {
+    const std::int64_t units = compute_units();
     int shares[kMaxProjections];
     std::int64_t floats[kMaxProjections];
     for (int i = 0; i < count; ++i) {
-        const Plan least = plan(encodings[i], rows, output_dims[i], input_dim);
-        shares[i] = shares_with_room(least, rows, output_dims[i], input_dim);
+        int same = 0;
+        while (encodings[same] != encodings[i] || output_dims[same] != output_dims[i]) ++same;
+        if (same < i) {
+            shares[i] = shares[same];
+            floats[i] = floats[same];
+            continue;
+        }
+        const Plan least = plan(encodings[i], rows, output_dims[i], input_dim, units);
+        shares[i] = shares_with_room(least, rows, output_dims[i], input_dim, units);
         floats[i] = partial_floats(shares[i], rows, output_dims[i]);
         if (floats[i] > room) {
             shares[i] = least.shares;
@@ -1531,20 +1574,16 @@ void for_each_launch(const std::uint32_t* encodings, const std::int64_t* output_
 std::int64_t gemm_f16_required_bytes(std::int64_t rows, std::int64_t input_dim, std::int64_t output_dim) {
     // the activations, then one copy of the output per K share of a split
     // launch (the encoding with the most shares bounds the others)
-    const int shares = plan(kEncQ4K, rows, output_dim, input_dim).shares;
-    return activation_bytes(rows, input_dim) + (shares > 1 ? shares * rows * output_dim * 4 : 0) + 256;
+    return required_bytes(rows, input_dim, output_dim, plan(kEncQ4K, rows, output_dim, input_dim, compute_units()).shares);
 }
 
 std::int64_t gemm_f16_workspace_bytes(std::int64_t rows, std::int64_t input_dim, std::int64_t output_dim) {
-    return largest_up_to(rows, output_dim, [&](std::int64_t count) {
-        const std::int64_t required = gemm_f16_required_bytes(count, input_dim, output_dim);
-        return std::max(required, activation_bytes(count, input_dim) + 4 * most_partial_floats(count, output_dim, input_dim) + 256);
-    });
+    return gemm_f16_multi_workspace_bytes(rows, input_dim, &output_dim, 1);
 }
 
 void gemm_f16_plan(std::uint32_t encoding, std::int64_t rows, std::int64_t input_dim,
                    std::int64_t output_dim, int* tile_rows, int* k_shares) {
-    const Plan chosen = plan(encoding, rows, output_dim, input_dim);
+    const Plan chosen = plan(encoding, rows, output_dim, input_dim, compute_units());
     *tile_rows = chosen.tile_rows;
     *k_shares = chosen.shares;
 }
@@ -1605,21 +1644,26 @@ void convert_gemm_activations(const float* input, std::int64_t rows, std::int64_
 
 std::int64_t gemm_f16_multi_workspace_bytes(std::int64_t rows, std::int64_t input_dim, const std::int64_t* output_dims,
                                             int count) {
-    std::int64_t narrowest = output_dims[0];
-    for (int i = 1; i < count; ++i) {
+    std::int64_t narrowest = output_dims[0], outputs = 0;
+    for (int i = 0; i < count; ++i) {
         if (output_dims[i] < narrowest) narrowest = output_dims[i];
+        outputs += output_dims[i];
     }
-    return largest_up_to(rows, narrowest, [&](std::int64_t chunk) {
+    const std::int64_t units = compute_units();
+    const auto needed = [&](std::int64_t chunk) {
         std::int64_t largest = 0, floats = 0;
+        std::int64_t here[kMaxProjections], required[kMaxProjections];
         for (int i = 0; i < count; ++i) {
-            std::int64_t single = gemm_f16_required_bytes(chunk, input_dim, output_dims[i]);
-            const std::int64_t here = most_partial_floats(chunk, output_dims[i], input_dim);
-            single = std::max(single, activation_bytes(chunk, input_dim) + 4 * here + 256);
-            if (single > largest) largest = single;
-            floats += here;
+            int same = 0;
+            while (output_dims[same] != output_dims[i]) ++same;
+            if (same == i) here[i] = most_partial_floats(chunk, output_dims[i], input_dim, units, &required[i]);
+            largest = std::max(largest, required[same]);
+            floats += here[same];
         }
-        const std::int64_t together = activation_bytes(chunk, input_dim) + 4 * floats + 256;
-        return together > largest ? together : largest;
+        return std::max(largest, activation_bytes(chunk, input_dim) + 4 * floats + 256);
+    };
+    return largest_up_to(rows, narrowest, units, needed, [&](std::int64_t chunk) {
+        return activation_bytes(chunk, input_dim) + 4 * kLowShares * chunk * outputs + 256;
     });
 }
 

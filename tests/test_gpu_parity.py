@@ -2120,6 +2120,18 @@ def test_prefill_gemm_cut_beyond_the_plan_beside_others(cuda, encoding, mixed):
         assert bool((workspace[nbytes:] == 0x5a).all())
 
 
+@pytest.mark.parametrize("rows,in_dim,out_dims", [(333, 6656, [4096, 256, 256, 4096]), (1000, 4096, [6656]), (2048, 16384, [6656]),
+                                                  (1100, 11520, [2080, 4097]), (700, 1536, [16384, 130, 2073]), (40, 512, [64])])
+def test_prefill_gemm_workspace_lets_every_shorter_call_take_its_shares(rows, in_dim, out_dims):
+    """Host logic only.  The query looks at few row counts, the largest first, and at none that cannot need more; with
+    its workspace a call of any count takes the shares and tiles that it would with all the room there is."""
+    nbytes = gemm_query(rows, in_dim, *out_dims)
+    for encoding in (kquant.Q4_K, kquant.Q6_K):
+        for count in sorted({*range(1, rows, 23), *range(128, rows, 128), 32, 33, rows}):
+            assert (tile_ops.gemm_launch(encoding, count, in_dim, out_dims, nbytes) ==
+                    tile_ops.gemm_launch(encoding, count, in_dim, out_dims, 1 << 60)), count
+
+
 def test_prefill_gemm_launch_says_what_runs():
     """Host logic only.  The height and the shares that the queries report are those of a call with the workspace at
     hand: 257 rows of 8,704 -> 2,999 are cut in two by the plan (tiles of 128 rows), in four with room for it (256)."""
