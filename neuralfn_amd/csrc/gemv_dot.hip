@@ -580,9 +580,16 @@ void launch_variant(ProjectionSet set, const float* first, const float* second,
     const std::size_t lds = static_cast<std::size_t>(T) * token_image_bytes_host(blocks);
     const int passes = (tokens + T - 1) / T;
     // (up to six workgroups per unit: 6,656 -> 65,536 streams at 5.25 TB/s with six, 5.0 with four)
-    // Normalising workgroups: one a unit.  Each normalises the row for itself, and two on a unit take turns
-    // at it: 6,656 -> 6,144 + 256 + 256 + 6,144 of Q4_K 17.3 -> 15.6 us, of Q5_K 25.3 -> 18.8 (the norms in a launch of
-    // their own: 16.0 and 19.1); + 1,024 + 1,024 18.2 -> 16.9 and 26.1 -> 21.5 (16.8, 20.1).
+    // Normalising workgroups: one a unit, at any size.  Each normalises the row for itself, and two on a unit take
+    // turns at it; a launch of many rows loses less to the loads that are then in flight than it gains.  One / two /
+    // three / as many as six workgroups a unit / the norms in a launch of their own, us, Q4_K and Q5_K:
+    //   2,048 -> 12,800   10.4 / 11.8 /  -   /  -   / 11.3   11.8 / 17.6 /  -   /  -   / 13.1
+    //   2,048 -> 65,536   25.1 / 26.1 / 31.9 / 37.1 / 27.0   30.4 / 40.5 / 45.3 / 59.3 / 35.6
+    //   4,096 -> 32,768   19.7 / 19.6 / 25.0 / 30.0 / 22.8   23.5 / 29.6 / 34.3 / 44.2 / 28.2
+    //   6,656 -> 18,432   20.3 / 20.0 / 25.1 /  -   / 21.3   22.6 / 29.5 / 34.6 /  -   / 25.7
+    //   8,192 -> 18,432   21.9 / 21.4 / 27.1 /  -   / 23.3   26.6 / 31.8 / 36.7 /  -   / 28.5
+    //   8,192 -> 65,536   62.9 / 63.4 / 67.6 / 67.1 / 63.6   75.8 / 78.7 / 84.1 / 96.9 / 75.6
+    // (the largest loss of one against two in 24 sizes is that of 8,192 -> 18,432 of Q4_K)
     const std::int64_t groups = decode_groups(rows, kDotWaves, P == kDualNorm ? 1 : 6);
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups), passes), dim3(kDotThreads), lds,
@@ -596,26 +603,19 @@ void launch_variant(ProjectionSet set, const float* first, const float* second,
     if constexpr (T == 1) {
         // one workgroup per compute unit: three stages, the third requested late
         const bool small = groups <= compute_units();
-        if (slices == 1) {
-            if (small) {
-                allow_large_lds<gemv_dot_kernel<ENC, T, P, 1, 3>>(kDynamicLds);
-                launch(gemv_dot_kernel<ENC, T, P, 1, 3>);
-            } else {
-                allow_large_lds<gemv_dot_kernel<ENC, T, P, 1, 2>>(kDynamicLds);
-                launch(gemv_dot_kernel<ENC, T, P, 1, 2>);
+        const auto in_registers = [&](auto count) {
+            constexpr int kSlices = decltype(count)::value;
+            if constexpr (P != kDualNorm) {
+                if (!small) {
+                    allow_large_lds<gemv_dot_kernel<ENC, T, P, kSlices, 2>>(kDynamicLds);
+                    return launch(gemv_dot_kernel<ENC, T, P, kSlices, 2>);
+                }
             }
-            return;
-        }
-        if (slices == 2) {
-            if (small) {
-                allow_large_lds<gemv_dot_kernel<ENC, T, P, 2, 3>>(kDynamicLds);
-                launch(gemv_dot_kernel<ENC, T, P, 2, 3>);
-            } else {
-                allow_large_lds<gemv_dot_kernel<ENC, T, P, 2, 2>>(kDynamicLds);
-                launch(gemv_dot_kernel<ENC, T, P, 2, 2>);
-            }
-            return;
-        }
+            allow_large_lds<gemv_dot_kernel<ENC, T, P, kSlices, 3>>(kDynamicLds);
+            launch(gemv_dot_kernel<ENC, T, P, kSlices, 3>);
+        };
+        if (slices == 1) return in_registers(std::integral_constant<int, 1>{});
+        if (P == kDualNorm || slices == 2) return in_registers(std::integral_constant<int, 2>{});
         if (small) {
             if constexpr (P == kGated || P == kSwiGlu) {
                 // rows of more than 8,192 columns behind an activation prologue: sixteen waves per
@@ -632,13 +632,16 @@ void launch_variant(ProjectionSet set, const float* first, const float* second,
                                    tail);
                 return;
             }
-            allow_large_lds<gemv_dot_kernel<ENC, T, P, 0, 3>>(kDynamicLds);
-            launch(gemv_dot_kernel<ENC, T, P, 0, 3>);
-            return;
+            if constexpr (P != kDualNorm) {
+                allow_large_lds<gemv_dot_kernel<ENC, T, P, 0, 3>>(kDynamicLds);
+                return launch(gemv_dot_kernel<ENC, T, P, 0, 3>);
+            }
         }
     }
-    allow_large_lds<gemv_dot_kernel<ENC, T, P, 0, 2>>(kDynamicLds);
-    launch(gemv_dot_kernel<ENC, T, P, 0, 2>);
+    if constexpr (P != kDualNorm) {  // (whose rows are at most 8,192 columns long: two slices)
+        allow_large_lds<gemv_dot_kernel<ENC, T, P, 0, 2>>(kDynamicLds);
+        launch(gemv_dot_kernel<ENC, T, P, 0, 2>);
+    }
 }
 
 // Pair mode: `set` holds two projections of one shape and one output (slot 0), one token.

@@ -1690,6 +1690,21 @@ def test_dual_rms_inside_the_projection_launch_equals_the_two_calls(cuda, oracle
         assert_bits_equal(a, b, f"projection of {n} rows")
 
 
+@pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K])
+@pytest.mark.parametrize("width,outputs", [(256, 30001), (4096, 20000), (8192, 12803)])
+def test_dual_rms_inside_a_projection_launch_of_many_rows(cuda, encoding, width, outputs):
+    """One normalising workgroup a compute unit, however many rows it then has: the bits of the two calls."""
+    packed = torch_().from_numpy(random_packed(encoding, 64, width, 55).reshape(64, -1)).to(cuda)
+    chosen = torch_().from_numpy(np.random.default_rng(56).integers(0, 64, outputs)).to(cuda)
+    weights = [tile_ops.PackedWeight(encoding, n, width, packed.index_select(0, chosen[:n]).reshape(-1)) for n in (outputs, 33)]
+    x, residual = (to_device(kquant.synthetic_activations(seed, 1, width), cuda) for seed in (57, 58))
+    ordinary = tile_ops.dual_rms_add_capture(x, residual)
+    fused = tile_ops.dual_rms_multi_linear(x, residual, weights)
+    for a, b in zip((*ordinary, *tile_ops.multi_linear(weights, ordinary[1], tile_ops.small_batch_workspace(1, width))),
+                    (*fused[:3], *fused[3])):
+        assert_bits_equal(a, b, f"{outputs} rows")
+
+
 def test_dual_rms_inside_the_projection_launch_fails_closed(cuda):
     lib = tile_ops.load()
     width = 512
