@@ -83,25 +83,42 @@ Projection make_projection(const Descriptor& descriptor, float* output) {
 // Whether two or three rows of the verifier family run on its matrix-core kernel behind a quantizer launch
 // (gemv_rows.hip), as from four rows on, or on the dot kernels: the same bits on either, a question of time.
 // Two launches that read the activations once, against one in which every workgroup makes their codes (and a
-// prologue's functions) for itself; K: input_dim.  Times of the call before -> with it, us, one box, weights from
-// memory.
-//   Three rows: K-Quants always (2,048 -> 6,144 of Q4_K 9.3 -> 7.0, 7,936 -> 39,936 76 -> 43, Q6_K 132 -> 68, SwiGLU
-//     16,384 -> 6,656 of Q4_K 37 -> 21); Q8_0 gains from long rows or many outputs (16,384 -> 6,656 34 -> 30, 4,096 ->
-//     32,768 35 -> 32; 4,096 -> 6,656 would lose, 12.4 -> 13.1).
-//   Two rows: K above 12,288 (SwiGLU 18,432 -> 2,304 21 -> 14, 16,384 -> 6,656 of Q6_K 38 -> 33) or, Q4_K and Q5_K, many
-//     outputs (4,096 -> 16,384 twice 25 -> 22); 6,656 -> 8,704 would lose, 13.4 -> 15.2.
+// prologue's functions) for itself: the longer the rows and the more of them, the more the dot kernels lose; short
+// rows of few outputs gain nothing that pays for a second launch.  outputs: of all projections of the call in this
+// encoding.  Lines from 1,500 calls of 1,024 to 19,968 columns into 128 to 40,000 outputs (weights from memory), us,
+// dot kernel and this one:
+//   Three rows, Q4_K and Q5_K: 7,936 -> 39,936 76 and 43; SwiGLU 16,384 -> 6,656 37 and 21; 2,304 -> 1,504 6.2 and 6.9,
+//     4,096 -> 982 of Q5_K 7.5 and 7.7; gated 1,536 -> 1,488 6.8 and 6.8.
+//   Q6_K: the streaming form of its dot kernel, from 4,096 columns on, is the slower one (5,120 -> 1,822 14.4 and 11.0)
+//     but for few long rows (14,848 -> 659 15.9 and 18.3); the form for shorter rows is the faster one (3,072 ->
+//     1,691 7.5 and 9.1, 2,560 -> 9,954 15.8 and 18.0) but for many (2,048 -> 5,136 11.0 and 9.1, 3,584 -> 22,087 31.6 and
+//     29.0).
+//   Q8_0: 16,384 -> 6,656 34 and 30; 6,656 -> 1,087 9.5 and 10.5, 8,192 -> 4,768 16.6 and 18.5; gated 7,168 -> 2,715
+//     14.5 and 13.1.
+//   Two rows: SwiGLU 18,432 -> 2,304 21 and 14, 18,432 -> 640 15.0 and 11.1; 15,872 -> 4,676 19.6 and 21.4 (a few
+//     workgroups have a second tile then); Q6_K 16,384 -> 2,312 23.3 and 21.1, 14,592 -> 511 15.7 and 18.2.  Shorter rows
+//     of Q4_K and Q5_K: 4,096 -> 16,384 twice 25 and 22, 2,304 -> 20,000 1.09 times as long, 6,656 -> 8,704 13.4 and 15.2.
 // The other family stays on its own kernels, although they take longer for some shapes (SwiGLU 18,432 -> 2,304 of Q4_K,
 // three rows, 34 us and not 14): the quantizer launch would overwrite activation records that a verifier call left in
 // the workspace, and at three and four rows the results would not be the logits that the fused lm_head takes its
 // maximum of.
-bool rows_kernel_pays(std::uint32_t encoding, int prologue, std::int64_t rows, std::int64_t output_dim,
+bool rows_kernel_pays(std::uint32_t encoding, int prologue, std::int64_t rows, std::int64_t outputs,
                       std::int64_t input_dim) {
-    constexpr std::int64_t kLongRows = 12288, kManyOutputs = 12288;
     if (prologue == kRecords || rows < 2) return false;
-    const bool q45 = encoding == kEncQ4K || encoding == kEncQ5K;
-    const bool q8 = encoding == kEncQ8_0;
-    if (rows == 2) return (!q8 && input_dim > kLongRows) || (q45 && output_dim >= kManyOutputs);
-    return !q8 || input_dim >= 6144 || output_dim >= kManyOutputs;
+    const bool plain = prologue == kPlain;
+    if (rows == 2) {
+        if (encoding == kEncQ8_0) return false;
+        if (input_dim <= 12288) return encoding != kEncQ6K && outputs > (plain ? 24576 : 12288);
+        if (!plain) return true;
+        return !(outputs > 4096 && outputs <= 5120) && (encoding != kEncQ6K || outputs > 2048);
+    }
+    switch (encoding) {
+        case kEncQ6K:
+            if (input_dim < 4096) return outputs > (input_dim <= 2048 ? 4608 : 20480);
+            return input_dim <= 10240 || !plain || outputs > 1024;
+        case kEncQ8_0: return plain ? input_dim > 8192 || outputs > 16384 : input_dim >= 6144 || outputs >= 12288;
+        default: return input_dim > (plain ? 4096 : 2304) || outputs > 3072;
+    }
 }
 
 // Shared body of the small-batch entry points.
@@ -146,7 +163,9 @@ int run_small_batch(bool verifier, const Descriptor* const* descriptors, const f
     for (int index = 0; index < set.count; ++index) {
         const std::uint32_t encoding = set.op[index].encoding;
         ProjectionSet* target = &exact;
-        if ((always_rows || (room && rows_kernel_pays(encoding, prologue, rows, set.op[index].output_dim, input_dim))) &&
+        std::int64_t outputs = 0;
+        for (int i = 0; i < set.count; ++i) outputs += set.op[i].encoding == encoding ? set.op[i].output_dim : 0;
+        if ((always_rows || (room && rows_kernel_pays(encoding, prologue, rows, outputs, input_dim))) &&
             gemv_rows_supports(encoding, input_dim)) {
             target = &verifier_rows;
         } else if (one_row_arithmetic && gemv_dot_supports(encoding, input_dim)) {
