@@ -352,12 +352,13 @@ def test_exact_linear_small_tiles_of_special_operands(cuda, oracle, encoding):
         test_exact_linear_of_tiny_operands(cuda, oracle, encoding, rows, out_dim, in_dim, -36)
 
 
-@pytest.mark.parametrize("out_dim", [90, 94, 325, 326, 581, 582, 605, 606, 1117, 1118])
+@pytest.mark.parametrize("in_dim,out_dim", [*((1024, n) for n in (90, 94, 320, 321, 576, 577, 606)),
+                                            *((1280, n) for n in (368, 369, 544, 545)), (2048, 368), (2048, 545),
+                                            *((2304, n) for n in (368, 369, 592, 593, 928, 929)), (4352, 640), (4352, 641)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
-def test_exact_linear_carries_the_same_bits_from_four_to_32_rows(cuda, encoding, out_dim):
-    """Which kernel and which form of it runs from four to 32 rows hangs on the outputs alone (their counts on
+def test_exact_linear_carries_the_same_bits_from_four_to_32_rows(cuda, encoding, in_dim, out_dim):
+    """Which kernel and which form of it runs from four to 32 rows hangs on the weight alone (outputs and widths on
     both sides of every line)."""
-    in_dim = 1024
     weight = tile_ops.PackedWeight.from_numpy(
         encoding, kquant.quantize(encoding, kquant.synthetic_weights(60, out_dim, in_dim)), out_dim, in_dim)
     x = to_device(kquant.synthetic_activations(61, 32, in_dim), cuda)
@@ -366,14 +367,14 @@ def test_exact_linear_carries_the_same_bits_from_four_to_32_rows(cuda, encoding,
         assert_bits_equal(tile_ops.linear(weight, x[:rows].contiguous()), all_rows[:rows].contiguous(), f"{rows} rows")
 
 
-@pytest.mark.parametrize("rows,out_dim,in_dim", [(4, 300, 2048), (5, 33, 512), (7, 605, 256), (12, 372, 8192), (17, 2, 64), (97, 65, 4096)])
+@pytest.mark.parametrize("rows,out_dim,in_dim", [(4, 300, 2048), (5, 33, 1280), (7, 368, 1536), (12, 352, 8192), (17, 2, 1088), (97, 65, 4096)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
 def test_exact_linear_of_row_groups(cuda, oracle, encoding, rows, out_dim, in_dim):
     """More than three rows into few outputs on the vector kernel, two or three of them a workgroup: row for
     row the bits of the call of three rows (F32 and bf16, whose waves may share a row or not: its bound), a
     last group of one or two, nothing written past the end."""
     if encoding not in (kquant.F32, kquant.BF16, kquant.Q8_0):
-        in_dim = max(in_dim, 256)
+        in_dim = -(-in_dim // 256) * 256
     packed = kquant.quantize(encoding, kquant.synthetic_weights(50, out_dim, in_dim))
     x = kquant.synthetic_activations(51, rows, in_dim)
     weight = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
