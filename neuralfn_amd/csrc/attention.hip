@@ -1385,10 +1385,11 @@ void launch_split(AttentionArguments a, std::int64_t query_rows, std::int64_t ti
     // in 16 shares of two waves takes 11.1 us with its merge, in 32 shares of one wave 12.1 us
     // (12 or 24 shares: 11.7; 8: 11.9); long contexts and blocks are not touched by this
     // (32,768 keys: 128 shares 15.1 us, 96: 15.4, 64: 17.1; a 16-row block: 8..24 shares 16.1 us).
-    // Sixteen shares up to 48 tiles: 3,000 keys in 24 of two waves 11.9 to 12.5 us, in 16 of three 11.1 to 11.6.
+    // Sixteen shares of three waves at 41 to 48 tiles: 300 calls of 33 to 48 tiles and 16 to 48 heads over 2 to 8 take
+    // 1.5 % less with them there (2,620 keys of 16 heads over 2 12.4 -> 11.5 us), and 1 % more at 33 to 40 tiles.
     if (query_rows == 1 && grouped && 2 * splits > tiles && tiles >= 4) {
         splits = (tiles + 1) / 2;
-        if (tiles <= 48 && splits > 16) splits = 16;
+        if (tiles > 40 && tiles <= 48) splits = 16;
     }
     if (splits < 2) splits = 2;
     if (splits > partial_bytes / share_bytes) splits = partial_bytes / share_bytes;
