@@ -169,10 +169,14 @@ std::int64_t lm_head_f32_blocks(std::int64_t output_dim) {
 // many workgroups as that takes (64 rows each would leave most units idle, or waves with four pairs
 // where others have none to hide behind): 4,608 -> 4,000 / 9,000 / 16,000 rows of Q4_K 24.4 / 24.4 / 25.2 ->
 // 11.3 / 19.1 / 22.8 us; 30,000 would take 39.3 instead of 37.0.
+std::int64_t row_pairs(std::int64_t output_dim) { return (output_dim + kExactPair - 1) / kExactPair; }
+std::int64_t row_turns(std::int64_t output_dim) {  // of eight waves, three workgroups a unit
+    const std::int64_t at_once = 24 * std::int64_t(compute_units());
+    return (row_pairs(output_dim) + at_once - 1) / at_once;
+}
 std::int64_t lm_head_row_groups(std::int64_t output_dim) {
     const std::int64_t resident = 2 * std::int64_t(compute_units());
-    const std::int64_t pairs = (output_dim + kExactPair - 1) / kExactPair;
-    const std::int64_t turns = (pairs + 12 * resident - 1) / (12 * resident);  // of eight waves, three a unit
+    const std::int64_t pairs = row_pairs(output_dim), turns = row_turns(output_dim);
     if (turns <= 2) return (pairs + kExactWaves * turns - 1) / (kExactWaves * turns);
     const std::int64_t blocks = lm_head_f32_blocks(output_dim);
     return blocks < resident ? blocks : resident;
@@ -192,6 +196,10 @@ void launch_lm_head_f32(const Descriptor& descriptor, const float* input, std::i
     if (rows == 1 && descriptor.input_dim % 64 == 0 &&
         exact_rows_lds(1, descriptor.input_dim) <= 159 * 1024) {
         std::int64_t groups = lm_head_row_groups(descriptor.output_dim);
+        // (Q8_0, 12,289 to 16,384 rows: 64 each, one workgroup a unit.  In two turns some units would have two workgroups
+        // and take as long as its four: 6,656 -> 13,001 and 7,936 -> 12,617 1.10 times, 2,560 to 5,120 columns as long;
+        // more rows, where 64 each leave some units with two, take 0.85 to 0.89 times, like the other formats.)
+        if (descriptor.encoding == kEncQ8_0 && row_turns(descriptor.output_dim) == 2 && blocks <= compute_units()) groups = blocks;
         if (groups > room) groups = room;
         bool launched = true;
         switch (descriptor.encoding) {
