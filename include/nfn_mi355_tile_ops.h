@@ -999,7 +999,8 @@ int nfn_mi355_k_quant_gemm_multi_float32_v1(
 /* One-token attention with a workspace: nfn_native_tile_glimmer_gqa_decode_float32_v1
  * runs one workgroup per query head because it has nowhere to put partial
  * results; with a workspace the keys of every head are dealt over many
- * workgroups (up to 128 shares) and a second launch merges their partial sums.
+ * workgroups (up to 128 shares) and a second launch merges their partial sums
+ * (keys that one workgroup takes in less time than the merge are not dealt).
  * With head_dim 128 and four or more query heads per key/value head a
  * workgroup serves up to 16 query heads of one key/value head on the matrix
  * cores, so a cache row is read once for all of them.  Same descriptor,
