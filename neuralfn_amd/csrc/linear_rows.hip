@@ -11,8 +11,6 @@
 #include "exact_rows.hpp"
 #include "kernels.hpp"
 
-#include <algorithm>
-
 namespace nfn {
 
 namespace {
@@ -265,35 +263,36 @@ void launch_for(const Descriptor& weight, const float* input, const float* bias,
 
 namespace {
 
-// Four rows and more: while the workgroups, of sixteen weight rows and three input rows each, are few enough.  Weight
-// rows per compute unit (sixteen are a workgroup a unit, 17 to 32 two on some, and take twice as long) up to which
-// it wins over linear_exact.hip, from 3,700 calls of 256 to 8,192 columns, 4 to 512 rows and up to 60 weight rows a unit; both in us, this one second, 32 rows:
+// Four rows and more: while the workgroups, of sixteen weight rows and three input rows each, are few enough.  A
+// unit with two of them takes twice as long as one with one, so that the lines lie at whole workgroups a unit.
+// Where it wins over linear_exact.hip, from 3,700 calls of 256 to 8,192 columns, 4 to 512 rows and up to four workgroups a
+// unit; both in us, this one second, 32 rows:
 //   Q4_K, Q8_0   none up to 1,024 columns, where that kernel needs a turn or two (1,024 -> 439 6.1 and 8.0; Q8_0 512 ->
-//     213 5.3 and 5.9), 24 up to 2,048 (2,048 -> 525 9.8 and 8.8, -> 915 9.8 and 11.7), 40 up to 4,096, 28 beyond (4,608 ->
-//     592 19.1 and 14.9, -> 854 19.2 and 20.2)
-//   Q5_K         none up to 1,024 (512 -> 571 6.0 and 10.1), 16 up to 2,048 (-> 360 10.4 and 6.7, -> 447 10.4 and 10.9), 26
-//     beyond (4,608 -> 603 19.8 and 17.3)
-//   Q6_K         none up to 1,024 (512 -> 246 5.7 and 10.6), 16 beyond (2,304 -> 312 17.6 and 8.9; 4,608 -> 305 24.8 and
-//     15.5, -> 408 24.8 and 29.0; 2,048 -> 471 12.6 and 17.5)
-//   bf16, F32    14 and 25: 8 rows of 6,400 into 300 18.5 and 8.9, 31.6 and 9.2; 33 rows into 64 22.8 and 8.3, 37.5 and 7.4
+//     213 5.3 and 5.9); three from 2,049 to 4,096 columns (Q4_K 0.80 to 1.00 of the time, Q8_0 0.72 to 0.99), else two (2,048 ->
+//     720 9.8 and 8.8, -> 915 9.8 and 11.7; 4,608 -> 592 19.1 and 14.9, -> 854 19.2 and 20.2)
+//   Q5_K         none up to 1,024 (512 -> 571 6.0 and 10.1), one up to 2,048 (-> 360 10.4 and 6.7, -> 447 10.4 and 10.9), two
+//     beyond (4,608 -> 603 19.8 and 17.3, 0.67 to 0.92 of the time)
+//   Q6_K         none up to 1,024 (512 -> 246 5.7 and 10.6); two from 3,073 to 4,352 columns and beyond 5,120 (0.58 to 0.96 of
+//     the time); else one (2,304 -> 312 17.6 and 8.9; 4,608 -> 305 24.8 and 15.5, -> 408 24.8 and 29.0; 2,048 -> 471 12.6 and
+//     17.5)
+//   bf16         one (0.57 to 0.84; two 0.85 to 1.2): 8 rows of 6,400 into 300 18.5 and 8.9; 33 rows into 64 22.8 and 8.3
+//   F32          one up to 256 columns, two beyond (0.36 to 0.89): 8 rows of 6,400 into 300 31.6 and 9.2
 bool rows_pay(const Descriptor& weight, std::int64_t rows) {
     rows = rows_chosen_for(rows);
     const std::int64_t columns = weight.input_dim;
-    std::int64_t most = 0;
+    std::int64_t most = 0;  // workgroups a unit
     switch (weight.encoding) {
-        case kEncQ4K: case kEncQ8_0: most = columns <= 1024 ? 0 : columns <= 2048 ? 24 : columns <= 4096 ? 40 : 28; break;
-        case kEncQ5K: most = columns <= 1024 ? 0 : columns <= 2048 ? 16 : 26; break;
-        case kEncQ6K: most = columns <= 1024 ? 0 : 16; break;
-        case kEncBF16: most = 14; break;
-        case kEncF32: most = 25; break;
+        case kEncQ4K: case kEncQ8_0: most = columns <= 1024 ? 0 : columns > 2048 && columns <= 4096 ? 3 : 2; break;
+        case kEncQ5K: most = columns <= 1024 ? 0 : columns <= 2048 ? 1 : 2; break;
+        case kEncQ6K: most = columns <= 1024 ? 0 : columns > 5120 || (columns > 3072 && columns <= 4352) ? 2 : 1; break;
+        case kEncBF16: most = 1; break;
+        case kEncF32: most = columns <= 256 ? 1 : 2; break;
         default: return false;
     }
-    // (three rows that leave a compute unit room for one workgroup: 5 rows of 7,168 into 2,937 of Q4_K 16.7 and 17.8)
-    if (exact_rows_lds(kMostRows, weight.input_dim) > 80 * 1024) most = std::min<std::int64_t>(most, 16);
     const std::int64_t groups = (rows + kMostRows - 1) / kMostRows;
     constexpr std::int64_t kWorkgroupRows = kExactWaves * kExactPair;
     const std::int64_t workgroups = (weight.output_dim + kWorkgroupRows - 1) / kWorkgroupRows;
-    return groups <= 65535 && workgroups <= most * compute_units() / (kWorkgroupRows * groups);
+    return groups <= 65535 && workgroups <= most * compute_units() / groups;
 }
 
 }  // namespace

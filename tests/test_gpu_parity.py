@@ -352,9 +352,9 @@ def test_exact_linear_small_tiles_of_special_operands(cuda, oracle, encoding):
         test_exact_linear_of_tiny_operands(cuda, oracle, encoding, rows, out_dim, in_dim, -36)
 
 
-@pytest.mark.parametrize("in_dim,out_dim", [*((1024, n) for n in (90, 94, 320, 321, 576, 577, 606)),
-                                            *((1280, n) for n in (368, 369, 544, 545)), (2048, 368), (2048, 545),
-                                            *((2304, n) for n in (368, 369, 592, 593, 928, 929)), (4352, 640), (4352, 641)])
+@pytest.mark.parametrize("in_dim,out_dim", [(256, 368), (256, 369), (512, 736), (512, 737), *((1024, n) for n in (90, 94, 368, 369)),
+                                            *((1280, n) for n in (368, 369, 736, 737)), (2304, 368), (2304, 369),
+                                            *((3328, n) for n in (736, 737, 1104, 1105)), (4352, 737), (5376, 736)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
 def test_exact_linear_carries_the_same_bits_from_four_to_32_rows(cuda, encoding, in_dim, out_dim):
     """Which kernel and which form of it runs from four to 32 rows hangs on the weight alone (outputs and widths on
