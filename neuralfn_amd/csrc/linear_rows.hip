@@ -265,30 +265,38 @@ namespace {
 
 // Four rows and more: while the workgroups, of sixteen weight rows and three input rows each, are few enough.  A
 // unit with two of them takes twice as long as one with one, so that the lines lie at whole workgroups a unit.
-// Where it wins over linear_exact.hip, from 3,700 calls of 256 to 8,192 columns, 4 to 512 rows and up to four workgroups a
-// unit; both in us, this one second, 32 rows:
-//   Q4_K, Q8_0   none up to 1,024 columns, where that kernel needs a turn or two (1,024 -> 439 6.1 and 8.0; Q8_0 512 ->
-//     213 5.3 and 5.9); three from 2,049 to 4,096 columns (Q4_K 0.80 to 1.00 of the time, Q8_0 0.72 to 0.99), else two (2,048 ->
-//     720 9.8 and 8.8, -> 915 9.8 and 11.7; 4,608 -> 592 19.1 and 14.9, -> 854 19.2 and 20.2)
-//   Q5_K         none up to 1,024 (512 -> 571 6.0 and 10.1), one up to 2,048 (-> 360 10.4 and 6.7, -> 447 10.4 and 10.9), two
-//     beyond (4,608 -> 603 19.8 and 17.3, 0.67 to 0.92 of the time)
-//   Q6_K         none up to 1,024 (512 -> 246 5.7 and 10.6); two from 3,073 to 4,352 columns and beyond 5,120 (0.58 to 0.96 of
-//     the time); else one (2,304 -> 312 17.6 and 8.9; 4,608 -> 305 24.8 and 15.5, -> 408 24.8 and 29.0; 2,048 -> 471 12.6 and
-//     17.5)
+// Where it wins over linear_exact.hip, from 5,000 calls of 256 to 8,192 columns, 4 to 512 rows and up to four workgroups
+// a unit; both in us, this one second, 32 rows if not named.  (Four to 32 rows, which take one form: where 32 lose up to
+// a sixth, fewer gain up to half.)
+//   None up to 1,024 columns, where that kernel needs a turn or two: 1,024 -> 439 of Q4_K 6.1 and 8.0, 512 -> 213 of Q8_0
+//     5.3 and 5.9, -> 571 of Q5_K 6.0 and 10.1, -> 246 of Q6_K 5.7 and 10.6.
+//   Q4_K, Q8_0   two: 2,048 -> 720 of Q4_K 9.8 and 8.8 (-> 915 9.8 and 11.7), 4,608 -> 592 19.1 and 14.9.  Three, up to 6,400
+//     columns (three rows then leave a unit room for two) and from 2,049 (Q8_0: 2,048) on: 0.72 to 1.00 of the time up to
+//     4,096, 0.85 to 1.07 from 5,121; between, 1.01 to 1.15, for up to 32 rows only: 4,608 -> 854 19.2 and 20.2, 8 rows of
+//     4,608 -> 991 12.7 and 9.8, 19 of 6,144 -> 1,010 of Q8_0 28.3 and 15.4
+//   Q5_K         two beyond 2,048 columns (4,608 -> 603 19.8 and 17.3; 0.67 to 0.92), and below for up to 32 rows (2,048 ->
+//     447 10.4 and 10.9, -> 360 10.4 and 6.7)
+//   Q6_K         two beyond 2,048 (0.58 to 1.06; 17 rows of 4,864 -> 467 31.7 and 13.2), around 4,608 for up to 32 rows only
+//     (-> 408 24.8 and 29.0, -> 305 24.8 and 15.5); below one (2,048 -> 471 12.6 and 17.5, -> 350 12.6 and 9.8)
 //   bf16         one (0.57 to 0.84; two 0.85 to 1.2): 8 rows of 6,400 into 300 18.5 and 8.9; 33 rows into 64 22.8 and 8.3
 //   F32          one up to 256 columns, two beyond (0.36 to 0.89): 8 rows of 6,400 into 300 31.6 and 9.2
 bool rows_pay(const Descriptor& weight, std::int64_t rows) {
     rows = rows_chosen_for(rows);
     const std::int64_t columns = weight.input_dim;
+    const bool few = rows <= 32, q8 = weight.encoding == kEncQ8_0;
+    const auto within = [columns](std::int64_t first, std::int64_t last) { return columns >= first && columns <= last; };
     std::int64_t most = 0;  // workgroups a unit
     switch (weight.encoding) {
-        case kEncQ4K: case kEncQ8_0: most = columns <= 1024 ? 0 : columns > 2048 && columns <= 4096 ? 3 : 2; break;
-        case kEncQ5K: most = columns <= 1024 ? 0 : columns <= 2048 ? 1 : 2; break;
-        case kEncQ6K: most = columns <= 1024 ? 0 : columns > 5120 || (columns > 3072 && columns <= 4352) ? 2 : 1; break;
+        case kEncQ4K: case kEncQ8_0:
+            most = within(q8 ? 2048 : 2049, few ? 6400 : 4096) || within(5121, 6400) ? 3 : 2;
+            break;
+        case kEncQ5K: most = columns > 2048 || few ? 2 : 1; break;
+        case kEncQ6K: most = columns > 2048 && (few || !within(4353, 4863)) ? 2 : 1; break;
         case kEncBF16: most = 1; break;
         case kEncF32: most = columns <= 256 ? 1 : 2; break;
         default: return false;
     }
+    if (columns <= 1024 && weight.encoding != kEncF32 && weight.encoding != kEncBF16) return false;
     const std::int64_t groups = (rows + kMostRows - 1) / kMostRows;
     constexpr std::int64_t kWorkgroupRows = kExactWaves * kExactPair;
     const std::int64_t workgroups = (weight.output_dim + kWorkgroupRows - 1) / kWorkgroupRows;
