@@ -85,7 +85,7 @@ Projection make_projection(const Descriptor& descriptor, float* output) {
 // Two launches that read the activations once, against one in which every workgroup makes their codes (and a
 // prologue's functions) for itself: the longer the rows and the more of them, the more the dot kernels lose; short
 // rows of few outputs gain nothing that pays for a second launch.  outputs: of all projections of the call in this
-// encoding.  Lines from 1,500 calls of 1,024 to 19,968 columns into 128 to 40,000 outputs (weights from memory), us,
+// encoding.  Lines from 2,400 calls of 768 to 19,968 columns into 128 to 40,000 outputs (weights from memory), us,
 // dot kernel and this one:
 //   Three rows, Q4_K and Q5_K: 7,936 -> 39,936 76 and 43; SwiGLU 16,384 -> 6,656 37 and 21; 2,304 -> 1,504 6.2 and 6.9,
 //     4,096 -> 982 of Q5_K 7.5 and 7.7; gated 1,536 -> 1,488 6.8 and 6.8.
@@ -97,7 +97,9 @@ Projection make_projection(const Descriptor& descriptor, float* output) {
 //     14.5 and 13.1.
 //   Two rows: SwiGLU 18,432 -> 2,304 21 and 14, 18,432 -> 640 15.0 and 11.1; 15,872 -> 4,676 19.6 and 21.4 (a few
 //     workgroups have a second tile then); Q6_K 16,384 -> 2,312 23.3 and 21.1, 14,592 -> 511 15.7 and 18.2.  Shorter rows
-//     of Q4_K and Q5_K: 4,096 -> 16,384 twice 25 and 22, 2,304 -> 20,000 1.09 times as long, 6,656 -> 8,704 13.4 and 15.2.
+//     of Q4_K and Q5_K from 12,289 outputs on: 0.6 to 0.99 of the time up to 2,048 columns, 0.76 to 1.08 from 4,097 to 6,144
+//     and from 8,193 to 11,264 (8,704 -> 15,904 of Q5_K 32.6 and 27.6); between and beyond 1.0 to 1.2 up to some 20,000 outputs;
+//     behind a prologue 0.71 to 1.0 but from 2,049 to 4,096 (up to 1.11 to 18,432 outputs).  6,656 -> 8,704 13.4 and 15.2.
 // The other family stays on its own kernels, although they take longer for some shapes (SwiGLU 18,432 -> 2,304 of Q4_K,
 // three rows, 34 us and not 14): the quantizer launch would overwrite activation records that a verifier call left in
 // the workspace, and at three and four rows the results would not be the logits that the fused lm_head takes its
@@ -108,7 +110,16 @@ bool rows_kernel_pays(std::uint32_t encoding, int prologue, std::int64_t rows, s
     const bool plain = prologue == kPlain;
     if (rows == 2) {
         if (encoding == kEncQ8_0) return false;
-        if (input_dim <= 12288) return encoding != kEncQ6K && outputs > (plain ? 24576 : 12288);
+        if (input_dim <= 12288) {
+            if (encoding == kEncQ6K) return false;
+            const auto within = [input_dim](std::int64_t first, std::int64_t last) {
+                return input_dim >= first && input_dim <= last;
+            };
+            if (input_dim <= 2048) return outputs > 12288;
+            if (!plain) return outputs > (within(2049, 4096) ? 18432 : 12288);
+            if (within(4097, 6144) || within(8193, 11264)) return outputs > 12288;
+            return encoding == kEncQ5K ? outputs > 20480 : outputs > 24576 && input_dim <= 7168;
+        }
         if (!plain) return true;
         return !(outputs > 4096 && outputs <= 5120) && (encoding != kEncQ6K || outputs > 2048);
     }
@@ -116,7 +127,9 @@ bool rows_kernel_pays(std::uint32_t encoding, int prologue, std::int64_t rows, s
         case kEncQ6K:
             if (input_dim < 4096) return outputs > (input_dim <= 2048 ? 4608 : 20480);
             return input_dim <= 10240 || !plain || outputs > 1024;
-        case kEncQ8_0: return plain ? input_dim > 8192 || outputs > 16384 : input_dim >= 6144 || outputs >= 12288;
+        case kEncQ8_0:
+            if (!plain) return input_dim >= 6144 || outputs >= 12288;
+            return input_dim > 8192 || outputs > (input_dim <= 2048 ? 12288 : 16384);
         default: return input_dim > (plain ? 4096 : 2304) || outputs > 3072;
     }
 }

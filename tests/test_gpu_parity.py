@@ -853,7 +853,7 @@ def test_verifier_matrix_core_rows_equal_the_one_row_kernel(cuda, oracle, encodi
                 assert_bits_equal(whole[row:row + 1].contiguous(), part, f"row {row} of {rows}")
 
 
-@pytest.mark.parametrize("in_dim,out_dim", [(256, 40), (2304, 33), (6656, 70), (4096, 12289), (12544, 31), (512, 24577), (12544, 4100)])
+@pytest.mark.parametrize("in_dim,out_dim", [(256, 40), (2304, 33), (6656, 70), (4096, 12289), (12544, 31), (512, 24577), (12544, 4100), (4352, 12289)])
 @pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q6_K, kquant.Q8_0])
 def test_two_and_three_rows_equal_the_one_row_kernel_on_either_kernel(cuda, oracle, encoding, in_dim, out_dim):
     """Two and three rows of the one-row arithmetic run on the matrix cores where that is faster and the
