@@ -20,6 +20,7 @@
 #include <utility>
 
 #include "common.hpp"
+#include "wave_rows.hpp"
 
 namespace nfn {
 
@@ -189,10 +190,67 @@ __device__ __forceinline__ void for_each_piece(F&& f, std::integer_sequence<int,
     (f(std::integral_constant<int, I>{}), ...);
 }
 
+// Lanes of both halves: lanes 0 to 31 return the sum of `a` over l and l + 32, the others that of `b`.
+// (The instruction swaps the upper half of its first operand with the lower half of its second.)
+__device__ __forceinline__ double fold_halves(double a, double b) {
+    const std::uint64_t x = __builtin_bit_cast(std::uint64_t, a), y = __builtin_bit_cast(std::uint64_t, b);
+    const auto low = __builtin_amdgcn_permlane32_swap(static_cast<std::uint32_t>(x), static_cast<std::uint32_t>(y), false, false);
+    const auto high = __builtin_amdgcn_permlane32_swap(static_cast<std::uint32_t>(x >> 32), static_cast<std::uint32_t>(y >> 32),
+                                                       false, false);
+    return __builtin_bit_cast(double, low[0] | static_cast<std::uint64_t>(high[0]) << 32) +
+        __builtin_bit_cast(double, low[1] | static_cast<std::uint64_t>(high[1]) << 32);
+}
+// ... of neighbouring rows of sixteen lanes: rows 0 and 2 return `a` over their pair of rows, rows 1 and 3 `b`.
+__device__ __forceinline__ double fold_rows(double a, double b) {
+    const std::uint64_t x = __builtin_bit_cast(std::uint64_t, a), y = __builtin_bit_cast(std::uint64_t, b);
+    const auto low = __builtin_amdgcn_permlane16_swap(static_cast<std::uint32_t>(x), static_cast<std::uint32_t>(y), false, false);
+    const auto high = __builtin_amdgcn_permlane16_swap(static_cast<std::uint32_t>(x >> 32), static_cast<std::uint32_t>(y >> 32),
+                                                       false, false);
+    return __builtin_bit_cast(double, low[0] | static_cast<std::uint64_t>(high[0]) << 32) +
+        __builtin_bit_cast(double, low[1] | static_cast<std::uint64_t>(high[1]) << 32);
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double value) {
+    const std::uint64_t x = __builtin_bit_cast(std::uint64_t, value);
+    const std::uint32_t low = static_cast<std::uint32_t>(dpp_move<CTRL>(static_cast<int>(x)));
+    const std::uint32_t high = static_cast<std::uint32_t>(dpp_move<CTRL>(static_cast<int>(x >> 32)));
+    return value + __builtin_bit_cast(double, low | static_cast<std::uint64_t>(high) << 32);
+}
+
+// The wave's sums of R values each for two weight rows, in every lane, rounded once: four values at a time are
+// folded into the four rows of sixteen lanes, which costs a third of a butterfly for each.
+template <int R>
+__device__ __forceinline__ void wave_sums(const double (&values)[kExactPair][R], float (&totals)[kExactPair][R]) {
+    static_assert(kExactPair == 2);
+    const auto within_row = [](double value) {
+        value = dpp_add<kQuadXor1>(value);
+        value = dpp_add<kQuadXor2>(value);
+        value = dpp_add<kHalfMirror>(value);
+        return static_cast<float>(dpp_add<kRowMirror>(value));
+    };
+#pragma unroll
+    for (int r = 0; r < R; r += 2) {
+        const double first = fold_halves(values[0][r], values[1][r]);
+        const bool two = r + 1 < R;
+        const double second = two ? fold_halves(values[0][two ? r + 1 : r], values[1][two ? r + 1 : r]) : first;
+        const float folded = within_row(fold_rows(first, second));
+        totals[0][r] = lane_value(folded, 0);
+        totals[1][r] = lane_value(folded, 32);
+        if (two) {
+            totals[0][two ? r + 1 : r] = lane_value(folded, 16);
+            totals[1][two ? r + 1 : r] = lane_value(folded, 48);
+        }
+    }
+}
+
 // Calls take(row, sums) for the weight rows `first`, `first + step`, ... below `output_dim`, two at a
 // time (rows 2 p and 2 p + 1); sums[r]: this wave's total for input row r, in every lane.  A row's
-// sum does not depend on the launch: lane l adds the units l, l + 64, ... in rising order, the even
-// and the odd columns in a chain each, and the lanes meet in a butterfly.
+// sum does not depend on the launch: lane l adds the units l, l + span, ... in rising order and the lanes
+// meet in doubles.  Every fourth column is added in a chain of its own; of Q8_0 sixteen columns are added in two
+// chains of eight and go to one of two sums in turn, for 12 % more additions (4,352 columns, three rows 11.0 -> 11.9 us).
+// Rounding against float64 at 4,096 / 8,192 columns: 7.7e-8 / 1.02e-7 (Q4_K, Q5_K), 7.4e-8 / 9.7e-8 (Q6_K), 6.8e-8 / 7.4e-8
+// (Q8_0); on the matrix-core kernel, which more rows run on, 1.2e-7 / 1.4e-7, 8.7e-8 / 1.1e-7 and 7.4e-8 / 8.9e-8.  (Two
+// chains a lane and a float butterfly: 1.2e-7 / 1.6e-7, and 1 % slower.)
 template <std::uint32_t ENC, int R, typename Take>
 __device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__ data, std::int64_t row_stride,
                                                 std::int64_t output_dim, std::int64_t input_dim,
@@ -201,10 +259,14 @@ __device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__
     const int lane = threadIdx.x & 63;
     const int units = static_cast<int>(input_dim >> 6);
     const int turns = (units + 63) / 64;
+    // A last turn of eight lanes or fewer takes twice as long as one of twelve or more (4,608 columns, one row 8.2 us,
+    // 4,864 6.5): it gets sixteen units at least.
+    constexpr int kLeastUnits = 16;
+    const int span = turns > 1 && units - 64 * (turns - 1) < kLeastUnits ? (units - kLeastUnits + turns - 2) / (turns - 1) : 64;
     if (first_pair >= end_pair) return;
     ExactUnit<ENC> now[kExactPair], next[kExactPair];
     auto load = [&](ExactUnit<ENC> (&into)[kExactPair], std::int64_t pair, int turn) {
-        const int unit = min(lane + 64 * turn, units - 1);
+        const int unit = min(lane + span * turn, units - 1);
 #pragma unroll
         for (int k = 0; k < kExactPair; ++k) {
             into[k].load(data + min(pair * kExactPair + k, output_dim - 1) * row_stride, unit);
@@ -212,16 +274,19 @@ __device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__
     };
     load(now, first_pair, 0);
     for (std::int64_t pair = first_pair; pair < end_pair; pair += pair_step) {
-        float sums[kExactPair][R][2] = {};  // even and odd columns: shorter chains, smaller errors
+        constexpr bool kShort = ENC == kEncQ8_0;
+        constexpr int kSums = kShort ? 2 : 4;
+        float sums[kExactPair][R][kSums] = {};
         for (int turn = 0; turn < turns; ++turn) {
             const bool more = turn + 1 < turns;
             // (unconditional: behind the last pair its own bytes are read again)
             load(next, more ? pair : pair + pair_step < end_pair ? pair + pair_step : pair, more ? turn + 1 : 0);
-            const int unit = lane + 64 * turn;
-            if (unit < units) {
+            const int unit = lane + span * turn;
+            if (lane < span && unit < units) {
 #pragma unroll
                 for (int k = 0; k < kExactPair; ++k) now[k].prepare(unit);
                 const float* x = staged + unit * kExactPitch;
+                float chains[kExactPair][R][2];  // (Q8_0)
                 const auto four = [&](auto index) {
                     constexpr int kI = decltype(index)::value;
                     exact_f32x4 w[kExactPair];
@@ -233,8 +298,16 @@ __device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__
                             *reinterpret_cast<const exact_f32x4*>(x + r * units * kExactPitch + 4 * kI);
 #pragma unroll
                         for (int k = 0; k < kExactPair; ++k) {
+                            float (&chain)[2] = chains[k][r];
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) sums[k][r][j & 1] = fmaf(v[j], w[k][j], sums[k][r][j & 1]);
+                            for (int j = 0; j < 4; ++j) {
+                                if constexpr (!kShort) {
+                                    sums[k][r][j] = fmaf(v[j], w[k][j], sums[k][r][j]);
+                                } else {
+                                    chain[j & 1] = kI % 4 == 0 && j < 2 ? v[j] * w[k][j] : fmaf(v[j], w[k][j], chain[j & 1]);
+                                }
+                            }
+                            if constexpr (kShort && kI % 4 == 3) sums[k][r][kI / 4 & 1] += chain[0] + chain[1];
                         }
                     }
                 };
@@ -243,13 +316,21 @@ __device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__
 #pragma unroll
             for (int k = 0; k < kExactPair; ++k) now[k] = next[k];
         }
+        double both[kExactPair][R];
+        float totals[kExactPair][R];
+#pragma unroll
+        for (int k = 0; k < kExactPair; ++k) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                both[k][r] = static_cast<double>(sums[k][r][0]) + static_cast<double>(sums[k][r][1]);
+                if constexpr (!kShort) both[k][r] += static_cast<double>(sums[k][r][2]) + static_cast<double>(sums[k][r][3]);
+            }
+        }
+        wave_sums<R>(both, totals);
 #pragma unroll
         for (int k = 0; k < kExactPair; ++k) {
             const std::int64_t row = pair * kExactPair + k;
-            float totals[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) totals[r] = wave_sum(sums[k][r][0] + sums[k][r][1]);
-            if (row < output_dim) take(row, totals);
+            if (row < output_dim) take(row, totals[k]);
         }
     }
 }

@@ -389,6 +389,23 @@ def test_exact_linear_of_row_groups(cuda, oracle, encoding, rows, out_dim, in_di
             assert_bits_equal(y[first:first + 3].contiguous(), part, f"rows {first} on")
 
 
+@pytest.mark.parametrize("in_dim", [4096, 4352, 8192])
+@pytest.mark.parametrize("encoding", ALL_PACKED)
+def test_exact_linear_of_few_outputs_rounds_no_more_than_of_many(cuda, encoding, in_dim):
+    """Few outputs run on the vector kernel and many on the matrix-core one (eight rows of 320 and of 8,192): against
+    float64 the former are no further off, over 2,560 values each, whose root mean squares are known to 1.4 percent
+    (1 / sqrt(2 x 2,560)): three times that for their ratio is 6 percent."""
+    packed = torch_().from_numpy(kquant.quantize(encoding, kquant.synthetic_weights(62, 256, in_dim)).reshape(256, -1)).to(cuda)
+    chosen = torch_().from_numpy(np.random.default_rng(64).integers(0, 256, 8192)).to(cuda)
+    weight = tile_ops.PackedWeight(encoding, 8192, in_dim, packed.index_select(0, chosen).reshape(-1))
+    few = tile_ops.PackedWeight(encoding, 320, in_dim, packed.index_select(0, chosen[:320]).reshape(-1))
+    x = to_device(kquant.synthetic_activations(63, 8, in_dim), cuda)
+    exact = x.double() @ tile_ops.dequantize(few).reshape(320, in_dim).double().T.contiguous()
+    error = [((y.double() - exact).norm() / exact.norm()).item()
+             for y in (tile_ops.linear(few, x), tile_ops.linear(weight, x)[:, :320])]
+    assert error[0] <= 1.06 * error[1], error
+
+
 @pytest.mark.parametrize("exponent", [-33, -35, -36, -37])
 @pytest.mark.parametrize("rows,out_dim,in_dim", [(3, 67, 512), (5, 67, 512), (60, 5000, 256), (100, 6600, 256), (200, 6600, 256)])
 @pytest.mark.parametrize("encoding", ALL_PACKED + [kquant.F32, kquant.BF16])
