@@ -1357,9 +1357,10 @@ namespace {
 
 // Keys of a row that a workgroup takes alone in one launch although there is a workspace: what the merge
 // takes is more than a few tiles side by side gain.  One row / seven rows of 32 heads over 2, us, split -> alone:
-// 90 keys 11.6 / 12.3 -> 7.2 / 9.1, 137 11.5 / 12.2 -> 7.3 / 9.8, 230 10.7 / 12.4 -> 9.3 / 9.9; 350 (six tiles) 10.8 / 12.7 and
-// 11.2 / 12.4.  A block's rows on the matrix cores, where the head size allows (7 rows of 137 keys on the vector
-// kernel 11.8), else up to three tiles (16 heads over 4, 4 rows of 137 keys 13.5 -> 11.8).
+// 90 keys 12.4 / 12.3 -> 9.0 / 9.1, 137 12.3 / 12.2 -> 9.5 / 9.8, 230 11.7 / 12.4 -> 9.5 / 9.9; seven rows of 350 (six tiles)
+// 12.7 and 12.4.  On the matrix cores, where the head size allows, as with shares: the vector kernel takes one row of 90
+// keys in 7.3 and of 230 in 10.0, but is 3.6e-7 off float64 where this is 1.9e-7 (7 rows of 137 keys 11.8).  Else up to
+// three tiles (16 heads over 4, 4 rows of 137 keys 13.5 -> 11.8).
 bool one_launch(const AttentionArguments& a, std::int64_t tiles) {
     return tiles <= (grouped_form_fits(a) ? 4 : 3);
 }
@@ -1413,7 +1414,8 @@ void launch_gqa_decode_split(const NfnNativeTileGlimmerGqaDecodeDescriptorV1& d,
     const AttentionArguments a = decode_arguments(d);
     const std::int64_t tiles = tiles_of(a.sliding_window);
     if (!vector_form_fits(a) || one_launch(a, tiles)) {
-        launch_attention(a, 1, tiles, stream);  // little to split, or no vector form: one launch
+        // little to split, or no vector form: one launch
+        launch_attention(a, 1, tiles, stream, tiles >= 2);
         return;
     }
     launch_split(a, 1, tiles, partials, gqa_decode_split_workspace_bytes(d.query_heads, d.head_dim),
@@ -1466,7 +1468,7 @@ void launch_block_attention(const NfnNativeTileDFlashBlockAttentionDescriptorV1&
     if (partials != nullptr && vector_form_fits(a) && !one_launch(a, tiles)) {
         launch_split(a, d.query_rows, tiles, partials, partial_bytes, stream);
     } else {
-        launch_attention(a, d.query_rows, tiles, stream, partials != nullptr && tiles >= 2 && d.query_rows > 1);
+        launch_attention(a, d.query_rows, tiles, stream, partials != nullptr && tiles >= 2);
     }
 }
 
