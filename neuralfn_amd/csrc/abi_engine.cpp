@@ -2,6 +2,7 @@
 // argument checks as the reference's wrappers make them
 // (neuralfn/csrc/native_train/tile_ops.cu:3601-3800, 4734-4775, 5013-5030,
 // 5150-5260, 5348-5362, 5421-5445, 6377-6388, 6944-6951), then one launch.
+#include "attention.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -180,16 +181,6 @@ int run_fused_decode(const NfnNativeTileGlimmerFusedDecodeAttentionDescriptorV1*
     // holds for every key range shorter than the ring (and for the device
     // form, whose window is at most the ring).  Otherwise the commit follows.
     const bool commit_first = on_device || d->position - d->first_key_position < d->cache_capacity;
-    launch_qk_norm_scale_rope(d->query, d->key, query_source != nullptr ? &query_weight : nullptr,
-                              d->query_norm_centered != 0,
-                              key_source != nullptr ? &key_weight : nullptr,
-                              d->key_norm_centered != 0, 1, d->query_heads, d->kv_heads,
-                              d->head_dim, d->norm_eps, d->query_scale, d->position,
-                              device_position, d->rope_theta,
-                              d->rope_layout == NFN_NATIVE_TILE_GLIMMER_ROPE_INTERLEAVED,
-                              d->apply_rope != 0, commit_first ? d->key_cache_bf16 : nullptr,
-                              d->value_cache_bf16, d->current_value, d->cache_capacity,
-                              d->cache_row_stride, stream);
     NfnNativeTileGlimmerGqaDecodeDescriptorV1 attention{};
     attention.query = d->query;
     attention.current_key = d->key;
@@ -205,6 +196,34 @@ int run_fused_decode(const NfnNativeTileGlimmerFusedDecodeAttentionDescriptorV1*
     attention.cache_capacity = d->cache_capacity;
     attention.cache_row_stride = d->cache_row_stride;
     attention.scale = d->attention_scale;
+    if (split_partials != nullptr && commit_first) {
+        RowPreparation preparation{};
+        preparation.query = d->query;
+        preparation.key = d->key;
+        preparation.key_cache = d->key_cache_bf16;
+        preparation.value_cache = d->value_cache_bf16;
+        preparation.query_weight = norm_weight(query_source != nullptr ? &query_weight : nullptr, d->query_norm_centered != 0);
+        preparation.key_weight = norm_weight(key_source != nullptr ? &key_weight : nullptr, d->key_norm_centered != 0);
+        preparation.eps = d->norm_eps;
+        preparation.query_scale = d->query_scale;
+        preparation.theta = static_cast<double>(d->rope_theta);
+        preparation.interleaved = d->rope_layout == NFN_NATIVE_TILE_GLIMMER_ROPE_INTERLEAVED;
+        preparation.apply_rope = d->apply_rope != 0;
+        if (launch_prepared_gqa_decode_split(attention, preparation, device_position, sliding_window,
+                                             on_device && d->apply_rope == 0, split_partials, stream)) {
+            return launch_status();
+        }
+    }
+    launch_qk_norm_scale_rope(d->query, d->key, query_source != nullptr ? &query_weight : nullptr,
+                              d->query_norm_centered != 0,
+                              key_source != nullptr ? &key_weight : nullptr,
+                              d->key_norm_centered != 0, 1, d->query_heads, d->kv_heads,
+                              d->head_dim, d->norm_eps, d->query_scale, d->position,
+                              device_position, d->rope_theta,
+                              d->rope_layout == NFN_NATIVE_TILE_GLIMMER_ROPE_INTERLEAVED,
+                              d->apply_rope != 0, commit_first ? d->key_cache_bf16 : nullptr,
+                              d->value_cache_bf16, d->current_value, d->cache_capacity,
+                              d->cache_row_stride, stream);
     if (on_device && split_partials != nullptr) {
         launch_gqa_decode_split_device_position(attention, device_position, sliding_window,
                                                 d->apply_rope == 0, split_partials, stream);

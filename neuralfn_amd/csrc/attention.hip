@@ -12,7 +12,8 @@
 // The one-token form is the block form with one query row whose own key is
 // the only block row.  A third kernel serves head_dim 128 with four or more
 // query heads per key/value head on the matrix cores, one workgroup per group
-// of up to 16 such heads: the split one-token form and blocks of many rows.
+// of up to 16 such heads: blocks of rows.  (One row with a workspace: attention_row.hip.)
+#include "attention.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -22,8 +23,7 @@ namespace {
 
 constexpr int kMaxWaves = 8;   // 512 threads: 256 vector registers per lane
 constexpr int kMaxHeadDim = 256;
-constexpr int kMaxSplits = 128;    // most shares of one head's keys in the split form
-constexpr int kVectorSplits = 32;  // ... when every query head has workgroups of its own
+constexpr int kVectorSplits = 32;  // most shares of one head's keys when every query head has workgroups of its own
 constexpr int kOwned = kMaxHeadDim / kWave;  // output dimensions per lane
 
 struct AttentionArguments {
@@ -63,11 +63,6 @@ __device__ __forceinline__ void resolve_position(AttentionArguments& a) {
     const std::int64_t position = a.device_position[0];
     a.context_length = position;
     if (a.whole_context) a.sliding_window = position + 1;
-}
-
-// floats per (query row, query head, split) in the partial buffer
-__host__ __device__ constexpr std::int64_t partial_floats(std::int64_t head_dim) {
-    return head_dim + 2;
 }
 
 __device__ __forceinline__ float wave_max_f(float value) {
@@ -662,24 +657,45 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void attention_vector_kernel(Att
 // Split form, second launch: one workgroup per (query row, query head) merges
 // the shares.  Four threads share an output dimension and take every fourth
 // share each, so that the loads of many shares are in flight together (read
-// one after the other, 32 shares cost more than the attention itself).
+// one after the other, 32 shares cost more than the attention itself); the first
+// kMergeAhead of a thread are requested before the factors are worked out.
+// With `query` the output row holds the prepared query of the head, which moves there; workgroups past
+// the heads copy the prepared key (RowPreparation, attention.hpp).
 constexpr int kMergeLanes = 4;
+constexpr int kMergeAhead = 8;
 
 __global__ __launch_bounds__(kMaxHeadDim * kMergeLanes) void attention_merge_kernel(
-    const float* __restrict__ partials, float* __restrict__ output, int splits, int head_dim) {
+    const float* __restrict__ partials, float* output, int splits, int head_dim, int heads, float* query,
+    const float* key_copy, float* key, int key_floats) {
     __shared__ float factor[kMaxSplits];
     __shared__ float wave_part[2][kMaxHeadDim * kMergeLanes / kWave];
     __shared__ float lane_sum[kMergeLanes][kMaxHeadDim];
+    const int tid = threadIdx.x;
+    if (static_cast<int>(blockIdx.x) >= heads) {
+        const int index = (static_cast<int>(blockIdx.x) - heads) * static_cast<int>(blockDim.x) + tid;
+        if (index < key_floats) key[index] = key_copy[index];
+        return;
+    }
     const std::int64_t stride = partial_floats(head_dim);
     const float* mine = partials + static_cast<std::int64_t>(blockIdx.x) * splits * stride;
-    const int tid = threadIdx.x;
+    float* row = output + static_cast<std::int64_t>(blockIdx.x) * head_dim;
     const int wave = tid >> 6;
     const int lane = tid & 63;
     const int dims = static_cast<int>(blockDim.x) / kMergeLanes;  // head_dim rounded up to waves
+    const int d = tid % dims;
+    const int share_lane = tid / dims;
 
     // thread s holds share s (at most 128 shares, at least 256 threads)
     const float maximum = tid < splits ? mine[tid * stride] : -INFINITY;
     const float denominator = tid < splits ? mine[tid * stride + 1] : 0.0f;
+    float ahead[kMergeAhead];
+#pragma unroll
+    for (int n = 0; n < kMergeAhead; ++n) {
+        const int s = share_lane + n * kMergeLanes;
+        ahead[n] = d < head_dim && s < splits ? mine[s * stride + 2 + d] : 0.0f;
+    }
+    const bool moves = query != nullptr && share_lane == 0 && d < head_dim;
+    const float moved = moves ? row[d] : 0.0f;
     const float wave_maximum = wave_max_f(maximum);
     if (lane == 0) wave_part[0][wave] = wave_maximum;
     __syncthreads();
@@ -691,20 +707,24 @@ __global__ __launch_bounds__(kMaxHeadDim * kMergeLanes) void attention_merge_ker
     __syncthreads();
     const float total = wave_part[1][0] + wave_part[1][1];
 
-    const int d = tid % dims;
-    const int share_lane = tid / dims;
     float sum = 0.0f;
     if (d < head_dim) {
+#pragma unroll
+        for (int n = 0; n < kMergeAhead; ++n) {
+            const int s = share_lane + n * kMergeLanes;
+            if (s < splits) sum = fmaf(ahead[n], factor[s], sum);
+        }
 #pragma unroll 4
-        for (int s = share_lane; s < splits; s += kMergeLanes) {
+        for (int s = share_lane + kMergeAhead * kMergeLanes; s < splits; s += kMergeLanes) {
             sum = fmaf(mine[s * stride + 2 + d], factor[s], sum);
         }
     }
     lane_sum[share_lane][d] = sum;
     __syncthreads();
+    if (moves) query[static_cast<std::int64_t>(blockIdx.x) * head_dim + d] = moved;
     if (share_lane == 0 && d < head_dim) {
         const float all = (lane_sum[0][d] + lane_sum[1][d]) + (lane_sum[2][d] + lane_sum[3][d]);
-        output[static_cast<std::int64_t>(blockIdx.x) * head_dim + d] = all / total;
+        row[d] = all / total;
     }
 }
 
@@ -732,42 +752,17 @@ __global__ __launch_bounds__(kMaxHeadDim * kMergeLanes) void attention_merge_ker
 // of a key, whose halves go to two instructions (column i standing for dimension
 // 32p + 2i in one and 32p + 2i + 1 in the other).
 // ---------------------------------------------------------------------------
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int kGroupWaves = 8;
-constexpr int kGroupHeads = 16;
-constexpr int kGroupHeadDim = 128;
 constexpr int kGroupRowPad = 4;  // floats between the rows of a wave's result in LDS
-constexpr int kStageRowBytes = 2 * kGroupHeadDim + 16;  // a staged value row and its pad
 constexpr int kStageBytes = kWave * kStageRowBytes;      // a wave's tile of value rows
-constexpr int kGroupMinHeads = 4;  // fewer query heads per key/value head: the vector form
 
 struct QueryTerms {
     bf16x8 high, middle, low;
 };
 
-// x = high + middle + low exactly, every term a bf16: each term takes the next eight
-// significant bits of what is left (truncation, so the remainders are exact)
 __device__ __forceinline__ QueryTerms split_query(const float (&x)[8]) {
     std::uint32_t words[3][4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        std::uint32_t term[3][2];
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            float rest = x[2 * w + half];
-#pragma unroll
-            for (int t = 0; t < 3; ++t) {
-                term[t][half] = __float_as_uint(rest) & 0xffff0000u;
-                rest -= __uint_as_float(term[t][half]);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            words[t][w] = __builtin_amdgcn_perm(term[t][1], term[t][0], 0x07060302u);
-        }
-    }
+    split_terms(x, words);
     QueryTerms terms;
     terms.high = __builtin_bit_cast(bf16x8, make_uint4(words[0][0], words[0][1], words[0][2], words[0][3]));
     terms.middle = __builtin_bit_cast(bf16x8, make_uint4(words[1][0], words[1][1], words[1][2], words[1][3]));
@@ -785,9 +780,6 @@ __device__ __forceinline__ uint4 pack_as_cached(float4 low, float4 high) {
                       pair(high.z, high.w));
 }
 
-// BLOCK: of several query rows.  (One row's tiles have no rows of a block: the code for them in its kernel makes a
-// decode step of eight layers 0.5 to 1 us a layer longer.)
-template <bool BLOCK>
 __global__ __launch_bounds__(kGroupWaves * kWave) void attention_grouped_kernel(AttentionArguments a) {
     // waves x kStageBytes: a value tile per wave; at the end the waves' results
     // (maxima, denominators, accumulators: less than that) in the same memory
@@ -1004,19 +996,13 @@ __global__ __launch_bounds__(kGroupWaves * kWave) void attention_grouped_kernel(
          tile += tile_step, tile_slot = ring_row(tile_slot + slot_step)) {
         const int in_tile =
             static_cast<int>(tiled_last - tile < kWave - 1 ? tiled_last - tile : kWave - 1);
-        if constexpr (BLOCK) {
-            // keys of the tile from here on are rows of the block
-            const int left = a.context_length <= tile ? 0
-                : static_cast<int>(a.context_length - tile < kWave ? a.context_length - tile : kWave);
-            if (is_straight(tile, tile_slot)) {
-                load_straight(tile_slot);
-            } else if (left <= in_tile && in_tile - left < kStaged) {
-                load_mixed(tile, tile_slot, in_tile, left);
-            } else {
-                load_general(tile, tile_slot, in_tile);
-            }
-        } else if (is_straight(tile, tile_slot)) {
+        // keys of the tile from here on are rows of the block
+        const int left = a.context_length <= tile ? 0
+            : static_cast<int>(a.context_length - tile < kWave ? a.context_length - tile : kWave);
+        if (is_straight(tile, tile_slot)) {
             load_straight(tile_slot);
+        } else if (left <= in_tile && in_tile - left < kStaged) {
+            load_mixed(tile, tile_slot, in_tile, left);
         } else {
             load_general(tile, tile_slot, in_tile);
         }
@@ -1281,13 +1267,8 @@ void launch_attention(const AttentionArguments& arguments, std::int64_t query_ro
             ((arguments.heads_per_kv + kGroupHeads - 1) / kGroupHeads);
         const dim3 grid(static_cast<unsigned>(query_rows * groups), splits), block(static_cast<unsigned>(waves * kWave));
         const std::size_t lds = static_cast<std::size_t>(waves) * kStageBytes;
-        if (query_rows == 1) {
-            allow_large_lds<attention_grouped_kernel<false>>(kGroupWaves * kStageBytes);
-            hipLaunchKernelGGL(attention_grouped_kernel<false>, grid, block, lds, stream, arguments);
-        } else {
-            allow_large_lds<attention_grouped_kernel<true>>(kGroupWaves * kStageBytes);
-            hipLaunchKernelGGL(attention_grouped_kernel<true>, grid, block, lds, stream, arguments);
-        }
+        allow_large_lds<attention_grouped_kernel>(kGroupWaves * kStageBytes);
+        hipLaunchKernelGGL(attention_grouped_kernel, grid, block, lds, stream, arguments);
         return;
     }
     const dim3 grid(static_cast<unsigned>(query_rows * arguments.query_heads), splits);
@@ -1382,16 +1363,6 @@ void launch_split(AttentionArguments a, std::int64_t query_rows, std::int64_t ti
     std::int64_t splits = compute_units() / groups;
     if (splits > (grouped ? kMaxSplits : kVectorSplits)) splits = grouped ? kMaxSplits : kVectorSplits;
     if (splits > tiles) splits = tiles;
-    // One query row: at least two tiles a share, two waves a workgroup.  A 2,048-key window
-    // in 16 shares of two waves takes 11.1 us with its merge, in 32 shares of one wave 12.1 us
-    // (12 or 24 shares: 11.7; 8: 11.9); long contexts and blocks are not touched by this
-    // (32,768 keys: 128 shares 15.1 us, 96: 15.4, 64: 17.1; a 16-row block: 8..24 shares 16.1 us).
-    // Sixteen shares of three waves at 41 to 48 tiles: 300 calls of 33 to 48 tiles and 16 to 48 heads over 2 to 8 take
-    // 1.5 % less with them there (2,620 keys of 16 heads over 2 12.4 -> 11.5 us), and 1 % more at 33 to 40 tiles.
-    if (query_rows == 1 && grouped && 2 * splits > tiles && tiles >= 4) {
-        splits = (tiles + 1) / 2;
-        if (tiles > 40 && tiles <= 48) splits = 16;
-    }
     if (splits < 2) splits = 2;
     if (splits > partial_bytes / share_bytes) splits = partial_bytes / share_bytes;
     if (splits < 2) {
@@ -1401,16 +1372,59 @@ void launch_split(AttentionArguments a, std::int64_t query_rows, std::int64_t ti
     }
     a.splits = static_cast<int>(splits);
     launch_attention(a, query_rows, (tiles + splits - 1) / splits, stream);
-    const int threads = static_cast<int>((a.head_dim + kWave - 1) / kWave * kWave) * kMergeLanes;
-    hipLaunchKernelGGL(attention_merge_kernel,
-                       dim3(static_cast<unsigned>(query_rows * a.query_heads)), dim3(threads), 0,
-                       stream, partials, a.output, a.splits, static_cast<int>(a.head_dim));
+    launch_attention_merge(partials, a.output, a.splits, query_rows * a.query_heads, a.head_dim, nullptr, nullptr,
+                           nullptr, 0, stream);
+}
+
+RowAttention row_call(const NfnNativeTileGlimmerGqaDecodeDescriptorV1& d, const RowPreparation* preparation) {
+    RowAttention call{};
+    call.query = d.query;
+    call.current_key = d.current_key;
+    call.current_value = d.current_value;
+    call.key_cache = d.key_cache_bf16;
+    call.value_cache = d.value_cache_bf16;
+    call.output = d.output;
+    call.query_heads = d.query_heads;
+    call.kv_heads = d.kv_heads;
+    call.head_dim = d.head_dim;
+    call.position = d.position;
+    call.first_key_position = d.first_key_position;
+    call.cache_capacity = d.cache_capacity;
+    call.cache_row_stride = d.cache_row_stride;
+    call.scale = d.scale;
+    call.preparation = preparation;
+    return call;
 }
 
 }  // namespace
 
+void launch_attention_merge(const float* partials, float* output, int splits, std::int64_t heads, std::int64_t head_dim,
+                            float* query, const float* key_copy, float* key, std::int64_t key_floats,
+                            hipStream_t stream) {
+    const int threads = static_cast<int>((head_dim + kWave - 1) / kWave * kWave) * kMergeLanes;
+    const std::int64_t copies = key_copy != nullptr ? (key_floats + threads - 1) / threads : 0;
+    hipLaunchKernelGGL(attention_merge_kernel, dim3(static_cast<unsigned>(heads + copies)), dim3(threads), 0, stream,
+                       partials, output, splits, static_cast<int>(head_dim), static_cast<int>(heads), query, key_copy,
+                       key, static_cast<int>(key_floats));
+}
+
+bool launch_prepared_gqa_decode_split(const NfnNativeTileGlimmerGqaDecodeDescriptorV1& d,
+                                      const RowPreparation& preparation, const std::int64_t* device_position,
+                                      std::int64_t sliding_window, bool whole_context, float* partials,
+                                      hipStream_t stream) {
+    RowAttention call = row_call(d, &preparation);
+    call.device_position = device_position;
+    call.sliding_window = sliding_window;
+    call.whole_context = whole_context;
+    return launch_attention_row(call, partials, gqa_decode_split_workspace_bytes(d.query_heads, d.head_dim), stream);
+}
+
 void launch_gqa_decode_split(const NfnNativeTileGlimmerGqaDecodeDescriptorV1& d, float* partials,
                              hipStream_t stream) {
+    if (launch_attention_row(row_call(d, nullptr), partials,
+                             gqa_decode_split_workspace_bytes(d.query_heads, d.head_dim), stream)) {
+        return;
+    }
     const AttentionArguments a = decode_arguments(d);
     const std::int64_t tiles = tiles_of(a.sliding_window);
     if (!vector_form_fits(a) || one_launch(a, tiles)) {
@@ -1426,6 +1440,13 @@ void launch_gqa_decode_split_device_position(const NfnNativeTileGlimmerGqaDecode
                                              const std::int64_t* device_position,
                                              std::int64_t sliding_window, bool whole_context,
                                              float* partials, hipStream_t stream) {
+    RowAttention call = row_call(d, nullptr);
+    call.device_position = device_position;
+    call.sliding_window = sliding_window;
+    call.whole_context = whole_context;
+    if (launch_attention_row(call, partials, gqa_decode_split_workspace_bytes(d.query_heads, d.head_dim), stream)) {
+        return;
+    }
     AttentionArguments a = decode_arguments(d);
     a.device_position = device_position;
     a.sliding_window = sliding_window;
@@ -1465,6 +1486,26 @@ void launch_block_attention(const NfnNativeTileDFlashBlockAttentionDescriptorV1&
         if (window < longest) longest = window;
     }
     const std::int64_t tiles = tiles_of(longest);
+    // one row that sees no other row of a block
+    if (partials != nullptr && d.query_rows == 1 && (a.causal != 0 || d.block_rows == 1)) {
+        RowAttention call{};
+        call.query = d.query;
+        call.current_key = d.block_key;
+        call.current_value = d.block_value;
+        call.key_cache = d.key_cache_bf16;
+        call.value_cache = d.value_cache_bf16;
+        call.output = d.output;
+        call.query_heads = d.query_heads;
+        call.kv_heads = d.kv_heads;
+        call.head_dim = d.head_dim;
+        call.position = d.context_length;
+        const std::int64_t first = d.context_length - d.sliding_window + (a.causal != 0 ? 1 : 0);
+        call.first_key_position = first > 0 ? first : 0;
+        call.cache_capacity = d.cache_capacity;
+        call.cache_row_stride = d.cache_row_stride;
+        call.scale = d.scale;
+        if (launch_attention_row(call, partials, partial_bytes, stream)) return;
+    }
     if (partials != nullptr && vector_form_fits(a) && !one_launch(a, tiles)) {
         launch_split(a, d.query_rows, tiles, partials, partial_bytes, stream);
     } else {

@@ -122,6 +122,13 @@ void launch_gqa_decode_device_position(const NfnNativeTileGlimmerGqaDecodeDescri
 std::int64_t gqa_decode_split_workspace_bytes(std::int64_t query_heads, std::int64_t head_dim);
 void launch_gqa_decode_split(const NfnNativeTileGlimmerGqaDecodeDescriptorV1& descriptor,
                              float* partials, hipStream_t stream);
+// ... with the per-head norms, scale, rotation and cache commit of launch_qk_norm_scale_rope in the same launches
+// (device_position null: at the descriptor's position); false, and nothing launched, where that does not apply.
+struct RowPreparation;
+bool launch_prepared_gqa_decode_split(const NfnNativeTileGlimmerGqaDecodeDescriptorV1& descriptor,
+                                      const RowPreparation& preparation, const std::int64_t* device_position,
+                                      std::int64_t sliding_window, bool whole_context, float* partials,
+                                      hipStream_t stream);
 // The same with the position read from device memory when the kernels run (the
 // meaning of `sliding_window` and `whole_context` as in the one-launch form).
 void launch_gqa_decode_split_device_position(

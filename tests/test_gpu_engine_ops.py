@@ -665,6 +665,86 @@ def test_fused_decode_attention_equals_the_separate_calls(cuda, oracle, apply_ro
     assert lib.nfn_native_tile_glimmer_fused_decode_attention_float32_v1(ctypes.byref(empty)) == 1
 
 
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("query_heads,kv_heads,position,first,capacity", [
+    (32, 2, 0, 0, 64),           # the current key alone
+    (16, 4, 1, 0, 64),           # one cached key, the fewest heads a group has
+    (32, 2, 15, 0, 64), (32, 2, 16, 0, 64), (32, 2, 17, 0, 64),      # around the keys of a wave
+    (32, 2, 127, 0, 256), (32, 2, 128, 0, 256), (32, 2, 129, 0, 256),  # ... of a step
+    (48, 8, 255, 0, 256), (48, 8, 256, 0, 512), (48, 8, 257, 0, 512),  # ... of a workgroup without shares
+    (40, 2, 100, 0, 128),        # two groups of query heads read a key: the norms keep a launch of their own
+    (48, 2, 900, 133, 777),      # ... in six shares, the ring wraps
+    (24, 1, 20000, 0, 32768),    # ... as many shares as there may be with the copy
+    (32, 2, 163, 100, 64),       # as many cached keys as the smallest ring allows
+    (32, 2, 9000, 0, 16384),     # shares of more than one step, ragged at the end
+])
+def test_fused_decode_attention_split_form_at_its_edges(cuda, oracle, query_heads, kv_heads, position, first, capacity,
+                                                        interleaved):
+    """Norms, rotation, attention and commit in the launches of the split form: the bits of the separate calls
+    (attention in its split form too), and of the call with the position on the device where that is a window.
+    Ring rows outside the keys hold NaN, the workspace and the output hold NaN patterns, none of which may be seen."""
+    rng = np.random.default_rng(position + query_heads)
+    head_dim, scale = 128, 128 ** -0.5
+    query = rng.standard_normal((query_heads, head_dim)).astype(np.float32)
+    key = rng.standard_normal((kv_heads, head_dim)).astype(np.float32)
+    value = rng.standard_normal((kv_heads, head_dim)).astype(np.float32)
+    keys = oracle.to_bf16(rng.standard_normal((capacity, kv_heads * head_dim)).astype(np.float32))
+    values = oracle.to_bf16(rng.standard_normal((capacity, kv_heads * head_dim)).astype(np.float32))
+    dead = np.setdiff1d(np.arange(capacity), np.arange(first, position) % capacity)
+    keys[dead], values[dead] = 0x7FC0, 0x7FC0
+    weights = [_norm_row((1.0 + 0.1 * rng.standard_normal(head_dim)).astype(np.float32)) for _ in range(2)]
+    layout = engine_ops.ROPE_INTERLEAVED if interleaved else engine_ops.ROPE_HALF_SPLIT
+    workspace = engine_ops.gqa_decode_workspace(query_heads, head_dim)
+
+    def state():
+        workspace.fill_(0xFF)
+        return [to_device(query, cuda), to_device(key, cuda), to_device(value, cuda), bf16_tensor(keys, cuda),
+                bf16_tensor(values, cuda)]
+
+    separate = state()
+    q, k, v, kc, vc = separate
+    engine_ops.qk_norm_scale_rope(q, k, *weights, 1e-5, 0.5, position, 500000.0, layout, True)
+    expected = oracle.gqa_decode(q.cpu().numpy(), k.cpu().numpy(), value, keys, values, position, first, scale)
+    out = engine_ops.gqa_decode(q, k, v, kc, vc, position, first, scale, workspace=workspace)
+    # 2e-7 relative at most for products of exact terms and float sums; outputs are weighted means of N(0, 1)
+    assert np.abs(out.cpu().numpy() - expected).max() <= 4e-6
+    engine_ops.cache_commit(k, v, kc, vc, position)
+    forms = [dict()]
+    if position - first + 1 <= capacity:
+        forms.append(dict(device_position=to_device(np.array([position], dtype=np.int64), cuda),
+                          sliding_window=position - first + 1))
+    for form in forms:
+        fused = state()
+        result = torch_().full_like(out, float("nan"))
+        engine_ops.fused_decode_attention(*fused, position, first, scale, *weights, 1e-5, 0.5, 500000.0, layout, True,
+                                          out=result, workspace=workspace, **form)
+        for name, one, other in zip(("query", "key", "value"), fused, separate):
+            assert_bits_equal(one, other, name)
+        assert np.array_equal(bits_of(fused[3]), bits_of(kc)) and np.array_equal(bits_of(fused[4]), bits_of(vc))
+        if form:  # shares may be cut at other keys
+            assert np.abs(result.cpu().numpy() - expected).max() <= 4e-6
+        else:
+            assert_bits_equal(result, out, "attention output")
+
+
+def test_fused_decode_attention_split_form_over_its_own_inputs(cuda):
+    """An output that lies over the query takes the launches that never read a row after another wrote it."""
+    torch = torch_()
+    generator = torch.Generator(device=cuda).manual_seed(5)
+    def draw(*shape):
+        return torch.randn(shape, generator=generator, device=cuda)
+    query, key, value, rings = draw(32, 128), draw(2, 128), draw(2, 128), draw(2, 1024, 256).to(torch.bfloat16).view(torch.int16)
+    workspace = engine_ops.gqa_decode_workspace(32, 128)
+    results = []
+    for over in (False, True):
+        q, k, caches = query.clone(), key.clone(), rings.clone()
+        out = q if over else torch.empty_like(q)
+        engine_ops.fused_decode_attention(q, k, value, caches[0], caches[1], 1000, 0, 128 ** -0.5, out=out, workspace=workspace)
+        results.append((out, k, caches))
+    for one, other in zip(*results):
+        assert torch.equal(one, other)
+
+
 @pytest.mark.parametrize("apply_rope,position", [(True, 4100), (True, 70), (False, 1500), (False, 0)])
 def test_fused_decode_attention_with_the_position_on_the_device(cuda, oracle, apply_rope, position):
     """The graph form reads the position when the kernels run: same bits as the host form at
