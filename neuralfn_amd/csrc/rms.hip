@@ -153,13 +153,16 @@ constexpr int kLoaded = kOwned / kLoaders;  // columns per thread
 // the small-batch workspace of gridDim.x rows; 3: the activation records of gridDim.x rows
 // (token by token) and, at `operand_image`, the same codes in matrix-operand order: what
 // the exact verifier's quantizer launch leaves for its matrix-core kernel (gemv_rows.hpp).
+// The leading arguments (13 dwords) are what the requests need and arrive in registers: by way of the argument block the
+// kernel's first request waited for one from memory (half a microsecond of 5.5).  `kinds`: norm_kind of the two weights.
 template <int HANDOFF>
 __global__ __launch_bounds__(kWideThreads) void dual_rms_resident_kernel(
-    const float* __restrict__ input, NormWeight first_weight,
-    const float* __restrict__ residual_input, float* __restrict__ hidden_output,
-    NormWeight second_weight, float* __restrict__ normalized_output,
-    float* __restrict__ residual_output, int width, float first_eps, float second_eps,
+    const float* __restrict__ input, const float* __restrict__ residual_input, const std::uint8_t* first_data,
+    const std::uint8_t* second_data, std::uint32_t kinds, int width, float first_eps, float second_eps,
+    float* __restrict__ hidden_output, float* __restrict__ normalized_output, float* __restrict__ residual_output,
     std::uint8_t* __restrict__ records, std::uint8_t* __restrict__ operand_image) {
+    const NormWeight first_weight = norm_weight_of(first_data, kinds & 0xffffu);
+    const NormWeight second_weight = norm_weight_of(second_data, kinds >> 16);
     __shared__ float partials[kRmsThreads + 1];
     __shared__ __attribute__((aligned(16))) float handed[kOwned * kRmsThreads];  // [k][t]: column t + 256 k
     extern __shared__ __attribute__((aligned(16))) float staged[];  // HANDOFF 1, 3: the normalized row
@@ -401,11 +404,14 @@ struct CacheRow {
 // three calls bit for bit.  For the fused decode step the key heads' workgroups
 // also write the bf16 cache row of the new key and value (the row a one-token
 // attention at this position never reads).
+// (the leading 13 dwords arrive in registers, as in dual_rms_resident_kernel)
 __global__ __launch_bounds__(kRmsThreads) void qk_norm_scale_rope_kernel(
-    float* __restrict__ query, float* __restrict__ key, NormWeight query_weight,
-    NormWeight key_weight, int query_heads, int kv_heads, int head_dim, float eps,
-    float query_scale, std::int64_t position, const std::int64_t* __restrict__ device_position,
-    double theta, bool interleaved, bool apply_rope, CacheRow commit) {
+    float* __restrict__ query, float* __restrict__ key, const std::uint8_t* query_data, const std::uint8_t* key_data,
+    std::uint32_t kinds, int query_heads, int kv_heads, int head_dim, float eps, float query_scale,
+    std::int64_t position, const std::int64_t* __restrict__ device_position, double theta, bool interleaved,
+    bool apply_rope, CacheRow commit) {
+    const NormWeight query_weight = norm_weight_of(query_data, kinds & 0xffffu);
+    const NormWeight key_weight = norm_weight_of(key_data, kinds >> 16);
     __shared__ float partials[kRmsThreads];
     __shared__ float normalized[kRmsThreads];
     if (device_position != nullptr) position = device_position[0];
@@ -483,27 +489,21 @@ void launch_dual_rms_add_capture(const float* input, const Descriptor* first_wei
     const dim3 grid(static_cast<unsigned>(rows));
     if (width <= kOwned * kRmsThreads) {
         const int columns = static_cast<int>(width);
-        std::uint8_t* const none = nullptr;
+        const std::uint32_t kinds = norm_kind(first) | (norm_kind(second) << 16);
+        const auto launch = [&](auto kernel, std::size_t lds, std::uint8_t* left, std::uint8_t* image) {
+            hipLaunchKernelGGL(kernel, grid, dim3(kWideThreads), lds, stream, input, residual_input, first.data,
+                               second.data, kinds, columns, first_eps, second_eps, hidden_output, normalized_output,
+                               residual_output, left, image);
+        };
+        const std::size_t row = static_cast<std::size_t>(columns) * sizeof(float);
         if (half_image != nullptr) {
-            hipLaunchKernelGGL((dual_rms_resident_kernel<2>), grid, dim3(kWideThreads), 0, stream, input,
-                               first, residual_input, hidden_output, second, normalized_output,
-                               residual_output, columns, first_eps, second_eps, half_image, none);
+            launch(dual_rms_resident_kernel<2>, 0, half_image, nullptr);
         } else if (records != nullptr && operand_image != nullptr) {
-            hipLaunchKernelGGL((dual_rms_resident_kernel<3>), grid, dim3(kWideThreads),
-                               static_cast<std::size_t>(columns) * sizeof(float), stream, input,
-                               first, residual_input, hidden_output, second, normalized_output,
-                               residual_output, columns, first_eps, second_eps, records,
-                               operand_image);
+            launch(dual_rms_resident_kernel<3>, row, records, operand_image);
         } else if (records != nullptr) {
-            hipLaunchKernelGGL((dual_rms_resident_kernel<1>), grid, dim3(kWideThreads),
-                               static_cast<std::size_t>(columns) * sizeof(float), stream, input,
-                               first, residual_input, hidden_output, second, normalized_output,
-                               residual_output, columns, first_eps, second_eps, records, none);
+            launch(dual_rms_resident_kernel<1>, row, records, nullptr);
         } else {
-            hipLaunchKernelGGL((dual_rms_resident_kernel<0>), grid, dim3(kWideThreads), 0, stream,
-                               input, first, residual_input, hidden_output, second,
-                               normalized_output, residual_output, columns, first_eps, second_eps,
-                               records, none);
+            launch(dual_rms_resident_kernel<0>, 0, nullptr, nullptr);
         }
         return;
     }
@@ -568,12 +568,13 @@ void launch_qk_norm_scale_rope(float* query, float* key, const Descriptor* query
                                std::uint16_t* value_cache, const float* current_value,
                                std::int64_t cache_capacity, std::int64_t cache_row_stride,
                                hipStream_t stream) {
+    const NormWeight first = norm_weight(query_weight, query_centered);
+    const NormWeight second = norm_weight(key_weight, key_centered);
     const CacheRow commit{key_cache, value_cache, current_value, cache_capacity, cache_row_stride};
     hipLaunchKernelGGL(qk_norm_scale_rope_kernel,
                        dim3(static_cast<unsigned>(rows * (query_heads + kv_heads))),
-                       dim3(kRmsThreads), 0, stream, query, key,
-                       norm_weight(query_weight, query_centered),
-                       norm_weight(key_weight, key_centered), static_cast<int>(query_heads),
+                       dim3(kRmsThreads), 0, stream, query, key, first.data, second.data,
+                       norm_kind(first) | (norm_kind(second) << 16), static_cast<int>(query_heads),
                        static_cast<int>(kv_heads), static_cast<int>(head_dim), eps, query_scale,
                        position, device_position, static_cast<double>(theta), interleaved,
                        apply_rope, commit);

@@ -20,6 +20,14 @@ struct NormWeight {
     int centered;  // the stored weight is (scale - 1)
 };
 
+// All of it but the pointer in sixteen bits, for kernels that take the pointer among their leading arguments.
+inline std::uint32_t norm_kind(const NormWeight& weight) {
+    return weight.encoding | (weight.present != 0 ? 0x4000u : 0u) | (weight.centered != 0 ? 0x8000u : 0u);
+}
+__device__ __forceinline__ NormWeight norm_weight_of(const std::uint8_t* data, std::uint32_t kind) {
+    return NormWeight{data, kind & 0x3fffu, (kind & 0x4000u) != 0 ? 1 : 0, (kind & 0x8000u) != 0 ? 1 : 0};
+}
+
 __device__ __forceinline__ float norm_scale(const NormWeight& weight, std::int64_t column) {
     if (!weight.present) return 1.0f;
     float scale = weight_value(weight.encoding, weight.data, column);
