@@ -1384,6 +1384,7 @@ RowAttention row_call(const NfnNativeTileGlimmerGqaDecodeDescriptorV1& d, const 
     call.key_cache = d.key_cache_bf16;
     call.value_cache = d.value_cache_bf16;
     call.output = d.output;
+    call.query_rows = 1;
     call.query_heads = d.query_heads;
     call.kv_heads = d.kv_heads;
     call.head_dim = d.head_dim;
@@ -1486,8 +1487,8 @@ void launch_block_attention(const NfnNativeTileDFlashBlockAttentionDescriptorV1&
         if (window < longest) longest = window;
     }
     const std::int64_t tiles = tiles_of(longest);
-    // one row that sees no other row of a block
-    if (partials != nullptr && d.query_rows == 1 && (a.causal != 0 || d.block_rows == 1)) {
+    // a causal block, or one row that sees no other row
+    if (partials != nullptr && (a.causal != 0 || (d.query_rows == 1 && d.block_rows == 1))) {
         RowAttention call{};
         call.query = d.query;
         call.current_key = d.block_key;
@@ -1495,10 +1496,12 @@ void launch_block_attention(const NfnNativeTileDFlashBlockAttentionDescriptorV1&
         call.key_cache = d.key_cache_bf16;
         call.value_cache = d.value_cache_bf16;
         call.output = d.output;
+        call.query_rows = d.query_rows;
         call.query_heads = d.query_heads;
         call.kv_heads = d.kv_heads;
         call.head_dim = d.head_dim;
         call.position = d.context_length;
+        call.sliding_window = d.sliding_window;
         const std::int64_t first = d.context_length - d.sliding_window + (a.causal != 0 ? 1 : 0);
         call.first_key_position = first > 0 ? first : 0;
         call.cache_capacity = d.cache_capacity;

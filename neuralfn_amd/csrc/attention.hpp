@@ -36,6 +36,8 @@ struct RowPreparation {
 
 // One query row over a cache.  The keys are first_key_position .. position - 1 of the ring and the current one;
 // with `device_position` the last `sliding_window` ones up to *device_position, or all when `whole_context`.
+// With query_rows > 1 the rows of a causal block: row r at position + r, with the last `sliding_window` keys up to its
+// own of the ring and of the block's rows (current_key, current_value).
 struct RowAttention {
     const float* query;
     const float* current_key;
@@ -43,7 +45,7 @@ struct RowAttention {
     const std::uint16_t* key_cache;
     const std::uint16_t* value_cache;
     float* output;
-    std::int64_t query_heads, kv_heads, head_dim;
+    std::int64_t query_rows, query_heads, kv_heads, head_dim;
     std::int64_t position, first_key_position;
     std::int64_t cache_capacity, cache_row_stride;
     float scale;

@@ -1,9 +1,10 @@
-// One query row on the matrix cores (head_dim 128, four and more query heads per key/value head): the
-// one-token attention of the decode loop, alone or with the per-head norms, the rotation and the cache
-// commit before it (semantics: neuralfn/csrc/native_train/tile_ops.h:308-339, 905-943).
+// One query row, or each row of a causal block, on the matrix cores (head_dim 128, four and more query
+// heads per key/value head): the one-token attention of the decode loop, alone or with the per-head norms,
+// the rotation and the cache commit before it, and the verifier's block attention where a row's share of
+// the keys is short (semantics: neuralfn/csrc/native_train/tile_ops.h:308-339, 445-486, 905-943).
 //
-// One workgroup of eight waves per (key/value head, group of up to 16 of its query heads, share of the
-// keys).  All query heads of a group read a key/value row once.
+// One workgroup of eight waves per (query row, key/value head, group of up to 16 of its query heads, share
+// of the keys).  All query heads of a group read a key/value row once.
 //
 // What bounds it is the number of instructions a wave issues one after the other (2 to 3 ns each for a
 // wave that is alone on its SIMD) behind one round of requests, not memory: a 2,048-key window of two
@@ -41,6 +42,8 @@
 #include "kernels.hpp"
 #include "wave_rows.hpp"
 
+#include <algorithm>
+
 namespace nfn {
 
 namespace {
@@ -58,6 +61,7 @@ static_assert(kGroupHeadDim == 16 * kRowWaves && kGroupHeadDim == 2 * kWave, "di
 struct RowTail {
     const float* block_key;
     const float* block_value;
+    std::int64_t block_stride;  // floats from a row of the block to the next
     float* output;
     float* partials;
     const std::int64_t* device_position;
@@ -67,6 +71,14 @@ struct RowTail {
     float* key_copy;  // where the prepared key goes (in place where no other workgroup reads it)
     RowPreparation preparation;
 };
+
+// eight floats as the bf16 row the cache would hold of them
+__device__ __forceinline__ uint4 pack_as_cached(float4 low, float4 high) {
+    const auto pair = [](float first, float second) {
+        return static_cast<std::uint32_t>(to_bf16(first)) | (static_cast<std::uint32_t>(to_bf16(second)) << 16);
+    };
+    return make_uint4(pair(low.x, low.y), pair(low.z, low.w), pair(high.x, high.y), pair(high.z, high.w));
+}
 
 // the four lanes (., i) of a wave meet
 __device__ __forceinline__ float across_j_max(float value) {
@@ -136,13 +148,18 @@ __device__ __forceinline__ HeadPair prepare_head(HeadPair raw, const float (&sca
     return HeadPair{a, b};
 }
 
-// The leading arguments (13 dwords) arrive in registers.  `heads_splits`: query heads per key/value head, and from
+// kBlock: several query rows, row r at context + r behind the cache's keys and the block's rows before it, which enter as
+// the cache will hold them; `keys` is then the context and `first_slot` the most keys that a row sees before its own.
+enum class RowMode { kPlain, kPrepare, kBlock };
+
+// The leading arguments (14 dwords) arrive in registers.  `heads_splits`: query heads per key/value head, and from
 // bit 16 on the shares; share_keys = 0: the position is in device memory.  first_slot: ring row of the first of `keys` cached keys.
-template <bool PREPARE>
+template <RowMode MODE>
 __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
     const float* query, const std::uint16_t* key_cache, const std::uint16_t* value_cache, std::uint32_t row_stride,
     std::uint32_t capacity, std::uint32_t first_slot, std::uint32_t keys, std::uint32_t share_keys,
-    std::uint32_t heads_splits, float scale, RowTail tail) {
+    std::uint32_t heads_splits, std::uint32_t kv_heads, float scale, RowTail tail) {
+    constexpr bool PREPARE = MODE == RowMode::kPrepare, BLOCK = MODE == RowMode::kBlock;
     __shared__ __attribute__((aligned(16))) std::uint8_t staged_values[kStepKeys * kStageRowBytes];
     // the weights' terms: [term][wave][head] x sixteen keys
     __shared__ __attribute__((aligned(16))) std::uint8_t staged_weights[3][kRowWaves][kGroupHeads][2 * kWaveKeys];
@@ -160,11 +177,13 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
     const int i = lane & 15;
     const std::uint32_t heads = heads_splits & 0xffffu, splits = heads_splits >> 16;
     const std::uint32_t groups_per_kv = (heads + kGroupHeads - 1) / kGroupHeads;
-    const std::uint32_t kv_head = groups_per_kv == 1 ? blockIdx.x : blockIdx.x / groups_per_kv;
-    const std::uint32_t head_group = blockIdx.x - kv_head * groups_per_kv;
+    const std::uint32_t query_row = BLOCK ? blockIdx.x / (kv_heads * groups_per_kv) : 0;
+    const std::uint32_t group = blockIdx.x - query_row * kv_heads * groups_per_kv;
+    const std::uint32_t kv_head = groups_per_kv == 1 ? group : group / groups_per_kv;
+    const std::uint32_t head_group = group - kv_head * groups_per_kv;
     const int heads_here = static_cast<int>(
         heads - head_group * kGroupHeads < kGroupHeads ? heads - head_group * kGroupHeads : kGroupHeads);
-    const std::int64_t first_head = kv_head * heads + head_group * kGroupHeads;
+    const std::int64_t first_head = query_row * kv_heads * heads + kv_head * heads + head_group * kGroupHeads;
     const std::int64_t head_offset = static_cast<std::int64_t>(kv_head) * kGroupHeadDim;
     // the current key goes with the last share
     const bool has_row = blockIdx.y + 1 == splits;
@@ -193,9 +212,18 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
     } else if constexpr (PREPARE) {
         position = tail.position;
     }
+    [[maybe_unused]] int cached = 0;  // kBlock: keys of the share (later) that lie in the cache
+    if constexpr (BLOCK) {
+        const std::uint32_t end = keys + query_row;
+        const std::uint32_t before = end < first_slot ? end : first_slot;
+        cached = static_cast<int>(before) - static_cast<int>(query_row);  // (a window inside the block: negative)
+        first_slot = cached > 0 ? (end - before) % capacity : 0;
+        keys = before;
+    }
     // the share's keys: `here` of them, the first at ring row `slot`
     const std::uint32_t share_begin = blockIdx.y * share_keys < keys ? blockIdx.y * share_keys : keys;
     const int here = static_cast<int>(keys - share_begin < share_keys ? keys - share_begin : share_keys);
+    if constexpr (BLOCK) cached -= static_cast<int>(share_begin);
     const auto ring_row = [capacity](std::uint32_t slot) {  // slot < 2 * capacity
         return slot >= capacity ? slot - capacity : slot;
     };
@@ -218,6 +246,27 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
     const auto request_keys = [&](int begin, std::uint32_t at) {
         const int count = keys_left(begin);
         if (count == 0) return;
+        if constexpr (BLOCK) {
+            if (begin + count > cached) {
+                // every lane requests both kinds of row, so that nothing waits in between
+                const int key = i < count ? i : count - 1, in_block = begin + key - cached;
+                const bool from_block = in_block >= 0;
+                const std::uint32_t row = from_block ? 0 : ring_row(at + key);
+                const std::uint16_t* source = key_cache + static_cast<std::uint64_t>(row) * row_stride + head_offset + 8 * j;
+                const float* floats = tail.block_key + (from_block ? in_block : 0) * tail.block_stride + head_offset + 8 * j;
+                uint4 raw[4];
+                float4 low[4], high[4];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    raw[s] = *reinterpret_cast<const uint4*>(source + 32 * s);
+                    low[s] = *reinterpret_cast<const float4*>(floats + 32 * s);
+                    high[s] = *reinterpret_cast<const float4*>(floats + 32 * s + 4);
+                }
+#pragma unroll
+                for (int s = 0; s < 4; ++s) key_raw[s] = from_block ? pack_as_cached(low[s], high[s]) : raw[s];
+                return;
+            }
+        }
         const std::uint32_t row = ring_row(at + (i < count ? i : count - 1));
         const std::uint16_t* source = key_cache + static_cast<std::uint64_t>(row) * row_stride + head_offset + 8 * j;
 #pragma unroll
@@ -226,6 +275,28 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
     const auto request_values = [&](int begin, std::uint32_t at) {
         const int count = keys_left(begin);
         if (count == 0) return;
+        if constexpr (BLOCK) {
+            if (begin + count > cached) {
+                uint4 raw[4];
+                float4 low[4], high[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int key = 4 * r + j < count ? 4 * r + j : count - 1, in_block = begin + key - cached;
+                    const std::uint32_t row = in_block >= 0 ? 0 : ring_row(at + key);
+                    const float* floats = tail.block_value + (in_block >= 0 ? in_block : 0) * tail.block_stride + head_offset + 8 * i;
+                    raw[r] = *reinterpret_cast<const uint4*>(
+                        value_cache + static_cast<std::uint64_t>(row) * row_stride + head_offset + 8 * i);
+                    low[r] = *reinterpret_cast<const float4*>(floats);
+                    high[r] = *reinterpret_cast<const float4*>(floats + 4);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int key = 4 * r + j < count ? 4 * r + j : count - 1;
+                    value_raw[r] = begin + key >= cached ? pack_as_cached(low[r], high[r]) : raw[r];
+                }
+                return;
+            }
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const std::uint32_t row = ring_row(at + (4 * r + j < count ? 4 * r + j : count - 1));
@@ -240,8 +311,9 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
     HeadPair row_key{0.0f, 0.0f}, row_value{0.0f, 0.0f};
     float4 row_sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (has_row) {
-        const float* key = tail.block_key + head_offset;
-        const float* value = tail.block_value + head_offset;
+        const std::int64_t own = BLOCK ? query_row * tail.block_stride + head_offset : head_offset;
+        const float* key = tail.block_key + own;
+        const float* value = tail.block_value + own;
         row_key = HeadPair{key[lane], key[lane + kWave]};
         row_sum = *reinterpret_cast<const float4*>(value + 16 * wave + 4 * j);
         if constexpr (PREPARE) row_value = HeadPair{value[lane], value[lane + kWave]};
@@ -448,6 +520,13 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
 // 100 -> 200 keys 5.1 -> 6.6), shares with their merge from 300 keys on 7.7.
 constexpr std::int64_t kAloneKeys = 256;
 
+// The longest share of a block's row, in keys.  Many steps are 2 us each for a workgroup that has a unit alone, since its waves
+// meet twice a step; the waves of attention_grouped_kernel walk alone.  With merge, us, that kernel / this one: 128 keys a
+// share (7 rows of 32 heads over 2, 2,048 keys) 13.4 / 11.5; 512 (10 of 32 over 8, 1,500) 16.6 / 16.3; 1,024 (12 of 16 over
+// 4, 4,000) 20.2 / 18.6; 1,280 (16 of 32 over 4, 4,802) 24.0 / 23.9; 2,176 (16 of 48 over 2, 8,192) 35.4 / 37.2; 4,224 (16
+// of 32 over 8, 8,192) 61.6 / 72.2.  (Two workgroups a unit: 128 registers, of which 31 go to scratch memory, 64.7 and 117.)
+constexpr std::int64_t kBlockKeys = 1024;
+
 bool overlap(const void* a, std::int64_t a_bytes, const void* b, std::int64_t b_bytes) {
     const auto first = reinterpret_cast<std::uintptr_t>(a), second = reinterpret_cast<std::uintptr_t>(b);
     return first < second + static_cast<std::uintptr_t>(b_bytes) && second < first + static_cast<std::uintptr_t>(a_bytes);
@@ -459,19 +538,23 @@ bool launch_attention_row(const RowAttention& call, float* partials, std::int64_
     const auto aligned = [](const void* pointer) { return reinterpret_cast<std::uintptr_t>(pointer) % 16 == 0; };
     const bool on_device = call.device_position != nullptr;
     // a position in device memory can be anything up to the ring's end, and a window is no longer than the ring
-    const std::int64_t keys = !on_device ? call.position - call.first_key_position
-        : call.whole_context             ? call.cache_capacity
-                                         : call.sliding_window - 1;
+    // (several rows: the most that one sees before its own)
+    const bool block = call.query_rows > 1;
+    const std::int64_t keys = block ? std::min(call.position + call.query_rows, call.sliding_window) - 1
+        : !on_device                ? call.position - call.first_key_position
+        : call.whole_context        ? call.cache_capacity
+                                    : call.sliding_window - 1;
     const std::int64_t heads_per_kv = call.query_heads / call.kv_heads;
     if (call.head_dim != kGroupHeadDim || heads_per_kv < kGroupMinHeads || call.query_heads > 65535 ||
         call.cache_row_stride % 8 != 0 || call.cache_row_stride >= (1 << 24) || call.cache_capacity < kWave ||
         call.cache_capacity > kMostKeys || keys > kMostKeys || !aligned(call.key_cache) || !aligned(call.value_cache) ||
-        !aligned(call.current_value) || !aligned(call.output)) {
+        !aligned(call.current_value) || !aligned(call.output) ||
+        (block && (call.position > kMostKeys || !aligned(call.current_key)))) {
         return false;
     }
     const std::int64_t groups_per_kv = (heads_per_kv + kGroupHeads - 1) / kGroupHeads;
-    const std::int64_t groups = call.kv_heads * groups_per_kv;
-    const std::int64_t share_bytes = call.query_heads * partial_floats(kGroupHeadDim) * 4;
+    const std::int64_t groups = call.query_rows * call.kv_heads * groups_per_kv;
+    const std::int64_t share_bytes = call.query_rows * call.query_heads * partial_floats(kGroupHeadDim) * 4;
     std::int64_t most = compute_units() / groups;
     if (most > kMaxSplits) most = kMaxSplits;
     if (partials == nullptr) most = 1;
@@ -479,6 +562,7 @@ bool launch_attention_row(const RowAttention& call, float* partials, std::int64_
     RowTail tail{};
     tail.block_key = call.current_key;
     tail.block_value = call.current_value;
+    tail.block_stride = call.kv_heads * kGroupHeadDim;
     tail.output = call.output;
     tail.device_position = call.device_position;
     tail.position = call.position;
@@ -517,18 +601,23 @@ bool launch_attention_row(const RowAttention& call, float* partials, std::int64_
     } else {
         share = kAloneKeys;
     }
+    if (block && share > kBlockKeys) return false;
     if (splits > 1) tail.partials = partials;
-    const std::uint32_t first_slot =
-        on_device ? 0 : static_cast<std::uint32_t>(call.first_key_position % call.cache_capacity);
-    const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(splits)), block(kRowWaves * kWave);
-    const auto kernel = call.preparation != nullptr ? attention_row_kernel<true> : attention_row_kernel<false>;
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream, call.query, call.key_cache, call.value_cache,
+    const std::uint32_t first_slot = static_cast<std::uint32_t>(
+        block ? keys : on_device ? 0 : call.first_key_position % call.cache_capacity);
+    const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(splits)), threads(kRowWaves * kWave);
+    const auto kernel = block               ? attention_row_kernel<RowMode::kBlock>
+        : call.preparation != nullptr ? attention_row_kernel<RowMode::kPrepare>
+                                      : attention_row_kernel<RowMode::kPlain>;
+    hipLaunchKernelGGL(kernel, grid, threads, 0, stream, call.query, call.key_cache, call.value_cache,
                        static_cast<std::uint32_t>(call.cache_row_stride),
-                       static_cast<std::uint32_t>(call.cache_capacity), first_slot, static_cast<std::uint32_t>(keys),
+                       static_cast<std::uint32_t>(call.cache_capacity), first_slot,
+                       static_cast<std::uint32_t>(block ? call.position : keys),
                        on_device ? 0u : static_cast<std::uint32_t>(share),
-                       static_cast<std::uint32_t>(heads_per_kv | splits << 16), call.scale, tail);
+                       static_cast<std::uint32_t>(heads_per_kv | splits << 16),
+                       static_cast<std::uint32_t>(call.kv_heads), call.scale, tail);
     if (splits > 1) {
-        launch_attention_merge(partials, call.output, static_cast<int>(splits), call.query_heads, kGroupHeadDim,
+        launch_attention_merge(partials, call.output, static_cast<int>(splits), call.query_rows * call.query_heads, kGroupHeadDim,
                                call.preparation != nullptr ? call.preparation->query : nullptr, key_copy,
                                call.preparation != nullptr ? call.preparation->key : nullptr,
                                call.kv_heads * kGroupHeadDim, stream);

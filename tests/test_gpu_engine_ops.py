@@ -456,6 +456,35 @@ def test_block_attention_tiles_with_rows_of_the_block(cuda, oracle, rows, contex
         test_block_attention_split_form(cuda, oracle, True, rows, rows, query_heads, kv_heads, context, window, capacity, 128)
 
 
+@pytest.mark.parametrize("rows,context,window,query_heads,kv_heads", [
+    (5, 0, 64, 32, 2), (9, 3, 4, 40, 2), (16, 40, 7, 16, 4),      # no cache; windows inside the block
+    (7, 121, 1000, 32, 2), (7, 122, 1000, 32, 2), (4, 255, 1000, 48, 8), (4, 253, 200, 48, 8),  # steps, one launch or shares
+    (16, 1017, 1033, 96, 8), (16, 1010, 1010, 96, 8),             # one unit a row's heads: shares as long as they get
+    (16, 2040, 2056, 96, 8), (16, 2050, 2066, 96, 8),             # ... and past that
+])
+def test_block_attention_rows_see_nothing_but_their_keys(cuda, oracle, rows, context, window, query_heads, kv_heads):
+    """The last row of the block is NaN, as are the ring's rows outside the first row's keys: only the last row may
+    show it, and a row past the others' windows nobody."""
+    rng = np.random.default_rng(rows + context)
+    capacity = max(window, 64) + 3
+    query = rng.standard_normal((rows, query_heads, 128)).astype(np.float32)
+    key, value = (rng.standard_normal((rows, kv_heads, 128)).astype(np.float32) for _ in range(2))
+    key[rows - 1], value[rows - 1] = np.nan, np.nan
+    rings = [oracle.to_bf16(rng.standard_normal((capacity, kv_heads * 128)).astype(np.float32)) for _ in range(2)]
+    dead = np.setdiff1d(np.arange(capacity), np.arange(max(0, context - window + 1), context) % capacity)
+    for ring in rings:
+        ring[dead] = 0x7FC0
+    workspace = engine_ops.gqa_decode_workspace(query_heads, 128)
+    workspace.fill_(0xFF)
+    out = engine_ops.block_attention(to_device(query, cuda), to_device(key, cuda), to_device(value, cuda),
+                                     *(bf16_tensor(ring, cuda) for ring in rings), context, window, 128 ** -0.5, True,
+                                     workspace=workspace).cpu().numpy().reshape(query.shape)
+    expected = oracle.block_attention(query, key, value, *rings, context, window, 128 ** -0.5, True).reshape(query.shape)
+    assert np.isnan(out[rows - 1]).all() and np.isnan(expected[rows - 1]).all()
+    # float sums of exact products, outputs weighted means of N(0, 1), as for one row
+    assert np.abs(out[:-1] - expected[:-1]).max() <= 4e-6
+
+
 @pytest.mark.parametrize("keys", [1, 63, 64, 128, 191, 192, 255, 256, 257, 2049, 3000, 3072, 3073])
 def test_one_row_attention_in_one_launch_and_in_shares(cuda, oracle, keys):
     """Both sides of the key counts that the number of workgroups a row is shared out over turns at."""
