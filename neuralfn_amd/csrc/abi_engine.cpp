@@ -206,7 +206,7 @@ int run_fused_decode(const NfnNativeTileGlimmerFusedDecodeAttentionDescriptorV1*
         preparation.key_weight = norm_weight(key_source != nullptr ? &key_weight : nullptr, d->key_norm_centered != 0);
         preparation.eps = d->norm_eps;
         preparation.query_scale = d->query_scale;
-        preparation.theta = static_cast<double>(d->rope_theta);
+        preparation.theta = rope_base(d->rope_theta);
         preparation.interleaved = d->rope_layout == NFN_NATIVE_TILE_GLIMMER_ROPE_INTERLEAVED;
         preparation.apply_rope = d->apply_rope != 0;
         if (launch_prepared_gqa_decode_split(attention, preparation, device_position, sliding_window,

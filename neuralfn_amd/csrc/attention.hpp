@@ -30,7 +30,7 @@ struct RowPreparation {
     std::uint16_t* value_cache;
     NormWeight query_weight, key_weight;
     float eps, query_scale;
-    double theta;
+    RopeBase theta;
     bool interleaved, apply_rope;
 };
 

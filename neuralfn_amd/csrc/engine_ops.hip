@@ -50,7 +50,7 @@ __global__ __launch_bounds__(kThreads) void embedding_kernel(
 __global__ __launch_bounds__(kThreads) void rope_kernel(
     float* __restrict__ query, float* __restrict__ key, std::int64_t rows,
     std::int64_t query_heads, std::int64_t kv_heads, std::int64_t head_dim,
-    std::int64_t start_position, double theta, bool interleaved, bool inverse) {
+    std::int64_t start_position, RopeBase theta, bool interleaved, bool inverse) {
     const std::int64_t half = head_dim / 2;
     const std::int64_t pairs_per_row = (query_heads + kv_heads) * half;
     const std::int64_t index = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -180,7 +180,7 @@ void launch_rope(float* query, float* key, std::int64_t rows, std::int64_t query
     const std::int64_t count = rows * (query_heads + kv_heads) * (head_dim / 2);
     hipLaunchKernelGGL(rope_kernel, dim3(blocks_for(count, std::int64_t(1) << 31)), dim3(kThreads),
                        0, stream, query, key, rows, query_heads, kv_heads, head_dim,
-                       start_position, static_cast<double>(theta), interleaved, inverse);
+                       start_position, rope_base(theta), interleaved, inverse);
 }
 
 void launch_cache_commit(const float* keys, const float* values, std::uint16_t* key_cache,

@@ -408,7 +408,7 @@ struct CacheRow {
 __global__ __launch_bounds__(kRmsThreads) void qk_norm_scale_rope_kernel(
     float* __restrict__ query, float* __restrict__ key, const std::uint8_t* query_data, const std::uint8_t* key_data,
     std::uint32_t kinds, int query_heads, int kv_heads, int head_dim, float eps, float query_scale,
-    std::int64_t position, const std::int64_t* __restrict__ device_position, double theta, bool interleaved,
+    std::int64_t position, const std::int64_t* __restrict__ device_position, RopeBase theta, bool interleaved,
     bool apply_rope, CacheRow commit) {
     const NormWeight query_weight = norm_weight_of(query_data, kinds & 0xffffu);
     const NormWeight key_weight = norm_weight_of(key_data, kinds >> 16);
@@ -576,7 +576,7 @@ void launch_qk_norm_scale_rope(float* query, float* key, const Descriptor* query
                        dim3(kRmsThreads), 0, stream, query, key, first.data, second.data,
                        norm_kind(first) | (norm_kind(second) << 16), static_cast<int>(query_heads),
                        static_cast<int>(kv_heads), static_cast<int>(head_dim), eps, query_scale,
-                       position, device_position, static_cast<double>(theta), interleaved,
+                       position, device_position, rope_base(theta), interleaved,
                        apply_rope, commit);
 }
 
