@@ -72,25 +72,22 @@ __device__ __forceinline__ TokenImage token_image(std::uint8_t* lds, int token, 
     return image;
 }
 
-// Scatter the codes of block `block`, four values per lane, into the image.
-__device__ __forceinline__ void quantize_block(const ActivationCodes& codes, int lane, int block,
-                                               int blocks, const TokenImage& image) {
-    const std::uint32_t hi = codes.hi, lo = codes.lo;
-    const float maximum = codes.maximum;
-    int sum = codes.sum;
-    sum += dpp_move<kQuadXor1>(sum);
-    sum += dpp_move<kQuadXor2>(sum);
-    sum += dpp_move<kHalfMirror>(sum);
-    // lane L holds values 4L..4L+3: sub-block L/8, 16-value half (L%8)/4, byte (L%4)*4
+// Scatter the codes of block `block` into the image; lane c of its LANES holds words LANES k + c: unit 4 block + word /
+// 16, sub-block (word / 8) % 2 of the pair, 16-value half (word / 4) % 2, byte 4 (word % 4).
+template <int LANES>
+__device__ __forceinline__ void quantize_block(const QuadCodes<LANES>& codes, int c, int block, int blocks,
+                                               const TokenImage& image) {
     const int units = 4 * blocks;
-    const int sub = lane >> 3;
-    const int unit = 4 * block + (sub >> 1);
-    const int array_high = 4 * (sub & 1) + ((lane >> 2) & 1);
-    std::uint8_t* slot = image.planes + (array_high * units + unit) * 16 + (lane & 3) * 4;
-    *reinterpret_cast<std::uint32_t*>(slot) = hi;
-    *reinterpret_cast<std::uint32_t*>(slot + 2 * units * 16) = lo;
-    if ((lane & 7) == 0) image.sums[block * 8 + sub] = sum;
-    if (lane == 0) image.scale[block] = maximum * (1.0f / kCodeRange);
+    const int array_high = 4 * ((c >> 3) & 1) + ((c >> 2) & 1);
+    std::uint8_t* slot = image.planes + (array_high * units + 4 * block + (c >> 4)) * 16 + (c & 3) * 4;
+#pragma unroll
+    for (int k = 0; k < 64 / LANES; ++k) {
+        *reinterpret_cast<std::uint32_t*>(slot + LANES * k) = codes.hi[k];
+        *reinterpret_cast<std::uint32_t*>(slot + 2 * units * 16 + LANES * k) = codes.lo[k];
+        const int sum = sum_of_thirty_two(codes.sum[k]);
+        if ((c & 7) == 0) image.sums[block * 8 + ((LANES * k + c) >> 3)] = sum;
+    }
+    if (c == 0) image.scale[block] = codes.maximum * (1.0f / kCodeRange);
 }
 
 template <bool Q5>
@@ -214,7 +211,6 @@ __device__ __forceinline__ void accumulate_unit(const Stage<Q5>& stage, const st
     }
 }
 
-typedef const __attribute__((address_space(1))) std::uint8_t* GlobalBytes;
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(1))) v4u* GlobalVec;
 
@@ -231,40 +227,10 @@ struct DotTail {
 };
 
 
-// Four 48-bit device addresses in three 64-bit words.
-struct PackedPointers {
-    std::uint64_t a, b, c;
-};
-constexpr std::uint64_t kAddressMask = (std::uint64_t(1) << 48) - 1;
-inline PackedPointers pack_pointers(const void* const p[4]) {
-    std::uint64_t v[4];
-    for (int i = 0; i < 4; ++i) v[i] = reinterpret_cast<std::uint64_t>(p[i]) & kAddressMask;
-    PackedPointers packed;
-    packed.a = v[0] | (v[1] << 48);
-    packed.b = (v[1] >> 16) | (v[2] << 32);
-    packed.c = (v[2] >> 32) | (v[3] << 16);
-    return packed;
-}
-__device__ __forceinline__ GlobalBytes unpack_pointer(std::uint64_t a, std::uint64_t b,
-                                                      std::uint64_t c, int index) {
-    const std::uint64_t p0 = a & kAddressMask;
-    const std::uint64_t p1 = (a >> 48) | ((b & 0xffffffffull) << 16);
-    const std::uint64_t p2 = (b >> 32) | ((c & 0xffffull) << 32);
-    const std::uint64_t p3 = c >> 16;
-    std::uint64_t p = p0;
-    p = index == 1 ? p1 : p;
-    p = index == 2 ? p2 : p;
-    p = index == 3 ? p3 : p;
-    return reinterpret_cast<GlobalBytes>(p);
-}
-
 // Walks the (row, 64-unit slice) pairs of one wave; everything is uniform.
-// HALF > 0 (pair mode, one projection slot): "row" r stands for row r of the first
-// projection followed by row r of the second, HALF slices each.
 struct DotCursor {
     int op, row, first_row, next_bound, iteration;
     GlobalBytes row_ptr;
-    std::int64_t second_minus_first;  // pair mode: from a row of the first projection to its partner
 
     __device__ __forceinline__ void bounds(int b1, int b2, int b3) {
         first_row = op == 0 ? 0 : op == 1 ? b1 : op == 2 ? b2 : b3;
@@ -278,27 +244,16 @@ struct DotCursor {
         bounds(b1, b2, b3);
         row_ptr = unpack_pointer(a, b, c, op) + (row - first_row) * stride;
     }
-    template <int HALF>
-    __device__ __forceinline__ void advance(int iterations, std::int64_t stride, std::uint64_t a,
-                                            std::uint64_t b, std::uint64_t c, int b1, int b2, int b3) {
-        ++iteration;
-        if constexpr (HALF > 0) {
-            if (iteration == HALF) row_ptr += second_minus_first;
-            if (iteration < 2 * HALF) return;
-            iteration = 0;
-            ++row;
-            row_ptr += stride - second_minus_first;
-            return;
-        }
-        if (iteration < iterations) return;
-        iteration = 0;
+    // true where the next row is the first one of another projection
+    __device__ __forceinline__ bool next_row(std::int64_t stride, std::uint64_t a, std::uint64_t b, std::uint64_t c,
+                                             int b1, int b2, int b3) {
         ++row;
         row_ptr += stride;
-        if (row == next_bound) {
-            ++op;
-            bounds(b1, b2, b3);
-            row_ptr = unpack_pointer(a, b, c, op);
-        }
+        if (row != next_bound) return false;
+        ++op;
+        bounds(b1, b2, b3);
+        row_ptr = unpack_pointer(a, b, c, op);
+        return true;
     }
 };
 
@@ -322,7 +277,6 @@ __global__ __launch_bounds__(WAVES * kWave) void gemv_dot_kernel(
     int bound2, int bound3, DotTail tail) {
     static_assert(ITER == 0 || (T == 1 && ITER <= 2), "register-resident activations: one token, two slices");
     static_assert(!PAIRS || (ITER > 0 && P == kPlain), "pair mode: register-resident activations, plain input");
-    constexpr int kHalf = PAIRS ? ITER : 0;
     constexpr bool kQ5 = ENC == kEncQ5K;
     constexpr int kBlockBytes = kQ5 ? 176 : 144;
     constexpr int kQuants = kQ5 ? 48 : 16;
@@ -351,9 +305,10 @@ __global__ __launch_bounds__(WAVES * kWave) void gemv_dot_kernel(
     // that their short latency does not queue behind the weight loads.  All
     // loads are unconditional (clamped indices) to keep the load counters exact.
     const int records = pass_tokens * blocks;
-    // (rows of more than 8,192 columns: eight, i.e. every record of a 16,384-column row)
-    constexpr int kEarly = ITER > 0 ? 4 : 8;
-    float4 early[kEarly];
+    constexpr int kLanes = ITER == 1 ? 32 : 16;
+    // (rows of more than 8,192 columns, eight waves: two groups of four a wave, i.e. every record of a 16,384-column row)
+    constexpr int kEarly = ITER > 0 || WAVES > kDotWaves ? 1 : 2;
+    RecordQuads<P, kLanes> early[kEarly];
     constexpr int kNormLoaders = (WAVES * kWave) / kRmsThreads;
     DualRmsOperands<kNormLoaders> norm_operands;
     if constexpr (P == kDualNorm) {
@@ -363,20 +318,18 @@ __global__ __launch_bounds__(WAVES * kWave) void gemv_dot_kernel(
     } else {
 #pragma unroll
         for (int e = 0; e < kEarly; ++e) {
-            const int record = min(wave + e * WAVES, records - 1);
-            const int token = token_of_record<T>(record, blocks);
-            const int block = record - token * blocks;
-            early[e] = load_activations<P>(pass_first, pass_second,
-                                           static_cast<std::int64_t>(token) * input_dim + block * 256 + lane * 4);
+            request_records<T, P, kLanes>(early[e], pass_first, pass_second, wave + e * WAVES, records, blocks, input_dim, lane);
         }
+        __builtin_amdgcn_sched_barrier(0);  // (the compiler would put them behind what follows)
     }
 
     // (2) weight loads of the first two (row, slice) pairs.  A stage beyond the wave's
     // last pair loads one fixed address in every lane (one cache line per instruction),
     // so the number of loads in flight is the same on every path.
-    DotCursor fetch;
-    fetch.second_minus_first = PAIRS ? unpack_pointer(data_a, data_b, data_c, 1) -
+    // pair mode: from a row of the first projection to its partner
+    const std::int64_t second_minus_first = PAIRS ? unpack_pointer(data_a, data_b, data_c, 1) -
             unpack_pointer(data_a, data_b, data_c, 0) : 0;
+    DotCursor fetch;
     fetch.start(row_count > 0 ? row_begin : 0, stride, data_a, data_b, data_c, bound1, bound2, bound3);
     int fetch_left = total;  // pairs not fetched yet
     // A lane's byte offsets inside a row depend on the slice only (and a slice of a
@@ -417,8 +370,16 @@ __global__ __launch_bounds__(WAVES * kWave) void gemv_dot_kernel(
             stage.h0 = make_uint4(h0.x, h0.y, h0.z, h0.w);
             stage.h1 = make_uint4(h1.x, h1.y, h1.z, h1.w);
         }
-        if (--fetch_left > 0) {
-            fetch.template advance<kHalf>(iterations, stride, data_a, data_b, data_c, bound1, bound2, bound3);
+        // (with ITER > 0 the slice is known where this is inlined: most steps move nothing)
+        --fetch_left;
+        if constexpr (PAIRS) {
+            if (slice == ITER - 1 && fetch_left > 0) fetch.row_ptr += second_minus_first;
+            if (slice == 2 * ITER - 1 && fetch_left > 0) fetch.row_ptr += stride - second_minus_first;
+        } else if constexpr (ITER > 0) {
+            if (slice == ITER - 1 && fetch_left > 0) fetch.next_row(stride, data_a, data_b, data_c, bound1, bound2, bound3);
+        } else if (fetch_left > 0 && ++fetch.iteration == iterations) {
+            fetch.iteration = 0;
+            fetch.next_row(stride, data_a, data_b, data_c, bound1, bound2, bound3);
         }
     };
     // STAGES register stages.  Two are requested here; a third only once this wave's
@@ -455,33 +416,39 @@ __global__ __launch_bounds__(WAVES * kWave) void gemv_dot_kernel(
                                       norm_partials);
 #pragma unroll
         for (int e = 0; e < kEarly; ++e) {
-            const int record = min(wave + e * WAVES, records - 1);
-            early[e] = *reinterpret_cast<const float4*>(normalized_row + record * 256 + lane * 4);
+            const int record = min(record_of_lane<kLanes>(wave + e * WAVES, lane), records - 1);
+#pragma unroll
+            for (int k = 0; k < 64 / kLanes; ++k) {
+                early[e].quad[k] = *reinterpret_cast<const float4*>(
+                    normalized_row + record * 256 + 4 * (kLanes * k + lane % kLanes));
+            }
         }
     }
-    auto quantize_record = [&](float4 loaded, int record) {
+    auto quantize_group = [&](const RecordQuads<P, kLanes>& loaded, int group) {
+        const QuadCodes<kLanes> codes = quad_codes<P, kLanes>(loaded);
+        const int record = record_of_lane<kLanes>(group, lane);
+        if (record >= records) return;
         const int token = token_of_record<T>(record, blocks);
         const int block = record - token * blocks;
-        const ActivationCodes codes = activation_codes<P>(loaded);
-        quantize_block(codes, lane, block, blocks, token_image(lds, token, blocks));
+        quantize_block<kLanes>(codes, lane % kLanes, block, blocks, token_image(lds, token, blocks));
         if (keep_records) {
-            store_record(records_out + (static_cast<std::int64_t>(token0 + token) * blocks + block) *
-                             kActRecord, lane, codes);
+            store_record_quads<kLanes>(records_out + (static_cast<std::int64_t>(token0 + token) * blocks + block) * kActRecord,
+                               lane % kLanes, codes);
         }
     };
 #pragma unroll
     for (int e = 0; e < kEarly; ++e) {
-        const int record = wave + e * WAVES;
-        if (record < records) quantize_record(early[e], record);
+        if (records_of_group(kLanes) * (wave + e * WAVES) < records) {
+            quantize_group(early[e], wave + e * WAVES);
+        } else {
+            drop_records(early[e]);
+        }
     }
     if constexpr (P != kDualNorm) {  // (a normalised row has at most 32 records: all early)
-        for (int record = wave + kEarly * WAVES; record < records; record += WAVES) {
-            const int token = token_of_record<T>(record, blocks);
-            const int block = record - token * blocks;
-            const float4 x = load_activations<P>(
-                pass_first, pass_second,
-                static_cast<std::int64_t>(token) * input_dim + block * 256 + lane * 4);
-            quantize_record(x, record);
+        for (int group = wave + kEarly * WAVES; records_of_group(kLanes) * group < records; group += WAVES) {
+            RecordQuads<P, kLanes> x;
+            request_records<T, P, kLanes>(x, pass_first, pass_second, group, records, blocks, input_dim, lane);
+            quantize_group(x, group);
         }
     }
     if constexpr (kStages == 3) issue(stages[2], 2 % kSlices);
@@ -499,13 +466,25 @@ __global__ __launch_bounds__(WAVES * kWave) void gemv_dot_kernel(
 #pragma unroll
     for (int t = 0; t < T; ++t) acc[t] = 0.0f;
 
-    DotCursor work;
-    work.second_minus_first = 0;  // only its row and iteration counters are used in pair mode
+    DotCursor work;  // (its row pointer is not used)
     work.start(row_count > 0 ? row_begin : 0, stride, data_a, data_b, data_c, bound1, bound2, bound3);
+    // where the first token's sum of the current row goes
+    std::int64_t output_dim = 0;
+    const auto output_of_row = [&]() {
+        float* base = tail.output[0];
+        output_dim = tail.output_dim[0];
+#pragma unroll
+        for (int k = 1; k < 4; ++k) {
+            base = work.op == k ? tail.output[k] : base;
+            output_dim = work.op == k ? tail.output_dim[k] : output_dim;
+        }
+        return base + static_cast<std::int64_t>(token0) * output_dim + (work.row - work.first_row);
+    };
+    float* output = output_of_row();
     float first_total = 0.0f;  // pair mode: the finished sum of the first projection's row
     // `slice`: for ITER > 0 the slice of its row this step works on
     auto compute = [&](const Stage<kQ5>& stage, int slice) {
-        const int iteration = work.iteration;
+        const int iteration = ITER > 0 ? slice : work.iteration;
         const int raw_unit = (PAIRS ? iteration % (ITER > 0 ? ITER : 1) : iteration) * kWave + lane;
         const bool live = raw_unit < units;
         const int unit = min(raw_unit, units - 1);
@@ -520,31 +499,24 @@ __global__ __launch_bounds__(WAVES * kWave) void gemv_dot_kernel(
                 acc[0] = 0.0f;
             } else if (iteration == 2 * ITER - 1) {
                 const float second_total = wave_total(acc[0]);
-                if (lane == 0) {
-                    tail.output[0][work.row] = apply_prologue<kSwiGlu>(first_total, second_total);
-                }
+                if (lane == 0) *output = apply_prologue<kSwiGlu>(first_total, second_total);
+                ++output;
                 acc[0] = 0.0f;
             }
-        } else if (iteration == iterations - 1) {
+        } else if (iteration == (ITER > 0 ? ITER : iterations) - 1) {
             // the row is complete: fixed-order butterfly, lane 0 writes
-            float* base = tail.output[0];
-            std::int64_t output_dim = tail.output_dim[0];
-#pragma unroll
-            for (int k = 1; k < 4; ++k) {
-                base = work.op == k ? tail.output[k] : base;
-                output_dim = work.op == k ? tail.output_dim[k] : output_dim;
-            }
-            float* output = base + (work.row - work.first_row);
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 const float total_value = wave_total(acc[t]);
-                if (lane == 0 && t < pass_tokens) {
-                    output[static_cast<std::int64_t>(token0 + t) * output_dim] = total_value;
-                }
+                if (lane == 0 && t < pass_tokens) output[t * output_dim] = total_value;
                 acc[t] = 0.0f;
             }
+            ++output;
+            if (work.next_row(stride, data_a, data_b, data_c, bound1, bound2, bound3)) output = output_of_row();
+            work.iteration = 0;
+        } else {
+            ++work.iteration;
         }
-        work.template advance<kHalf>(iterations, stride, data_a, data_b, data_c, bound1, bound2, bound3);
     };
 
     for (int n = 0; n < total; n += kPeriod) {

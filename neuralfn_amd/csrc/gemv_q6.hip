@@ -79,21 +79,24 @@ __device__ __forceinline__ TokenImage token_image(std::uint8_t* lds, int token, 
     return image;
 }
 
-// Quantize the 256 activations of block `block`, four per lane: lane L holds
-// positions 4L..4L+3 = half L/32, quarter (L/8)%4, sixteen (L/4)%2, bytes 4*(L%4)..
-__device__ __forceinline__ void quantize_block(const ActivationCodes& codes, int lane, int block,
-                                               int blocks, const TokenImage& image) {
-    int sum = codes.sum;
-    sum += dpp_move<kQuadXor1>(sum);
-    sum += dpp_move<kQuadXor2>(sum);
+// The codes of block `block`; lane c of its LANES holds words LANES k + c: half word / 32, quarter (word / 8) % 4,
+// sixteen (word / 4) % 2, bytes 4 (word % 4)..
+template <int LANES>
+__device__ __forceinline__ void quantize_block(const QuadCodes<LANES>& codes, int c, int block, int blocks,
+                                               const TokenImage& image) {
     const int units = 4 * blocks;
-    const int quarter = (lane >> 3) & 3;
-    const int unit = 4 * block + 2 * (lane >> 5) + ((lane >> 2) & 1);
-    std::uint8_t* slot = image.planes + (2 * quarter * units + unit) * 16 + (lane & 3) * 4;
-    *reinterpret_cast<std::uint32_t*>(slot) = codes.hi;
-    *reinterpret_cast<std::uint32_t*>(slot + units * 16) = codes.lo;
-    if ((lane & 3) == 0) image.sums[unit * 4 + quarter] = sum;
-    if (lane == 0) image.scale[block] = codes.maximum * (1.0f / kCodeRange);
+#pragma unroll
+    for (int k = 0; k < 64 / LANES; ++k) {
+        const int word = LANES * k + c;
+        const int quarter = (word >> 3) & 3;
+        const int unit = 4 * block + 2 * (word >> 5) + ((word >> 2) & 1);
+        std::uint8_t* slot = image.planes + (2 * quarter * units + unit) * 16 + (c & 3) * 4;
+        *reinterpret_cast<std::uint32_t*>(slot) = codes.hi[k];
+        *reinterpret_cast<std::uint32_t*>(slot + units * 16) = codes.lo[k];
+        const int sum = sum_of_sixteen(codes.sum[k]);
+        if ((c & 3) == 0) image.sums[unit * 4 + quarter] = sum;
+    }
+    if (c == 0) image.scale[block] = codes.maximum * (1.0f / kCodeRange);
 }
 
 struct Stage {
@@ -206,17 +209,10 @@ __global__ __launch_bounds__(kThreads) void gemv_q6_kernel(
     // that their short latency does not queue behind the weight loads.  All
     // loads are unconditional (clamped indices) to keep the load counters exact.
     const int records = pass_tokens * blocks;
-    constexpr int kEarly = 4;
-    float4 early[kEarly];
-#pragma unroll
-    for (int e = 0; e < kEarly; ++e) {
-        const int record = min(wave + e * kWaves, records - 1);
-        const int token = token_of_record<T>(record, blocks);
-        const int block = record - token * blocks;
-        early[e] = load_activations<P>(
-            pass_first, pass_second,
-            static_cast<std::int64_t>(token) * input_dim + block * 256 + lane * 4);
-    }
+    constexpr int kLanes = T == 1 ? 32 : 16;  // (fewer than sixteen records a token)
+    RecordQuads<P, kLanes> early;
+    request_records<T, P, kLanes>(early, pass_first, pass_second, wave, records, blocks, input_dim, lane);
+    __builtin_amdgcn_sched_barrier(0);  // (the compiler would put them behind what follows)
 
     // (2) weight loads of the first two (row, slice) pairs
     PairCursor fetch;
@@ -243,28 +239,27 @@ __global__ __launch_bounds__(kThreads) void gemv_q6_kernel(
     // (the first workgroup also leaves the records in the caller's workspace
     // for a later launch that shares this input)
     const bool keep_records = P != kRecords && records_out != nullptr && blockIdx.x == 0;
-    auto quantize_record = [&](float4 loaded, int record) {
+    auto quantize_group = [&](const RecordQuads<P, kLanes>& loaded, int group) {
+        const QuadCodes<kLanes> codes = quad_codes<P, kLanes>(loaded);
+        const int record = record_of_lane<kLanes>(group, lane);
+        if (record >= records) return;
         const int token = token_of_record<T>(record, blocks);
         const int block = record - token * blocks;
-        const ActivationCodes codes = activation_codes<P>(loaded);
-        quantize_block(codes, lane, block, blocks, token_image(lds, token, blocks));
+        quantize_block<kLanes>(codes, lane % kLanes, block, blocks, token_image(lds, token, blocks));
         if (keep_records) {
-            store_record(records_out + (static_cast<std::int64_t>(token0 + token) * blocks + block) *
-                             kActRecord, lane, codes);
+            store_record_quads<kLanes>(records_out + (static_cast<std::int64_t>(token0 + token) * blocks + block) * kActRecord,
+                               lane % kLanes, codes);
         }
     };
-#pragma unroll
-    for (int e = 0; e < kEarly; ++e) {
-        const int record = wave + e * kWaves;
-        if (record < records) quantize_record(early[e], record);
+    if (records_of_group(kLanes) * wave < records) {
+        quantize_group(early, wave);
+    } else {
+        drop_records(early);
     }
-    for (int record = wave + kEarly * kWaves; record < records; record += kWaves) {
-        const int token = token_of_record<T>(record, blocks);
-        const int block = record - token * blocks;
-        const float4 x = load_activations<P>(
-            pass_first, pass_second,
-            static_cast<std::int64_t>(token) * input_dim + block * 256 + lane * 4);
-        quantize_record(x, record);
+    for (int group = wave + kWaves; records_of_group(kLanes) * group < records; group += kWaves) {
+        RecordQuads<P, kLanes> x;
+        request_records<T, P, kLanes>(x, pass_first, pass_second, group, records, blocks, input_dim, lane);
+        quantize_group(x, group);
     }
     __syncthreads();
 
@@ -393,43 +388,66 @@ struct PassLoads {
 // projection (16,384 -> 6,656) 21.9 us at 6 to 8 and 13 to 16 KB past a multiple of 16, 21.45 at 0 to 5
 // (deep into a context; a short one 21.65 and 21.75).  Presumably the instruction cache, which keeps a layer's
 // kernels from one layer to the next; a counter run, whose launches start cold, shows the same misses.
+// The leading arguments (13 dwords) arrive in registers: what the first requests need.  The activations' go out before
+// anything else is worked out.  (With the projections read from a struct, five trips to the argument block, one behind
+// the other, came before a wave's first request: 2 to 5 us of the down projection's 7 before its barrier.)
+// `shape`: blocks of a row, from bit 10 on the tokens, from 16 on the rows of a wave.  starts_a, starts_b: four
+// sixteen-bit wave numbers, the first waves of projections 1 to 3 (0xffff: none) and the waves of the launch.
+// missing_a, missing_b: how many rows each projection's last wave has less than the others.
+struct Q6Tail {
+    const float* second;
+    LmHeadCandidate* candidates;
+    std::uint8_t* records_out;
+    float* output[4];
+    std::int64_t output_dim[4];
+};
+
 template <int T, int P, bool ARGMAX, int W, bool FEWER>
 __global__ __attribute__((aligned(16384))) __launch_bounds__(W * kWave) void gemv_q6_stream_kernel(
-    const float* __restrict__ first, const float* __restrict__ second, std::int64_t input_dim,
-    int tokens, int rows_per_wave, LmHeadCandidate* __restrict__ candidates,
-    std::uint8_t* __restrict__ records_out, ProjectionSet set) {
+    const float* __restrict__ first, std::uint64_t data_a, std::uint64_t data_b, std::uint64_t data_c,
+    std::uint32_t shape, std::uint32_t starts_a, std::uint32_t starts_b, std::uint32_t missing_a,
+    std::uint32_t missing_b, Q6Tail tail) {
     extern __shared__ __attribute__((aligned(16))) std::uint8_t lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int waves = FEWER ? static_cast<int>(blockDim.x) / kWave : W;
-    const int blocks = static_cast<int>(input_dim >> 8);  // per row, >= 16
+    const int blocks = static_cast<int>(shape & 0x3ffu);  // per row, >= 16
+    const int tokens = static_cast<int>((shape >> 10) & 0x3fu);
+    const int rows_per_wave = static_cast<int>(shape >> 16);
+    const int input_dim = blocks * 256;
     const int token0 = blockIdx.y * T;
-    const int pass_tokens = min(tokens - token0, T);
-    const float* pass_first = pass_input<P>(first, token0, static_cast<int>(input_dim));
+    const int pass_tokens = T == 1 ? 1 : min(tokens - token0, T);
+    const float* pass_first = pass_input<P>(first, token0, input_dim);
     const float* pass_second = P == kGated || P == kSwiGlu
-        ? second + static_cast<std::int64_t>(token0) * input_dim : nullptr;
+        ? tail.second + static_cast<std::int64_t>(token0) * input_dim : nullptr;
     std::uint8_t* staging = lds + T * token_image_bytes(blocks) + wave * kStagingBytes;
 
-    // rows and blocks of this wave: every projection owns a range of waves
-    // (first_tile is its first wave), a wave a contiguous range of its rows
+    // (1) activations of the first records this wave quantizes
+    const int records = pass_tokens * blocks;
+    constexpr int kLanes = 16;
+    RecordQuads<P, kLanes> early;
+    request_records<T, P, kLanes>(early, pass_first, pass_second, wave, records, blocks, input_dim, lane);
+    __builtin_amdgcn_sched_barrier(0);  // (the compiler would put them behind what follows)
+
+    // rows and blocks of this wave: every projection owns a range of waves, a wave a contiguous range of its rows
     const int wave_index = static_cast<int>(blockIdx.x) * waves + wave;
-    int which = 0;
-#pragma unroll
-    for (int index = 1; index < 4; ++index) {
-        if (index < set.count && wave_index >= static_cast<int>(set.op[index].first_tile)) which = index;
-    }
-    const Projection op = pick(set, which);
-    const std::int64_t row_begin =
-        static_cast<std::int64_t>(wave_index - static_cast<int>(op.first_tile)) * rows_per_wave;
-    const int row_count = static_cast<int>(max(
-        static_cast<std::int64_t>(0),
-        min(static_cast<std::int64_t>(rows_per_wave), op.output_dim - row_begin)));
+    const int start1 = static_cast<int>(starts_a & 0xffffu), start2 = static_cast<int>(starts_a >> 16);
+    const int start3 = static_cast<int>(starts_b & 0xffffu), wave_total_count = static_cast<int>(starts_b >> 16);
+    const int which = (wave_index >= start1 ? 1 : 0) + (wave_index >= start2 ? 1 : 0) + (wave_index >= start3 ? 1 : 0);
+    const int op_begin = which == 0 ? 0 : which == 1 ? start1 : which == 2 ? start2 : start3;
+    const int op_end = min(which == 0 ? start1 : which == 1 ? start2 : which == 2 ? start3 : 0xffff, wave_total_count);
+    const std::uint32_t missing_pair = which < 2 ? missing_a : missing_b;
+    const int missing = static_cast<int>((which & 1) != 0 ? missing_pair >> 16 : missing_pair & 0xffffu);
+    // (a wave past the last one stands at the last one's rows and has none)
+    const int op_wave = min(wave_index, op_end - 1) - op_begin;
+    const int rows_to_end = (op_end - op_begin - op_wave) * rows_per_wave - missing;  // of the tensor
+    const int row_count = wave_index < op_end ? min(rows_per_wave, rows_to_end) : 0;
+    const std::int64_t row_begin = static_cast<std::int64_t>(op_wave) * rows_per_wave;
     const int wave_blocks = row_count * blocks;
     const int passes = (wave_blocks + kPassBlocks - 1) / kPassBlocks;
-    // first byte of the wave's first block; a wave without rows points at the
-    // last row so that its (unused) loads stay inside the tensor
-    const std::uint8_t* stream = op.data +
-        min(row_begin, op.output_dim - 1) * op.row_stride;
+    // first byte of the wave's first block (a wave without rows reads, and does not use, blocks of the last row)
+    const std::uint8_t* op_data = (const std::uint8_t*)unpack_pointer(data_a, data_b, data_c, which);
+    const std::uint8_t* stream = op_data + row_begin * (static_cast<std::int64_t>(blocks) * kBlockBytes);
     const int stream_blocks = max(wave_blocks, 1);  // blocks that may be read from `stream`
 
     // Blocks are 210 bytes long, so every other block of a tensor that starts on a
@@ -446,14 +464,12 @@ __global__ __attribute__((aligned(16384))) __launch_bounds__(W * kWave) void gem
     // one: a pass that holds the last block of the tensor, or blocks that only
     // stand in for ones past the wave's range, reads every piece the plain way.
     // A tensor that does not start on a word is read the plain way throughout.
-    const bool realign = (reinterpret_cast<std::uintptr_t>(op.data) & 3u) == 0;
+    const bool realign = (reinterpret_cast<std::uintptr_t>(op_data) & 3u) == 0;
     const int stream_parity =
         static_cast<int>((reinterpret_cast<std::uintptr_t>(stream) >> 1) & 1u);
     // the tensor's last block as a block of this wave's stream (beyond it for most waves)
-    const std::int64_t blocks_to_end =
-        (op.output_dim - min(row_begin, op.output_dim - 1)) * static_cast<std::int64_t>(blocks);
     const int tensor_last_block =
-        static_cast<int>(min(blocks_to_end - 1, static_cast<std::int64_t>(0x7fffffff)));
+        static_cast<int>(min(static_cast<std::int64_t>(rows_to_end) * blocks - 1, static_cast<std::int64_t>(0x7fffffff)));
     static_assert(kPassBlocks % 2 == 0, "a block of a pass keeps its alignment from pass to pass");
     // passes read the plain way: from plain_from on, and plain_also
     const int plain_from = realign ? stream_blocks / kPassBlocks : 0;
@@ -489,55 +505,56 @@ __global__ __attribute__((aligned(16384))) __launch_bounds__(W * kWave) void gem
         }
     };
 
-    // (1) activations of the first records this wave quantizes, then (2) the
-    // packed bytes of the first two passes: all in flight together
-    const int records = pass_tokens * blocks;
-    constexpr int kEarly = 4;
-    float4 early[kEarly];
-#pragma unroll
-    for (int e = 0; e < kEarly; ++e) {
-        const int record = min(wave + e * waves, records - 1);
-        const int token = token_of_record<T>(record, blocks);
-        const int block = record - token * blocks;
-        early[e] = load_activations<P>(
-            pass_first, pass_second,
-            static_cast<std::int64_t>(token) * input_dim + block * 256 + lane * 4);
-    }
+    // (2) the packed bytes of the first pass
     PassLoads loads0, loads1;
     issue(loads0, 0);
 
     // (3) quantize; one barrier
     // (the first workgroup also leaves the records in the caller's workspace
     // for a later launch that shares this input)
+    std::uint8_t* const records_out = tail.records_out;
     const bool keep_records = P != kRecords && records_out != nullptr && blockIdx.x == 0;
-    auto quantize_record = [&](float4 loaded, int record) {
+    auto quantize_group = [&](const RecordQuads<P, kLanes>& loaded, int group) {
+        const QuadCodes<kLanes> codes = quad_codes<P, kLanes>(loaded);
+        const int record = record_of_lane<kLanes>(group, lane);
+        if (record >= records) return;
         const int token = token_of_record<T>(record, blocks);
         const int block = record - token * blocks;
-        const ActivationCodes codes = activation_codes<P>(loaded);
-        quantize_block(codes, lane, block, blocks, token_image(lds, token, blocks));
+        quantize_block<kLanes>(codes, lane % kLanes, block, blocks, token_image(lds, token, blocks));
         if (keep_records) {
-            store_record(records_out + (static_cast<std::int64_t>(token0 + token) * blocks + block) *
-                             kActRecord, lane, codes);
+            store_record_quads<kLanes>(records_out + (static_cast<std::int64_t>(token0 + token) * blocks + block) * kActRecord,
+                               lane % kLanes, codes);
         }
     };
-#pragma unroll
-    for (int e = 0; e < kEarly; ++e) {
-        const int record = wave + e * waves;
-        if (record < records) quantize_record(early[e], record);
+    if (records_of_group(kLanes) * wave < records) {
+        quantize_group(early, wave);
+    } else {
+        drop_records(early);
     }
-    for (int record = wave + kEarly * waves; record < records; record += waves) {
-        const int token = token_of_record<T>(record, blocks);
-        const int block = record - token * blocks;
-        const float4 x = load_activations<P>(
-            pass_first, pass_second,
-            static_cast<std::int64_t>(token) * input_dim + block * 256 + lane * 4);
-        quantize_record(x, record);
+    for (int group = wave + waves; records_of_group(kLanes) * group < records; group += waves) {
+        RecordQuads<P, kLanes> x;
+        request_records<T, P, kLanes>(x, pass_first, pass_second, group, records, blocks, input_dim, lane);
+        quantize_group(x, group);
     }
     // the second pass's weights are requested only now: requests that go out ahead of the
     // activation loads of waves that start later delay those, and every wave waits at
     // the barrier for all activations
     issue(loads1, min(1, max(passes - 1, 0)));
     __syncthreads();
+
+    // where the first token's sum of the wave's first row goes
+    float* output = nullptr;
+    std::int64_t output_dim = 0;
+    if constexpr (!ARGMAX) {
+        output = tail.output[0];
+        output_dim = tail.output_dim[0];
+#pragma unroll
+        for (int k = 1; k < 4; ++k) {
+            output = which == k ? tail.output[k] : output;
+            output_dim = which == k ? tail.output_dim[k] : output_dim;
+        }
+        output += token0 * output_dim + row_begin;
+    }
 
     float acc_current[T], acc_next[T];
     float best_value[T];
@@ -642,10 +659,7 @@ __global__ __attribute__((aligned(16384))) __launch_bounds__(W * kWave) void gem
                         best_index[t] = row_begin + row;
                     }
                 } else {
-                    if (lane == 0 && t < pass_tokens) {
-                        op.output[static_cast<std::int64_t>(token0 + t) * op.output_dim +
-                                  row_begin + row] = total_value;
-                    }
+                    if (lane == 0 && t < pass_tokens) output[t * output_dim + row] = total_value;
                 }
                 acc_current[t] = acc_next[t];
                 acc_next[t] = 0.0f;
@@ -684,7 +698,7 @@ __global__ __attribute__((aligned(16384))) __launch_bounds__(W * kWave) void gem
             candidate.index = index;
             candidate.value = value;
             candidate.pad = 0;
-            candidates[static_cast<std::int64_t>(token0 + t) * gridDim.x + blockIdx.x] = candidate;
+            tail.candidates[static_cast<std::int64_t>(token0 + t) * gridDim.x + blockIdx.x] = candidate;
         }
     }
 }
@@ -761,17 +775,36 @@ std::int64_t launch_stream(const ProjectionSet& set, const float* first, const f
     std::int64_t rows = 0;
     for (int index = 0; index < set.count; ++index) rows += set.op[index].output_dim;
     const std::int64_t rows_per_wave = stream_geometry(rows, W).rows_per_wave;
-    ProjectionSet placed = set;
+    Q6Tail tail{};
+    tail.second = second;
+    tail.candidates = candidates;
+    tail.records_out = records_out;
+    const void* data[4] = {};
+    std::uint32_t starts[4] = {0xffffu, 0xffffu, 0xffffu, 0}, missing[4] = {};
     std::int64_t waves = 0;
-    for (int index = 0; index < placed.count; ++index) {
-        placed.op[index].first_tile = static_cast<std::uint32_t>(waves);
-        waves += (placed.op[index].output_dim + rows_per_wave - 1) / rows_per_wave;
+    for (int index = 0; index < set.count; ++index) {
+        const std::int64_t output_dim = set.op[index].output_dim;
+        const std::int64_t op_waves = (output_dim + rows_per_wave - 1) / rows_per_wave;
+        data[index] = set.op[index].data;
+        tail.output[index] = set.op[index].output;
+        tail.output_dim[index] = output_dim;
+        if (index > 0) starts[index - 1] = static_cast<std::uint32_t>(waves);
+        missing[index] = static_cast<std::uint32_t>(op_waves * rows_per_wave - output_dim);
+        waves += op_waves;
     }
+    const std::int64_t blocks = set.input_dim >> 8;
+    if (waves >= 0xffff || rows_per_wave > 0xffff || tokens > 0x3f || blocks > 0x3ff) {
+        return launch_variant<T, P, ARGMAX>(set, first, second, records_out, tokens, candidates, stream);
+    }
+    starts[3] = static_cast<std::uint32_t>(waves);
+    const PackedPointers packed = pack_pointers(data);
+    const std::uint32_t shape = static_cast<std::uint32_t>(blocks | tokens << 10 | rows_per_wave << 16);
     const auto launch = [&](auto kernel, int waves_per_group) {
         const std::int64_t groups = (waves + waves_per_group - 1) / waves_per_group;
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups), passes), dim3(waves_per_group * kWave),
-                           lds, stream, first, second, set.input_dim, tokens, static_cast<int>(rows_per_wave),
-                           candidates, records_out, placed);
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups), passes), dim3(waves_per_group * kWave), lds,
+                           stream, first, packed.a, packed.b, packed.c, shape, starts[0] | starts[1] << 16,
+                           starts[2] | starts[3] << 16, missing[0] | missing[1] << 16, missing[2] | missing[3] << 16,
+                           tail);
         return groups;
     };
     if constexpr (T == 1 && W == 16 && !ARGMAX) {

@@ -58,17 +58,19 @@ __device__ __forceinline__ TokenImage token_image(std::uint8_t* lds, int token, 
     return image;
 }
 
-// Quantize the 256 activations of block `block`, four per lane: lane L holds
-// values 4L..4L+3 = unit L/16 of the block, sixteen (L/4)%4, bytes 4*(L%4)..
-__device__ __forceinline__ void quantize_block(const ActivationCodes& codes, int lane, int block,
-                                               int blocks, const TokenImage& image) {
+// The codes of block `block`; lane c of its LANES holds words LANES k + c: unit word / 16 of the block, sixteen
+// (word / 4) % 4, bytes 4 (word % 4)..
+template <int LANES>
+__device__ __forceinline__ void quantize_block(const QuadCodes<LANES>& codes, int c, int block, int blocks,
+                                               const TokenImage& image) {
     const int units = 4 * blocks;
-    const int unit = 4 * block + (lane >> 4);
-    const int sixteen = (lane >> 2) & 3;
-    std::uint8_t* slot = image.planes + (2 * sixteen * units + unit) * 16 + (lane & 3) * 4;
-    *reinterpret_cast<std::uint32_t*>(slot) = codes.hi;
-    *reinterpret_cast<std::uint32_t*>(slot + units * 16) = codes.lo;
-    if (lane == 0) image.scale[block] = codes.maximum * (1.0f / kCodeRange);
+    std::uint8_t* slot = image.planes + (2 * ((c >> 2) & 3) * units + 4 * block + (c >> 4)) * 16 + (c & 3) * 4;
+#pragma unroll
+    for (int k = 0; k < 64 / LANES; ++k) {
+        *reinterpret_cast<std::uint32_t*>(slot + LANES * k) = codes.hi[k];
+        *reinterpret_cast<std::uint32_t*>(slot + units * 16 + LANES * k) = codes.lo[k];
+    }
+    if (c == 0) image.scale[block] = codes.maximum * (1.0f / kCodeRange);
 }
 
 struct Stage {
@@ -76,7 +78,8 @@ struct Stage {
     std::uint32_t last;
 };
 
-template <int T, int P>
+// FEW: at most two records a wave.
+template <int T, int P, bool FEW>
 __global__ __launch_bounds__(kThreads) void gemv_q8_kernel(
     const float* __restrict__ first, const float* __restrict__ second, int tokens, int input_dim,
     int total_rows, int rows_per_group, int longer_groups, std::uint8_t* __restrict__ records_out,
@@ -104,17 +107,10 @@ __global__ __launch_bounds__(kThreads) void gemv_q8_kernel(
     // that their short latency does not queue behind the weight loads.  All
     // loads are unconditional (clamped indices) to keep the load counters exact.
     const int records = pass_tokens * blocks;
-    constexpr int kEarly = 4;
-    float4 early[kEarly];
-#pragma unroll
-    for (int e = 0; e < kEarly; ++e) {
-        const int record = min(wave + e * kWaves, records - 1);
-        const int token = token_of_record<T>(record, blocks);
-        const int block = record - token * blocks;
-        early[e] = load_activations<P>(
-            pass_first, pass_second,
-            static_cast<std::int64_t>(token) * input_dim + block * 256 + lane * 4);
-    }
+    constexpr int kLanes = FEW ? 32 : 16;
+    RecordQuads<P, kLanes> early;
+    request_records<T, P, kLanes>(early, pass_first, pass_second, wave, records, blocks, input_dim, lane);
+    __builtin_amdgcn_sched_barrier(0);  // (the compiler would put them behind what follows)
 
     // (2) weight loads of the first two (row, slice) pairs
     PairCursor fetch;
@@ -137,28 +133,27 @@ __global__ __launch_bounds__(kThreads) void gemv_q8_kernel(
     // (the first workgroup also leaves the records in the caller's workspace
     // for a later launch that shares this input)
     const bool keep_records = P != kRecords && records_out != nullptr && blockIdx.x == 0;
-    auto quantize_record = [&](float4 loaded, int record) {
+    auto quantize_group = [&](const RecordQuads<P, kLanes>& loaded, int group) {
+        const QuadCodes<kLanes> codes = quad_codes<P, kLanes>(loaded);
+        const int record = record_of_lane<kLanes>(group, lane);
+        if (record >= records) return;
         const int token = token_of_record<T>(record, blocks);
         const int block = record - token * blocks;
-        const ActivationCodes codes = activation_codes<P>(loaded);
-        quantize_block(codes, lane, block, blocks, token_image(lds, token, blocks));
+        quantize_block<kLanes>(codes, lane % kLanes, block, blocks, token_image(lds, token, blocks));
         if (keep_records) {
-            store_record(records_out + (static_cast<std::int64_t>(token0 + token) * blocks + block) *
-                             kActRecord, lane, codes);
+            store_record_quads<kLanes>(records_out + (static_cast<std::int64_t>(token0 + token) * blocks + block) * kActRecord,
+                               lane % kLanes, codes);
         }
     };
-#pragma unroll
-    for (int e = 0; e < kEarly; ++e) {
-        const int record = wave + e * kWaves;
-        if (record < records) quantize_record(early[e], record);
+    if (records_of_group(kLanes) * wave < records) {
+        quantize_group(early, wave);
+    } else {
+        drop_records(early);
     }
-    for (int record = wave + kEarly * kWaves; record < records; record += kWaves) {
-        const int token = token_of_record<T>(record, blocks);
-        const int block = record - token * blocks;
-        const float4 x = load_activations<P>(
-            pass_first, pass_second,
-            static_cast<std::int64_t>(token) * input_dim + block * 256 + lane * 4);
-        quantize_record(x, record);
+    for (int group = wave + kWaves; records_of_group(kLanes) * group < records; group += kWaves) {
+        RecordQuads<P, kLanes> x;
+        request_records<T, P, kLanes>(x, pass_first, pass_second, group, records, blocks, input_dim, lane);
+        quantize_group(x, group);
     }
     // the second stage's weights are requested only now: requests that go out ahead of the
     // activation loads of waves that start later delay those, and every wave waits at
@@ -258,8 +253,13 @@ void launch_variant(ProjectionSet set, const float* first, const float* second,
         rows += set.op[index].output_dim;
     }
     const std::size_t lds = static_cast<std::size_t>(T) * token_image_bytes(set.input_dim >> 8);
-    auto kernel = gemv_q8_kernel<T, P>;
-    allow_large_lds<gemv_q8_kernel<T, P>>();
+    const bool few = T * (set.input_dim >> 8) <= 2 * kWaves;
+    auto kernel = few ? gemv_q8_kernel<T, P, true> : gemv_q8_kernel<T, P, false>;
+    if (few) {
+        allow_large_lds<gemv_q8_kernel<T, P, true>>();
+    } else {
+        allow_large_lds<gemv_q8_kernel<T, P, false>>();
+    }
     const int passes = (tokens + T - 1) / T;
     const std::int64_t groups = decode_groups(rows, kWaves);
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups), passes), dim3(kThreads), lds,

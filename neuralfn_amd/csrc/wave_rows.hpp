@@ -51,7 +51,11 @@ __device__ __forceinline__ float wave_total(float v) {
     v += dpp_move<kQuadXor2>(v);
     v += dpp_move<kHalfMirror>(v);
     v += dpp_move<kRowMirror>(v);
-    return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+    // (row 0 + row 1) + (row 2 + row 3)
+    auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+    rows = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
 }
 
 __device__ __forceinline__ std::uint32_t perm(std::uint32_t hi, std::uint32_t lo, std::uint32_t sel) {
@@ -69,24 +73,29 @@ struct ActivationCodes {
     float maximum;         // the wave's largest magnitude; scale = maximum / 32512
 };
 
+__device__ __forceinline__ float code_factor(float maximum) {
+    return maximum > 1.0e-30f ? kCodeRange * __builtin_amdgcn_rcpf(maximum) : 0.0f;
+}
+__device__ __forceinline__ void encode_quad(float4 x, float factor, std::uint32_t& hi, std::uint32_t& lo) {
+    // 1.5*2^23 + 128: the low 16 bits of the sum's bit pattern are
+    // round-to-nearest-even(x*factor) + 128 in two's complement.
+    constexpr float kMagic = 12582912.0f + 128.0f;
+    const std::uint32_t u0 = __float_as_uint(fmaf(x.x, factor, kMagic));
+    const std::uint32_t u1 = __float_as_uint(fmaf(x.y, factor, kMagic));
+    const std::uint32_t u2 = __float_as_uint(fmaf(x.z, factor, kMagic));
+    const std::uint32_t u3 = __float_as_uint(fmaf(x.w, factor, kMagic));
+    // code + 128 = 256*hi + (lo + 128): hi is byte 1, lo is byte 0 with its top bit flipped
+    const std::uint32_t p01 = perm(u1, u0, 0x05010400u);  // [u0.b0, u1.b0, u0.b1, u1.b1]
+    const std::uint32_t p23 = perm(u3, u2, 0x05010400u);
+    lo = perm(p23, p01, 0x05040100u) ^ 0x80808080u;
+    hi = perm(p23, p01, 0x07060302u);
+}
+
 __device__ __forceinline__ ActivationCodes encode_activations(float4 x) {
     const float local = fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)));
     ActivationCodes codes;
     codes.maximum = wave_max(local);
-    const float inverse =
-        codes.maximum > 1.0e-30f ? kCodeRange * __builtin_amdgcn_rcpf(codes.maximum) : 0.0f;
-    // 1.5*2^23 + 128: the low 16 bits of the sum's bit pattern are
-    // round-to-nearest-even(x*inverse) + 128 in two's complement.
-    constexpr float kMagic = 12582912.0f + 128.0f;
-    const std::uint32_t u0 = __float_as_uint(fmaf(x.x, inverse, kMagic));
-    const std::uint32_t u1 = __float_as_uint(fmaf(x.y, inverse, kMagic));
-    const std::uint32_t u2 = __float_as_uint(fmaf(x.z, inverse, kMagic));
-    const std::uint32_t u3 = __float_as_uint(fmaf(x.w, inverse, kMagic));
-    // code + 128 = 256*hi + (lo + 128): hi is byte 1, lo is byte 0 with its top bit flipped
-    const std::uint32_t p01 = perm(u1, u0, 0x05010400u);  // [u0.b0, u1.b0, u0.b1, u1.b1]
-    const std::uint32_t p23 = perm(u3, u2, 0x05010400u);
-    codes.lo = perm(p23, p01, 0x05040100u) ^ 0x80808080u;
-    codes.hi = perm(p23, p01, 0x07060302u);
+    encode_quad(x, code_factor(codes.maximum), codes.hi, codes.lo);
     codes.sum = (__builtin_amdgcn_sdot4(static_cast<int>(codes.hi), 0x01010101, 0, false) << 8) +
         __builtin_amdgcn_sdot4(static_cast<int>(codes.lo), 0x01010101, 0, false);
     return codes;
@@ -174,14 +183,177 @@ __device__ __forceinline__ void store_record(std::uint8_t* record, int lane,
 }
 
 // Token of activation record `record` (records run token by token, `blocks`
-// per token).  One token per pass: no division on the way to the first loads.
+// per token), of T tokens at most: no division on the way to the first loads.
 template <int T>
 __device__ __forceinline__ int token_of_record(int record, int blocks) {
-    if constexpr (T == 1) {
-        return 0;
-    } else {
-        return record / blocks;
+    int token = 0;
+#pragma unroll
+    for (int t = 1; t < T; ++t) token += record >= t * blocks ? 1 : 0;
+    return token;
+}
+
+// ---- several records at once by a wave: the one-row kernels' quantizer.  LANES lanes to a record (16 or 32): lane c of
+// them holds its words LANES k + c of four values, k = 0..64 / LANES (each load reads 16 LANES bytes in a row a record).
+// What bounds it is instructions, since every workgroup quantizes the whole row for itself: a record a wave and pass, as
+// encode_activations has it, takes 60 of them a record, this 25 (of 16 lanes), for the same codes, sums and maximum.
+// Thirty-two lanes where sixteen would leave half of the waves without a record (rows of up to 4,096 columns).
+// With the rows' bookkeeping at compile time (gemv_dot.hip), us: two rows of 6,656 columns into 4,608 of Q4_K 9.5 -> 8.3,
+// one of 16,384 into 6,656 of Q4_K 15.8 -> 14.7, of Q5_K 19.0 -> 17.9, of Q8_0 25.5 -> 24.7.
+constexpr int records_of_group(int lanes) { return kWave / lanes; }
+
+template <int P, int LANES>
+struct RecordQuads {
+    static constexpr int kQuads = 64 / LANES;
+    float4 quad[kQuads];
+    float4 other[P == kGated || P == kSwiGlu ? kQuads : 1];  // the prologue's second operand
+};
+template <int LANES>
+struct QuadCodes {
+    std::uint32_t hi[64 / LANES], lo[64 / LANES];  // four bytes each, value order
+    int sum[64 / LANES];                           // of a quad's four codes
+    float maximum;                                 // the record's largest magnitude
+};
+
+// The lane's record of group `group`; from the number of records on there is none.
+template <int LANES>
+__device__ __forceinline__ int record_of_lane(int group, int lane) {
+    return records_of_group(LANES) * group + lane / LANES;
+}
+
+// ... its values as they lie in memory (records past the last repeat it).
+template <int T, int P, int LANES>
+__device__ __forceinline__ void request_records(RecordQuads<P, LANES>& x, const float* __restrict__ first,
+                                                const float* __restrict__ second, int group, int records, int blocks,
+                                                int input_dim, int lane) {
+    const int record = min(record_of_lane<LANES>(group, lane), records - 1);
+    const int token = token_of_record<T>(record, blocks);
+    const std::int64_t column =
+        static_cast<std::int64_t>(token) * input_dim + (record - token * blocks) * 256 + 4 * (lane % LANES);
+#pragma unroll
+    for (int k = 0; k < x.kQuads; ++k) {
+        x.quad[k] = load_activations<P == kRecords ? kRecords : kPlain>(first, second, column + 4 * LANES * k);
     }
+    if constexpr (P == kGated || P == kSwiGlu) {
+#pragma unroll
+        for (int k = 0; k < x.kQuads; ++k) x.other[k] = *reinterpret_cast<const float4*>(second + column + 4 * LANES * k);
+    }
+}
+
+// For a wave that has no record of a group it has requested: without a use on every path the compiler moves the
+// requests to the one that has it, behind the weights' requests.
+template <int P, int LANES>
+__device__ __forceinline__ void drop_records(const RecordQuads<P, LANES>& x) {
+#pragma unroll
+    for (int k = 0; k < x.kQuads; ++k) {
+        asm volatile("" : : "v"(x.quad[k].x), "v"(x.quad[k].y), "v"(x.quad[k].z), "v"(x.quad[k].w));
+        if constexpr (P == kGated || P == kSwiGlu) {
+            asm volatile("" : : "v"(x.other[k].x), "v"(x.other[k].y), "v"(x.other[k].z), "v"(x.other[k].w));
+        }
+    }
+}
+
+template <int P, int LANES>
+__device__ __forceinline__ QuadCodes<LANES> quad_codes(const RecordQuads<P, LANES>& x) {
+    static_assert(LANES == 16 || LANES == 32, "a row or two of lanes");
+    constexpr int kQuads = 64 / LANES;
+    QuadCodes<LANES> codes;
+    if constexpr (P == kRecords) {
+#pragma unroll
+        for (int k = 0; k < kQuads; ++k) {
+            codes.hi[k] = __float_as_uint(x.quad[k].x);
+            codes.lo[k] = __float_as_uint(x.quad[k].y);
+        }
+        codes.maximum = x.quad[0].z;
+    } else {
+        float4 values[kQuads];
+        std::uint32_t largest = 0;  // (wave_max's order of magnitudes)
+#pragma unroll
+        for (int k = 0; k < kQuads; ++k) {
+            float4 q = x.quad[k];
+            if constexpr (P == kGated || P == kSwiGlu) {
+                q.x = apply_prologue<P>(q.x, x.other[k].x);
+                q.y = apply_prologue<P>(q.y, x.other[k].y);
+                q.z = apply_prologue<P>(q.z, x.other[k].z);
+                q.w = apply_prologue<P>(q.w, x.other[k].w);
+            }
+            values[k] = q;
+            largest = max(largest, __float_as_uint(fmaxf(fmaxf(fabsf(q.x), fabsf(q.y)), fmaxf(fabsf(q.z), fabsf(q.w)))));
+        }
+        largest = max(largest, static_cast<std::uint32_t>(dpp_move<kQuadXor1>(static_cast<int>(largest))));
+        largest = max(largest, static_cast<std::uint32_t>(dpp_move<kQuadXor2>(static_cast<int>(largest))));
+        largest = max(largest, static_cast<std::uint32_t>(dpp_move<kHalfMirror>(static_cast<int>(largest))));
+        largest = max(largest, static_cast<std::uint32_t>(dpp_move<kRowMirror>(static_cast<int>(largest))));
+        if constexpr (LANES == 32) {
+            const auto rows = __builtin_amdgcn_permlane16_swap(largest, largest, false, false);
+            largest = max(rows[0], rows[1]);
+        }
+        codes.maximum = __uint_as_float(largest);
+        const float inverse = code_factor(codes.maximum);
+#pragma unroll
+        for (int k = 0; k < kQuads; ++k) encode_quad(values[k], inverse, codes.hi[k], codes.lo[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < kQuads; ++k) {
+        codes.sum[k] = (__builtin_amdgcn_sdot4(static_cast<int>(codes.hi[k]), 0x01010101, 0, false) << 8) +
+            __builtin_amdgcn_sdot4(static_cast<int>(codes.lo[k]), 0x01010101, 0, false);
+    }
+    return codes;
+}
+
+// The sum over the lane's four (eight) neighbours of the record: of sixteen (32) values in a row.
+__device__ __forceinline__ int sum_of_sixteen(int sum) {
+    sum += dpp_move<kQuadXor1>(sum);
+    return sum + dpp_move<kQuadXor2>(sum);
+}
+__device__ __forceinline__ int sum_of_thirty_two(int sum) {
+    sum = sum_of_sixteen(sum);
+    return sum + dpp_move<kHalfMirror>(sum);
+}
+
+// store_record from such lanes; `c` = lane % LANES.
+template <int LANES>
+__device__ __forceinline__ void store_record_quads(std::uint8_t* record, int c, const QuadCodes<LANES>& codes) {
+#pragma unroll
+    for (int k = 0; k < 64 / LANES; ++k) {
+        const int word = LANES * k + c;
+        *reinterpret_cast<std::uint32_t*>(record + 4 * word) = codes.hi[k];
+        *reinterpret_cast<std::uint32_t*>(record + 256 + 4 * word) = codes.lo[k];
+        const int sum = sum_of_thirty_two(codes.sum[k]);
+        if ((c & 7) == 0) *reinterpret_cast<int*>(record + kRecordSums + (word >> 3) * 4) = sum;
+    }
+    if (c == 0) {
+        *reinterpret_cast<float*>(record + kRecordScale) = codes.maximum * (1.0f / kCodeRange);
+        *reinterpret_cast<float*>(record + kRecordMaximum) = codes.maximum;
+    }
+}
+
+typedef const __attribute__((address_space(1))) std::uint8_t* GlobalBytes;
+
+// Four 48-bit device addresses in three 64-bit words.
+struct PackedPointers {
+    std::uint64_t a, b, c;
+};
+constexpr std::uint64_t kAddressMask = (std::uint64_t(1) << 48) - 1;
+inline PackedPointers pack_pointers(const void* const p[4]) {
+    std::uint64_t v[4];
+    for (int i = 0; i < 4; ++i) v[i] = reinterpret_cast<std::uint64_t>(p[i]) & kAddressMask;
+    PackedPointers packed;
+    packed.a = v[0] | (v[1] << 48);
+    packed.b = (v[1] >> 16) | (v[2] << 32);
+    packed.c = (v[2] >> 32) | (v[3] << 16);
+    return packed;
+}
+__device__ __forceinline__ GlobalBytes unpack_pointer(std::uint64_t a, std::uint64_t b,
+                                                      std::uint64_t c, int index) {
+    const std::uint64_t p0 = a & kAddressMask;
+    const std::uint64_t p1 = (a >> 48) | ((b & 0xffffffffull) << 16);
+    const std::uint64_t p2 = (b >> 32) | ((c & 0xffffull) << 32);
+    const std::uint64_t p3 = c >> 16;
+    std::uint64_t p = p0;
+    p = index == 1 ? p1 : p;
+    p = index == 2 ? p2 : p;
+    p = index == 3 ? p3 : p;
+    return reinterpret_cast<GlobalBytes>(p);
 }
 
 // Projection `index` of the set, chosen with scalar selects from fields that
