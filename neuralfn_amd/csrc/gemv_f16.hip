@@ -40,6 +40,8 @@
 #include "lm_head.hpp"
 #include "wave_rows.hpp"
 
+#include <type_traits>
+
 namespace nfn {
 
 namespace {
@@ -50,7 +52,8 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 constexpr int kTileRows = 16;
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * kWave;
-constexpr int kDepth = 4;  // blocks in flight per wave
+constexpr int kDepth = 4;       // blocks in flight per wave
+constexpr int kShortDepth = 2;  // ... of a tile, in rows of so many blocks a wave: of two tiles
 
 // ---- activations: fp32 -> fp16 scaled per row and K share, [column / 8][row][8] ----
 
@@ -129,7 +132,6 @@ __global__ __launch_bounds__(kImageThreads) void f16_image_kernel(
 
 typedef const __attribute__((address_space(1))) std::uint8_t* GlobalBytes;
 typedef const __attribute__((address_space(1))) u32x4* GlobalVec;
-typedef const __attribute__((address_space(1))) f16x8* GlobalFragment;
 
 __device__ __forceinline__ f16x8 as_operand(std::uint32_t a, std::uint32_t b, std::uint32_t c,
                                             std::uint32_t d) {
@@ -492,7 +494,8 @@ struct TileShape {
     int final_row;         // the projection's last row if it is one of the tile's, else -1
 };
 
-template <std::uint32_t ENC, int MODE, bool RING>
+// DEPTH: blocks of a wave's share of K that it holds the fragments of (kDepth, or kShortDepth where no share has more).
+template <std::uint32_t ENC, int MODE, bool RING, int DEPTH>
 __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
     const std::uint8_t* __restrict__ image, const float* __restrict__ inverse_scale, int tokens,
     std::uint32_t total_tiles, int input_dim, LmHeadCandidate* __restrict__ candidates,
@@ -519,26 +522,34 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
     const int begin = blocks * share / kWaves;
     const int end = blocks * (share + 1) / kWaves;
     const int count = end - begin;
-    const int chunks = ((blocks + kWaves - 1) / kWaves + kDepth - 1) / kDepth;  // the same for every wave
+    const int chunks = ((blocks + kWaves - 1) / kWaves + DEPTH - 1) / DEPTH;  // the same for every wave
 
     // The 16 bytes of group g of eight columns for token i: image + (g * tokens + i) * 16, as
     // a uniform part (block and instruction) and this lane's part (its quarter and token).
-    // Lanes past the last token read token 0 again: a row of A only reaches its own row of
-    // the result, and those rows are never stored.
-    const GlobalBytes global_image = (GlobalBytes)image;
+    // Lanes past the last token and steps past the wave's last block ask for bytes past the image's end, which a
+    // buffer load answers with zeros from nowhere (a row of A only reaches its own row of the result, and those rows
+    // are never stored): a compute unit takes the fragments of all eight waves in at 64 bytes a cycle, and asking
+    // for token 0 or the last block again cost eight rows of 4,096 columns 0.2 of 10.3 us, sixteen of 6,656 columns
+    // 0.6 of 14.7.  (A condition around the loads has every wait behind it wait for all of them: sixteen rows of
+    // 8,192 columns 14.9 -> 15.8 us.)
     const std::uint32_t group_bytes = static_cast<std::uint32_t>(tokens) * 16;
     const std::uint32_t lane_fragment =
-        static_cast<std::uint32_t>(Block::lane_group(j)) * group_bytes + (i < tokens ? i : 0) * 16;
-    f16x8 fragments[kDepth][8];
+        static_cast<std::uint32_t>(Block::lane_group(j)) * group_bytes + i * 16;
+    constexpr std::uint32_t kNowhere = 0x80000000u;
+    const auto image_buffer = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<std::uint8_t*>(image), 0, static_cast<int>(blocks * 32 * group_bytes), 0x00027000);
+    f16x8 fragments[DEPTH][8];
     auto load_fragments = [&](int chunk) {
 #pragma unroll
-        for (int s = 0; s < kDepth; ++s) {
-            const int block = begin + max(min(chunk * kDepth + s, count - 1), 0);
-            const GlobalBytes block_image = global_image + static_cast<std::int64_t>(block) * 32 * group_bytes;
+        for (int s = 0; s < DEPTH; ++s) {
+            const int local = chunk * DEPTH + s;
+            const std::uint32_t mine = local < count && i < tokens ? lane_fragment : kNowhere;
+            const std::uint32_t block_offset =
+                static_cast<std::uint32_t>(begin + min(local, max(count - 1, 0))) * 32 * group_bytes;
 #pragma unroll
             for (int m = 0; m < 8; ++m) {
-                fragments[s][m] = *reinterpret_cast<GlobalFragment>(
-                    block_image + Block::step_group(m) * group_bytes + lane_fragment);
+                fragments[s][m] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                    image_buffer, mine, block_offset + Block::step_group(m) * group_bytes, 0));
             }
         }
     };
@@ -608,13 +619,14 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
         fetch_setup();
     };
     auto fetch = [&](PackedBlock<ENC>& stage, int s) {
-        const int local = fetch_chunk * kDepth + s;  // block of this wave's K range
+        const int local = fetch_chunk * DEPTH + s;  // block of this wave's K range
         const bool work = fetch_live && local < count;
         const GlobalBytes source = work
             ? fetch_tile + static_cast<std::int64_t>(begin + local) * Block::kBytes : (GlobalBytes)set.op[0].data;
         stage.load(source, work ? fetch_row : 0u, work ? load_quarter : 0);
     };
-    PackedBlock<ENC> stages[RING ? 1 : kDepth];
+    constexpr int kAhead = DEPTH == kShortDepth ? kGroupTiles : 1;  // tiles that a step's load runs ahead
+    PackedBlock<ENC> stages[RING ? 1 : kAhead * DEPTH];
 
     // RING form: a cursor over the steps that have work runs kStages - 1 of them ahead.  A
     // step's kLoads instructions each bring the block of kRowsPerLoad rows; lane l of one has
@@ -653,11 +665,11 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
                 for (int q = 0; q < Lds::kLoads; ++q) ring_offset[q] = 0;
                 return;
             }
-            ring_steps = min(kDepth, count - ring_chunk * kDepth);
+            ring_steps = min(DEPTH, count - ring_chunk * DEPTH);
             if (ring_steps > 0) break;
         }
         const TileShape shape = tile_shape(ring_group, ring_slot);
-        const int first = begin + ring_chunk * kDepth;
+        const int first = begin + ring_chunk * DEPTH;
         ring_ptr = shape.base + static_cast<std::int64_t>(first) * Block::kBytes;
         ring_bump = Block::kBytes;
         ring_step = 0;
@@ -733,8 +745,11 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
     } else {
         fetch_setup();
 #pragma unroll
-        for (int s = 0; s < kDepth; ++s) fetch(stages[s], s);
-        fetch_advance();
+        for (int t = 0; t < kAhead; ++t) {
+#pragma unroll
+            for (int s = 0; s < DEPTH; ++s) fetch(stages[t * DEPTH + s], s);
+            fetch_advance();
+        }
     }
 
     // ARGMAX: the running best of every (lane, result register) of the waves that add up tiles
@@ -755,14 +770,14 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
         const int group_tiles = tiles_of_group(group);
         for (int chunk = 0; chunk < chunks; ++chunk) {
             if (chunks > 1 || (group == 0 && !fragments_first)) load_fragments(chunk);
-            const int chunk_count = min(kDepth, count - chunk * kDepth);  // this wave's blocks of the chunk
+            const int chunk_count = min(DEPTH, count - chunk * DEPTH);  // this wave's blocks of the chunk
 #pragma unroll
             for (int t = 0; t < kGroupTiles; ++t) {
                 if (t >= group_tiles) break;
 #pragma unroll
-                for (int s = 0; s < kDepth; ++s) {
+                for (int s = 0; s < DEPTH; ++s) {
                     if (RING && s >= chunk_count) break;  // (the plain form fetches in every step)
-                    PackedBlock<ENC>& stage = stages[RING ? 0 : s];
+                    PackedBlock<ENC>& stage = stages[RING ? 0 : (kAhead > 1 ? t : 0) * DEPTH + s];
                     if (s < chunk_count) {
                         const f16x8 (&a)[8] = fragments[s];
                         if constexpr (RING) {
@@ -913,6 +928,14 @@ bool ring_form(const ProjectionSet& set) {
     return false;
 }
 
+// Rows of up to 4,096 columns: a wave's share of K has kShortDepth blocks at most.  With kDepth, half of such a
+// launch's steps stood empty and still asked for their fragments and a block of weights; with kShortDepth they are
+// gone, and the registers hold the weights of two tiles instead.  Medians in us, kDepth -> kShortDepth: Q4_K
+// 2,048 -> 7,168 of 5 rows 11.2 -> 9.3, 4,096 -> 4,096 of 8 rows 10.5 -> 9.2, gate and up 4,096 -> 16,384 of 8 rows
+// 28.0 -> 25.9; Q6_K 4,096 -> 8,192 of 8 rows 14.9 -> 14.1; Q8_0 2,560 -> 10,240 of 16 rows 15.7 -> 14.4.  Longer rows
+// need the deeper pipeline: their shares would take twice the chunks, each a wait of its own for its fragments.
+bool short_rows(std::int64_t input_dim) { return input_dim <= kShortDepth * kWaves * 256; }
+
 // `candidates` non-null: the lm_head form (one projection), which returns its workgroup count.
 template <std::uint32_t ENC>
 std::uint32_t launch_encoding(ProjectionSet set, const std::uint8_t* image, const float* inverse_scale,
@@ -923,27 +946,30 @@ std::uint32_t launch_encoding(ProjectionSet set, const std::uint8_t* image, cons
         tiles += static_cast<std::uint32_t>((set.op[index].output_dim + kTileRows - 1) / kTileRows);
     }
     const std::uint32_t grid = grid_of(tiles, candidates != nullptr);
+    const bool few = short_rows(set.input_dim);
+    const auto launch = [&](auto kernel, unsigned lds) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, image, inverse_scale, tokens, tiles,
+                           static_cast<int>(set.input_dim), candidates, set);
+    };
+    const auto launch_ring = [&](auto mode, auto depth) {
+        constexpr unsigned kLds = Ring<ENC>::kLdsBytes;  // (beside 36 KB of static LDS)
+        allow_large_lds<gemv_f16_kernel<ENC, mode(), true, depth()>>(kLds);
+        launch(gemv_f16_kernel<ENC, mode(), true, depth()>, kLds);
+    };
+    const std::integral_constant<int, kDepth> deep;
+    const std::integral_constant<int, kShortDepth> shallow;
+    const std::integral_constant<int, kArgmax> argmax;
+    const std::integral_constant<int, kStore> store;
     if (ring_form<ENC>(set)) {
-        constexpr unsigned kLds = Ring<ENC>::kLdsBytes;
         if (candidates != nullptr) {
-            allow_large_lds<gemv_f16_kernel<ENC, kArgmax, true>>(kLds);  // (beside 36 KB of static LDS)
-            hipLaunchKernelGGL((gemv_f16_kernel<ENC, kArgmax, true>), dim3(grid), dim3(kThreads), kLds,
-                               stream, image, inverse_scale, tokens, tiles,
-                               static_cast<int>(set.input_dim), candidates, set);
+            few ? launch_ring(argmax, shallow) : launch_ring(argmax, deep);
         } else {
-            allow_large_lds<gemv_f16_kernel<ENC, kStore, true>>(kLds);
-            hipLaunchKernelGGL((gemv_f16_kernel<ENC, kStore, true>), dim3(grid), dim3(kThreads), kLds,
-                               stream, image, inverse_scale, tokens, tiles,
-                               static_cast<int>(set.input_dim), candidates, set);
+            few ? launch_ring(store, shallow) : launch_ring(store, deep);
         }
     } else if (candidates != nullptr) {
-        hipLaunchKernelGGL((gemv_f16_kernel<ENC, kArgmax, false>), dim3(grid), dim3(kThreads), 0, stream,
-                           image, inverse_scale, tokens, tiles, static_cast<int>(set.input_dim),
-                           candidates, set);
+        launch(few ? gemv_f16_kernel<ENC, kArgmax, false, kShortDepth> : gemv_f16_kernel<ENC, kArgmax, false, kDepth>, 0);
     } else {
-        hipLaunchKernelGGL((gemv_f16_kernel<ENC, kStore, false>), dim3(grid), dim3(kThreads), 0, stream,
-                           image, inverse_scale, tokens, tiles, static_cast<int>(set.input_dim),
-                           candidates, set);
+        launch(few ? gemv_f16_kernel<ENC, kStore, false, kShortDepth> : gemv_f16_kernel<ENC, kStore, false, kDepth>, 0);
     }
     return grid;
 }
@@ -954,15 +980,19 @@ void launch_pair(const ProjectionSet& set, const std::uint8_t* image, const floa
                  int tokens, hipStream_t stream) {
     const std::uint32_t tiles =
         static_cast<std::uint32_t>((set.op[0].output_dim + kTileRows - 1) / kTileRows);
-    if (ring_form<ENC>(set)) {
-        allow_large_lds<gemv_f16_kernel<ENC, kPairs, true>>(Ring<ENC>::kLdsBytes);
-        hipLaunchKernelGGL((gemv_f16_kernel<ENC, kPairs, true>), dim3(grid_of(tiles, false)), dim3(kThreads),
-                           Ring<ENC>::kLdsBytes, stream, image, inverse_scale, tokens, tiles,
-                           static_cast<int>(set.input_dim), static_cast<LmHeadCandidate*>(nullptr), set);
+    const auto launch = [&](auto kernel, unsigned lds) {
+        hipLaunchKernelGGL(kernel, dim3(grid_of(tiles, false)), dim3(kThreads), lds, stream, image, inverse_scale, tokens,
+                           tiles, static_cast<int>(set.input_dim), static_cast<LmHeadCandidate*>(nullptr), set);
+    };
+    const bool few = short_rows(set.input_dim);
+    if (!ring_form<ENC>(set)) {
+        launch(few ? gemv_f16_kernel<ENC, kPairs, false, kShortDepth> : gemv_f16_kernel<ENC, kPairs, false, kDepth>, 0);
+    } else if (few) {
+        allow_large_lds<gemv_f16_kernel<ENC, kPairs, true, kShortDepth>>(Ring<ENC>::kLdsBytes);
+        launch(gemv_f16_kernel<ENC, kPairs, true, kShortDepth>, Ring<ENC>::kLdsBytes);
     } else {
-        hipLaunchKernelGGL((gemv_f16_kernel<ENC, kPairs, false>), dim3(grid_of(tiles, false)), dim3(kThreads),
-                           0, stream, image, inverse_scale, tokens, tiles,
-                           static_cast<int>(set.input_dim), static_cast<LmHeadCandidate*>(nullptr), set);
+        allow_large_lds<gemv_f16_kernel<ENC, kPairs, true, kDepth>>(Ring<ENC>::kLdsBytes);
+        launch(gemv_f16_kernel<ENC, kPairs, true, kDepth>, Ring<ENC>::kLdsBytes);
     }
 }
 

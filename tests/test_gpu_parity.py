@@ -820,6 +820,27 @@ def test_small_batch_half_kernel_many_tiles(cuda, oracle, in_dim):
             assert normalised_error(y.cpu().numpy(), expected) <= TOLERANCE
 
 
+@pytest.mark.parametrize("in_dim", [2048, 3840, 4096, 4352])
+@pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q6_K, kquant.Q8_0])
+def test_small_batch_half_kernel_short_rows(cuda, oracle, encoding, in_dim):
+    """Rows of up to 4,096 columns (two blocks a wave) keep two tiles of weights in flight: one tile a
+    workgroup, three (a group of two and a group of one), shares of one and of two blocks, and the
+    first length past the line.  A tile's rows are the same bits wherever the tile lies."""
+    rows = 9
+    units = torch_().cuda.get_device_properties(0).multi_processor_count
+    packed = random_packed(encoding, 16 * 2 * units + 24, in_dim, 97).reshape(16 * 2 * units + 24, -1)
+    x = kquant.synthetic_activations(98, rows, in_dim)
+    workspace = tile_ops.small_batch_workspace(rows, in_dim)
+    outputs = []
+    for out_dim in (24, 16 * 2 * units + 24):
+        weight = tile_ops.PackedWeight.from_numpy(encoding, packed[:out_dim].reshape(-1), out_dim, in_dim)
+        outputs.append(tile_ops.multi_linear([weight], to_device(x, cuda), workspace)[0].cpu())
+    checked = np.r_[0:24, 16 * units - 8:16 * units + 40, 16 * 2 * units - 16:16 * 2 * units + 24]
+    expected = oracle.linear(encoding, packed[checked].reshape(-1), len(checked), in_dim, x)
+    assert normalised_error(outputs[1].numpy()[:, checked], expected) <= TOLERANCE
+    assert_bits_equal(outputs[0], outputs[1][:, :24].contiguous(), "one tile = its place among many")
+
+
 @pytest.mark.parametrize("in_dim", [4096, 8192, 8448, 16384])
 @pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K])
 def test_decode_dot_kernel_row_lengths(cuda, oracle, encoding, in_dim):
