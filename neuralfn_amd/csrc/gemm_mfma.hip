@@ -50,6 +50,7 @@ namespace nfn {
 
 namespace {
 
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int kBM = 256;
@@ -733,68 +734,93 @@ struct Slices {
 template <std::uint32_t ENC, int RB, int WAVES>
 constexpr bool kWholeBlocks = (ENC == kEncQ4K && RB == 2) || (ENC == kEncQ5K && RB == 1);
 
-// The projections of one launch: one encoding, one input.  Workgroup numbers run through the
-// projections, inside each through its K shares, inside each through its tiles.
+// The projections of one launch: one encoding, one input.
 struct GemmGroup {
     const std::uint8_t* weights[kMaxProjections];
     float* output[kMaxProjections];    // share 0
     float* partials[kMaxProjections];  // the other shares, one copy of the output each
     std::int64_t output_dim[kMaxProjections];
     std::int64_t row_stride;
-    int first[kMaxProjections];   // workgroup number (past the end for slots without a projection)
-    int tiles[kMaxProjections];
     int shares[kMaxProjections];
 };
 
-// this workgroup's projection, share and tile
+// ... as the kernels take them.  Workgroup numbers run through the projections, inside each through its K
+// shares, inside each through its tiles.  Where the projections behind the first begin is among the leading
+// arguments, which lie in registers when a wave starts, so that what a workgroup needs to know of its own is
+// one request to the argument block.  Picked from arrays by branches it was eight, one behind the other, and the
+// first bytes of the weights were asked for 1.2 us after a workgroup's start instead of 0.8.
+struct GemmSlot {
+    const std::uint8_t* weights;
+    float* output;
+    float* partials;
+    std::int64_t output_dim;
+    int first;  // workgroup number
+    int tiles;
+    int shares;
+    std::uint32_t by_tiles, by_shares;  // what `divided` divides by the two with
+    int pad[3];
+};
+static_assert(sizeof(GemmSlot) == 64, "a slot begins at a multiple of 64 bytes");
+struct GemmSlots {
+    GemmSlot slot[kMaxProjections];
+};
+static_assert(kMaxProjections == 4, "three starts among the kernels' leading arguments");
+
+// n / d for n < 2^31 by the host's inverse of d: the product's upper half is the quotient or one less, because
+// the inverse falls short of 2^32 / d by at most one.
+inline std::uint32_t inverse_of(int d) { return 0xffffffffu / static_cast<std::uint32_t>(d); }
+__device__ __forceinline__ int divided(int n, int d, std::uint32_t inverse) {
+    const int quotient = static_cast<int>(__umulhi(static_cast<std::uint32_t>(n), inverse));
+    return n - quotient * d >= d ? quotient + 1 : quotient;
+}
+
+// this workgroup's projection, share and tile, and the blocks of 256 columns that its share has
 struct GroupPlace {
     const std::uint8_t* weights;
     float *output, *partials;
     std::int64_t output_dim;
-    int share, shares, tile;
+    int share, tile, first_block, end_block;
 };
 // (a macro: a reference to a kernel's argument makes the compiler copy it to scratch memory)
-#define NFN_PLACE(place, group)                                              \
-    GroupPlace place;                                                        \
-    place.weights = group.weights[0];                                        \
-    place.output = group.output[0];                                          \
-    place.partials = group.partials[0];                                      \
-    place.output_dim = group.output_dim[0];                                  \
-    place.shares = group.shares[0];                                          \
-    {                                                                        \
-        int first = 0, tiles = group.tiles[0];                               \
-        _Pragma("unroll") for (int i = 1; i < kMaxProjections; ++i) {        \
-            if (static_cast<int>(blockIdx.x) >= group.first[i]) {            \
-                place.weights = group.weights[i];                            \
-                place.output = group.output[i];                              \
-                place.partials = group.partials[i];                          \
-                place.output_dim = group.output_dim[i];                      \
-                place.shares = group.shares[i];                              \
-                first = group.first[i];                                      \
-                tiles = group.tiles[i];                                      \
-            }                                                                \
-        }                                                                    \
-        place.share = (static_cast<int>(blockIdx.x) - first) / tiles;        \
-        place.tile = (static_cast<int>(blockIdx.x) - first) % tiles;         \
+#define NFN_PLACE(place, slots)                                                                             \
+    GroupPlace place;                                                                                       \
+    {                                                                                                       \
+        const int number = static_cast<int>(blockIdx.x);                                                    \
+        int index = number >= first1 ? 1 : 0;                                                               \
+        index = number >= first2 ? 2 : index;                                                               \
+        index = number >= first3 ? 3 : index;                                                               \
+        const GemmSlot& mine = slots.slot[index];                                                           \
+        place.weights = mine.weights;                                                                       \
+        place.output = mine.output;                                                                         \
+        place.partials = mine.partials;                                                                     \
+        asm volatile("" : "+s"(place.partials)); /* (requested with the others, in every share) */          \
+        place.output_dim = mine.output_dim;                                                                 \
+        const int tiles = mine.tiles, shares = mine.shares, whole = number - mine.first;                    \
+        const std::uint32_t by_shares = mine.by_shares;                                                     \
+        place.share = divided(whole, tiles, mine.by_tiles);                                                 \
+        place.tile = whole - place.share * tiles;                                                           \
+        place.first_block = divided(total_blocks * place.share, shares, by_shares);                         \
+        place.end_block = divided(total_blocks * (place.share + 1), shares, by_shares);                     \
     }
 
 // RB: 32-row blocks per wave; the workgroup's tile is 32 * RB * WAVES rows by 128 columns.
 template <std::uint32_t ENC, int RB, int WAVES>
 __global__ __launch_bounds__(WAVES * kWave)
 __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB, WAVES>, kWavesPerSimd<ENC, RB, WAVES>))) void gemm_f16_kernel(
-    const std::uint8_t* __restrict__ activations, const float* __restrict__ inverse_scale, std::int64_t input_dim,
-    std::int64_t rows, int m_tiles, GemmGroup group) {
+    const std::uint8_t* __restrict__ activations, const float* __restrict__ inverse_scale, std::int64_t row_stride,
+    std::int64_t rows, int total_blocks, int m_tiles, std::uint32_t by_m_tiles, int first1, int first2, int first3,
+    GemmSlots slots) {
     extern __shared__ __attribute__((aligned(16))) std::uint8_t lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // rows 64*wave .. +63 of the tile
-    NFN_PLACE(place, group)
+    NFN_PLACE(place, slots)
     const std::uint8_t* weights = place.weights;
     float* output = place.output;
     const std::int64_t output_dim = place.output_dim;
-    const int share = place.share, shares = place.shares;
-    const int m_tile = place.tile % m_tiles;
-    const int n_tile = place.tile / m_tiles;
+    const int share = place.share;
+    const int n_tile = divided(place.tile, m_tiles, by_m_tiles);
+    const int m_tile = place.tile - n_tile * m_tiles;
     using Slice = typename Held<ENC, WAVES>::Slice;
     using Header = typename Held<ENC, WAVES>::Header;
     constexpr int kTileRows = 32 * RB * WAVES;
@@ -802,16 +828,13 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB, WAVES>, kWavesPerSimd<
     const std::int64_t n0 = static_cast<std::int64_t>(n_tile) * kBN;
     // which share of the K dimension (whole 256-value blocks) this workgroup sums; each share
     // writes its own copy of the output
-    const int total_blocks = static_cast<int>(input_dim >> 8);
-    const int first_block = total_blocks * share / shares;
-    const int end_block = total_blocks * (share + 1) / shares;
-    const int steps = (end_block - first_block) * 4;  // a positive multiple of 4
+    const int first_block = place.first_block;
+    const int steps = (place.end_block - first_block) * 4;  // a positive multiple of 4
     const int last = steps - 1;
-    const std::int64_t row_stride = group.row_stride;
     if (share > 0) output = place.partials + (share - 1) * rows * output_dim;
 
     // activations: fragment (row block, K chunk) is 1 KB, a row block's chunks are consecutive
-    const std::int64_t row_block_bytes = (input_dim / 16) * kFragmentBytes;
+    const std::int64_t row_block_bytes = static_cast<std::int64_t>(total_blocks) * 16 * kFragmentBytes;
     // (a tile of 512 rows can reach past the rows the copy is padded to: its last waves take blocks
     // that are there and store nothing)
     int row_block = static_cast<int>(m0 / 32) + wave * RB;
@@ -966,32 +989,52 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB, WAVES>, kWavesPerSimd<
         block += 2;
     }
 
-    // D register r of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32
-    const int column = lane & 31;
-    const int row_base = (lane >> 5) * 4;
-    const bool whole = m0 + kTileRows <= rows && n0 + kBN <= output_dim;
+    // D register r of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32.  A store of it as it lies is 128 bytes of
+    // two rows; a wave turns it in its part of the stages into whole rows of the tile and stores 512 bytes of each at
+    // once (256 where the output's rows do not begin at 16 bytes).  Workgroups that start together end together, and
+    // what they then have to write is megabytes: 1,316 rows of 2,048 -> 7,680 (Q5_K), 40 MB, spent 10 to 15 of 62 us
+    // here with the stores as the results lie, and now take 58; 1,148 rows of 2,048 -> 4,864 (Q8_0) 46.0 -> 40.7, 250
+    // rows of 3,328 into Q, K, V and gate (Q4_K) 42.8 -> 36.9, 36 rows of 2,048 -> 6,144 (Q6_K) 31.4 -> 28.0; a launch
+    // of one long round (2,048 rows of 16,384 -> 6,656, 433) gains nothing.
+    const int end_lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));  // (no register held for it)
+    const int column = end_lane & 31;
+    const int half = end_lane >> 5;
+    constexpr int kPitch = kBN + 8;               // floats: rows that lie four apart begin in different banks
+    constexpr int kTurned = WAVES == 8 ? 8 : 16;  // rows at a time
+    static_assert(kTurned * kPitch * 4 * WAVES <= 2 * kStageBytes, "the waves' parts fit the stages");
+    const bool wide = output_dim % 4 == 0 && reinterpret_cast<std::uintptr_t>(output) % 16 == 0;
+    __syncthreads();
+    float* const turned = reinterpret_cast<float*>(lds) + wave * (kTurned * kPitch);
 #pragma unroll
     for (int i = 0; i < RB; ++i) {
-        const std::int64_t tile_row = m0 + wave * (32 * RB) + i * 32 + row_base;
-        float inverse[16];
+        const std::int64_t first_row = m0 + wave * (32 * RB) + i * 32;
+        const float* const scales = inverse_scale + (WAVES == 8 ? row_block * 32 + i * 32 : first_row) + 4 * half;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) inverse[r] = inverse_scale[(WAVES == 8 ? row_block * 32 + i * 32 + row_base : tile_row) + 8 * (r >> 2) + (r & 3)];
+        for (int part = 0; part < 32 / kTurned; ++part) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const std::int64_t n = n0 + j * 32 + column;
-            float* target = output + tile_row * output_dim + n;
-            if (whole) {
+            for (int r = part * kTurned / 2; r < (part + 1) * kTurned / 2; ++r) {
+                const float inverse = scales[8 * (r >> 2) + (r & 3)];
+                const int row = 4 * half + 8 * (r >> 2) + (r & 3) - part * kTurned;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    target[(8 * (r >> 2) + (r & 3)) * output_dim] = acc[i][j][r] * inverse[r];
+                for (int j = 0; j < 4; ++j) turned[row * kPitch + j * 32 + column] = acc[i][j][r] * inverse;
+            }
+            const std::int64_t m = first_row + part * kTurned;
+            if (wide) {
+                const std::int64_t n = n0 + 4 * column;
+#pragma unroll
+                for (int t = 0; t < kTurned; t += 2) {
+                    const v4f four = *reinterpret_cast<const v4f*>(turned + (t + half) * kPitch + 4 * column);
+                    if (m + t + half < rows && n < output_dim) {
+                        *reinterpret_cast<v4f*>(output + (m + t + half) * output_dim + n) = four;
+                    }
                 }
             } else {
+                const std::int64_t n = n0 + end_lane;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const std::int64_t m = tile_row + 8 * (r >> 2) + (r & 3);
-                    if (m < rows && n < output_dim) {
-                        output[m * output_dim + n] = acc[i][j][r] * inverse[r];
-                    }
+                for (int t = 0; t < kTurned; ++t) {
+                    const float first = turned[t * kPitch + end_lane], second = turned[t * kPitch + end_lane + 64];
+                    if (m + t < rows && n < output_dim) output[(m + t) * output_dim + n] = first;
+                    if (m + t < rows && n + 64 < output_dim) output[(m + t) * output_dim + n + 64] = second;
                 }
             }
         }
@@ -1071,18 +1114,16 @@ struct LowBlock {
 
 template <std::uint32_t ENC>
 __global__ __launch_bounds__(kThreads, 2) void gemm_f16_low_kernel(
-    const std::uint8_t* __restrict__ activations, const float* __restrict__ inverse_scale, std::int64_t input_dim,
-    std::int64_t rows, GemmGroup group) {
+    const std::uint8_t* __restrict__ activations, const float* __restrict__ inverse_scale, std::int64_t row_stride,
+    std::int64_t rows, int total_blocks, int first1, int first2, int first3, GemmSlots slots) {
     extern __shared__ __attribute__((aligned(16))) std::uint8_t lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-    NFN_PLACE(place, group)
+    NFN_PLACE(place, slots)
     const std::int64_t output_dim = place.output_dim;
     const std::int64_t n0 = static_cast<std::int64_t>(place.tile) * kBN + 32 * wave;
-    const int total_blocks = static_cast<int>(input_dim >> 8);
-    const int first_block = total_blocks * place.share / place.shares;
-    const int end_block = total_blocks * (place.share + 1) / place.shares;
-    const int steps = (end_block - first_block) * 4;
+    const int first_block = place.first_block;
+    const int steps = (place.end_block - first_block) * 4;
     const int last = steps - 1;
     const int last_block = (steps >> 2) - 1;
     float* const output = place.share > 0 ? place.partials + (place.share - 1) * rows * output_dim : place.output;
@@ -1099,8 +1140,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f16_low_kernel(
     const int b_row = kParts<ENC> == 4 ? b_turn : (b_turn & ~6) | ((b_turn & 2) << 1) | ((b_turn & 4) >> 1);
     const std::int64_t b_skip = static_cast<std::int64_t>(first_block) * kBlockBytes<ENC>;
     WeightRows b_global;
-    b_global.first = place.weights + min(n0 + b_row, output_dim - 1) * group.row_stride + b_skip;
-    b_global.second = place.weights + min(n0 + b_row + 16, output_dim - 1) * group.row_stride + b_skip;
+    b_global.first = place.weights + min(n0 + b_row, output_dim - 1) * row_stride + b_skip;
+    b_global.second = place.weights + min(n0 + b_row + 16, output_dim - 1) * row_stride + b_skip;
 
     v16f acc;
 #pragma unroll
@@ -1281,22 +1322,28 @@ Plan plan(std::uint32_t encoding, std::int64_t rows, std::int64_t output_dim, st
 }
 
 template <std::uint32_t ENC, int RB, int WAVES>
-void launch_tiles(GemmGroup group, int count, const std::uint8_t* activations, const float* inverse_scale,
+void launch_tiles(const GemmGroup& group, int count, const std::uint8_t* activations, const float* inverse_scale,
                   std::int64_t rows, std::int64_t input_dim, hipStream_t stream) {
     const int m_tiles = static_cast<int>((rows + 32 * RB * WAVES - 1) / (32 * RB * WAVES));
-    int workgroups = 0;
+    GemmSlots slots{};
+    int workgroups = 0, first[kMaxProjections];
     for (int i = 0; i < kMaxProjections; ++i) {
-        group.first[i] = i < count ? workgroups : 0x7fffffff;
+        first[i] = i < count ? workgroups : 0x7fffffff;
         if (i >= count) continue;
-        group.tiles[i] = m_tiles * static_cast<int>((group.output_dim[i] + kBN - 1) / kBN);
-        workgroups += group.tiles[i] * group.shares[i];
+        const int tiles = m_tiles * static_cast<int>((group.output_dim[i] + kBN - 1) / kBN);
+        slots.slot[i] = GemmSlot{group.weights[i], group.output[i], group.partials[i], group.output_dim[i],
+                                 workgroups, tiles, group.shares[i], inverse_of(tiles), inverse_of(group.shares[i]), {}};
+        workgroups += tiles * group.shares[i];
     }
+    const int blocks = static_cast<int>(input_dim >> 8);
     if (rows > kLowRows) {
         hipLaunchKernelGGL((gemm_f16_kernel<ENC, RB, WAVES>), dim3(static_cast<unsigned>(workgroups)), dim3(WAVES * kWave),
-                           2 * kStageBytes, stream, activations, inverse_scale, input_dim, rows, m_tiles, group);
+                           2 * kStageBytes, stream, activations, inverse_scale, group.row_stride, rows, blocks, m_tiles,
+                           inverse_of(m_tiles), first[1], first[2], first[3], slots);
     } else {
         hipLaunchKernelGGL(gemm_f16_low_kernel<ENC>, dim3(static_cast<unsigned>(workgroups)), dim3(kThreads),
-                           2 * kStageBytes, stream, activations, inverse_scale, input_dim, rows, group);
+                           2 * kStageBytes, stream, activations, inverse_scale, group.row_stride, rows, blocks, first[1],
+                           first[2], first[3], slots);
     }
 }
 
