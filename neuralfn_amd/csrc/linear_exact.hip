@@ -29,8 +29,8 @@
 // eight lanes a row instead, eight rows an instruction, and so loads and cuts only the rows that are there (by
 // eights: 8, 16 or 32), which every tile of weight rows does again: 4,096 -> 6,656 at 5 / 16 / 25 / 64 rows Q4_K
 // 15.2 / 17.4 / 19.6 / 28.7 -> 12.2 / 15.1 / 18.1 / 28.4 us, Q5_K 16.8 / 19.7 / 22.2 / 34.0 -> 13.7 / 16.3 /
-// 20.0 / 30.8, Q6_K 21.8 / 24.1 / 27.6 / 46.6 -> 20.5 / 21.5 / 25.6 / 42.0, Q8_0 24.2 / 28.2 / 31.0 / 45.9 ->
-// 21.6 / 22.8 / 25.6 / 38.3, bf16 20.4 / 23.9 / 27.1 / 38.4 -> 18.1 / 21.1 / 23.2 / 31.5, F32 32.4 / 33.5 / 35.7 /
+// 20.0 / 30.8, Q6_K 21.8 / 24.1 / 27.6 / 46.6 -> 15.4 / 18 / 20 / 35.9, Q8_0 24.2 / 28.2 / 31.0 / 45.9 ->
+// 12.9 / 15 / 16.5 / 26.2, bf16 20.4 / 23.9 / 27.1 / 38.4 -> 18.1 / 21.1 / 23.2 / 31.5, F32 32.4 / 33.5 / 35.7 /
 // 55.9 -> 28.4 / 31.2 / 33.1 / 51.6, at 200 rows 135 -> 114.  (Its buffer loads of activations as global ones take
 // registers that Q5_K does not have: 25 rows 20.0 -> 24.3.  Weights requested behind the next step's activations:
 // Q8_0 2 % faster, F32 of 64 rows 46.6 -> 55.0.)  What is left is the cut and the decode (16 waves'
@@ -48,7 +48,7 @@
 // once instead of tile by tile: no difference.  Requests two steps ahead instead of one, and the matrix
 // instructions of a step before its other work instead of between it: neither.)  The 64 x 128 form of Q6_K
 // keeps six registers that do not change in its loop in scratch (28 bytes a lane), read outside of it; the
-// 32 x 32 form of Q6_K for 17 rows and more five (32 bytes); the others none.
+// others none.
 // Measured at 4,096 -> 6,656, against the vector kernel (16 rows) and the float matrix instruction (200,
 // 512 rows) before: Q4_K 134 -> 15 us at 16 rows, 203 -> 62 at 200, 311 -> 121 at 512; Q8_0 368 -> 23,
 // 180 -> 55, 279 -> 108; F32 406 -> 31, 172 -> 114, 271 -> 217.
@@ -154,8 +154,13 @@ __device__ __forceinline__ void signed_codes_to_bf16(std::uint32_t bytes, std::u
 // Every load looks up a cache line for each of its lanes, however few bytes it brings, and those
 // look-ups bound the kernels: the two lanes of a row (half 0 and 1, 32 lanes apart) therefore
 // fetch different pieces, 16 bytes wherever a piece has them, and trade words in arrange().  Q6_K
-// takes four loads a unit instead of nine, Q8_0 three instead of four: 4,096 -> 6,656 at 16 / 200 /
-// 512 rows 24.2 / 112 / 223 -> 21.6 / 107 / 211 us for Q6_K, 28.9 / 92 / 179 -> 26.8 / 87 / 169 for Q8_0.
+// takes five loads a unit instead of nine, Q8_0 three instead of four.
+// Sixteen bytes that start two past a word keep the address unit four times as long as sixteen that start at one (a
+// wave's load of 32 rows 55 ns a compute unit, aligned 15; of two words twice, of one word or less as long as ever),
+// and half of Q6_K's and of Q8_0's pieces do.  The small form asks for the words that hold a piece and moves them
+// up by two bytes: 4,096 / 6,400 -> 1,700 of Q6_K, 4 rows 17.0 / 39.1 -> 13.4 / 21.8 us, 32 rows 22.4 / 46.1 -> 18.9 /
+// 30.5; of Q8_0 17.4 / 20.2 -> 10.6 / 14.3 and 21.9 / 27.6 -> 15.7 / 22.4; 64 rows -> 6,656 of Q6_K 40.8 / 76.6 ->
+// 35.9 / 53.9.  (Q6_K rows of an odd number of blocks begin past a word by turns, so that every load was a slow one.)
 // -----------------------------------------------------------------------------------------------
 // first: the lower 32 lanes' `a` and `b` (in the lower and the upper lanes), second: the upper lanes'
 struct Traded {
@@ -224,21 +229,42 @@ struct Unit<kEncQ5K> : UnitOfQ4KOrQ5K<kEncQ5K> {};
 template <>
 struct Unit<kEncQ6K> {
     static constexpr bool kWide = false, kScaled = true, kMinimum = false, kScalePerChunk = true;
-    // as loaded: the 16 columns of chunk `half`; arranged: words 0 and 1 the lane's columns of
-    // chunk 0, words 2 and 3 those of chunk 1
-    u32x4_a2 low[2], high;  // low: [step]
+    // as loaded: the 16 columns of chunk `half`, from the word at or before the first (every other block of a row
+    // starts two bytes past a word); aligned: the columns; arranged: words 0 and 1 the lane's columns of chunk 0, words 2 and 3 those of chunk 1
+    u32x4_a4 low[2], high;  // low: [step]
+    std::uint32_t beyond;   // the word behind the lower bits (half 0), the upper ones (half 1)
     std::uint32_t scales;   // the unit's four sub-scales, (step, chunk) at byte 2 step + chunk
     std::uint32_t d;        // in the upper half
     int upper;
+    __device__ __forceinline__ static std::uint32_t past_word(const std::uint8_t* row, int unit) {
+        return (static_cast<std::uint32_t>(reinterpret_cast<std::uintptr_t>(row)) + 2u * (unit >> 2)) & 2u;
+    }
     __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half) {
         typedef std::uint32_t u32_a2 __attribute__((aligned(2)));
         const std::uint8_t* block = row + (unit >> 2) * 210;
         const int half_block = (unit >> 1) & 1;
         upper = unit & 1;  // quarters 2 and 3 of the half block: high nibbles, high-bit pairs 2 and 3
-        low[0] = *reinterpret_cast<const u32x4_a2*>(block + half_block * 64 + 16 * half);
-        low[1] = *reinterpret_cast<const u32x4_a2*>(block + half_block * 64 + 32 + 16 * half);
-        high = *reinterpret_cast<const u32x4_a2*>(block + 128 + half_block * 32 + 16 * half);
+        const std::uint8_t* word = block - past_word(row, unit);
+        low[0] = *reinterpret_cast<const u32x4_a4*>(word + half_block * 64 + 16 * half);
+        low[1] = *reinterpret_cast<const u32x4_a4*>(word + half_block * 64 + 32 + 16 * half);
+        high = *reinterpret_cast<const u32x4_a4*>(word + 128 + half_block * 32 + 16 * half);
+        beyond = *reinterpret_cast<const std::uint32_t*>(word + (half != 0 ? 160 + 32 * half_block : 64 + 64 * half_block));
         scales = *reinterpret_cast<const u32_a2*>(block + (half != 0 ? 192 + 4 * (unit & 3) : 206));
+    }
+    __device__ __forceinline__ void align(const std::uint8_t* row, int unit) {
+        const std::uint32_t shift = past_word(row, unit);
+        if (__ballot(shift != 0) == 0) return;
+        // each piece's following word lies in the other lane of the row or, behind the last, in `beyond`
+        const bool second = (threadIdx.x & 32) != 0;
+        const Traded a = trade(low[0][0], low[1][0]), b = trade(low[1][0], beyond), c = trade(high[0], high[0]);
+        const std::uint32_t behind[3] = {second ? a.first : a.second, second ? b.first : b.second,
+                                         second ? beyond : c.second};
+#pragma unroll
+        for (int word = 0; word < 4; ++word) {
+            low[0][word] = __builtin_amdgcn_alignbyte(word < 3 ? low[0][word + 1] : behind[0], low[0][word], shift);
+            low[1][word] = __builtin_amdgcn_alignbyte(word < 3 ? low[1][word + 1] : behind[1], low[1][word], shift);
+            high[word] = __builtin_amdgcn_alignbyte(word < 3 ? high[word + 1] : behind[2], high[word], shift);
+        }
     }
     __device__ __forceinline__ void arrange() {
 #pragma unroll
@@ -273,7 +299,31 @@ template <>
 struct Unit<kEncQ8_0> {
     static constexpr bool kWide = true, kScaled = true, kMinimum = false, kScalePerChunk = false;
     u32x4_a2 codes[2];
-    std::uint32_t d[2];  // as loaded: [0] the scale of block `half`
+    std::uint32_t d[2];  // as loaded: [0] the scale of block `half`; of a pair: [0] the word behind it
+    // Rows of whole units: a pair of blocks is 68 bytes, whole words where the tensor begins at one.
+    __device__ __forceinline__ void load_pair(const std::uint8_t* row, int unit, int half) {
+        const std::uint8_t* pair = row + 68 * unit;
+        codes[0] = *reinterpret_cast<const u32x4_a2*>(pair + 16 * half);
+        codes[1] = *reinterpret_cast<const u32x4_a2*>(pair + 32 + 16 * half);
+        typedef std::uint32_t u32_a2 __attribute__((aligned(2)));
+        d[0] = *reinterpret_cast<const u32_a2*>(pair + 64);
+    }
+    // The lane has words 4 half .. 4 half + 3 and 8 + 4 half .. 11 + 4 half of the pair's seventeen.  The first
+    // block's codes begin in the middle of word 0, the second one's are words 9 to 16, behind its scale.
+    __device__ __forceinline__ void arrange_pair() {
+        const bool second = (threadIdx.x & 32) != 0;
+        const Traded a = trade(codes[0][0], codes[1][0]), b = trade(codes[1][0], codes[1][0]);
+        const std::uint32_t behind0 = second ? a.first : a.second, behind1 = second ? d[0] : b.second;
+        const std::uint32_t scales = (codes[0][0] & 0xffffu) | (codes[1][0] & 0xffff0000u);  // (of the lower lanes)
+        const Traded t = trade(scales, scales);
+        d[0] = t.first & 0xffffu;
+        d[1] = t.first >> 16;
+#pragma unroll
+        for (int word = 0; word < 4; ++word) {
+            codes[0][word] = __builtin_amdgcn_alignbyte(word < 3 ? codes[0][word + 1] : behind0, codes[0][word], 2);
+            codes[1][word] = word < 3 ? codes[1][word + 1] : behind1;
+        }
+    }
     // (`steps`: the row's 32-column blocks; a row of an odd number of them reads its last one twice)
     __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half, int steps) {
 #pragma unroll
@@ -633,7 +683,8 @@ constexpr int kSmallLds = WAVES * (kOwnTerms<MT> + 4 * 32 * MT * 4);
 // WAVES waves share a tile of 32 MT input rows x 32 NT weight rows, of which the first 8 ITEMS of each
 // 32 exist (the products of the others are not stored).  ITEMS = 0: each lane loads and cuts what it
 // multiplies, which spares a short walk over K the way through LDS.
-template <std::uint32_t ENC, int MT, int NT, int WAVES, int ITEMS>
+// PAIRS: Q8_0 rows of whole units.
+template <std::uint32_t ENC, int MT, int NT, int WAVES, int ITEMS, bool PAIRS>
 __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exact_small_kernel(
     const std::uint8_t* __restrict__ data, std::int64_t row_stride, const float* __restrict__ input,
     const float* __restrict__ bias, float* __restrict__ output, std::int64_t rows, std::int64_t input_dim,
@@ -663,18 +714,24 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
     // Cutter: quad lane % 8 of the rows 8 item + lane / 8; a load instruction reads whole lines.
     float* const sums = reinterpret_cast<float*>(lds + WAVES * kOwnTerms<MT>) + wave * 4 * 32 * MT;  // [step % 4][row]
     const int quad = lane & 7;
+    // Rows past the end: the last one again.  Q6_K has no registers for every item's place (five ended up in
+    // scratch): there they lie past the buffer's end, and a load has zeros for them from nowhere.
+    constexpr bool kSpare = ENC == kEncQ6K;
+    const std::int64_t tile_rows = min(rows - row0, std::int64_t(32 * MT));
     const __amdgpu_buffer_rsrc_t x_tile = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(input + row0 * input_dim), 0, 0xffffffff, 0x00020000);
+        const_cast<float*>(input + row0 * input_dim), 0, kSpare ? static_cast<int>(tile_rows * input_dim * 4) : -1, 0x00020000);
     // (ITEMS = 0: columns 16 half + 8 chunk (kWide), 8 half + 16 chunk of row `inner`)
     const float* const x_row = input + min(row0 + inner, rows - 1) * input_dim + (Slice::kWide ? 16 : 8) * half;
-    const int last_row = static_cast<int>(min(rows - 1 - row0, std::int64_t(32 * MT)));
+    const int last_row = static_cast<int>(tile_rows - 1);
     constexpr int kLoads = ITEMS == 0 ? 4 : ITEMS;
-    std::uint32_t x_from[MT][kLoads];
+    const std::uint32_t eight_rows = 32 * static_cast<std::uint32_t>(input_dim);
+    std::uint32_t x_from[kSpare ? 1 : MT][kSpare ? 1 : kLoads];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
+    for (int m = 0; m < (kSpare ? 1 : MT); ++m) {
 #pragma unroll
-        for (int item = 0; item < kLoads; ++item) {
-            x_from[m][item] = 4 * (static_cast<std::uint32_t>(min(32 * m + 8 * item + (lane >> 3), last_row)) *
+        for (int item = 0; item < (kSpare ? 1 : kLoads); ++item) {
+            const int row = 32 * m + 8 * item + (lane >> 3);
+            x_from[m][item] = 4 * (static_cast<std::uint32_t>(kSpare ? row : min(row, last_row)) *
                                        static_cast<std::uint32_t>(input_dim) + 4 * quad);
         }
     }
@@ -690,7 +747,10 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
                         x_row + static_cast<std::int64_t>(min(step, last_step)) * 32 + kNext * (item >> 1) + 4 * (item & 1));
                 } else {
                     x[m][item] = __builtin_bit_cast(f32x4_a4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                                  x_tile, x_from[m][item], min(step, last_step) * 128, 0));
+                                                                  x_tile,
+                                                                  kSpare ? x_from[0][0] + (4 * m + item) * eight_rows
+                                                                         : x_from[kSpare ? 0 : m][kSpare ? 0 : item],
+                                                                  min(step, last_step) * 128, 0));
                 }
             }
         }
@@ -731,8 +791,15 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
         // (2 x 2 tiles leave no registers for a second unit of float weights: a step's, as they are used up)
         constexpr bool kAhead = MT * NT < 4;
         Slice now[NT], next[NT];
+        const auto load_weights = [&](Slice& into, const std::uint8_t* row, int unit) {
+            if constexpr (PAIRS) {
+                into.load_pair(row, unit, half);
+            } else {
+                load_unit<ENC>(into, row, unit, half, steps);
+            }
+        };
 #pragma unroll
-        for (int n = 0; n < NT; ++n) load_unit<ENC>(now[n], w_row[n], first_unit, half, steps);
+        for (int n = 0; n < NT; ++n) load_weights(now[n], w_row[n], first_unit);
         load_inputs(2 * first_unit);
         if constexpr (ITEMS > 0) {
             cut_inputs(2 * first_unit);
@@ -740,10 +807,17 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
         }
         for (int unit = first_unit; unit < end_unit; ++unit) {
 #pragma unroll
-            for (int n = 0; n < NT; ++n) now[n].arrange();
+            for (int n = 0; n < NT; ++n) {
+                if constexpr (ENC == kEncQ6K) now[n].align(w_row[n], unit);
+                if constexpr (PAIRS) {
+                    now[n].arrange_pair();
+                } else {
+                    now[n].arrange();
+                }
+            }
             if constexpr (kAhead) {
 #pragma unroll
-                for (int n = 0; n < NT; ++n) load_unit<ENC>(next[n], w_row[n], min(unit + 1, end_unit - 1), half, steps);
+                for (int n = 0; n < NT; ++n) load_weights(next[n], w_row[n], min(unit + 1, end_unit - 1));
             }
             float partial[2];  // (ITEMS == 0: the lane's half of its row's sums)
 #pragma unroll
@@ -1281,23 +1355,31 @@ void launch_small_form(const Descriptor& weight, const float* input, const float
     const std::int64_t column_tiles = (weight.output_dim + 32 * NT - 1) / (32 * NT);
     constexpr int kLds = ITEMS == 0 ? WAVES * 16 * kWave * 4 : kSmallLds<MT, NT, WAVES>;
     static_assert(kLds >= WAVES * 16 * kWave * 4, "the waves' sums meet in the same memory");
-    allow_large_lds<linear_exact_small_kernel<ENC, MT, NT, WAVES, ITEMS>>();
-    hipLaunchKernelGGL((linear_exact_small_kernel<ENC, MT, NT, WAVES, ITEMS>),
-                       dim3(static_cast<unsigned>(row_tiles * column_tiles)), dim3(WAVES * kWave), kLds, stream,
-                       weight.data, weight.row_stride_bytes, input, bias, output, rows, weight.input_dim,
-                       weight.output_dim, static_cast<int>(row_tiles));
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(row_tiles * column_tiles)), dim3(WAVES * kWave), kLds, stream,
+                           weight.data, weight.row_stride_bytes, input, bias, output, rows, weight.input_dim,
+                           weight.output_dim, static_cast<int>(row_tiles));
+    };
+    if constexpr (ENC == kEncQ8_0) {
+        if (weight.input_dim % 64 == 0) {
+            allow_large_lds<linear_exact_small_kernel<ENC, MT, NT, WAVES, ITEMS, true>>();
+            return launch(linear_exact_small_kernel<ENC, MT, NT, WAVES, ITEMS, true>);
+        }
+    }
+    allow_large_lds<linear_exact_small_kernel<ENC, MT, NT, WAVES, ITEMS, false>>();
+    launch(linear_exact_small_kernel<ENC, MT, NT, WAVES, ITEMS, false>);
 }
 
 template <std::uint32_t ENC, int MT, int NT, int WAVES>
 void launch_small(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
                   hipStream_t stream) {
     if constexpr (WAVES == 16 && kWholeBlocks<ENC>) {
-        // Walks of two or three units a wave, through LDS and not: 25 rows of Q6_K 2,048 -> 300 13.2 and 11.0 us,
-        // 3,328 -> 8,000 27.0 and 26.4, 4,096 -> 6,656 25.6 and 27.5; 16 rows 10.9 and 10.3, 15.0 and 16.2 (3,072 ->
-        // 2,000), 21.5 and 24.2; 25 rows of Q4_K 2,560 -> 8,000 14.3 and 13.7, 3,072 -> 2,000 12.9 and 13.4, and
-        // 2,048 -> 300 9.1 and 10.3.
+        // Walks of up to three units a wave, through LDS and not: 16 rows of Q6_K 512 -> 300 5.8 and 5.5 us, 768 -> 300
+        // 6.1 and 6.4, 17 rows 2,048 -> 1,700 10.9 and 10.0, 32 rows 1,024 -> 300 7.5 and 7.2, 1,280 -> 1,700 10.5 and
+        // 11.5; 25 rows of Q4_K 2,560 -> 8,000 14.3 and 13.7, 3,072 -> 2,000 12.9 and 13.4, and 2,048 -> 300 9.1 and 10.3.
         const bool wide = (weight.output_dim + 31) / 32 * 3 > compute_units();
-        if (ENC == kEncQ6K ? weight.input_dim <= (rows > 16 ? 3328 : 2048) : rows > 16 && weight.input_dim <= 2560 && wide) {
+        const std::int64_t q6_columns = rows > 20 ? 1024 : rows > 16 ? 2048 : 512;
+        if (ENC == kEncQ6K ? weight.input_dim <= q6_columns : rows > 16 && weight.input_dim <= 2560 && wide) {
             return launch_small_form<ENC, MT, NT, WAVES, 0>(weight, input, bias, output, rows, stream);
         }
     }

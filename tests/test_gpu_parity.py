@@ -1371,6 +1371,25 @@ def test_exact_linear_on_tensors_off_a_word(cuda, encoding, rows, out_dim, in_di
     assert_bits_equal(tile_ops.linear(shifted, shifted_floats(x, cuda), shifted_floats(bias, cuda)), expected)
 
 
+@pytest.mark.parametrize("rows", [1, 3, 4, 16, 17, 21, 40])
+@pytest.mark.parametrize("in_dim", [256, 512, 768, 1280, 2304])
+@pytest.mark.parametrize("encoding", [kquant.Q6_K, kquant.Q8_0])
+def test_exact_linear_of_blocks_past_a_word(cuda, oracle, encoding, in_dim, rows):
+    """Blocks that start two bytes past a word are read from the word before them: rows of odd and even
+    numbers of blocks, tensors that start at a word and two bytes past it, the first and the last block of
+    a tensor.  Bound as for the forms' edges above."""
+    out_dim = 35 if rows < 40 else 5000  # (32 x 64 tiles)
+    packed = random_packed(encoding, out_dim, in_dim, 64)
+    x = kquant.synthetic_activations(65, rows, in_dim)
+    aligned = tile_ops.PackedWeight.from_numpy(encoding, packed, out_dim, in_dim)
+    shifted = tile_ops.PackedWeight(encoding, out_dim, in_dim, shifted_copy(packed, 2, cuda))
+    y = tile_ops.linear(aligned, to_device(x, cuda))
+    assert_bits_equal(tile_ops.linear(shifted, to_device(x, cuda)), y)
+    checked = np.r_[0:35] if out_dim == 35 else np.r_[0:33, 4960:5000]
+    expected = oracle.linear(encoding, packed.reshape(out_dim, -1)[checked].reshape(-1), len(checked), in_dim, x)
+    assert normalised_error(y.cpu().numpy()[:, checked], expected) <= 1e-5
+
+
 @pytest.mark.parametrize("encoding", ALL_PACKED)
 def test_lm_head_one_row_on_tensors_off_a_word(cuda, encoding):
     out_dim, in_dim = 4099, 1280
