@@ -73,6 +73,9 @@ struct __attribute__((packed, aligned(2))) Chunk16 {
 struct __attribute__((packed, aligned(2))) Chunk8 {
     std::uint32_t v[2];
 };
+struct __attribute__((packed, aligned(2))) Chunk4 {
+    std::uint32_t v;
+};
 
 // ---------------------------------------------------------------------------
 // activations: fp32 -> row-scaled fp16 in operand order, whole 256-row tiles
@@ -354,6 +357,57 @@ template <>
 struct PackedSlice<kEncQ8_0> {
     // a K step of 64 is two 34-byte blocks; `pair` counts K steps inside 256 values
     u32x4 codes_a, codes_b;
+    std::uint32_t behind_a, behind_b;
+    f16x2 scale_a, scale_b;
+    // The two are seventeen words: the first one's codes start in the middle of word 0, the second one's
+    // scale is the upper half of word 8.  Four lanes take words 0..3, 4..7, 9..12 and 13..16, and word 4
+    // or 8 beside them: from where the first one's codes begin, two bytes past a word, sixteen bytes take the
+    // address unit four times as long.  Loaded as they lie -> from words, us: 17 rows of 6,656 into Q, K, V and gate 39.7 ->
+    // 33.7, 32 of gate and up 4,096 -> 11,264 64.5 -> 57.8, 100 of Q, K, V and gate 47.4 -> 42.7, 333 of down 11,264 ->
+    // 5,632 103 -> 93, 1,400 of it 282 -> 254.  (Q6_K's pieces, of which half begin past a word, the same way: three to
+    // eight more instructions a piece for as many loads, 17 to 2,048 rows 0 to 5 % slower.)
+    __device__ __forceinline__ static void load_row(const std::uint8_t* p, int part, u32x4& codes, std::uint32_t& behind) {
+        const Chunk16 c = *reinterpret_cast<const Chunk16*>(p + part * 16 + (part >> 1) * 4);
+        codes = u32x4{c.v[0], c.v[1], c.v[2], c.v[3]};
+        behind = reinterpret_cast<const Chunk4*>(p + (part == 0 ? 16 : 32))->v;
+    }
+    __device__ __forceinline__ static void arrange_row(int part, u32x4& codes, std::uint32_t behind, f16x2& scale) {
+        // (of the first lane, for the first two)
+        const std::uint32_t first = __builtin_amdgcn_update_dpp(0, static_cast<int>(codes[0]), 0xe0, 0xf, 0xf, true);
+        scale = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(behind, first, part < 2 ? 0x01000100u : 0x07060706u));
+        const std::uint32_t shift = part < 2 ? 2 : 0;
+#pragma unroll
+        for (int word = 0; word < 4; ++word) {
+            codes[word] = __builtin_amdgcn_alignbyte(word < 3 ? codes[word + 1] : behind, codes[word], shift);
+        }
+    }
+    __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
+        const int offset = (block * 4 + pair) * 68;
+        load_row(rows.first + offset, part, codes_a, behind_a);
+        load_row(rows.second + offset, part, codes_b, behind_b);
+    }
+    __device__ __forceinline__ void prepare_bits(const BlockHeader<kEncQ8_0>&, int, int part) {
+        arrange_row(part, codes_a, behind_a, scale_a);
+        arrange_row(part, codes_b, behind_b, scale_b);
+    }
+    __device__ __forceinline__ void prepare_scales(const BlockHeader<kEncQ8_0>&) {}
+    // flipping the sign bit turns the int8 code q into the byte q+128: bias 1024+128
+    template <int I>
+    __device__ __forceinline__ void group_a(std::uint32_t (&out)[2]) const {
+        scale_bytes(codes_a[I] ^ 0x80808080u, splat(-1152.0f), scale_a, splat(0.0f), out[0], out[1]);
+    }
+    template <int I>
+    __device__ __forceinline__ void group_b(std::uint32_t (&out)[2]) const {
+        scale_bytes(codes_b[I] ^ 0x80808080u, splat(-1152.0f), scale_b, splat(0.0f), out[0], out[1]);
+    }
+};
+
+// The same with every lane's codes loaded from where they begin, two bytes past a word for half the lanes, for
+// the tiles of 256 rows, which have no register left for the words' way (six in scratch: 200 rows of gate and up
+// 4,096 -> 11,264 80 -> 92 us).
+struct CodesAsTheyLie {
+    // a K step of 64 is two 34-byte blocks; `pair` counts K steps inside 256 values
+    u32x4 codes_a, codes_b;
     std::uint32_t d_a, d_b;
     f16x2 scale_a, scale_b;
     __device__ __forceinline__ static void load_row(const std::uint8_t* p, int part, u32x4& codes, std::uint32_t& d) {
@@ -491,33 +545,45 @@ struct PackedRun<kEncQ6K> {
 template <>
 struct PackedRun<kEncQ8_0> {
     u32x4 codes;
-    std::uint32_t d;
+    std::uint32_t behind;
     f16x2 scale;
     __device__ __forceinline__ void load(const WeightRows& rows, int block, int pair, int part) {
-        PackedSlice<kEncQ8_0>::load_row(rows.first + (block * 8 + pair * 2 + (part >> 1)) * 34, part, codes, d);
+        PackedSlice<kEncQ8_0>::load_row(rows.first + (block * 4 + pair) * 68, part, codes, behind);
     }
-    __device__ __forceinline__ void prepare_bits(const RunHeader<kEncQ8_0>&, int, int) {}
-    __device__ __forceinline__ void prepare_scales(const RunHeader<kEncQ8_0>&) {
-        const _Float16 h = __builtin_bit_cast(_Float16, static_cast<std::uint16_t>(d));
-        scale = f16x2{h, h};
+    __device__ __forceinline__ void prepare_bits(const RunHeader<kEncQ8_0>&, int, int part) {
+        PackedSlice<kEncQ8_0>::arrange_row(part, codes, behind, scale);
     }
+    __device__ __forceinline__ void prepare_scales(const RunHeader<kEncQ8_0>&) {}
     template <int I>
     __device__ __forceinline__ void decode(std::uint32_t (&out)[2]) const {
         scale_bytes(codes[I] ^ 0x80808080u, splat(-1152.0f), scale, splat(0.0f), out[0], out[1]);
     }
 };
 
-// what a thread holds and decodes with WAVES waves a workgroup
-template <std::uint32_t ENC, int WAVES>
+// what a thread holds and decodes with WAVES waves a workgroup and RB 32-row blocks a wave
+template <std::uint32_t ENC, int RB, int WAVES>
 struct Held {
     using Slice = PackedSlice<ENC>;
     using Header = BlockHeader<ENC>;
 };
-template <std::uint32_t ENC>
-struct Held<ENC, 8> {
+template <std::uint32_t ENC, int RB>
+struct Held<ENC, RB, 8> {
     using Slice = PackedRun<ENC>;
     using Header = RunHeader<ENC>;
 };
+template <>
+struct Held<kEncQ8_0, 2, 4> {
+    using Slice = CodesAsTheyLie;
+    using Header = BlockHeader<kEncQ8_0>;
+};
+template <int I>
+__device__ __forceinline__ void decode(const CodesAsTheyLie& slice, std::uint32_t (&out)[2]) {
+    if constexpr (I < 4) {
+        slice.template group_a<I>(out);
+    } else {
+        slice.template group_b<I - 4>(out);
+    }
+}
 template <int I, std::uint32_t ENC>
 __device__ __forceinline__ void decode(const PackedSlice<ENC>& slice, std::uint32_t (&out)[2]) {
     if constexpr (I < 4) {
@@ -586,7 +652,7 @@ template <std::uint32_t ENC, int RB, int WAVES, bool REFILL>
 __device__ __forceinline__ void k_step(
     v16f (&acc)[RB][4], ActivationSlice& a_now, WeightFragments& current,
     const std::uint8_t* b_read, const std::uint8_t* b_read_next, std::uint8_t* b_write,
-    typename Held<ENC, WAVES>::Slice& b_next, const typename Held<ENC, WAVES>::Header& header, int decode_pair,
+    typename Held<ENC, RB, WAVES>::Slice& b_next, const typename Held<ENC, RB, WAVES>::Header& header, int decode_pair,
     int b_part, const std::uint8_t* a_fetch, std::int64_t row_block_bytes, const WeightRows& b_global,
     int fetch_step) {
     WeightFragments ahead;
@@ -714,9 +780,9 @@ template <std::uint32_t ENC, int RB, int WAVES>
 constexpr int kWavesPerSimd = WAVES == 8 ? 2 : ENC == kEncQ6K ? RB == 1 ? 2 : 1 : RB == 1 && ENC == kEncQ4K ? 3 : 2;
 
 // The packed bytes of a block of a lane's rows.
-template <std::uint32_t ENC, int WAVES>
+template <std::uint32_t ENC, int RB, int WAVES>
 struct Slices {
-    typename Held<ENC, WAVES>::Slice b0, b1, b2, b3;  // of its four steps; Q6_K: b0 the first half, b1 the second
+    typename Held<ENC, RB, WAVES>::Slice b0, b1, b2, b3;  // of its four steps; Q6_K: b0 the first half, b1 the second
     __device__ __forceinline__ void load(const WeightRows& rows, int block, int part) {
         b0.load(rows, block, 0, part);
         b1.load(rows, block, kHalfBlocks<ENC> ? 2 : 1, part);
@@ -821,8 +887,8 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB, WAVES>, kWavesPerSimd<
     const int share = place.share;
     const int n_tile = divided(place.tile, m_tiles, by_m_tiles);
     const int m_tile = place.tile - n_tile * m_tiles;
-    using Slice = typename Held<ENC, WAVES>::Slice;
-    using Header = typename Held<ENC, WAVES>::Header;
+    using Slice = typename Held<ENC, RB, WAVES>::Slice;
+    using Header = typename Held<ENC, RB, WAVES>::Header;
     constexpr int kTileRows = 32 * RB * WAVES;
     const std::int64_t m0 = static_cast<std::int64_t>(m_tile) * kTileRows;
     const std::int64_t n0 = static_cast<std::int64_t>(n_tile) * kBN;
@@ -876,7 +942,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB, WAVES>, kWavesPerSimd<
     // before the first of its four steps is decoded.
     ActivationSlice a_now;
     constexpr bool kWhole = kWholeBlocks<ENC, RB, WAVES>;
-    Slices<ENC, WAVES> set0, set1;  // (set1: whole blocks only; the sets swap roles like the headers)
+    Slices<ENC, RB, WAVES> set0, set1;  // (set1: whole blocks only; the sets swap roles like the headers)
     Header header_even, header_odd;  // blocks 0, 2, 4 ... and 1, 3, 5 ...
     const int last_block = (steps >> 2) - 1;
     header_even.load(b_global.first, 0, b_part);
@@ -943,11 +1009,11 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB, WAVES>, kWavesPerSimd<
     // (Whole blocks: the next block goes to the other set at the start instead.
     // Q6_K: b0 holds a block's first half, which the first and, of the next block, the fourth step
     // decode, b1 the second.)
-    auto block_of_four = [&](int step, const Header& now, const Header& next, Slices<ENC, WAVES>& mine,
-                             Slices<ENC, WAVES>& other) {
+    auto block_of_four = [&](int step, const Header& now, const Header& next, Slices<ENC, RB, WAVES>& mine,
+                             Slices<ENC, RB, WAVES>& other) {
         constexpr bool kHalves = kHalfBlocks<ENC>;
         constexpr int kAhead = kHalves ? 3 : 4;  // from the step that is decoded to the one that is fetched
-        Slices<ENC, WAVES>& after = kWhole ? other : mine;
+        Slices<ENC, RB, WAVES>& after = kWhole ? other : mine;
         if constexpr (kWhole) {
             const int block = min((step >> 2) + 1, last_block);
             other.load(b_global, block, b_part);
@@ -1105,7 +1171,7 @@ __device__ __forceinline__ void low_step(v16f& acc, LowActivations& a, const std
 template <std::uint32_t ENC>
 struct LowBlock {
     BlockHeader<ENC> header;
-    Slices<ENC, 4> slices;
+    Slices<ENC, 1, 4> slices;
     __device__ __forceinline__ void load(const WeightRows& rows, int block, int part) {
         header.load(rows.first, block, part);
         slices.load(rows, block, part);
