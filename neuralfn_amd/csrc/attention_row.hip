@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
         position = tail.device_position[0];
         std::int64_t first = tail.whole_context != 0 ? 0 : position - tail.sliding_window + 1;
         if (first < 0) first = 0;
-        keys = static_cast<std::uint32_t>(position - first);
+        keys = static_cast<std::uint32_t>(position > first ? position - first : 0);
         first_slot = static_cast<std::uint32_t>(
             first < 2 * kMostKeys ? static_cast<std::uint32_t>(first) % capacity
                                   : static_cast<std::uint32_t>(first % static_cast<std::int64_t>(capacity)));
