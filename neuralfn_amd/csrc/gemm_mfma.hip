@@ -612,6 +612,13 @@ constexpr int kRunSecond = ENC == kEncQ4K || ENC == kEncQ5K ? 64 : 16;
 
 // The activation fragments of one K step for one wave: row blocks 0 and 1,
 // K chunks 0..3, in named registers (an array here ends up in scratch memory).
+// What a lane wrote to LDS is seen by the wave's other lanes, and no access moves across (no instruction of its own).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 struct ActivationSlice {
     f16x8 r0k0, r0k1, r0k2, r0k3, r1k0, r1k1, r1k2, r1k3;
 };
@@ -1084,6 +1091,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB, WAVES>, kWavesPerSimd<
 #pragma unroll
                 for (int j = 0; j < 4; ++j) turned[row * kPitch + j * 32 + column] = acc[i][j][r] * inverse;
             }
+            wave_sync();
             const std::int64_t m = first_row + part * kTurned;
             if (wide) {
                 const std::int64_t n = n0 + 4 * column;
@@ -1103,6 +1111,7 @@ __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<ENC, RB, WAVES>, kWavesPerSimd<
                     if (m + t < rows && n + 64 < output_dim) output[(m + t) * output_dim + n + 64] = second;
                 }
             }
+            wave_sync();
         }
     }
 }
@@ -1132,12 +1141,6 @@ __device__ __forceinline__ void low_step(v16f& acc, LowActivations& a, const std
                                          std::uint8_t* next_stage, PackedSlice<ENC>& b_next,
                                          const BlockHeader<ENC>& header, int decode_pair, int b_part,
                                          const std::uint8_t* a_fetch) {
-    // what a lane wrote is seen by the wave's other lanes, and no LDS access moves across
-    const auto wave_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
     wave_sync();
     f16x8 weights[4];
 #pragma unroll
