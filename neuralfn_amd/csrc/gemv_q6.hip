@@ -793,7 +793,7 @@ std::int64_t launch_stream(const ProjectionSet& set, const float* first, const f
         waves += op_waves;
     }
     const std::int64_t blocks = set.input_dim >> 8;
-    if (waves >= 0xffff || rows_per_wave > 0xffff || tokens > 0x3f || blocks > 0x3ff) {
+    if (waves > 0xffff - W || rows_per_wave > 0xffff || tokens > 0x3f || blocks > 0x3ff) {
         return launch_variant<T, P, ARGMAX>(set, first, second, records_out, tokens, candidates, stream);
     }
     starts[3] = static_cast<std::uint32_t>(waves);
