@@ -486,7 +486,7 @@ struct Ring {
     static constexpr unsigned kLdsBytes = kWaves * kStages * kStageBytes;
 };
 
-// A tile of 16 weight rows as both the fetching and the multiplying side see it (uniform).
+// A tile of up to 16 weight rows as both the fetching and the multiplying side see it (uniform).
 struct TileShape {
     const __attribute__((address_space(1))) std::uint8_t* base;  // its first row
     std::uint32_t stride;  // bytes between rows
@@ -494,10 +494,11 @@ struct TileShape {
     int final_row;         // the projection's last row if it is one of the tile's, else -1
 };
 
+// tile_rows: weight rows of a tile (the rule is rows_of_tile's).
 // DEPTH: blocks of a wave's share of K that it holds the fragments of (kDepth, or kShortDepth where no share has more).
 template <std::uint32_t ENC, int MODE, bool RING, int DEPTH>
 __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
-    const std::uint8_t* __restrict__ image, const float* __restrict__ inverse_scale, int tokens,
+    const std::uint8_t* __restrict__ image, const float* __restrict__ inverse_scale, int tokens, int tile_rows,
     std::uint32_t total_tiles, int input_dim, LmHeadCandidate* __restrict__ candidates,
     ProjectionSet set) {
     using Block = PackedBlock<ENC>;
@@ -573,9 +574,9 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
         const int index = PAIRS ? group : group * kGroupTiles + slot;
         const std::uint32_t tile = blockIdx.x + static_cast<std::uint32_t>(index) * gridDim.x;
         const Projection op = PAIRS ? pick(set, slot) : tile_projection(set, tile);
-        const std::int64_t row0 = static_cast<std::int64_t>(tile - (PAIRS ? 0u : op.first_tile)) * kTileRows;
+        const std::int64_t row0 = static_cast<std::int64_t>(tile - (PAIRS ? 0u : op.first_tile)) * tile_rows;
         TileShape shape;
-        shape.last = static_cast<int>(min(static_cast<std::int64_t>(kTileRows - 1), op.output_dim - 1 - row0));
+        shape.last = static_cast<int>(min(static_cast<std::int64_t>(tile_rows - 1), op.output_dim - 1 - row0));
         shape.base = (GlobalBytes)op.data + row0 * op.row_stride;
         shape.stride = static_cast<std::uint32_t>(op.row_stride);
         shape.final_row = row0 + shape.last == op.output_dim - 1 ? shape.last : -1;
@@ -819,7 +820,7 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
         if constexpr (PAIRS) {
             if (wave == 0) {
                 const std::uint32_t tile = blockIdx.x + static_cast<std::uint32_t>(group) * gridDim.x;
-                const std::int64_t row = static_cast<std::int64_t>(tile) * kTileRows + i;
+                const std::int64_t row = static_cast<std::int64_t>(tile) * tile_rows + i;
                 f32x4 first = *reinterpret_cast<const f32x4*>(buffer + lane * 4);
                 f32x4 second = *reinterpret_cast<const f32x4*>(buffer + (kWaves * kWave + lane) * 4);
 #pragma unroll
@@ -830,7 +831,7 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int token = 4 * j + r;
-                    if (token < tokens && row < set.op[0].output_dim) {
+                    if (token < tokens && i < tile_rows && row < set.op[0].output_dim) {
                         set.op[0].output[static_cast<std::int64_t>(token) * set.op[0].output_dim + row] =
                             apply_prologue<kSwiGlu>(first[r], second[r]);
                     }
@@ -843,7 +844,7 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
             const std::uint32_t tile =
                 blockIdx.x + static_cast<std::uint32_t>(group * kGroupTiles + wave) * gridDim.x;
             const Projection op = tile_projection(set, tile);
-            const std::int64_t row = static_cast<std::int64_t>(tile - op.first_tile) * kTileRows + i;
+            const std::int64_t row = static_cast<std::int64_t>(tile - op.first_tile) * tile_rows + i;
             f32x4 sum = *reinterpret_cast<const f32x4*>(mine + lane * 4);
 #pragma unroll
             for (int w = 1; w < kWaves; ++w) {
@@ -867,7 +868,7 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int token = 4 * j + r;
-                    if (token < tokens && row < op.output_dim) {
+                    if (token < tokens && i < tile_rows && row < op.output_dim) {
                         op.output[static_cast<std::int64_t>(token) * op.output_dim + row] = sum[r];
                     }
                 }
@@ -936,20 +937,38 @@ bool ring_form(const ProjectionSet& set) {
 // need the deeper pipeline: their shares would take twice the chunks, each a wait of its own for its fragments.
 bool short_rows(std::int64_t input_dim) { return input_dim <= kShortDepth * kWaves * 256; }
 
+// Rows of a tile for the first `count` projections of a set (a pair counts once).  Tiles of sixteen rows rarely come out
+// even: 6,656 rows are 416 of them, two for 160 of 256 workgroups and one for the others, which then stand still.  The
+// fewest rows that send no workgroup round once more (there: thirteen) give all of them the same, for one row's bits as before;
+// lanes without a row repeat the tile's last one's requests.  us, sixteen rows -> fewer, of 16 tokens: 16,384 -> 6,656 Q4_K
+// 27.9 -> 27.0, Q5_K 32.4 -> 30.6, Q6_K 35.5 -> 33.7, Q8_0 34.7 -> 33.3; 6,656 -> 4,096, 256, 256 and 4,096 Q4_K 19.0 -> 18.2;
+// 5,000 calls of 5 to 16 tokens, geometric means: two tiles a workgroup 1.04 (no format under 1.025), three 1.03, four to
+// six 1.02 (the slowest 3 % longer), seven and more 1.00: whole tiles.  One tile and more workgroups: Q4_K 1.03 and
+// Q5_K 1.03; Q6_K 1.00 and down to 0.92 (whole); Q8_0 1.02 from six rows and 6,144 columns on, 0.99 below (whole).
+int rows_of_tile(std::uint32_t encoding, const ProjectionSet& set, int count) {
+    const EvenTiles even = even_tiles(set, count, kTileRows, 4);
+    if (even.each > 6) return kTileRows;
+    if (even.each == 1 && (encoding == kEncQ6K || (encoding == kEncQ8_0 && (set.input_dim < 6144 || even.rows < 6)))) {
+        return kTileRows;
+    }
+    return even.rows;
+}
+
 // `candidates` non-null: the lm_head form (one projection), which returns its workgroup count.
 template <std::uint32_t ENC>
 std::uint32_t launch_encoding(ProjectionSet set, const std::uint8_t* image, const float* inverse_scale,
                               int tokens, LmHeadCandidate* candidates, hipStream_t stream) {
+    const int tile_rows = candidates != nullptr ? kTileRows : rows_of_tile(ENC, set, set.count);
     std::uint32_t tiles = 0;
     for (int index = 0; index < set.count; ++index) {
         set.op[index].first_tile = tiles;
-        tiles += static_cast<std::uint32_t>((set.op[index].output_dim + kTileRows - 1) / kTileRows);
+        tiles += static_cast<std::uint32_t>((set.op[index].output_dim + tile_rows - 1) / tile_rows);
     }
     const std::uint32_t grid = grid_of(tiles, candidates != nullptr);
     const bool few = short_rows(set.input_dim);
     const auto launch = [&](auto kernel, unsigned lds) {
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, image, inverse_scale, tokens, tiles,
-                           static_cast<int>(set.input_dim), candidates, set);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, image, inverse_scale, tokens, tile_rows,
+                           tiles, static_cast<int>(set.input_dim), candidates, set);
     };
     const auto launch_ring = [&](auto mode, auto depth) {
         constexpr unsigned kLds = Ring<ENC>::kLdsBytes;  // (beside 36 KB of static LDS)
@@ -978,11 +997,11 @@ std::uint32_t launch_encoding(ProjectionSet set, const std::uint8_t* image, cons
 template <std::uint32_t ENC>
 void launch_pair(const ProjectionSet& set, const std::uint8_t* image, const float* inverse_scale,
                  int tokens, hipStream_t stream) {
-    const std::uint32_t tiles =
-        static_cast<std::uint32_t>((set.op[0].output_dim + kTileRows - 1) / kTileRows);
+    const int tile_rows = rows_of_tile(ENC, set, 1);
+    const std::uint32_t tiles = static_cast<std::uint32_t>((set.op[0].output_dim + tile_rows - 1) / tile_rows);
     const auto launch = [&](auto kernel, unsigned lds) {
         hipLaunchKernelGGL(kernel, dim3(grid_of(tiles, false)), dim3(kThreads), lds, stream, image, inverse_scale, tokens,
-                           tiles, static_cast<int>(set.input_dim), static_cast<LmHeadCandidate*>(nullptr), set);
+                           tile_rows, tiles, static_cast<int>(set.input_dim), static_cast<LmHeadCandidate*>(nullptr), set);
     };
     const bool few = short_rows(set.input_dim);
     if (!ring_form<ENC>(set)) {

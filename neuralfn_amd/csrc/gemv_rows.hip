@@ -15,7 +15,7 @@
 //   * which terms form a chain: the units 4b + p of the blocks b = c, c + 16, c + 32, ...
 //     ("class" c = 0..15, p = 0..3; a block: 256 values), in that order,
 //   * the balanced binary tree over the 64 chains in the order (c, p).
-// Here a workgroup of 8 waves owns 32 consecutive weight rows.  A matrix instruction takes
+// Here a workgroup of 8 waves owns up to 32 consecutive weight rows.  A matrix instruction takes
 // the values of a scale group (K: 32 values, 16 for Q6_K), 32 weight rows (operand B, lane l:
 // row l % 32, half l / 32 of the group; the packed bytes are loaded coalesced and change lanes
 // through a private LDS tile per wave) and the two int8 planes of up to 16 tokens (operand A,
@@ -208,10 +208,11 @@ __device__ __forceinline__ void rows_wait_for_all(std::uint32_t words, int count
 // about half the length, shared out over the workgroups by what the halves cost (a row of 26
 // blocks has 16 on the left and 10 on the right): for tile counts that leave much of the
 // chip idle in the last pass over whole tiles (272 tiles on 256 units).
+// rows_a_tile: kRowsTile; where whole tiles would not come out even, fewer (rows_of_tile).
 template <std::uint32_t ENC, int S, bool SPLIT>
 __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
     const std::uint8_t* __restrict__ image, const std::uint8_t* __restrict__ records, int tokens,
-    int input_dim, std::uint32_t total_tiles, std::uint32_t left_groups, ProjectionSet set) {
+    int input_dim, std::uint32_t total_tiles, std::uint32_t left_groups, int rows_a_tile, ProjectionSet set) {
     constexpr bool kQ5 = ENC == kEncQ5K;
     using F = RowsFormat<ENC>;
     constexpr int kBlockBytes = F::kBlockBytes;
@@ -279,9 +280,9 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
     const int last_slot = min((F::kLoads - 1) * kWave + lane, F::kTileChunks - 1) * 16;
     auto aim = [&](std::uint32_t tile) {
         const Projection op = projection_of(tile);
-        const std::int64_t row0 = static_cast<std::int64_t>(tile - op.first_tile) * kRowsTile;
+        const std::int64_t row0 = static_cast<std::int64_t>(tile - op.first_tile) * rows_a_tile;
         const int valid_rows =
-            static_cast<int>(min(static_cast<std::int64_t>(kRowsTile), op.output_dim - row0));
+            static_cast<int>(min(static_cast<std::int64_t>(rows_a_tile), op.output_dim - row0));
         tile_rows = op.data + row0 * op.row_stride;
         row_parity = 0;
 #pragma unroll
@@ -727,9 +728,9 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
     auto add_classes = [&](int index) {
         const std::uint32_t tile = first_tile + static_cast<std::uint32_t>(index) * tile_stride;
         const Projection op = projection_of(tile);
-        const std::int64_t row0 = static_cast<std::int64_t>(tile - op.first_tile) * kRowsTile;
+        const std::int64_t row0 = static_cast<std::int64_t>(tile - op.first_tile) * rows_a_tile;
         const int valid_rows =
-            static_cast<int>(min(static_cast<std::int64_t>(kRowsTile), op.output_dim - row0));
+            static_cast<int>(min(static_cast<std::int64_t>(rows_a_tile), op.output_dim - row0));
         if (token < kTokens && token < tokens && j < valid_rows) {
             const auto& sums = class_sums[index % kTilesHeld];
             float pairs[kOwnClasses / 2];
@@ -986,20 +987,31 @@ RowsPlan plan_rows(std::uint32_t tiles, std::int64_t input_dim, std::int64_t tok
     return plan;
 }
 
+// Rows of a tile of the whole form: the fewest that send no workgroup round once more, so that 6,656 rows are 256 tiles of
+// 26 and not 208 of 32.  us, seven tokens, 32 rows -> fewer: 16,384 -> 6,656 Q4_K 26.2 -> 24.2, Q5_K 28.0 -> 26.7, Q8_0 32.8 ->
+// 31.0; 4,608 -> 4,608 Q4_K 11.6 -> 11.0.  1,700 calls of 5 to 16 tokens, geometric means: several tiles a workgroup 1.015 of
+// all formats (the slowest 2 % longer), one of sixteen rows and more 1.02 of Q4_K and Q5_K, 1.03 of Q8_0; of fewer rows
+// 1.00, and of Q6_K 0.99, down to 0.95: whole tiles.
+int rows_of_tile(std::uint32_t encoding, const ProjectionSet& set) {
+    const EvenTiles even = even_tiles(set, set.count, kRowsTile, 4);
+    if (even.each > 6 || (even.each == 1 && (even.rows < 16 || encoding == kEncQ6K))) return kRowsTile;
+    return even.rows;
+}
+
 template <std::uint32_t ENC, bool SPLIT>
 void launch_form(const ProjectionSet& set, const std::uint8_t* image, const std::uint8_t* records,
-                 int tokens, std::uint32_t tiles, const RowsPlan& plan, hipStream_t stream) {
+                 int tokens, std::uint32_t tiles, int rows_a_tile, const RowsPlan& plan, hipStream_t stream) {
     const dim3 grid(plan.groups), block(kRowsThreads);
     const int input_dim = static_cast<int>(set.input_dim);
     if (tokens <= 4) {
         hipLaunchKernelGGL((gemv_rows_kernel<ENC, 2, SPLIT>), grid, block, 0, stream, image, records, tokens,
-                           input_dim, tiles, plan.left_groups, set);
+                           input_dim, tiles, plan.left_groups, rows_a_tile, set);
     } else if (tokens <= 8) {
         hipLaunchKernelGGL((gemv_rows_kernel<ENC, 4, SPLIT>), grid, block, 0, stream, image, records, tokens,
-                           input_dim, tiles, plan.left_groups, set);
+                           input_dim, tiles, plan.left_groups, rows_a_tile, set);
     } else {
         hipLaunchKernelGGL((gemv_rows_kernel<ENC, 8, SPLIT>), grid, block, 0, stream, image, records, tokens,
-                           input_dim, tiles, plan.left_groups, set);
+                           input_dim, tiles, plan.left_groups, rows_a_tile, set);
     }
 }
 
@@ -1011,11 +1023,22 @@ void launch_encoding(ProjectionSet set, const std::uint8_t* image, const std::ui
         set.op[index].first_tile = tiles;
         tiles += static_cast<std::uint32_t>((set.op[index].output_dim + kRowsTile - 1) / kRowsTile);
     }
-    const RowsPlan plan = plan_rows(tiles, set.input_dim, tokens, outputs_cleared, fill_launch);
+    RowsPlan plan = plan_rows(tiles, set.input_dim, tokens, outputs_cleared, fill_launch);
+    int rows = kRowsTile;
+    if (!plan.split) {
+        rows = rows_of_tile(ENC, set);
+        tiles = 0;
+        for (int index = 0; index < set.count; ++index) {
+            set.op[index].first_tile = tiles;
+            tiles += static_cast<std::uint32_t>((set.op[index].output_dim + rows - 1) / rows);
+        }
+        const std::uint32_t units = static_cast<std::uint32_t>(compute_units());
+        plan.groups = tiles < units ? tiles : units;
+    }
     if (plan.split) {
-        launch_form<ENC, true>(set, image, records, tokens, tiles, plan, stream);
+        launch_form<ENC, true>(set, image, records, tokens, tiles, rows, plan, stream);
     } else {
-        launch_form<ENC, false>(set, image, records, tokens, tiles, plan, stream);
+        launch_form<ENC, false>(set, image, records, tokens, tiles, rows, plan, stream);
     }
 }
 

@@ -431,6 +431,32 @@ __device__ __forceinline__ WaveRows wave_rows(int group, int wave, int rows_per_
     return rows;
 }
 
+// How many tiles of up to `whole` rows of a set's first `count` projections a workgroup takes where every unit has one, and
+// the fewest rows a tile, `fewest` at least, with which no workgroup takes more.
+struct EvenTiles {
+    std::int64_t each;
+    int rows;
+};
+inline EvenTiles even_tiles(const ProjectionSet& set, int count, int whole, int fewest) {
+    const std::int64_t units = compute_units();
+    const auto tiles_of = [&](int rows) {
+        std::int64_t tiles = 0;
+        for (int index = 0; index < count; ++index) tiles += (set.op[index].output_dim + rows - 1) / rows;
+        return tiles;
+    };
+    EvenTiles even{(tiles_of(whole) + units - 1) / units, whole};
+    int low = fewest;
+    while (low < even.rows) {  // fewer rows make no fewer tiles
+        const int middle = (low + even.rows) / 2;
+        if (tiles_of(middle) <= even.each * units) {
+            even.rows = middle;
+        } else {
+            low = middle + 1;
+        }
+    }
+    return even;
+}
+
 // Workgroups of a wave-per-row decode launch.  Small launches are bound by
 // fixed costs: waves start at a limited rate and every workgroup quantizes the
 // whole activation vector, so one workgroup per compute unit (all resident at

@@ -841,6 +841,61 @@ def test_small_batch_half_kernel_short_rows(cuda, oracle, encoding, in_dim):
     assert_bits_equal(outputs[0], outputs[1][:, :24].contiguous(), "one tile = its place among many")
 
 
+@pytest.mark.parametrize("family,rows", [("mmq", 5), ("mmq", 16), ("mmvq", 7), ("mmvq", 16)])
+@pytest.mark.parametrize("encoding,in_dim", [(kquant.Q4_K, 512), (kquant.Q5_K, 768), (kquant.Q6_K, 768), (kquant.Q8_0, 512),
+                                             (kquant.Q8_0, 6144)])
+def test_small_batch_tiles_of_fewer_rows(cuda, oracle, encoding, in_dim, family, rows):
+    """Tiles of as few rows as keep every workgroup at its number of tiles: the fewest rows there are, one tile a
+    workgroup with and without a remainder, two, three, and so many that tiles stay whole; alone and beside another
+    projection.  A row has the bits it has in a launch of its own."""
+    units = torch_().cuda.get_device_properties(0).multi_processor_count
+    most = 7 * 32 * units + 9
+    packed = random_packed(encoding, most, in_dim, 31).reshape(most, -1)
+    x = kquant.synthetic_activations(32, rows, in_dim)
+    workspace = tile_ops.small_batch_workspace(rows, in_dim)
+
+    def run(*spans):
+        weights = [tile_ops.PackedWeight.from_numpy(encoding, packed[a:b].reshape(-1), b - a, in_dim) for a, b in spans]
+        return [y.cpu() for y in tile_ops.multi_linear(weights, to_device(x, cuda), workspace, family=family)]
+
+    (own,) = run((0, 40))
+    expected = oracle.linear(encoding, packed[:40].reshape(-1), 40, in_dim, x)
+    assert normalised_error(own.numpy(), expected) <= TOLERANCE
+    sizes = [4 * units - 3, 4 * units + 1, 13 * units, 16 * units + 5, 26 * units, 26 * units + 1, 2 * 32 * units + 7, most]
+    for out_dim in sizes if in_dim < 6144 else sizes[:5]:
+        (y,) = run((0, out_dim))
+        assert_bits_equal(y[:, :40].contiguous(), own, f"first rows of {out_dim}")
+        (last,) = run((out_dim - 40, out_dim))
+        assert_bits_equal(y[:, -40:].contiguous(), last, f"last rows of {out_dim}")
+        middle = out_dim // 2
+        (between,) = run((middle - 20, middle + 20))
+        assert_bits_equal(y[:, middle - 20:middle + 20].contiguous(), between, f"middle rows of {out_dim}")
+    first, second = run((0, 13 * units + 2), (40, 40 + 9 * units))
+    assert_bits_equal(first[:, :40].contiguous(), own, "beside another projection")
+    (alone,) = run((40, 80))
+    assert_bits_equal(second[:, :40].contiguous(), alone, "the other projection")
+
+
+@pytest.mark.parametrize("rows", [5, 16])
+@pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K, kquant.Q6_K, kquant.Q8_0])
+def test_gate_up_swiglu_rows_tiles_of_fewer_rows(cuda, encoding, rows):
+    """The pair form's tiles likewise."""
+    units = torch_().cuda.get_device_properties(0).multi_processor_count
+    in_dim, most = 512, 16 * units + 9
+    packed = [random_packed(encoding, most, in_dim, seed).reshape(most, -1) for seed in (41, 42)]
+    x = to_device(kquant.synthetic_activations(43, rows, in_dim), cuda)
+    workspace = tile_ops.small_batch_workspace(rows, in_dim)
+
+    def run(begin, end):
+        gate, up = (tile_ops.PackedWeight.from_numpy(encoding, p[begin:end].reshape(-1), end - begin, in_dim) for p in packed)
+        return tile_ops.gate_up_swiglu_rows(gate, up, x, rows, workspace).cpu()
+
+    for out_dim in (4 * units + 1, 13 * units, most):
+        y = run(0, out_dim)
+        assert_bits_equal(y[:, :40].contiguous(), run(0, 40), f"first rows of {out_dim}")
+        assert_bits_equal(y[:, -40:].contiguous(), run(out_dim - 40, out_dim), f"last rows of {out_dim}")
+
+
 @pytest.mark.parametrize("in_dim", [4096, 8192, 8448, 16384])
 @pytest.mark.parametrize("encoding", [kquant.Q4_K, kquant.Q5_K])
 def test_decode_dot_kernel_row_lengths(cuda, oracle, encoding, in_dim):
