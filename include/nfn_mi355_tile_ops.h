@@ -672,7 +672,7 @@ int nfn_native_tile_glimmer_cache_commit_rows_bf16_v1(
  * 946-947): qk_norm_scale_rope on query/key (in place), gqa_decode with key as
  * the current key, and the bf16 cache commit of key/current_value at
  * `position`.  The norm weights are embedded by value; has_*_norm_weight == 0
- * makes the corresponding descriptor inert.  Here it is two launches on the
+ * makes the corresponding descriptor inert.  Here it is, without a workspace, two launches on the
  * descriptor's stream (the norm/rope kernel also writes the cache row, which a
  * one-token attention at this position does not read; a key range as long as
  * the ring gets the commit as a third launch, after the attention), with the
@@ -1017,8 +1017,10 @@ int nfn_mi355_gqa_decode_split_v1(
     int64_t workspace_nbytes);
 
 /* nfn_native_tile_glimmer_fused_decode_attention_float32_v1 with the split
- * attention form above: three launches (norm/rope/commit, attention shares,
- * merge).  Same descriptor, same workspace as nfn_mi355_gqa_decode_split_v1. */
+ * attention form above: attention shares and their merge, with the norms, the
+ * rotation and the commit inside (head_dim 128, four or more query heads per
+ * key/value head; else in a launch before).  Same descriptor, same workspace
+ * as nfn_mi355_gqa_decode_split_v1. */
 int nfn_mi355_fused_decode_attention_split_v1(
     const NfnNativeTileGlimmerFusedDecodeAttentionDescriptorV1* descriptor,
     void* workspace,

@@ -9,8 +9,9 @@ down projection; post-feed-forward norm + residual.  The grouping into calls is 
 engine's: one grouped small-batch call per shared input, the sigmoid gate and SwiGLU as prologues
 of the projection that consumes them, two adjacent norms in one dual-RMS call
 (neuralfn/csrc/native_gpt2/resident_glimmer_cuda.cpp:2233-2585, 2913-2960), and the Q/K norms,
-rope, attention and cache commit in its fused decode-attention call (two launches here).
-Eight launches per layer and token.
+rope, attention and cache commit in its fused decode-attention call (two launches here: norms and
+attention, or with a workspace the attention's shares and their merge).  Eight launches per layer
+and token, seven with the first norm inside the projections' launch.
 
 This is host-side sequencing for tests and benchmarks, not an engine: no sampling, no prompt
 handling, one token per step.
@@ -216,5 +217,5 @@ def verify_layer(geometry: LayerGeometry, weights: LayerWeights, cache: LayerCac
 
 
 LAUNCHES_PER_LAYER = 8           # with the reference's fused attention call
-LAUNCHES_PER_LAYER_SPLIT = 9     # with the split attention form (one more: the merge)
-LAUNCHES_PER_LAYER_FUSED = 8     # ... and the first dual norm inside the Q/K/V/gate launch
+LAUNCHES_PER_LAYER_SPLIT = 8     # with the split attention form (its merge, but norms, rope and commit inside)
+LAUNCHES_PER_LAYER_FUSED = 7     # ... and the first dual norm inside the Q/K/V/gate launch
