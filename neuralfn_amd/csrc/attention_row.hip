@@ -43,6 +43,7 @@
 #include "wave_rows.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace nfn {
 
@@ -53,6 +54,7 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 constexpr int kRowWaves = 8;
 constexpr int kWaveKeys = 16;  // keys a wave scores in a step
 constexpr int kStepKeys = kRowWaves * kWaveKeys;
+constexpr int kLoadsDone = 0x0f70;  // s_waitcnt: no load in flight
 constexpr int kWaveHeads = kGroupHeads / kRowWaves;
 constexpr std::int64_t kMostKeys = std::int64_t(1) << 30;  // of a ring or a call: sums of two fit 32 bits
 static_assert(kGroupHeadDim == 16 * kRowWaves && kGroupHeadDim == 2 * kWave, "dimensions of a wave and a lane");
@@ -239,11 +241,15 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
     uint4 key_raw[4], value_raw[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) key_raw[r] = value_raw[r] = make_uint4(0u, 0u, 0u, 0u);
+    // (settle: requests of both kinds of row have landed where they end.  The lanes that keep the cache's row need not wait for
+    // the block's, but the compiler then takes those loads for possibly in flight in every step and waits for the next
+    // step's rows where their registers are used again: 7 rows of 48 heads over 8, 2,048 keys 16.8 -> 14.9 us, 12 of 16 over
+    // 4, 4,000 20.4 -> 17.4.  A wave's first requests are waited for soon enough.)
     const auto keys_left = [&](int begin) {  // of the wave's sixteen, wave-uniform
         const int left = here - begin;
         return left < 0 ? 0 : left < kWaveKeys ? left : kWaveKeys;
     };
-    const auto request_keys = [&](int begin, std::uint32_t at) {
+    const auto request_keys = [&](int begin, std::uint32_t at, [[maybe_unused]] auto settle) {
         const int count = keys_left(begin);
         if (count == 0) return;
         if constexpr (BLOCK) {
@@ -264,6 +270,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
                 }
 #pragma unroll
                 for (int s = 0; s < 4; ++s) key_raw[s] = from_block ? pack_as_cached(low[s], high[s]) : raw[s];
+                if constexpr (settle()) __builtin_amdgcn_s_waitcnt(kLoadsDone);
                 return;
             }
         }
@@ -272,7 +279,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
 #pragma unroll
         for (int s = 0; s < 4; ++s) key_raw[s] = *reinterpret_cast<const uint4*>(source + 32 * s);
     };
-    const auto request_values = [&](int begin, std::uint32_t at) {
+    const auto request_values = [&](int begin, std::uint32_t at, [[maybe_unused]] auto settle) {
         const int count = keys_left(begin);
         if (count == 0) return;
         if constexpr (BLOCK) {
@@ -294,6 +301,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
                     const int key = 4 * r + j < count ? 4 * r + j : count - 1;
                     value_raw[r] = begin + key >= cached ? pack_as_cached(low[r], high[r]) : raw[r];
                 }
+                if constexpr (settle()) __builtin_amdgcn_s_waitcnt(kLoadsDone);
                 return;
             }
         }
@@ -304,8 +312,8 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
                 value_cache + static_cast<std::uint64_t>(row) * row_stride + head_offset + 8 * i);
         }
     };
-    request_keys(wave * kWaveKeys, slot);
-    request_values(wave * kWaveKeys, slot);
+    request_keys(wave * kWaveKeys, slot, std::false_type());
+    request_values(wave * kWaveKeys, slot, std::false_type());
 
     // the current row's key and, of its value, the dimensions this lane adds up
     HeadPair row_key{0.0f, 0.0f}, row_value{0.0f, 0.0f};
@@ -414,7 +422,10 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
     for (int begin = 0; begin < here; begin += kStepKeys) {
         const int wave_begin = begin + wave * kWaveKeys;
         const int count = keys_left(wave_begin);
-        // a chain per term of the query
+        // A chain per term of the query.  Where they meet, the sum is as large as the score and rounds like it; the exponent
+        // below takes them one by one on top of the maximum instead, where what is left of a key that matters is small.
+        // Against float64, 100 to 2,047 keys: 1.53 to 1.86e-7, attention_grouped_kernel 1.59 to 1.98e-7 (the exponent from
+        // the rounded score: 1.64 to 1.98e-7; one chain with the large term last: 1.50 to 1.86e-7, five steps 2 us longer).
         f32x4 chains[3] = {};
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -427,13 +438,13 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
         // the next step's keys are requested as soon as these have been used
         const std::uint32_t next_slot = ring_row(slot + slot_step);
         const bool more = begin + kStepKeys < here;
-        if (more) request_keys(wave_begin + kStepKeys, next_slot);
-        float score[4];
+        if (more) request_keys(wave_begin + kStepKeys, next_slot, std::true_type());
+        float lower[4];  // of the products, the lower terms' part
         float largest = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            score[r] = 4 * j + r < count ? ((chains[2][r] + chains[1][r]) + chains[0][r]) * scale : -INFINITY;
-            largest = fmaxf(largest, score[r]);
+            lower[r] = chains[2][r] + chains[1][r];
+            largest = fmaxf(largest, 4 * j + r < count ? (lower[r] + chains[0][r]) * scale : -INFINITY);
         }
         largest = across_j_max(largest);
         if (j == 0) wave_maximum[i][wave] = largest;
@@ -448,7 +459,10 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
         maximum = next_maximum;
         float weight[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) weight[r] = __expf(score[r] - next_maximum);  // 0 for a dead key
+        for (int r = 0; r < 4; ++r) {
+            const float exponent = fmaf(lower[r], scale, fmaf(chains[0][r], scale, -next_maximum));
+            weight[r] = 4 * j + r < count ? __expf(exponent) : 0.0f;
+        }
         const float sum = across_j_sum((weight[0] + weight[1]) + (weight[2] + weight[3]));
         if (j == 0) wave_sum[i][wave] = sum;
         std::uint32_t words[3][2];
@@ -464,7 +478,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
             if (4 * r + j >= count) value = make_uint4(0u, 0u, 0u, 0u);
             *reinterpret_cast<uint4*>(staged_values + (wave * kWaveKeys + 4 * r + j) * kStageRowBytes + 16 * i) = value;
         }
-        if (more) request_values(wave_begin + kStepKeys, next_slot);
+        if (more) request_values(wave_begin + kStepKeys, next_slot, std::true_type());
         slot = next_slot;
         __syncthreads();
 
@@ -520,11 +534,12 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
 // 100 -> 200 keys 5.1 -> 6.6), shares with their merge from 300 keys on 7.7.
 constexpr std::int64_t kAloneKeys = 256;
 
-// The longest share of a block's row, in keys.  Many steps are 2 us each for a workgroup that has a unit alone, since its waves
+// The longest share of a block's row, in keys.  A step is 1.6 to 2 us for a workgroup that has a unit alone, since its waves
 // meet twice a step; the waves of attention_grouped_kernel walk alone.  With merge, us, that kernel / this one: 128 keys a
-// share (7 rows of 32 heads over 2, 2,048 keys) 13.4 / 11.5; 512 (10 of 32 over 8, 1,500) 16.6 / 16.3; 1,024 (12 of 16 over
-// 4, 4,000) 20.2 / 18.6; 1,280 (16 of 32 over 4, 4,802) 24.0 / 23.9; 2,176 (16 of 48 over 2, 8,192) 35.4 / 37.2; 4,224 (16
-// of 32 over 8, 8,192) 61.6 / 72.2.  (Two workgroups a unit: 128 registers, of which 31 go to scratch memory, 64.7 and 117.)
+// share (7 rows of 32 heads over 2, 2,048 keys) 12.8 / 10.9; 640 (7 of 48 over 8, 2,048) 16.0 / 14.7; 512 (10 of 32 over 8,
+// 1,500) 16.8 / 16.3; 768 (16 of 32 over 8, 1,500) 19.6 / 19.5; 1,024 (16 of 32 over 8, 2,000) 23.4 / 22.2; 1,280 (16 of 32
+// over 4, 4,802) 24.0 / 22.4, but (of 32 over 8, 2,500) 24.6 / 25.3; 2,176 (16 of 48 over 2, 8,192) 34.6 / 35.1; 4,224 (16
+// of 32 over 8, 8,192) 57.4 / 58.4.  (Two workgroups a unit: 128 registers, of which 31 go to scratch memory, 64.7 and 117.)
 constexpr std::int64_t kBlockKeys = 1024;
 
 bool overlap(const void* a, std::int64_t a_bytes, const void* b, std::int64_t b_bytes) {

@@ -515,6 +515,36 @@ def test_one_row_attention_in_one_launch_rounds_no_more_than_in_shares(cuda, que
     assert max(errors[1:]) <= 1.25 * errors[0], errors
 
 
+@pytest.mark.parametrize("query_heads,kv_heads", [(32, 2), (48, 8)])
+@pytest.mark.parametrize("keys", [180, 500])
+def test_one_row_attention_rounds_no_more_than_a_block_of_every_row(cuda, query_heads, kv_heads, keys):
+    """The one-token call, and rows of a causal block, against float64: no further off than the kernel of blocks whose
+    rows all see each other, over sixty draws, whose mean is known to one percent."""
+    generator = torch_().Generator(device=cuda).manual_seed(11)
+    normal = lambda *shape: torch_().randn(shape, generator=generator, device=cuda)
+    scale, heads_per_kv = 128 ** -0.5, query_heads // kv_heads
+    workspace = engine_ops.gqa_decode_workspace(8 * query_heads, 128)
+    errors = {"row": 0.0, "causal": 0.0, "all": 0.0}
+    for _ in range(60):
+        query, key, value = normal(2, query_heads, 128), normal(2, kv_heads, 128), normal(2, kv_heads, 128)
+        key, value = (t.to(torch_().bfloat16).float() for t in (key, value))  # (a causal block's earlier row is rounded)
+        rings = [normal(keys + 64, kv_heads * 128).to(torch_().bfloat16) for _ in range(2)]
+        bits = [ring.view(torch_().int16) for ring in rings]
+        outputs = {
+            "row": (engine_ops.gqa_decode(query[0], key[0], value[0], *bits, keys, 0, scale, workspace=workspace), query[0], 1),
+            "causal": (engine_ops.block_attention(query, key, value, *bits, keys, keys + 2, scale, True, workspace=workspace)
+                       .reshape(query.shape)[1], query[1], 2),
+            "all": (engine_ops.block_attention(query, key, value, *bits, keys, keys + 2, scale, False, workspace=workspace)
+                    .reshape(query.shape)[1], query[1], 2)}
+        for name, (out, q, own) in outputs.items():
+            k, v = (torch_().cat([ring[:keys].double().reshape(keys, kv_heads, 128), rows[:own].double()]).permute(1, 0, 2)
+                    .repeat_interleave(heads_per_kv, 0) for ring, rows in zip(rings, (key, value)))
+            weights = torch_().softmax((k * q.double()[:, None]).sum(-1) * scale, 1)
+            exact = (weights[:, :, None] * v).sum(1)
+            errors[name] += ((out.double().reshape(exact.shape) - exact).norm() / exact.norm()).item() / 60
+    assert max(errors["row"], errors["causal"]) <= 1.01 * errors["all"], errors
+
+
 def test_block_attention_fails_closed(cuda):
     lib = tile_ops.load()
     x = torch_().zeros(1 << 16, dtype=torch_().float32, device=cuda)
