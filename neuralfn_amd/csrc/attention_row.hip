@@ -43,6 +43,7 @@
 #include "wave_rows.hpp"
 
 #include <algorithm>
+#include <cfloat>
 #include <type_traits>
 
 namespace nfn {
@@ -409,13 +410,14 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
     }
 
     // The running maximum and denominator of head i (the same in every wave) and dimensions 16w + 4j + r of its sum
-    // start with the current row, of weight 1 (NaN for an infinite score).
+    // start with the current row, of weight 1; NaN for a score of +inf, and 0 for -inf, which leaves NaN only where no
+    // other key has a finite score (0 / 0).
     float maximum = -INFINITY;
     float denominator = 0.0f;
     f32x4 accumulator = {0.0f, 0.0f, 0.0f, 0.0f};
     if (has_row) {
         maximum = row_score[i];
-        denominator = expf(maximum - maximum);
+        denominator = maximum == -INFINITY ? 0.0f : expf(maximum - maximum);
         accumulator = f32x4{row_sum.x * denominator, row_sum.y * denominator, row_sum.z * denominator,
                             row_sum.w * denominator};
     }
@@ -455,12 +457,14 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
         const float next_maximum = fmaxf(
             maximum, fmaxf(fmaxf(fmaxf(maxima[0].x, maxima[0].y), fmaxf(maxima[0].z, maxima[0].w)),
                            fmaxf(fmaxf(maxima[1].x, maxima[1].y), fmaxf(maxima[1].z, maxima[1].w))));
-        const float keep = __expf(maximum - next_maximum);
+        // (without a finite score so far every weight is 0)
+        const float reference = fmaxf(next_maximum, -FLT_MAX);
+        const float keep = __expf(maximum - reference);
         maximum = next_maximum;
         float weight[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float exponent = fmaf(lower[r], scale, fmaf(chains[0][r], scale, -next_maximum));
+            const float exponent = fmaf(lower[r], scale, fmaf(chains[0][r], scale, -reference));
             weight[r] = 4 * j + r < count ? __expf(exponent) : 0.0f;
         }
         const float sum = across_j_sum((weight[0] + weight[1]) + (weight[2] + weight[3]));

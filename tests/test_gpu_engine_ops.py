@@ -545,6 +545,51 @@ def test_one_row_attention_rounds_no_more_than_a_block_of_every_row(cuda, query_
     assert max(errors["row"], errors["causal"]) <= 1.01 * errors["all"], errors
 
 
+@pytest.mark.parametrize("query_heads,kv_heads,keys,far", [
+    (32, 2, 0, 0), (32, 2, 5, 0), (48, 8, 250, 0), (32, 2, 700, 0),   # the current key alone, in one launch, in shares
+    (48, 8, 250, 130), (32, 2, 700, 300),                             # a whole step, whole shares without a finite score
+    (128, 32, 2100, 300),                                             # ... the first steps of a longer share
+])
+@pytest.mark.parametrize("own", [-np.inf, np.inf, -1e30, 0.0])
+def test_one_row_attention_of_infinite_scores(cuda, oracle, query_heads, kv_heads, keys, far, own):
+    """A key of score -inf (an infinite element, or products past float's range) has no weight beside others, alone it
+    leaves NaN; one of +inf leaves NaN.  `far`: cached keys from the first on of score -inf."""
+    if own == -1e30 and keys == 0:
+        own = -np.inf  # (the oracle's doubles reach further: alone, its score is finite)
+    rng = np.random.default_rng(keys + query_heads)
+    rows, scale = 3, 128 ** -0.5
+    query = rng.standard_normal((rows, query_heads, 128)).astype(np.float32)
+    key, value = (rng.standard_normal((rows, kv_heads, 128)).astype(np.float32) for _ in range(2))
+    rings = [rng.standard_normal((keys + 64, kv_heads, 128)).astype(np.float32) for _ in range(2)]
+    query[:, :, 3] = 1e30
+    key[:, :, 3], rings[0][:, :, 3], rings[0][:far, :, 3] = 0.0, 0.0, -1e30
+    key[rows - 1, :, 3] = own
+    rings = [oracle.to_bf16(ring.reshape(keys + 64, -1)) for ring in rings]
+    device_rings = [bf16_tensor(ring, cuda) for ring in rings]
+    workspace = engine_ops.gqa_decode_workspace(4 * query_heads, 128)
+    workspace.fill_(0xFF)
+
+    def compare(out, expected):
+        out, expected = out.cpu().numpy().reshape(-1, 128), np.asarray(expected).reshape(-1, 128)
+        assert np.array_equal(np.isnan(out), np.isnan(expected))
+        finite = ~np.isnan(expected)
+        assert np.abs(out[finite] - expected[finite]).max(initial=0.0) <= 4e-6
+
+    one = [to_device(a[rows - 1], cuda) for a in (query, key, value)]
+    with np.errstate(all="ignore"):
+        expected = oracle.gqa_decode(query[rows - 1], key[rows - 1], value[rows - 1], *rings, keys, 0, scale)
+        block = oracle.block_attention(query, key, value, *rings, keys, keys + rows, scale, True)
+    compare(engine_ops.gqa_decode(*one, *device_rings, keys, 0, scale, workspace=workspace), expected)
+    engine_ops.lend_attention_workspace(workspace)
+    try:
+        compare(engine_ops.gqa_decode(*one, *device_rings, keys, 0, scale), expected)
+    finally:
+        engine_ops.lend_attention_workspace(None)
+    if kv_heads < 32:  # (there, three rows' shares are too long for this kernel)
+        compare(engine_ops.block_attention(*(to_device(a, cuda) for a in (query, key, value)), *device_rings, keys,
+                                           keys + rows, scale, True, workspace=workspace), block)
+
+
 def test_block_attention_fails_closed(cuda):
     lib = tile_ops.load()
     x = torch_().zeros(1 << 16, dtype=torch_().float32, device=cuda)
