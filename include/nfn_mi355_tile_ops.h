@@ -717,7 +717,9 @@ int nfn_native_tile_glimmer_fused_decode_attention_float32_v1(
  * and `first_key_position` of the descriptor are ignored, the kernels read
  * *device_position when they run, so one captured graph serves every token.
  * With apply_rope (a local layer) the keys are the last `sliding_window` ones,
- * otherwise all from key 0.  1 <= sliding_window <= cache_capacity. */
+ * otherwise all from key 0.  1 <= sliding_window <= cache_capacity.  The caller
+ * sees to *device_position >= 0: of a negative one the cache takes no row, and
+ * the outputs are unspecified. */
 int nfn_native_tile_glimmer_fused_decode_attention_device_position_float32_v1(
     const NfnNativeTileGlimmerFusedDecodeAttentionDescriptorV1* descriptor,
     const int64_t* device_position,

@@ -386,15 +386,18 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
             float* key = tail.key_copy + head_offset;
             key[lane] = row_key.first;
             key[lane + kWave] = row_key.second;
-            // (the ring row that the new key takes is none that this call reads)
-            const std::uint32_t ring = static_cast<std::uint64_t>(position) < static_cast<std::uint64_t>(2 * kMostKeys)
-                ? static_cast<std::uint32_t>(position) % capacity
-                : static_cast<std::uint32_t>(position % static_cast<std::int64_t>(capacity));
-            const std::uint64_t cache_row = static_cast<std::uint64_t>(ring) * row_stride + head_offset;
-            how.key_cache[cache_row + lane] = to_bf16(row_key.first);
-            how.key_cache[cache_row + lane + kWave] = to_bf16(row_key.second);
-            how.value_cache[cache_row + lane] = to_bf16(row_value.first);
-            how.value_cache[cache_row + lane + kWave] = to_bf16(row_value.second);
+            // (the ring row that the new key takes is none that this call reads; a position below 0, which only device memory
+            // can hold, has none)
+            if (position >= 0) {
+                const std::uint32_t ring = position < 2 * kMostKeys
+                    ? static_cast<std::uint32_t>(position) % capacity
+                    : static_cast<std::uint32_t>(position % static_cast<std::int64_t>(capacity));
+                const std::uint64_t cache_row = static_cast<std::uint64_t>(ring) * row_stride + head_offset;
+                how.key_cache[cache_row + lane] = to_bf16(row_key.first);
+                how.key_cache[cache_row + lane + kWave] = to_bf16(row_key.second);
+                how.value_cache[cache_row + lane] = to_bf16(row_value.first);
+                how.value_cache[cache_row + lane + kWave] = to_bf16(row_value.second);
+            }
         }
     }
 

@@ -439,8 +439,9 @@ __global__ __launch_bounds__(kRmsThreads) void qk_norm_scale_rope_kernel(
                                            static_cast<float>(head_dim) + eps);
     float result = __fmul_rn(__fmul_rn(value, inverse), scale[0]);
     if (is_query) result = __fmul_rn(result, query_scale);
-    // a key head also goes to the cache (one row only), with its value head
-    const bool commits = !is_query && commit.key_cache != nullptr;
+    // a key head also goes to the cache (one row only; none for a position below 0, which only device memory can hold),
+    // with its value head
+    const bool commits = !is_query && commit.key_cache != nullptr && position >= 0;
     const std::int64_t cache_index = commits
         ? (position % commit.capacity) * commit.row_stride +
             static_cast<std::int64_t>(combined - query_heads) * head_dim

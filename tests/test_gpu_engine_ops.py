@@ -903,6 +903,21 @@ def test_fused_decode_attention_with_the_position_on_the_device(cuda, oracle, ap
                       workspace.numel()) == 1
 
 
+@pytest.mark.parametrize("apply_rope", [True, False])  # norms and commit in the attention's launch, and in their own
+def test_a_negative_position_on_the_device_commits_nothing(cuda, apply_rope):
+    torch = torch_()
+    generator = torch.Generator(device=cuda).manual_seed(8)
+    def draw(*shape):
+        return torch.randn(shape, generator=generator, device=cuda)
+    query, key, value, rings = draw(32, 128), draw(2, 128), draw(2, 128), draw(2, 512, 256).to(torch.bfloat16).view(torch.int16)
+    before = rings.clone()
+    out = engine_ops.fused_decode_attention(
+        query, key, value, rings[0][128:256], rings[1][128:256], 0, 0, 128 ** -0.5, apply_rope=apply_rope,
+        device_position=torch.tensor([-3], device=cuda), sliding_window=100, workspace=engine_ops.gqa_decode_workspace(32, 128))
+    assert torch.equal(rings, before)  # neither the ring nor the rows around it
+    assert torch.equal(out.reshape(2, 16, 128), value[:, None].expand(2, 16, 128))  # the current key alone
+
+
 def test_lent_workspace_turns_the_reference_named_calls_into_their_split_forms(cuda, oracle):
     rng = np.random.default_rng(41)
     query_heads, kv_heads, head_dim, capacity, position = 32, 2, 128, 2048, 3000
