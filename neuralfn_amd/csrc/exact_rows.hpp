@@ -20,6 +20,7 @@
 #include <utility>
 
 #include "common.hpp"
+#include "q6_words.hpp"
 #include "wave_rows.hpp"
 
 namespace nfn {
@@ -105,9 +106,9 @@ struct ExactUnit<kEncQ6K> {
     std::uint32_t codes_of_scale, d;
     float scale[4];
     int upper;
-    __device__ __forceinline__ void load(const std::uint8_t* row, int unit) {
+    __device__ __forceinline__ void load(const std::uint8_t* tensor, const std::uint8_t* row, int unit) {
         const std::uint8_t* block = row + (unit >> 2) * 210;
-        shift = static_cast<std::uint32_t>(reinterpret_cast<std::uintptr_t>(block)) & 2u;
+        shift = q6_past_word(reinterpret_cast<std::uintptr_t>(tensor), reinterpret_cast<std::uintptr_t>(block));
         const std::uint8_t* lower = block - shift + ((unit >> 1) & 1) * 64;
         const std::uint8_t* top = block - shift + 128 + ((unit >> 1) & 1) * 32;
 #pragma unroll
@@ -287,7 +288,12 @@ __device__ __forceinline__ void exact_rows_walk(const std::uint8_t* __restrict__
         const int unit = min(lane + span * turn, units - 1);
 #pragma unroll
         for (int k = 0; k < kExactPair; ++k) {
-            into[k].load(data + min(pair * kExactPair + k, output_dim - 1) * row_stride, unit);
+            const std::uint8_t* row = data + min(pair * kExactPair + k, output_dim - 1) * row_stride;
+            if constexpr (ENC == kEncQ6K) {
+                into[k].load(data, row, unit);
+            } else {
+                into[k].load(row, unit);
+            }
         }
     };
     load(now, first_pair, 0);

@@ -374,7 +374,8 @@ __global__ __launch_bounds__(kRowsThreads, 2) void gemv_rows_kernel(
 #pragma unroll
         for (int i = 0; i < F::kLoads; ++i) {
             if constexpr (F::kQ6 || F::kQ8) {
-                // (Q8_0 rows are only as aligned as the tensor; Q6_K pieces start on a word)
+                // (Q8_0 rows are only as aligned as the tensor; Q6_K pieces start on a word, those of a tensor that does not
+                // two bytes before it: the same aligned word, which is there, and what it brings is shifted out)
                 const std::uint32_t back = F::kQ6 ? ((shifted >> i) & 1u) * 2u : 0u;
                 const RowsPiece piece = *reinterpret_cast<const RowsPiece*>(weights + chunk_offset[i] - back);
                 stage.chunk[i] = v4u{piece.v[0], piece.v[1], piece.v[2], piece.v[3]};

@@ -59,6 +59,7 @@
 // Weight layouts and decode: neuralfn/csrc/native_gpt2/resident_glimmer.cpp:542-616.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "q6_words.hpp"
 
 #include <algorithm>
 
@@ -236,23 +237,23 @@ struct Unit<kEncQ6K> {
     std::uint32_t scales;   // the unit's four sub-scales, (step, chunk) at byte 2 step + chunk
     std::uint32_t d;        // in the upper half
     int upper;
-    __device__ __forceinline__ static std::uint32_t past_word(const std::uint8_t* row, int unit) {
-        return (static_cast<std::uint32_t>(reinterpret_cast<std::uintptr_t>(row)) + 2u * (unit >> 2)) & 2u;
+    __device__ __forceinline__ static std::uint32_t past_word(const std::uint8_t* tensor, const std::uint8_t* row, int unit) {
+        return q6_past_word(reinterpret_cast<std::uintptr_t>(tensor), reinterpret_cast<std::uintptr_t>(row) + 2u * (unit >> 2));
     }
-    __device__ __forceinline__ void load(const std::uint8_t* row, int unit, int half) {
+    __device__ __forceinline__ void load(const std::uint8_t* tensor, const std::uint8_t* row, int unit, int half) {
         typedef std::uint32_t u32_a2 __attribute__((aligned(2)));
         const std::uint8_t* block = row + (unit >> 2) * 210;
         const int half_block = (unit >> 1) & 1;
         upper = unit & 1;  // quarters 2 and 3 of the half block: high nibbles, high-bit pairs 2 and 3
-        const std::uint8_t* word = block - past_word(row, unit);
+        const std::uint8_t* word = block - past_word(tensor, row, unit);
         low[0] = *reinterpret_cast<const u32x4_a4*>(word + half_block * 64 + 16 * half);
         low[1] = *reinterpret_cast<const u32x4_a4*>(word + half_block * 64 + 32 + 16 * half);
         high = *reinterpret_cast<const u32x4_a4*>(word + 128 + half_block * 32 + 16 * half);
         beyond = *reinterpret_cast<const std::uint32_t*>(word + (half != 0 ? 160 + 32 * half_block : 64 + 64 * half_block));
         scales = *reinterpret_cast<const u32_a2*>(block + (half != 0 ? 192 + 4 * (unit & 3) : 206));
     }
-    __device__ __forceinline__ void align(const std::uint8_t* row, int unit) {
-        const std::uint32_t shift = past_word(row, unit);
+    __device__ __forceinline__ void align(const std::uint8_t* tensor, const std::uint8_t* row, int unit) {
+        const std::uint32_t shift = past_word(tensor, row, unit);
         if (__ballot(shift != 0) == 0) return;
         // each piece's following word lies in the other lane of the row or, behind the last, in `beyond`
         const bool second = (threadIdx.x & 32) != 0;
@@ -482,8 +483,11 @@ __device__ __forceinline__ void multiply(f32x16 (&acc)[MT], const Terms (&a)[MT]
 }
 
 template <std::uint32_t ENC>
-__device__ __forceinline__ void load_unit(Unit<ENC>& into, const std::uint8_t* row, int unit, int half, int steps) {
-    if constexpr (kWholeBlocks<ENC>) {
+__device__ __forceinline__ void load_unit(Unit<ENC>& into, const std::uint8_t* tensor, const std::uint8_t* row, int unit,
+                                          int half, int steps) {
+    if constexpr (ENC == kEncQ6K) {
+        into.load(tensor, row, unit, half);
+    } else if constexpr (kWholeBlocks<ENC>) {
         into.load(row, unit, half);
     } else {
         into.load(row, unit, half, steps);
@@ -795,7 +799,7 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
             if constexpr (PAIRS) {
                 into.load_pair(row, unit, half);
             } else {
-                load_unit<ENC>(into, row, unit, half, steps);
+                load_unit<ENC>(into, data, row, unit, half, steps);
             }
         };
 #pragma unroll
@@ -808,7 +812,7 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES >= 16 ? 4 : 2) void linear_exa
         for (int unit = first_unit; unit < end_unit; ++unit) {
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
-                if constexpr (ENC == kEncQ6K) now[n].align(w_row[n], unit);
+                if constexpr (ENC == kEncQ6K) now[n].align(data, w_row[n], unit);
                 if constexpr (PAIRS) {
                     now[n].arrange_pair();
                 } else {
