@@ -1378,11 +1378,14 @@ template <std::uint32_t ENC, int MT, int NT, int WAVES>
 void launch_small(const Descriptor& weight, const float* input, const float* bias, float* output, std::int64_t rows,
                   hipStream_t stream) {
     if constexpr (WAVES == 16 && kWholeBlocks<ENC>) {
-        // Walks of up to three units a wave, through LDS and not: 16 rows of Q6_K 512 -> 300 5.8 and 5.5 us, 768 -> 300
-        // 6.1 and 6.4, 17 rows 2,048 -> 1,700 10.9 and 10.0, 32 rows 1,024 -> 300 7.5 and 7.2, 1,280 -> 1,700 10.5 and
-        // 11.5; 25 rows of Q4_K 2,560 -> 8,000 14.3 and 13.7, 3,072 -> 2,000 12.9 and 13.4, and 2,048 -> 300 9.1 and 10.3.
+        // Short walks, the same bits with or without the way through LDS.  Q6_K from 1,155 shapes of 7 to 64 rows, 512 to 3,072
+        // columns and 64 to 6,656 outputs, geometric means of the time through LDS over the time without: up to 8 rows 0.95 to
+        // 0.97 at 512 to 1,024 columns; 9 to 16 rows 1.03 to 1.05 there, 0.94 to 0.96 at 1,280; 17 to 20 rows 1.17 to 1.21 there,
+        // 1.01 to 1.07 at 1,280 to 2,560, 0.97 to 0.99 at 2,816; more rows 1.04 to 1.21 up to 1,024, 1.00 to 1.05 up to 1,536,
+        // 0.95 to 1.02 at 1,792.  Q4_K and Q5_K: 25 rows of Q4_K 2,560 -> 8,000 14.3 and 13.7 us, 3,072 -> 2,000 12.9 and
+        // 13.4, and 2,048 -> 300 9.1 and 10.3.
         const bool wide = (weight.output_dim + 31) / 32 * 3 > compute_units();
-        const std::int64_t q6_columns = rows > 20 ? 1024 : rows > 16 ? 2048 : 512;
+        const std::int64_t q6_columns = rows <= 8 ? 0 : rows <= 16 ? 1024 : rows <= 20 ? 2560 : 1536;
         if (ENC == kEncQ6K ? weight.input_dim <= q6_columns : rows > 16 && weight.input_dim <= 2560 && wide) {
             return launch_small_form<ENC, MT, NT, WAVES, 0>(weight, input, bias, output, rows, stream);
         }
