@@ -547,6 +547,9 @@ constexpr std::int64_t kAloneKeys = 256;
 // 1,500) 16.8 / 16.3; 768 (16 of 32 over 8, 1,500) 19.6 / 19.5; 1,024 (16 of 32 over 8, 2,000) 23.4 / 22.2; 1,280 (16 of 32
 // over 4, 4,802) 24.0 / 22.4, but (of 32 over 8, 2,500) 24.6 / 25.3; 2,176 (16 of 48 over 2, 8,192) 34.6 / 35.1; 4,224 (16
 // of 32 over 8, 8,192) 57.4 / 58.4.  (Two workgroups a unit: 128 registers, of which 31 go to scratch memory, 64.7 and 117.)
+// One row alone has no such limit: at 512 to 8,192 keys a share (16 heads over 1 to 256 over 64, up to 524,288 keys) it takes
+// 0.80 to 0.95 of attention_grouped_kernel's time, with norms, rotation and commit 0.76 to 0.95; at 1,024 and 2,048 keys a
+// share, which lie whole powers of two apart in the ring, 0.88 to 1.00 and 0.82 to 0.96.
 constexpr std::int64_t kBlockKeys = 1024;
 
 bool overlap(const void* a, std::int64_t a_bytes, const void* b, std::int64_t b_bytes) {
