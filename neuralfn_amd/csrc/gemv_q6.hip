@@ -793,6 +793,8 @@ std::int64_t launch_stream(const ProjectionSet& set, const float* first, const f
         waves += op_waves;
     }
     const std::int64_t blocks = set.input_dim >> 8;
+    // (a guard for the packed arguments, which no call on this chip comes to: 256 units have some 33,000 waves at most, 65,536
+    // rows a wave would be a billion rows, a row has a few hundred blocks and a call sixteen tokens)
     if (waves > 0xffff - W || rows_per_wave > 0xffff || tokens > 0x3f || blocks > 0x3ff) {
         return launch_variant<T, P, ARGMAX>(set, first, second, records_out, tokens, candidates, stream);
     }

@@ -1327,6 +1327,24 @@ def test_q6_k_long_rows_one_token_and_verifier(cuda, oracle, shape):
     assert_bits_equal(one, batched[:1], "mmq at one row")
 
 
+@pytest.mark.parametrize("out_dims", [(1301, 257, 63, 910), (1, 4097, 2), (513, 1)])
+@pytest.mark.parametrize("in_dim", [4352, 6656])
+def test_q6_k_long_rows_grouped_projections_end_in_partial_waves(cuda, oracle, in_dim, out_dims):
+    """Where each projection's waves begin and how many rows its last one lacks reach the streaming kernel packed: every
+    projection of a call has the bits of its own call, for one token and for two and three of the verifier."""
+    x = kquant.synthetic_activations(66, 3, in_dim)
+    packed = [random_packed(kquant.Q6_K, out_dim, in_dim, 67 + out_dim) for out_dim in out_dims]
+    weights = [tile_ops.PackedWeight.from_numpy(kquant.Q6_K, p, out_dim, in_dim) for p, out_dim in zip(packed, out_dims)]
+    workspace = tile_ops.small_batch_workspace(3, in_dim)
+    for rows, family in ((1, "mmq"), (1, "mmvq"), (2, "mmvq"), (3, "mmvq")):
+        together = tile_ops.multi_linear(weights, to_device(x[:rows], cuda), workspace, family=family)
+        for weight, y in zip(weights, together):
+            alone = tile_ops.multi_linear([weight], to_device(x[:rows], cuda), workspace, family=family)[0]
+            assert_bits_equal(y, alone, f"{weight.output_dim} outputs, {rows} rows")
+    for p, out_dim, y in zip(packed, out_dims, together):
+        assert normalised_error(y.cpu().numpy(), oracle.linear(kquant.Q6_K, p, out_dim, in_dim, x)) <= TOLERANCE
+
+
 @pytest.mark.parametrize("per_unit,in_dim,prologue", [(8.0, 12288, "plain"), (11.99, 12544, "swiglu"),
                                                       (17.3, 16384, "plain"), (23.9, 12288, "gated")])
 def test_q6_k_long_rows_with_fewer_waves_a_workgroup(cuda, oracle, per_unit, in_dim, prologue):
