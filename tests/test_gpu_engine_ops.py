@@ -137,6 +137,19 @@ def test_rope_batch_against_oracle(cuda, oracle, layout, inverse):
         assert_bits_equal(k1, k[0])
 
 
+@pytest.mark.parametrize("head_dim", [80, 96, 192, 256])
+@pytest.mark.parametrize("position,theta", [(1_000_003, 500000.0), (9_999_999, 10000.0), (131071, 3.0)])
+def test_rope_of_head_sizes_that_are_no_power_of_two(cuda, oracle, head_dim, position, theta):
+    """The frequency's exponent is a rounded quotient then.  An angle of 10^7 in double is 1e-9 off, the result a rounding
+    of float each for two products and a sum of numbers up to 5."""
+    query = np.random.default_rng(head_dim).standard_normal((4, head_dim)).astype(np.float32)
+    for layout in (engine_ops.ROPE_HALF_SPLIT, engine_ops.ROPE_INTERLEAVED):
+        q, k = to_device(query, cuda), to_device(query[:2], cuda)
+        engine_ops.rope(q, k, position, theta, layout)
+        assert np.abs(q.cpu().numpy() - oracle.rope(query, position, theta, layout == 1, False)).max() <= 5e-7
+        assert_bits_equal(k, q[:2])
+
+
 def test_rope_fails_closed(cuda):
     lib = tile_ops.load()
     x = torch_().zeros(64, dtype=torch_().float32, device=cuda)
