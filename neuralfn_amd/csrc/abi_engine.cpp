@@ -176,8 +176,9 @@ int run_fused_decode(const NfnNativeTileGlimmerFusedDecodeAttentionDescriptorV1*
     }
     const hipStream_t stream = as_stream(d->cuda_stream);
     if (split_partials == nullptr) split_partials = lent_partials(d->cuda_stream, d->query_heads, d->head_dim);
-    // The new cache row is written by the first launch, before the attention
-    // runs: right as long as the attention does not read that ring row, which
+    // The new cache row is written by the norm launch, before the attention
+    // runs, or by the attention launch itself where that takes the norms along:
+    // right as long as the attention does not read that ring row, which
     // holds for every key range shorter than the ring (and for the device
     // form, whose window is at most the ring).  Otherwise the commit follows.
     const bool commit_first = on_device || d->position - d->first_key_position < d->cache_capacity;

@@ -104,10 +104,13 @@ __device__ __forceinline__ float score_block_key(const float* q, const float* ke
     return dot;
 }
 
-// The key range of one query row, and how many waves share it.  The split
-// depends on the row's key count only, not on the launch: a row of a causal
-// block then sums in the same order as the one-token call at the same
-// position, and gives the same bits.
+// The key range of one query row, and how many waves share it.  Without shares
+// (a.partials) that depends on the row's key count only, not on the launch: a row
+// of a causal block then sums in the same order as the one-token call at the
+// same position, and gives the same bits while both run on the same kernel.
+// Shares are cut by what else the launch has to do: to rounding then, here as
+// in attention_row.hip (whose blocks of up to 256 keys a row have no shares, nor
+// has the one-token call of so many, and agree bit for bit).
 struct KeyRange {
     std::int64_t first, last;
     int active;
@@ -768,16 +771,6 @@ __device__ __forceinline__ QueryTerms split_query(const float (&x)[8]) {
     terms.middle = __builtin_bit_cast(bf16x8, make_uint4(words[1][0], words[1][1], words[1][2], words[1][3]));
     terms.low = __builtin_bit_cast(bf16x8, make_uint4(words[2][0], words[2][1], words[2][2], words[2][3]));
     return terms;
-}
-
-// eight floats as the bf16 row the cache would hold of them
-__device__ __forceinline__ uint4 pack_as_cached(float4 low, float4 high) {
-    const auto pair = [](float first, float second) {
-        return static_cast<std::uint32_t>(to_bf16(first)) |
-            (static_cast<std::uint32_t>(to_bf16(second)) << 16);
-    };
-    return make_uint4(pair(low.x, low.y), pair(low.z, low.w), pair(high.x, high.y),
-                      pair(high.z, high.w));
 }
 
 __global__ __launch_bounds__(kGroupWaves * kWave) void attention_grouped_kernel(AttentionArguments a) {

@@ -65,6 +65,14 @@ void launch_attention_merge(const float* partials, float* output, int splits, st
                             float* query, const float* key_copy, float* key, std::int64_t key_floats,
                             hipStream_t stream);
 
+// eight floats as the bf16 row the cache would hold of them
+__device__ __forceinline__ uint4 pack_as_cached(float4 low, float4 high) {
+    const auto pair = [](float first, float second) {
+        return static_cast<std::uint32_t>(to_bf16(first)) | (static_cast<std::uint32_t>(to_bf16(second)) << 16);
+    };
+    return make_uint4(pair(low.x, low.y), pair(low.z, low.w), pair(high.x, high.y), pair(high.z, high.w));
+}
+
 // x = high + middle + low exactly, every term a bf16 in the upper half of a word: each takes the next eight
 // significant bits of what is left (truncation, so the remainders are exact; eight at most are left for the last,
 // whose lower half holds none of them)

@@ -75,14 +75,6 @@ struct RowTail {
     RowPreparation preparation;
 };
 
-// eight floats as the bf16 row the cache would hold of them
-__device__ __forceinline__ uint4 pack_as_cached(float4 low, float4 high) {
-    const auto pair = [](float first, float second) {
-        return static_cast<std::uint32_t>(to_bf16(first)) | (static_cast<std::uint32_t>(to_bf16(second)) << 16);
-    };
-    return make_uint4(pair(low.x, low.y), pair(low.z, low.w), pair(high.x, high.y), pair(high.z, high.w));
-}
-
 // the four lanes (., i) of a wave meet
 __device__ __forceinline__ float across_j_max(float value) {
     auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(value), __float_as_uint(value), false, false);

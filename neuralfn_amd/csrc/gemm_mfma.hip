@@ -610,8 +610,6 @@ constexpr int kSecondRun = kParts<ENC> == 2 ? 64 : 64 * kRowBytes;
 template <std::uint32_t ENC>
 constexpr int kRunSecond = ENC == kEncQ4K || ENC == kEncQ5K ? 64 : 16;
 
-// The activation fragments of one K step for one wave: row blocks 0 and 1,
-// K chunks 0..3, in named registers (an array here ends up in scratch memory).
 // What a lane wrote to LDS is seen by the wave's other lanes, and no access moves across (no instruction of its own).
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -619,6 +617,8 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The activation fragments of one K step for one wave: row blocks 0 and 1,
+// K chunks 0..3, in named registers (an array here ends up in scratch memory).
 struct ActivationSlice {
     f16x8 r0k0, r0k1, r0k2, r0k3, r1k0, r1k1, r1k2, r1k3;
 };

@@ -437,11 +437,12 @@ __device__ __forceinline__ Projection tile_projection(const ProjectionSet& set, 
 constexpr int kGroupTiles = 2;  // tiles a workgroup accumulates side by side
 
 // A workgroup takes its tiles in groups of up to kGroupTiles and K in chunks of
-// 8 x kDepth blocks.  Per (group, chunk) a wave loads the activation fragments
-// of its share of the chunk (at most kDepth blocks) once, into registers, and
-// walks the group's tiles: step s of every tile uses fragment set s and stage
-// s, so only packed weights stream, kDepth steps (one tile) ahead.  Rows of up
-// to 8,192 columns are one chunk: the fragments are loaded once per launch.
+// 8 x DEPTH blocks.  Per (group, chunk) a wave loads the activation fragments
+// of its share of the chunk (at most DEPTH blocks) once, into registers, and
+// walks the group's tiles: step s of every tile uses fragment set s, so only packed
+// weights stream: kDepth steps (one tile) ahead into stage s, or with kShortDepth the
+// steps of two tiles into the stages of both.  Rows of up to 8,192 columns (kShortDepth:
+// all that it takes) are one chunk: the fragments are loaded once per launch.
 // After the last chunk the eight waves' partial sums of the group meet in LDS.
 //
 // kArgmax (the lm_head, one projection): instead of storing the results, the wave that adds up
@@ -586,10 +587,10 @@ __global__ __launch_bounds__(kThreads) void gemv_f16_kernel(
     // Every wave walks the same stream of (group, chunk, tile of the group, step)
     // in uniform control flow (a group's tiles: kGroupTiles, fewer in the last group).
     //
-    // Plain form: weight loads run kDepth steps ahead; they are
+    // Plain form: weight loads run kAhead tiles of DEPTH steps ahead; they are
     // unconditional (a step without work reads the first bytes of the first
     // projection, one line for the whole wave), so a step waits for nothing but
-    // its own.  The fetch cursor walks the same stream, one tile ahead.
+    // its own.  The fetch cursor walks the same stream, kAhead tiles ahead.
     // kQuadFetch: lane l asks for quarter l % 4 of row l / 4, so that the four lanes of a quad
     // read neighbouring bytes of one row; the matrix instruction wants quarter l / 16 of row
     // l % 16 in lane l, and a step's registers change lanes before use (Q6_K at 16 rows,

@@ -217,5 +217,5 @@ def verify_layer(geometry: LayerGeometry, weights: LayerWeights, cache: LayerCac
 
 
 LAUNCHES_PER_LAYER = 8           # with the reference's fused attention call
-LAUNCHES_PER_LAYER_SPLIT = 8     # with the split attention form (its merge, but norms, rope and commit inside)
-LAUNCHES_PER_LAYER_FUSED = 7     # ... and the first dual norm inside the Q/K/V/gate launch
+LAUNCHES_PER_LAYER_FUSED = 7     # with the split attention form (its merge, but norms, rope and commit inside) and the first
+                                 # dual norm inside the Q/K/V/gate launch
