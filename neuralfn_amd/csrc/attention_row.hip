@@ -75,6 +75,10 @@ struct RowTail {
     RowPreparation preparation;
 };
 
+// What the lower two terms of a float contribute to its products with a bf16.  Where that is infinite and a lower term 0 the
+// contribution is NaN and the upper term's product, an infinity, says it all; NaN for any other reason is in both.
+__device__ __forceinline__ float finite_part(float lower) { return __builtin_amdgcn_fmed3f(lower, -FLT_MAX, FLT_MAX); }
+
 // the four lanes (., i) of a wave meet
 __device__ __forceinline__ float across_j_max(float value) {
     auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(value), __float_as_uint(value), false, false);
@@ -440,7 +444,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
         float largest = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            lower[r] = chains[2][r] + chains[1][r];
+            lower[r] = finite_part(chains[2][r] + chains[1][r]);
             largest = fmaxf(largest, 4 * j + r < count ? (lower[r] + chains[0][r]) * scale : -INFINITY);
         }
         largest = across_j_max(largest);
@@ -507,7 +511,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void attention_row_kernel(
              ((parts[1].x + parts[1].y) + (parts[1].z + parts[1].w)));
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            accumulator[r] = accumulator[r] * keep + ((sums[2][r] + sums[1][r]) + sums[0][r]);
+            accumulator[r] = accumulator[r] * keep + (finite_part(sums[2][r] + sums[1][r]) + sums[0][r]);
         }
     }
 

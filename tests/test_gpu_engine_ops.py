@@ -603,6 +603,40 @@ def test_one_row_attention_of_infinite_scores(cuda, oracle, query_heads, kv_head
                                            keys + rows, scale, True, workspace=workspace), block)
 
 
+@pytest.mark.parametrize("query_heads,kv_heads,keys", [(32, 2, 1), (16, 4, 20), (32, 2, 63), (48, 8, 200), (32, 2, 700)])
+@pytest.mark.parametrize("where", ["key", "value", "own value"])
+def test_one_row_attention_of_infinite_keys_and_values(cuda, oracle, query_heads, kv_heads, keys, where):
+    """Queries of bf16 values and keys whose weights are 1 have lower terms of 0 on the matrix cores: with an infinite key
+    or value they give what the number itself gives, an infinity or no weight, and not NaN."""
+    rng = np.random.default_rng(keys)
+    rows, scale = 2, 128 ** -0.5
+    query = oracle.bf16_to_float(oracle.to_bf16(rng.standard_normal((rows, query_heads, 128)).astype(np.float32)))
+    key, value = (rng.standard_normal((rows, kv_heads, 128)).astype(np.float32) for _ in range(2))
+    rings = [rng.standard_normal((keys + 64, kv_heads * 128)).astype(np.float32) for _ in range(2)]
+    if where == "key":  # of score -inf for queries above 0, +inf (NaN) below
+        rings[0][keys // 2, 7] = -np.inf
+    elif where == "value":
+        rings[1][keys // 2, 7], rings[1][0, 9] = np.inf, -np.inf
+    else:
+        value[rows - 1, :, 7] = np.inf
+    rings = [oracle.to_bf16(ring) for ring in rings]
+    device_rings = [bf16_tensor(ring, cuda) for ring in rings]
+    workspace = engine_ops.gqa_decode_workspace(2 * query_heads, 128)
+    workspace.fill_(0xFF)
+    with np.errstate(all="ignore"):
+        cases = ((engine_ops.gqa_decode(*(to_device(a[-1], cuda) for a in (query, key, value)), *device_rings, keys, 0, scale,
+                                        workspace=workspace),
+                  oracle.gqa_decode(query[-1], key[-1], value[-1], *rings, keys, 0, scale)),
+                 (engine_ops.block_attention(*(to_device(a, cuda) for a in (query, key, value)), *device_rings, keys, keys + rows,
+                                             scale, True, workspace=workspace),
+                  oracle.block_attention(query, key, value, *rings, keys, keys + rows, scale, True)))
+    for out, expected in cases:
+        out, expected = out.cpu().numpy().reshape(-1), np.asarray(expected).reshape(-1)
+        finite = np.isfinite(expected)
+        assert np.array_equal(out[~finite], expected[~finite], equal_nan=True) and np.isfinite(out[finite]).all()
+        assert np.abs(out[finite] - expected[finite]).max(initial=0.0) <= 4e-6
+
+
 def test_block_attention_fails_closed(cuda):
     lib = tile_ops.load()
     x = torch_().zeros(1 << 16, dtype=torch_().float32, device=cuda)
